@@ -45,28 +45,28 @@ def _case(name, model, size="", weights="bf16", prompts=0, lo=0, hi=0, past=0, d
 def listed():
     return [
         # one user waiting for one token: the latency of a step that is nothing but launches and weights
-        _case("dense decode, one sequence", "dense", decodes=1, past_lo=128, past_hi=128),
+        _case("dense decode 1 x 128", "dense", decodes=1, past_lo=128, past_hi=128),
         # the headline workload: 32 sequences at 1024 tokens of context
-        _case("dense decode, 32 x 1024", "dense", decodes=32, past_lo=1024, past_hi=1024),
+        _case("dense decode 32 x 1024", "dense", decodes=32, past_lo=1024, past_hi=1024),
         # a busy server (up to 256 requests in flight, 100-1024 tokens each): ragged contexts
-        _case("dense decode, 200 ragged", "dense", decodes=200, past_lo=100, past_hi=1024),
+        _case("dense decode 200 ragged", "dense", decodes=200, past_lo=100, past_hi=1024),
         # fp8 weights, the batch of the shared-prefix workload
-        _case("dense decode, fp8 weights", "dense", weights="fp8", decodes=64, past_lo=512, past_hi=1100),
+        _case("dense decode fp8 weights", "dense", weights="fp8", decodes=64, past_lo=512, past_hi=1100),
         # one short question arriving: what its time to first token consists of
-        _case("dense prefill, 137 tokens", "dense", prompts=1, lo=137, hi=137),
+        _case("dense prefill 137 tokens", "dense", prompts=1, lo=137, hi=137),
         # a full house of prompts: the step that sets the headline's time to first token
-        _case("dense prefill, 16 x 1024", "dense", prompts=16, lo=1024, hi=1024),
+        _case("dense prefill 16 x 1024", "dense", prompts=16, lo=1024, hi=1024),
         # sparse feed-forwards: every expert is hit in a decode batch
-        _case("moe decode, 32 x 1024", "moe", "w2048", decodes=32, past_lo=1024, past_hi=1024),
+        _case("moe decode 32 x 1024", "moe", "w2048", decodes=32, past_lo=1024, past_hi=1024),
         # recurrent + window-attention layers: a decode batch, ...
-        _case("gazutar decode, 32 x 1024", "gazutar", "w2048", decodes=32, past_lo=1024, past_hi=1024),
+        _case("gazutar decode 32 x 1024", "gazutar", "w2048", decodes=32, past_lo=1024, past_hi=1024),
         # ... a prefill step of ragged prompts, ...
-        _case("gazutar prefill, 11 ragged", "gazutar", "w1024", prompts=11, lo=77, hi=1400),
+        _case("gazutar prefill 11 ragged", "gazutar", "w1024", prompts=11, lo=77, hi=1400),
         # ... and the exact serving mode: portions of prompts beside decoded tokens, everything in 32 bits
         _case("gazutar float32 mixed step", "gazutar", "w1024", "f32", prompts=3, lo=101, hi=400, past=130, decodes=13, past_lo=60, past_hi=700),
         # latent attention and linear attention: a prefill step at the larger size, a decode batch at the smaller one
-        _case("felolorn prefill, 8 x 1024", "felolorn", "w2048", prompts=8, lo=1024, hi=1024),
-        _case("felolorn decode, 24 ragged", "felolorn", "w1024", decodes=24, past_lo=30, past_hi=1500),
+        _case("felolorn prefill 8 x 1024", "felolorn", "w2048", prompts=8, lo=1024, hi=1024),
+        _case("felolorn decode 24 ragged", "felolorn", "w1024", decodes=24, past_lo=30, past_hi=1500),
     ]
 
 
