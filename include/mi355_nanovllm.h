@@ -753,6 +753,20 @@ int mi_gemm_any_act(const float* x, int64_t ldx, const void* w, const void* w2, 
  * act2_from (>= act_from) on - projections of one input that need different activations as one product. */
 int mi_gemm_any_segments(const float* x, int64_t ldx, const void* w, int w_dtype, const float* bias, int act, int act_from,
                          int act2, int act2_from, float* y, int64_t ldy, int M, int N, int K, int exact, mi_stream stream);
+/* The same products for prompt-sized steps over bf16 weights, in two parts: x rounded to bf16 once - gathered into the groups'
+ * order - and the MFMA tile kernels over it.  mi_gemm_any_tile_rows: rows of a tile (128 or 256) or 0 when the shape does not
+ * pay or is not taken (bf16 weights, K % 64 == 0, N % 4 == 0, activations of the shapes in use, n_groups <= 1024; n_groups 0:
+ * no groups).  mi_gemm_any_table_ints: int32s of the tile table of a grouped operand.  mi_gemm_any_operand: xb[r] = bf16 of
+ * x[x_rows ? x_rows[r] : r] for the rows r before group_offsets[n_groups] (all rows without groups), and the table (may be NULL).
+ * mi_gemm_any_tile: y[y_rows ? y_rows[r] : r] = epilogue of mi_gemm_any_act / mi_gemm_any_grouped_glu, fp32 or bf16. */
+int mi_gemm_any_tile_rows(int rows, int N, int K, int n_groups, int dual, int act);
+int64_t mi_gemm_any_table_ints(int rows, int n_groups, int tile_rows);
+int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets, int n_groups,
+                        int tile_rows, int rows, int K, mi_bf16* xb, int32_t* table, mi_stream stream);
+int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int tile_rows, const mi_bf16* w, const mi_bf16* w2,
+                     const float* bias, const float* bias2, int act, float limit, const float* row_scale,
+                     const int32_t* row_scale_rows, int n_groups, void* y, int y_is_bf16, int64_t ldy,
+                     const int32_t* y_rows, int rows, int N, int K, float alpha, mi_stream stream);
 /* mi_gemm_any_grouped with the activation named: y = act(x w^T) (* (x w2^T) with w2). */
 int mi_gemm_any_grouped_act(const float* x, int64_t ldx, const int32_t* x_rows, const void* w, const void* w2, int w_dtype,
                             int act, const int32_t* group_offsets, int n_groups, int rows_per_group_max, float* y,

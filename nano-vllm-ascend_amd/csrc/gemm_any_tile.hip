@@ -1,0 +1,231 @@
+// The prompt-sized projections of the 32-bit-residual model families on the large MFMA tile kernels: fp32 activations are
+// rounded to bf16 once, into an operand buffer (gathered into the experts' order on the way), and multiplied by the tile
+// kernels of gemm_tile.hip with an fp32 epilogue.
+//
+// What bounds it: the products are MFMA-bound from a few hundred rows on.  The kernel these shapes ran on before
+// (gemm_any_mfma_kernel: x converted by every feature tile again, operands through registers into LDS, two barriers per K
+// step) reached 200-350 TFLOP/s; the tile kernels fetch both operands with LDS-DMA, which needs them in bf16 - hence the
+// pass over x, which reads and writes 6 bytes per element once and is paid back from the second feature tile on.
+// Measured, 8192 rows: 2048 x 2048 207 -> 75 us + 15 us of operand pass; 64 experts x 8 per row, 2048 -> 2 x 768 with SwiGLU
+// 1192 -> 523 us (790 TFLOP/s), back to 2048 1050 -> 250 us.  Bits: one fp32 chain over k per result, k ascending, from
+// the same rounded operands as gemm_any_mfma_kernel's - the same bits.
+#include "gemm_tile_args.hpp"
+
+namespace mi {
+
+// Table of a grouped operand: {row tiles, 0, 0, 0}, then per row tile {group, first row, end of the group's rows, 0}.
+template <int ACT, bool DUAL>
+struct AnyTileArgs : TileArgs {
+  static constexpr int kAct = ACT;
+  static constexpr bool kDual = DUAL;
+  const uint16_t* w2;
+  int groups;
+  const int32_t* table;  // nullptr: one group of M rows
+  float* y32;
+  uint16_t* y16;         // != nullptr: the results as bf16 instead
+  const int32_t* y_rows;
+  const float* bias1;
+  const float* bias2;
+  float alpha, limit;
+  const float* row_scale;
+  const int32_t* row_scale_rows;
+};
+
+// the operand's table is read through the scalar cache: it was written by an earlier launch and is the same for a whole wave
+typedef const __attribute__((address_space(4))) int32_t* ConstInts;
+template <class A>
+__device__ __forceinline__ int any_tiles(const A& a) {
+  return a.tiles_f * (a.table ? ((ConstInts)(uintptr_t)a.table)[0] : a.tiles_t);
+}
+template <class A>
+__device__ __forceinline__ AnyTile any_tile(const A& a, int b, int tile_rows, int tile_features) {
+  const int mt = b / a.tiles_f, nt = b - mt * a.tiles_f;
+  if (!a.table) return AnyTile{0, mt * tile_rows, a.M, nt * tile_features};
+  ConstInts e = (ConstInts)(uintptr_t)a.table + 4 + 4 * mt;
+  return AnyTile{e[0], e[1], e[2], nt * tile_features};
+}
+template <class A>
+__device__ __forceinline__ AnyRow any_row(const A& a, int m, int m_end) {
+  AnyRow r{-1, 1.f};
+  if (m >= m_end) return r;
+  r.y = a.y_rows ? a.y_rows[m] : m;
+  if (a.row_scale) r.scale = a.row_scale[a.row_scale_rows ? a.row_scale_rows[m] : m];
+  return r;
+}
+// four consecutive features of one row: the epilogue of gemm_any.hip's finish(), operation for operation
+template <class A>
+__device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, f32x4 v, f32x4 v2) {
+  if (row.y < 0 || n >= a.N) return;
+  if (a.row_scale) {
+    v *= row.scale;
+    if (A::kDual) v2 *= row.scale;
+  }
+  if (a.bias1) v += *reinterpret_cast<const f32x4*>(a.bias1 + n);
+  if (A::kDual && a.bias2) v2 += *reinterpret_cast<const f32x4*>(a.bias2 + n);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float z = v[e];
+    float o = z;
+    if constexpr (A::kAct == MI_ACT_CLAMPED_GLU) {
+      const float g = fminf(z, a.limit), u = fminf(fmaxf(v2[e], -a.limit), a.limit);
+      o = g / (1.f + expf(-1.702f * g)) * (u + 1.f);
+    } else {
+      if constexpr (A::kAct == MI_ACT_SILU) o = z / (1.f + expf(-z));
+      if constexpr (A::kAct == MI_ACT_GELU_TANH) o = 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+      if constexpr (A::kAct == MI_ACT_GELU_ERF) o = 0.5f * z * (1.f + erff(z * 0.7071067811865476f));
+      if constexpr (A::kAct == MI_ACT_RELU2) o = fmaxf(z, 0.f) * fmaxf(z, 0.f);
+      if (A::kDual) o *= v2[e];
+    }
+    v[e] = o * a.alpha;
+  }
+  if (a.y16) *reinterpret_cast<u32x2*>(a.y16 + row.y * a.ldy + n) = u32x2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+  else *reinterpret_cast<f32x4*>(a.y32 + row.y * a.ldy + n) = v;
+}
+
+
+#include "gemm_w16_kernel.hpp"
+#include "gemm_mid_kernel.hpp"
+
+// x rows -> bf16 rows (eight elements a thread), gathered by x_rows; rows from the groups' end on are left as they are.
+// The grid's last workgroup writes the tile table.
+__global__ __launch_bounds__(256) void any_operand_kernel(const float* __restrict__ x, int64_t ldx,
+                                                          const int32_t* __restrict__ x_rows,
+                                                          const int32_t* __restrict__ group_offsets, int n_groups,
+                                                          int tile_rows, int rows, int K, uint16_t* __restrict__ xb,
+                                                          int32_t* __restrict__ table) {
+  __shared__ int tiles[1024];
+  const int tid = threadIdx.x;
+  if (table && blockIdx.x == gridDim.x - 1) {
+    for (int g = tid; g < n_groups; g += 256) tiles[g] = (group_offsets[g + 1] - group_offsets[g] + tile_rows - 1) / tile_rows;
+    __syncthreads();
+    for (int g = tid; g < n_groups; g += 256) {
+      int at = 0;
+      for (int j = 0; j < g; ++j) at += tiles[j];
+      const int lo = group_offsets[g], hi = group_offsets[g + 1];
+      for (int i = 0; i < tiles[g]; ++i)
+        *reinterpret_cast<int4*>(table + 4 + 4 * (at + i)) = int4{g, lo + i * tile_rows, hi, 0};
+      if (g == n_groups - 1) *reinterpret_cast<int4*>(table) = int4{at + tiles[g], 0, 0, 0};
+    }
+    return;
+  }
+  const int per_row = K >> 3;
+  const int64_t i = (int64_t)blockIdx.x * 256 + tid;
+  const int row = (int)(i / per_row), c = (int)(i - (int64_t)row * per_row) * 8;
+  if (row >= rows || (group_offsets && row >= group_offsets[n_groups])) return;
+  const float* src = x + (int64_t)(x_rows ? x_rows[row] : row) * ldx + c;
+  float4 a, b;
+  if ((ldx & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
+    a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+  } else {
+    a = float4{src[0], src[1], src[2], src[3]}, b = float4{src[4], src[5], src[6], src[7]};
+  }
+  *reinterpret_cast<u32x4*>(xb + (int64_t)row * K + c) =
+      u32x4{pack_bf(a.x, a.y), pack_bf(a.z, a.w), pack_bf(b.x, b.y), pack_bf(b.z, b.w)};
+}
+
+// the row tiles of `rows` rows in at most n_groups groups (0: one, its tiles known)
+static int64_t row_tiles(int rows, int n_groups, int t) { return n_groups ? rows / t + n_groups : (rows + t - 1) / t; }
+
+// 0: not taken; else the rows of a tile (256: the persistent kernel, 128: the small-tile kernel)
+static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int act) {
+  if (rows < 1 || N < 1 || K < BK || K % BK || N % 4 || n_groups < 0 || n_groups > 1024) return 0;
+  const bool known = dual ? act == MI_ACT_SILU || act == MI_ACT_GELU_TANH || act == MI_ACT_CLAMPED_GLU
+                          : act == MI_ACT_NONE || act == MI_ACT_GELU_ERF || act == MI_ACT_RELU2;
+  if (!known) return 0;
+  // 32-bit byte offsets from the operand bases, and 0xF0000000 beyond both (the persistent kernel's "fetch nothing")
+  const int64_t limit = (int64_t)1 << 31;
+  if (((int64_t)(n_groups ? n_groups : 1) * N + 256) * K * 2 >= limit || ((int64_t)rows + 256) * K * 2 >= limit) return 0;
+  // Where the lines lie (us, this kernel incl. the operand pass against gemm_any.hip's):
+  //   no groups, N 2048, K 2048: 128 rows 25 / 30, 512 rows 28 / 88, 4096 rows 53 / 96; N 512, K 1024: 128 rows 16 / 17.
+  //   Experts' pair of products, 32 of 512 x 1024 (64 of 768 x 2048): 4 rows each 29 / 36 (153 / 170), 16 rows 30 / 109
+  //   (148 / 364), 512 rows 131 / 265 (541 / 1236).
+  // 256-row tiles from about 160 of them on (N 3072, K 1024, 4096 rows: 40, with 128-row tiles 48; N 2048, K 2048, 4096 rows
+  // = 128 tiles: 57 / 53), with groups from 128 rows and some 350 tiles on, where the groups' last, part-filled tiles no
+  // longer weigh (64 experts: 128 rows each 246 / 253, 64 rows 215 / 175; 32 experts of 512 rows = 320 tiles: 142 / 131).
+  if (rows < 128 || N < 128 || rows < n_groups) return 0;
+  const int tf = dual ? 128 : 256;
+  if (n_groups) return rows >= 128 * n_groups && (rows / 256 + n_groups / 2) * (int64_t)((N + tf - 1) / tf) >= 350 ? 256 : 128;
+  return ((rows + 255) / 256) * (int64_t)((N + tf - 1) / tf) >= 160 ? 256 : 128;
+}
+
+template <int ACT, bool DUAL>
+static int launch_any_tile(const AnyTileArgs<ACT, DUAL>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
+  using A = AnyTileArgs<ACT, DUAL>;
+  A a = args;
+  if (tile_rows == 256) {
+    a.tiles_f = (a.N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
+    a.tiles_t = (a.M + 255) / 256;
+    const int64_t tiles = row_tiles_max * a.tiles_f;
+    hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 0, A>), dim3((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid)),
+                       dim3(256), 0, st, a);
+  } else {
+    a.tiles_f = (a.N + (DUAL ? 63 : 127)) / (DUAL ? 64 : 128);
+    a.tiles_t = (a.M + 127) / 128;
+    const int64_t tiles = row_tiles_max * a.tiles_f;
+    if (tiles > 0x7fffffff) return MI_EUNSUPPORTED;
+    if (tiles > kPersistentGrid)
+      hipLaunchKernelGGL((gemm_mid_kernel<TEPI_ANY, false, 2, A>), dim3((unsigned)tiles), dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((gemm_mid_kernel<TEPI_ANY, false, 4, A>), dim3((unsigned)tiles), dim3(256), 0, st, a);
+  }
+  return check_launch();
+}
+
+}  // namespace mi
+
+using namespace mi;
+
+extern "C" int mi_gemm_any_tile_rows(int rows, int N, int K, int n_groups, int dual, int act) {
+  return tile_rows_for(rows, N, K, n_groups, dual != 0, act);
+}
+
+extern "C" int64_t mi_gemm_any_table_ints(int rows, int n_groups, int tile_rows) {
+  if (rows < 0 || n_groups < 1 || (tile_rows != 128 && tile_rows != 256)) return 0;
+  return 4 + 4 * row_tiles(rows, n_groups, tile_rows);
+}
+
+extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets,
+                                   int n_groups, int tile_rows, int rows, int K, mi_bf16* xb, int32_t* table,
+                                   mi_stream stream) {
+  if (!x || !xb || rows < 0 || K < 8 || K % 8 || ldx < K || !aligned16(xb)) return MI_EINVAL;
+  if (n_groups < 0 || n_groups > 1024 || (n_groups > 0) != (group_offsets != nullptr)) return MI_EINVAL;
+  if (table && (!n_groups || !aligned16(table) || (tile_rows != 128 && tile_rows != 256))) return MI_EINVAL;
+  if (rows == 0) return MI_OK;
+  const int64_t blocks = ((int64_t)rows * (K / 8) + 255) / 256 + (table ? 1 : 0);
+  if (blocks > 0x7fffffff) return MI_EUNSUPPORTED;
+  hipLaunchKernelGGL(any_operand_kernel, dim3((unsigned)blocks), dim3(256), 0, S(stream), x, ldx, x_rows, group_offsets, n_groups,
+                     tile_rows, rows, K, xb, table);
+  return check_launch();
+}
+
+extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int tile_rows, const mi_bf16* w, const mi_bf16* w2,
+                                const float* bias, const float* bias2, int act, float limit, const float* row_scale,
+                                const int32_t* row_scale_rows, int n_groups, void* y, int y_is_bf16, int64_t ldy,
+                                const int32_t* y_rows, int rows, int N, int K, float alpha, mi_stream stream) {
+  if (!xb || !w || !y || rows < 0 || (n_groups > 0) != (table != nullptr) || (row_scale_rows && !row_scale)) return MI_EINVAL;
+  if (act == MI_ACT_CLAMPED_GLU && !(limit > 0.f)) return MI_EINVAL;
+  if (rows == 0) return MI_OK;
+  if (tile_rows != 128 && tile_rows != 256) return MI_EINVAL;
+  if (tile_rows_for(rows, N, K, n_groups, w2 != nullptr, act) == 0) return MI_EUNSUPPORTED;
+  if (ldy < N || ldy % 4 || !aligned16(xb) || !aligned16(w) || (w2 && !aligned16(w2)) || !aligned16(y) || (bias && !aligned16(bias)) ||
+      (bias2 && (!w2 || !aligned16(bias2))))
+    return MI_EINVAL;
+  const int64_t tiles = row_tiles(rows, n_groups, tile_rows);
+  auto go = [&](auto args) {
+    args.x = xb, args.w = w, args.w2 = w2, args.bias = nullptr, args.y = nullptr, args.part = nullptr;
+    args.ldx = K, args.ldy = ldy, args.M = rows, args.N = N, args.K = K;
+    args.groups = n_groups ? n_groups : 1, args.table = table;
+    args.y32 = y_is_bf16 ? nullptr : static_cast<float*>(y), args.y16 = y_is_bf16 ? static_cast<uint16_t*>(y) : nullptr;
+    args.y_rows = y_rows, args.bias1 = bias, args.bias2 = bias2, args.alpha = alpha, args.limit = limit;
+    args.row_scale = row_scale, args.row_scale_rows = row_scale_rows;
+    return launch_any_tile(args, tile_rows, tiles, S(stream));
+  };
+  if (w2) {
+    if (act == MI_ACT_SILU) return go(AnyTileArgs<MI_ACT_SILU, true>{});
+    if (act == MI_ACT_GELU_TANH) return go(AnyTileArgs<MI_ACT_GELU_TANH, true>{});
+    return go(AnyTileArgs<MI_ACT_CLAMPED_GLU, true>{});
+  }
+  if (act == MI_ACT_NONE) return go(AnyTileArgs<MI_ACT_NONE, false>{});
+  if (act == MI_ACT_GELU_ERF) return go(AnyTileArgs<MI_ACT_GELU_ERF, false>{});
+  return go(AnyTileArgs<MI_ACT_RELU2, false>{});
+}

@@ -41,31 +41,9 @@
 namespace mi {
 using namespace gt;
 
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-enum { TEPI_NONE = 0, TEPI_SILU = 1, TEPI_PARTIAL = 2, TEPI_QKV = 3 };
-
-struct TileArgs {
-  const uint16_t* x;
-  const uint16_t* w;
-  const uint16_t* bias;
-  uint16_t* y;
-  int64_t ldx, ldy;
-  int M, N, K;
-  int tiles_f, tiles_t;
-  float* part;  // split-K (gridDim.y > 1): fp32 partial sums [gridDim.y][M][N] instead of y
-  // TEPI_QKV (mi_gemm_bf16_qkv_store): the K and V heads of the packed qkv projection go straight to the paged cache
-  struct QkvStore {
-    const uint16_t* k_w;       // k-norm weight [128] or null
-    const int64_t* positions;  // [M]
-    const float* cos_sin;      // [max_position][128]
-    uint16_t* k_cache;
-    uint16_t* v_cache;
-    const int32_t* slots;      // [M] flat slots (block * block_size + offset; negative: not stored)
-    float eps;
-    int n_q_heads, n_kv_heads, block_size;
-  } qkv;
-};
+}  // namespace mi
+#include "gemm_tile_args.hpp"
+namespace mi {
 
 // Tuning variants of the eight-wave kernel below (mi_gemm_bf16_ex instantiates the combinations it lists - the staggered
 // start V & 1024 and the never-waited DMA V & 256 measured no effect and are not instantiated any more; the timing-only
@@ -83,30 +61,6 @@ struct TileArgs {
 //   V & 32 / 64 / 128   ABLATIONS for timing only (wrong results): no DMA in the K loop / no fragment reads in the K
 //            loop / no workgroup barriers in the K loop
 constexpr int kDefaultV = 0;
-constexpr int kPersistentGrid = 256;  // one workgroup per CU
-
-#define MI_GT_BARRIER() asm volatile("s_barrier" ::: "memory")
-
-// tile of "block" b.  Plain order (the default): tile b, feature tiles fastest.  The dispatcher places workgroup b
-// on XCD b % 8 (a speed assumption only) and a persistent workgroup keeps b % 8 - and, the feature-tile count dividing
-// 256 for every shape of the path, its feature tile - over its tiles: its 256 x K weight panel stays in the XCD's L2
-// while the activation panels stream through.  The alternative (rect): the 32 workgroups an XCD runs together are
-// given a GT x GF rectangle of tiles, GT activation + GF weight panels per K step; measured equal or slower
-// (tools/gemm_bench.py), kept as a tuning variant.
-__device__ __forceinline__ int tile_of_block(int b, int tiles_t, int tiles_f, bool rect) {
-  const int ntiles = tiles_t * tiles_f;
-  if (!rect) return b;
-  const int gf = tiles_f % 8 == 0 ? 8 : (tiles_f % 4 == 0 ? 4 : (tiles_f % 2 == 0 ? 2 : 1)), gt = 32 / gf;
-  const int xcd = b & 7, idx = b >> 3;
-  if (ntiles % 256 == 0 && tiles_t % gt == 0) {
-    const int r = (idx >> 5) * 8 + xcd, local = idx & 31, rc = tiles_f / gf;
-    return ((r / rc) * gt + local / gf) * tiles_f + (r % rc) * gf + local % gf;
-  }
-  // any other grid: XCD x takes the x-th contiguous run of tiles (bijective for every ntiles)
-  const int qn = ntiles >> 3, rn = ntiles & 7;
-  return (xcd < rn ? xcd * (qn + 1) : rn * (qn + 1) + (xcd - rn) * qn) + idx;
-}
-
 template <int EPI, bool BIAS, int V>
 __global__ __launch_bounds__(512, 2) void gemm_tile_kernel(const TileArgs a) {
   // ONE LDS object (a second one makes hipcc drain the DMA queue before every fragment read)
@@ -471,165 +425,7 @@ __global__ __launch_bounds__(512, 2) void gemm_tile_kernel(const TileArgs a) {
 #include "gemm_w4_kernel.hpp"
 #include "gemm_w16_kernel.hpp"
 
-// ---------------------------------------------------------------------------
-// The same GEMM on 128 x 128 tiles, for shapes whose 256 x 256 tiles cannot fill the chip (64 < M <= ~2048 rows:
-// large decode batches, short prompts).  Four waves, each 64 features x 64 tokens (2 x 2 accumulators); one K step of
-// the tile is two 16 KiB half-tiles in the layout of gemm_tile_index.hpp (A: local row = tile feature row, B: local
-// row = tile token row) in a ring of NST stages.  One barrier per K step: "my pieces of step t have landed" (a COUNTED
-// wait: the pieces of the NST - 2 steps behind it may still fly) -> barrier (everybody's have, and everybody is done
-// reading step t - 1) -> request step t + NST - 1 into the buffer step t - 1 used -> fragments of step t -> sixteen
-// MFMAs.  These shapes have at most a workgroup or two per CU and a K loop of 16-80 steps: with one step of
-// prefetch (NST = 2, two workgroups per CU) every step waits out most of a DMA round trip (0.75 us per step
-// measured); NST = 4 (128 KiB, one workgroup per CU) keeps three steps in flight.
-// Same summation order and epilogues as the large kernel: results are bit-identical.
-// SwiGLU: the tile's 128 weight rows are, per wave, 32 gate rows (fragment 0) and the 32 up rows that pair with them.
-// ---------------------------------------------------------------------------
-constexpr int MID_STAGE = 2 * HALF_BYTES;  // (MID_F, MID_T and the index arithmetic: gemm_tile_index.hpp)
-
-template <int EPI, bool BIAS, int NST>
-__global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const TileArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[NST * MID_STAGE];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int fw = wave >> 1, tw = wave & 1, hi = lane >> 5, l31 = lane & 31;
-  const int KT_all = a.K / BK;
-  const int KT = EPI == TEPI_PARTIAL ? KT_all / (int)gridDim.y : KT_all;
-  const int64_t kbeg_bytes = EPI == TEPI_PARTIAL ? (int64_t)blockIdx.y * KT * (BK * 2) : 0;
-  const int n0 = ((int)blockIdx.x % a.tiles_f) * MID_F, m0 = ((int)blockIdx.x / a.tiles_f) * MID_T;
-
-  // LDS-DMA: wave w moves the 1 KiB blocks 4 w .. 4 w + 3 (8 local rows each) of both half-tiles
-  const char* srcA[4];
-  const char* srcB[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int lr = mid_dma_local_row(wave, i, lane), c = mid_dma_chunk(wave, i, lane);
-    const int rowA = mid_weight_row(lr, n0, a.N, EPI == TEPI_SILU);
-    srcA[i] = reinterpret_cast<const char*>(a.w) + kbeg_bytes + ((int64_t)min(rowA, a.N - 1) * a.K + c * 8) * 2;
-    srcB[i] = reinterpret_cast<const char*>(a.x) + kbeg_bytes + ((int64_t)min(m0 + lr, a.M - 1) * a.ldx + c * 8) * 2;
-  }
-  auto issue = [&](int kt, int p) __attribute__((always_inline)) {
-    char* dst = lds + p * MID_STAGE + wave * 4096;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcA[i] + (int64_t)kt * (BK * 2)),
-                                       (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcB[i] + (int64_t)kt * (BK * 2)),
-                                       (__attribute__((address_space(3))) void*)(dst + HALF_BYTES + i * 1024), 16, 0, 0);
-    }
-  };
-  int kx[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk)
-    kx[kk] = (l31 >> 3) * 1024 + (l31 & 7) * 128 + ((frag_chunk(kk, hi) ^ swizzle(l31)) << 4);
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int f = 0; f < 2; ++f)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[f][b][r] = 0.f;
-
-#pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < KT) issue(s, s);
-  int p = 0, pn = NST - 1;  // ring slots of step kt and of step kt + NST - 1
-  for (int kt = 0; kt < KT; ++kt) {
-    // requested so far: steps <= kt + NST - 2; eight pieces per step and wave, completing in order
-    const int behind = min(KT - 1 - kt, NST - 2);
-    if (behind >= 2) asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
-    else if (behind == 1) asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    if (kt + NST - 1 < KT) issue(kt + NST - 1, pn);
-    const char* sa = lds + p * MID_STAGE + fw * 8192;
-    const char* sb = lds + p * MID_STAGE + HALF_BYTES + tw * 8192;
-    u32x4 A[2][4], B[2][4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-#pragma unroll
-      for (int f = 0; f < 2; ++f) A[f][kk] = *reinterpret_cast<const u32x4*>(sa + f * 4096 + kx[kk]);
-#pragma unroll
-      for (int b = 0; b < 2; ++b) B[b][kk] = *reinterpret_cast<const u32x4*>(sb + b * 4096 + kx[kk]);
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[f][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(A[f][kk]), as_frag(B[b][kk]), acc[f][b], 0, 0, 0);
-    p = p + 1 == NST ? 0 : p + 1;
-    pn = pn + 1 == NST ? 0 : pn + 1;
-  }
-
-  // epilogue: lane (hi, l31) holds token tw * 64 + b * 32 + l31, features 8 rq + 4 hi + {0..3} of each 32-row fragment
-  const int n_out = EPI == TEPI_SILU ? a.N >> 1 : a.N;
-  const bool wide = n_out % 8 == 0 && a.ldy % 8 == 0;
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int tok = m0 + tw * 64 + b * 32 + l31;
-    const bool tok_ok = tok < a.M;
-    if (EPI == TEPI_PARTIAL) {
-      float* prow = a.part + ((int64_t)blockIdx.y * a.M + min(tok, a.M - 1)) * a.N;
-#pragma unroll
-      for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int rq = 0; rq < 4; ++rq) {
-          const int col = n0 + fw * 64 + f * 32 + 8 * rq + 4 * hi;
-          if (tok_ok && col < a.N)
-            *reinterpret_cast<f32x4*>(prow + col) =
-                f32x4{acc[f][b][4 * rq], acc[f][b][4 * rq + 1], acc[f][b][4 * rq + 2], acc[f][b][4 * rq + 3]};
-        }
-      continue;
-    }
-    uint16_t* yrow = a.y + (int64_t)min(tok, a.M - 1) * a.ldy;
-#pragma unroll
-    for (int f = 0; f < (EPI == TEPI_SILU ? 1 : 2); ++f) {
-      const int col0 = EPI == TEPI_SILU ? (n0 >> 1) + fw * 32 : n0 + fw * 64 + f * 32;
-      u32x2 pk[4];
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int col = col0 + 8 * rq + 4 * hi;
-        float o[4];
-        if (EPI == TEPI_SILU) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {  // the roundings and the silu form of the large kernel's epilogue
-            const float gb = rbf(acc[0][b][4 * rq + e]);
-            const float sb = rbf(gb * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gb * -1.4426950408889634f)));
-            o[e] = sb * rbf(acc[1][b][4 * rq + e]);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = acc[f][b][4 * rq + e];
-          if (BIAS && col < n_out) {
-            const u32x2 bw = *reinterpret_cast<const u32x2*>(a.bias + col);
-            o[0] += lo_bf(bw[0]);
-            o[1] += hi_bf(bw[0]);
-            o[2] += lo_bf(bw[1]);
-            o[3] += hi_bf(bw[1]);
-          }
-        }
-        pk[rq] = u32x2{pack_bf(o[0], o[1]), pack_bf(o[2], o[3])};
-      }
-      if (wide) {
-#pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2) {
-          const auto sx = __builtin_amdgcn_permlane32_swap(pk[2 * p2][0], pk[2 * p2 + 1][0], false, false);
-          const auto sy = __builtin_amdgcn_permlane32_swap(pk[2 * p2][1], pk[2 * p2 + 1][1], false, false);
-          const int col = col0 + 8 * (2 * p2 + hi);
-          if (tok_ok && col < n_out) *reinterpret_cast<u32x4*>(yrow + col) = u32x4{sx[0], sy[0], sx[1], sy[1]};
-        }
-      } else {
-#pragma unroll
-        for (int rq = 0; rq < 4; ++rq) {
-          const int col = col0 + 8 * rq + 4 * hi;
-          if (tok_ok && col < n_out) *reinterpret_cast<u32x2*>(yrow + col) = pk[rq];
-        }
-      }
-    }
-  }
-}
+#include "gemm_mid_kernel.hpp"
 
 // sum of the split-K slices in slice order, (+ bias), one rounding to bf16: four features per thread
 static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int nsplit,

@@ -23,9 +23,10 @@
 // (tests/test_gemm_tile_gpu.py holds the two MFMA shapes against each other and against the library).
 #pragma once
 
-template <int EPI, bool BIAS, int V>
-__global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
-  constexpr bool LINES = (V & 32768) != 0 && EPI != TEPI_PARTIAL;
+template <int EPI, bool BIAS, int V, class ARGS = TileArgs>
+__global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
+  constexpr bool LINES = (V & 32768) != 0 && EPI != TEPI_PARTIAL && EPI != TEPI_ANY;
+  constexpr bool PAIRED = EPI == TEPI_ANY && ARGS::kDual;  // two weights: half 0 of the A region holds 128 rows of w, half 1 of w2
   __shared__ __attribute__((aligned(1024))) char lds[2 * W16_STEP_BYTES + (LINES ? 4 * W4_STAGE_BYTES : 0)];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -33,14 +34,21 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
   const int KT_all = a.K / BK;
   const int KT = EPI == TEPI_PARTIAL ? KT_all / (int)gridDim.y : KT_all;
   const uint32_t kbeg_bytes = EPI == TEPI_PARTIAL ? (uint32_t)blockIdx.y * KT * (BK * 2) : 0u;
-  const int ntiles = a.tiles_f * a.tiles_t, stride = (int)gridDim.x;
+  int ntiles = a.tiles_f * a.tiles_t;
+  if constexpr (EPI == TEPI_ANY) ntiles = any_tiles(a);
+  const int stride = (int)gridDim.x;
+  if (EPI == TEPI_ANY && (int)blockIdx.x >= ntiles) return;  // (the grid is the host's bound on the grouped tiles)
 
   // ---- the feed (as gemm_w4_kernel): waves 0, 1 the A region (weight rows), waves 2, 3 the B region ----
   const bool wgt = w4_wave_is_weight(wave);
   const uint32_t ld2 = (uint32_t)(wgt ? a.K : a.ldx) * 2;
-  const uint32_t records = (uint32_t)(wgt ? a.N : a.M) * ld2;
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wgt ? a.w : a.x), 0, records, 0x00020000);
+  uint32_t records = (uint32_t)(wgt ? a.N : a.M) * ld2;
+  const uint16_t* src = wgt ? a.w : a.x;
+  if constexpr (EPI == TEPI_ANY) {
+    if (wgt) records *= (uint32_t)a.groups;
+    if (PAIRED && wave == 1) src = a.w2;
+  }
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(src), 0, records, 0x00020000);
   // per-lane part of a piece's source offset: the rows of slice lane >> 3 depend on the piece through ONE bit (x3 of the
   // piece, gemm_tile_index.hpp): two variants.  SwiGLU weights: rows 64..127 of a wave's half are the up rows N / 2 on.
   uint32_t voff[2];
@@ -55,6 +63,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
   auto fetch_tile = [&](int b) __attribute__((always_inline)) {
     if (b >= ntiles) {  // past the workgroup's last tile: every row beyond the descriptor - the pieces fetch nothing
       f_row = 0xF0000000u;
+      return;
+    }
+    if constexpr (EPI == TEPI_ANY) {
+      const AnyTile t = any_tile(a, b, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
+      if (!wgt) f_row = (uint32_t)(t.m0 + (wave & 1) * 128) * ld2;
+      else f_row = (uint32_t)(t.group * a.N + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
       return;
     }
     const int tid = tile_of_block(b, a.tiles_t, a.tiles_f, (V & 4) != 0);
@@ -82,7 +96,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
   };
 
   // ---- fragment reads: one per-lane byte offset per operand; fragment and k half are immediates ----
-  int offa = w16_frag_lane(n16, q4) + fw * (16 * W16_PIECE_BYTES);
+  // (PAIRED: a wave's eight A fragments are rows 64 fw .. + 63 of BOTH halves - 64 rows of w, then the same rows of w2;
+  // + 64 rows of a half = slice bit 2 = 512 bytes)
+  int offa = w16_frag_lane(n16, q4) + (PAIRED ? fw * 512 : fw * (16 * W16_PIECE_BYTES));
   int offb = w16_frag_lane(n16, q4) + (32 + tw * 16) * W16_PIECE_BYTES;
   int flip = W16_STEP_BYTES;
   u32x4 Ra[2][8], Rb[2][8];  // [k half][fragment]
@@ -92,7 +108,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
   auto read1 = [&](int kh, int q) __attribute__((always_inline)) {
     if (q == 0 || q > 8) {
       const int f = q == 0 ? 0 : q - 8;
-      Ra[kh][f] = *reinterpret_cast<const u32x4*>(lds + w16_frag_imm(f, kh) + offa);
+      const int imm = PAIRED ? (f >> 2) * (16 * W16_PIECE_BYTES) + w16_frag_imm(f & 3, kh) : w16_frag_imm(f, kh);
+      Ra[kh][f] = *reinterpret_cast<const u32x4*>(lds + imm + offa);
     } else {
       Rb[kh][q - 1] = *reinterpret_cast<const u32x4*>(lds + w16_frag_imm(q - 1, kh) + offb);
     }
@@ -284,7 +301,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
 
   for (int blk = (int)blockIdx.x; blk < ntiles; blk += stride) {
     const int tid = tile_of_block(blk, a.tiles_t, a.tiles_f, (V & 4) != 0);
-    const int m0 = (tid / a.tiles_f) * TILE_T, n0 = (tid % a.tiles_f) * TILE_F;
+    int m0 = (tid / a.tiles_f) * TILE_T, n0 = (tid % a.tiles_f) * TILE_F, m_end = a.M;
+    if constexpr (EPI == TEPI_ANY) {
+      const AnyTile t = any_tile(a, blk, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
+      m0 = t.m0, n0 = t.n0, m_end = t.m_end;
+    }
     kstep(std::true_type{});
     for (int kt = 1; kt < KT; ++kt) kstep(std::false_type{});
     __builtin_amdgcn_sched_barrier(0);
@@ -298,8 +319,23 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const TileArgs a) {
     asm volatile("" : "+a"(acc[5][3]), "+a"(acc[5][4]), "+a"(acc[5][5]), "+a"(acc[5][6]), "+a"(acc[5][7]), "+a"(acc[6][0]), "+a"(acc[6][1]), "+a"(acc[6][2]), "+a"(acc[6][3]), "+a"(acc[6][4]), "+a"(acc[6][5]), "+a"(acc[6][6]), "+a"(acc[6][7]), "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]), "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7]));
     // A workgroup's last tile: its (empty) past-the-end pieces must not outlive the workgroup's LDS
     if (blk + stride >= ntiles) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (LINES) epilogue_lines(m0, n0);
-    else epilogue(m0, n0);
+    if constexpr (EPI == TEPI_ANY) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const AnyRow row = any_row(a, m0 + w16_acc_token(tw, t, n16), m_end);
+#pragma unroll
+        for (int f = 0; f < (PAIRED ? 4 : 8); ++f) {
+          // (the next tile's first fragments are live here: accumulators copied out early would spill them)
+          if constexpr (PAIRED) asm volatile("" : "+a"(acc[f][t]), "+a"(acc[f + 4][t]));
+          any_store(a, row, n0 + fw * (PAIRED ? 64 : 128) + 16 * f + 4 * q4, acc[f][t], acc[PAIRED ? f + 4 : f][t]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    } else if constexpr (LINES) {
+      epilogue_lines(m0, n0);
+    } else {
+      epilogue(m0, n0);
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
   if (V & 4096) {

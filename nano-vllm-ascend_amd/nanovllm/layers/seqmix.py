@@ -211,8 +211,7 @@ class GroupedSparseMLP(nn.Module):
                                      self.group_kind)
         offsets, pair_token, pair_index = ops.moe_sort(ids, self.n_out)
         P = ids.numel()
-        act = ops.gemm_any_grouped(x, pair_token, self.gate, self.up, offsets, P, None, P)
-        y = ops.gemm_any_grouped(act, None, self.down, None, offsets, P, pair_index, P)
+        y = ops.expert_ff(x, pair_token, self.gate, self.up, self.down, _C.ACT_SILU, offsets, P, pair_index)
         return ops.moe_combine_f32(y, x, ids, wts, self.E)
 
 
@@ -405,8 +404,7 @@ class SharedSparseMLP(nn.Module):
         ids, wts = ops.route_topk(z, self.E, self.top_k, self.weight_scale)
         offsets, pair_token, pair_index = ops.moe_sort(ids, self.E)
         P = ids.numel()
-        a = ops.gemm_any_grouped_act(h, pair_token, self.up, None, self.act, offsets, P, None, P)
-        y = ops.gemm_any_grouped_act(a, None, self.down, None, _C.ACT_NONE, offsets, P, pair_index, P)
+        y = ops.expert_ff(h, pair_token, self.up, None, self.down, self.act, offsets, P, pair_index)
         sh = ops.gemm_any(ops.gemm_any_act(h, self.shared_up, act=self.act), self.shared_down) if self.shared else None
         return y, ids, wts, sh, z[:, self.E:] if self.gated else None
 
@@ -715,9 +713,8 @@ class InputWeightedSparseMLP(nn.Module):
         ids, wts = ops.route_grouped(z, self.no_correction, self.top_k, 1, 1, _C.ROUTE_SIGMOID, _C.ROUTE_GROUP_MAX)
         offsets, pair_token, pair_index = ops.moe_sort(ids, self.E)
         P = ids.numel()
-        a = ops.gemm_any_grouped_glu(h, pair_token, self.gate, self.up, _C.ACT_CLAMPED_GLU, self.limit, wts, pair_index,
-                                     offsets, P, None, P)
-        y = ops.gemm_any_grouped(a, None, self.down, None, offsets, P, pair_index, P)
+        y = ops.expert_ff(h, pair_token, self.gate, self.up, self.down, _C.ACT_CLAMPED_GLU, offsets, P, pair_index, self.limit, wts,
+                          pair_index)
         return ops.moe_combine_shared(y, ids, None, h.shape[1])
 
 

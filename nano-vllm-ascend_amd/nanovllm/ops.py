@@ -956,6 +956,39 @@ def _i32(*ts: torch.Tensor) -> None:
             raise _C.MiError("expected a contiguous int32 tensor")
 
 
+def _tile_rows(rows: int, w, w2, act: int, exact: bool, groups: int, *fp32: torch.Tensor) -> int:
+    """Rows of a tile if this product goes through the tile kernels (mi_gemm_any_tile), else 0.  fp32: what its epilogue reads
+    or writes in 16-byte pieces (None: absent)."""
+    if exact or w.dtype != _BF16 or rows < 128:
+        return 0
+    if any(t is not None and (t.data_ptr() % 16 or (t.dim() == 2 and t.stride(0) % 4)) for t in fp32):
+        return 0
+    if w.data_ptr() % 16 or (w2 is not None and w2.data_ptr() % 16):
+        return 0
+    return lib.mi_gemm_any_tile_rows(rows, w.shape[-2], w.shape[-1], groups, int(w2 is not None), int(act))
+
+
+def _tile_operand(x, tile_rows: int, x_rows=None, offsets=None, groups: int = 0, rows: int | None = None):
+    """-> (x rounded to bf16, in sorted order with x_rows; the groups' tile table or None)"""
+    rows, K = x.shape[0] if rows is None else rows, x.shape[1]
+    xb = torch.empty((rows, K), dtype=_BF16, device=x.device)
+    table = torch.empty(lib.mi_gemm_any_table_ints(rows, groups, tile_rows), dtype=torch.int32, device=x.device) if groups else None
+    check(lib.mi_gemm_any_operand(ptr(x), x.stride(0) if x.shape[0] > 1 else K, ptr(x_rows), ptr(offsets), groups, tile_rows, rows, K,
+                                  ptr(xb), ptr(table), stream()), "mi_gemm_any_operand")
+    return xb, table
+
+
+def _tile_gemm(operand, tile_rows: int, w, w2, out, act: int, groups: int = 0, y_rows=None, bias=None, bias2=None, alpha: float = 1.0,
+               limit: float = 0.0, row_scale=None, row_scale_rows=None):
+    xb, table = operand
+    N, K = w.shape[-2], w.shape[-1]
+    check(lib.mi_gemm_any_tile(ptr(xb), ptr(table), tile_rows, ptr(w), ptr(w2), ptr(bias), ptr(bias2), int(act), float(limit),
+                               ptr(row_scale), ptr(row_scale_rows), groups, ptr(out), int(out.dtype == _BF16),
+                               out.stride(0) if out.shape[0] > 1 else N, ptr(y_rows), xb.shape[0], N, K, float(alpha), stream()),
+          "mi_gemm_any_tile")
+    return out
+
+
 def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None) -> torch.Tensor:
     """alpha * x @ w.T for any shapes; x may be a column slice of a wider buffer (unit inner stride)."""
     require_gpu(x, w)
@@ -966,6 +999,9 @@ def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None) -> torch.T
     if out is None:
         out = torch.empty((M, N), dtype=_F32, device=x.device)
     assert out.shape == (M, N)
+    t = _tile_rows(M, w, None, _C.ACT_NONE, exact, 0, out)
+    if t:
+        return _tile_gemm(_tile_operand(x, t), t, w, None, out, _C.ACT_NONE, alpha=alpha)
     check(lib.mi_gemm_any(ptr(x), x.stride(0) if M > 1 else K, ptr(w), _dt(w), ptr(out), out.stride(0) if M > 1 else N,
                           M, N, K, float(alpha), int(exact), stream()), "mi_gemm_any")
     return out
@@ -980,9 +1016,34 @@ def gemm_any_grouped(x, x_rows, w, w2, group_offsets, rows_max: int, y_rows, y_r
     G, N, K = w.shape
     assert x.shape[1] == K and group_offsets.numel() >= G + 1
     y = torch.empty((y_rows_total, N), dtype=_F32, device=x.device)
+    act = _C.ACT_NONE if w2 is None else _C.ACT_SILU
+    t = _tile_rows(rows_max, w, w2, act, exact, G, y)
+    if t:
+        return _tile_gemm(_tile_operand(x, t, x_rows, group_offsets, G, rows_max), t, w, w2, y, act, G, y_rows)
     check(lib.mi_gemm_any_grouped(ptr(x), x.stride(0), ptr(x_rows), ptr(w), ptr(w2), _dt(w), ptr(group_offsets), G,
                                   rows_max, ptr(y), N, ptr(y_rows), N, K, int(exact), stream()), "mi_gemm_any_grouped")
     return y
+
+
+def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_index, limit: float = 0.0, row_scale=None,
+              row_scale_rows=None) -> torch.Tensor:
+    """Both products of the experts' feed-forwards over expert-sorted pairs: down[e] (act(w[e] x) (* w2[e] x)) of every pair at
+    its place pair_index.  Prompt-sized steps over bf16 weights: the inner activations leave the first product as the bf16 rows
+    that the second one multiplies (it would round the same numbers itself)."""
+    t = min(_tile_rows(pairs, w, w2, act, False, w.shape[0]), _tile_rows(pairs, down, None, _C.ACT_NONE, False, w.shape[0]))
+    if t:
+        require_gpu(x, w, offsets)
+        _f32(x, row_scale)
+        _i32(pair_token, pair_index, offsets, row_scale_rows)
+        assert x.shape[1] == w.shape[2] and down.shape == (w.shape[0], w.shape[2], w.shape[1]) and offsets.numel() > w.shape[0]
+        G, ff, width = w.shape
+        operand = _tile_operand(x, t, pair_token, offsets, G, pairs)
+        inner = torch.empty((pairs, ff), dtype=_BF16, device=x.device)
+        _tile_gemm(operand, t, w, w2, inner, act, G, limit=limit, row_scale=row_scale, row_scale_rows=row_scale_rows)
+        y = torch.empty((pairs, width), dtype=_F32, device=x.device)
+        return _tile_gemm((inner, operand[1]), t, down, None, y, _C.ACT_NONE, G, pair_index)
+    a = gemm_any_grouped_glu(x, pair_token, w, w2, act, limit, row_scale, row_scale_rows, offsets, pairs, None, pairs)
+    return gemm_any_grouped(a, None, down, None, offsets, pairs, pair_index, pairs)
 
 
 def embedding_f32(ids, table, out=None, scale: float = 1.0) -> torch.Tensor:
@@ -1178,6 +1239,9 @@ def gemm_any_act(x, w, bias=None, act: int = _C.ACT_NONE, w2=None, bias2=None, a
     if out is None:
         out = torch.empty((M, N), dtype=_F32, device=x.device)
     assert out.shape == (M, N)
+    t = _tile_rows(M, w, w2, act, exact, 0, out, bias, bias2)
+    if t:
+        return _tile_gemm(_tile_operand(x, t), t, w, w2, out, act, bias=bias, bias2=bias2, alpha=alpha)
     check(lib.mi_gemm_any_act(ptr(x), x.stride(0) if M > 1 else K, ptr(w), ptr(w2), _dt(w), ptr(bias), ptr(bias2), int(act),
                               ptr(out), out.stride(0) if M > 1 else N, M, N, K, float(alpha), int(exact), stream()),
           "mi_gemm_any_act")
@@ -1194,6 +1258,9 @@ def gemm_any_grouped_act(x, x_rows, w, w2, act: int, group_offsets, rows_max: in
     G, N, K = w.shape
     assert x.shape[1] == K and group_offsets.numel() >= G + 1
     y = torch.empty((y_rows_total, N), dtype=_F32, device=x.device)
+    t = _tile_rows(rows_max, w, w2, act, exact, G, y)
+    if t:
+        return _tile_gemm(_tile_operand(x, t, x_rows, group_offsets, G, rows_max), t, w, w2, y, act, G, y_rows)
     check(lib.mi_gemm_any_grouped_act(ptr(x), x.stride(0), ptr(x_rows), ptr(w), ptr(w2), _dt(w), int(act), ptr(group_offsets),
                                       G, rows_max, ptr(y), N, ptr(y_rows), N, K, int(exact), stream()),
           "mi_gemm_any_grouped_act")
@@ -1450,6 +1517,10 @@ def gemm_any_grouped_glu(x, x_rows, w, w2, act: int, limit: float, row_scale, ro
     G, N, K = w.shape
     assert x.shape[1] == K and group_offsets.numel() >= G + 1
     y = torch.empty((y_rows_total, N), dtype=_F32, device=x.device)
+    t = _tile_rows(rows_max, w, w2, act, exact, G, y)
+    if t:
+        return _tile_gemm(_tile_operand(x, t, x_rows, group_offsets, G, rows_max), t, w, w2, y, act, G, y_rows, limit=limit,
+                          row_scale=row_scale, row_scale_rows=row_scale_rows)
     check(lib.mi_gemm_any_grouped_glu(ptr(x), x.stride(0), ptr(x_rows), ptr(w), ptr(w2), _dt(w), int(act), float(limit),
                                       ptr(row_scale), ptr(row_scale_rows), ptr(group_offsets), G, rows_max, ptr(y), N,
                                       ptr(y_rows), N, K, int(exact), stream()), "mi_gemm_any_grouped_glu")

@@ -1,0 +1,98 @@
+"""Prompt-sized projections of the 32-bit-residual families on the tile kernels (mi_gemm_any_tile): edges of row, feature and
+group tiles, both kernels, every epilogue, scattered rows, against a float64 statement over the rounded operands.
+
+Bound: the operands' products are exact in fp32, the sum over K carries at most K roundings of 2^-24 of the absolute sum, the
+epilogue a handful more; activations are 1.13-Lipschitz at most (gelu, silu), relu^2 and the clamped pair scale with their
+arguments - so: error <= (K + 16) * 2^-24 * (what the same expression gives on absolute values) + 1e-6."""
+import pytest
+import torch
+
+from nanovllm import _C, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(z, z2, act, limit):
+    if act == _C.ACT_CLAMPED_GLU:
+        g, u = z.clamp(max=limit), z2.clamp(-limit, limit)
+        return g * torch.sigmoid(1.702 * g) * (u + 1)
+    a = {_C.ACT_NONE: lambda t: t, _C.ACT_SILU: torch.nn.functional.silu, _C.ACT_GELU_ERF: torch.nn.functional.gelu,
+         _C.ACT_GELU_TANH: lambda t: torch.nn.functional.gelu(t, approximate="tanh"), _C.ACT_RELU2: lambda t: t.clamp(min=0) ** 2}[act](z)
+    return a if z2 is None else a * z2
+
+
+def _close(got, want, size, K):
+    err = (got.double() - want).abs()
+    bound = (K + 16) * 2.0 ** -24 * size + 1e-6
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("M,N,K", [(256, 128, 64), (257, 132, 128), (511, 260, 192), (1030, 644, 320)])
+@pytest.mark.parametrize("act,dual", [(_C.ACT_NONE, False), (_C.ACT_GELU_ERF, False), (_C.ACT_RELU2, False), (_C.ACT_SILU, True),
+                                      (_C.ACT_GELU_TANH, True)])
+def test_plain_rows(tile, M, N, K, act, dual):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K + act)
+    x = torch.randn(M, K + 3, device="cuda", generator=g)[:, :K]   # rows that do not start on 16 bytes
+    w, w2 = (torch.randn(N, K, device="cuda", generator=g).mul(K ** -0.5).bfloat16() for _ in range(2))
+    bias, bias2 = torch.randn(N, device="cuda", generator=g), torch.randn(N, device="cuda", generator=g)
+    w2, bias2 = (w2, bias2) if dual else (None, None)
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    ops._tile_gemm(ops._tile_operand(x, tile), tile, w, w2, out[:M], act, bias=bias, bias2=bias2, alpha=0.5)
+    xr = x.bfloat16().double()
+    z = xr @ w.double().T + bias
+    z2 = xr @ w2.double().T + bias2 if dual else None
+    s = xr.abs() @ w.double().abs().T + bias.abs()
+    s2 = xr.abs() @ w2.double().abs().T + bias2.abs() if dual else 1.0
+    size = 2 * s * (s if act == _C.ACT_RELU2 else 1.0) * s2
+    _close(out[:M], 0.5 * _ref(z, z2, act, 0.0), size, K)
+    assert bool((out[M] == 7.0).all())
+
+
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("counts", [(300, 0, 1, 128, 129), (0, 0, 256, 257), (64,) * 8, (5, 700)])
+@pytest.mark.parametrize("act", [_C.ACT_SILU, _C.ACT_CLAMPED_GLU])
+def test_grouped_rows(tile, counts, act):
+    G, N, K, T = len(counts), 196, 128, 211
+    g = torch.Generator(device="cuda").manual_seed(sum(counts) + act)
+    P = sum(counts) + 9   # the last nine rows belong to no group
+    x = torch.randn(T, K, device="cuda", generator=g)
+    rows = torch.randint(0, T, (P,), device="cuda", generator=g, dtype=torch.int32)
+    rows[sum(counts):] = 1 << 30   # (never looked at)
+    place = torch.randperm(P, device="cuda", generator=g).to(torch.int32)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device="cuda")
+    w, w2 = (torch.randn(G, N, K, device="cuda", generator=g).mul(K ** -0.5).bfloat16() for _ in range(2))
+    scale = torch.rand(P, device="cuda", generator=g) if act == _C.ACT_CLAMPED_GLU else None
+    y = torch.full((P, N), 7.0, device="cuda")
+    operand = ops._tile_operand(x, tile, rows, off, G, P)
+    ops._tile_gemm(operand, tile, w, w2, y, act, G, place, limit=1.5, row_scale=scale, row_scale_rows=place if scale is not None else None)
+    y16 = torch.zeros((P, N), device="cuda", dtype=torch.bfloat16)
+    ops._tile_gemm(operand, tile, w, w2, y16, act, G, place, limit=1.5, row_scale=scale, row_scale_rows=place if scale is not None else None)
+    want, size = torch.full((P, N), 7.0, device="cuda", dtype=torch.float64), torch.ones(P, N, device="cuda", dtype=torch.float64)
+    for e in range(G):
+        r = slice(int(off[e]), int(off[e + 1]))
+        xr, at = x[rows[r].long()].bfloat16().double(), place[r].long()
+        f = scale[at].double().unsqueeze(1) if scale is not None else 1.0
+        z, z2 = xr @ w[e].double().T * f, xr @ w2[e].double().T * f
+        want[at] = _ref(z, z2, act, 1.5)
+        size[at] = 4 * (xr.abs() @ w[e].double().abs().T) * (xr.abs() @ w2[e].double().abs().T + 1)
+    _close(y, want, size, K)
+    done = place[:sum(counts)].long()
+    assert torch.equal(y16[done], y[done].bfloat16())
+
+
+@pytest.mark.parametrize("act,limit", [(_C.ACT_SILU, 0.0), (_C.ACT_CLAMPED_GLU, 7.0)])
+def test_expert_pair_takes_the_same_bits_as_two_products(act, limit):
+    E, top, T, W, ff = 8, 2, 500, 256, 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+    h = torch.randn(T, W, device="cuda", generator=g)
+    ids = torch.randint(0, E, (T, top), device="cuda", generator=g, dtype=torch.int32)
+    wts = torch.rand(T, top, device="cuda", generator=g)
+    off, tok, place = ops.moe_sort(ids, E)
+    gate, up = (torch.randn(E, ff, W, device="cuda", generator=g).mul(W ** -0.5).bfloat16() for _ in range(2))
+    down = torch.randn(E, W, ff, device="cuda", generator=g).mul(ff ** -0.5).bfloat16()
+    scale = wts if act == _C.ACT_CLAMPED_GLU else None
+    a = ops.gemm_any_grouped_glu(h, tok, gate, up, act, limit, scale, place if scale is not None else None, off, T * top, None, T * top)
+    two = ops.gemm_any_grouped(a, None, down, None, off, T * top, place, T * top)
+    one = ops.expert_ff(h, tok, gate, up, down, act, off, T * top, place, limit, scale, place if scale is not None else None)
+    assert ops._tile_rows(T * top, gate, up, act, False, E) and torch.equal(one, two)
