@@ -5,15 +5,16 @@
 // (From 128 rows on, bf16 products of the shapes in use - K a multiple of 64, no segments - go to gemm_any_tile.hip.)
 //
 // These serve the model families whose residual stream, norms and recurrences are kept in 32-bit floats and whose
-// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): four kernels,
+// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): five kernels,
 //
 //   gemm_any_mfma_kernel   bf16 weights: a 64 x 64 (from 512 rows: 128 x 128, with SwiGLU 128 x 64) output tile per 4-wave
 //                          workgroup, x rounded to bf16 on its way into LDS, v_mfma_f32_16x16x32_bf16, the next K
 //                          step's operands fetched while the current one is multiplied, edges zero-filled
 //   gemm_any_skinny_kernel bf16 weights, up to 64 rows per tile (decode batches, a decode step's experts): 16 features per
 //                          workgroup, the waves split K, fragments straight from memory
-//   gemm_any_fma_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, plain FMA chains in k
-//                          order - the float32 serving mode, and the routers of sparse feed-forwards in either mode
+//   gemm_any_f32_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, on the fp32 matrix instruction
+//                          - the float32 serving mode, and the routers of sparse feed-forwards in either mode
+//   gemm_any_fma_kernel    the same in plain FMA chains, for operands whose rows are not whole 128-byte lines
 //   gemm_any_rows_kernel   M <= 8 rows, and the exact mode up to 64: one wave per (output feature, batch of rows)
 //                          streams its weight row once, lanes split K in 16-byte pieces, butterfly reduction; both
 //                          dtypes, x not rounded
@@ -155,11 +156,11 @@ __device__ __forceinline__ void load8<float>(const float* p, int n_valid, bool v
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// exact kernel: 64 x 64 tile, 256 threads, 4 x 4 outputs per thread, k ascending
+// exact kernel for any alignment and K: 64 x 64 tile, 256 threads, 4 x 4 outputs per thread, k ascending
 // ---------------------------------------------------------------------------------------------------------------
-template <typename TW, bool DUAL, int RT, bool EXT>  // RT rows per thread: a 64 x 64 tile (4) or 16 x 64 (1: few features, many rows)
+template <typename TW, bool DUAL, bool EXT>
 __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
-  constexpr int BM = 16 * RT, BN = 64, BK = 32, PAD = 4;
+  constexpr int RT = 4, BM = 16 * RT, BN = 64, BK = 32, PAD = 4;
   __shared__ float As[BK][BM + PAD];
   __shared__ float Bs[DUAL ? 2 : 1][BK][BN + PAD];
   const int tid = threadIdx.x;
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
   const int n0 = blockIdx.x * BN;
   const int lr = tid >> 2, lk = (tid & 3) * 8;  // this thread stages 8 consecutive k of one row
   int64_t xrow = -1;
-  if (lr < BM && m0 + lr < m_hi) xrow = a.x_rows ? a.x_rows[m0 + lr] : m0 + lr;
+  if (m0 + lr < m_hi) xrow = a.x_rows ? a.x_rows[m0 + lr] : m0 + lr;
   const int wrow = n0 + lr < a.N ? n0 + lr : -1;
   float acc[DUAL ? 2 : 1][RT][4] = {};
   const int ty = tid >> 4, tx = tid & 15;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int k = k0 + lk + i;
-      if (lr < BM) As[lk + i][lr] = (xrow >= 0 && k < a.K) ? a.x[xrow * a.ldx + k] : 0.f;
+      As[lk + i][lr] = (xrow >= 0 && k < a.K) ? a.x[xrow * a.ldx + k] : 0.f;
       Bs[0][lk + i][lr] = (wrow >= 0 && k < a.K) ? w_load<TW>(w + (int64_t)wrow * a.K + k) : 0.f;
       if (DUAL) Bs[1][lk + i][lr] = (wrow >= 0 && k < a.K) ? w_load<TW>(w2 + (int64_t)wrow * a.K + k) : 0.f;
     }
@@ -212,6 +213,142 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
       const int n = n0 + tx * 4 + j;
       if (n >= a.N) continue;
       a.y[yrow * a.ldy + n] = finish<DUAL, EXT>(a, m, yrow, n, acc[0][i][j], acc[DUAL ? 1 : 0][i][j]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// exact kernel on the matrix cores: v_mfma_f32_16x16x4_f32 (fp32 operands, fp32 products and sums; twice the vector rate)
+// ---------------------------------------------------------------------------------------------------------------
+// Four waves (WM x WN) with FM x FN fragments of 16 x 16 each.  K in steps of 32 floats = one 128-byte line of a row, by
+// LDS-DMA (global_load_lds, 16 bytes a lane: eight rows an instruction; bf16 weights: sixteen rows of 64 bytes) into a ring of
+// four images, so that three steps are in flight: these products are latency-bound, not rate-bound, at the sizes they come in
+// (a router's 32 features, an expert's hundred rows).  A row's 16-byte chunks are XOR-swizzled by its number, on the source
+// side of the DMA and at the fragment reads: sixteen rows at one chunk are sixteen different bank groups.  A lane reads four
+// consecutive k of its row at once (ds_read_b128; bf16: 8 bytes, widened): element j goes into the j-th MFMA of a group
+// of 16 k, which then contracts k = 4 (lane >> 4) + j - a fixed order of the sum, whatever the tile.
+// Rows beyond the group's end and features beyond N are read from the last valid one and not stored.
+// Needs K % 32 == 0, 16-byte aligned rows of x and w; anything else: gemm_any_fma_kernel.
+// Measured against gemm_any_fma_kernel (64 x 64 tiles, element-wise loads, plain FMA chains), us: see launch_exact.
+template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT>
+__global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
+  constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN, BK = 32, NST = 4, ND = DUAL ? 2 : 1;
+  constexpr bool WF = sizeof(TW) == 4;
+  constexpr int WROW = BK * (int)sizeof(TW), WRP = 1024 / WROW;           // bytes of a weight row's step, rows of a piece
+  constexpr int XB = BM * 128, WB = BN * WROW, STAGE = XB + ND * WB;
+  constexpr int PIECES = STAGE / 1024, PP = (PIECES + 3) / 4;             // 1 KiB each; PP per wave (the last may repeat)
+  static_assert(WM * WN == 4 && XB % 1024 == 0 && WB % 1024 == 0, "whole pieces");
+  __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int m_lo, m_hi;
+  const TW *w, *w2;
+  select_group<TW, DUAL>(a, w, w2, m_lo, m_hi);
+  const int m0 = m_lo + blockIdx.y * BM;
+  if (m0 >= m_hi) return;
+  const int n0 = blockIdx.x * BN;
+  const char* src[PP];
+  int dst[PP];
+#pragma unroll
+  for (int i = 0; i < PP; ++i) {
+    const int p = min(wave * PP + i, PIECES - 1);
+    dst[i] = p * 1024;
+    if (p < XB / 1024) {
+      const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+      const int m = min(m0 + r, m_hi - 1);
+      const int64_t row = a.x_rows ? a.x_rows[m] : m;
+      src[i] = reinterpret_cast<const char*>(a.x + row * a.ldx) + c * 16;
+    } else {
+      const int q = p - XB / 1024, d = q / (WB / 1024);
+      constexpr int CH = WROW / 16;
+      const int r = (q - d * (WB / 1024)) * WRP + lane / CH;
+      const int c = (lane % CH) ^ (WF ? (r >> 1) & 7 : (r >> 2) & 3);
+      src[i] = reinterpret_cast<const char*>((DUAL && d ? w2 : w) + (int64_t)min(n0 + r, a.N - 1) * a.K) + c * 16;
+    }
+  }
+  const int KT = a.K / BK;
+  auto issue = [&](int kt) __attribute__((always_inline)) {
+    char* base = lds + (kt & (NST - 1)) * STAGE;
+#pragma unroll
+    for (int i = 0; i < PP; ++i) {
+      const bool x = dst[i] < XB;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)kt * (x ? 128 : WROW)),
+                                       (__attribute__((address_space(3))) void*)(base + dst[i]), 16, 0, 0);
+    }
+  };
+  const int wm = (wave / WN) * 16 * FM, wn = (wave % WN) * 16 * FN;
+  const int r16 = lane & 15, kg = lane >> 4;
+  f32x4 acc[ND][FM][FN];
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[d][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < KT) issue(s);
+  for (int kt = 0; kt < KT; ++kt) {
+    const int behind = min(KT - 1 - kt, NST - 2);  // steps requested behind this one: their pieces may still fly
+    if (behind == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PP) : "memory");
+    else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PP) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (kt + NST - 1 < KT) issue(kt + NST - 1);  // (into the image everybody finished reading before the barrier)
+    const char* sx = lds + (kt & (NST - 1)) * STAGE;
+    const char* sw = sx + XB;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      f32x4 xf[FM], wf[ND][FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int r = wm + i * 16 + r16;
+        xf[i] = *reinterpret_cast<const f32x4*>(sx + r * 128 + (((ks * 4 + kg) ^ ((r >> 1) & 7)) << 4));
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const int r = wn + j * 16 + r16;
+          if constexpr (WF) {
+            wf[d][j] = *reinterpret_cast<const f32x4*>(sw + d * WB + r * 128 + (((ks * 4 + kg) ^ ((r >> 1) & 7)) << 4));
+          } else {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(sw + d * WB + r * 64 + (((ks * 2 + (kg >> 1)) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8);
+            wf[d][j] = f32x4{lo_bf(v[0]), hi_bf(v[0]), lo_bf(v[1]), hi_bf(v[1])};
+          }
+        }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+              acc[d][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[d][j][e], xf[i][e], acc[d][i][j], 0, 0, 0);
+    }
+  }
+  const bool y_vec = (a.ldy % 4 == 0) && dev_aligned16(a.y);
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + wm + i * 16 + r16;
+    if (m >= m_hi) continue;
+    const int64_t yrow = a.y_rows ? a.y_rows[m] : m;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int n = n0 + wn + j * 16 + kg * 4;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        v[r] = n + r < a.N ? finish<DUAL, EXT>(a, m, yrow, n + r, acc[0][i][j][r], acc[ND - 1][i][j][r]) : 0.f;
+      float* yp = a.y + yrow * a.ldy + n;
+      if (n + 4 <= a.N && y_vec) {
+        *reinterpret_cast<float4*>(yp) = float4{v[0], v[1], v[2], v[3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < a.N) yp[r] = v[r];
+      }
     }
   }
 }
@@ -495,6 +632,34 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
   }
 }
 
+// Exact mode beyond a few rows.  The tile of gemm_any_f32_kernel: the largest of 64 x 64, 32 x 64, 32 x 32 whose grid puts a
+// workgroup on most of the 256 CUs; groups of less than 256 rows (an even share is assumed) in 32-row tiles, whose last one
+// is padded by less.  us, gemm_any_fma_kernel / here: 733 rows, K 1024: N 1024 64 / 17, N 3072 202 / 67, N 32 113 / 12; 32
+// experts of 92 rows, 1024 -> 2 x 512 with SwiGLU 351 / 96 (64-row tiles: 141), back to 1024 216 / 55 (66); a router, 8192
+// rows, K 2048, 64 bf16 rows 235 / 36.
+template <typename TW, bool DUAL, bool EXT>
+static int launch_exact(const GemmAnyArgs& a, int groups, int rows_per_group_max, hipStream_t st) {
+  constexpr int W16 = 16 / (int)sizeof(TW);
+  const bool grouped = a.group_offsets != nullptr;
+  const bool vec = a.K % 32 == 0 && a.ldx % 4 == 0 && aligned16(a.x) && aligned16(a.w) && (!DUAL || aligned16(a.w2)) && a.K % W16 == 0 &&
+                   a.x_batch % 4 == 0;
+  if (vec) {
+    const int rows = grouped ? (rows_per_group_max + groups - 1) / groups : rows_per_group_max;
+    auto tiles = [&](int bm, int bn) { return (int64_t)((rows + bm - 1) / bm) * ((a.N + bn - 1) / bn) * groups; };
+    auto grid = [&](int bm, int bn) { return dim3((a.N + bn - 1) / bn, (rows_per_group_max + bm - 1) / bm, groups); };
+    if (rows > 32 && a.N > 32 && tiles(64, 64) >= 180 && !(grouped && rows < 256)) {
+      hipLaunchKernelGGL((gemm_any_f32_kernel<TW, DUAL, 2, 2, 2, 2, EXT>), grid(64, 64), dim3(256), 0, st, a);
+    } else if (a.N > 32 && tiles(32, 64) >= 180) {
+      hipLaunchKernelGGL((gemm_any_f32_kernel<TW, DUAL, 2, 1, 1, 4, EXT>), grid(32, 64), dim3(256), 0, st, a);
+    } else {
+      hipLaunchKernelGGL((gemm_any_f32_kernel<TW, DUAL, 1, 1, 2, 2, EXT>), grid(32, 32), dim3(256), 0, st, a);
+    }
+    return check_launch();
+  }
+  hipLaunchKernelGGL((gemm_any_fma_kernel<TW, DUAL, EXT>), dim3((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups), dim3(256), 0, st, a);
+  return check_launch();
+}
+
 template <typename TW, bool DUAL, bool EXT>
 static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, int mode, hipStream_t st) {
   // mode 0: product (MFMA for bf16 weights, the row kernel for few rows); 1: exact (FMA chains / row kernel, x unrounded)
@@ -537,12 +702,7 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
       return check_launch();
     }
   }
-  if (a.N <= 64 && rows_per_group_max >= 1024) {  // a router over a prompt: one column of tiles - short tiles, more of them
-    hipLaunchKernelGGL((gemm_any_fma_kernel<TW, DUAL, 1, EXT>), dim3(1, (rows_per_group_max + 15) / 16, groups), dim3(256), 0, st, a);
-    return check_launch();
-  }
-  hipLaunchKernelGGL((gemm_any_fma_kernel<TW, DUAL, 4, EXT>), grid, dim3(256), 0, st, a);
-  return check_launch();
+  return launch_exact<TW, DUAL, EXT>(a, groups, rows_per_group_max, st);
 }
 
 }  // namespace mi
