@@ -11,8 +11,8 @@
 //                               s_ij = scale q_i.k_j - slope_h (i - j), keys 0 <= i - j < window, separate key and value
 //                               head sizes, grouped heads, optional sigmoid output gate; prompt portions and single
 //                               decoded tokens in one launch (a row's keys are addressed through its sequence's block
-//                               table and total length); three kernels: matrix cores for prompt portions over a bf16
-//                               cache, 16-byte-load VALU form (decode: four waves per row and head), element-wise form
+//                               table and total length); four kernels: matrix cores for prompt portions (attn_prompt.hip) and
+//                               for decode over a bf16 cache, 16-byte-load VALU form, element-wise form
 //   mi_causal_conv_silu         short causal depthwise convolution over time + SiLU, carried across steps by a
 //   mi_causal_conv_state        per-sequence state slot holding the last taps - 1 inputs
 //   mi_channel_delta            gated delta rule with one decay per head AND key channel:
@@ -36,6 +36,7 @@
 // A step's rows are described by cu_q [n_seqs + 1] (row range of each sequence) and kv_lens [n_seqs] (the sequence's
 // length INCLUDING this step's rows): row r of sequence s sits at position kv_lens[s] - (cu_q[s+1] - cu_q[s]) + r.
 #include "seqmix_common.hpp"
+#include "attn_bias.hpp"
 
 namespace mi {
 
@@ -136,76 +137,6 @@ __global__ __launch_bounds__(256) void swa_prepare_kernel(float* __restrict__ pr
     }
     if (slot >= 0) st_f<TC>(v_cache + ((blk * G + c / Dv) * block_size + off) * Dv + c % Dv, v);
   }
-}
-
-// Distance bias of a score, taken off it: kind MI_BIAS_SLOPE: 2^(-8 (h + 1) / H) * dist (p1 == nullptr) or p1[h] * dist;
-// MI_BIAS_LOG: p1[h] * ln(1 + p2[h] * dist); MI_BIAS_NONE: nothing.  ldv: elements between two tokens' value rows (Dv,
-// or the key row's length when the values are the leading channels of the key rows of the same cache).
-// sink != nullptr: a row's softmax normalises by sum_j exp(s_j) + exp(sink[h]): the extra term is a learned per-head
-// logit taken as it is (the score scale does not touch it) that only soaks up weight - nothing is added to the output
-// for it.
-// softcap > 0: the scaled, biased score s becomes softcap * tanh(s / softcap) before the mask and the softmax.
-// value_heads: the value cache has this many heads (a divisor of the key heads G; query head h reads value head
-// h / (H / value_heads)) - fewer, wider value heads than key heads let every query head weigh the values of SEVERAL
-// key/value heads at once (value rows holding the heads side by side), which is what mixing the heads' softmax weights
-// afterwards needs.
-// chunk > 0: position i sees the keys of its own chunk only (floor(i / chunk) = floor(j / chunk), positions counted from
-// the sequence's start); with the window: both hold.
-// kept > 0: the first `kept` keys of a sequence stay visible from everywhere behind them, whatever window and chunk say.
-struct AttnBias {
-  int kind;
-  const float* p1;
-  const float* p2;
-  const float* sink;
-  float softcap;
-  int value_heads;
-  int chunk;
-  int kept;
-};
-// the oldest key position `pos` sees
-__device__ __forceinline__ int first_key(const AttnBias& bias, int pos, int window) {
-  int lo = max(0, pos - window + 1);
-  if (bias.chunk > 0) lo = max(lo, pos - pos % bias.chunk);
-  return lo;
-}
-// Kept keys lie away from the window: a walk over the keys counts u from lo - min(kept, lo) on, the u below lo stand for
-// the kept keys that are older than lo (gap = lo - min(kept, lo) further down), the others for themselves - one run of
-// numbers without holes, so that kept and window keys share the rounds of 32 / 64.  lo: the oldest key of the walk's first
-// row by window and chunk.
-__device__ __forceinline__ int kept_gap(const AttnBias& bias, int lo) { return lo - min(bias.kept, lo); }
-template <bool KEEP>
-__device__ __forceinline__ int key_at(int u, int lo, int gap) { return KEEP && u < lo ? u - gap : u; }
-__device__ __forceinline__ float capped(const AttnBias& bias, float s) {
-  return bias.softcap > 0.f ? bias.softcap * tanhf(s / bias.softcap) : s;
-}
-// the denominator of a finished row: its keys' sum l (relative to the running maximum m) plus the head's sink
-__device__ __forceinline__ float with_sink(const AttnBias& bias, int h, float m, float l) {
-  return bias.sink ? l + expf(bias.sink[h] - m) : l;
-}
-struct HeadBias {
-  float a, b;
-  bool log;
-};
-__device__ __forceinline__ HeadBias head_bias(const AttnBias& bias, int h, int H) {
-  HeadBias r{0.f, 0.f, bias.kind == MI_BIAS_LOG};
-  if (bias.kind == MI_BIAS_SLOPE) r.a = bias.p1 ? bias.p1[h] : exp2f(-8.f * (float)(h + 1) / (float)H);
-  else if (bias.kind == MI_BIAS_LOG) r.a = bias.p1[h], r.b = bias.p2[h];
-  return r;
-}
-__device__ __forceinline__ float dist_bias(const HeadBias& hb, int dist) {
-  return hb.log ? hb.a * log1pf(hb.b * (float)dist) : hb.a * (float)dist;
-}
-
-// Row of a token in a paged cache [blocks][kv heads][block_size][.]: (table[key / block_size] * G + g) * block_size +
-// key % block_size, in 32-bit arithmetic (rows of a cache are far fewer than 2^32; the byte offset is formed from it with
-// one 32 x 32 -> 64-bit multiply-add), the division a shift when block_size is a power of two (bs_shift >= 0).
-__device__ __forceinline__ int block_shift(int block_size) {
-  return (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
-}
-__device__ __forceinline__ uint32_t cache_row(const int32_t* table, int key, int G, int g, int block_size, int bs_shift) {
-  const int blk = bs_shift >= 0 ? key >> bs_shift : key / block_size;
-  const int off = bs_shift >= 0 ? key & (block_size - 1) : key - blk * block_size;
-  return ((uint32_t)table[blk] * (uint32_t)G + (uint32_t)g) * (uint32_t)block_size + (uint32_t)off;
 }
 
 // The general form (any head sizes): one wave per (row, head); lanes over keys for the scores, over value channels for
@@ -453,202 +384,6 @@ __global__ __launch_bounds__(256) void swa_attention_vec_kernel(const float* __r
           float o = acc[r][e] * inv;
           if (gate) o *= sigmoid_f(gate[row * ldg + h * Dv + d]);
           out[row * ldo + h * Dv + d] = o;
-        }
-      }
-    }
-    first = end;
-  }
-}
-
-// The matrix-core form for prompt portions over a bf16 cache (D a multiple of 32, Dv of 16): a wave takes 16 consecutive
-// step rows of one head.  S^T = K Q^T on v_mfma_f32_16x16x32_bf16 with the KEYS on the row axis (the A operand is a key's
-// cache row as stored: 16-byte loads), 32 keys per round; O^T += V^T P^T with the contraction slots ordered as the score
-// registers are (slot 8 g + e of lane group g = key 4 g + e of the first 16-key tile for e < 4, of the second for
-// e >= 4), so the softmax weights go from the accumulators into the B operand without leaving their lane; the V^T
-// operand gathers its eight keys' elements.  Scores and weights stay fp32 quantities: q and p enter the MFMAs as
-// bf16 hi + lo pairs (two MFMAs each, products exact, fp32 accumulation: 16 mantissa bits of q and p against the 8 of a
-// plain bf16 operand), scale, distance bias, mask, running maximum and sum are fp32 VALU work on the accumulators.
-template <int DKM, int DVM, bool PAIR, bool KEEP>  // KEEP: bias.kept > 0
-__global__ __launch_bounds__(256) void swa_attention_mfma_kernel(const float* __restrict__ q, int64_t ldq,
-                                                                 const uint16_t* __restrict__ k_cache,
-                                                                 const uint16_t* __restrict__ v_cache,
-                                                                 const int32_t* __restrict__ block_tables, int table_cols,
-                                                                 const int32_t* __restrict__ cu_q,
-                                                                 const int32_t* __restrict__ kv_lens, int n_seqs,
-                                                                 int n_rows, int H, int G, int D, int Dv, int block_size,
-                                                                 int window, float scale, AttnBias bias, int64_t ldv,
-                                                                 const float* __restrict__ gate, int64_t ldg,
-                                                                 float* __restrict__ out, int64_t ldo) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wid = blockIdx.x * 4 + wave;
-  const int n_groups = (n_rows + 15) / 16;
-  if (wid >= n_groups * H) return;
-  const int rg = wid / H, h = wid % H;
-  const int g = h / (H / G);
-  const int Gv = bias.value_heads, gv = h / (H / Gv);
-  const HeadBias hb = head_bias(bias, h, H);
-  const int qi = lane & 15, kg = lane >> 4;
-  const int dk = D / 32, dvt = Dv / 16;
-  const int bs_shift = block_shift(block_size);
-  const bool q_vec = (ldq % 4 == 0) && ((reinterpret_cast<uintptr_t>(q) & 15u) == 0) && (D % 4 == 0);
-  const int group_end = min(rg * 16 + 16, n_rows);
-  for (int first = rg * 16; first < group_end;) {
-    const int s = seq_of_row(cu_q, n_seqs, first);
-    const int end = min(cu_q[s + 1], group_end), nr = end - first;
-    const int pos0 = kv_lens[s] - (cu_q[s + 1] - cu_q[s]) + (first - cu_q[s]);
-    const int32_t* table = block_tables + (int64_t)s * table_cols;
-    bf16x8 qh[DKM], ql[DKM];
-#pragma unroll
-    for (int ks = 0; ks < DKM; ++ks) {
-      float xv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (ks < dk && qi < nr) {
-        const float* qp = q + (int64_t)(first + qi) * ldq + h * D + ks * 32 + kg * 8;
-        if (q_vec) {
-          const float4 a = *reinterpret_cast<const float4*>(qp), b = *reinterpret_cast<const float4*>(qp + 4);
-          xv[0] = a.x, xv[1] = a.y, xv[2] = a.z, xv[3] = a.w, xv[4] = b.x, xv[5] = b.y, xv[6] = b.z, xv[7] = b.w;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xv[e] = qp[e];
-        }
-      }
-      float lo[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) lo[e] = xv[e] - rbf(xv[e]);
-      qh[ks] = as_frag(u32x4{pack_bf(xv[0], xv[1]), pack_bf(xv[2], xv[3]), pack_bf(xv[4], xv[5]), pack_bf(xv[6], xv[7])});
-      ql[ks] = as_frag(u32x4{pack_bf(lo[0], lo[1]), pack_bf(lo[2], lo[3]), pack_bf(lo[4], lo[5]), pack_bf(lo[6], lo[7])});
-    }
-    const int lo_key = first_key(bias, pos0, window), hi_key = pos0 + nr - 1;
-    const int gap = KEEP ? kept_gap(bias, lo_key) : lo_key;
-    const int my_pos = pos0 + qi;
-    const int my_lo = first_key(bias, my_pos, window);
-    float m = -INFINITY, l = 0.f;
-    f32x4 oacc[DVM];
-#pragma unroll
-    for (int dt = 0; dt < DVM; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int j0 = gap; j0 <= hi_key; j0 += 32) {
-      f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        // this lane's row of the K operand; rows beyond the last key repeat it (their scores are masked below), so
-        // that every load is unconditional and a round's loads are all in flight together
-        const int key = key_at<KEEP>(min(j0 + t * 16 + qi, hi_key), lo_key, gap);
-        const uint16_t* kr =
-            k_cache + (int64_t)cache_row(table, key, G, g, block_size, bs_shift) * D + kg * 8;
-#pragma unroll
-        for (int ks = 0; ks < DKM; ++ks) {
-          if (ks < dk) {
-            const bf16x8 kf = as_frag(*reinterpret_cast<const u32x4*>(kr + ks * 32));
-            sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qh[ks], sacc[t], 0, 0, 0);
-            sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, ql[ks], sacc[t], 0, 0, 0);
-          }
-        }
-      }
-      float sc[8];
-      bool vis[8];
-      int dist[8];
-      float mx = -INFINITY;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = key_at<KEEP>(j0 + (e >> 2) * 16 + kg * 4 + (e & 3), lo_key, gap);
-        vis[e] = qi < nr && key <= my_pos && (key >= my_lo || (KEEP && key < bias.kept));
-        sc[e] = sacc[e >> 2][e & 3] * scale;
-        dist[e] = my_pos - key;
-      }
-      // the bias kind is the same for the whole launch: a branch every wave takes the same way, so that the logarithms
-      // are not evaluated (and thrown away) where the bias is linear or absent
-      if (bias.kind == MI_BIAS_LOG) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sc[e] -= hb.a * log1pf(hb.b * (float)max(dist[e], 0));
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sc[e] -= hb.a * (float)dist[e];
-      }
-      if (bias.softcap > 0.f) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sc[e] = bias.softcap * tanhf(sc[e] / bias.softcap);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        sc[e] = vis[e] ? sc[e] : -INFINITY;
-        mx = fmaxf(mx, sc[e]);
-      }
-      mx = xor_max<32>(xor_max<16>(mx));
-      const float m_new = fmaxf(m, mx);
-      const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
-      float pv[8], psum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pv[e] = vis[e] ? expf(sc[e] - m_new) : 0.f;
-        psum += pv[e];
-      }
-      psum = xor_sum<32>(xor_sum<16>(psum));
-      l = l * corr + psum;
-      m = m_new;
-      float plo[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) plo[e] = pv[e] - rbf(pv[e]);
-      const bf16x8 ph = as_frag(u32x4{pack_bf(pv[0], pv[1]), pack_bf(pv[2], pv[3]), pack_bf(pv[4], pv[5]), pack_bf(pv[6], pv[7])});
-      const bf16x8 pl = as_frag(u32x4{pack_bf(plo[0], plo[1]), pack_bf(plo[2], plo[3]), pack_bf(plo[4], plo[5]), pack_bf(plo[6], plo[7])});
-      // V^T operand: the lane's eight keys (its contraction slots) at ONE channel per 16-channel tile - or, when Dv is a
-      // multiple of 32 (PAIR), at TWO neighbouring channels per 32-channel pair of tiles with one 4-byte load: the low
-      // halves feed the tile of the pair's even channels, the high halves the tile of its odd channels
-      const uint16_t* vrow[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        // (beyond the last key: weight 0)
-        const int key = key_at<KEEP>(min(j0 + (e >> 2) * 16 + kg * 4 + (e & 3), hi_key), lo_key, gap);
-        vrow[e] = v_cache + (int64_t)cache_row(table, key, Gv, gv, block_size, bs_shift) * (int)ldv +
-                  (PAIR ? 2 * qi : qi);
-      }
-      if constexpr (PAIR) {
-#pragma unroll
-        for (int dp = 0; dp < DVM / 2; ++dp) {
-          if (2 * dp < dvt) {
-            uint32_t w[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) w[e] = *reinterpret_cast<const uint32_t*>(vrow[e] + dp * 32);
-            const bf16x8 v_even = as_frag(u32x4{(w[0] & 0xffffu) | (w[1] << 16), (w[2] & 0xffffu) | (w[3] << 16),
-                                                (w[4] & 0xffffu) | (w[5] << 16), (w[6] & 0xffffu) | (w[7] << 16)});
-            const bf16x8 v_odd = as_frag(u32x4{(w[0] >> 16) | (w[1] & 0xffff0000u), (w[2] >> 16) | (w[3] & 0xffff0000u),
-                                               (w[4] >> 16) | (w[5] & 0xffff0000u), (w[6] >> 16) | (w[7] & 0xffff0000u)});
-            oacc[2 * dp] *= corr;
-            oacc[2 * dp + 1] *= corr;
-            oacc[2 * dp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_even, ph, oacc[2 * dp], 0, 0, 0);
-            oacc[2 * dp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_even, pl, oacc[2 * dp], 0, 0, 0);
-            oacc[2 * dp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_odd, ph, oacc[2 * dp + 1], 0, 0, 0);
-            oacc[2 * dp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_odd, pl, oacc[2 * dp + 1], 0, 0, 0);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int dt = 0; dt < DVM; ++dt) {
-          if (dt < dvt) {
-            uint32_t ve[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ve[e] = (uint32_t)vrow[e][dt * 16];
-            const bf16x8 vf = as_frag(u32x4{ve[0] | (ve[1] << 16), ve[2] | (ve[3] << 16), ve[4] | (ve[5] << 16), ve[6] | (ve[7] << 16)});
-            oacc[dt] *= corr;
-            oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph, oacc[dt], 0, 0, 0);
-            oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, oacc[dt], 0, 0, 0);
-          }
-        }
-      }
-    }
-    if (qi < nr) {
-      // the lane holds channels 16 dt + 4 kg + r of its query's output (PAIR: tile 2 dp + b holds the channels
-      // 32 dp + 2 (4 kg + r) + b, i.e. the lane has the eight consecutive channels 32 dp + 8 kg .. + 7)
-      const float inv = 1.f / with_sink(bias, h, m, l);
-      const int64_t row = first + qi;
-#pragma unroll
-      for (int dt = 0; dt < DVM; ++dt) {
-        if (dt < dvt) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int d = PAIR ? (dt >> 1) * 32 + 2 * (kg * 4 + r) + (dt & 1) : dt * 16 + kg * 4 + r;
-            float o = oacc[dt][r] * inv;
-            if (gate) o *= sigmoid_f(gate[row * ldg + h * Dv + d]);
-            out[row * ldo + h * Dv + d] = o;
-          }
         }
       }
     }
@@ -2093,27 +1828,10 @@ static int launch_swa(const float* q, int64_t ldq, const void* kc, const void* v
   constexpr int VEC = 16 / sizeof(TC);
   // (v may point at a column of wider value rows: the fast forms load it in 16-byte / 4-byte pieces)
   const bool v16 = (reinterpret_cast<uintptr_t>(vc) & 15u) == 0;
-  if constexpr (sizeof(TC) == 2) {
-    // prompt portions over a bf16 cache: the matrix-core form
-    if (v16 && rows > n_seqs && D % 32 == 0 && Dv % 16 == 0 && D <= 256 && Dv <= 256 && ldv % 2 == 0) {
-      const dim3 grid_m((((rows + 15) / 16) * H + 3) / 4);
-#define MI_SWA_MFMA(DKM, DVM, PAIR, KEEP)                                                                             \
-  hipLaunchKernelGGL((swa_attention_mfma_kernel<DKM, DVM, PAIR, KEEP>), grid_m, dim3(256), 0, st, q, ldq, k, v, bt, cols, \
-                     cu_q, kv_lens, n_seqs, rows, H, G, D, Dv, block_size, window, scale, bias, ldv, gate, ldg, out, ldo)
-#define MI_SWA_MFMA_KEEP(DKM, DVM, PAIR)                    \
-  do {                                                      \
-    if (bias.kept > 0) MI_SWA_MFMA(DKM, DVM, PAIR, true);   \
-    else MI_SWA_MFMA(DKM, DVM, PAIR, false);                \
-  } while (0)
-      const bool small = D <= 128 && Dv <= 128, pair = Dv % 32 == 0;
-      if (small && pair) MI_SWA_MFMA_KEEP(4, 8, true);
-      else if (small) MI_SWA_MFMA_KEEP(4, 8, false);
-      else if (pair) MI_SWA_MFMA_KEEP(8, 16, true);
-      else MI_SWA_MFMA_KEEP(8, 16, false);
-#undef MI_SWA_MFMA_KEEP
-#undef MI_SWA_MFMA
-      return check_launch();
-    }
+  if (rows > n_seqs) {  // prompt portions: matrix cores, a workgroup's K / V rows shared by 128 (row, head) columns
+    const int rc = launch_prompt_attention(q, ldq, kc, vc, sizeof(TC) == 2, bt, cols, cu_q, kv_lens, n_seqs, rows, H, G, D, Dv,
+                                           block_size, window, scale, bias, ldv, gate, ldg, out, ldo, st);
+    if (rc != MI_EUNSUPPORTED) return rc;
   }
   if constexpr (sizeof(TC) == 2) {
     // decode steps (a row per sequence) over a bf16 cache: the matrix-core form with a kv head's query heads as columns

@@ -1,0 +1,100 @@
+"""Attention of prompt portions (csrc/attn_prompt.hip): the forms its images, tiles and page look-ups branch on, against float64.
+
+Bounds.  bf16 pages: q and the weights enter the products as hi + lo pairs (2^-17 of each), the rest is fp32; fp32 pages: fp32
+throughout, scores in units of ln 2 (2^-23 of a score's size in a weight's exponent).  With |scores| <= 30: 2e-5 of the largest value
+on bf16 pages, 1e-5 on fp32 pages."""
+import math
+
+import pytest
+import torch
+
+from nanovllm import _C, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(dtype, H, G, D, Dv, block, seqs, window=2 ** 31 - 1, kept=0, chunk=0, softcap=0.0, sink=False, bias=_C.BIAS_NONE, vik=False,
+          gate=False, value_heads=None):
+    g = torch.Generator(device="cuda").manual_seed(H * 131 + D * 7 + Dv + block + len(seqs))
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    Gv = value_heads or G
+    pages = [-(-(a + n) // block) for a, n in seqs]
+    order = torch.randperm(sum(pages) + 1, device="cuda", generator=g).int()
+    table = torch.full((len(seqs), max(pages)), -1, dtype=torch.int32, device="cuda")
+    at = 0
+    for i, n in enumerate(pages):
+        table[i, :n] = order[at:at + n]
+        at += n
+    k_cache = torch.full((len(order), G, block, D), float("nan"), device="cuda").to(dtype)   # rows nobody wrote stay NaN
+    v_cache = k_cache if vik else torch.full((len(order), Gv, block, Dv), float("nan"), device="cuda").to(dtype)
+    ks, vs = [], []
+    for i, (a, n) in enumerate(seqs):
+        p = torch.arange(a + n, device="cuda")
+        k = rnd(a + n, G, D).to(dtype)
+        k_cache[table[i, p // block].long(), :, p % block] = k
+        if not vik:
+            v = rnd(a + n, Gv, Dv).to(dtype)
+            v_cache[table[i, p // block].long(), :, p % block] = v
+        ks.append(k.double())
+        vs.append(k.double()[..., :Dv] if vik else v.double())
+    rows = sum(n for _, n in seqs)
+    q, gt = rnd(rows, H * D), rnd(rows, H * Dv) if gate else None
+    cu = torch.tensor([0] + list(torch.tensor([n for _, n in seqs]).cumsum(0)), dtype=torch.int32, device="cuda")
+    kv = torch.tensor([a + n for a, n in seqs], dtype=torch.int32, device="cuda")
+    sk = rnd(H) if sink else None
+    p1, p2 = (torch.rand(H, device="cuda", generator=g), torch.rand(H, device="cuda", generator=g)) if bias == _C.BIAS_LOG else (None, None)
+    scale = D ** -0.5
+    got = ops.paged_attention_f32(q, k_cache, v_cache, D if vik else Dv, table, cu, kv, H, G, D, Dv, block, window, scale, bias, p1, p2,
+                                  gate=gt, sink=sk, softcap=softcap, chunk=chunk, kept=kept, value_heads=Gv)
+    want = torch.empty(rows, H, Dv, dtype=torch.float64, device="cuda")
+    for i, (a, n) in enumerate(seqs):
+        qq = q[int(cu[i]):int(cu[i + 1])].double().view(n, H, D)
+        pos, key = torch.arange(a, a + n, device="cuda").view(-1, 1), torch.arange(a + n, device="cuda").view(1, -1)
+        dist = pos - key
+        seen = (dist >= 0) & (((dist < window) & ((pos // chunk == key // chunk) if chunk else True)) | (key < kept))
+        for h in range(H):
+            s = qq[:, h] @ ks[i][:, h // (H // G)].T * scale
+            if bias == _C.BIAS_SLOPE:
+                s = s - 2.0 ** (-8.0 * (h + 1) / H) * dist
+            elif bias == _C.BIAS_LOG:
+                s = s - p1[h].double() * torch.log1p(p2[h].double() * dist.clamp(min=0))
+            if softcap:
+                s = softcap * torch.tanh(s / softcap)
+            s = s.masked_fill(~seen, -math.inf)
+            if sink:
+                s = torch.cat([s, sk[h].double().expand(n, 1)], 1)
+            want[int(cu[i]):int(cu[i + 1]), h] = torch.softmax(s, 1)[:, :a + n] @ vs[i][:, h // (H // Gv)]
+    want = want.view(rows, H * Dv)
+    if gate:
+        want = want * torch.sigmoid(gt.double())
+    tol = (2e-5 if dtype == torch.bfloat16 else 1e-5) * float(want.abs().max())
+    assert float((got.double() - want).abs().max()) <= tol
+
+
+SEQS = ((0, 1), (130, 70), (0, 33), (17, 1), (31, 2))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,G,D,Dv", [(6, 2, 64, 64), (5, 1, 64, 128), (8, 8, 128, 128), (4, 4, 96, 48), (7, 1, 256, 192), (2, 1, 32, 256),
+                                      (130, 1, 32, 16)])
+def test_head_shapes(dtype, H, G, D, Dv):
+    _case(dtype, H, G, D, Dv, 16, SEQS, gate=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("block", [8, 16, 48, 64, 256])
+def test_page_sizes(dtype, block):
+    _case(dtype, 4, 2, 64, 64, block, SEQS, window=50, bias=_C.BIAS_SLOPE)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", [dict(window=1), dict(window=40, kept=5), dict(window=64, kept=70), dict(chunk=48), dict(chunk=33, kept=3),
+                                  dict(softcap=5.0, sink=True), dict(bias=_C.BIAS_LOG, sink=True), dict(value_heads=1), dict(kept=500)])
+def test_masks_and_biases(dtype, form):
+    _case(dtype, 4, 2, 64, 128, 32, SEQS + ((200, 97),), **form)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,Dv", [(256, 256), (224, 160)])
+def test_values_inside_the_key_rows(dtype, D, Dv):
+    _case(dtype, 16, 1, D, Dv, 64, SEQS, vik=True, sink=True)
