@@ -718,6 +718,15 @@ int mi_channel_delta(const float* qkv, int64_t ld, int q_off, int k_off, int v_o
                      const float* a_log, const float* gate_pre, int64_t ld_gate, const float* norm_w, float* state,
                      const int32_t* cu_q, const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows, int H,
                      int G, int D, int Dv, float eps, float* workspace, float* out, int64_t ldo, mi_stream stream);
+/* mi_channel_delta for prompt portions, sixteen rows at a time (csrc/delta_blocks.hip): the same state and results.
+ * mi_channel_delta_blocks_elems: floats of 16-byte aligned workspace, 0 where the row-by-row call is the better one (max_rows: the most
+ * rows that one sequence brings), -1 beyond the compiled kernels (D <= 256). */
+int64_t mi_channel_delta_blocks_elems(int n_rows, int n_seqs, int max_rows, int H, int D);
+int mi_channel_delta_blocks(const float* qkv, int64_t ld, int q_off, int k_off, int v_off, const float* beta_pre,
+                            int64_t ld_beta, const float* decay_pre, int64_t ld_decay, const float* dt_bias, const float* a_log,
+                            const float* gate_pre, int64_t ld_gate, const float* norm_w, float* state, const int32_t* cu_q,
+                            const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows, int H, int G, int D, int Dv,
+                            float eps, float* workspace, int64_t ws_elems, float* out, int64_t ldo, mi_stream stream);
 #define MI_ROUTE_SOFTMAX 0    /* scores = softmax(logits) over n_outputs */
 #define MI_ROUTE_SIGMOID 1    /* scores = sigmoid(logits), each output for itself */
 #define MI_ROUTE_GROUP_MAX  0 /* a group's value: its largest choice score */

@@ -1,0 +1,402 @@
+// The channel-wise gated delta rule over prompt portions, sixteen rows at a time on the fp32 matrix instruction
+// (mi_channel_delta_blocks); short steps walk row by row (seqmix.hip: channel_delta_kernel).
+//
+//   S <- diag(g_t) S;   u_t = beta_t (v_t - S^T k_t);   S <- S + k_t u_t^T;   o_t = S^T q_t
+//
+// Over a block of rows t = 0..15 behind the state S0, with P_t = g_0 .. g_t and P_jt = g_{j+1} .. g_t (products per key channel, all at
+// most 1: nothing is divided by a decay, so nothing can overflow):
+//   the decayed state read with k_t:  D_t = (k_t P_t)^T S0,   A_tj = sum_d k_t P_jt k_j  (j < t)
+//   read with q_t:                    E_t = (q_t P_t)^T S0,   B_tj = sum_d q_t P_jt k_j  (j <= t)
+//   u_t = beta_t (v_t - D_t - sum_j A_tj u_j)   =>   U = T (V - D),  T = (1 + diag(beta) A)^-1 diag(beta)   (16 x 16, lower triangular)
+//   O = E + B U,      S <- diag(P_15) S0 + sum_j (k_j P_j15) u_j^T
+// blocks_prepare_kernel (a workgroup per block and head, all blocks at once) leaves (k P), (q P), (k P_.15), P_15, B and T of a block as
+// one record in MFMA operand order; blocks_walk_kernel (a wave per 16 value columns, S in its registers as MFMA accumulators, which
+// are the next block's B operand as they stand) walks a sequence's records.
+//
+// What bounds it: the chain of a sequence's blocks; 104 matrix instructions of 32 cycles each (128 channels) are 1.4 us, the vector
+// work between them brings a block to 2.7 us, against 0.71 us per ROW of the row-by-row walk (LDS reads, cross-lane sums, plain FMAs).
+// 8 sequences of 1024 rows, 8 heads, 128 x 128: 809 us row by row, 294 so (preparation 83, walk 175).  The error against 64 bits is
+// the row-by-row one's (rms within 3 % at 5 .. 100 rows).  A NaN or an infinity in a row reaches the rows of its own block, of the
+// same sequence, in front of it too (zero times NaN), not only the ones behind it, whose state it spoils either way.
+#include "seqmix_common.hpp"
+
+namespace mi {
+
+constexpr int kB = 16;                     // rows of a block
+constexpr int kStateCols = 32;             // value columns of a block of the state's memory layout (seqmix.hip: kDeltaCols)
+
+// floats of a record, DP = 16 DT key channels: [k P: DP * 16][q P: DP * 16][k P_.15: DP * 16][B: 256][T: 256][P_15: DP], rounded up to
+// whole KiB
+constexpr int record_floats(int dp) { return (3 * dp * kB + 512 + dp + 255) & ~255; }
+
+// First record of sequence s, whose rows begin at r0: r0 / 16 + s, at least as far from the next sequence's as it has blocks
+// (ceil(n / 16) <= (r0 + n) / 16 - r0 / 16 + 1), so that no block has to add up the sequences before it.
+__host__ __device__ constexpr int first_record(int r0, int s) { return r0 / kB + s; }
+
+struct BlockArgs {
+  const float* qkv;
+  int64_t ld;
+  int q_off, k_off, v_off;
+  const float* beta_pre;   // [rows][H]
+  int64_t ld_beta;
+  const float* decay_pre;  // [rows][H * D]
+  int64_t ld_decay;
+  const float* dt_bias;    // [H * D]
+  const float* a_log;      // [H]
+  const int32_t* cu_q;
+  const int32_t* kv_lens;
+  const int32_t* slot_ids;
+  int n_seqs, H, G, D, Dv;
+  float* state;
+  float* records;
+  float* out;
+  int64_t ldo;
+};
+
+__device__ __forceinline__ f32x4 sum8(const f32x4 (&x)[8]) { return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])); }
+
+template <int DT>
+__global__ __launch_bounds__(256) void blocks_prepare_kernel(BlockArgs a) {
+  constexpr int DP = 16 * DT, LD = DP + 4;   // (rows 16 bytes apart in their banks: sixteen of them are read at one channel group)
+  __shared__ __attribute__((aligned(16))) float kk[kB][LD], qq[kB][LD], gg[kB][LD];
+  __shared__ float am[kB][kB + 1], bm[kB][kB + 1], gamma[DP], beta[kB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.y;
+  // the block's sequence: the last one whose records begin at or before it
+  int s = -1;
+  for (int i0 = 0; i0 < a.n_seqs; i0 += 64) {
+    const int i = i0 + lane;
+    const int found = __popcll(__ballot(i < a.n_seqs && first_record(a.cu_q[min(i, a.n_seqs - 1)], i) <= (int)blockIdx.x));
+    s += found;
+    if (found < 64) break;
+  }
+  s = __builtin_amdgcn_readfirstlane(s);
+  const int r0 = a.cu_q[s] + ((int)blockIdx.x - first_record(a.cu_q[s], s)) * kB, n = min(kB, a.cu_q[s + 1] - r0);
+  if (n <= 0) return;  // (a record that no block uses)
+  // ---- the rows' q, k and decays; rows beyond the sequence's end change nothing: k = q = 0, g = 1, beta = 0 ----
+  const int hq = h / (a.H / a.G);
+  const float rate = expf(a.a_log[h]);
+  constexpr int RW = kB / 4, C = DP / 64;
+  float qv[RW][C], kv[RW][C], gv[RW][C], bv[RW];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {   // (every load first, at clamped places: none waits for another)
+    const int64_t r = r0 + min(wave * RW + i, n - 1);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int d = min(lane + 64 * c, a.D - 1);
+      qv[i][c] = a.qkv[r * a.ld + a.q_off + hq * a.D + d];
+      kv[i][c] = a.qkv[r * a.ld + a.k_off + hq * a.D + d];
+      gv[i][c] = a.decay_pre[r * a.ld_decay + h * a.D + d];
+    }
+    bv[i] = a.beta_pre[r * a.ld_beta + h];
+  }
+  float bias[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) bias[c] = a.dt_bias[h * a.D + min(lane + 64 * c, a.D - 1)];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const int t = wave * RW + i;
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const bool ok = t < n && lane + 64 * c < a.D;
+      const float q = ok ? qv[i][c] : 0.f, k = ok ? kv[i][c] : 0.f;
+      qv[i][c] = q, kv[i][c] = k;
+      gg[t][lane + 64 * c] = ok ? expf(-rate * softplus_f(gv[i][c] + bias[c])) : 1.f;
+      sq = fmaf(q, q, sq);
+      sk = fmaf(k, k, sk);
+    }
+    const float nq = (1.f / sqrtf((float)a.D)) / sqrtf(wave_sum(sq) + 1e-6f), nk = 1.f / sqrtf(wave_sum(sk) + 1e-6f);
+    if (lane == 0) beta[t] = t < n ? sigmoid_f(bv[i]) : 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) qq[t][lane + 64 * c] = qv[i][c] * nq, kk[t][lane + 64 * c] = kv[i][c] * nk;
+  }
+  __syncthreads();
+  // ---- A and B: sixteen lanes per j walk t = 0..15 with p = k_j P_jt (0 before t = j) ----
+  {
+    const int j = tid >> 4, c = tid & 15;
+    float p[DT];
+#pragma unroll
+    for (int i = 0; i < DT; ++i) p[i] = 0.f;
+#pragma unroll 4
+    for (int t = 0; t < kB; ++t) {
+      float sa = 0.f, sb = 0.f;
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        const float k = kk[t][16 * i + c];
+        p[i] = t == j ? k : p[i] * gg[t][16 * i + c];
+        sa = fmaf(p[i], k, sa);
+        sb = fmaf(p[i], qq[t][16 * i + c], sb);
+      }
+      sa = xor_sum<8>(xor_sum<4>(xor_sum<2>(xor_sum<1>(sa))));
+      sb = xor_sum<8>(xor_sum<4>(xor_sum<2>(xor_sum<1>(sb))));
+      if (c == 0) am[t][j] = sa, bm[t][j] = sb;
+    }
+  }
+  __syncthreads();
+  // ---- the decayed vectors in place (a thread per channel and direction): kk <- k P, qq <- q P, gg <- k P_.15; T column by column ----
+  float* const rec = a.records + ((int64_t)blockIdx.x * a.H + h) * record_floats(DP);
+  float* const rec_q = rec + DP * kB;
+  float* const rec_k = rec_q + DP * kB;
+  float* const rec_b = rec_k + DP * kB;
+  // (products of up to sixteen decays in 64 bits, rounded once: the walk applies them to what it has summed over all rows)
+  float back[2][kB];
+#pragma unroll
+  for (int i = 0; i < (2 * DP + 255) / 256; ++i) {
+    const int id = tid + 256 * i, d = id < DP ? id : id - DP;
+    if (id < 2 * DP) {
+      double p = 1.;
+      if (id < DP) {
+#pragma unroll
+        for (int t = 0; t < kB; ++t) {
+          p *= gg[t][d];
+          qq[t][d] = (float)(qq[t][d] * p);
+        }
+        gamma[d] = (float)p;
+      } else {
+#pragma unroll
+        for (int t = kB - 1; t >= 0; --t) {
+          back[i][t] = (float)(kk[t][d] * p);
+          p *= gg[t][d];
+        }
+        p = 1.;
+#pragma unroll
+        for (int t = 0; t < kB; ++t) {
+          p *= gg[t][d];
+          kk[t][d] = (float)(kk[t][d] * p);
+        }
+      }
+    }
+  }
+  if (tid < kB) {
+    const int c = tid;
+    float col[kB];
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) sum = fmaf(am[i][j], col[j], sum);
+      col[i] = beta[i] * ((i == c ? 1.f : 0.f) - sum);
+    }
+#pragma unroll
+    for (int i = 0; i < kB; ++i) rec_b[256 + ((c >> 2) * 16 + i) * 4 + (c & 3)] = col[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < (2 * DP + 255) / 256; ++i) {
+    const int id = tid + 256 * i;
+    if (id >= DP && id < 2 * DP)
+#pragma unroll
+      for (int t = 0; t < kB; ++t) gg[t][id - DP] = back[i][t];
+  }
+  __syncthreads();
+  // ---- the record, 16 bytes a thread: slot (tile m of 16 channels, lane group g, r) ----
+  for (int i = tid; i < DT * 64; i += 256) {
+    const int m = i >> 6, kg = (i >> 4) & 3, r = i & 15;
+    *reinterpret_cast<float4*>(rec + i * 4) = *reinterpret_cast<const float4*>(&kk[r][16 * m + 4 * kg]);
+    *reinterpret_cast<float4*>(rec_q + i * 4) = *reinterpret_cast<const float4*>(&qq[r][16 * m + 4 * kg]);
+    *reinterpret_cast<float4*>(rec_k + i * 4) = float4{gg[4 * kg][16 * m + r], gg[4 * kg + 1][16 * m + r], gg[4 * kg + 2][16 * m + r], gg[4 * kg + 3][16 * m + r]};
+  }
+  if (tid < 64) {
+    const int kg = tid >> 4, r = tid & 15;
+    *reinterpret_cast<float4*>(rec_b + tid * 4) = float4{bm[r][4 * kg], bm[r][4 * kg + 1], bm[r][4 * kg + 2], bm[r][4 * kg + 3]};
+  }
+  for (int d = tid; d < DP; d += 256) rec_b[512 + d] = gamma[d];
+}
+
+// grid: (sequences, heads, value columns / 64); a wave takes 16 columns.  Ring of three records (two where three do not fit: 256 channels) (with the rows' values behind each, a
+// wave's own 16 columns) by LDS-DMA two blocks ahead; in front of a group's matrix instructions stand the LDS reads of the next one.
+template <int DT>
+__global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
+  constexpr int DP = 16 * DT, REC = record_floats(DP), PIECES = REC / 256, PP = (PIECES + 3) / 4, IMG = REC * 4 + 4096;
+  constexpr int NST = 3 * IMG <= 163840 ? 3 : 2;
+  __shared__ __attribute__((aligned(1024))) char lds[NST * IMG];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int s = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 64 + wave * 16 + r16;
+  const int r0 = a.cu_q[s], n = a.cu_q[s + 1] - r0;
+  if (n == 0) return;
+  const int nb = (n + kB - 1) / kB;
+  const char* const recs = reinterpret_cast<const char*>(a.records + ((int64_t)first_record(r0, s) * a.H + h) * REC);
+  const int64_t rec_stride = (int64_t)a.H * REC * 4;
+  const float* vp[4];   // the next block's rows 4 kg + r at this lane's column
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    vp[r] = a.qkv + (int64_t)(r0 + min(4 * kg + r, n - 1)) * a.ld + a.v_off + (int64_t)h * a.Dv + min(col, a.Dv - 1);
+  // PP + 4 requests, whatever the block (beyond the end: the last one's again; rows beyond the end: the last row's)
+  auto issue = [&](int b, int st) __attribute__((always_inline)) {
+    const int bb = min(b, nb - 1);
+    char* const to = lds + st * IMG;
+#pragma unroll
+    for (int i = 0; i < PP; ++i) {
+      const int p = min(wave * PP + i, PIECES - 1);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(recs + bb * rec_stride + p * 1024 + (uint32_t)(lane * 16)),
+                                       (__attribute__((address_space(3))) void*)(to + p * 1024), 16, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vp[r],
+                                       (__attribute__((address_space(3))) void*)(to + REC * 4 + wave * 1024 + r * 256), 4, 0, 0);
+    const int left = n - 1 - (b + 1) * kB;   // rows behind the next block's first
+    if (left >= kB - 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vp[r] += (int64_t)kB * a.ld;
+    } else if (left >= 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vp[r] += (int64_t)(kB + min(4 * kg + r, left) - (4 * kg + r)) * a.ld;
+    }
+  };
+  // the state: S[m][r] = key channel 16 m + 4 kg + r of this lane's column; in memory as the row-by-row kernels keep it
+  const int cb = col / kStateCols, cbs = (a.Dv + kStateCols - 1) / kStateCols, cc = col % kStateCols;
+  const bool has_state = cb < cbs, has_col = col < a.Dv;
+  float* const st = a.state + (((int64_t)a.slot_ids[s] * a.H + h) * cbs + cb) * (DP * kStateCols);
+  f32x4 S[DT];
+#pragma unroll
+  for (int m = 0; m < DT; ++m) S[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (has_state && a.kv_lens[s] > n) {
+#pragma unroll
+    for (int m = 0; m < DT; ++m) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[m][r] = st[(4 * m + r) * (4 * kStateCols) + cc * 4 + kg];
+    }
+  }
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  float* op = a.out + (int64_t)(r0 + 4 * kg) * a.ldo + (int64_t)h * a.Dv + col;   // (formed beyond the columns, not used there)
+  auto store = [&](int b) __attribute__((always_inline)) {
+    if (b * kB + kB <= n) {
+      if (has_col)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) op[r * a.ldo] = o[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (has_col && b * kB + 4 * kg + r < n) op[r * a.ldo] = o[r];
+    }
+    op += (int64_t)kB * a.ldo;
+  };
+#pragma unroll
+  for (int i = 0; i + 1 < NST; ++i) issue(i, i);
+  int cur = 0;
+  for (int b = 0; b < nb; ++b) {
+    // record b has landed (a ring of three: record b + 1's requests may be out); everybody is done with record b - 1: its place is free
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * (PP + 4)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (b > 0) store(b - 1);   // (here, not behind the block: the wait above would have to see them home)
+    issue(b + NST - 1, cur == 0 ? NST - 1 : cur - 1);
+    const char* const img = lds + cur * IMG;
+    cur = cur == NST - 1 ? 0 : cur + 1;
+    const char* const rec = img + lane * 16;
+    const char* const rec_q = rec + DP * kB * 4;
+    const char* const rec_k = rec_q + DP * kB * 4;
+    const char* const rec_b = rec_k + DP * kB * 4;
+    const char* const gam = rec_b - lane * 16 + 2048 + kg * 16;   // P_15 of this lane's channels 16 m + 4 kg ..
+    auto vec = [](const char* p) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(p); };
+    f32x4 d[8], e[8];   // (eight chains: each is an eighth as long, and so is its rounding)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) d[r] = e[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 pf[2][2], qf[2][2], gf[2][2], kf[2][4], u, tf = vec(rec_b + 1024), bf = vec(rec_b);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = *reinterpret_cast<const float*>(img + REC * 4 + wave * 1024 + r * 256 + lane * 4);
+    auto read_q = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        pf[c & 1][i] = vec(rec + (2 * c + i) * 1024);
+        qf[c & 1][i] = vec(rec_q + (2 * c + i) * 1024);
+        gf[c & 1][i] = vec(gam + (2 * c + i) * 64);
+      }
+    };
+    auto read_k = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kf[c & 1][i] = vec(rec_k + (4 * c + i) * 1024);
+    };
+    read_q(0);
+#pragma unroll
+    for (int c = 0; c < DT / 2; ++c) {
+      if (c + 1 < DT / 2) read_q(c + 1);
+      else read_k(0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          f32x4 &dx = d[4 * i + r], &ex = e[4 * i + r];
+          dx = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[c & 1][i][r], S[2 * c + i][r], dx, 0, 0, 0);
+          ex = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c & 1][i][r], S[2 * c + i][r], ex, 0, 0, 0);
+        }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) S[2 * c + i] *= gf[c & 1][i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = has_col && b * kB + 4 * kg + r < n ? u[r] : 0.f;
+    const f32x4 w = u - sum8(d);
+    u = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[r], w[r], u, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < DT / 4; ++c) {
+      if (c + 1 < DT / 4) read_k(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)   // (r outside i: a tile's four products wait for each other)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c & 1][i][r], u[r], S[4 * c + i], 0, 0, 0);
+    }
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[r], u[r], x, 0, 0, 0);
+    o = sum8(e) + x;
+  }
+  store(nb - 1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the requests beyond the end land before the workgroup's LDS is given away)
+  if (!has_state) return;
+#pragma unroll
+  for (int m = 0; m < DT; ++m) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) st[(4 * m + r) * (4 * kStateCols) + cc * 4 + kg] = S[m][r];
+  }
+}
+
+static int tiles_of(int D) { return D <= 64 ? 4 : D <= 128 ? 8 : D <= 256 ? 16 : 0; }
+
+}  // namespace mi
+
+using namespace mi;
+
+// Where the block form is used: a sequence's chain of blocks is 2.7 us per 16 rows against 0.71 us a row, but every sequence, also one
+// that brings a single row, costs a record.  us, rows / blocks, 8 heads of 128 x 128: one sequence of 16 rows 24 / 30, of 64 58 / 38;
+// 32 sequences of 16 rows 32 / 45, of 64 86 / 76; 64 rows beside 31 single ones 63 / 59, 256 beside 255 281 / 274, 1024 beside 255
+// 986 / 606; 256 sequences of 2 rows 64 / 179.
+extern "C" int64_t mi_channel_delta_blocks_elems(int n_rows, int n_seqs, int max_rows, int H, int D) {
+  const int dt = tiles_of(D);
+  if (n_rows < 0 || n_seqs < 1 || H < 1 || D < 1 || dt == 0) return -1;
+  if (max_rows < 64 + n_seqs / 2) return 0;
+  return ((int64_t)n_rows / kB + n_seqs) * H * record_floats(16 * dt);
+}
+
+extern "C" int mi_channel_delta_blocks(const float* qkv, int64_t ld, int q_off, int k_off, int v_off, const float* beta_pre,
+                                       int64_t ld_beta, const float* decay_pre, int64_t ld_decay, const float* dt_bias,
+                                       const float* a_log, const float* gate_pre, int64_t ld_gate, const float* norm_w, float* state,
+                                       const int32_t* cu_q, const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows,
+                                       int H, int G, int D, int Dv, float eps, float* workspace, int64_t ws_elems, float* out,
+                                       int64_t ldo, mi_stream stream) {
+  if (!qkv || !beta_pre || !decay_pre || !dt_bias || !a_log || !gate_pre || !norm_w || !state || !cu_q || !kv_lens || !slot_ids || !out ||
+      !workspace || n_seqs < 1 || n_rows < 0 || H < 1 || G < 1 || H % G || D < 1 || Dv < 1)
+    return MI_EINVAL;
+  const int dt = tiles_of(D);
+  if (dt == 0 || H > 65535 || Dv > 65535) return MI_EUNSUPPORTED;
+  if (n_rows == 0) return MI_OK;
+  if (!aligned16(workspace) || ws_elems < ((int64_t)n_rows / kB + n_seqs) * H * record_floats(16 * dt)) return MI_EWORKSPACE;
+  const BlockArgs a{qkv, ld, q_off, k_off, v_off, beta_pre, ld_beta, decay_pre, ld_decay, dt_bias, a_log, cu_q, kv_lens, slot_ids,
+                    n_seqs, H, G, D, Dv, state, workspace, out, ldo};
+  const dim3 prep(n_rows / kB + n_seqs, H), walk(n_seqs, H, (Dv + 63) / 64);   // (64 columns hold whole blocks of the state's layout)
+  const auto launch = [&](auto prepare, auto walk_kernel) -> int {
+    hipLaunchKernelGGL(prepare, prep, dim3(256), 0, S(stream), a);
+    if (check_launch() != MI_OK) return MI_ELAUNCH;
+    hipLaunchKernelGGL(walk_kernel, walk, dim3(256), 0, S(stream), a);
+    return check_launch();
+  };
+  const int rc = dt == 4   ? launch(blocks_prepare_kernel<4>, blocks_walk_kernel<4>)
+                 : dt == 8 ? launch(blocks_prepare_kernel<8>, blocks_walk_kernel<8>)
+                           : launch(blocks_prepare_kernel<16>, blocks_walk_kernel<16>);
+  return rc != MI_OK ? rc : launch_head_norm(out, ldo, gate_pre, ld_gate, norm_w, n_rows, H, Dv, eps, S(stream));
+}

@@ -770,7 +770,7 @@ __global__ __launch_bounds__(256) void causal_conv_step_kernel(const float* __re
 // ---------------------------------------------------------------------------------------------------------------
 // Three launches.  delta_prepare_kernel (parallel over rows): the row's unit q and k per q/k head, its decay vector and
 // beta per head - everything with a transcendental in it - into a workspace [rows][2 G D + H D + H].
-// channel_delta_kernel (the recurrence): the columns of S (one per value channel) never exchange anything: S^T k, the
+// channel_delta_kernel (the recurrence; long prompt portions go sixteen rows at a time, delta_blocks.hip): the columns of S (one per value channel) never exchange anything: S^T k, the
 // rank-one update and S^T q are per-column sums over the key channels.  One workgroup = 32 value columns of one
 // (sequence, head); a column is held by FOUR lanes (a quad), each keeping DR of the (padded) 4 * DR key channels of it
 // in registers for the whole walk over the sequence's rows of this step - lane r of the quad owns the channels
@@ -1999,6 +1999,13 @@ extern "C" int mi_causal_conv_state(const float* x, int64_t ldx, int taps, float
   return check_launch();
 }
 
+int mi::launch_head_norm(float* out, int64_t ldo, const float* gate_pre, int64_t ld_gate, const float* norm_w, int n_rows, int H,
+                         int Dv, float eps, hipStream_t st) {
+  hipLaunchKernelGGL(delta_finish_kernel, dim3((n_rows * H + 3) / 4), dim3(256), 0, st, out, ldo, gate_pre, ld_gate, norm_w, 0, n_rows,
+                     H, Dv, eps, MI_ACT_SIGMOID, 1.f);
+  return check_launch();
+}
+
 static int delta_dr(int D) { return D <= 64 ? 16 : D <= 128 ? 32 : D <= 256 ? 64 : 0; }
 
 extern "C" int64_t mi_channel_delta_state_elems(int H, int D, int Dv) {
@@ -2037,9 +2044,7 @@ extern "C" int mi_channel_delta(const float* qkv, int64_t ld, int q_off, int k_o
   else MI_DELTA(64);
 #undef MI_DELTA
   if (check_launch() != MI_OK) return MI_ELAUNCH;
-  hipLaunchKernelGGL(delta_finish_kernel, dim3((n_rows * H + 3) / 4), dim3(256), 0, S(stream), out, ldo, gate_pre,
-                     ld_gate, norm_w, 0, n_rows, H, Dv, eps, MI_ACT_SIGMOID, 1.f);
-  return check_launch();
+  return launch_head_norm(out, ldo, gate_pre, ld_gate, norm_w, n_rows, H, Dv, eps, S(stream));
 }
 
 extern "C" int mi_route_grouped(const float* logits, int64_t ld, const float* correction, int n_tokens, int n_outputs,

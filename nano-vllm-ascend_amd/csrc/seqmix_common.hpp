@@ -36,4 +36,9 @@ __device__ __forceinline__ int seq_of_row(const int32_t* cu_q, int n_seqs, int r
   return s;
 }
 
+// Read-out norm of the recurrences (seqmix.hip), in place: every head's Dv channels to unit rms, times norm_w [Dv], times sigmoid(gate)
+// with a gate.
+int launch_head_norm(float* out, int64_t ldo, const float* gate_pre, int64_t ld_gate, const float* norm_w, int n_rows, int H, int Dv,
+                     float eps, hipStream_t st);
+
 }  // namespace mi

@@ -184,7 +184,7 @@ class ChannelDeltaMixer(nn.Module):
         off = self.qkv.offsets
         o = ops.channel_delta(qkv, off["q"][0], off["k"][0], off["v"][0], self.low.cols(low, "b"), decay_pre, self.dt_bias,
                               self.A_log, gate_pre, self.norm, self.state, cu, kv, slots, self.H, self.G, self.D, self.Dv,
-                              self.eps)
+                              self.eps, ctx.max_seqlen_q)
         return ops.gemm_any(o, self.o)
 
 

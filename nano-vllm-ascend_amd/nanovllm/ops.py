@@ -1169,7 +1169,8 @@ def channel_delta_state_elems(H: int, D: int, Dv: int) -> int:
 
 
 def channel_delta(qkv, q_off: int, k_off: int, v_off: int, beta_pre, decay_pre, dt_bias, a_log, gate_pre, norm_w, state,
-                  cu_q, kv_lens, slot_ids, H: int, G: int, D: int, Dv: int, eps: float) -> torch.Tensor:
+                  cu_q, kv_lens, slot_ids, H: int, G: int, D: int, Dv: int, eps: float, max_rows: int = 1) -> torch.Tensor:
+    """max_rows: the most rows that one sequence brings (it only chooses the kernels)."""
     require_gpu(qkv, state)
     _f32(qkv, beta_pre, decay_pre, dt_bias, a_log, gate_pre, norm_w, state)
     _i32(cu_q, kv_lens, slot_ids)
@@ -1178,6 +1179,15 @@ def channel_delta(qkv, q_off: int, k_off: int, v_off: int, beta_pre, decay_pre, 
     assert beta_pre.shape == (rows, H) and decay_pre.shape == (rows, H * D) and gate_pre.shape == (rows, H * Dv)
     assert dt_bias.numel() == H * D and a_log.numel() == H and norm_w.numel() == Dv
     out = torch.empty((rows, H * Dv), dtype=_F32, device=qkv.device)
+    n = lib.mi_channel_delta_blocks_elems(rows, kv_lens.numel(), max_rows, H, D)
+    if n > 0:   # prompt portions: sixteen rows at a time
+        scratch = torch.empty(n, dtype=_F32, device=qkv.device)
+        check(lib.mi_channel_delta_blocks(ptr(qkv), qkv.stride(0), q_off, k_off, v_off, ptr(beta_pre), beta_pre.stride(0),
+                                          ptr(decay_pre), decay_pre.stride(0), ptr(dt_bias), ptr(a_log), ptr(gate_pre),
+                                          gate_pre.stride(0), ptr(norm_w), ptr(state), ptr(cu_q), ptr(kv_lens), ptr(slot_ids),
+                                          kv_lens.numel(), rows, H, G, D, Dv, float(eps), ptr(scratch), n, ptr(out), out.stride(0),
+                                          stream()), "mi_channel_delta_blocks")
+        return out
     scratch = torch.empty(max(1, lib.mi_channel_delta_workspace_elems(rows, H, G, D)), dtype=_F32, device=qkv.device)
     check(lib.mi_channel_delta(ptr(qkv), qkv.stride(0), q_off, k_off, v_off, ptr(beta_pre), beta_pre.stride(0),
                                ptr(decay_pre), decay_pre.stride(0), ptr(dt_bias), ptr(a_log), ptr(gate_pre),
