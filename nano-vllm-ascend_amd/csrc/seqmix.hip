@@ -74,27 +74,73 @@ __global__ __launch_bounds__(256) void embedding_sinusoid_f32_kernel(const int64
   }
 }
 
-// one workgroup per row; mean, then the mean of squared deviations (two passes over the row, which stays in L1)
+// VEC floats at p (VEC 4: 16-byte aligned; the row-wise kernels below take VEC 4 where every pointer, stride and width allows it, and
+// one float at a time otherwise)
+template <int VEC>
+using fvec = float __attribute__((ext_vector_type(VEC)));
+template <int VEC>
+__device__ __forceinline__ fvec<VEC> vat(const float* p) { return *reinterpret_cast<const fvec<VEC>*>(p); }
+template <int VEC>
+__device__ __forceinline__ float vsum(fvec<VEC> v) {
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) s += reinterpret_cast<const float*>(&v)[e];
+  return s;
+}
+
+// One workgroup per row; mean, then the mean of squared deviations.  Bound by the rows' bytes: a thread asks for all of its pieces (the
+// residual's too) before the first sum and keeps them (VEC 4: rows up to 4096 wide; the rest of wider ones is read again), so that a CU
+// has its whole share of requests out at once.  8112 rows of 2048, added to the residual: 37 us with a float per request, each pass over
+// the row again; now 19.
+template <int VEC>
 __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ y, int64_t ldy,
                                                             const float* __restrict__ w, const float* __restrict__ b,
                                                             float* __restrict__ out, int64_t ldo, int width, float eps,
                                                             int add) {
+  using vec = fvec<VEC>;
   __shared__ float red[4];
+  constexpr int KEEP = 4, STEP = 256 * VEC;
   const float* yr = y + (int64_t)blockIdx.x * ldy;
+  float* o = out + (int64_t)blockIdx.x * ldo;
+  const int c0 = threadIdx.x * VEC;
+  vec kept[KEEP], base[KEEP];
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = c0 + i * STEP;
+    kept[i] = base[i] = (vec)(0.f);
+    if (c < width) {
+      kept[i] = vat<VEC>(yr + c);
+      if (add) base[i] = vat<VEC>(o + c);
+    }
+  }
   float s = 0.f;
-  for (int c = threadIdx.x; c < width; c += 256) s += yr[c];
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) s += vsum<VEC>(kept[i]);
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP) s += vsum<VEC>(vat<VEC>(yr + c));
   const float mean = block_sum256(s, red) / (float)width;
   float q = 0.f;
-  for (int c = threadIdx.x; c < width; c += 256) {
-    const float d = yr[c] - mean;
-    q += d * d;
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i)
+    if (c0 + i * STEP < width) {
+      const vec d = kept[i] - mean;
+      q += vsum<VEC>(d * d);
+    }
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP) {
+    const vec d = vat<VEC>(yr + c) - mean;
+    q += vsum<VEC>(d * d);
   }
-  const float var = block_sum256(q, red) / (float)width;
-  const float rstd = 1.f / sqrtf(var + eps);
-  float* o = out + (int64_t)blockIdx.x * ldo;
-  for (int c = threadIdx.x; c < width; c += 256) {
-    const float v = (yr[c] - mean) * rstd * w[c] + b[c];
-    o[c] = add ? o[c] + v : v;
+  const float rstd = 1.f / sqrtf(block_sum256(q, red) / (float)width + eps);
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = c0 + i * STEP;
+    if (c < width) {
+      const vec v = (kept[i] - mean) * rstd * vat<VEC>(w + c) + vat<VEC>(b + c);
+      *reinterpret_cast<vec*>(o + c) = add ? base[i] + v : v;
+    }
+  }
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP) {
+    const vec v = (vat<VEC>(yr + c) - mean) * rstd * vat<VEC>(w + c) + vat<VEC>(b + c);
+    *reinterpret_cast<vec*>(o + c) = add ? vat<VEC>(o + c) + v : v;
   }
 }
 
@@ -693,6 +739,62 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(const float* __restric
   y[(int64_t)row * ldy + c] = acc;
 }
 
+// The same for 2 .. 5 taps over rows that can be read 16 bytes at a time: a thread takes four channels of eight rows in a row, their
+// filters once and the 7 + taps input rows in flight together; the taps are summed in the order above.  8192 rows of 2048 channels,
+// 4 taps: 102 us a row per workgroup (a walk over the sequences' borders and uncoalesced filters for every row); now 28.
+constexpr int kConvRows = 8;
+template <int TAPS>
+__global__ __launch_bounds__(256) void causal_conv_rows_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w,
+                                                               const float* __restrict__ state, const int32_t* __restrict__ cu_q,
+                                                               const int32_t* __restrict__ kv_lens,
+                                                               const int32_t* __restrict__ slot_ids, int n_seqs, int rows, int C, int silu,
+                                                               int add_input, float* __restrict__ y, int64_t ldy) {
+  const int row0 = blockIdx.x * kConvRows, c = (blockIdx.y * 256 + threadIdx.x) * 4, lane = threadIdx.x & 63;
+  int s = 0;   // row0's sequence: as many ends of sequences in front of the last one lie at or before it
+  for (int i0 = 0; i0 < n_seqs - 1; i0 += 64) {
+    const int i = i0 + lane;
+    const int found = __popcll(__ballot(i < n_seqs - 1 && cu_q[min(i + 1, n_seqs)] <= row0));
+    s += found;
+    if (found < 64) break;
+  }
+  s = __builtin_amdgcn_readfirstlane(s);
+  if (c >= C) return;
+  float4 xs[kConvRows + TAPS - 1], f[TAPS];
+#pragma unroll
+  for (int i = 0; i < kConvRows + TAPS - 1; ++i)   // (a row that no tap uses: the first or the last one again)
+    xs[i] = *reinterpret_cast<const float4*>(x + (int64_t)min(max(row0 + i - (TAPS - 1), 0), rows - 1) * ldx + c);
+#pragma unroll
+  for (int i = 0; i < TAPS; ++i) f[i] = *reinterpret_cast<const float4*>(w + (int64_t)c * TAPS + 4 * i);
+  const float* wt = reinterpret_cast<const float*>(f);   // [channel][tap]
+  int r0 = cu_q[s];
+#pragma unroll
+  for (int i = 0; i < kConvRows; ++i) {
+    const int row = row0 + i;
+    if (row >= rows) return;
+    while (s + 1 < n_seqs && row >= cu_q[s + 1]) ++s, r0 = cu_q[s];
+    float4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      float4 v = xs[i + j];
+      const int rr = row - r0 - (TAPS - 1) + j;
+      if (rr < 0) {   // in front of the step's rows: the state, zeros before the sequence
+        v = float4{0.f, 0.f, 0.f, 0.f};
+        if (kv_lens[s] - (cu_q[s + 1] - r0) > 0)
+          v = *reinterpret_cast<const float4*>(state + ((int64_t)slot_ids[s] * (TAPS - 1) + (TAPS - 1 + rr)) * C + c);
+      }
+      acc.x = fmaf(wt[j], v.x, acc.x), acc.y = fmaf(wt[TAPS + j], v.y, acc.y);
+      acc.z = fmaf(wt[2 * TAPS + j], v.z, acc.z), acc.w = fmaf(wt[3 * TAPS + j], v.w, acc.w);
+    }
+    if (silu) {
+      acc.x = acc.x / (1.f + expf(-acc.x)), acc.y = acc.y / (1.f + expf(-acc.y));
+      acc.z = acc.z / (1.f + expf(-acc.z)), acc.w = acc.w / (1.f + expf(-acc.w));
+    }
+    const float4 own = xs[i + TAPS - 1];
+    if (add_input) acc.x += own.x, acc.y += own.y, acc.z += own.z, acc.w += own.w;
+    *reinterpret_cast<float4*>(y + (int64_t)row * ldy + c) = acc;
+  }
+}
+
 // the new tail: the last taps - 1 inputs of (old tail ++ this step's rows).  One thread per (sequence, channel) reads
 // everything it needs before it writes, and no other thread touches its entries.
 __global__ __launch_bounds__(256) void causal_conv_state_kernel(const float* __restrict__ x, int64_t ldx, int taps,
@@ -1053,20 +1155,35 @@ __global__ __launch_bounds__(256) void route_grouped_kernel(const float* __restr
   }
 }
 
+// grid (token, 256 * VEC channels); the parts' pieces are asked for CH at a time (beyond top_k: the last one again, not added).  Bound by
+// the experts' outputs: 8192 tokens of 8 x 2048 floats, 191 us with a float per request and one part after the other; now 134 (4.8 TB/s).
+template <int VEC, int CH>
 __global__ __launch_bounds__(256) void moe_combine_f32_kernel(const float* __restrict__ y, const float* __restrict__ h,
                                                               int64_t ldh, const int32_t* __restrict__ ids,
                                                               const float* __restrict__ wts, int top_k, int n_experts,
                                                               int width, float* __restrict__ out, int64_t ldo) {
-  const int t = blockIdx.x;
-  for (int c = threadIdx.x; c < width; c += 256) {
-    float acc = 0.f;
-    for (int k = 0; k < top_k; ++k) {
-      const int e = ids[(int64_t)t * top_k + k];
-      const float v = e >= n_experts ? h[(int64_t)t * ldh + c] : y[((int64_t)t * top_k + k) * width + c];
-      acc = fmaf(wts[(int64_t)t * top_k + k], v, acc);
+  using vec = fvec<VEC>;
+  const int64_t t = blockIdx.x;
+  const int c = ((int)blockIdx.y * 256 + (int)threadIdx.x) * VEC;
+  if (c >= width) return;
+  vec acc = (vec)(0.f);
+  for (int k0 = 0; k0 < top_k; k0 += CH) {
+    vec v[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k = min(k0 + j, top_k - 1);
+      v[j] = vat<VEC>((ids[t * top_k + k] >= n_experts ? h + t * ldh : y + (t * top_k + k) * width) + c);
     }
-    out[(int64_t)t * ldo + c] = acc;
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      if (k0 + j < top_k) {
+        const float wt = wts[t * top_k + k0 + j];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          reinterpret_cast<float*>(&acc)[e] = fmaf(wt, reinterpret_cast<const float*>(&v[j])[e], reinterpret_cast<const float*>(&acc)[e]);
+      }
   }
+  *reinterpret_cast<vec*>(out + t * ldo + c) = acc;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1386,69 +1503,120 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
 
 // out[t] = sum_k w[t][k] y[t * top_k + k] + sigmoid(shared_gate[t]) * shared[t]   (shared == nullptr: no shared part;
 // shared_gate == nullptr: the shared part as it is; wts == nullptr: every weight 1 - experts whose weight already went into their input)
-__global__ __launch_bounds__(256) void moe_combine_shared_kernel(const float* __restrict__ y, const int32_t* __restrict__ ids,
-                                                                 const float* __restrict__ wts, int top_k, int width,
-                                                                 const float* __restrict__ shared, int64_t lds_,
+// (grid and requests as moe_combine_f32_kernel's)
+template <int VEC, int CH>
+__global__ __launch_bounds__(256) void moe_combine_shared_kernel(const float* __restrict__ y, const float* __restrict__ wts, int top_k,
+                                                                 int width, const float* __restrict__ shared, int64_t lds_,
                                                                  const float* __restrict__ shared_gate, int64_t ldsg,
                                                                  float* __restrict__ out, int64_t ldo) {
-  const int t = blockIdx.x;
-  const float sgate = shared_gate ? sigmoid_f(shared_gate[(int64_t)t * ldsg]) : 1.f;
-  for (int c = threadIdx.x; c < width; c += 256) {
-    float acc = 0.f;
-    for (int k = 0; k < top_k; ++k)
-      acc = fmaf(wts ? wts[(int64_t)t * top_k + k] : 1.f, y[((int64_t)t * top_k + k) * width + c], acc);
-    if (shared) acc = fmaf(sgate, shared[(int64_t)t * lds_ + c], acc);
-    out[(int64_t)t * ldo + c] = acc;
+  using vec = fvec<VEC>;
+  const int64_t t = blockIdx.x;
+  const int c = ((int)blockIdx.y * 256 + (int)threadIdx.x) * VEC;
+  if (c >= width) return;
+  const float sgate = shared_gate ? sigmoid_f(shared_gate[t * ldsg]) : 1.f;
+  vec acc = (vec)(0.f), sh = (vec)(0.f);
+  if (shared) sh = vat<VEC>(shared + t * lds_ + c);
+  auto add = [&](float wt, vec v) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+      reinterpret_cast<float*>(&acc)[e] = fmaf(wt, reinterpret_cast<const float*>(&v)[e], reinterpret_cast<const float*>(&acc)[e]);
+  };
+  for (int k0 = 0; k0 < top_k; k0 += CH) {
+    vec v[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) v[j] = vat<VEC>(y + (t * top_k + min(k0 + j, top_k - 1)) * width + c);
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      if (k0 + j < top_k) add(wts ? wts[t * top_k + k0 + j] : 1.f, v[j]);
   }
+  if (shared) add(sgate, sh);
+  *reinterpret_cast<vec*>(out + t * ldo + c) = acc;
 }
-
 
 // ---------------------------------------------------------------------------------------------------------------
 // gated sublayer output behind its own norm, added to the residual: res += rms(y * sigmoid(gate)) * w_post
 // ---------------------------------------------------------------------------------------------------------------
 // One workgroup per row.  v = y * sigmoid(gate_pre) (gate_pre may be nullptr: v = y); res += v / sqrt(mean(v^2) + eps) *
-// w_post; w_next != nullptr: out = res / sqrt(mean(res^2) + eps) * w_next - what the next sublayer reads.  A thread keeps
-// its (up to eight) gated values in registers between the two passes; wider rows recompute them.
+// w_post; w_next != nullptr: out = res / sqrt(mean(res^2) + eps) * w_next - what the next sublayer reads.  Bound by the rows' bytes: all of
+// a thread's pieces (VEC 4: rows up to 4096 wide; the rest of wider ones is read again) are asked for before the first sum.  8192 rows
+// of 2048 with a gate, 335 MB: 130 us with a float per request; now 57 (5.9 TB/s).
+template <int VEC>
 __global__ __launch_bounds__(256) void gated_norm_add_f32_kernel(float* __restrict__ res, int64_t ldr,
                                                                  const float* __restrict__ y, int64_t ldy,
                                                                  const float* __restrict__ gate_pre, int64_t ldg,
                                                                  const float* __restrict__ w_post, float eps,
                                                                  const float* __restrict__ w_next,
                                                                  float* __restrict__ out, int64_t ldo, int width) {
+  using vec = fvec<VEC>;
   __shared__ float red[4];
-  constexpr int KEEP = 8;
+  constexpr int KEEP = 4, STEP = 256 * VEC;
   float* r = res + (int64_t)blockIdx.x * ldr;
   const float* yr = y + (int64_t)blockIdx.x * ldy;
   const float* gr = gate_pre ? gate_pre + (int64_t)blockIdx.x * ldg : nullptr;
-  float kept[KEEP];
-  float sq = 0.f;
-  int i = 0;
-  for (int c = threadIdx.x; c < width; c += 256, ++i) {
-    float v = yr[c];
-    if (gr) v *= sigmoid_f(gr[c]);
-    if (i < KEEP) kept[i] = v;
-    sq = fmaf(v, v, sq);
+  auto gated = [&](vec v, vec g) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) reinterpret_cast<float*>(&v)[e] *= sigmoid_f(reinterpret_cast<const float*>(&g)[e]);
+    return v;
+  };
+  auto square = [](vec v, float s) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) s = fmaf(reinterpret_cast<const float*>(&v)[e], reinterpret_cast<const float*>(&v)[e], s);
+    return s;
+  };
+  auto again = [&](int c) { return gr ? gated(vat<VEC>(yr + c), vat<VEC>(gr + c)) : vat<VEC>(yr + c); };
+  auto added = [&](vec v, float scale, int c, vec to) {
+    const vec w = vat<VEC>(w_post + c);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+      reinterpret_cast<float*>(&to)[e] = fmaf(reinterpret_cast<const float*>(&v)[e] * scale, reinterpret_cast<const float*>(&w)[e],
+                                              reinterpret_cast<const float*>(&to)[e]);
+    return to;
+  };
+  const int c0 = threadIdx.x * VEC;
+  vec kept[KEEP], gv[KEEP], rv[KEEP];
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = c0 + i * STEP;
+    if (c < width) {
+      kept[i] = vat<VEC>(yr + c);
+      if (gr) gv[i] = vat<VEC>(gr + c);
+      rv[i] = vat<VEC>(r + c);
+    }
   }
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i)
+    if (c0 + i * STEP < width) {
+      if (gr) kept[i] = gated(kept[i], gv[i]);
+      sq = square(kept[i], sq);
+    }
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP) sq = square(again(c), sq);
   const float rstd = 1.f / sqrtf(block_sum256(sq, red) / (float)width + eps);
   float sq2 = 0.f;
-  i = 0;
-  for (int c = threadIdx.x; c < width; c += 256, ++i) {
-    float v;
-    if (i < KEEP) v = kept[i];
-    else {
-      v = yr[c];
-      if (gr) v *= sigmoid_f(gr[c]);
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = c0 + i * STEP;
+    if (c < width) {
+      kept[i] = added(kept[i], rstd, c, rv[i]);
+      *reinterpret_cast<vec*>(r + c) = kept[i];
+      sq2 = square(kept[i], sq2);
     }
-    const float x = fmaf(v * rstd, w_post[c], r[c]);
-    r[c] = x;
-    if (i < KEEP) kept[i] = x;
-    sq2 = fmaf(x, x, sq2);
+  }
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP) {
+    const vec x = added(again(c), rstd, c, vat<VEC>(r + c));
+    *reinterpret_cast<vec*>(r + c) = x;
+    sq2 = square(x, sq2);
   }
   if (!w_next) return;
   const float rstd2 = 1.f / sqrtf(block_sum256(sq2, red) / (float)width + eps);
   float* o = out + (int64_t)blockIdx.x * ldo;
-  i = 0;
-  for (int c = threadIdx.x; c < width; c += 256, ++i) o[c] = (i < KEEP ? kept[i] : r[c]) * rstd2 * w_next[c];
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = c0 + i * STEP;
+    if (c < width) *reinterpret_cast<vec*>(o + c) = kept[i] * rstd2 * vat<VEC>(w_next + c);
+  }
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP)  // (a thread re-reads its own writes)
+    *reinterpret_cast<vec*>(o + c) = vat<VEC>(r + c) * rstd2 * vat<VEC>(w_next + c);
 }
 
 // The same without a gate, for a sublayer output that is still in parts: v = sum_k wts[row][k] y[row * parts + k] +
@@ -1794,8 +1962,9 @@ extern "C" int mi_layernorm_f32(const float* y, int64_t ldy, const float* w, con
                                 int rows, int width, float eps, int add_to_out, mi_stream stream) {
   if (!y || !w || !b || !out || rows < 0 || width < 1 || ldy < width || ldo < width) return MI_EINVAL;
   if (rows == 0) return MI_OK;
-  hipLaunchKernelGGL(layernorm_f32_kernel, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out, ldo, width, eps,
-                     add_to_out);
+  const bool vec = width % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(w) && aligned16(b) && aligned16(out);
+  hipLaunchKernelGGL(vec ? layernorm_f32_kernel<4> : layernorm_f32_kernel<1>, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out,
+                     ldo, width, eps, add_to_out);
   return check_launch();
 }
 
@@ -1959,6 +2128,16 @@ extern "C" int mi_causal_conv(const float* x, int64_t ldx, const float* w, int t
   if (!x || !w || !state || !cu_q || !kv_lens || !slot_ids || !y || rows < 0 || n_seqs < 1 || channels < 1) return MI_EINVAL;
   if (taps < 1 || taps > 17) return MI_EUNSUPPORTED;
   if (rows == 0) return MI_OK;
+  if (taps >= 2 && taps <= 5 && channels % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && aligned16(x) && aligned16(w) && aligned16(state) &&
+      aligned16(y)) {
+    const auto kernel = taps == 2   ? causal_conv_rows_kernel<2>
+                        : taps == 3 ? causal_conv_rows_kernel<3>
+                        : taps == 4 ? causal_conv_rows_kernel<4>
+                                    : causal_conv_rows_kernel<5>;
+    hipLaunchKernelGGL(kernel, dim3((rows + kConvRows - 1) / kConvRows, (channels + 1023) / 1024), dim3(256), 0, S(stream), x, ldx, w,
+                       state, cu_q, kv_lens, slot_ids, n_seqs, rows, channels, silu, add_input, y, ldy);
+    return check_launch();
+  }
   hipLaunchKernelGGL(causal_conv_kernel, dim3(rows, (channels + 255) / 256), dim3(256), 0, S(stream), x, ldx, w, taps,
                      state, cu_q, kv_lens, slot_ids, n_seqs, channels, silu, add_input, y, ldy);
   return check_launch();
@@ -2068,7 +2247,10 @@ extern "C" int mi_moe_combine_f32(const float* y, const float* h, int64_t ldh, c
                                   mi_stream stream) {
   if (!y || !h || !ids || !weights || !out || n_tokens < 0 || top_k < 1 || width < 1) return MI_EINVAL;
   if (n_tokens == 0) return MI_OK;
-  hipLaunchKernelGGL(moe_combine_f32_kernel, dim3(n_tokens), dim3(256), 0, S(stream), y, h, ldh, ids, weights, top_k,
+  const bool vec = width % 4 == 0 && ldh % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(h) && aligned16(out);
+  const auto kernel = vec ? (top_k <= 4 ? moe_combine_f32_kernel<4, 4> : moe_combine_f32_kernel<4, 8>) : moe_combine_f32_kernel<1, 4>;
+  const int cols = vec ? 1024 : 256;
+  hipLaunchKernelGGL(kernel, dim3(n_tokens, (width + cols - 1) / cols), dim3(256), 0, S(stream), y, h, ldh, ids, weights, top_k,
                      n_experts, width, out, ldo);
   return check_launch();
 }
@@ -2186,8 +2368,12 @@ extern "C" int mi_moe_combine_shared(const float* y, const int32_t* ids, const f
                                      int64_t ld_gate, float* out, int64_t ldo, mi_stream stream) {
   if (!y || !ids || !out || n_tokens < 0 || top_k < 1 || width < 1) return MI_EINVAL;
   if (n_tokens == 0) return MI_OK;
-  hipLaunchKernelGGL(moe_combine_shared_kernel, dim3(n_tokens), dim3(256), 0, S(stream), y, ids, weights, top_k, width,
-                     shared, ld_shared, shared_gate, ld_gate, out, ldo);
+  const bool vec = width % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(out) &&
+                   (!shared || (ld_shared % 4 == 0 && aligned16(shared)));
+  const auto kernel = vec ? (top_k <= 4 ? moe_combine_shared_kernel<4, 4> : moe_combine_shared_kernel<4, 8>) : moe_combine_shared_kernel<1, 4>;
+  const int cols = vec ? 1024 : 256;
+  hipLaunchKernelGGL(kernel, dim3(n_tokens, (width + cols - 1) / cols), dim3(256), 0, S(stream), y, weights, top_k, width, shared,
+                     ld_shared, shared_gate, ld_gate, out, ldo);
   return check_launch();
 }
 
@@ -2196,8 +2382,10 @@ extern "C" int mi_gated_norm_add_f32(float* res, int64_t ldr, const float* y, in
                                      int64_t ldo, int rows, int width, mi_stream stream) {
   if (!res || !y || !w_post || rows < 0 || width < 1 || (w_next && !out)) return MI_EINVAL;
   if (rows == 0) return MI_OK;
-  hipLaunchKernelGGL(gated_norm_add_f32_kernel, dim3(rows), dim3(256), 0, S(stream), res, ldr, y, ldy, gate_pre, ldg,
-                     w_post, eps, w_next, out, ldo, width);
+  const bool vec = width % 4 == 0 && ldr % 4 == 0 && ldy % 4 == 0 && aligned16(res) && aligned16(y) && aligned16(w_post) &&
+                   (!gate_pre || (ldg % 4 == 0 && aligned16(gate_pre))) && (!w_next || (ldo % 4 == 0 && aligned16(out) && aligned16(w_next)));
+  hipLaunchKernelGGL(vec ? gated_norm_add_f32_kernel<4> : gated_norm_add_f32_kernel<1>, dim3(rows), dim3(256), 0, S(stream), res, ldr, y,
+                     ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, width);
   return check_launch();
 }
 
