@@ -20,6 +20,8 @@
 // does (:104-115); the bf16 partial outputs of mi_moe_down are summed over the ranks before mi_moe_combine.
 #include "mi_common.hpp"
 
+#include <algorithm>
+
 namespace mi {
 
 // ---------------------------------------------------------------------------------------------------
@@ -101,32 +103,64 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const uint16_t* __restri
 }
 
 // ---------------------------------------------------------------------------------------------------
-// grouping: one workgroup; pairs (t, slot) -> position in the expert-sorted list
+// grouping: pairs (t, slot) -> position in the expert-sorted list
 // ---------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ topk_ids, int n_pairs, int top_k, int E,
+// Workgroup b places the pairs [b * chunk, (b + 1) * chunk).  Each counts ALL pairs by itself (the list is at most a few hundred KiB of
+// L2; no workgroup waits for another): how many of an expert lie in front of its chunk and how many there are, a scan over the
+// experts, then a cursor per expert for its own pairs.  What bounds one workgroup is the scattered stores, 64 lines per request: 65536
+// pairs of 64 experts 62 us from one CU, 19 from 32 (2048 pairs each); 16384 pairs 17 / 8, 1024 pairs 6.9 / 6.4.
+constexpr int kSortLoads = 4;   // pairs of a thread that are asked for together, in fours
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ topk_ids, int n_pairs, int top_k, int E, int chunk,
                                                         int32_t* __restrict__ offsets, int32_t* __restrict__ pair_token,
                                                         int32_t* __restrict__ pair_index) {
-  __shared__ int cnt[513], cursor[512];
-  for (int e = threadIdx.x; e <= E; e += blockDim.x) cnt[e] = 0;
+  __shared__ int before[512], total[512], wave_sums[8];   // (E <= 512)
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lo = blockIdx.x * chunk, hi = min(lo + chunk, n_pairs);
+  if (tid < 512) before[tid] = total[tid] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) atomicAdd(&cnt[topk_ids[i]], 1);
+  // (lo is a multiple of four: a piece of four lies on one side of it)
+  for (int i0 = 4 * tid; i0 < n_pairs; i0 += kSortLoads * 4096) {
+    int id[kSortLoads][4];
+#pragma unroll
+    for (int u = 0; u < kSortLoads; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = i0 + u * 4096 + e;
+        id[u][e] = i < n_pairs ? topk_ids[i] : -1;
+      }
+#pragma unroll
+    for (int u = 0; u < kSortLoads; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i0 + u * 4096 + e < n_pairs) atomicAdd(i0 + u * 4096 < lo ? &before[id[u][e]] : &total[id[u][e]], 1);
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {  // exclusive scan (E <= 512)
-    int run = 0;
-    for (int e = 0; e < E; ++e) {
-      const int c = cnt[e];
-      offsets[e] = run;
-      cursor[e] = run;
-      run += c;
+  // exclusive scan of before + total over the experts, a thread each
+  int mine = 0, run = 0;
+  if (tid < 512) {
+    mine = run = before[tid] + total[tid];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(run, off);
+      if (lane >= off) run += o;
     }
-    offsets[E] = run;
+    if (lane == 63) wave_sums[wave] = run;
+  }
+  __syncthreads();
+  if (tid < 512) {
+    for (int w = 0; w < wave; ++w) run += wave_sums[w];
+    before[tid] += run - mine;   // this chunk's cursor
+    if (blockIdx.x == 0) {
+      if (tid < E) offsets[tid] = run - mine;
+      if (tid == E - 1) offsets[E] = run;
+    }
   }
   __syncthreads();
   // which slot inside an expert's run a pair gets is irrelevant to every result (the pairs of a run are
   // independent MFMA columns, and results are written back by pair index), so the order the atomics happen
   // to produce - different from rank to rank and run to run - is fine
-  for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
-    const int pos = atomicAdd(&cursor[topk_ids[i]], 1);
+  for (int i = lo + tid; i < hi; i += 1024) {
+    const int pos = atomicAdd(&before[topk_ids[i]], 1);
     pair_token[pos] = i / top_k;
     pair_index[pos] = i;
   }
@@ -329,7 +363,9 @@ extern "C" int mi_moe_sort(const int32_t* topk_ids, int n_tokens, int top_k, int
                            int32_t* pair_token, int32_t* pair_index, mi_stream stream) {
   if (!topk_ids || !expert_offsets || !pair_token || !pair_index || n_tokens < 0) return MI_EINVAL;
   if (n_experts < 1 || n_experts > 512 || top_k < 1) return MI_EUNSUPPORTED;
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, S(stream), topk_ids, n_tokens * top_k, top_k, n_experts,
+  const int n_pairs = n_tokens * top_k, wgs = std::max(1, std::min(32, n_pairs / 2048));
+  const int chunk = ((n_pairs + wgs - 1) / wgs + 3) & ~3;
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(wgs), dim3(1024), 0, S(stream), topk_ids, n_pairs, top_k, n_experts, chunk,
                      expert_offsets, pair_token, pair_index);
   return check_launch();
 }
