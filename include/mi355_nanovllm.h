@@ -324,6 +324,9 @@ int64_t mi_gemm_bf16_max_rows(int N, int K, int64_t ldx);
 size_t mi_gemm_bf16_workspace(int M, int N, int K, int epilogue);
 int mi_gemm_bf16(const mi_bf16* x, int64_t ldx, const mi_bf16* w, const mi_bf16* bias, mi_bf16* y, int64_t ldy,
                  int M, int N, int K, int epilogue, void* workspace, size_t ws_bytes, mi_stream stream);
+/* fp32 sums [ksplit][M][N] of K slices of x w^T (mi_gemm_bf16's operands; K % (64 ksplit) == 0), for mi_add_rmsnorm_splitk. */
+int mi_gemm_bf16_splitk(const mi_bf16* x, int64_t ldx, const mi_bf16* w, float* partials, int M, int N, int K, int ksplit,
+                        mi_stream stream);
 /* The packed qkv projection of a prefill step with the K / V side of qwen3.py:79-90 + attention.py:55-58 in its
  * epilogue (round 4): qkv[M][N] = x @ w^T (+ bias) as mi_gemm_bf16, but only the q heads (columns
  * [0, n_q_heads * 128)) are written to `qkv`; every k head is k-normed (k_w, or NULL: none), rotated (positions,
@@ -524,6 +527,11 @@ int mi_pick_final_pairs(const void* candidates, int n_groups, int rows, void* pa
 int mi_gemm_fp8w_packed_pick(const mi_bf16* x, const uint8_t* w_packed, const float* scale,
                              mi_bf16* y, int M, int N, int K, const float* temperatures,
                              const uint64_t* rng, void* candidates, mi_stream stream);
+/* The candidates of mi_gemm_bf16_packed_pick_shard from bf16 logits [M][N] that are already in memory (N % 8 == 0): candidates
+ * [M][mi_logits_pick_groups(N)] of 8 bytes, for mi_pick_final / mi_pick_final_pairs. */
+int mi_logits_pick_groups(int N);
+int mi_logits_pick(const mi_bf16* logits, int M, int N, const float* temperatures, const uint64_t* rng, void* candidates,
+                   int col_offset, mi_stream stream);
 int mi_pick_final(const void* candidates, int n_groups, int rows, int64_t* out,
                   mi_stream stream);
 

@@ -12,31 +12,43 @@
 // Same summation order and epilogues as the large kernel: results are bit-identical.
 // SwiGLU: the tile's 128 weight rows are, per wave, 32 gate rows (fragment 0) and the 32 up rows that pair with them.
 // ---------------------------------------------------------------------------
-constexpr int MID_STAGE = 2 * HALF_BYTES;  // (MID_F, MID_T and the index arithmetic: gemm_tile_index.hpp)
+// Other shapes (MidShape): fewer features or tokens per tile where 128 x 128 tiles leave CUs without work or are filled with repeated
+// rows - the ring then holds more of the shorter K steps, and about as many bytes are on their way.
+template <int N, int PER_STEP>
+__device__ __forceinline__ void mid_wait(int behind) {  // all but the pieces of the `behind` (<= N) newest K steps have landed
+  if constexpr (N == 0) {
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  } else {
+    if (behind >= N) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N * PER_STEP) : "memory");
+    else mid_wait<N - 1, PER_STEP>(behind);
+  }
+}
 
-template <int EPI, bool BIAS, int NST, class ARGS = TileArgs>
-__global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const ARGS a) {
-  __shared__ __attribute__((aligned(1024))) char lds[NST * MID_STAGE];
+template <int EPI, bool BIAS, int NST, class ARGS = TileArgs, class SH = Mid128>
+__global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void gemm_mid_kernel(const ARGS a) {
+  constexpr int WF = SH::WF, WT = SH::WT;
+  static_assert(WF == 2 || (EPI != TEPI_SILU && !ARGS::kDual), "a wave holds the gate and the up fragment of its outputs");
+  __shared__ __attribute__((aligned(1024))) char lds[NST * SH::STAGE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int fw = wave >> 1, tw = wave & 1, hi = lane >> 5, l31 = lane & 31;
+  const int fw = wave / SH::TW, tw = wave % SH::TW, hi = lane >> 5, l31 = lane & 31;
   const int KT_all = a.K / BK;
   const int KT = EPI == TEPI_PARTIAL ? KT_all / (int)gridDim.y : KT_all;
   const int64_t kbeg_bytes = EPI == TEPI_PARTIAL ? (int64_t)blockIdx.y * KT * (BK * 2) : 0;
-  int n0 = ((int)blockIdx.x % a.tiles_f) * MID_F, m0 = ((int)blockIdx.x / a.tiles_f) * MID_T, m_end = a.M;
+  int n0 = ((int)blockIdx.x % a.tiles_f) * SH::F, m0 = ((int)blockIdx.x / a.tiles_f) * SH::T, m_end = a.M;
   int64_t wrow0 = 0;
   if constexpr (EPI == TEPI_ANY) {
     if ((int)blockIdx.x >= any_tiles(a)) return;  // (the grid is the host's bound on the grouped tiles)
-    const AnyTile t = any_tile(a, (int)blockIdx.x, MID_T, ARGS::kDual ? MID_F / 2 : MID_F);
+    const AnyTile t = any_tile(a, (int)blockIdx.x, SH::T, ARGS::kDual ? SH::F / 2 : SH::F);
     n0 = t.n0, m0 = t.m0, m_end = t.m_end, wrow0 = (int64_t)t.group * a.N;
   }
 
-  // LDS-DMA: wave w moves the 1 KiB blocks 4 w .. 4 w + 3 (8 local rows each) of both half-tiles
-  const char* srcA[4];
-  const char* srcB[4];
+  // LDS-DMA: wave w moves its share of the 1 KiB pieces (8 local rows each) of the feature rows and of the token rows
+  const char* srcA[SH::A_PIECES];
+  const char* srcB[SH::B_PIECES];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int lr = mid_dma_local_row(wave, i, lane), c = mid_dma_chunk(wave, i, lane);
+  for (int i = 0; i < SH::A_PIECES; ++i) {
+    const int lr = (wave * SH::A_PIECES + i) * 8 + (lane >> 3), c = (lane & 7) ^ swizzle(lr);
     if constexpr (EPI == TEPI_ANY) {
       // two weights: every wave's first fragment holds 32 rows of w, its second the rows of w2 that pair with them
       const bool second = ARGS::kDual && ((lr >> 5) & 1);
@@ -46,16 +58,22 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const A
       const int rowA = mid_weight_row(lr, n0, a.N, EPI == TEPI_SILU);
       srcA[i] = reinterpret_cast<const char*>(a.w) + kbeg_bytes + ((int64_t)min(rowA, a.N - 1) * a.K + c * 8) * 2;
     }
+  }
+#pragma unroll
+  for (int i = 0; i < SH::B_PIECES; ++i) {
+    const int lr = (wave * SH::B_PIECES + i) * 8 + (lane >> 3), c = (lane & 7) ^ swizzle(lr);
     srcB[i] = reinterpret_cast<const char*>(a.x) + kbeg_bytes + ((int64_t)min(m0 + lr, m_end - 1) * a.ldx + c * 8) * 2;
   }
   auto issue = [&](int kt, int p) __attribute__((always_inline)) {
-    char* dst = lds + p * MID_STAGE + wave * 4096;
+    char* dst = lds + p * SH::STAGE;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcA[i] + (int64_t)kt * (BK * 2)),
-                                       (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcB[i] + (int64_t)kt * (BK * 2)),
-                                       (__attribute__((address_space(3))) void*)(dst + HALF_BYTES + i * 1024), 16, 0, 0);
+    for (int i = 0; i < (SH::A_PIECES > SH::B_PIECES ? SH::A_PIECES : SH::B_PIECES); ++i) {
+      if (i < SH::A_PIECES)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcA[i < SH::A_PIECES ? i : 0] + (int64_t)kt * (BK * 2)),
+                                         (__attribute__((address_space(3))) void*)(dst + (wave * SH::A_PIECES + i) * 1024), 16, 0, 0);
+      if (i < SH::B_PIECES)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcB[i < SH::B_PIECES ? i : 0] + (int64_t)kt * (BK * 2)),
+                                         (__attribute__((address_space(3))) void*)(dst + SH::F * 128 + (wave * SH::B_PIECES + i) * 1024), 16, 0, 0);
     }
   };
   int kx[4];
@@ -63,11 +81,11 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const A
   for (int kk = 0; kk < 4; ++kk)
     kx[kk] = (l31 >> 3) * 1024 + (l31 & 7) * 128 + ((frag_chunk(kk, hi) ^ swizzle(l31)) << 4);
 
-  f32x16 acc[2][2];
+  f32x16 acc[WF][WT];
 #pragma unroll
-  for (int f = 0; f < 2; ++f)
+  for (int f = 0; f < WF; ++f)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < WT; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[f][b][r] = 0.f;
 
@@ -76,49 +94,46 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const A
     if (s < KT) issue(s, s);
   int p = 0, pn = NST - 1;  // ring slots of step kt and of step kt + NST - 1
   for (int kt = 0; kt < KT; ++kt) {
-    // requested so far: steps <= kt + NST - 2; eight pieces per step and wave, completing in order
-    const int behind = min(KT - 1 - kt, NST - 2);
-    if (behind >= 2) asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
-    else if (behind == 1) asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    // requested so far: steps <= kt + NST - 2; the same number of pieces per step and wave, completing in order
+    mid_wait<NST - 2, SH::A_PIECES + SH::B_PIECES>(min(KT - 1 - kt, NST - 2));
     __builtin_amdgcn_sched_barrier(0);
     if (kt + NST - 1 < KT) issue(kt + NST - 1, pn);
-    const char* sa = lds + p * MID_STAGE + fw * 8192;
-    const char* sb = lds + p * MID_STAGE + HALF_BYTES + tw * 8192;
-    u32x4 A[2][4], B[2][4];
+    const char* sa = lds + p * SH::STAGE + fw * WF * 4096;
+    const char* sb = lds + p * SH::STAGE + SH::F * 128 + tw * WT * 4096;
+    u32x4 A[WF][4], B[WT][4];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
-      for (int f = 0; f < 2; ++f) A[f][kk] = *reinterpret_cast<const u32x4*>(sa + f * 4096 + kx[kk]);
+      for (int f = 0; f < WF; ++f) A[f][kk] = *reinterpret_cast<const u32x4*>(sa + f * 4096 + kx[kk]);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) B[b][kk] = *reinterpret_cast<const u32x4*>(sb + b * 4096 + kx[kk]);
+      for (int b = 0; b < WT; ++b) B[b][kk] = *reinterpret_cast<const u32x4*>(sb + b * 4096 + kx[kk]);
     }
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < WF; ++f)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < WT; ++b)
           acc[f][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(A[f][kk]), as_frag(B[b][kk]), acc[f][b], 0, 0, 0);
     p = p + 1 == NST ? 0 : p + 1;
     pn = pn + 1 == NST ? 0 : pn + 1;
   }
 
-  // epilogue: lane (hi, l31) holds token tw * 64 + b * 32 + l31, features 8 rq + 4 hi + {0..3} of each 32-row fragment
+  // epilogue: lane (hi, l31) holds token (tw WT + b) 32 + l31, features 8 rq + 4 hi + {0..3} of each 32-row fragment
   if constexpr (EPI == TEPI_ANY) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const AnyRow row = any_row(a, m0 + tw * 64 + b * 32 + l31, m_end);
+    for (int b = 0; b < WT; ++b) {
+      const AnyRow row = any_row(a, m0 + (tw * WT + b) * 32 + l31, m_end);
 #pragma unroll
-      for (int f = 0; f < (ARGS::kDual ? 1 : 2); ++f)
+      for (int f = 0; f < (ARGS::kDual ? 1 : WF); ++f)
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) {
-          const int col = n0 + (ARGS::kDual ? fw * 32 : fw * 64 + f * 32) + 8 * rq + 4 * hi;
+          const int col = n0 + (ARGS::kDual ? fw : fw * WF + f) * 32 + 8 * rq + 4 * hi;
           f32x4 v, v2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             v[e] = acc[f][b][4 * rq + e];
-            if (ARGS::kDual) v2[e] = acc[1][b][4 * rq + e];
+            if (ARGS::kDual) v2[e] = acc[WF - 1][b][4 * rq + e];
           }
           any_store(a, row, col, v, v2);
         }
@@ -128,16 +143,16 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const A
   const int n_out = EPI == TEPI_SILU ? a.N >> 1 : a.N;
   const bool wide = n_out % 8 == 0 && a.ldy % 8 == 0;
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int tok = m0 + tw * 64 + b * 32 + l31;
+  for (int b = 0; b < WT; ++b) {
+    const int tok = m0 + (tw * WT + b) * 32 + l31;
     const bool tok_ok = tok < a.M;
     if (EPI == TEPI_PARTIAL) {
       float* prow = a.part + ((int64_t)blockIdx.y * a.M + min(tok, a.M - 1)) * a.N;
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < WF; ++f)
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) {
-          const int col = n0 + fw * 64 + f * 32 + 8 * rq + 4 * hi;
+          const int col = n0 + (fw * WF + f) * 32 + 8 * rq + 4 * hi;
           if (tok_ok && col < a.N)
             *reinterpret_cast<f32x4*>(prow + col) =
                 f32x4{acc[f][b][4 * rq], acc[f][b][4 * rq + 1], acc[f][b][4 * rq + 2], acc[f][b][4 * rq + 3]};
@@ -146,8 +161,8 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const A
     }
     uint16_t* yrow = a.y + (int64_t)min(tok, a.M - 1) * a.ldy;
 #pragma unroll
-    for (int f = 0; f < (EPI == TEPI_SILU ? 1 : 2); ++f) {
-      const int col0 = EPI == TEPI_SILU ? (n0 >> 1) + fw * 32 : n0 + fw * 64 + f * 32;
+    for (int f = 0; f < (EPI == TEPI_SILU ? 1 : WF); ++f) {
+      const int col0 = EPI == TEPI_SILU ? (n0 >> 1) + fw * 32 : n0 + (fw * WF + f) * 32;
       u32x2 pk[4];
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
@@ -158,7 +173,7 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void gemm_mid_kernel(const A
           for (int e = 0; e < 4; ++e) {  // the roundings and the silu form of the large kernel's epilogue
             const float gb = rbf(acc[0][b][4 * rq + e]);
             const float sb = rbf(gb * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gb * -1.4426950408889634f)));
-            o[e] = sb * rbf(acc[1][b][4 * rq + e]);
+            o[e] = sb * rbf(acc[WF - 1][b][4 * rq + e]);
           }
         } else {
 #pragma unroll

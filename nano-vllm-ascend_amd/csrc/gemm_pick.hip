@@ -57,9 +57,64 @@ __global__ __launch_bounds__(1024) void pick_final_kernel(const uint2* __restric
   }
 }
 
+// The same candidates from logits that are already in memory (more than 64 rows: the head product is a tile GEMM then): grid
+// (pieces of kScanCols columns, rows), keys and ties as EPI_PICK forms them.
+constexpr int kScanCols = 8192;
+__global__ __launch_bounds__(256) void pick_scan_kernel(const uint16_t* __restrict__ logits, int N, PickArgs pk) {
+  const int row = blockIdx.y, c0 = blockIdx.x * kScanCols;
+  const uint16_t* p = logits + (int64_t)row * N;
+  const float tmp = pk.temperatures ? pk.temperatures[row] : 0.f;
+  const bool noisy = tmp > 0.f;
+  const float inv_t = noisy ? 1.0f / tmp : 1.0f;
+  const uint64_t rkey = sample_row_key(pk.rng[0], pk.rng[1], row);
+  u32x4 v[kScanCols / 2048];
+#pragma unroll
+  for (int i = 0; i < kScanCols / 2048; ++i)   // (past the end: the last piece again, not looked at)
+    v[i] = *reinterpret_cast<const u32x4*>(p + min(c0 + 2048 * i + 8 * (int)threadIdx.x, N - 8));
+  float best = -INFINITY;
+  int best_c = 0x7fffffff;
+#pragma unroll
+  for (int i = 0; i < kScanCols / 2048; ++i) {
+    const int c = c0 + 2048 * i + 8 * (int)threadIdx.x;
+    if (c >= N) break;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float l = e & 1 ? hi_bf(v[i][e >> 1]) : lo_bf(v[i][e >> 1]);
+      const float key = noisy ? gumbel_key(l, inv_t, rkey, pk.col0 + c + e) : l;
+      if (key > best) best = key, best_c = pk.col0 + c + e;   // (ascending columns: the first of equal keys stays)
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float ob = __shfl_xor(best, o, 64);
+    const int oc = __shfl_xor(best_c, o, 64);
+    if (ob > best || (ob == best && oc < best_c)) best = ob, best_c = oc;
+  }
+  __shared__ float sb[4];
+  __shared__ int sc[4];
+  if ((threadIdx.x & 63) == 0) sb[threadIdx.x >> 6] = best, sc[threadIdx.x >> 6] = best_c;
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int w = 1; w < 4; ++w)
+    if (sb[w] > best || (sb[w] == best && sc[w] < best_c)) best = sb[w], best_c = sc[w];
+  pk.cand[(int64_t)row * gridDim.x + blockIdx.x] = uint2{__float_as_uint(best), (uint32_t)best_c};
+}
+
 }  // namespace mi
 
 using namespace mi;
+
+extern "C" int mi_logits_pick_groups(int N) { return N <= 0 || N % 8 ? 0 : (N + kScanCols - 1) / kScanCols; }
+
+extern "C" int mi_logits_pick(const mi_bf16* logits, int M, int N, const float* temperatures, const uint64_t* rng, void* candidates,
+                              int col_offset, mi_stream stream) {
+  if (!logits || !rng || !candidates || M < 0 || N <= 0 || col_offset < 0 || !aligned16(logits)) return MI_EINVAL;
+  if (N % 8 || M > 65535) return MI_EUNSUPPORTED;
+  if (M == 0) return MI_OK;
+  hipLaunchKernelGGL(pick_scan_kernel, dim3(mi_logits_pick_groups(N), M), dim3(256), 0, S(stream), logits, N,
+                     PickArgs{temperatures, rng, static_cast<uint2*>(candidates), col_offset});
+  return check_launch();
+}
 
 // head GEMM with the pick epilogue: the same workgroup geometry as mi_gemm_bf16_packed for this (M, N)
 extern "C" int mi_gemm_pick_groups(int M, int N, int K, int fp8_weights) {

@@ -487,50 +487,71 @@ static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
 // The 128-tile kernel takes the shapes whose 256-tiles are too few for the chip; both kernels give the same bits,
 // the choice is a matter of time only.  Modelled time of a launch: rounds of workgroups x K steps x time per step
 // (measured: tools/gemm_bench.py), plus - with K slices - the fp32 partial sums out and back and the second launch.
-constexpr double kMidStepUs = 0.5, kMidPairStepUs = 0.62, kLaunchUs = 3.8, kPartialBytesPerUs = 4.0e6;
+// gemm_mid_kernel's shapes (features x tokens): its time per K step with one workgroup on a CU (what the ring's requests take), and for
+// two sharing it.  us, one launch: 200 rows x 4096 features x 1024 with 128 x 128 / 64 x 128 / 64 x 64 tiles 12.5 / 9.3 / 7.1
+// (64 / 128 / 256 workgroups; the weight-streaming kernel 18.6), 400 rows 12.5 / 9.3 / 9.6; 200 x 5120 x 2048 21.2 / 15.8 / 14.5;
+// SwiGLU of 6144 rows x 1024 at 200 tokens 12.7 / 9.4, at 400 12.9 / 12.5; 1024 rows of 6144 x 1024 stay with 128 x 128 (22).
+using Mid64x128 = MidShape<1, 4, 2, 1>;   // (a wave holds a gate and an up fragment: SwiGLU too)
+using Mid64 = MidShape<2, 2, 1, 1>;
+struct MidTile {
+  int f, t;
+  double step_us, pair_us;
+};
+constexpr MidTile kMidTiles[3] = {{128, 128, 0.52, 0.62}, {64, 128, 0.36, 0.50}, {64, 64, 0.22, 0.35}};
+constexpr double kLaunchUs = 3.8, kPartialBytesPerUs = 4.0e6;
 
 // fewer 256-tiles than CUs: the 128-tile kernel
 static bool use_mid(int M, int N, int K) {
   return (int64_t)((M + TILE_T - 1) / TILE_T) * ((N + TILE_F - 1) / TILE_F) < kPersistentGrid;
 }
 
-static int mid_ksplit(int M, int N, int K) {
-  const int tiles = ((M + MID_T - 1) / MID_T) * ((N + MID_F - 1) / MID_F), kt = K / BK;
+struct MidPick {
+  int tile, ksplit;
+};
+// fixed_ks: the caller wants that many slices' sums; 0: whatever is fastest, the sum of the slices included
+static MidPick pick_mid(int M, int N, int K, bool silu, int fixed_ks = 0) {
+  const int kt = K / BK;
   double best = 1e30;
-  int best_ks = 1;
-  for (int ks = 1; ks <= 16; ks *= 2) {
-    if (kt % ks || (ks > 1 && kt / ks < 2)) break;
-    // one workgroup on a CU takes ~0.5 us per K step (DMA issue and MFMAs of a wave do not overlap), two sharing
-    // it ~0.62 us for both
-    const int per_cu = (tiles * ks + kPersistentGrid - 1) / kPersistentGrid;
-    double t = (per_cu == 1 ? kMidStepUs : (per_cu + 1) / 2 * kMidPairStepUs) * (kt / ks) + kLaunchUs;
-    if (ks > 1) t += 2.0 * ks * (double)M * N * sizeof(float) / kPartialBytesPerUs + kLaunchUs;
-    if (t < best) {
-      best = t;
-      best_ks = ks;
+  MidPick pick{0, 1};
+  for (int i = 0; i < (silu ? 2 : 3); ++i) {
+    const MidTile& s = kMidTiles[i];
+    const int64_t tiles = (int64_t)((M + s.t - 1) / s.t) * ((N + s.f - 1) / s.f);
+    for (int ks = fixed_ks ? fixed_ks : 1; ks <= (fixed_ks ? fixed_ks : silu ? 1 : 16); ks *= 2) {
+      if (!fixed_ks && (kt % ks || (ks > 1 && kt / ks < 2))) break;
+      const int64_t per_cu = (tiles * ks + kPersistentGrid - 1) / kPersistentGrid;
+      double t = (per_cu == 1 ? s.step_us : (per_cu + 1) / 2 * s.pair_us) * (kt / ks) + kLaunchUs;
+      if (!fixed_ks && ks > 1) t += 2.0 * ks * (double)M * N * sizeof(float) / kPartialBytesPerUs + kLaunchUs;
+      if (t < best) best = t, pick = MidPick{i, ks};
     }
   }
-  return best_ks;
+  return pick;
 }
 
-// NST = 0: by workgroup count - at most one workgroup per CU: the deep ring (nothing else hides the DMA round trip);
-// more: the two-stage ring, two workgroups per CU (measured, tools/gemm_bench.py GEMM_MID=1: 22 vs 27 us on
-// 1024 x 6144 x 1024, 31 vs 34 the other way round on 1024 x 1024 x 3072)
+// NST = 0: by shape and workgroup count.  128 x 128: at most one workgroup per CU - the deep ring (nothing else hides the DMA round
+// trip); more: the two-stage ring, two workgroups per CU (22 vs 27 us on 1024 x 6144 x 1024, 31 vs 34 the other way round on
+// 1024 x 1024 x 3072).  The smaller shapes: rings of which two fit a CU (64 x 64, five stages: 7.1 us above, nine 7.7).
 template <int EPI, bool BIAS, int NST = 0>
-static int launch_mid(TileArgs a, hipStream_t st, int ksplit = 1) {
-  a.tiles_f = (a.N + MID_F - 1) / MID_F;
-  a.tiles_t = (a.M + MID_T - 1) / MID_T;
-  const dim3 grid(a.tiles_f * a.tiles_t, ksplit);
-  if (NST == 0) {
-    if ((int64_t)grid.x * grid.y > kPersistentGrid) hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 2>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 4>), grid, dim3(256), 0, st, a);
+static int launch_mid(TileArgs a, hipStream_t st, MidPick pick = {0, 1}) {
+  const MidTile& s = kMidTiles[pick.tile];
+  a.tiles_f = (a.N + s.f - 1) / s.f;
+  a.tiles_t = (a.M + s.t - 1) / s.t;
+  const dim3 grid(a.tiles_f * a.tiles_t, pick.ksplit);
+  if constexpr (NST != 0) {
+    hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, NST>), grid, dim3(256), 0, st, a);
   } else {
-    hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, (NST ? NST : 2)>), grid, dim3(256), 0, st, a);
+    if constexpr (EPI != TEPI_SILU)
+      if (pick.tile == 2) {
+        hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 5, TileArgs, Mid64>), grid, dim3(256), 0, st, a);
+        return check_launch();
+      }
+    if (pick.tile == 1) hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 3, TileArgs, Mid64x128>), grid, dim3(256), 0, st, a);
+    else if ((int64_t)grid.x * grid.y > kPersistentGrid) hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 2>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 4>), grid, dim3(256), 0, st, a);
   }
   return check_launch();
 }
 
-static int gemm_ksplit(int M, int N, int K) { return use_mid(M, N, K) ? mid_ksplit(M, N, K) : tile_ksplit(M, N, K); }
+static int gemm_ksplit(int M, int N, int K) { return use_mid(M, N, K) ? pick_mid(M, N, K, false).ksplit : tile_ksplit(M, N, K); }
 
 static int check_tile_gemm(const void* x, int64_t ldx, const void* w, const void* bias, const void* y, int64_t ldy,
                            int M, int N, int K, int epilogue) {
@@ -573,20 +594,33 @@ extern "C" int mi_gemm_bf16(const mi_bf16* x, int64_t ldx, const mi_bf16* w, con
   TileArgs a{x, w, bias, y, ldx, ldy, M, N, K, (N + TILE_F - 1) / TILE_F, (M + TILE_T - 1) / TILE_T, nullptr};
   hipStream_t st = S(stream);
   const bool mid = use_mid(M, N, K);
-  if (epilogue == 1) return mid ? launch_mid<TEPI_SILU, false>(a, st) : launch_tile<TEPI_SILU, false>(a, st);
-  const int ks = gemm_ksplit(M, N, K);
+  const MidPick pick = mid ? pick_mid(M, N, K, epilogue == 1) : MidPick{0, 1};
+  if (epilogue == 1) return mid ? launch_mid<TEPI_SILU, false>(a, st, pick) : launch_tile<TEPI_SILU, false>(a, st);
+  const int ks = mid ? pick.ksplit : tile_ksplit(M, N, K);
   if (ks > 1) {  // two launches: K slices as fp32 partial sums, then their sum (+ bias) rounded once
     if (!workspace || !aligned16(workspace) || ws_bytes < mi_gemm_bf16_workspace(M, N, K, 0)) return MI_EWORKSPACE;
     a.part = static_cast<float*>(workspace);
-    const int rc2 = mid ? launch_mid<TEPI_PARTIAL, false>(a, st, ks) : launch_tile<TEPI_PARTIAL, false>(a, st, ks);
+    const int rc2 = mid ? launch_mid<TEPI_PARTIAL, false>(a, st, pick) : launch_tile<TEPI_PARTIAL, false>(a, st, ks);
     if (rc2 != MI_OK) return rc2;
     const int64_t quads = (int64_t)M * (N / 4);
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a.part, ks, bias, y,
                        ldy, M, N);
     return check_launch();
   }
-  if (mid) return bias ? launch_mid<TEPI_NONE, true>(a, st) : launch_mid<TEPI_NONE, false>(a, st);
+  if (mid) return bias ? launch_mid<TEPI_NONE, true>(a, st, pick) : launch_mid<TEPI_NONE, false>(a, st, pick);
   return bias ? launch_tile<TEPI_NONE, true>(a, st) : launch_tile<TEPI_NONE, false>(a, st);
+}
+
+// fp32 sums of `ksplit` K slices [ksplit][M][N] (mi_gemm_bf16_packed_splitk's result for the weight as stored), for the norm that adds
+// them up
+extern "C" int mi_gemm_bf16_splitk(const mi_bf16* x, int64_t ldx, const mi_bf16* w, float* partials, int M, int N, int K, int ksplit,
+                                   mi_stream stream) {
+  const int rc = check_tile_gemm(x, ldx, w, nullptr, partials, N, M, N, K, 0);
+  if (rc != MI_OK) return rc;
+  if (ksplit < 1 || ksplit > 65535 || K % ((int64_t)BK * ksplit)) return MI_EUNSUPPORTED;
+  if (M == 0) return MI_OK;
+  TileArgs a{x, w, nullptr, nullptr, ldx, N, M, N, K, 0, 0, partials};
+  return launch_mid<TEPI_PARTIAL, false>(a, S(stream), pick_mid(M, N, K, false, ksplit));
 }
 
 // The packed qkv projection with the K / V heads stored straight into the paged cache (TEPI_QKV, gemm_w4_kernel.hpp)

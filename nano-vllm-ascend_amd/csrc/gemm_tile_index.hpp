@@ -86,6 +86,17 @@ MI_HD constexpr int mid_b_local_row(int tw, int b, int l31) { return tw * 64 + b
 MI_HD constexpr int mid_acc_feature(int fw, int f, int r, int hi) { return fw * 64 + f * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi; }
 MI_HD constexpr int mid_acc_token(int tw, int b, int l31) { return tw * 64 + b * 32 + l31; }
 
+// A tile shape of gemm_mid_kernel: FW x TW waves of WF x WT accumulators of 32 x 32; a K step in LDS = the tile's feature rows, then its
+// token rows, 128 bytes each, in 1 KiB pieces of eight rows that the waves move in equal shares.
+template <int FW_, int TW_, int WF_, int WT_>
+struct MidShape {
+  static constexpr int FW = FW_, TW = TW_, WF = WF_, WT = WT_, NW = FW * TW, F = 32 * FW * WF, T = 32 * TW * WT;
+  static constexpr int A_PIECES = F / 8 / NW, B_PIECES = T / 8 / NW;  // per wave and K step
+  static constexpr int STAGE = (F + T) * 128;
+};
+using Mid128 = MidShape<2, 2, 2, 2>;
+static_assert(Mid128::F == MID_F && Mid128::T == MID_T, "the 128 x 128 tile");
+
 // ---- the four-wave 256 x 256 x 64 kernel (gemm_w4_kernel, the product kernel for large M since round 4) ----
 // One wave per SIMD: fw = wave >> 1 (128 features), tw = wave & 1 (128 tokens), wave tile 128 x 128 = 4 x 4 accumulators.
 // One K step of the tile in LDS is ONE image of 64 PIECES: a piece is what one `buffer_load_dwordx4 ... lds` wave

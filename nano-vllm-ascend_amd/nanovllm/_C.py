@@ -144,6 +144,9 @@ _SIGNATURES = {
     "mi_gemm_pick_groups": (c_int, [c_int, c_int, c_int, c_int]),
     "mi_gemm_bf16_packed_pick": (c_int, [_p, _p, _p, c_int, c_int, c_int, _p, _p, _p, _p]),
     "mi_gemm_fp8w_packed_pick": (c_int, [_p, _p, _p, _p, c_int, c_int, c_int, _p, _p, _p, _p]),
+    "mi_logits_pick_groups": (c_int, [c_int]),
+    "mi_logits_pick": (c_int, [_p, c_int, c_int, _p, _p, _p, c_int, _p]),
+    "mi_gemm_bf16_splitk": (c_int, [_p, c_int64, _p, _p, c_int, c_int, c_int, c_int, _p]),
     "mi_pick_final": (c_int, [_p, c_int, c_int, _p, _p]),
     "mi_gemm_bf16_packed_pick_shard": (c_int, [_p, _p, _p, c_int, c_int, c_int, _p, _p, _p, c_int, _p]),
     "mi_pick_final_pairs": (c_int, [_p, c_int, c_int, _p, _p]),

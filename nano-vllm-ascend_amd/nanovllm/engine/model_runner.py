@@ -698,13 +698,14 @@ class ModelRunner(RowSteps):
             hidden = self.model(d["ids"][:tb], d["pos"][:tb])
             x = ops.gather_last_tokens(hidden, d["cu_q"][:sb + 1])
             if self.world_size == 1:
-                logits, _ = ops.gemm_packed_pick(x, head.weight_packed, d["temps"][:sb], d["rng"], self.tokens_dev[:sb])
+                logits, _ = ops.gemm_packed_pick(x, head.weight_packed, d["temps"][:sb], d["rng"], self.tokens_dev[:sb],
+                                                 w=head.weight)
                 return logits
             # tensor parallelism: every rank picks in its vocabulary shard, the ranks exchange {key, token} pairs over the
             # region and take the same winner (ParallelLMHead.local_logits_pick, the decode graphs' last launches)
             pairs = torch.empty((sb, 2), dtype=torch.int32, device=x.device)
             logits, _ = ops.gemm_packed_pick(x, head.weight_packed, d["temps"][:sb], d["rng"], self.tokens_dev[:sb],
-                                             col_offset=head.vocab_start_idx, pairs_out=pairs)
+                                             col_offset=head.vocab_start_idx, pairs_out=pairs, w=head.weight)
             self.xgmi.pick_exchange(pairs, self.tokens_dev[:sb])
             return logits
 

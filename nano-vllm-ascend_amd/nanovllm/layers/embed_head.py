@@ -74,12 +74,12 @@ class ParallelLMHead(VocabParallelEmbedding):
         on every rank's device, inside the captured graph."""
         assert not get_context().is_prefill and self.can_pick()
         if self.tp_size == 1:
-            logits, _ = ops.gemm_packed_pick(x, self.weight_packed, temperatures, rng, out_tokens)
+            logits, _ = ops.gemm_packed_pick(x, self.weight_packed, temperatures, rng, out_tokens, w=self.weight)
             return logits
         rows = x.shape[0]
         pairs = torch.empty((rows, 2), dtype=torch.int32, device=x.device)
         logits, _ = ops.gemm_packed_pick(x, self.weight_packed, temperatures, rng, out_tokens,
-                                         col_offset=self.vocab_start_idx, pairs_out=pairs)
+                                         col_offset=self.vocab_start_idx, pairs_out=pairs, w=self.weight)
         get_xgmi_comm().pick_exchange(pairs, out_tokens)
         return logits
 

@@ -227,13 +227,20 @@ class Qwen3Model(nn.Module):
         self.norm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     # prefill steps up to this many tokens take the seven-launch streaming path of the decode step, longer ones the
-    # module-by-module path on the tile GEMMs.  Measured on the captured prefill steps of a Qwen3-0.6B-shaped engine
-    # (profiles/r05_prefill_bucket_times.txt; ms per step with the switch at 512 / 128 tokens): 192 tokens 2.11 / 1.98,
-    # 256: 2.32 / 2.05, 384: 2.77 / 2.57, 512: 3.19 / 2.63; at 128 tokens the streaming path wins (1.73 vs 1.93).
-    PREFILL_STREAM_MAX = int(os.environ.get("MI355_PREFILL_STREAM_MAX", "128"))
+    # module-by-module path on the tile GEMMs.  Above 64 rows the dense bf16 projections of the streaming path are tile GEMMs too,
+    # the narrow ones in K slices that the norm adds up (ms per captured step of a Qwen3-0.6B-shaped model, streaming / module path:
+    # 130 tokens 1.51 / 1.66, 256: 1.65 / 1.83, 512: 2.20 / 2.40, 8 x 64: 1.94 / 2.15); fp8 weights, experts and ranks still read
+    # their weights once per 64 rows there and stay at 128 (192 tokens, before: 2.11 / 1.98).
+    PREFILL_STREAM_MAX = int(os.environ.get("MI355_PREFILL_STREAM_MAX", "512"))
+
+    def _prefill_stream_max(self) -> int:
+        l0 = self.layers[0]
+        tile = (tp_size() == 1 and not collectives_on() and not isinstance(l0.self_attn.qkv_proj.weight_packed, ops.Fp8Weight)
+                and not any(hasattr(l.mlp, "experts") for l in self.layers))
+        return min(ops.SKINNY_MAX_M, self.PREFILL_STREAM_MAX if tile else min(self.PREFILL_STREAM_MAX, 128))
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
-        limit = min(ops.SKINNY_MAX_M, self.PREFILL_STREAM_MAX) if get_context().is_prefill else ops.SKINNY_MAX_M
+        limit = self._prefill_stream_max() if get_context().is_prefill else ops.SKINNY_MAX_M
         if self.fused and input_ids.numel() <= limit and self._can_stream():
             return self._forward_streaming(input_ids, positions)
         hidden_states = self.embed_tokens(input_ids)
@@ -296,7 +303,8 @@ class Qwen3Model(nn.Module):
           add+RMSNorm (summing the previous projection's split-K partials)      (mi_add_rmsnorm_splitk)
           -> packed qkv GEMM                                                     (mi_gemm_bf16_packed)
           -> q/k-norm + RoPE + KV store + paged attention in one launch          (mi_paged_attn_decode_fused)
-          -> split-K o_proj -> add+RMSNorm -> gate_up GEMM + SwiGLU epilogue -> split-K down_proj.
+          -> split-K o_proj -> add+RMSNorm -> gate_up GEMM + SwiGLU epilogue -> split-K down_proj
+        (above 64 rows the bf16 projections are tile GEMMs on the weights as stored: ops.gemm_tile, ops.gemm_tile_splitk).
         MI355_ATTN_FUSED=0 keeps q/k-norm+RoPE+store as its own launch (mi_qknorm_rope_store).
         With tensor parallelism the two row-parallel projections produce bf16 partial sums as complete
         rows (mi_gemm_bf16_rows4); the all-reduce over the ranks (linear.py:149-153) and the following
@@ -337,7 +345,11 @@ class Qwen3Model(nn.Module):
             if rows4 and lin.weight_rows4 is not None:
                 y = ops.gemm_rows4(x, lin.weight_rows4)
             elif not exchange:
-                return ops.gemm_packed_splitk(x, lin.weight_packed, self._ksplit(lin.weight)), True
+                ks, k = self._ksplit(lin.weight), lin.weight.shape[1]
+                if (rows > ops.TILE_MIN_ROWS and k % (64 * ks) == 0 and not isinstance(lin.weight_packed, ops.Fp8Weight)
+                        and ops.tile_gemm_max_rows(*lin.weight.shape) >= rows):
+                    return ops.gemm_tile_splitk(x, lin.weight, ks), True
+                return ops.gemm_packed_splitk(x, lin.weight_packed, ks), True
             else:
                 y = ops.gemm_packed(x, lin.weight_packed)  # this rank's bf16 partial sums
             if exchange and not fused_seam:
@@ -354,8 +366,8 @@ class Qwen3Model(nn.Module):
             return ops.add_rmsnorm(y, res, ln.weight, ln.eps)
 
         def column_parallel(x, lin, silu_mul=False):
-            """qkv / gate_up (+ SwiGLU): the weight-streaming kernel, or - large batches, wide projections - the
-            128-tile MFMA kernel on the weight as stored (ops.prefers_tile)"""
+            """qkv / gate_up (+ SwiGLU): the weight-streaming kernel, or - more than 64 rows, wide projections - the
+            small-tile MFMA kernel on the weight as stored (ops.prefers_tile)"""
             w = lin.weight
             if (ops.prefers_tile(rows, w.shape[0]) and w.shape[1] % 64 == 0
                     and not isinstance(lin.weight_packed, ops.Fp8Weight)

@@ -411,16 +411,15 @@ def silu_mul(x, out=None) -> torch.Tensor:
 # rows the weight-streaming decode kernels take in one launch (chunks of 64 rows, csrc kSkinnyMaxRows); the decode
 # fast path of the models, the in-graph sampler and the engine's lookahead all go up to this many sequences
 SKINNY_MAX_M = 512
-# ... but above this many rows a WIDE projection (qkv, gate_up: thousands of output features = enough 128 x 128 tiles
-# for the chip) is faster on the MFMA tile kernel: 12.7 vs 15.1 us (qkv) and 13.1 vs 21.7 us (gate_up + SwiGLU) at 256
-# rows, 13.4 vs 28.0 and 14.3 vs 50.0 at 512; the narrow row-parallel projections (o_proj, down: N = hidden) stay on
-# the streaming kernels up to SKINNY_MAX_M rows (7.4 vs 13.2 us at 256) - tools/gemm_bench.py, GEMM_MID=1
-TILE_MIN_ROWS = 128
-TILE_MIN_FEATURES = 2048
+# ... but a WIDE projection (qkv, gate_up) goes to the MFMA tile kernels above 64 rows, where the streaming kernel begins to read the
+# rows' weights once per 64 (us: 4096 x 1024 at 72 rows 7.1 vs 10.5, at 200 7.1 vs 18.6; gate_up + SwiGLU of 6144 9.2 vs 11.5 and
+# 9.4 vs 17.1; 2048 x 2048 at 100 rows 10.2 vs 8.1, at 137 10.1 vs 14.0), the narrow ones above 256 (1024 x 2048 without K slices
+# at 256 rows 10.6 vs 7.6, at 400 10.7 vs 13.1; 1024 x 3072 14.7 vs 9.4 and 14.8 vs 16.5)
+TILE_MIN_ROWS = 64
 
 
 def prefers_tile(rows: int, n_features: int) -> bool:
-    return rows > SKINNY_MAX_M or (rows > TILE_MIN_ROWS and n_features >= TILE_MIN_FEATURES)
+    return rows > SKINNY_MAX_M // 2 or (rows > 2 * TILE_MIN_ROWS and n_features >= 2048) or (rows > TILE_MIN_ROWS and n_features >= 4096)
 
 
 def gemm_skinny(x, w, bias=None, out=None) -> torch.Tensor:
@@ -647,6 +646,20 @@ def gemm_packed_splitk(x, w_packed, ksplit: int, out=None) -> torch.Tensor:
     return out
 
 
+def gemm_tile_splitk(x, w, ksplit: int, out=None) -> torch.Tensor:
+    """fp32 partials [ksplit, M, N] of x @ w.T on the tile kernels (w as stored): gemm_packed_splitk above 64 rows (200 rows, four
+    slices: 1024 x 2048 6.7 vs 8.8 us, 1024 x 3072 6.9 vs 15.2)."""
+    require_gpu(x, w)
+    _bf16(x, w)
+    assert x.is_contiguous() and w.is_contiguous() and w.dim() == 2 and x.shape[-1] == w.shape[1]
+    N, K = w.shape
+    M = x.numel() // K
+    if out is None:
+        out = torch.empty((ksplit, M, N), dtype=torch.float32, device=x.device)
+    check(lib.mi_gemm_bf16_splitk(ptr(x), K, ptr(w), ptr(out), M, N, K, ksplit, stream()), "mi_gemm_bf16_splitk")
+    return out
+
+
 def add_rmsnorm_splitk(partials, residual, w, eps: float, out=None, residual_out=None):
     require_gpu(partials, residual, w)
     _bf16(residual, w)
@@ -807,12 +820,13 @@ def sample(logits, temperatures, seed: int, step: int, out=None) -> torch.Tensor
 
 
 def gemm_packed_pick(x, w_packed, temperatures, rng, out_tokens, logits=None, candidates=None, col_offset: int = 0,
-                     pairs_out=None):
+                     pairs_out=None, w=None):
     """logits = x @ w.T (as gemm_packed) and, in the same pass, the sampler's token per row
     (as sample(logits, temperatures, seed, step) with {seed, step} = the two uint64 of the device tensor `rng`).
     Returns (logits, tokens).  Tensor parallelism: w_packed is a vocabulary shard starting at `col_offset` and
     `pairs_out` [M, 2] int32 receives this rank's best {key bits, global token} per row instead of tokens (the
-    ranks then pick among themselves: XgmiComm.pick_exchange)."""
+    ranks then pick among themselves: XgmiComm.pick_exchange).  w: the same weight as stored; above 64 rows the logits are a tile
+    GEMM over it and the tokens come from a pass over them (151936 x 1024, us: 72 rows 171 / 88, 200 rows 364 / 111; the pass over 200 rows 14)."""
     require_gpu(x, rng, out_tokens)
     _bf16(x)
     assert x.is_contiguous() and rng.dtype == torch.int64 and rng.numel() == 2 and out_tokens.dtype == torch.int64
@@ -821,14 +835,20 @@ def gemm_packed_pick(x, w_packed, temperatures, rng, out_tokens, logits=None, ca
     N = w_packed.shape[0]
     assert w_packed.shape[1] == K and out_tokens.numel() >= M
     assert temperatures is None or (temperatures.dtype == torch.float32 and temperatures.numel() >= M)
-    groups = lib.mi_gemm_pick_groups(M, N, K, int(isinstance(w_packed, Fp8Weight)))
+    tile = (w is not None and M > TILE_MIN_ROWS and not isinstance(w_packed, Fp8Weight) and x.dim() == 2
+            and tile_gemm_max_rows(N, K) >= M)
+    groups = lib.mi_logits_pick_groups(N) if tile else lib.mi_gemm_pick_groups(M, N, K, int(isinstance(w_packed, Fp8Weight)))
     assert groups > 0
     if logits is None:
         logits = torch.empty((M, N), dtype=_BF16, device=x.device)
     if candidates is None:
         candidates = torch.empty((M, groups, 2), dtype=torch.int32, device=x.device)
     assert candidates.numel() >= groups * M * 2
-    if isinstance(w_packed, Fp8Weight):
+    if tile:
+        gemm_tile(x, w, out=logits)
+        check(lib.mi_logits_pick(ptr(logits), M, N, ptr(temperatures), ptr(rng), ptr(candidates), int(col_offset), stream()),
+              "mi_logits_pick")
+    elif isinstance(w_packed, Fp8Weight):
         assert col_offset == 0, "fp8 head shards are not picked in the graph"
         check(lib.mi_gemm_fp8w_packed_pick(ptr(x), ptr(w_packed.data), ptr(w_packed.scale), ptr(logits), M, N, K,
                                            ptr(temperatures), ptr(rng), ptr(candidates), stream()),
