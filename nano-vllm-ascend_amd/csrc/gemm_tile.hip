@@ -32,6 +32,7 @@
 // Summation order: one fp32 MFMA chain over K per output element (k ascending), rounded to bf16 once -
 // the same rounding points as F.linear; the SwiGLU epilogue keeps the reference's three roundings
 // (bf16 gate_up output, bf16 silu, bf16 product).
+#include <algorithm>
 #include <type_traits>
 
 #include "mi_common.hpp"
@@ -490,14 +491,16 @@ static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
 // gemm_mid_kernel's shapes (features x tokens): its time per K step with one workgroup on a CU (what the ring's requests take), and for
 // two sharing it.  us, one launch: 200 rows x 4096 features x 1024 with 128 x 128 / 64 x 128 / 64 x 64 tiles 12.5 / 9.3 / 7.1
 // (64 / 128 / 256 workgroups; the weight-streaming kernel 18.6), 400 rows 12.5 / 9.3 / 9.6; 200 x 5120 x 2048 21.2 / 15.8 / 14.5;
-// SwiGLU of 6144 rows x 1024 at 200 tokens 12.7 / 9.4, at 400 12.9 / 12.5; 1024 rows of 6144 x 1024 stay with 128 x 128 (22).
+// SwiGLU of 6144 rows x 1024 at 200 tokens 12.7 / 9.4, at 400 12.9 / 12.5; 1024 rows x 1024 features x 3072: 128 x 128 in four K
+// slices 19.8, 64 x 64 14.1.  Beyond 2048 rows the smaller tiles only read the operands more often (4096 rows x 1024 x 2048:
+// 26.4 / 31.2).
 using Mid64x128 = MidShape<1, 4, 2, 1>;   // (a wave holds a gate and an up fragment: SwiGLU too)
 using Mid64 = MidShape<2, 2, 1, 1>;
 struct MidTile {
   int f, t;
   double step_us, pair_us;
 };
-constexpr MidTile kMidTiles[3] = {{128, 128, 0.52, 0.62}, {64, 128, 0.36, 0.50}, {64, 64, 0.22, 0.35}};
+constexpr MidTile kMidTiles[3] = {{128, 128, 0.52, 0.62}, {64, 128, 0.36, 0.56}, {64, 64, 0.22, 0.35}};
 constexpr double kLaunchUs = 3.8, kPartialBytesPerUs = 4.0e6;
 
 // fewer 256-tiles than CUs: the 128-tile kernel
@@ -509,11 +512,12 @@ struct MidPick {
   int tile, ksplit;
 };
 // fixed_ks: the caller wants that many slices' sums; 0: whatever is fastest, the sum of the slices included
-static MidPick pick_mid(int M, int N, int K, bool silu, int fixed_ks = 0) {
+static MidPick pick_mid(int M, int N, int K, bool silu, int fixed_ks = 0, bool only128 = false) {
   const int kt = K / BK;
+  const int shapes = only128 || M > 2048 ? 1 : silu ? 2 : 3;
   double best = 1e30;
   MidPick pick{0, 1};
-  for (int i = 0; i < (silu ? 2 : 3); ++i) {
+  for (int i = 0; i < shapes; ++i) {
     const MidTile& s = kMidTiles[i];
     const int64_t tiles = (int64_t)((M + s.t - 1) / s.t) * ((N + s.f - 1) / s.f);
     for (int ks = fixed_ks ? fixed_ks : 1; ks <= (fixed_ks ? fixed_ks : silu ? 1 : 16); ks *= 2) {
@@ -551,8 +555,6 @@ static int launch_mid(TileArgs a, hipStream_t st, MidPick pick = {0, 1}) {
   return check_launch();
 }
 
-static int gemm_ksplit(int M, int N, int K) { return use_mid(M, N, K) ? pick_mid(M, N, K, false).ksplit : tile_ksplit(M, N, K); }
-
 static int check_tile_gemm(const void* x, int64_t ldx, const void* w, const void* bias, const void* y, int64_t ldy,
                            int M, int N, int K, int epilogue) {
   if (!x || !w || !y || M < 0 || N <= 0 || K <= 0 || ldx < K) return MI_EINVAL;
@@ -582,7 +584,8 @@ extern "C" int64_t mi_gemm_bf16_max_rows(int N, int K, int64_t ldx) {
 
 extern "C" size_t mi_gemm_bf16_workspace(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK || epilogue != 0) return 0;
-  const int ks = gemm_ksplit(M, N, K);
+  // the most that a plan for the shape has: 128 x 128 tiles in K slices (the smaller tiles are often done without slices)
+  const int ks = use_mid(M, N, K) ? std::max(pick_mid(M, N, K, false).ksplit, pick_mid(M, N, K, false, 0, true).ksplit) : tile_ksplit(M, N, K);
   return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
 }
 
@@ -598,7 +601,7 @@ extern "C" int mi_gemm_bf16(const mi_bf16* x, int64_t ldx, const mi_bf16* w, con
   if (epilogue == 1) return mid ? launch_mid<TEPI_SILU, false>(a, st, pick) : launch_tile<TEPI_SILU, false>(a, st);
   const int ks = mid ? pick.ksplit : tile_ksplit(M, N, K);
   if (ks > 1) {  // two launches: K slices as fp32 partial sums, then their sum (+ bias) rounded once
-    if (!workspace || !aligned16(workspace) || ws_bytes < mi_gemm_bf16_workspace(M, N, K, 0)) return MI_EWORKSPACE;
+    if (!workspace || !aligned16(workspace) || ws_bytes < (size_t)ks * M * N * sizeof(float)) return MI_EWORKSPACE;
     a.part = static_cast<float*>(workspace);
     const int rc2 = mid ? launch_mid<TEPI_PARTIAL, false>(a, st, pick) : launch_tile<TEPI_PARTIAL, false>(a, st, ks);
     if (rc2 != MI_OK) return rc2;
