@@ -771,7 +771,7 @@ int mi_gemm_any_act(const float* x, int64_t ldx, const void* w, const void* w2, 
 int mi_gemm_any_segments(const float* x, int64_t ldx, const void* w, int w_dtype, const float* bias, int act, int act_from,
                          int act2, int act2_from, float* y, int64_t ldy, int M, int N, int K, int exact, mi_stream stream);
 /* The same products for prompt-sized steps over bf16 weights, in two parts: x rounded to bf16 once - gathered into the groups'
- * order - and the MFMA tile kernels over it.  mi_gemm_any_tile_rows: rows of a tile (128 or 256) or 0 when the shape does not
+ * order - and the MFMA tile kernels over it.  mi_gemm_any_tile_rows: rows of a tile (64, 128 or 256) or 0 when the shape does not
  * pay or is not taken (bf16 weights, K % 64 == 0, N % 4 == 0, activations of the shapes in use, n_groups <= 1024; n_groups 0:
  * no groups).  mi_gemm_any_table_ints: int32s of the tile table of a grouped operand.  mi_gemm_any_operand: xb[r] = bf16 of
  * x[x_rows ? x_rows[r] : r] for the rows r before group_offsets[n_groups] (all rows without groups), and the table (may be NULL).

@@ -2,7 +2,7 @@
 // weights bf16 or fp32 as stored ([N][K] row-major), fp32 accumulation, fp32 output - plain, and grouped over
 // expert-sorted rows (one launch for all experts of a sparse feed-forward, SwiGLU optionally in the epilogue).
 //
-// (From 128 rows on, bf16 products of the shapes in use - K a multiple of 64, no segments - go to gemm_any_tile.hip.)
+// (bf16 products of more than 8 to 64 rows, by K - a multiple of 64, no segments - go to gemm_any_tile.hip.)
 //
 // These serve the model families whose residual stream, norms and recurrences are kept in 32-bit floats and whose
 // widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): five kernels,

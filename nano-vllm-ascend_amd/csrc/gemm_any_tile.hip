@@ -1,4 +1,5 @@
-// The prompt-sized projections of the 32-bit-residual model families on the large MFMA tile kernels: fp32 activations are
+// The projections of the 32-bit-residual model families on the MFMA tile kernels (prompt steps, decode batches of more than 8 rows,
+// experts of 16 pairs and more): fp32 activations are
 // rounded to bf16 once, into an operand buffer (gathered into the experts' order on the way), and multiplied by the tile
 // kernels of gemm_tile.hip with an fp32 epilogue.
 //
@@ -123,10 +124,12 @@ __global__ __launch_bounds__(256) void any_operand_kernel(const float* __restric
       u32x4{pack_bf(a.x, a.y), pack_bf(a.z, a.w), pack_bf(b.x, b.y), pack_bf(b.z, b.w)};
 }
 
+static bool tile_rows_ok(int t) { return t == 64 || t == 128 || t == 256; }
+
 // the row tiles of `rows` rows in at most n_groups groups (0: one, its tiles known)
 static int64_t row_tiles(int rows, int n_groups, int t) { return n_groups ? rows / t + n_groups : (rows + t - 1) / t; }
 
-// 0: not taken; else the rows of a tile (256: the persistent kernel, 128: the small-tile kernel)
+// 0: not taken; else the rows of a tile (256: the persistent kernel, 128 and 64: the small-tile kernel)
 static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int act) {
   if (rows < 1 || N < 1 || K < BK || K % BK || N % 4 || n_groups < 0 || n_groups > 1024) return 0;
   const bool known = dual ? act == MI_ACT_SILU || act == MI_ACT_GELU_TANH || act == MI_ACT_CLAMPED_GLU
@@ -135,16 +138,26 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   // 32-bit byte offsets from the operand bases, and 0xF0000000 beyond both (the persistent kernel's "fetch nothing")
   const int64_t limit = (int64_t)1 << 31;
   if (((int64_t)(n_groups ? n_groups : 1) * N + 256) * K * 2 >= limit || ((int64_t)rows + 256) * K * 2 >= limit) return 0;
-  // Where the lines lie (us, this kernel incl. the operand pass against gemm_any.hip's):
-  //   no groups, N 2048, K 2048: 128 rows 25 / 30, 512 rows 28 / 88, 4096 rows 53 / 96; N 512, K 1024: 128 rows 16 / 17.
-  //   Experts' pair of products, 32 of 512 x 1024 (64 of 768 x 2048): 4 rows each 29 / 36 (153 / 170), 16 rows 30 / 109
-  //   (148 / 364), 512 rows 131 / 265 (541 / 1236).
-  // 256-row tiles from about 160 of them on (N 3072, K 1024, 4096 rows: 40, with 128-row tiles 48; N 2048, K 2048, 4096 rows
-  // = 128 tiles: 57 / 53), with groups from 128 rows and some 350 tiles on, where the groups' last, part-filled tiles no
-  // longer weigh (64 experts: 128 rows each 246 / 253, 64 rows 215 / 175; 32 experts of 512 rows = 320 tiles: 142 / 131).
-  if (rows < 128 || N < 128 || rows < n_groups) return 0;
+  if (N < 64) return 0;
+  // Where the lines lie (us, these kernels incl. the 2 us of the operand pass against gemm_any.hip's; up to 8 rows those do not round x,
+  // and they stay).  No groups, N 2048: K 2048 at 9 rows 13.0 / 13.2, at 32 13.2 / 19.1, at 128 14.4 / 43.2; K 512 at 16 rows 7.1 / 5.9,
+  // at 24 7.2 / 7.2, at 64 7.3 / 10.8; K 256 at 32 rows 6.3 / 5.4, at 64 6.4 / 7.9; K 64 from 65 rows on 5.1 / 5.2.  Experts' pair of
+  // products, 32 of 512 x 1024 (64 of 768 x 2048): 16 pairs 19 / 20 (32 / 50), 128 pairs 28 / 37, (64 pairs 82 / 106).
+  if (n_groups ? rows < 16 || (rows < 128 && K < 256) : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) || (rows > 8 && K >= 2048 && !dual)))
+    return 0;
   const int tf = dual ? 128 : 256;
-  if (n_groups) return rows >= 128 * n_groups && (rows / 256 + n_groups / 2) * (int64_t)((N + tf - 1) / tf) >= 350 ? 256 : 128;
+  if (n_groups) {
+    // 64-row tiles while a group's rows are fewer than its last tile's padding would be: 32 rows of 64 experts each 129 / 147 us with
+    // 128-row tiles (32 experts 28 / 36), 64 rows 163 / 156 (37 / 38)
+    if (rows < 48 * (int64_t)n_groups) return 64;
+    // 256-row tiles from 128 rows and some 350 tiles on, where the groups' last, part-filled tiles no longer weigh (64 experts: 128
+    // rows each 246 / 253; 32 experts of 512 rows = 320 tiles: 142 / 131)
+    return rows >= 128 * n_groups && (rows / 256 + n_groups / 2) * (int64_t)((N + tf - 1) / tf) >= 350 ? 256 : 128;
+  }
+  // 64-row tiles while they are at most two per CU (N 2048, K 2048, 512 rows: 13.0, with 128-row tiles 24.7; N 6144: 256 rows 16.7 /
+  // 25.1, 512 rows 29.5 / 26.7); 256-row tiles from about 160 of them on (N 3072, K 1024, 4096 rows: 40, with 128-row tiles 48;
+  // N 2048, K 2048, 4096 rows = 128 tiles: 57 / 53)
+  if ((int64_t)((rows + 63) / 64) * ((N + 63) / 64) <= 512) return 64;
   return ((rows + 255) / 256) * (int64_t)((N + tf - 1) / tf) >= 160 ? 256 : 128;
 }
 
@@ -158,6 +171,21 @@ static int launch_any_tile(const AnyTileArgs<ACT, DUAL>& args, int tile_rows, in
     const int64_t tiles = row_tiles_max * a.tiles_f;
     hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 0, A>), dim3((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid)),
                        dim3(256), 0, st, a);
+  } else if (tile_rows == 64) {
+    // two weights: 128 feature rows (64 outputs); one: 64, or 128 where that leaves at least four tiles per CU (the experts' second
+    // product, us, 64 / 128 features: 32 experts of 1024 x 512 8.9 / 9.6, 64 of 2048 x 768 41 / 39.5)
+    const int64_t narrow = row_tiles_max * ((a.N + 63) / 64);
+    const bool wide = DUAL || narrow > 4 * kPersistentGrid;
+    a.tiles_f = !DUAL && wide ? (a.N + 127) / 128 : (a.N + 63) / 64;
+    a.tiles_t = (a.M + 63) / 64;
+    const int64_t tiles = row_tiles_max * a.tiles_f;
+    if (tiles > 0x7fffffff) return MI_EUNSUPPORTED;
+    if (wide) {
+      hipLaunchKernelGGL((gemm_mid_kernel<TEPI_ANY, false, 3, A, MidShape<2, 2, 2, 1>>), dim3((unsigned)tiles), dim3(256), 0, st, a);
+    } else {
+      if constexpr (!DUAL)
+        hipLaunchKernelGGL((gemm_mid_kernel<TEPI_ANY, false, 5, A, MidShape<2, 2, 1, 1>>), dim3((unsigned)tiles), dim3(256), 0, st, a);
+    }
   } else {
     a.tiles_f = (a.N + (DUAL ? 63 : 127)) / (DUAL ? 64 : 128);
     a.tiles_t = (a.M + 127) / 128;
@@ -180,7 +208,7 @@ extern "C" int mi_gemm_any_tile_rows(int rows, int N, int K, int n_groups, int d
 }
 
 extern "C" int64_t mi_gemm_any_table_ints(int rows, int n_groups, int tile_rows) {
-  if (rows < 0 || n_groups < 1 || (tile_rows != 128 && tile_rows != 256)) return 0;
+  if (rows < 0 || n_groups < 1 || !tile_rows_ok(tile_rows)) return 0;
   return 4 + 4 * row_tiles(rows, n_groups, tile_rows);
 }
 
@@ -189,7 +217,7 @@ extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x
                                    mi_stream stream) {
   if (!x || !xb || rows < 0 || K < 8 || K % 8 || ldx < K || !aligned16(xb)) return MI_EINVAL;
   if (n_groups < 0 || n_groups > 1024 || (n_groups > 0) != (group_offsets != nullptr)) return MI_EINVAL;
-  if (table && (!n_groups || !aligned16(table) || (tile_rows != 128 && tile_rows != 256))) return MI_EINVAL;
+  if (table && (!n_groups || !aligned16(table) || !tile_rows_ok(tile_rows))) return MI_EINVAL;
   if (rows == 0) return MI_OK;
   const int64_t blocks = ((int64_t)rows * (K / 8) + 255) / 256 + (table ? 1 : 0);
   if (blocks > 0x7fffffff) return MI_EUNSUPPORTED;
@@ -205,7 +233,7 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
   if (!xb || !w || !y || rows < 0 || (n_groups > 0) != (table != nullptr) || (row_scale_rows && !row_scale)) return MI_EINVAL;
   if (act == MI_ACT_CLAMPED_GLU && !(limit > 0.f)) return MI_EINVAL;
   if (rows == 0) return MI_OK;
-  if (tile_rows != 128 && tile_rows != 256) return MI_EINVAL;
+  if (!tile_rows_ok(tile_rows)) return MI_EINVAL;
   if (tile_rows_for(rows, N, K, n_groups, w2 != nullptr, act) == 0) return MI_EUNSUPPORTED;
   if (ldy < N || ldy % 4 || !aligned16(xb) || !aligned16(w) || (w2 && !aligned16(w2)) || !aligned16(y) || (bias && !aligned16(bias)) ||
       (bias2 && (!w2 || !aligned16(bias2))))

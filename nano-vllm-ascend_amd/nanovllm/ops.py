@@ -979,7 +979,7 @@ def _i32(*ts: torch.Tensor) -> None:
 def _tile_rows(rows: int, w, w2, act: int, exact: bool, groups: int, *fp32: torch.Tensor) -> int:
     """Rows of a tile if this product goes through the tile kernels (mi_gemm_any_tile), else 0.  fp32: what its epilogue reads
     or writes in 16-byte pieces (None: absent)."""
-    if exact or w.dtype != _BF16 or rows < 128:
+    if exact or w.dtype != _BF16 or rows <= 8:
         return 0
     if any(t is not None and (t.data_ptr() % 16 or (t.dim() == 2 and t.stride(0) % 4)) for t in fp32):
         return 0
@@ -1048,7 +1048,7 @@ def gemm_any_grouped(x, x_rows, w, w2, group_offsets, rows_max: int, y_rows, y_r
 def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_index, limit: float = 0.0, row_scale=None,
               row_scale_rows=None) -> torch.Tensor:
     """Both products of the experts' feed-forwards over expert-sorted pairs: down[e] (act(w[e] x) (* w2[e] x)) of every pair at
-    its place pair_index.  Prompt-sized steps over bf16 weights: the inner activations leave the first product as the bf16 rows
+    its place pair_index.  bf16 weights, 16 pairs and more: the inner activations leave the first product as the bf16 rows
     that the second one multiplies (it would round the same numbers itself)."""
     t = min(_tile_rows(pairs, w, w2, act, False, w.shape[0]), _tile_rows(pairs, down, None, _C.ACT_NONE, False, w.shape[0]))
     if t:

@@ -1,4 +1,4 @@
-"""Prompt-sized projections of the 32-bit-residual families on the tile kernels (mi_gemm_any_tile): edges of row, feature and
+"""Projections of the 32-bit-residual families on the tile kernels (mi_gemm_any_tile): edges of row, feature and
 group tiles, both kernels, every epilogue, scattered rows, against a float64 statement over the rounded operands.
 
 Bound: the operands' products are exact in fp32, the sum over K carries at most K roundings of 2^-24 of the absolute sum, the
@@ -27,8 +27,8 @@ def _close(got, want, size, K):
     assert bool((err <= bound).all()), float((err / bound).max())
 
 
-@pytest.mark.parametrize("tile", [128, 256])
-@pytest.mark.parametrize("M,N,K", [(256, 128, 64), (257, 132, 128), (511, 260, 192), (1030, 644, 320)])
+@pytest.mark.parametrize("tile", [64, 128, 256])
+@pytest.mark.parametrize("M,N,K", [(65, 64, 64), (17, 68, 512), (256, 128, 64), (257, 132, 128), (511, 260, 192), (1030, 644, 320)])
 @pytest.mark.parametrize("act,dual", [(_C.ACT_NONE, False), (_C.ACT_GELU_ERF, False), (_C.ACT_RELU2, False), (_C.ACT_SILU, True),
                                       (_C.ACT_GELU_TANH, True)])
 def test_plain_rows(tile, M, N, K, act, dual):
@@ -49,8 +49,8 @@ def test_plain_rows(tile, M, N, K, act, dual):
     assert bool((out[M] == 7.0).all())
 
 
-@pytest.mark.parametrize("tile", [128, 256])
-@pytest.mark.parametrize("counts", [(300, 0, 1, 128, 129), (0, 0, 256, 257), (64,) * 8, (5, 700)])
+@pytest.mark.parametrize("tile", [64, 128, 256])
+@pytest.mark.parametrize("counts", [(300, 0, 1, 128, 129), (0, 0, 256, 257), (64,) * 8, (5, 700), (1, 0, 65, 3, 64, 2)])
 @pytest.mark.parametrize("act", [_C.ACT_SILU, _C.ACT_CLAMPED_GLU])
 def test_grouped_rows(tile, counts, act):
     G, N, K, T = len(counts), 196, 128, 211
