@@ -15,7 +15,7 @@
 //   gemm_any_f32_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, on the fp32 matrix instruction
 //                          - the float32 serving mode, and the routers of sparse feed-forwards in either mode
 //   gemm_any_fma_kernel    the same in plain FMA chains, for operands whose rows are not whole 128-byte lines
-//   gemm_any_rows_kernel   M <= 8 rows, and the exact mode up to 64: one wave per (output feature, batch of rows)
+//   gemm_any_rows_kernel   M <= 8 rows, and the exact mode up to 64: one wave per (one or four output features, batch of rows)
 //                          streams its weight row once, lanes split K in 16-byte pieces, butterfly reduction; both
 //                          dtypes, x not rounded
 //
@@ -588,13 +588,19 @@ __global__ __launch_bounds__(256) void gemm_any_skinny_kernel(GemmAnyArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// few rows: one wave per output feature and batch of MT rows (blockIdx.y); the lanes take K in pieces of 8, ascending,
+// few rows: one wave per FT output features and batch of MT rows (blockIdx.y); the lanes take K in pieces of 8, ascending,
 // 16-byte loads where the operands allow it, then a butterfly over the lanes
 // ---------------------------------------------------------------------------------------------------------------
-template <typename TW, int MT, bool DUAL, bool EXT>
+// Bound by what is asked for at a time: the rows' pieces are loaded without a branch (rows beyond the end: the last one again, not
+// stored), so that a K piece is one round trip and not one per row - a router's 32 rows x 64 features x 2048 10.7 -> 6.7 us - and
+// four features share the rows' pieces where there are enough features for the chip (N 32768, K 2048: 8 rows 110 us with one feature
+// and a branch per row, now 76, 4 rows 62 / 40; a single row 31 with one feature, 36 with four).
+template <typename TW, int MT, int FT, bool DUAL, bool EXT>
 __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
+  static_assert(FT == 1 || !DUAL, "several features: one weight");
+  constexpr int WN = DUAL ? 2 : FT;
   const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int n = (blockIdx.x * 4 + (threadIdx.x >> 6)) * FT;
   int m_lo, m_hi;
   const TW *w, *w2;
   select_group<TW, DUAL>(a, w, w2, m_lo, m_hi);
@@ -602,34 +608,47 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
   if (n >= a.N || m0 >= m_hi) return;  // (whole waves: the reductions below see all 64 lanes)
   const bool w_vec = a.K % 8 == 0 && dev_aligned16(a.w) && (!DUAL || dev_aligned16(a.w2));
   const bool x_vec = a.ldx % 4 == 0 && dev_aligned16(a.x);
-  float acc[DUAL ? 2 : 1][MT] = {};
-  int64_t xr[MT];
+  float acc[WN][MT] = {};
+  const float* xp[MT];
+  const TW* wp[WN];
 #pragma unroll
-  for (int r = 0; r < MT; ++r) xr[r] = m0 + r < m_hi ? (a.x_rows ? a.x_rows[m0 + r] : m0 + r) : -1;
-  for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) {
-    float wv[DUAL ? 2 : 1][8];
-    load8<TW>(w + (int64_t)n * a.K + k0, a.K - k0, w_vec, wv[0]);
-    if (DUAL) load8<TW>(w2 + (int64_t)n * a.K + k0, a.K - k0, w_vec, wv[DUAL ? 1 : 0]);
+  for (int r = 0; r < MT; ++r) {
+    const int m = min(m0 + r, m_hi - 1);
+    xp[r] = a.x + (int64_t)(a.x_rows ? a.x_rows[m] : m) * a.ldx;
+  }
 #pragma unroll
-    for (int r = 0; r < MT; ++r) {
-      if (xr[r] < 0) continue;
-      float xv[8];
-      load8<float>(a.x + xr[r] * a.ldx + k0, a.K - k0, x_vec, xv);
+  for (int f = 0; f < FT; ++f) wp[f] = w + (int64_t)min(n + f, a.N - 1) * a.K;
+  if (DUAL) wp[WN - 1] = w2 + (int64_t)n * a.K;
+  auto piece = [&](int k0, bool wv_, bool xv_) __attribute__((always_inline)) {
+    float wv[WN][8], xv[MT][8];
+#pragma unroll
+    for (int f = 0; f < WN; ++f) load8<TW>(wp[f] + k0, a.K - k0, wv_, wv[f]);
+#pragma unroll
+    for (int r = 0; r < MT; ++r) load8<float>(xp[r] + k0, a.K - k0, xv_, xv[r]);
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int d = 0; d < (DUAL ? 2 : 1); ++d) acc[d][r] = fmaf(xv[i], wv[d][i], acc[d][r]);
-    }
+        for (int f = 0; f < WN; ++f) acc[f][r] = fmaf(xv[r][i], wv[f][i], acc[f][r]);
+  };
+  if (w_vec && x_vec) {   // (K % 8 == 0: every piece is whole)
+#pragma unroll FT == 1 ? 2 : 1
+    for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, true, true);
+  } else {
+    for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, w_vec, x_vec);
   }
 #pragma unroll
-  for (int r = 0; r < MT; ++r) {
-    const float v = wave_sum(acc[0][r]);
-    const float v2 = DUAL ? wave_sum(acc[DUAL ? 1 : 0][r]) : 0.f;
-    if (lane == 0 && xr[r] >= 0) {
-      const int64_t yrow = a.y_rows ? a.y_rows[m0 + r] : m0 + r;
-      a.y[yrow * a.ldy + n] = finish<DUAL, EXT>(a, m0 + r, yrow, n, v, v2);
+  for (int f = 0; f < FT; ++f)
+#pragma unroll
+    for (int r = 0; r < MT; ++r) {
+      const float v = wave_sum(acc[f][r]);
+      const float v2 = DUAL ? wave_sum(acc[WN - 1][r]) : 0.f;
+      if (lane == 0 && m0 + r < m_hi && n + f < a.N) {
+        const int64_t yrow = a.y_rows ? a.y_rows[m0 + r] : m0 + r;
+        a.y[yrow * a.ldy + n + f] = finish<DUAL, EXT>(a, m0 + r, yrow, n + f, v, v2);
+      }
     }
-  }
 }
 
 // Exact mode beyond a few rows.  The tile of gemm_any_f32_kernel: the largest of 64 x 64, 32 x 64, 32 x 32 whose grid puts a
@@ -668,10 +687,17 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
   const bool few = rows_per_group_max <= 8 || (mode == 1 && rows_per_group_max <= 64);
   if (few) {
     const int mt = rows_per_group_max <= 1 ? 1 : rows_per_group_max <= 4 ? 4 : 8;
-    const dim3 grid((a.N + 3) / 4, (rows_per_group_max + mt - 1) / mt, groups);
-    if (mt == 1) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
-    else if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 4, DUAL, EXT>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 8, DUAL, EXT>), grid, dim3(256), 0, st, a);
+    const int ft = !DUAL && mt > 1 && a.N >= 8192 ? 4 : 1;   // (a wave per four features: from two workgroups per CU on)
+    const dim3 grid((a.N + 4 * ft - 1) / (4 * ft), (rows_per_group_max + mt - 1) / mt, groups);
+    if constexpr (!DUAL)
+      if (ft == 4) {
+        if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 4, 4, DUAL, EXT>), grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 8, 4, DUAL, EXT>), grid, dim3(256), 0, st, a);
+        return check_launch();
+      }
+    if (mt == 1) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 1, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
+    else if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 4, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 8, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
     return check_launch();
   }
   const dim3 grid((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups);

@@ -74,6 +74,7 @@ __device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, 
       if constexpr (A::kAct == MI_ACT_SILU) o = z / (1.f + expf(-z));
       if constexpr (A::kAct == MI_ACT_GELU_TANH) o = 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
       if constexpr (A::kAct == MI_ACT_GELU_ERF) o = 0.5f * z * (1.f + erff(z * 0.7071067811865476f));
+      if constexpr (A::kAct == MI_ACT_SOFTCAP) o = tanhf(z / a.alpha);   // (times alpha below: alpha tanh(z / alpha))
       if constexpr (A::kAct == MI_ACT_RELU2) o = fmaxf(z, 0.f) * fmaxf(z, 0.f);
       if (A::kDual) o *= v2[e];
     }
@@ -133,7 +134,7 @@ static int64_t row_tiles(int rows, int n_groups, int t) { return n_groups ? rows
 static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int act) {
   if (rows < 1 || N < 1 || K < BK || K % BK || N % 4 || n_groups < 0 || n_groups > 1024) return 0;
   const bool known = dual ? act == MI_ACT_SILU || act == MI_ACT_GELU_TANH || act == MI_ACT_CLAMPED_GLU
-                          : act == MI_ACT_NONE || act == MI_ACT_GELU_ERF || act == MI_ACT_RELU2;
+                          : act == MI_ACT_NONE || act == MI_ACT_GELU_ERF || act == MI_ACT_RELU2 || act == MI_ACT_SOFTCAP;
   if (!known) return 0;
   // 32-bit byte offsets from the operand bases, and 0xF0000000 beyond both (the persistent kernel's "fetch nothing")
   const int64_t limit = (int64_t)1 << 31;
@@ -143,7 +144,7 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   // and they stay).  No groups, N 2048: K 2048 at 9 rows 13.0 / 13.2, at 32 13.2 / 19.1, at 128 14.4 / 43.2; K 512 at 16 rows 7.1 / 5.9,
   // at 24 7.2 / 7.2, at 64 7.3 / 10.8; K 256 at 32 rows 6.3 / 5.4, at 64 6.4 / 7.9; K 64 from 65 rows on 5.1 / 5.2.  Experts' pair of
   // products, 32 of 512 x 1024 (64 of 768 x 2048): 16 pairs 19 / 20 (32 / 50), 128 pairs 28 / 37, (64 pairs 82 / 106).
-  if (n_groups ? rows < 16 || (rows < 128 && K < 256) : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) || (rows > 8 && K >= 2048 && !dual)))
+  if (n_groups ? rows < 16 || (rows < 128 && K < 256) : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) || (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
     return 0;
   const int tf = dual ? 128 : 256;
   if (n_groups) {
@@ -254,6 +255,7 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
     return go(AnyTileArgs<MI_ACT_CLAMPED_GLU, true>{});
   }
   if (act == MI_ACT_NONE) return go(AnyTileArgs<MI_ACT_NONE, false>{});
+  if (act == MI_ACT_SOFTCAP) return alpha > 0.f ? go(AnyTileArgs<MI_ACT_SOFTCAP, false>{}) : MI_EINVAL;
   if (act == MI_ACT_GELU_ERF) return go(AnyTileArgs<MI_ACT_GELU_ERF, false>{});
   return go(AnyTileArgs<MI_ACT_RELU2, false>{});
 }

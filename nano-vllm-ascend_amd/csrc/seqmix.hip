@@ -1040,18 +1040,33 @@ __global__ __launch_bounds__(256) void delta_finish_kernel(float* __restrict__ o
 // One wave per token; a lane holds the outputs lane, lane + 64, ... (n <= 512: eight per lane).  Choice scores go through
 // LDS for the group maxima; groups and then outputs are picked by repeated arg-max over the wave (larger value first,
 // equal values: the lower index), NaN scores counting as 0.
+// (v as an integer of the same order - a NaN counts as the lowest value, -0 as 0 - and two DPP reductions: of the keys, then of the
+// indexes that have the best one.  Exchanging value and index over the wave step by step took 12 LDS-latency shuffles per pick: 32 tokens
+// x 64 outputs, 2 of 4 groups and 8 of them 15.4 us, now 6.4.)
+__device__ __forceinline__ int wave_max_int(int v) {
+  float x, y;
+  xor_pair<32>(__int_as_float(v), x, y);
+  v = max(__float_as_int(x), __float_as_int(y));
+  xor_pair<16>(__int_as_float(v), x, y);
+  v = max(__float_as_int(x), __float_as_int(y));
+  v = max(v, __float_as_int(xor_get<8>(__int_as_float(v))));
+  v = max(v, __float_as_int(xor_get<4>(__int_as_float(v))));
+  v = max(v, __float_as_int(xor_get<2>(__int_as_float(v))));
+  return max(v, __float_as_int(xor_get<1>(__int_as_float(v))));
+}
+constexpr int kNoIndex = 1 << 30;   // a lane without a candidate; the result where no lane has one
 __device__ __forceinline__ void wave_argmax(float& v, int& idx) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const float ov = __shfl_xor(v, off);
-    const int oi = __shfl_xor(idx, off);
-    if (ov > v || (ov == v && oi < idx)) v = ov, idx = oi;
-  }
+  const int bits = __float_as_int(v == v ? v + 0.f : -INFINITY);
+  const int key = idx == kNoIndex ? -0x7fffffff - 1 : bits ^ ((bits >> 31) & 0x7fffffff);
+  const int best = wave_max_int(key);
+  idx = -wave_max_int(key == best ? -idx : -kNoIndex);
+  v = __int_as_float(best ^ ((best >> 31) & 0x7fffffff));
 }
 
 // score_kind: MI_ROUTE_SOFTMAX (scores = softmax over the outputs) or MI_ROUTE_SIGMOID (each output's own sigmoid);
 // group_kind: a group's value is its best choice score (MI_ROUTE_GROUP_MAX) or the sum of its two best
 // (MI_ROUTE_GROUP_TOP2; a group of one output: that output's score).
+template <int EPL>   // outputs per lane: n <= 64 EPL
 __global__ __launch_bounds__(256) void route_grouped_kernel(const float* __restrict__ logits, int64_t ld,
                                                             const float* __restrict__ correction, int T, int n, int top_k,
                                                             int n_groups, int keep, int score_kind, int group_kind,
@@ -1062,8 +1077,7 @@ __global__ __launch_bounds__(256) void route_grouped_kernel(const float* __restr
   const int t = blockIdx.x * 4 + wave;
   if (t >= T) return;
   const float* z = logits + (int64_t)t * ld;
-  constexpr int EPL = 8;
-  const int big = 1 << 30;
+  const int big = kNoIndex;
   float sc[EPL], ch[EPL];
   float mx = -INFINITY;
 #pragma unroll
@@ -1104,6 +1118,7 @@ __global__ __launch_bounds__(256) void route_grouped_kernel(const float* __restr
     float gv = -INFINITY;
     if (gi < n_groups) {
       float second = -INFINITY;
+#pragma unroll 4
       for (int e = gi * per; e < (gi + 1) * per; ++e) {
         const float c = choice_s[wave][e];
         if (c > gv) second = gv, gv = c;
@@ -1462,7 +1477,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
   if (t >= T) return;
   const float* z = logits + (int64_t)t * ld;
   constexpr int EPL = 8;
-  const int big = 1 << 30;
+  const int big = kNoIndex;
   float sc[EPL];
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
@@ -2237,8 +2252,11 @@ extern "C" int mi_route_grouped(const float* logits, int64_t ld, const float* co
       top_k < 1 || top_k > keep * (n_outputs / n_groups))
     return MI_EUNSUPPORTED;
   if (n_tokens == 0) return MI_OK;
-  hipLaunchKernelGGL(route_grouped_kernel, dim3((n_tokens + 3) / 4), dim3(256), 0, S(stream), logits, ld, correction,
-                     n_tokens, n_outputs, top_k, n_groups, keep, score_kind, group_kind, ids, weights);
+  const auto kernel = n_outputs <= 64    ? route_grouped_kernel<1>
+                      : n_outputs <= 128 ? route_grouped_kernel<2>
+                      : n_outputs <= 256 ? route_grouped_kernel<4>
+                                         : route_grouped_kernel<8>;
+  hipLaunchKernelGGL(kernel, dim3((n_tokens + 3) / 4), dim3(256), 0, S(stream), logits, ld, correction, n_tokens, n_outputs, top_k, n_groups, keep, score_kind, group_kind, ids, weights);
   return check_launch();
 }
 
