@@ -38,8 +38,14 @@ template <class A>
 __device__ __forceinline__ int any_tiles(const A& a) {
   return a.tiles_f * (a.table ? ((ConstInts)(uintptr_t)a.table)[0] : a.tiles_t);
 }
+// "Block" b's tile: the b & 7-th XCD takes the b & 7-th contiguous run of the tiles (workgroups go to the XCDs in turn: a speed
+// assumption only; one to one for any count).  The 32 workgroups an XCD runs together then share row tiles and an expert's weights in
+// its L2; with tile b each XCD read nearly every operand row for itself (64 experts of 2 x 768 x 2048 over 65536 rows 526 -> 473 us,
+// 32 of 2 x 512 x 1024 over some 32000 124 -> 117).
 template <class A>
-__device__ __forceinline__ AnyTile any_tile(const A& a, int b, int tile_rows, int tile_features) {
+__device__ __forceinline__ AnyTile any_tile(const A& a, int block, int ntiles, int tile_rows, int tile_features) {
+  const int qn = ntiles >> 3, rn = ntiles & 7, xcd = block & 7;
+  const int b = xcd * qn + min(xcd, rn) + (block >> 3);
   const int mt = b / a.tiles_f, nt = b - mt * a.tiles_f;
   if (!a.table) return AnyTile{0, mt * tile_rows, a.M, nt * tile_features};
   ConstInts e = (ConstInts)(uintptr_t)a.table + 4 + 4 * mt;
@@ -147,6 +153,7 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   if (n_groups ? rows < 16 || (rows < 128 && K < 256) : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) || (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
     return 0;
   const int tf = dual ? 128 : 256;
+  if (n_groups && act == MI_ACT_SOFTCAP) return 0;   // (no group has one)
   if (n_groups) {
     // 64-row tiles while a group's rows are fewer than its last tile's padding would be: 32 rows of 64 experts each 129 / 147 us with
     // 128-row tiles (32 experts 28 / 36), 64 rows 163 / 156 (37 / 38)
@@ -159,19 +166,20 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   // 25.1, 512 rows 29.5 / 26.7); 256-row tiles from about 160 of them on (N 3072, K 1024, 4096 rows: 40, with 128-row tiles 48;
   // N 2048, K 2048, 4096 rows = 128 tiles: 57 / 53)
   if ((int64_t)((rows + 63) / 64) * ((N + 63) / 64) <= 512) return 64;
-  return ((rows + 255) / 256) * (int64_t)((N + tf - 1) / tf) >= 160 ? 256 : 128;
+  return act != MI_ACT_SOFTCAP && ((rows + 255) / 256) * (int64_t)((N + tf - 1) / tf) >= 160 ? 256 : 128;
 }
 
 template <int ACT, bool DUAL>
 static int launch_any_tile(const AnyTileArgs<ACT, DUAL>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
   using A = AnyTileArgs<ACT, DUAL>;
   A a = args;
-  if (tile_rows == 256) {
+  if (tile_rows == 256 && ACT != MI_ACT_SOFTCAP) {
     a.tiles_f = (a.N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
     a.tiles_t = (a.M + 255) / 256;
     const int64_t tiles = row_tiles_max * a.tiles_f;
-    hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 0, A>), dim3((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid)),
-                       dim3(256), 0, st, a);
+    if constexpr (ACT != MI_ACT_SOFTCAP)   // (a head's product: never that many rows; it would not fit the persistent kernel's registers)
+      hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 0, A>), dim3((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid)),
+                         dim3(256), 0, st, a);
   } else if (tile_rows == 64) {
     // two weights: 128 feature rows (64 outputs); one: 64, or 128 where that leaves at least four tiles per CU (the experts' second
     // product, us, 64 / 128 features: 32 experts of 1024 x 512 8.9 / 9.6, 64 of 2048 x 768 41 / 39.5)

@@ -38,8 +38,9 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
   int n0 = ((int)blockIdx.x % a.tiles_f) * SH::F, m0 = ((int)blockIdx.x / a.tiles_f) * SH::T, m_end = a.M;
   int64_t wrow0 = 0;
   if constexpr (EPI == TEPI_ANY) {
-    if ((int)blockIdx.x >= any_tiles(a)) return;  // (the grid is the host's bound on the grouped tiles)
-    const AnyTile t = any_tile(a, (int)blockIdx.x, SH::T, ARGS::kDual ? SH::F / 2 : SH::F);
+    const int ntiles = any_tiles(a);
+    if ((int)blockIdx.x >= ntiles) return;  // (the grid is the host's bound on the grouped tiles)
+    const AnyTile t = any_tile(a, (int)blockIdx.x, ntiles, SH::T, ARGS::kDual ? SH::F / 2 : SH::F);
     n0 = t.n0, m0 = t.m0, m_end = t.m_end, wrow0 = (int64_t)t.group * a.N;
   }
 

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
       return;
     }
     if constexpr (EPI == TEPI_ANY) {
-      const AnyTile t = any_tile(a, b, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
+      const AnyTile t = any_tile(a, b, ntiles, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
       if (!wgt) f_row = (uint32_t)(t.m0 + (wave & 1) * 128) * ld2;
       else f_row = (uint32_t)(t.group * a.N + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
       return;
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     const int tid = tile_of_block(blk, a.tiles_t, a.tiles_f, (V & 4) != 0);
     int m0 = (tid / a.tiles_f) * TILE_T, n0 = (tid % a.tiles_f) * TILE_F, m_end = a.M;
     if constexpr (EPI == TEPI_ANY) {
-      const AnyTile t = any_tile(a, blk, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
+      const AnyTile t = any_tile(a, blk, ntiles, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
       m0 = t.m0, n0 = t.n0, m_end = t.m_end;
     }
     kstep(std::true_type{});
