@@ -109,17 +109,27 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const uint16_t* __restri
 // L2; no workgroup waits for another): how many of an expert lie in front of its chunk and how many there are, a scan over the
 // experts, then a cursor per expert for its own pairs.  What bounds one workgroup is the scattered stores, 64 lines per request: 65536
 // pairs of 64 experts 62 us from one CU, 19 from 32 (2048 pairs each); 16384 pairs 17 / 8, 1024 pairs 6.9 / 6.4.
+// ONE: a single workgroup (fewer than 4096 pairs, at most four a thread), which keeps the pairs it has read.
 constexpr int kSortLoads = 4;   // pairs of a thread that are asked for together, in fours
+template <bool ONE>
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ topk_ids, int n_pairs, int top_k, int E, int chunk,
                                                         int32_t* __restrict__ offsets, int32_t* __restrict__ pair_token,
                                                         int32_t* __restrict__ pair_index) {
   __shared__ int before[512], total[512], wave_sums[8];   // (E <= 512)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lo = blockIdx.x * chunk, hi = min(lo + chunk, n_pairs);
+  int own[kSortLoads];
+  if (ONE)
+#pragma unroll
+    for (int u = 0; u < kSortLoads; ++u) own[u] = tid + u * 1024 < n_pairs ? topk_ids[tid + u * 1024] : -1;
   if (tid < 512) before[tid] = total[tid] = 0;
   __syncthreads();
+  if (ONE)
+#pragma unroll
+    for (int u = 0; u < kSortLoads; ++u)
+      if (own[u] >= 0) atomicAdd(&total[own[u]], 1);
   // (lo is a multiple of four: a piece of four lies on one side of it)
-  for (int i0 = 4 * tid; i0 < n_pairs; i0 += kSortLoads * 4096) {
+  for (int i0 = 4 * tid; !ONE && i0 < n_pairs; i0 += kSortLoads * 4096) {
     int id[kSortLoads][4];
 #pragma unroll
     for (int u = 0; u < kSortLoads; ++u)
@@ -146,9 +156,10 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restric
     }
     if (lane == 63) wave_sums[wave] = run;
   }
-  __syncthreads();
+  if (E > 64) __syncthreads();
   if (tid < 512) {
-    for (int w = 0; w < wave; ++w) run += wave_sums[w];
+    if (E > 64)
+      for (int w = 0; w < wave; ++w) run += wave_sums[w];
     before[tid] += run - mine;   // this chunk's cursor
     if (blockIdx.x == 0) {
       if (tid < E) offsets[tid] = run - mine;
@@ -159,10 +170,17 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restric
   // which slot inside an expert's run a pair gets is irrelevant to every result (the pairs of a run are
   // independent MFMA columns, and results are written back by pair index), so the order the atomics happen
   // to produce - different from rank to rank and run to run - is fine
-  for (int i = lo + tid; i < hi; i += 1024) {
-    const int pos = atomicAdd(&before[topk_ids[i]], 1);
+  auto place = [&](int i, int e) {
+    const int pos = atomicAdd(&before[e], 1);
     pair_token[pos] = i / top_k;
     pair_index[pos] = i;
+  };
+  if (ONE) {
+#pragma unroll
+    for (int u = 0; u < kSortLoads; ++u)
+      if (own[u] >= 0) place(tid + u * 1024, own[u]);
+  } else {
+    for (int i = lo + tid; i < hi; i += 1024) place(i, topk_ids[i]);
   }
 }
 
@@ -365,7 +383,7 @@ extern "C" int mi_moe_sort(const int32_t* topk_ids, int n_tokens, int top_k, int
   if (n_experts < 1 || n_experts > 512 || top_k < 1) return MI_EUNSUPPORTED;
   const int n_pairs = n_tokens * top_k, wgs = std::max(1, std::min(32, n_pairs / 2048));
   const int chunk = ((n_pairs + wgs - 1) / wgs + 3) & ~3;
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(wgs), dim3(1024), 0, S(stream), topk_ids, n_pairs, top_k, n_experts, chunk,
+  hipLaunchKernelGGL(wgs == 1 ? moe_sort_kernel<true> : moe_sort_kernel<false>, dim3(wgs), dim3(1024), 0, S(stream), topk_ids, n_pairs, top_k, n_experts, chunk,
                      expert_offsets, pair_token, pair_index);
   return check_launch();
 }
