@@ -112,3 +112,52 @@ def test_convolution_of_eight_rows_at_a_time(ops, taps, C, lens):
                 full = torch.cat([past, own])
                 want = own + sum(w[:, j].double() * full[j:j + l] for j in range(taps))
                 assert l == 0 or (got[cu[i]:cu[i + 1]].double() - want).abs().max() <= (taps + 1) * 2.0 ** -24 * 8 * want.abs().max()
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(8, 4, 128, 128), (3, 1, 12, 8), (40, 2, 128, 64), (2, 2, 20, 36)])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mix", [False, True])
+def test_keys_and_values_to_the_pages_in_pieces(ops, H, G, D, Dv, cache, mix):
+    """q and k normed over the whole projection, values mixed, rows to the pages (one row without a slot): 16-byte pieces and, from rows
+    an odd distance apart, one float at a time (5120 query channels: beyond what a thread keeps)."""
+    torch.manual_seed(H * D + Dv)
+    T, bs, nq, nk, nv = 7, 4, H * D, G * D, G * Dv
+    proj, qw, kw, vf = torch.randn(T, nq + nk + nv), 1 + 0.1 * torch.randn(nq), 1 + 0.1 * torch.randn(nk), torch.randn(T, nv)
+    slots = torch.tensor([5, 0, -1, 11, 2, 7, 8], dtype=torch.int32)
+    lam = torch.tensor([0.3])
+    rms = lambda x, w: x / (x.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w
+    q, k, v = proj.double().split([nq, nk, nv], 1)
+    v = 0.7 * v + 0.3 * vf.double() if mix else v
+    q, k = rms(q, qw.double()), rms(k, kw.double())
+    for place in (lambda t: t.cuda(), lambda t: _off(t.cuda())):
+        p = place(proj)
+        kc, vc = (torch.full((3, G, bs, d), 9.0, dtype=cache, device="cuda") for d in (D, Dv))
+        ops.swa_prepare(p, 0, nq, nq + nk, qw.cuda(), kw.cuda(), 1e-5, place(vf) if mix else None, lam.cuda() if mix else None, kc, vc,
+                        slots.cuda(), H, G, D, Dv, bs)
+        tol = _tol(max(nq, nk)) * 4
+        assert (p[:, :nq].cpu().double() - q).abs().max() <= tol
+        assert (p[:, nq + nk:].cpu().double() - v).abs().max() <= tol
+        used = torch.zeros(3 * bs, dtype=torch.bool)
+        for t, s in enumerate(slots.tolist()):
+            if s >= 0:
+                used[s] = True
+                for c, ref, d in ((kc, k, D), (vc, v, Dv)):
+                    got, want = c[s // bs, :, s % bs].cpu().double(), ref[t].view(G, d)
+                    assert ((got - want).abs() <= tol + (2.0 ** -8 * want.abs() if cache == torch.bfloat16 else 0)).all()
+        for c in (kc, vc):
+            assert (c.permute(0, 2, 1, 3).reshape(3 * bs, -1).cpu()[~used] == 9.0).all()
+
+
+@pytest.mark.parametrize("rows,H,Dv", [(4096, 4, 128), (5461, 3, 100), (16385, 1, 64), (8192, 2, 20)])
+@pytest.mark.parametrize("gate", [False, True])
+def test_head_norms_four_at_a_time(ops, rows, H, Dv, gate):
+    """From 16384 (row, head) pairs on four per wave (5461 x 3: one short of it), in place."""
+    from nanovllm import _C
+    torch.manual_seed(rows)
+    o, z, w = torch.randn(rows, H * Dv + 5), torch.randn(rows, H * Dv), 1 + 0.1 * torch.randn(Dv)
+    v = o[:, :H * Dv].double().view(rows, H, Dv)
+    want = (v / (v.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w.double()).reshape(rows, -1) * (z.double().sigmoid() if gate else 1)
+    got = o.cuda()
+    ops.head_norm_gate(got[:, :H * Dv], z.cuda() if gate else None, _C.ACT_SIGMOID, w.cuda(), H, Dv, 1e-5)
+    assert (got[:, :H * Dv].cpu().double() - want).abs().max() <= _tol(Dv) * want.abs().max()
+    assert torch.equal(got[:, H * Dv:].cpu(), o[:, H * Dv:])
