@@ -413,13 +413,14 @@ def silu_mul(x, out=None) -> torch.Tensor:
 SKINNY_MAX_M = 512
 # ... but a WIDE projection (qkv, gate_up) goes to the MFMA tile kernels above 64 rows, where the streaming kernel begins to read the
 # rows' weights once per 64 (us: 4096 x 1024 at 72 rows 7.1 vs 10.5, at 200 7.1 vs 18.6; gate_up + SwiGLU of 6144 9.2 vs 11.5 and
-# 9.4 vs 17.1; 2048 x 2048 at 100 rows 10.2 vs 8.1, at 137 10.1 vs 14.0), the narrow ones above 256 (1024 x 2048 without K slices
-# at 256 rows 10.6 vs 7.6, at 400 10.7 vs 13.1; 1024 x 3072 14.7 vs 9.4 and 14.8 vs 16.5)
+# 9.4 vs 17.1; 2048 x 2048 at 100 rows 10.2 vs 8.1, at 137 10.1 vs 14.0); the narrow ones (1024 x 2048 without K slices at 256 rows
+# 10.6 vs 7.6, at 400 10.7 vs 13.1) stay up to SKINNY_MAX_M rows: steps that are launched eagerly pay more on the host than that gains
+# (270 rows of a sparse model's 4 layers of width 1024: 770 us per step, 838 with tiles from 257 rows on)
 TILE_MIN_ROWS = 64
 
 
 def prefers_tile(rows: int, n_features: int) -> bool:
-    return rows > SKINNY_MAX_M // 2 or (rows > 2 * TILE_MIN_ROWS and n_features >= 2048) or (rows > TILE_MIN_ROWS and n_features >= 4096)
+    return rows > SKINNY_MAX_M or (rows > 2 * TILE_MIN_ROWS and n_features >= 2048) or (rows > TILE_MIN_ROWS and n_features >= 4096)
 
 
 def gemm_skinny(x, w, bias=None, out=None) -> torch.Tensor:
