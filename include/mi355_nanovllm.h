@@ -784,6 +784,18 @@ int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int tile_rows, con
                      const float* bias, const float* bias2, int act, float limit, const float* row_scale,
                      const int32_t* row_scale_rows, int n_groups, void* y, int y_is_bf16, int64_t ldy,
                      const int32_t* y_rows, int rows, int N, int K, float alpha, mi_stream stream);
+/* mi_gemm_any_act (exact 0) with the choice inside: through the tile kernels where mi_gemm_any_fit_elems gives the elements of the
+ * operand buffer xb (and pointers and strides are in 16-byte pieces), otherwise the general kernels (xb may be NULL). */
+int64_t mi_gemm_any_fit_elems(int M, int N, int K, int dual, int act);
+int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias, const float* bias2,
+                    int act, float* y, int64_t ldy, int M, int N, int K, float alpha, mi_bf16* xb, int64_t xb_elems, mi_stream stream);
+/* Both products of the experts' feed-forwards over expert-sorted pairs on the tile kernels: y[pair_index] = down[e] act(w[e] x) (* w2[e] x).
+ * mi_expert_ff_bytes: 16-byte aligned scratch, 0 where the shapes are not taken. */
+int64_t mi_expert_ff_bytes(int pairs, int n_groups, int ff, int width, int dual, int act);
+int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_token, const mi_bf16* w, const mi_bf16* w2, const mi_bf16* down,
+                 int act, float limit, const float* row_scale, const int32_t* row_scale_rows, const int32_t* offsets,
+                 const int32_t* pair_index, int pairs, int n_groups, int ff, int width, void* scratch, int64_t scratch_bytes, float* y,
+                 mi_stream stream);
 /* mi_gemm_any_grouped with the activation named: y = act(x w^T) (* (x w2^T) with w2). */
 int mi_gemm_any_grouped_act(const float* x, int64_t ldx, const int32_t* x_rows, const void* w, const void* w2, int w_dtype,
                             int act, const int32_t* group_offsets, int n_groups, int rows_per_group_max, float* y,

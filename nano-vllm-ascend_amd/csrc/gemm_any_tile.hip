@@ -267,3 +267,59 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
   if (act == MI_ACT_GELU_ERF) return go(AnyTileArgs<MI_ACT_GELU_ERF, false>{});
   return go(AnyTileArgs<MI_ACT_RELU2, false>{});
 }
+
+// ---- the two launches (operand pass, product) and the choice between these kernels and gemm_any.hip's behind one call: steps that are
+// launched eagerly are bound by the host, which pays for every call (a prompt of 40 rows through 4 layers of Felolorn at width 1024: some 1330 us with four calls per product, 1110 with two) ----
+
+extern "C" int64_t mi_gemm_any_fit_elems(int M, int N, int K, int dual, int act) {
+  return tile_rows_for(M, N, K, 0, dual != 0, act) ? (int64_t)M * K : 0;
+}
+
+extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias,
+                               const float* bias2, int act, float* y, int64_t ldy, int M, int N, int K, float alpha, mi_bf16* xb,
+                               int64_t xb_elems, mi_stream stream) {
+  const bool fits = xb && x && w && y && w_dtype == MI_DTYPE_BF16 && M > 0 && ldx >= K && ldy >= N && ldy % 4 == 0 && aligned16(w) &&
+                    (!w2 || aligned16(w2)) && aligned16(y) && (!bias || aligned16(bias)) && (!bias2 || (w2 && aligned16(bias2))) &&
+                    aligned16(xb) && xb_elems >= (int64_t)M * K && !(act == MI_ACT_SOFTCAP && !(alpha > 0.f));
+  const int t = fits ? tile_rows_for(M, N, K, 0, w2 != nullptr, act) : 0;
+  if (!t) return mi_gemm_any_act(x, ldx, w, w2, w_dtype, bias, bias2, act, y, ldy, M, N, K, alpha, 0, stream);
+  const int rc = mi_gemm_any_operand(x, ldx, nullptr, nullptr, 0, t, M, K, xb, nullptr, stream);
+  return rc != MI_OK ? rc
+                     : mi_gemm_any_tile(xb, nullptr, t, static_cast<const mi_bf16*>(w), static_cast<const mi_bf16*>(w2), bias, bias2, act,
+                                        0.f, nullptr, nullptr, 0, y, 0, ldy, nullptr, M, N, K, alpha, stream);
+}
+
+// scratch of mi_expert_ff: the gathered operand, the inner activations, the tile table (each rounded up to 16 bytes)
+static int expert_tile_rows(int pairs, int G, int ff, int width, bool dual, int act) {
+  const int a = tile_rows_for(pairs, ff, width, G, dual, act), b = tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE);
+  return a < b ? a : b;
+}
+static int64_t round16(int64_t bytes) { return (bytes + 15) & ~(int64_t)15; }
+
+extern "C" int64_t mi_expert_ff_bytes(int pairs, int G, int ff, int width, int dual, int act) {
+  if (pairs < 1 || G < 1) return 0;
+  const int t = expert_tile_rows(pairs, G, ff, width, dual != 0, act);
+  return t ? round16((int64_t)pairs * width * 2) + round16((int64_t)pairs * ff * 2) + 4 * mi_gemm_any_table_ints(pairs, G, t) : 0;
+}
+
+extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_token, const mi_bf16* w, const mi_bf16* w2,
+                            const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
+                            const int32_t* offsets, const int32_t* pair_index, int pairs, int G, int ff, int width, void* scratch,
+                            int64_t scratch_bytes, float* y, mi_stream stream) {
+  if (!x || !w || !down || !offsets || !scratch || !y || pairs < 1 || G < 1 || !aligned16(scratch)) return MI_EINVAL;
+  const int64_t need = mi_expert_ff_bytes(pairs, G, ff, width, w2 != nullptr, act);
+  if (need == 0) return MI_EUNSUPPORTED;
+  if (scratch_bytes < need) return MI_EWORKSPACE;
+  const int t = expert_tile_rows(pairs, G, ff, width, w2 != nullptr, act);
+  char* p = static_cast<char*>(scratch);
+  mi_bf16* xb = reinterpret_cast<mi_bf16*>(p);
+  mi_bf16* inner = reinterpret_cast<mi_bf16*>(p += round16((int64_t)pairs * width * 2));
+  int32_t* table = reinterpret_cast<int32_t*>(p += round16((int64_t)pairs * ff * 2));
+  int rc = mi_gemm_any_operand(x, ldx, pair_token, offsets, G, t, pairs, width, xb, table, stream);
+  if (rc == MI_OK)
+    rc = mi_gemm_any_tile(xb, table, t, w, w2, nullptr, nullptr, act, limit, row_scale, row_scale_rows, G, inner, 1, ff, nullptr, pairs, ff,
+                          width, 1.f, stream);
+  return rc != MI_OK ? rc
+                     : mi_gemm_any_tile(inner, table, t, down, nullptr, nullptr, nullptr, MI_ACT_NONE, 0.f, nullptr, nullptr, G, y, 0, width,
+                                        pair_index, pairs, width, ff, 1.f, stream);
+}

@@ -202,6 +202,11 @@ _SIGNATURES = {
                                 c_int, _p]),
     "mi_gemm_any_tile_rows": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mi_gemm_any_table_ints": (c_int64, [c_int, c_int, c_int]),
+    "mi_gemm_any_fit_elems": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
+    "mi_gemm_any_fit": (c_int, [_p, c_int64, _p, _p, c_int, _p, _p, c_int, _p, c_int64, c_int, c_int, c_int, c_float, _p, c_int64, _p]),
+    "mi_expert_ff_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int, c_int]),
+    "mi_expert_ff": (c_int, [_p, c_int64, _p, _p, _p, _p, c_int, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p, c_int64, _p,
+                             _p]),
     "mi_gemm_any_operand": (c_int, [_p, c_int64, _p, _p, c_int, c_int, c_int, c_int, _p, _p, _p]),
     "mi_gemm_any_tile": (c_int, [_p, _p, c_int, _p, _p, _p, _p, c_int, c_float, _p, _p, c_int, _p, c_int, c_int64, _p, c_int,
                                  c_int, c_int, c_float, _p]),

@@ -1010,6 +1010,13 @@ def _tile_gemm(operand, tile_rows: int, w, w2, out, act: int, groups: int = 0, y
     return out
 
 
+def _gemm_any_fit(x, w, w2, bias, bias2, act: int, out, M: int, N: int, K: int, alpha: float) -> None:
+    n = lib.mi_gemm_any_fit_elems(M, N, K, w2 is not None, act)
+    xb = torch.empty(n, dtype=_BF16, device=x.device) if n else None
+    check(lib.mi_gemm_any_fit(ptr(x), x.stride(0), ptr(w), ptr(w2), _C.DTYPE_BF16, ptr(bias), ptr(bias2), act, ptr(out), out.stride(0),
+                              M, N, K, alpha, ptr(xb), n, stream()), "mi_gemm_any_fit")
+
+
 def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None) -> torch.Tensor:
     """alpha * x @ w.T for any shapes; x may be a column slice of a wider buffer (unit inner stride)."""
     require_gpu(x, w)
@@ -1020,9 +1027,9 @@ def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None) -> torch.T
     if out is None:
         out = torch.empty((M, N), dtype=_F32, device=x.device)
     assert out.shape == (M, N)
-    t = _tile_rows(M, w, None, _C.ACT_NONE, exact, 0, out)
-    if t:
-        return _tile_gemm(_tile_operand(x, t), t, w, None, out, _C.ACT_NONE, alpha=alpha)
+    if M > 8 and not exact and w.dtype == _BF16:
+        _gemm_any_fit(x, w, None, None, None, _C.ACT_NONE, out, M, N, K, alpha)
+        return out
     check(lib.mi_gemm_any(ptr(x), x.stride(0) if M > 1 else K, ptr(w), _dt(w), ptr(out), out.stride(0) if M > 1 else N,
                           M, N, K, float(alpha), int(exact), stream()), "mi_gemm_any")
     return out
@@ -1051,18 +1058,20 @@ def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_in
     """Both products of the experts' feed-forwards over expert-sorted pairs: down[e] (act(w[e] x) (* w2[e] x)) of every pair at
     its place pair_index.  bf16 weights, 16 pairs and more: the inner activations leave the first product as the bf16 rows
     that the second one multiplies (it would round the same numbers itself)."""
-    t = min(_tile_rows(pairs, w, w2, act, False, w.shape[0]), _tile_rows(pairs, down, None, _C.ACT_NONE, False, w.shape[0]))
-    if t:
+    G, ff, width = w.shape
+    n = lib.mi_expert_ff_bytes(pairs, G, ff, width, w2 is not None, int(act)) if w.dtype == _BF16 and down.dtype == _BF16 else 0
+    if n and not (w.data_ptr() | down.data_ptr() | (0 if w2 is None else w2.data_ptr())) % 16:
         require_gpu(x, w, offsets)
         _f32(x, row_scale)
         _i32(pair_token, pair_index, offsets, row_scale_rows)
-        assert x.shape[1] == w.shape[2] and down.shape == (w.shape[0], w.shape[2], w.shape[1]) and offsets.numel() > w.shape[0]
-        G, ff, width = w.shape
-        operand = _tile_operand(x, t, pair_token, offsets, G, pairs)
-        inner = torch.empty((pairs, ff), dtype=_BF16, device=x.device)
-        _tile_gemm(operand, t, w, w2, inner, act, G, limit=limit, row_scale=row_scale, row_scale_rows=row_scale_rows)
+        assert x.shape[1] == width and down.shape == (G, width, ff) and offsets.numel() > G
+        assert w.is_contiguous() and down.is_contiguous() and (w2 is None or (w2.shape == w.shape and w2.is_contiguous() and w2.dtype == _BF16))
+        scratch = torch.empty(n, dtype=torch.uint8, device=x.device)
         y = torch.empty((pairs, width), dtype=_F32, device=x.device)
-        return _tile_gemm((inner, operand[1]), t, down, None, y, _C.ACT_NONE, G, pair_index)
+        check(lib.mi_expert_ff(ptr(x), x.stride(0) if x.shape[0] > 1 else width, ptr(pair_token), ptr(w), ptr(w2), ptr(down), int(act),
+                               float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets), ptr(pair_index), pairs, G, ff, width,
+                               ptr(scratch), n, ptr(y), stream()), "mi_expert_ff")
+        return y
     a = gemm_any_grouped_glu(x, pair_token, w, w2, act, limit, row_scale, row_scale_rows, offsets, pairs, None, pairs)
     return gemm_any_grouped(a, None, down, None, offsets, pairs, pair_index, pairs)
 
@@ -1270,9 +1279,9 @@ def gemm_any_act(x, w, bias=None, act: int = _C.ACT_NONE, w2=None, bias2=None, a
     if out is None:
         out = torch.empty((M, N), dtype=_F32, device=x.device)
     assert out.shape == (M, N)
-    t = _tile_rows(M, w, w2, act, exact, 0, out, bias, bias2)
-    if t:
-        return _tile_gemm(_tile_operand(x, t), t, w, w2, out, act, bias=bias, bias2=bias2, alpha=alpha)
+    if M > 8 and not exact and w.dtype == _BF16:
+        _gemm_any_fit(x, w, w2, bias, bias2, int(act), out, M, N, K, alpha)
+        return out
     check(lib.mi_gemm_any_act(ptr(x), x.stride(0) if M > 1 else K, ptr(w), ptr(w2), _dt(w), ptr(bias), ptr(bias2), int(act),
                               ptr(out), out.stride(0) if M > 1 else N, M, N, K, float(alpha), int(exact), stream()),
           "mi_gemm_any_act")
