@@ -95,24 +95,26 @@ __device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, 
 #include "gemm_mid_kernel.hpp"
 
 // x rows -> bf16 rows (eight elements a thread), gathered by x_rows; rows from the groups' end on are left as they are.
-// The grid's last workgroup writes the tile table.
+// The grid's last workgroup writes the tile table: `table_tiles` entries at most, of rows before `rows` - whatever the groups' ends say,
+// nothing is written or, by the product that follows the table, read beyond the buffers.
 __global__ __launch_bounds__(256) void any_operand_kernel(const float* __restrict__ x, int64_t ldx,
                                                           const int32_t* __restrict__ x_rows,
                                                           const int32_t* __restrict__ group_offsets, int n_groups,
                                                           int tile_rows, int rows, int K, uint16_t* __restrict__ xb,
-                                                          int32_t* __restrict__ table) {
+                                                          int32_t* __restrict__ table, int table_tiles) {
   __shared__ int tiles[1024];
   const int tid = threadIdx.x;
   if (table && blockIdx.x == gridDim.x - 1) {
-    for (int g = tid; g < n_groups; g += 256) tiles[g] = (group_offsets[g + 1] - group_offsets[g] + tile_rows - 1) / tile_rows;
+    auto end_of = [&](int g) { return min(max(group_offsets[g], 0), rows); };
+    for (int g = tid; g < n_groups; g += 256) tiles[g] = (max(end_of(g + 1) - end_of(g), 0) + tile_rows - 1) / tile_rows;
     __syncthreads();
     for (int g = tid; g < n_groups; g += 256) {
       int at = 0;
       for (int j = 0; j < g; ++j) at += tiles[j];
-      const int lo = group_offsets[g], hi = group_offsets[g + 1];
-      for (int i = 0; i < tiles[g]; ++i)
+      const int lo = end_of(g), hi = end_of(g + 1);
+      for (int i = 0; i < tiles[g] && at + i < table_tiles; ++i)
         *reinterpret_cast<int4*>(table + 4 + 4 * (at + i)) = int4{g, lo + i * tile_rows, hi, 0};
-      if (g == n_groups - 1) *reinterpret_cast<int4*>(table) = int4{at + tiles[g], 0, 0, 0};
+      if (g == n_groups - 1) *reinterpret_cast<int4*>(table) = int4{min(at + tiles[g], table_tiles), 0, 0, 0};
     }
     return;
   }
@@ -231,7 +233,7 @@ extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x
   const int64_t blocks = ((int64_t)rows * (K / 8) + 255) / 256 + (table ? 1 : 0);
   if (blocks > 0x7fffffff) return MI_EUNSUPPORTED;
   hipLaunchKernelGGL(any_operand_kernel, dim3((unsigned)blocks), dim3(256), 0, S(stream), x, ldx, x_rows, group_offsets, n_groups,
-                     tile_rows, rows, K, xb, table);
+                     tile_rows, rows, K, xb, table, table ? (int)row_tiles(rows, n_groups, tile_rows) : 0);
   return check_launch();
 }
 

@@ -1010,6 +1010,23 @@ def _tile_gemm(operand, tile_rows: int, w, w2, out, act: int, groups: int = 0, y
     return out
 
 
+def _grouped_tile_rows(total: int, rows_max: int, w, w2, act: int, exact: bool, *fp32: torch.Tensor) -> int:
+    """_tile_rows of a grouped product: `total` sorted rows of all groups, at most rows_max in one (up to 8 the general kernels do not
+    round x)."""
+    return _tile_rows(total, w, w2, act, exact, w.shape[0], *fp32) if rows_max > 8 else 0
+
+
+def _grouped_tiles(x, x_rows, w, w2, act: int, offsets, rows_max: int, y, y_rows, exact: bool, **epilogue) -> bool:
+    """A grouped product through the tile kernels, if it goes there.  Their operand and tile table hold the rows of ALL groups: as many
+    as there are places to take one from."""
+    total = x.shape[0] if x_rows is None else x_rows.numel()
+    t = _grouped_tile_rows(total, rows_max, w, w2, act, exact, y)
+    if t:
+        G = w.shape[0]
+        _tile_gemm(_tile_operand(x, t, x_rows, offsets, G, total), t, w, w2, y, act, G, y_rows, **epilogue)
+    return t > 0
+
+
 def _gemm_any_fit(x, w, w2, bias, bias2, act: int, out, M: int, N: int, K: int, alpha: float) -> None:
     n = lib.mi_gemm_any_fit_elems(M, N, K, w2 is not None, act)
     xb = torch.empty(n, dtype=_BF16, device=x.device) if n else None
@@ -1044,10 +1061,8 @@ def gemm_any_grouped(x, x_rows, w, w2, group_offsets, rows_max: int, y_rows, y_r
     G, N, K = w.shape
     assert x.shape[1] == K and group_offsets.numel() >= G + 1
     y = torch.empty((y_rows_total, N), dtype=_F32, device=x.device)
-    act = _C.ACT_NONE if w2 is None else _C.ACT_SILU
-    t = _tile_rows(rows_max, w, w2, act, exact, G, y)
-    if t:
-        return _tile_gemm(_tile_operand(x, t, x_rows, group_offsets, G, rows_max), t, w, w2, y, act, G, y_rows)
+    if _grouped_tiles(x, x_rows, w, w2, _C.ACT_NONE if w2 is None else _C.ACT_SILU, group_offsets, rows_max, y, y_rows, exact):
+        return y
     check(lib.mi_gemm_any_grouped(ptr(x), x.stride(0), ptr(x_rows), ptr(w), ptr(w2), _dt(w), ptr(group_offsets), G,
                                   rows_max, ptr(y), N, ptr(y_rows), N, K, int(exact), stream()), "mi_gemm_any_grouped")
     return y
@@ -1298,9 +1313,8 @@ def gemm_any_grouped_act(x, x_rows, w, w2, act: int, group_offsets, rows_max: in
     G, N, K = w.shape
     assert x.shape[1] == K and group_offsets.numel() >= G + 1
     y = torch.empty((y_rows_total, N), dtype=_F32, device=x.device)
-    t = _tile_rows(rows_max, w, w2, act, exact, G, y)
-    if t:
-        return _tile_gemm(_tile_operand(x, t, x_rows, group_offsets, G, rows_max), t, w, w2, y, act, G, y_rows)
+    if _grouped_tiles(x, x_rows, w, w2, act, group_offsets, rows_max, y, y_rows, exact):
+        return y
     check(lib.mi_gemm_any_grouped_act(ptr(x), x.stride(0), ptr(x_rows), ptr(w), ptr(w2), _dt(w), int(act), ptr(group_offsets),
                                       G, rows_max, ptr(y), N, ptr(y_rows), N, K, int(exact), stream()),
           "mi_gemm_any_grouped_act")
@@ -1557,10 +1571,9 @@ def gemm_any_grouped_glu(x, x_rows, w, w2, act: int, limit: float, row_scale, ro
     G, N, K = w.shape
     assert x.shape[1] == K and group_offsets.numel() >= G + 1
     y = torch.empty((y_rows_total, N), dtype=_F32, device=x.device)
-    t = _tile_rows(rows_max, w, w2, act, exact, G, y)
-    if t:
-        return _tile_gemm(_tile_operand(x, t, x_rows, group_offsets, G, rows_max), t, w, w2, y, act, G, y_rows, limit=limit,
-                          row_scale=row_scale, row_scale_rows=row_scale_rows)
+    if _grouped_tiles(x, x_rows, w, w2, act, group_offsets, rows_max, y, y_rows, exact, limit=limit, row_scale=row_scale,
+                      row_scale_rows=row_scale_rows):
+        return y
     check(lib.mi_gemm_any_grouped_glu(ptr(x), x.stride(0), ptr(x_rows), ptr(w), ptr(w2), _dt(w), int(act), float(limit),
                                       ptr(row_scale), ptr(row_scale_rows), ptr(group_offsets), G, rows_max, ptr(y), N,
                                       ptr(y_rows), N, K, int(exact), stream()), "mi_gemm_any_grouped_glu")

@@ -96,3 +96,28 @@ def test_expert_pair_takes_the_same_bits_as_two_products(act, limit):
     two = ops.gemm_any_grouped(a, None, down, None, off, T * top, place, T * top)
     one = ops.expert_ff(h, tok, gate, up, down, act, off, T * top, place, limit, scale, place if scale is not None else None)
     assert ops._tile_rows(T * top, gate, up, act, False, E) and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("counts", [(200,) * 8, (9, 0, 300, 1)])
+def test_bound_on_one_groups_rows(counts, gathered):
+    """rows_max bounds ONE group; the product covers the rows of all of them"""
+    G, N, K, T, P = len(counts), 68, 64, 111, sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(P)
+    x = torch.randn(T if gathered else P, K, device="cuda", generator=g)
+    rows = torch.randint(0, T, (P,), device="cuda", generator=g, dtype=torch.int32) if gathered else None
+    xs = (x[rows.long()] if gathered else x).bfloat16().double()
+    place = torch.randperm(P, device="cuda", generator=g).to(torch.int32)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device="cuda")
+    w, w2 = (torch.randn(G, N, K, device="cuda", generator=g).mul(K ** -0.5).bfloat16() for _ in range(2))
+    z, z2, s, s2 = (torch.empty(P, N, device="cuda", dtype=torch.float64) for _ in range(4))
+    for e in range(G):
+        r = slice(int(off[e]), int(off[e + 1]))
+        at = place[r].long()
+        z[at], z2[at] = xs[r] @ w[e].double().T, xs[r] @ w2[e].double().T
+        s[at], s2[at] = xs[r].abs() @ w[e].double().abs().T, xs[r].abs() @ w2[e].double().abs().T
+    most = max(counts)
+    _close(ops.gemm_any_grouped(x, rows, w, None, off, most, place, P), z, s, K)
+    _close(ops.gemm_any_grouped_act(x, rows, w, None, _C.ACT_RELU2, off, most, place, P), z.clamp(min=0) ** 2, 2 * s * s, K)
+    _close(ops.gemm_any_grouped_glu(x, rows, w, w2, _C.ACT_CLAMPED_GLU, 1.5, None, None, off, most, place, P),
+           _ref(z, z2, _C.ACT_CLAMPED_GLU, 1.5), 4 * s * (s2 + 1), K)

@@ -1,0 +1,57 @@
+"""Grouped products take `rows_max` as a bound on ONE group's rows: the operand buffer and the tile table of the tile path have to be
+sized for the rows of all groups.  The library calls are recorded, not made."""
+import pytest
+import torch
+
+from nanovllm import _C, ops
+
+
+class _Recorder:
+    """mi_gemm_any_operand / mi_gemm_any_tile recorded, everything else the library's own"""
+
+    def __init__(self, lib):
+        self.lib, self.calls = lib, {}
+
+    def __getattr__(self, name):
+        if name not in ("mi_gemm_any_operand", "mi_gemm_any_tile"):
+            return getattr(self.lib, name)
+        return lambda *a: self.calls.setdefault(name, a) and 0
+
+
+@pytest.mark.parametrize("name", ["gemm_any_grouped", "gemm_any_grouped_act", "gemm_any_grouped_glu"])
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("counts", [(200,) * 8, (9, 0, 300, 1)])
+def test_rows_of_all_groups(monkeypatch, name, gathered, counts):
+    G, N, K, total = len(counts), 64, 64, sum(counts)
+    rec = _Recorder(_C.lib)
+    made = []
+    empty = torch.empty
+    monkeypatch.setattr(ops, "lib", rec)
+    monkeypatch.setattr(ops, "require_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "stream", lambda: 0)
+    monkeypatch.setattr(ops.torch, "empty", lambda *a, **k: made.append(empty(*a, **k)) or made[-1])
+    w = torch.zeros(G, N, K, dtype=torch.bfloat16)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32)
+    x = torch.zeros(17 if gathered else total, K)
+    x_rows = torch.zeros(total, dtype=torch.int32) if gathered else None
+    y_rows = torch.arange(total, dtype=torch.int32)
+    most = max(counts)
+    if name == "gemm_any_grouped":
+        ops.gemm_any_grouped(x, x_rows, w, None, off, most, y_rows, total)
+    elif name == "gemm_any_grouped_act":
+        ops.gemm_any_grouped_act(x, x_rows, w, None, _C.ACT_NONE, off, most, y_rows, total)
+    else:
+        ops.gemm_any_grouped_glu(x, x_rows, w, None, _C.ACT_NONE, 0.0, None, None, off, most, y_rows, total)
+    operand, tile = rec.calls["mi_gemm_any_operand"], rec.calls["mi_gemm_any_tile"]
+    tile_rows, rows = operand[5], operand[6]
+    assert rows >= total and tile[16] >= total
+    xb = next(t for t in made if t.data_ptr() == operand[8])
+    table = next(t for t in made if t.data_ptr() == operand[9])
+    assert xb.shape[0] >= total
+    assert table.numel() >= 4 + 4 * sum(-(-c // tile_rows) for c in counts)
+
+
+def test_few_rows_per_group_stay_on_the_kernel_that_does_not_round_them():
+    w = torch.zeros(64, 64, 64, dtype=torch.bfloat16)
+    assert ops._grouped_tile_rows(512, 9, w, None, _C.ACT_NONE, False)
+    assert not ops._grouped_tile_rows(512, 8, w, None, _C.ACT_NONE, False)
