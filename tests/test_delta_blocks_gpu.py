@@ -89,3 +89,35 @@ def test_channel_delta_by_blocks(ops, lens, H, G, D, Dv):
     live = [len(lens) - 1 - i for i, n in enumerate(lens) if n]   # (slots are handed out in reverse; an empty sequence's stays as it was)
     assert (s_blocks[live] - s_rows[live]).abs().max() <= 4 * (D + 16) * 2.0 ** -24 * s_rows[live].abs().max()
     assert all((s_blocks[len(lens) - 1 - i] == 7.0).all() for i, n in enumerate(lens) if n == 0)
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "decay", "beta"])
+@pytest.mark.parametrize("at", [0, 5, 21, 32, 66])
+def test_values_that_are_not_finite_stay_behind_their_row(ops, where, value, at):
+    """A NaN or an infinity in a row: the rows in front of it, of its own block too, are what they are without it, and what is not finite
+    behind it is what the row-by-row kernel has not finite."""
+    torch.manual_seed(at)
+    n, H, G, D, Dv, eps = 70, 4, 2, 64, 40, 1e-6
+    t = dict(qkv=torch.randn(n, 2 * G * D + H * Dv), beta=torch.randn(n, H), gate=torch.randn(n, H * Dv), decay=torch.randn(n, H * D),
+             dt=torch.randn(H * D), a_log=torch.randn(H) * 0.5, w=1 + 0.1 * torch.randn(Dv))
+    g = {k: v.cuda() for k, v in t.items()}
+
+    def call(max_rows):
+        state = torch.full((2, ops.channel_delta_state_elems(H, D, Dv)), 7.0, device="cuda")
+        o = ops.channel_delta(g["qkv"], 0, G * D, 2 * G * D, g["beta"], g["decay"], g["dt"], g["a_log"], g["gate"], g["w"], state,
+                              torch.tensor([0, n - 3, n], dtype=torch.int32).cuda(), torch.tensor([n - 3, 3], dtype=torch.int32).cuda(),
+                              torch.tensor([1, 0], dtype=torch.int32).cuda(), H, G, D, Dv, eps, max_rows)
+        return o, state
+
+    clean, clean_state = call(4096)
+    assert torch.isfinite(clean).all()
+    name, col = {"q": ("qkv", 3), "k": ("qkv", G * D + D + 2), "v": ("qkv", 2 * G * D + 2 * Dv + 33), "decay": ("decay", D + 9), "beta": ("beta", 1)}[where]
+    g[name][at, col] = -value if where == "decay" else value   # (an infinite decay of 0 is a plain number)
+    (got, state), (by_row, row_state) = call(4096), call(1)
+    assert torch.equal(got[:at], clean[:at])
+    assert torch.equal(torch.isfinite(got), torch.isfinite(by_row))
+    assert torch.equal(torch.isfinite(state), torch.isfinite(row_state))
+    fine = torch.isfinite(by_row)
+    assert (got[fine] - by_row[fine]).abs().max() <= 8 * (D + 16) * 2.0 ** -24 * clean.abs().max() * (clean.abs().max() / clean.pow(2).mean().sqrt())
+    assert torch.equal(got[n - 3:][torch.isfinite(got[n - 3:])], clean[n - 3:][torch.isfinite(got[n - 3:])])
