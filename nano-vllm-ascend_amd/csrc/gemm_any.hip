@@ -5,7 +5,7 @@
 // (bf16 products of more than 8 to 64 rows, by K - a multiple of 64, no segments - go to gemm_any_tile.hip.)
 //
 // These serve the model families whose residual stream, norms and recurrences are kept in 32-bit floats and whose
-// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): five kernels,
+// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): six kernels,
 //
 //   gemm_any_mfma_kernel   bf16 weights: a 64 x 64 (from 512 rows: 128 x 128, with SwiGLU 128 x 64) output tile per 4-wave
 //                          workgroup, x rounded to bf16 on its way into LDS, v_mfma_f32_16x16x32_bf16, the next K
@@ -18,6 +18,7 @@
 //   gemm_any_rows_kernel   M <= 8 rows, and the exact mode up to 64: one wave per (one or four output features, batch of rows)
 //                          streams its weight row once, lanes split K in 16-byte pieces, butterfly reduction; both
 //                          dtypes, x not rounded
+//   gemm_any_each_row_kernel  the same for groups that have a row or none each
 //
 // A row of the result is a function of its own x row and the weights only: the summation order over k does not depend
 // on M, on the row's place in the batch or on the tile it falls into (each kernel has ONE fixed order), so the same
@@ -651,6 +652,50 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
     }
 }
 
+// The same one row after the other, for groups that have one or none each (the experts of a token or two): a batch would multiply its
+// empty places too, and its registers leave too few waves to keep the weights coming.  us, gate and up / down, batches of 8 | here:
+// 8 pairs of 64 experts of 768 x 2048 33.7 / 37.4 | 15.2 / 14.9, 4 of 32 of 512 x 1024 6.5 / 5.6 | 5.1 / 4.7 (fp32, 8 pairs: 12.1 / 11.1 |
+// 7.3 / 5.7); all eight in one expert 12.8 / 14.8 | 22.3 / 14.7.
+template <typename TW, bool DUAL, bool EXT>
+__global__ __launch_bounds__(256) void gemm_any_each_row_kernel(GemmAnyArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  int m_lo, m_hi;
+  const TW *w, *w2;
+  select_group<TW, DUAL>(a, w, w2, m_lo, m_hi);
+  if (n >= a.N) return;  // (whole waves)
+  const bool w_vec = a.K % 8 == 0 && dev_aligned16(a.w) && (!DUAL || dev_aligned16(a.w2));
+  const bool x_vec = a.ldx % 4 == 0 && dev_aligned16(a.x);
+  w += (int64_t)n * a.K;
+  if (DUAL) w2 += (int64_t)n * a.K;
+  for (int m = m_lo + blockIdx.y; m < m_hi; m += gridDim.y) {
+    const float* x = a.x + (int64_t)(a.x_rows ? a.x_rows[m] : m) * a.ldx;
+    float acc = 0.f, acc2 = 0.f;
+    auto piece = [&](int k0, bool wv_, bool xv_) __attribute__((always_inline)) {
+      float xv[8], wv[8], wv2[8];
+      load8<TW>(w + k0, a.K - k0, wv_, wv);
+      if (DUAL) load8<TW>(w2 + k0, a.K - k0, wv_, wv2);
+      load8<float>(x + k0, a.K - k0, xv_, xv);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        acc = fmaf(xv[i], wv[i], acc);
+        if (DUAL) acc2 = fmaf(xv[i], wv2[i], acc2);
+      }
+    };
+    if (w_vec && x_vec) {   // (K % 8 == 0: every piece is whole)
+#pragma unroll 2
+      for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, true, true);
+    } else {
+      for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, w_vec, x_vec);
+    }
+    const float v = wave_sum(acc), v2 = DUAL ? wave_sum(acc2) : 0.f;
+    if (lane == 0) {
+      const int64_t yrow = a.y_rows ? a.y_rows[m] : m;
+      a.y[yrow * a.ldy + n] = finish<DUAL, EXT>(a, m, yrow, n, v, v2);
+    }
+  }
+}
+
 // Exact mode beyond a few rows.  The tile of gemm_any_f32_kernel: the largest of 64 x 64, 32 x 64, 32 x 32 whose grid puts a
 // workgroup on most of the 256 CUs; groups of less than 256 rows (an even share is assumed) in 32-row tiles, whose last one
 // is padded by less.  us, gemm_any_fma_kernel / here: 733 rows, K 1024: N 1024 64 / 17, N 3072 202 / 67, N 32 113 / 12; 32
@@ -687,6 +732,10 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
   const bool few = rows_per_group_max <= 8 || (mode == 1 && rows_per_group_max <= 64);
   if (few) {
     const int mt = rows_per_group_max <= 1 ? 1 : rows_per_group_max <= 4 ? 4 : 8;
+    if (a.group_offsets && mt > 1 && rows_per_group_max <= groups) {   // (a group of eight rows and more: over several workgroups)
+      hipLaunchKernelGGL((gemm_any_each_row_kernel<TW, DUAL, EXT>), dim3((a.N + 3) / 4, (rows_per_group_max + 7) / 8, groups), dim3(256), 0, st, a);
+      return check_launch();
+    }
     const int ft = !DUAL && mt > 1 && a.N >= 8192 ? 4 : 1;   // (a wave per four features: from two workgroups per CU on)
     const dim3 grid((a.N + 4 * ft - 1) / (4 * ft), (rows_per_group_max + mt - 1) / mt, groups);
     if constexpr (!DUAL)

@@ -66,3 +66,30 @@ def test_grouped_picks(ops, n, groups, keep, top):
         want = sorted(allowed, key=lambda e: (-s[e].item(), e))[:top]
         assert ids[t].tolist() == want
         assert (wts[t].cpu() - score[t][want]).abs().max() <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("counts", [(1, 0, 1, 1, 0, 0, 0, 1), (0, 4, 0, 0), (1,) * 8, (0, 0, 0, 0, 0, 0, 0, 8), (0, 11, 1) + (0,) * 11])
+@pytest.mark.parametrize("K", [8, 100, 1032])
+@pytest.mark.parametrize("dtype,exact", [(torch.bfloat16, False), (torch.bfloat16, True), (torch.float32, False)])
+@pytest.mark.parametrize("dual", [False, True])
+def test_groups_of_a_row_or_none(ops, counts, K, dtype, exact, dual):
+    """no more rows than groups: one row after the other (gemm_any_each_row_kernel); the order of sums is a plain product's of a row"""
+    G, N, P = len(counts), 21, sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(K + P)
+    x = torch.randn(5, K, device="cuda", generator=g)
+    rows = torch.randint(0, 5, (P,), device="cuda", generator=g, dtype=torch.int32)
+    place = torch.randperm(P, device="cuda", generator=g).to(torch.int32)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device="cuda")
+    w, w2 = ((torch.randn(G, N, K, device="cuda", generator=g) * K ** -0.5).to(dtype) for _ in range(2))
+    got = ops.gemm_any_grouped(x, rows, w, w2 if dual else None, off, P, place, P, exact)
+    for e in range(G):
+        for m in range(int(off[e]), int(off[e + 1])):
+            one = x[rows[m].long()][None]
+            if P > 8 and not exact:   # (only then is x rounded, and not here)
+                continue
+            z = ops.gemm_any(one, w[e], exact=True)[0]
+            if dual:
+                z = torch.nn.functional.silu(z.double()) * ops.gemm_any(one, w2[e], exact=True)[0].double()
+                assert ((got[place[m].long()].double() - z).abs() <= 2.0 ** -20 * z.abs() + 1e-12).all()
+            else:
+                assert torch.equal(got[place[m].long()], z)
