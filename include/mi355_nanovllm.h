@@ -313,7 +313,7 @@ int mi_pack_weight(const mi_bf16* w, mi_bf16* w_packed, int N, int K, mi_stream 
  * MergedColumnParallelLinear (linear.py:76-93) and y[M][N/2] = SiluAndMul (activation.py:10-12) of the product,
  * with the reference's three bf16 roundings.  K % 64 == 0, N % 4 == 0 (epilogue 1: N/2 % 128 == 0, no bias),
  * ldx % 8 == 0, ldy % 4 == 0.
- * Shapes whose tiles cannot fill the chip (few token rows x a narrow projection, e.g. 1024 x 1024 x 3072) are
+ * Shapes whose tiles cannot fill the chip (few token rows x a narrow projection, e.g. 200 x 1024 x 3072) are
  * computed as K slices into `workspace` (fp32, mi_gemm_bf16_workspace bytes; 0 = not needed for this shape) and
  * summed in slice order by a second launch - deterministic, one rounding.
  * The operands are addressed with 32-bit byte offsets: (N + 256) * K * 2 and (M + 256) * ldx * 2 must stay below 2^31.

@@ -32,7 +32,6 @@
 // Summation order: one fp32 MFMA chain over K per output element (k ascending), rounded to bf16 once -
 // the same rounding points as F.linear; the SwiGLU epilogue keeps the reference's three roundings
 // (bf16 gate_up output, bf16 silu, bf16 product).
-#include <algorithm>
 #include <type_traits>
 
 #include "mi_common.hpp"
@@ -512,9 +511,9 @@ struct MidPick {
   int tile, ksplit;
 };
 // fixed_ks: the caller wants that many slices' sums; 0: whatever is fastest, the sum of the slices included
-static MidPick pick_mid(int M, int N, int K, bool silu, int fixed_ks = 0, bool only128 = false) {
+static MidPick pick_mid(int M, int N, int K, bool silu, int fixed_ks = 0) {
   const int kt = K / BK;
-  const int shapes = only128 || M > 2048 ? 1 : silu ? 2 : 3;
+  const int shapes = M > 2048 ? 1 : silu ? 2 : 3;
   double best = 1e30;
   MidPick pick{0, 1};
   for (int i = 0; i < shapes; ++i) {
@@ -584,8 +583,7 @@ extern "C" int64_t mi_gemm_bf16_max_rows(int N, int K, int64_t ldx) {
 
 extern "C" size_t mi_gemm_bf16_workspace(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK || epilogue != 0) return 0;
-  // the most that a plan for the shape has: 128 x 128 tiles in K slices (the smaller tiles are often done without slices)
-  const int ks = use_mid(M, N, K) ? std::max(pick_mid(M, N, K, false).ksplit, pick_mid(M, N, K, false, 0, true).ksplit) : tile_ksplit(M, N, K);
+  const int ks = use_mid(M, N, K) ? pick_mid(M, N, K, false).ksplit : tile_ksplit(M, N, K);   // (mi_gemm_bf16's own plan)
   return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
 }
 

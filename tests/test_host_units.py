@@ -238,8 +238,10 @@ def test_c_abi_exports_every_declared_symbol_and_rejects_bad_arguments():
     assert _C.lib.mi_gemm_bf16(1 << 20, 96, 1 << 20, None, 1 << 20, 64, 128, 64, 96, 0, None, 0, None) == -2  # K % 64
     assert _C.lib.mi_gemm_bf16(1 << 20, 64, 1 << 20, None, 1 << 20, 64, 128, 64, 64, 2, None, 0, None) == -1  # epilogue
     assert _C.lib.mi_gemm_bf16_workspace(16384, 4096, 1024, 0) == 0           # plenty of tiles: no K slices
-    ws = _C.lib.mi_gemm_bf16_workspace(1024, 1024, 3072, 0)  # 64 tiles of 128 x 128, 48 K steps: summed in K slices
-    assert ws % (1024 * 1024 * 4) == 0 and ws // (1024 * 1024 * 4) in (2, 4, 8, 16)
+    ws = _C.lib.mi_gemm_bf16_workspace(200, 1024, 3072, 0)  # 64 tiles of 64 x 64, 48 K steps: summed in K slices
+    assert ws % (200 * 1024 * 4) == 0 and ws // (200 * 1024 * 4) in (2, 4, 8, 16)
+    # ... and a workspace is asked for where mi_gemm_bf16 sums slices, not where it could: 256 tiles, 64 over 32 K steps
+    assert _C.lib.mi_gemm_bf16_workspace(1024, 1024, 3072, 0) == 0 and _C.lib.mi_gemm_bf16_workspace(200, 1024, 2048, 0) == 0
     assert _C.lib.mi_paged_attn_decode_workspace(32, 16) == 32 * 16 * 16 * 130 * 4
     # the Python side asks the library for mi_gemm_bf16's shape contract instead of restating it.  M = 0
     # makes mi_gemm_bf16 return its contract check without launching: both must agree on the weight side ...
