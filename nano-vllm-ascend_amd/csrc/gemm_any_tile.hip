@@ -175,7 +175,7 @@ template <int ACT, bool DUAL>
 static int launch_any_tile(const AnyTileArgs<ACT, DUAL>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
   using A = AnyTileArgs<ACT, DUAL>;
   A a = args;
-  if (tile_rows == 256 && ACT != MI_ACT_SOFTCAP) {
+  if (tile_rows == 256) {
     a.tiles_f = (a.N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
     a.tiles_t = (a.M + 255) / 256;
     const int64_t tiles = row_tiles_max * a.tiles_f;
@@ -243,6 +243,7 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
                                 const int32_t* y_rows, int rows, int N, int K, float alpha, mi_stream stream) {
   if (!xb || !w || !y || rows < 0 || (n_groups > 0) != (table != nullptr) || (row_scale_rows && !row_scale)) return MI_EINVAL;
   if (act == MI_ACT_CLAMPED_GLU && !(limit > 0.f)) return MI_EINVAL;
+  if (act == MI_ACT_SOFTCAP && tile_rows == 256) return MI_EUNSUPPORTED;   // (launch_any_tile)
   if (rows == 0) return MI_OK;
   if (!tile_rows_ok(tile_rows)) return MI_EINVAL;
   if (tile_rows_for(rows, N, K, n_groups, w2 != nullptr, act) == 0) return MI_EUNSUPPORTED;

@@ -55,3 +55,12 @@ def test_few_rows_per_group_stay_on_the_kernel_that_does_not_round_them():
     w = torch.zeros(64, 64, 64, dtype=torch.bfloat16)
     assert ops._grouped_tile_rows(512, 9, w, None, _C.ACT_NONE, False)
     assert not ops._grouped_tile_rows(512, 8, w, None, _C.ACT_NONE, False)
+
+
+def test_soft_capped_products_have_no_256_row_tiles():
+    """mi_gemm_any_tile: tiles of 256 rows are the persistent kernel's, which has no soft-capped form (no rows: nothing is launched)"""
+    p, run = 1 << 20, _C.lib.mi_gemm_any_tile
+    args = lambda act, tile, rows: (p, None, tile, p, None, None, None, act, 0.0, None, None, 0, p, 0, 8192, None, rows, 8192, 64, 30.0, None)
+    assert run(*args(_C.ACT_SOFTCAP, 256, 0)) == -2
+    for act, tile in ((_C.ACT_SOFTCAP, 128), (_C.ACT_SOFTCAP, 64), (_C.ACT_NONE, 256)):
+        assert run(*args(act, tile, 0)) == 0
