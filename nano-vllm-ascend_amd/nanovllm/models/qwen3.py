@@ -215,6 +215,11 @@ class Qwen3DecoderLayer(nn.Module):
         return hidden_states, residual
 
 
+def _env_int(name: str) -> int | None:
+    value = os.environ.get(name)
+    return None if value is None else int(value)
+
+
 class Qwen3Model(nn.Module):
     def __init__(self, config, fused: bool = True, layer_factory=None, **layer_overrides) -> None:
         """layer_factory(layer_idx) -> decoder layer: models whose layers differ (Qwen3-MoE) build ONLY their own
@@ -230,14 +235,17 @@ class Qwen3Model(nn.Module):
     # module-by-module path on the tile GEMMs.  Above 64 rows the dense bf16 projections of the streaming path are tile GEMMs too,
     # the narrow ones in K slices that the norm adds up (ms per captured step of a Qwen3-0.6B-shaped model, streaming / module path:
     # 130 tokens 1.51 / 1.66, 256: 1.65 / 1.83, 512: 2.20 / 2.40, 8 x 64: 1.94 / 2.15); fp8 weights, experts and ranks still read
-    # their weights once per 64 rows there and stay at 128 (192 tokens, before: 2.11 / 1.98).
-    PREFILL_STREAM_MAX = int(os.environ.get("MI355_PREFILL_STREAM_MAX", "512"))
+    # their weights once per 64 rows there and stay at 128 (192 tokens, before: 2.11 / 1.98).  MI355_PREFILL_STREAM_MAX, where it is set,
+    # holds for all of them.
+    PREFILL_STREAM_MAX: int | None = _env_int("MI355_PREFILL_STREAM_MAX")
 
     def _prefill_stream_max(self) -> int:
+        if self.PREFILL_STREAM_MAX is not None:
+            return min(ops.SKINNY_MAX_M, self.PREFILL_STREAM_MAX)
         l0 = self.layers[0]
         tile = (tp_size() == 1 and not collectives_on() and not isinstance(l0.self_attn.qkv_proj.weight_packed, ops.Fp8Weight)
                 and not any(hasattr(l.mlp, "experts") for l in self.layers))
-        return min(ops.SKINNY_MAX_M, self.PREFILL_STREAM_MAX if tile else min(self.PREFILL_STREAM_MAX, 128))
+        return min(ops.SKINNY_MAX_M, 512 if tile else 128)
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         limit = self._prefill_stream_max() if get_context().is_prefill else ops.SKINNY_MAX_M

@@ -1237,3 +1237,25 @@ def test_exchange_region_cap_for_eager_launches_and_the_scope_that_lifts_it():
     assert comm._large == 0 and not comm.fits_rows(112, 2048)
     comm.eager_max_bytes = comm.max_bytes  # (MI355_XGMI_EAGER_LARGE=1: the bring-up switch)
     assert comm.fits_rows(512, 2048)
+
+
+@pytest.mark.parametrize("kind", ["dense", "fp8", "experts", "ranks"])
+@pytest.mark.parametrize("said", [None, 64, 128, 200, 4096])
+def test_prefill_stream_limit_is_the_users_where_one_is_given(monkeypatch, kind, said):
+    """MI355_PREFILL_STREAM_MAX holds for every model; unset: 512 tokens where the projections above 64 rows are tile GEMMs, else 128."""
+    import types
+
+    from nanovllm import ops
+    from nanovllm.models import qwen3
+
+    monkeypatch.setattr(qwen3, "tp_size", lambda: 2 if kind == "ranks" else 1)
+    monkeypatch.setattr(qwen3, "collectives_on", lambda: kind == "ranks")
+    packed = object.__new__(ops.Fp8Weight) if kind == "fp8" else object()
+    mlp = types.SimpleNamespace(experts=1) if kind == "experts" else types.SimpleNamespace()
+    layer = types.SimpleNamespace(self_attn=types.SimpleNamespace(qkv_proj=types.SimpleNamespace(weight_packed=packed)), mlp=mlp)
+    model = types.SimpleNamespace(layers=[layer], PREFILL_STREAM_MAX=qwen3._env_int("MI355_PREFILL_STREAM_MAX_UNSET"))
+    if said is not None:
+        monkeypatch.setenv("MI355_PREFILL_STREAM_MAX", str(said))
+        model.PREFILL_STREAM_MAX = qwen3._env_int("MI355_PREFILL_STREAM_MAX")
+    want = (512 if kind == "dense" else 128) if said is None else min(said, ops.SKINNY_MAX_M)
+    assert qwen3.Qwen3Model._prefill_stream_max(model) == want
