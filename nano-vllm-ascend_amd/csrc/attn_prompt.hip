@@ -29,8 +29,8 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // up to 32 DKM key and 16 DVM value channels; smaller heads are zero-padded to that in the images: a branch per fragment would put
 // every fragment's LDS latency behind the one before.  VIK: the values are the leading channels of the key rows.  PAGED16: pages
-// of a multiple of 16 rows.
-template <typename TC, int DKM, int DVM, int NST, bool VIK, bool PAGED16>
+// of a multiple of 16 rows.  V4: value rows that start on 4 bytes only (bf16, an even stride), requested in 4-byte pieces.
+template <typename TC, int DKM, int DVM, int NST, bool VIK, bool PAGED16, bool V4 = false>
 __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
     const float* __restrict__ q, int64_t ldq, const TC* __restrict__ k_cache, const TC* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, int table_cols, const int32_t* __restrict__ cu_q,
@@ -44,6 +44,7 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
   // LDS-DMA instructions of 1 KiB; PP per wave, all of one operand and of one half (16 keys) of the step
   constexpr int KP = KB / 1024, VP = VB / 1024, PP = (KP + VP + kWaves - 1) / kWaves <= 2 ? (KP + VP + kWaves - 1) / kWaves
                                                      : (KP + VP <= 32 ? 4 : 8);
+  static_assert(!V4 || (BF && !VIK), "see above");
   static_assert(KP / 2 % PP == 0 && VP / 2 % PP == 0 && KP + VP <= PP * kWaves && (NST & (NST - 1)) == 0, "see above");
   __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE];
   // the chunk that lies at position p of row r is p ^ swizzle(r): sixteen rows at one chunk (a K fragment) and four or eight
@@ -111,20 +112,26 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                          (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 0);
     };
-    if constexpr (PAGED16) {
-      const int k0 = half_key(u);
-      const TC* base = cache + ((int64_t)((uint32_t)pg * heads + head) * block_size + (k0 - blk_of(k0) * block_size)) * ldr;
-      if (u + kKeys - 1 <= hi_key) {
+    const int k0 = half_key(u);   // (PAGED16)
+    const TC* base = cache + ((int64_t)((uint32_t)pg * heads + head) * block_size + (k0 - blk_of(k0) * block_size)) * ldr;
+    auto row_at = [&](int r) __attribute__((always_inline)) {   // row r of the step
+      const int key = min(u + r, hi_key);
+      return PAGED16 ? base + (key - k0) * ldr : cache + (int64_t)cache_row(table, key, heads, head, block_size, bs_shift) * ldr;
+    };
+    if (V4 && is_v) {
 #pragma unroll
-        for (int i = 0; i < PP; ++i) dma(base + poff[i], i);
-      } else {
-#pragma unroll
-        for (int i = 0; i < PP; ++i) dma(base + (min(u + prow[i], hi_key) - k0) * ldr + pchan[i], i);
+      for (int i = 0; i < PP * 4; ++i) {
+        const int at = (p0 - KP) * 1024 + i * 256 + lane * 4, r = at / VROW, c = ((at % VROW / 16) ^ swizzle(r, VROW)) * VEC + (at & 15) / 2;
+        if (c < Dv)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row_at(r) + c),
+                                           (__attribute__((address_space(3))) void*)(dst + i * 256), 4, 0, 0);
       }
+    } else if (PAGED16 && u + kKeys - 1 <= hi_key) {
+#pragma unroll
+      for (int i = 0; i < PP; ++i) dma(base + poff[i], i);
     } else {
 #pragma unroll
-      for (int i = 0; i < PP; ++i)
-        dma(cache + (int64_t)cache_row(table, min(u + prow[i], hi_key), heads, head, block_size, bs_shift) * ldr + pchan[i], i);
+      for (int i = 0; i < PP; ++i) dma(row_at(prow[i]) + pchan[i], i);
     }
   };
 
@@ -194,7 +201,9 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
     }
   for (int k = 0; k < n_steps; ++k, u0 = next_step(u0)) {
     const int behind = min(n_steps - 1 - k, NST - 2);   // steps requested behind this one: their pieces may still fly
-    if (NST > 2 && behind == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PP) : "memory");
+    if (V4 && is_v && NST > 2 && behind == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(8 * PP) : "memory");
+    else if (V4 && is_v && NST > 2 && behind == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(4 * PP) : "memory");
+    else if (NST > 2 && behind == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PP) : "memory");
     else if (NST > 2 && behind == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PP) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -337,7 +346,7 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
                             int Dv, int block_size, int window, float scale, const AttnBias& bias, int64_t ldv,
                             const float* gate, int64_t ldg, float* out, int64_t ldo, hipStream_t st) {
   const int vec = bf16 ? 8 : 4;
-  if (D % (bf16 ? 32 : 16) || Dv % 16 || D > 256 || Dv > 256 || ldv % vec || !aligned16(k_cache) || !aligned16(v_cache) || G > 65535)
+  if (D % (bf16 ? 32 : 16) || Dv % 16 || D > 256 || Dv > 256 || ldv % (bf16 ? 2 : vec) || !aligned16(k_cache) || !aligned16(v_cache) || G > 65535)
     return MI_EUNSUPPORTED;
   const int hpg = H / G, heads = hpg < kCols ? hpg : kCols, R = kCols / heads;
   const int64_t tiles = rows / R + n_seqs;
@@ -348,12 +357,19 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   // and V through registers into the image (V transposed on the way): 345, 104, 86.
   const bool vik = k_cache == v_cache && bias.value_heads == G && ldv == D && Dv <= D;
   const bool paged16 = block_size % 16 == 0;
-#define MI_PROMPT(TC, DKM, DVM, NST, VIK, PAGED16)                                                                         \
-  hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, VIK, PAGED16>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
+#define MI_PROMPT(TC, DKM, DVM, NST, ...)                                                                                  \
+  hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
                      static_cast<const TC*>(k_cache), static_cast<const TC*>(v_cache), bt, cols, cu_q, kv_lens, n_seqs, H, G, D, Dv, \
                      block_size, window, scale, bias, ldv, gate, ldg, out, ldo)
   if (bf16) {
-    if (!paged16) MI_PROMPT(uint16_t, 8, 16, 4, false, false);
+    // value rows on 4 bytes (us, the kernel before / element by element / so: 8 x 1024 rows, 8 / 4 heads x 128, window 512 199 / 2440 / 85;
+    // 4 x 1024 rows, 16 heads over one of 256 channels 428 / 3580 / 224; 4 x 300 rows, 8 / 4 heads x 64 and 48 34 / 165 / 18)
+    if (ldv % vec) {
+      if (!paged16) MI_PROMPT(uint16_t, 8, 16, 4, false, false, true);
+      else if (D <= 64 && Dv <= 64) MI_PROMPT(uint16_t, 2, 4, 4, false, true, true);
+      else if (D <= 128 && Dv <= 128) MI_PROMPT(uint16_t, 4, 8, 4, false, true, true);
+      else MI_PROMPT(uint16_t, 8, 16, 4, false, true, true);
+    } else if (!paged16) MI_PROMPT(uint16_t, 8, 16, 4, false, false);
     else if (D <= 64 && Dv <= 64) MI_PROMPT(uint16_t, 2, 4, 4, false, true);
     else if (D <= 64 && Dv <= 128) MI_PROMPT(uint16_t, 2, 8, 4, false, true);
     else if (D <= 128 && Dv <= 128) MI_PROMPT(uint16_t, 4, 8, 4, false, true);

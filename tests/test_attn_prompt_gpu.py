@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _case(dtype, H, G, D, Dv, block, seqs, window=2 ** 31 - 1, kept=0, chunk=0, softcap=0.0, sink=False, bias=_C.BIAS_NONE, vik=False,
-          gate=False, value_heads=None):
+          gate=False, value_heads=None, pad=0):
     g = torch.Generator(device="cuda").manual_seed(H * 131 + D * 7 + Dv + block + len(seqs))
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
     Gv = value_heads or G
@@ -26,7 +26,7 @@ def _case(dtype, H, G, D, Dv, block, seqs, window=2 ** 31 - 1, kept=0, chunk=0, 
         table[i, :n] = order[at:at + n]
         at += n
     k_cache = torch.full((len(order), G, block, D), float("nan"), device="cuda").to(dtype)   # rows nobody wrote stay NaN
-    v_cache = k_cache if vik else torch.full((len(order), Gv, block, Dv), float("nan"), device="cuda").to(dtype)
+    v_cache = k_cache if vik else torch.full((len(order), Gv, block, Dv + pad), float("nan"), device="cuda").to(dtype)
     ks, vs = [], []
     for i, (a, n) in enumerate(seqs):
         p = torch.arange(a + n, device="cuda")
@@ -34,7 +34,7 @@ def _case(dtype, H, G, D, Dv, block, seqs, window=2 ** 31 - 1, kept=0, chunk=0, 
         k_cache[table[i, p // block].long(), :, p % block] = k
         if not vik:
             v = rnd(a + n, Gv, Dv).to(dtype)
-            v_cache[table[i, p // block].long(), :, p % block] = v
+            v_cache[table[i, p // block].long(), :, p % block, :Dv] = v
         ks.append(k.double())
         vs.append(k.double()[..., :Dv] if vik else v.double())
     rows = sum(n for _, n in seqs)
@@ -44,7 +44,7 @@ def _case(dtype, H, G, D, Dv, block, seqs, window=2 ** 31 - 1, kept=0, chunk=0, 
     sk = rnd(H) if sink else None
     p1, p2 = (torch.rand(H, device="cuda", generator=g), torch.rand(H, device="cuda", generator=g)) if bias == _C.BIAS_LOG else (None, None)
     scale = D ** -0.5
-    got = ops.paged_attention_f32(q, k_cache, v_cache, D if vik else Dv, table, cu, kv, H, G, D, Dv, block, window, scale, bias, p1, p2,
+    got = ops.paged_attention_f32(q, k_cache, v_cache, D if vik else Dv + pad, table, cu, kv, H, G, D, Dv, block, window, scale, bias, p1, p2,
                                   gate=gt, sink=sk, softcap=softcap, chunk=chunk, kept=kept, value_heads=Gv)
     want = torch.empty(rows, H, Dv, dtype=torch.float64, device="cuda")
     for i, (a, n) in enumerate(seqs):
@@ -98,3 +98,11 @@ def test_masks_and_biases(dtype, form):
 @pytest.mark.parametrize("D,Dv", [(256, 256), (224, 160)])
 def test_values_inside_the_key_rows(dtype, D, Dv):
     _case(dtype, 16, 1, D, Dv, 64, SEQS, vik=True, sink=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("pad", [1, 2, 4, 6, 8])
+@pytest.mark.parametrize("H,G,D,Dv,block", [(4, 2, 64, 64, 16), (6, 1, 128, 48, 24), (2, 2, 256, 256, 64)])
+def test_value_rows_of_any_stride(dtype, pad, H, G, D, Dv, block):
+    """even strides of bf16 value rows stay on the matrix cores, odd ones go element by element"""
+    _case(dtype, H, G, D, Dv, block, SEQS, window=60, pad=pad, gate=True)
