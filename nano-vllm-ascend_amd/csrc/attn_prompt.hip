@@ -19,6 +19,9 @@
 // KiB of fragments per 16 columns and 32 keys at 256 channels) where it is long.  The kernels it replaces - a wave per 16
 // columns with K and V from L2 by every wave and V in 4-byte gathers; over fp32 rows plain FMA chains - waited for memory.
 // Measured: see launch_prompt_attention.
+//
+// Keys that a column does not see weigh 0 in its products, and 0 times a NaN or an infinity among their values is NaN: a column whose
+// result is not finite is taken again without them (attend_column; the look at the results costs 0.6 us of a launch).
 #include "attn_bias.hpp"
 
 namespace mi {
@@ -26,6 +29,51 @@ namespace mi {
 constexpr int kCols = 128, kKeys = 32, kPromptThreads = 512, kWaves = 8;
 constexpr float kLog2e = 1.44269504088896340736f;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// One column by one wave, keys it does not see left out instead of weighed with 0: for columns that the matrix instructions gave
+// something that is not finite, because a key of their step that they do not see has a NaN or an infinity among its values.
+template <typename TC>
+__device__ __forceinline__ void attend_column(const float* q, const TC* k_cache, const TC* v_cache, const int32_t* table, int pos, int h, int H,
+                                              int G, int D, int Dv, int block_size, int window, float scale, const AttnBias& bias, int64_t ldv,
+                                              const float* gate, float* out) {
+  const int lane = threadIdx.x & 63, g = h / (H / G), Gv = bias.value_heads, gv = h / (H / Gv), bs_shift = block_shift(block_size);
+  const int lo = first_key(bias, pos, window), gap = kept_gap(bias, lo);
+  const HeadBias hb = head_bias(bias, h, H);
+  float m = -INFINITY, l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};   // (Dv <= 256)
+  for (int j0 = gap; j0 <= pos; j0 += 64) {
+    const int j = key_at<true>(j0 + lane, lo, gap);
+    float sc = -INFINITY;
+    if (j <= pos) {
+      const TC* kr = k_cache + (int64_t)cache_row(table, j, G, g, block_size, bs_shift) * D;
+      float dot = 0.f;
+#pragma unroll 1
+      for (int d = 0; d < D; ++d) dot = fmaf(q[d], ld_f<TC>(kr + d), dot);
+      sc = capped(bias, dot * scale - dist_bias(hb, pos - j));
+    }
+    const float m_new = fmaxf(m, wave_max(sc));
+    const float mref = m_new == -INFINITY ? 0.f : m_new;
+    const float p = j <= pos ? expf(sc - mref) : 0.f, corr = expf(m - mref);
+    l = l * corr + wave_sum(p);
+    m = m_new;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] *= corr;
+    const int n = min(64, pos - j0 + 1);
+#pragma unroll 1
+    for (int jj = 0; jj < n; ++jj) {
+      const float pj = __shfl(p, jj);
+      const TC* vr = v_cache + (int64_t)cache_row(table, key_at<true>(j0 + jj, lo, gap), Gv, gv, block_size, bs_shift) * ldv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (lane + 64 * i < Dv) acc[i] = fmaf(pj, ld_f<TC>(vr + lane + 64 * i), acc[i]);
+    }
+  }
+  const float inv = 1.f / with_sink(bias, h, m, l);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int d = lane + 64 * i;
+    if (d < Dv) out[d] = acc[i] * inv * (gate ? sigmoid_f(gate[d]) : 1.f);
+  }
+}
 
 // up to 32 DKM key and 16 DVM value channels; smaller heads are zero-padded to that in the images: a branch per fragment would put
 // every fragment's LDS latency behind the one before.  VIK: the values are the leading channels of the key rows.  PAGED16: pages
@@ -314,7 +362,6 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
     }
   }
 
-  if (!live) return;
   // the lane holds channels 16 f + 4 kg + {0..3} of its column
   const float inv = 1.f / (bias.sink ? l + __builtin_amdgcn_exp2f(bias.sink[ch] * kLog2e - m) : l);
   const int64_t row = first + crow;
@@ -322,10 +369,13 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
   const float* gp = gate ? gate + row * ldg + (int64_t)ch * Dv + kg * 4 : nullptr;
   const bool ovec = (ldo % 4 == 0) && ((reinterpret_cast<uintptr_t>(out) & 15u) == 0);
   const bool gvec = gate && (ldg % 4 == 0) && ((reinterpret_cast<uintptr_t>(gate) & 15u) == 0);
+  f32x4 zero = {0.f, 0.f, 0.f, 0.f};   // (zero times the results: NaN where one of them is not finite)
 #pragma unroll
   for (int f = 0; f < DVM; ++f) {
-    if (f < dvt) {
+    if (live && f < dvt) {
       f32x4 o = oacc[f] * inv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zero[e] = fmaf(oacc[f][e], 0.f, zero[e]);
       if (gate) {
         const f32x4 z = gvec ? *reinterpret_cast<const f32x4*>(gp + f * 16) : f32x4{gp[f * 16], gp[f * 16 + 1], gp[f * 16 + 2], gp[f * 16 + 3]};
 #pragma unroll
@@ -338,6 +388,18 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
         for (int e = 0; e < 4; ++e) op[f * 16 + e] = o[e];
       }
     }
+  }
+  const float odd = (zero[0] + zero[1]) + (zero[2] + zero[3]);
+  uint64_t todo = __ballot(live && odd != 0.f);
+  if (todo == 0) return;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // (the columns above are home before they are written again)
+  __builtin_amdgcn_wave_barrier();
+  while (todo) {
+    const int r = __builtin_ctzll(todo) & 15, cr = (wave * 16 + r) / nh, c_ch = g * hpg + h0 + (wave * 16 + r - cr * nh);
+    todo &= ~(0x0001000100010001ull << r);   // (a column's four lanes)
+    const int64_t at = first + cr;
+    attend_column<TC>(q + at * ldq + (int64_t)c_ch * D, k_cache, v_cache, table, pos0 + cr, c_ch, H, G, D, Dv, block_size, window, scale, bias, ldv,
+                      gate ? gate + at * ldg + (int64_t)c_ch * Dv : nullptr, out + at * ldo + (int64_t)c_ch * Dv);
   }
 }
 

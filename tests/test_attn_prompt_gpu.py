@@ -106,3 +106,37 @@ def test_values_inside_the_key_rows(dtype, D, Dv):
 def test_value_rows_of_any_stride(dtype, pad, H, G, D, Dv, block):
     """even strides of bf16 value rows stay on the matrix cores, odd ones go element by element"""
     _case(dtype, H, G, D, Dv, block, SEQS, window=60, pad=pad, gate=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["k", "v"])
+@pytest.mark.parametrize("H,G,D,Dv,vik,window,kept", [(4, 2, 64, 64, False, 2 ** 31 - 1, 0), (8, 4, 128, 128, False, 50, 3), (3, 1, 256, 256, True, 40, 0),
+                                                      (2, 2, 96, 48, False, 64, 0)])
+def test_keys_and_values_that_are_not_finite_reach_the_rows_that_see_them(dtype, value, where, H, G, D, Dv, vik, window, kept):
+    """one such key or value row at position 40 of 150: rows in front of it, and rows whose window has passed it, are as without it"""
+    if vik and where == "v":
+        pytest.skip("the values are the keys")
+    n, bad, block = 150, 40, 16
+    g = torch.Generator(device="cuda").manual_seed(D)
+    k, v = (torch.randn(10, G, block, d, device="cuda", generator=g).to(dtype) for d in (D, Dv))
+    v = k if vik else v
+    q = torch.randn(n, H * D, device="cuda", generator=g)
+    table = torch.randperm(10, device="cuda", generator=g).int().view(1, 10)
+    cu, kv = torch.tensor([0, n], dtype=torch.int32, device="cuda"), torch.tensor([n], dtype=torch.int32, device="cuda")
+
+    def call():
+        return ops.paged_attention_f32(q, k, v, Dv, table, cu, kv, H, G, D, Dv, block, window, D ** -0.5, kept=kept)
+
+    clean = call()
+    (k if where == "k" else v)[table[0, bad // block].long(), G - 1, bad % block, 5] = value
+    got = call()
+    pos = torch.arange(n, device="cuda")
+    sees = (pos >= bad) & (pos - bad < window)
+    heads = (torch.arange(H, device="cuda") // (H // G) == G - 1).repeat_interleave(Dv)
+    channel = torch.arange(H * Dv, device="cuda") % Dv == 5
+    hit = sees.view(-1, 1) & (heads & channel if where == "v" else heads).view(1, -1)
+    tol = 2 * (2e-5 if dtype == torch.bfloat16 else 1e-5) * float(clean.abs().max())   # (two results, each within the bound above)
+    assert torch.isfinite(got[~hit]).all() and float((got - clean)[~hit].abs().max()) <= tol
+    if where == "v" or value != value:   # (an infinite key may just weigh nothing: -inf)
+        assert not torch.isfinite(got[hit]).any()
