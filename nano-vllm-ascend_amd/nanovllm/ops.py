@@ -1080,6 +1080,7 @@ def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_in
         _f32(x, row_scale)
         _i32(pair_token, pair_index, offsets, row_scale_rows)
         assert x.shape[1] == width and down.shape == (G, width, ff) and offsets.numel() > G
+        assert row_scale is None or row_scale.is_contiguous()
         assert w.is_contiguous() and down.is_contiguous() and (w2 is None or (w2.shape == w.shape and w2.is_contiguous() and w2.dtype == _BF16))
         scratch = torch.empty(n, dtype=torch.uint8, device=x.device)
         y = torch.empty((pairs, width), dtype=_F32, device=x.device)

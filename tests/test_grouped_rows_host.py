@@ -13,22 +13,27 @@ class _Recorder:
         self.lib, self.calls = lib, {}
 
     def __getattr__(self, name):
-        if name not in ("mi_gemm_any_operand", "mi_gemm_any_tile"):
+        if name not in ("mi_gemm_any_operand", "mi_gemm_any_tile", "mi_expert_ff"):
             return getattr(self.lib, name)
-        return lambda *a: self.calls.setdefault(name, a) and 0
+        return lambda *a: self.calls.__setitem__(name, a) or 0
+
+
+@pytest.fixture
+def recorded(monkeypatch):
+    rec = _Recorder(_C.lib)
+    monkeypatch.setattr(ops, "lib", rec)
+    monkeypatch.setattr(ops, "require_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "stream", lambda: 0)
+    return rec.calls
 
 
 @pytest.mark.parametrize("name", ["gemm_any_grouped", "gemm_any_grouped_act", "gemm_any_grouped_glu"])
 @pytest.mark.parametrize("gathered", [False, True])
 @pytest.mark.parametrize("counts", [(200,) * 8, (9, 0, 300, 1)])
-def test_rows_of_all_groups(monkeypatch, name, gathered, counts):
+def test_rows_of_all_groups(monkeypatch, recorded, name, gathered, counts):
     G, N, K, total = len(counts), 64, 64, sum(counts)
-    rec = _Recorder(_C.lib)
     made = []
     empty = torch.empty
-    monkeypatch.setattr(ops, "lib", rec)
-    monkeypatch.setattr(ops, "require_gpu", lambda *a: None)
-    monkeypatch.setattr(ops, "stream", lambda: 0)
     monkeypatch.setattr(ops.torch, "empty", lambda *a, **k: made.append(empty(*a, **k)) or made[-1])
     w = torch.zeros(G, N, K, dtype=torch.bfloat16)
     off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32)
@@ -42,7 +47,7 @@ def test_rows_of_all_groups(monkeypatch, name, gathered, counts):
         ops.gemm_any_grouped_act(x, x_rows, w, None, _C.ACT_NONE, off, most, y_rows, total)
     else:
         ops.gemm_any_grouped_glu(x, x_rows, w, None, _C.ACT_NONE, 0.0, None, None, off, most, y_rows, total)
-    operand, tile = rec.calls["mi_gemm_any_operand"], rec.calls["mi_gemm_any_tile"]
+    operand, tile = recorded["mi_gemm_any_operand"], recorded["mi_gemm_any_tile"]
     tile_rows, rows = operand[5], operand[6]
     assert rows >= total and tile[16] >= total
     xb = next(t for t in made if t.data_ptr() == operand[8])
@@ -64,3 +69,17 @@ def test_soft_capped_products_have_no_256_row_tiles():
     assert run(*args(_C.ACT_SOFTCAP, 256, 0)) == -2
     for act, tile in ((_C.ACT_SOFTCAP, 128), (_C.ACT_SOFTCAP, 64), (_C.ACT_NONE, 256)):
         assert run(*args(act, tile, 0)) == 0
+
+
+def test_expert_feed_forward_takes_the_operands_that_the_two_products_take(recorded):
+    """a scale per pair is read as it lies in memory: strided ones are refused by both routes"""
+    G, T, top, W, ff = 4, 10, 2, 64, 64
+    x, gate, down = torch.zeros(T, W), torch.zeros(G, ff, W, dtype=torch.bfloat16), torch.zeros(G, W, ff, dtype=torch.bfloat16)
+    i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
+    args = (x, i32(T * top), gate, gate, down, _C.ACT_CLAMPED_GLU, i32(G + 1), T * top, i32(T * top), 7.0)
+    ops.expert_ff(*args, torch.ones(T, top), i32(T * top))
+    assert "mi_expert_ff" in recorded
+    recorded.clear()
+    with pytest.raises(AssertionError):
+        ops.expert_ff(*args, torch.ones(T, 2 * top)[:, :top], i32(T * top))
+    assert not recorded
