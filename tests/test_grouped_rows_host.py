@@ -73,7 +73,7 @@ def test_soft_capped_products_have_no_256_row_tiles():
 
 def test_expert_feed_forward_takes_the_operands_that_the_two_products_take(recorded):
     """a scale per pair is read as it lies in memory: strided ones are refused by both routes"""
-    G, T, top, W, ff = 4, 10, 2, 64, 64
+    G, T, top, W, ff = 4, 10, 2, 256, 256
     x, gate, down = torch.zeros(T, W), torch.zeros(G, ff, W, dtype=torch.bfloat16), torch.zeros(G, W, ff, dtype=torch.bfloat16)
     i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
     args = (x, i32(T * top), gate, gate, down, _C.ACT_CLAMPED_GLU, i32(G + 1), T * top, i32(T * top), 7.0)
