@@ -423,28 +423,30 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
                      static_cast<const TC*>(k_cache), static_cast<const TC*>(v_cache), bt, cols, cu_q, kv_lens, n_seqs, H, G, D, Dv, \
                      block_size, window, scale, bias, ldv, gate, ldg, out, ldo)
-  if (bf16) {
+  // (WIDE: stages of the ring at 256 channels of keys and of values)
+#define MI_PROMPT_SIZES(TC, PAGED16, WIDE)                                   \
+  do {                                                                       \
+    if (D <= 64 && Dv <= 64) MI_PROMPT(TC, 2, 4, 4, false, PAGED16);         \
+    else if (D <= 64 && Dv <= 128) MI_PROMPT(TC, 2, 8, 4, false, PAGED16);   \
+    else if (D <= 128 && Dv <= 128) MI_PROMPT(TC, 4, 8, 4, false, PAGED16);  \
+    else if (vik) MI_PROMPT(TC, 8, 16, 4, true, PAGED16);                    \
+    else MI_PROMPT(TC, 8, 16, WIDE, false, PAGED16);                         \
+  } while (0)
+  if (bf16 && ldv % vec) {
     // value rows on 4 bytes (us, the kernel before / element by element / so: 8 x 1024 rows, 8 / 4 heads x 128, window 512 199 / 2440 / 85;
     // 4 x 1024 rows, 16 heads over one of 256 channels 428 / 3580 / 224; 4 x 300 rows, 8 / 4 heads x 64 and 48 34 / 165 / 18)
-    if (ldv % vec) {
-      if (!paged16) MI_PROMPT(uint16_t, 8, 16, 4, false, false, true);
-      else if (D <= 64 && Dv <= 64) MI_PROMPT(uint16_t, 2, 4, 4, false, true, true);
-      else if (D <= 128 && Dv <= 128) MI_PROMPT(uint16_t, 4, 8, 4, false, true, true);
-      else MI_PROMPT(uint16_t, 8, 16, 4, false, true, true);
-    } else if (!paged16) MI_PROMPT(uint16_t, 8, 16, 4, false, false);
-    else if (D <= 64 && Dv <= 64) MI_PROMPT(uint16_t, 2, 4, 4, false, true);
-    else if (D <= 64 && Dv <= 128) MI_PROMPT(uint16_t, 2, 8, 4, false, true);
-    else if (D <= 128 && Dv <= 128) MI_PROMPT(uint16_t, 4, 8, 4, false, true);
-    else if (vik) MI_PROMPT(uint16_t, 8, 16, 4, true, true);
-    else MI_PROMPT(uint16_t, 8, 16, 4, false, true);
+    if (!paged16) MI_PROMPT(uint16_t, 8, 16, 4, false, false, true);
+    else if (D <= 64 && Dv <= 64) MI_PROMPT(uint16_t, 2, 4, 4, false, true, true);
+    else if (D <= 128 && Dv <= 128) MI_PROMPT(uint16_t, 4, 8, 4, false, true, true);
+    else MI_PROMPT(uint16_t, 8, 16, 4, false, true, true);
+  } else if (bf16) {
+    if (paged16) MI_PROMPT_SIZES(uint16_t, true, 4);
+    else MI_PROMPT_SIZES(uint16_t, false, 4);
   } else {
-    if (!paged16) MI_PROMPT(float, 8, 16, 2, false, false);
-    else if (D <= 64 && Dv <= 64) MI_PROMPT(float, 2, 4, 4, false, true);
-    else if (D <= 64 && Dv <= 128) MI_PROMPT(float, 2, 8, 4, false, true);
-    else if (D <= 128 && Dv <= 128) MI_PROMPT(float, 4, 8, 4, false, true);
-    else if (vik) MI_PROMPT(float, 8, 16, 4, true, true);
-    else MI_PROMPT(float, 8, 16, 2, false, true);
+    if (paged16) MI_PROMPT_SIZES(float, true, 2);
+    else MI_PROMPT_SIZES(float, false, 2);
   }
+#undef MI_PROMPT_SIZES
 #undef MI_PROMPT
   return check_launch();
 }
