@@ -423,7 +423,8 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
                      static_cast<const TC*>(k_cache), static_cast<const TC*>(v_cache), bt, cols, cu_q, kv_lens, n_seqs, H, G, D, Dv, \
                      block_size, window, scale, bias, ldv, gate, ldg, out, ldo)
-  // (WIDE: stages of the ring at 256 channels of keys and of values)
+  // (WIDE: stages of the ring at 256 channels of keys and of values.  Pages of 24 rows, 400 rows of 4 sequences, 8 / 4 heads, us, the kernels
+  // before / 256 channels for every head / by head size: fp32 x 64 72 / 177 / 43, x 128 144 / 183 / 79; bf16 x 64 46 / 46 / 21.)
 #define MI_PROMPT_SIZES(TC, PAGED16, WIDE)                                   \
   do {                                                                       \
     if (D <= 64 && Dv <= 64) MI_PROMPT(TC, 2, 4, 4, false, PAGED16);         \

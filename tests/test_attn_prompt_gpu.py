@@ -88,6 +88,13 @@ def test_page_sizes(dtype, block):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("block", [8, 24])
+@pytest.mark.parametrize("D,Dv,vik", [(64, 128, False), (128, 112, False), (192, 256, False), (256, 224, True)])
+def test_head_sizes_over_pages_of_any_size(dtype, block, D, Dv, vik):
+    _case(dtype, 4, 2, D, Dv, block, SEQS, window=50, vik=vik)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("form", [dict(window=1), dict(window=40, kept=5), dict(window=64, kept=70), dict(chunk=48), dict(chunk=33, kept=3),
                                   dict(softcap=5.0, sink=True), dict(bias=_C.BIAS_LOG, sink=True), dict(value_heads=1), dict(kept=500)])
 def test_masks_and_biases(dtype, form):
