@@ -157,11 +157,12 @@ __device__ __forceinline__ void load8<float>(const float* p, int n_valid, bool v
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// exact kernel for any alignment and K: 64 x 64 tile, 256 threads, 4 x 4 outputs per thread, k ascending
+// exact kernel for any alignment and K: 256 threads, RT x 4 outputs per thread, k ascending: a 64 x 64 tile (RT 4) or 16 x 64 (1: few
+// features, many rows)
 // ---------------------------------------------------------------------------------------------------------------
-template <typename TW, bool DUAL, bool EXT>
+template <typename TW, bool DUAL, int RT, bool EXT>
 __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
-  constexpr int RT = 4, BM = 16 * RT, BN = 64, BK = 32, PAD = 4;
+  constexpr int BM = 16 * RT, BN = 64, BK = 32, PAD = 4;
   __shared__ float As[BK][BM + PAD];
   __shared__ float Bs[DUAL ? 2 : 1][BK][BN + PAD];
   const int tid = threadIdx.x;
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
   const int n0 = blockIdx.x * BN;
   const int lr = tid >> 2, lk = (tid & 3) * 8;  // this thread stages 8 consecutive k of one row
   int64_t xrow = -1;
-  if (m0 + lr < m_hi) xrow = a.x_rows ? a.x_rows[m0 + lr] : m0 + lr;
+  if (lr < BM && m0 + lr < m_hi) xrow = a.x_rows ? a.x_rows[m0 + lr] : m0 + lr;
   const int wrow = n0 + lr < a.N ? n0 + lr : -1;
   float acc[DUAL ? 2 : 1][RT][4] = {};
   const int ty = tid >> 4, tx = tid & 15;
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int k = k0 + lk + i;
-      As[lk + i][lr] = (xrow >= 0 && k < a.K) ? a.x[xrow * a.ldx + k] : 0.f;
+      if (lr < BM) As[lk + i][lr] = (xrow >= 0 && k < a.K) ? a.x[xrow * a.ldx + k] : 0.f;
       Bs[0][lk + i][lr] = (wrow >= 0 && k < a.K) ? w_load<TW>(w + (int64_t)wrow * a.K + k) : 0.f;
       if (DUAL) Bs[1][lk + i][lr] = (wrow >= 0 && k < a.K) ? w_load<TW>(w2 + (int64_t)wrow * a.K + k) : 0.f;
     }
@@ -720,7 +721,13 @@ static int launch_exact(const GemmAnyArgs& a, int groups, int rows_per_group_max
     }
     return check_launch();
   }
-  hipLaunchKernelGGL((gemm_any_fma_kernel<TW, DUAL, EXT>), dim3((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups), dim3(256), 0, st, a);
+  // a router over a prompt: one column of tiles - short tiles, more of them (us, 64 / 16 rows: 1024 rows x 64 features x 1000 93 / 75,
+  // 8192 rows x 32 x 1000 100 / 84)
+  if (a.N <= 64 && rows_per_group_max >= 1024) {
+    hipLaunchKernelGGL((gemm_any_fma_kernel<TW, DUAL, 1, EXT>), dim3(1, (rows_per_group_max + 15) / 16, groups), dim3(256), 0, st, a);
+    return check_launch();
+  }
+  hipLaunchKernelGGL((gemm_any_fma_kernel<TW, DUAL, 4, EXT>), dim3((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups), dim3(256), 0, st, a);
   return check_launch();
 }
 

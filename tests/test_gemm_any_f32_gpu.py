@@ -60,3 +60,15 @@ def test_a_row_has_the_same_bits_in_every_tile():
     x, w = torch.randn(5000, 256, device="cuda", generator=g), torch.randn(96, 256, device="cuda", generator=g)
     whole = ops.gemm_any(x, w, exact=True)
     assert torch.equal(whole[:700], ops.gemm_any(x[:700], w, exact=True)) and torch.equal(whole[17:90], ops.gemm_any(x[17:90], w, exact=True))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,odd", [(1024, 64, 40, 0), (1039, 5, 100, 0), (1500, 33, 64, 1), (1023, 64, 40, 0), (1024, 65, 40, 0)])
+def test_few_features_over_rows_that_are_no_whole_lines(dtype, M, N, K, odd):
+    """16-row tiles up to 64 features and from 1024 rows on, 64-row tiles beside that; the bound as above"""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K + odd, device="cuda", generator=g)[:, odd:]
+    w = torch.randn(N, K, device="cuda", generator=g).to(dtype)
+    got, want = ops.gemm_any(x, w, exact=True), x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    assert bool(((got.double() - want).abs() <= K * 2.0 ** -23 * size + 1e-12).all())
