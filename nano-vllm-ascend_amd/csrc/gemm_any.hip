@@ -597,7 +597,9 @@ __global__ __launch_bounds__(256) void gemm_any_skinny_kernel(GemmAnyArgs a) {
 // stored), so that a K piece is one round trip and not one per row - a router's 32 rows x 64 features x 2048 10.7 -> 6.7 us - and
 // four features share the rows' pieces where there are enough features for the chip (N 32768, K 2048: 8 rows 110 us with one feature
 // and a branch per row, now 76, 4 rows 62 / 40; a single row 31 with one feature, 36 with four).
-template <typename TW, int MT, int FT, bool DUAL, bool EXT>
+// UNROLL: K pieces that are asked for together; more than one only where all lanes have as many pieces - the last ones, which some lanes
+// lack, would be a pass of their own (64 rows x 1024 features x 1000 18.5 us, one at a time 13.2).
+template <typename TW, int MT, int FT, bool DUAL, bool EXT, int UNROLL = (FT == 1 ? 2 : 1)>
 __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
   static_assert(FT == 1 || !DUAL, "several features: one weight");
   constexpr int WN = DUAL ? 2 : FT;
@@ -634,8 +636,11 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
 #pragma unroll
         for (int f = 0; f < WN; ++f) acc[f][r] = fmaf(xv[r][i], wv[f][i], acc[f][r]);
   };
-  if (w_vec && x_vec) {   // (K % 8 == 0: every piece is whole)
-#pragma unroll FT == 1 ? 2 : 1
+  if (w_vec && x_vec && UNROLL > 1 && a.K % (64 * 8) == 0) {   // (K % 8 == 0: every piece is whole)
+#pragma unroll UNROLL
+    for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, true, true);
+  } else if (w_vec && x_vec) {
+#pragma unroll 1
     for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, true, true);
   } else {
     for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, w_vec, x_vec);
@@ -683,8 +688,11 @@ __global__ __launch_bounds__(256) void gemm_any_each_row_kernel(GemmAnyArgs a) {
         if (DUAL) acc2 = fmaf(xv[i], wv2[i], acc2);
       }
     };
-    if (w_vec && x_vec) {   // (K % 8 == 0: every piece is whole)
+    if (w_vec && x_vec && a.K % (64 * 8) == 0) {
 #pragma unroll 2
+      for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, true, true);
+    } else if (w_vec && x_vec) {
+#pragma unroll 1
       for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, true, true);
     } else {
       for (int k0 = lane * 8; k0 < a.K; k0 += 64 * 8) piece(k0, w_vec, x_vec);
@@ -733,9 +741,9 @@ static int launch_exact(const GemmAnyArgs& a, int groups, int rows_per_group_max
 
 template <typename TW, bool DUAL, bool EXT>
 static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, int mode, hipStream_t st) {
-  // mode 0: product (MFMA for bf16 weights, the row kernel for few rows); 1: exact (FMA chains / row kernel, x unrounded)
-  // few rows (per group): the weight-streaming row kernel.  Also the exact mode up to 64 rows: a router's few output
-  // features would make one tile of the FMA kernel walk all of K alone
+  // mode 0: product (MFMA for bf16 weights, the row kernels for few rows); 1: exact (x unrounded: the row kernels, beyond them launch_exact)
+  // few rows (per group): the weight-streaming row kernels.  Also the exact mode up to 64 rows: a router's few output
+  // features would be one or two tiles of launch_exact's kernels, each walking all of K alone
   const bool few = rows_per_group_max <= 8 || (mode == 1 && rows_per_group_max <= 64);
   if (few) {
     const int mt = rows_per_group_max <= 1 ? 1 : rows_per_group_max <= 4 ? 4 : 8;
@@ -751,10 +759,30 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
         else hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 8, 4, DUAL, EXT>), grid, dim3(256), 0, st, a);
         return check_launch();
       }
-    if (mt == 1) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 1, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
-    else if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 4, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 8, 1, DUAL, EXT>), grid, dim3(256), 0, st, a);
-    return check_launch();
+    const auto rows = [&](auto kernel, int batch) {
+      hipLaunchKernelGGL(kernel, dim3(grid.x, (rows_per_group_max + batch - 1) / batch, groups), dim3(256), 0, st, a);
+      return check_launch();
+    };
+    // A batch's empty places are multiplied too, and the registers of many rows and of two pieces leave few waves.  So up to seven rows are
+    // a batch of their own, and from five on the lanes take a piece at a time, at eight from 4096 weight rows on.  us, four or eight rows
+    // with two pieces / as here: 2 x 6144 x 2048 9.4 / 6.6, 5 x 6144 x 2048 16.8 / 11.6, 6 x 4096 x 2568 19.2 / 13.6, 8 x 8000 x 1000
+    // 19.9 / 13.4; 8 x 1024 x 1024 keeps two pieces (5.5, one 5.7).  Groups, and more than one batch (exact mode): four rows, a piece at a
+    // time (fp32 weights: 9 rows x 3072 x 1024 10.5 / 8.1, 64 rows 36 / 31, 64 x 1024 x 1000 18.5 / 12.9; experts' gate and up, 36 pairs
+    // of 32 of 512 x 1024 34.3 / 19.4) - except over weights beyond the L2s, which would be read twice as often (64 x 6144 x 2048, 50 MB:
+    // 119 / 139).
+    if (mt == 1) return rows(gemm_any_rows_kernel<TW, 1, 1, DUAL, EXT>, 1);
+    if (rows_per_group_max <= 8 && !a.group_offsets) {
+      if (rows_per_group_max == 2) return rows(gemm_any_rows_kernel<TW, 2, 1, DUAL, EXT>, 2);
+      if (rows_per_group_max == 3) return rows(gemm_any_rows_kernel<TW, 3, 1, DUAL, EXT>, 3);
+      if (rows_per_group_max == 4) return rows(gemm_any_rows_kernel<TW, 4, 1, DUAL, EXT>, 4);
+      if (rows_per_group_max == 5) return rows(gemm_any_rows_kernel<TW, 5, 1, DUAL, EXT, 1>, 5);
+      if (rows_per_group_max == 6) return rows(gemm_any_rows_kernel<TW, 6, 1, DUAL, EXT, 1>, 6);
+      if (rows_per_group_max == 7) return rows(gemm_any_rows_kernel<TW, 7, 1, DUAL, EXT, 1>, 7);
+      if ((int64_t)a.N * (DUAL ? 2 : 1) >= 4096) return rows(gemm_any_rows_kernel<TW, 8, 1, DUAL, EXT, 1>, 8);
+    } else if (a.group_offsets || (int64_t)a.N * a.K * (int64_t)sizeof(TW) <= (32 << 20)) {
+      return rows(gemm_any_rows_kernel<TW, 4, 1, DUAL, EXT, 1>, 4);
+    }
+    return rows(gemm_any_rows_kernel<TW, 8, 1, DUAL, EXT>, 8);
   }
   const dim3 grid((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups);
   if constexpr (sizeof(TW) == 2) {

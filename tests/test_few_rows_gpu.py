@@ -93,3 +93,41 @@ def test_groups_of_a_row_or_none(ops, counts, K, dtype, exact, dual):
                 assert ((got[place[m].long()].double() - z).abs() <= 2.0 ** -20 * z.abs() + 1e-12).all()
             else:
                 assert torch.equal(got[place[m].long()], z)
+
+
+@pytest.mark.parametrize("M", [2, 3, 5, 6, 7, 8, 9, 11, 13, 64])
+@pytest.mark.parametrize("K", [8, 520, 1000, 1024])
+@pytest.mark.parametrize("N", [33, 4100])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dual", [False, True])
+def test_batches_of_every_size(ops, M, K, N, dtype, dual):
+    """every row has the bits that it has alone, whatever its batch and however many pieces of K are asked for together"""
+    from nanovllm import _C
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn(M, K, device="cuda", generator=g)
+    w, w2 = ((torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(dtype) for _ in range(2))
+    kw = dict(act=_C.ACT_SILU, w2=w2) if dual else {}
+    got = ops.gemm_any_act(x, w, exact=True, **kw)
+    one = torch.cat([ops.gemm_any_act(x[r:r + 1], w, exact=True, **kw) for r in range(M)])
+    assert torch.equal(got, one)
+    z, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    bound = (K / 64 + 16) * 2.0 ** -24 * mag + 1e-12
+    if dual:   # (silu is 1.1-Lipschitz and at most its argument)
+        z2, mag2 = x.double() @ w2.double().T, x.double().abs() @ w2.double().abs().T
+        bound = 1.1 * bound * (z2.abs() + (K / 64 + 16) * 2.0 ** -24 * mag2) + z.abs() * (K / 64 + 16) * 2.0 ** -24 * mag2 + 2.0 ** -20 * (z * z2).abs() + 1e-12
+        z = torch.nn.functional.silu(z) * z2
+    assert ((got.double() - z).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("counts", [(8,), (3, 5), (0, 7, 1), (5, 0, 12, 4), (33, 31)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_groups_in_batches_of_four(ops, counts, dtype):
+    G, N, K, P = len(counts), 37, 600, sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(P)
+    x = torch.randn(P, K, device="cuda", generator=g)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device="cuda")
+    w = (torch.randn(G, N, K, device="cuda", generator=g) * K ** -0.5).to(dtype)
+    got = ops.gemm_any_grouped(x, None, w, None, off, P, None, P, True)
+    for e in range(G):
+        for m in range(int(off[e]), int(off[e + 1])):
+            assert torch.equal(got[m], ops.gemm_any(x[m:m + 1], w[e], exact=True)[0])
