@@ -121,3 +121,49 @@ def test_bound_on_one_groups_rows(counts, gathered):
     _close(ops.gemm_any_grouped_act(x, rows, w, None, _C.ACT_RELU2, off, most, place, P), z.clamp(min=0) ** 2, 2 * s * s, K)
     _close(ops.gemm_any_grouped_glu(x, rows, w, w2, _C.ACT_CLAMPED_GLU, 1.5, None, None, off, most, place, P),
            _ref(z, z2, _C.ACT_CLAMPED_GLU, 1.5), 4 * s * (s2 + 1), K)
+
+
+# what the dispatch picks for large work: the persistent kernel over several tiles per workgroup (more than 2 x 256 of them: the next
+# tile's group is fetched under the running one's products), 128-row tiles on the two-stage ring (more than 256 of them), 64-row tiles
+# of 128 features for one weight (more than 1024 of 64)
+LARGE = [(256, 24, 1028, 64, False, 33000), (256, 24, 516, 128, True, 33000), (256, 0, 1284, 64, False, 30000), (256, 0, 644, 64, True, 26000),
+         (128, 12, 516, 64, False, 9000), (128, 12, 260, 64, True, 9000), (128, 0, 516, 128, False, 9000), (64, 64, 2052, 64, False, 1500),
+         (64, 64, 1028, 256, True, 1500), (64, 0, 2052, 64, False, 3000)]
+
+
+@pytest.mark.parametrize("tile,G,N,K,dual,rows", LARGE)
+def test_more_tiles_than_the_chip_holds(tile, G, N, K, dual, rows):
+    g = torch.Generator(device="cuda").manual_seed(N + rows)
+    act = _C.ACT_SILU if dual else _C.ACT_NONE
+    row_tiles = rows // tile + G if G else -(-rows // tile)
+    wide = {256: 128 if dual else 256, 128: 64 if dual else 128, 64: 64}[tile]
+    assert row_tiles * -(-N // wide) > {256: 512, 128: 256, 64: 1024}[tile]
+    x = torch.randn(rows, K, device="cuda", generator=g)
+    place = torch.randperm(rows, device="cuda", generator=g).to(torch.int32)
+    if G:   # ragged, every fifth group empty, the last rows in none
+        share = torch.rand(G, generator=torch.Generator().manual_seed(G)) + 0.1
+        share[::5] = 0
+        counts = (share / share.sum() * (rows - 100)).long().tolist()
+        off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device="cuda")
+    else:
+        counts, off = [rows], None
+    w, w2 = (torch.randn(max(G, 1), N, K, device="cuda", generator=g).mul(K ** -0.5).bfloat16() for _ in range(2))
+    y = torch.full((rows, N), 7.0, device="cuda")
+    ww, ww2 = (w, w2) if G else (w[0], w2[0])
+    ops._tile_gemm(ops._tile_operand(x, tile, None, off, G, rows), tile, ww, ww2 if dual else None, y, act, G, place)
+    lo = 0
+    for e, n in enumerate(counts):
+        xr, at = x[lo:lo + n].bfloat16().double(), place[lo:lo + n].long()
+        z, s = xr @ w[e].double().T, xr.abs() @ w[e].double().abs().T
+        if dual:
+            z2, s2 = xr @ w2[e].double().T, xr.abs() @ w2[e].double().abs().T
+            z, s = torch.nn.functional.silu(z) * z2, 4 * s * (s2 + 1)
+        _close(y[at], z, s, K)
+        lo += n
+    assert bool((y[place[lo:].long()] == 7.0).all())
+
+
+@pytest.mark.parametrize("rows,N,K,G,dual,want", [(65536, 768, 2048, 64, True, 256), (65536, 2048, 768, 64, False, 256), (1024, 2048, 768, 64, False, 64),
+                                                  (256, 2048, 768, 64, False, 64), (8192, 2048, 2048, 0, False, 256), (2048, 768, 2048, 32, True, 128)])
+def test_rule_reaches_the_large_forms(rows, N, K, G, dual, want):
+    assert _C.lib.mi_gemm_any_tile_rows(rows, N, K, G, int(dual), _C.ACT_SILU if dual else _C.ACT_NONE) == want
