@@ -391,7 +391,7 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
   }
   const float odd = (zero[0] + zero[1]) + (zero[2] + zero[3]);
   uint64_t todo = __ballot(live && odd != 0.f);
-  if (todo == 0) return;
+  if (__builtin_expect(todo == 0, 1)) return;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // (the columns above are home before they are written again)
   __builtin_amdgcn_wave_barrier();
   while (todo) {

@@ -349,8 +349,6 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
     u = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 4; ++r) u = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[r], w[r], u, 0, 0, 0);
-    const bool odd = __any(!(finite(u[0]) && finite(u[1]) && finite(u[2]) && finite(u[3])));   // (the whole wave takes the branches)
-    if (odd) u = causal(tf, w, u, kg);
 #pragma unroll
     for (int c = 0; c < DT / 4; ++c) {
       if (c + 1 < DT / 4) read_k(c + 1);
@@ -363,8 +361,15 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
     f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 4; ++r) x = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[r], u[r], x, 0, 0, 0);
-    if (odd) x = causal(bf, u, x, kg);
     o = sum8(e) + x;
+    float zero = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) zero = fmaf(o[r], 0.f, zero);
+    // (the state has what is not finite either way; the whole wave takes the branch)
+    if (__builtin_expect(__any(zero != 0.f), 0)) {
+      const f32x4 x2 = causal(vec(rec_b), causal(vec(rec_b + 1024), w, u, kg), x, kg);
+      o = sum8(e) + x2;
+    }
   }
   store(nb - 1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the requests beyond the end land before the workgroup's LDS is given away)
