@@ -1,10 +1,10 @@
 """Tensor-parallel linear layers (reference: nanovllm/layers/linear.py) — same class
 names, constructor arguments and per-parameter `weight_loader` sharding rules.
 
-forward(): decode-sized activations (ops.prefers_tile: at most 64 rows, up to 512 for the narrow
-projections) go through the hand-written weight-streaming MFMA kernels (mi_gemm_bf16_packed / _skinny,
-the rows in chunks of 64); everything larger - every prefill projection - through the MFMA tile
-kernels of mi_gemm_bf16 (csrc/gemm_tile.hip).  No library GEMM anywhere on the path.
+forward(): decode-sized activations (ops.prefers_tile: at most 64 rows of 4096 features and more, 128 of 2048 and
+more, 512 of narrower projections) go through the hand-written weight-streaming MFMA kernels (mi_gemm_bf16_packed /
+_skinny, the rows in chunks of 64); everything larger through the MFMA tile kernels of mi_gemm_bf16
+(csrc/gemm_tile.hip).  No library GEMM anywhere on the path.
 """
 from __future__ import annotations
 
