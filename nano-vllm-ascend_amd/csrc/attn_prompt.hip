@@ -419,6 +419,14 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   // and V through registers into the image (V transposed on the way): 345, 104, 86.
   const bool vik = k_cache == v_cache && bias.value_heads == G && ldv == D && Dv <= D;
   const bool paged16 = block_size % 16 == 0;
+  // fp32 heads of more than 128 channels and a few dozen keys: 256 channels' padding and a ring of two cost more than the plain kernel's FMA
+  // chains until the walk is longer (us, that one / here: 8 / 4 heads x 160, 40 rows 23 / 34, 100 rows 46 / 57, 200 rows faster here; 16
+  // heads over one row of 256 channels 27 / 37, 100 rows 52 / 48; up to 32 keys are one step here: x 256, 30 rows 37 / 24)
+  const int64_t keys = (int64_t)cols * block_size;   // (at most so many for any sequence)
+  if (!bf16 && (D > 128 || Dv > 128) && keys > 32 && keys <= (vik ? 64 : 128) && rows > 32 * (int64_t)n_seqs) return MI_EUNSUPPORTED;
+  // ... and of at most 32 channels, padded to 64, where there are too few tiles for the chip (8 / 4 heads x 32: 1 x 400 rows 36 / 40, 1 x 1600 140 /
+  // 151; 4 x 1000 rows 171 / 115; x 16: 4 x 400 31 / 40, 4 x 1600 217 / 242)
+  if (!bf16 && D <= 32 && Dv <= 32 && keys > 32 && tiles * G * grid.z <= (D <= 16 && Dv <= 16 ? 420 : 108)) return MI_EUNSUPPORTED;
 #define MI_PROMPT(TC, DKM, DVM, NST, ...)                                                                                  \
   hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
                      static_cast<const TC*>(k_cache), static_cast<const TC*>(v_cache), bt, cols, cu_q, kv_lens, n_seqs, H, G, D, Dv, \

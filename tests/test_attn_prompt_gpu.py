@@ -95,6 +95,14 @@ def test_head_sizes_over_pages_of_any_size(dtype, block, D, Dv, vik):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("seqs", [((0, 33),), ((0, 64), (0, 40)), ((0, 65), (3, 60)), ((0, 128), (60, 40)), ((0, 129), (0, 40))])
+@pytest.mark.parametrize("D,Dv,vik", [(160, 128, False), (128, 192, False), (256, 256, True)])
+def test_wide_heads_over_few_keys(dtype, seqs, D, Dv, vik):
+    """both sides of the line beyond which fp32 heads of more than 128 channels go to the matrix cores"""
+    _case(dtype, 6, 2, D, Dv, 16, seqs, vik=vik, sink=True, gate=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("form", [dict(window=1), dict(window=40, kept=5), dict(window=64, kept=70), dict(chunk=48), dict(chunk=33, kept=3),
                                   dict(softcap=5.0, sink=True), dict(bias=_C.BIAS_LOG, sink=True), dict(value_heads=1), dict(kept=500)])
 def test_masks_and_biases(dtype, form):
