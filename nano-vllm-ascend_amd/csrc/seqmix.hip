@@ -2240,7 +2240,11 @@ extern "C" int mi_causal_conv(const float* x, int64_t ldx, const float* w, int t
   if (!x || !w || !state || !cu_q || !kv_lens || !slot_ids || !y || rows < 0 || n_seqs < 1 || channels < 1) return MI_EINVAL;
   if (taps < 1 || taps > 17) return MI_EUNSUPPORTED;
   if (rows == 0) return MI_OK;
-  if (taps >= 2 && taps <= 5 && channels % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && aligned16(x) && aligned16(w) && aligned16(state) &&
+  // A thread's eight rows are a chain of some 6 us whatever the step: small ones go a row per workgroup, whose walk over the sequences'
+  // borders costs 0.05 us for each (us, a row per workgroup / eight rows per thread, 4 taps: 64 rows x 2048 3.5 / 6.2, 200 x 3072 5.8 / 6.4,
+  // 300 x 3072 7.1 / 6.6; of 64 sequences 100 rows x 2048 8.0 / 9.4, 300 x 1024 8.8 / 7.4).
+  const bool large = (int64_t)rows * channels * (32 + n_seqs) >= 32 * 800000ll;
+  if (large && taps >= 2 && taps <= 5 && channels % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && aligned16(x) && aligned16(w) && aligned16(state) &&
       aligned16(y)) {
     const auto kernel = taps == 2   ? causal_conv_rows_kernel<2>
                         : taps == 3 ? causal_conv_rows_kernel<3>

@@ -94,7 +94,21 @@ def test_sums_of_experts_in_pieces(ops, width, top_k):
 @pytest.mark.parametrize("C", [4, 1028])
 @pytest.mark.parametrize("lens", [[9], [8, 8], [1, 0, 2, 30, 1, 1, 7], [1] * 70 + [11]])
 def test_convolution_of_eight_rows_at_a_time(ops, taps, C, lens):
+    """Steps as small as these go a row per workgroup (an odd row distance: always)."""
+    assert sum(lens) * C * (32 + len(lens)) < 32 * 800000
+    _convolution(ops, taps, C, lens)
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4, 5])
+@pytest.mark.parametrize("C,lens", [(1028, [803]), (1028, [8] * 99 + [9]), (1028, [1, 0, 2, 30, 1, 1, 7] * 20), (1028, [1] * 700 + [11]),
+                                    (4, [1] * 2000 + [5] * 400), (4100, [64, 63, 65, 9])])
+def test_convolution_of_eight_rows_in_large_steps(ops, taps, C, lens):
     """Eight rows per thread across the sequences' borders against one row per workgroup (an odd row distance): equal bits."""
+    assert sum(lens) * C * (32 + len(lens)) >= 32 * 800000
+    _convolution(ops, taps, C, lens)
+
+
+def _convolution(ops, taps, C, lens):
     torch.manual_seed(taps + C + len(lens))
     n, rows = len(lens), sum(lens)
     x, w = torch.randn(rows, C, device="cuda"), torch.randn(C, taps, device="cuda")
@@ -106,7 +120,7 @@ def test_convolution_of_eight_rows_at_a_time(ops, taps, C, lens):
         got = ops.causal_conv(x, w, state, cu, kv, slots, silu=silu, add_input=not silu)
         assert torch.equal(got, ops.causal_conv(_off(x), w, state, cu, kv, slots, silu=silu, add_input=not silu))
         if not silu:
-            for i, l in enumerate(lens):
+            for i, l in list(enumerate(lens))[-80:]:
                 own = x[cu[i]:cu[i + 1]].double()
                 past = state[n - 1 - i].double() if i % 2 else torch.zeros_like(state[0]).double()
                 full = torch.cat([past, own])
