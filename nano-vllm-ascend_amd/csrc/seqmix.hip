@@ -151,8 +151,8 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
 // mixed (written back in place, so that a later layer can take it as ITS v_first only if this layer is the first mixing
 // one - the caller keeps that tensor) and stored.  Cache layout [blocks][kv heads][block][dim], slot = block * block_size
 // + offset, slot < 0: not stored.
-// VEC 4: everything in 16-byte pieces (8-byte ones of a bf16 cache; a piece lies inside one head), a thread's first KEEP pieces of q and k
-// kept between the norm and its use.  8112 rows of 8 x 128 + 4 x 128 + 4 x 128: 45 us with a float per request, now 31.
+// VEC 4: everything in 16-byte pieces (8-byte ones of a bf16 cache; a piece lies inside one head).  A thread's first KEEP pieces of q and k
+// are kept between the norm and its use.  8112 rows of 8 x 128 + 4 x 128 + 4 x 128: 45 us with a float per request, now 31.
 template <typename TC, int VEC>
 __global__ __launch_bounds__(256) void swa_prepare_kernel(float* __restrict__ proj, int64_t ld, int q_off, int k_off,
                                                           int v_off, int nq, int nk, int nv,
@@ -2071,7 +2071,8 @@ extern "C" int mi_layernorm_f32(const float* y, int64_t ldy, const float* w, con
                                 int rows, int width, float eps, int add_to_out, mi_stream stream) {
   if (!y || !w || !b || !out || rows < 0 || width < 1 || ldy < width || ldo < width) return MI_EINVAL;
   if (rows == 0) return MI_OK;
-  const bool vec = width % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(w) && aligned16(b) && aligned16(out);
+  // (from 256 wide on: less leaves most of a workgroup without a piece - 8192 rows of 100 9.2 us a float at a time, 10.3 in pieces)
+  const bool vec = width >= 256 && width % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(w) && aligned16(b) && aligned16(out);
   hipLaunchKernelGGL(vec ? layernorm_f32_kernel<4> : layernorm_f32_kernel<1>, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out,
                      ldo, width, eps, add_to_out);
   return check_launch();
@@ -2366,7 +2367,11 @@ extern "C" int mi_moe_combine_f32(const float* y, const float* h, int64_t ldh, c
   if (!y || !h || !ids || !weights || !out || n_tokens < 0 || top_k < 1 || width < 1) return MI_EINVAL;
   if (n_tokens == 0) return MI_OK;
   const bool vec = width % 4 == 0 && ldh % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(h) && aligned16(out);
-  const auto kernel = vec ? (top_k <= 4 ? moe_combine_f32_kernel<4, 4> : moe_combine_f32_kernel<4, 8>) : moe_combine_f32_kernel<1, 4>;
+  // (no more requests than parts, about: 8192 tokens of one part of 250 6.7 us, four requests 9.5)
+  const auto kernel = vec ? (top_k <= 2   ? moe_combine_f32_kernel<4, 2>
+                             : top_k <= 4 ? moe_combine_f32_kernel<4, 4>
+                                          : moe_combine_f32_kernel<4, 8>)
+                          : (top_k <= 2 ? moe_combine_f32_kernel<1, 1> : moe_combine_f32_kernel<1, 4>);
   const int cols = vec ? 1024 : 256;
   hipLaunchKernelGGL(kernel, dim3(n_tokens, (width + cols - 1) / cols), dim3(256), 0, S(stream), y, h, ldh, ids, weights, top_k,
                      n_experts, width, out, ldo);
@@ -2488,7 +2493,10 @@ extern "C" int mi_moe_combine_shared(const float* y, const int32_t* ids, const f
   if (n_tokens == 0) return MI_OK;
   const bool vec = width % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(out) &&
                    (!shared || (ld_shared % 4 == 0 && aligned16(shared)));
-  const auto kernel = vec ? (top_k <= 4 ? moe_combine_shared_kernel<4, 4> : moe_combine_shared_kernel<4, 8>) : moe_combine_shared_kernel<1, 4>;
+  const auto kernel = vec ? (top_k <= 2   ? moe_combine_shared_kernel<4, 2>
+                             : top_k <= 4 ? moe_combine_shared_kernel<4, 4>
+                                          : moe_combine_shared_kernel<4, 8>)
+                          : (top_k <= 2 ? moe_combine_shared_kernel<1, 1> : moe_combine_shared_kernel<1, 4>);
   const int cols = vec ? 1024 : 256;
   hipLaunchKernelGGL(kernel, dim3(n_tokens, (width + cols - 1) / cols), dim3(256), 0, S(stream), y, weights, top_k, width, shared,
                      ld_shared, shared_gate, ld_gate, out, ldo);
@@ -2500,7 +2508,8 @@ extern "C" int mi_gated_norm_add_f32(float* res, int64_t ldr, const float* y, in
                                      int64_t ldo, int rows, int width, mi_stream stream) {
   if (!res || !y || !w_post || rows < 0 || width < 1 || (w_next && !out)) return MI_EINVAL;
   if (rows == 0) return MI_OK;
-  const bool vec = width % 4 == 0 && ldr % 4 == 0 && ldy % 4 == 0 && aligned16(res) && aligned16(y) && aligned16(w_post) &&
+  // (from 256 wide on, as layernorm: 8192 rows of 100 12.8 / 14.3 us)
+  const bool vec = width >= 256 && width % 4 == 0 && ldr % 4 == 0 && ldy % 4 == 0 && aligned16(res) && aligned16(y) && aligned16(w_post) &&
                    (!gate_pre || (ldg % 4 == 0 && aligned16(gate_pre))) && (!w_next || (ldo % 4 == 0 && aligned16(out) && aligned16(w_next)));
   hipLaunchKernelGGL(vec ? gated_norm_add_f32_kernel<4> : gated_norm_add_f32_kernel<1>, dim3(rows), dim3(256), 0, S(stream), res, ldr, y,
                      ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, width);

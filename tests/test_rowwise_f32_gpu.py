@@ -1,6 +1,6 @@
 """The row-wise fp32 kernels that read 16 bytes a lane where pointers, strides and widths allow it, and one float at a time otherwise
 (csrc/seqmix.hip: layernorm, gated norm-and-add, the experts' sum, the causal convolution): both forms over the same numbers, against
-the operation in 64 bits.  Widths: one piece, less than a workgroup's, what a thread keeps (4096 by pieces, 1024 by floats) and beyond.
+the operation in 64 bits.  Widths: below and at the 256 from which the norms go in pieces, what a thread keeps (4096 by pieces, 1024 by floats) and beyond.
 
 Tolerance: sums of `width` fp32 terms in chains of at most width / 256 + 14 additions, each rounded to 2^-24 of the partial sum; the
 results are of order one, so (width / 256 + 32) * 2^-24 * 8 covers sum, root, quotient and the products behind them."""
@@ -25,7 +25,7 @@ def _off(t):
     return base.copy_(t)
 
 
-WIDTHS = [4, 36, 1024, 1028, 2048, 4096, 4100, 9000]
+WIDTHS = [4, 36, 252, 256, 260, 1024, 1028, 2048, 4096, 4100, 9000]
 ROWS = 5
 
 
