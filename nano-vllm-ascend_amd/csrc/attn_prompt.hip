@@ -169,10 +169,11 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
     if (V4 && is_v) {
 #pragma unroll
       for (int i = 0; i < PP * 4; ++i) {
+        // (channels of the zero padding repeat the last ones, which nothing reads: a request without a lane, half a row beyond a head's
+        // channels, would be branched over, and the waits below count on every one)
         const int at = (p0 - KP) * 1024 + i * 256 + lane * 4, r = at / VROW, c = ((at % VROW / 16) ^ swizzle(r, VROW)) * VEC + (at & 15) / 2;
-        if (c < Dv)
-          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row_at(r) + c),
-                                           (__attribute__((address_space(3))) void*)(dst + i * 256), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row_at(r) + min(c, Dv - 2)),
+                                         (__attribute__((address_space(3))) void*)(dst + i * 256), 4, 0, 0);
       }
     } else if (PAGED16 && u + kKeys - 1 <= hi_key) {
 #pragma unroll

@@ -123,6 +123,13 @@ def test_value_rows_of_any_stride(dtype, pad, H, G, D, Dv, block):
     _case(dtype, H, G, D, Dv, block, SEQS, window=60, pad=pad, gate=True)
 
 
+@pytest.mark.parametrize("pad", [2, 6])
+@pytest.mark.parametrize("H,G,D,Dv,block", [(4, 2, 192, 96, 16), (8, 1, 256, 16, 64), (4, 4, 64, 128, 24)])
+def test_narrow_value_rows_of_even_strides_over_long_walks(pad, H, G, D, Dv, block):
+    """value heads of at most half the image's 256 channels: every request of a step's values counts in the ring's waits"""
+    _case(torch.bfloat16, H, G, D, Dv, block, ((1500, 70), (900, 33)), pad=pad)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 @pytest.mark.parametrize("where", ["k", "v"])
