@@ -138,8 +138,20 @@ static bool tile_rows_ok(int t) { return t == 64 || t == 128 || t == 256; }
 // the row tiles of `rows` rows in at most n_groups groups (0: one, its tiles known)
 static int64_t row_tiles(int rows, int n_groups, int t) { return n_groups ? rows / t + n_groups : (rows + t - 1) / t; }
 
-// 0: not taken; else the rows of a tile (256: the persistent kernel, 128 and 64: the small-tile kernel)
-static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int act) {
+// Few pairs over small experts: the operand pass and the rings' first round trips are longer than the general kernels' whole walk (us with
+// weights not in the L2s, both products, general / tile kernels: 8 experts of 256 x 1024, 64 pairs 15.8 / 18.2; 16 of 256 x 512, 96 pairs
+// 12.0 / 14.8; 32 of 256 x 512, 32 pairs 13.3 / 14.7, 48 pairs 16.6 / 14.6; 128 of 256 x 256, 24 pairs 12.4 / 13.3; 8 of 512 x 1024,
+// 32 pairs 17.0 / 19.1, 64 pairs 18.8 / 19.1; 128 of 192 x 512, 24 pairs 13.7 / 16.9).  Their time grows with the experts that have a pair
+// (some G P / (G + P)) and their rows of weights; beyond eight pairs an expert they take other kernels.
+static bool few_pairs(int64_t pairs, int N, int K, int64_t G) {
+  if (pairs > 192 || pairs > 8 * G || (pairs >= 128 && N >= 256 && K >= 256) || (int64_t)N * K > (512 << 10)) return false;
+  const bool narrow = pairs < 128 && (N < 256 || K < 256);   // (K < 256: on the general kernels either way, an operand pass for one product)
+  return G * pairs * (N + K) <= (narrow ? 22000 : (int64_t)N * K <= (256 << 10) ? 12800 : 10240) * (G + pairs);
+}
+
+// 0: not taken; else the rows of a tile (256: the persistent kernel, 128 and 64: the small-tile kernel).  pays: only where it is not slower
+// than the general kernels
+static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int act, bool pays = true) {
   if (rows < 1 || N < 1 || K < BK || K % BK || N % 4 || n_groups < 0 || n_groups > 1024) return 0;
   const bool known = dual ? act == MI_ACT_SILU || act == MI_ACT_GELU_TANH || act == MI_ACT_CLAMPED_GLU
                           : act == MI_ACT_NONE || act == MI_ACT_GELU_ERF || act == MI_ACT_RELU2 || act == MI_ACT_SOFTCAP;
@@ -152,7 +164,9 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   // and they stay).  No groups, N 2048: K 2048 at 9 rows 13.0 / 13.2, at 32 13.2 / 19.1, at 128 14.4 / 43.2; K 512 at 16 rows 7.1 / 5.9,
   // at 24 7.2 / 7.2, at 64 7.3 / 10.8; K 256 at 32 rows 6.3 / 5.4, at 64 6.4 / 7.9; K 64 from 65 rows on 5.1 / 5.2.  Experts' pair of
   // products, 32 of 512 x 1024 (64 of 768 x 2048): 16 pairs 19 / 20 (32 / 50), 128 pairs 28 / 37, (64 pairs 82 / 106).
-  if (n_groups ? rows < 16 || (rows < 128 && K < 256) : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) || (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
+  if (n_groups ? rows < 16 || (rows < 128 && K < 256) || (pays && few_pairs(rows, N, K, n_groups))
+               : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) ||
+                   (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
     return 0;
   const int tf = dual ? 128 : 256;
   if (n_groups && act == MI_ACT_SOFTCAP) return 0;   // (no group has one)
@@ -246,7 +260,7 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
   if (act == MI_ACT_SOFTCAP && tile_rows == 256) return MI_EUNSUPPORTED;   // (launch_any_tile)
   if (rows == 0) return MI_OK;
   if (!tile_rows_ok(tile_rows)) return MI_EINVAL;
-  if (tile_rows_for(rows, N, K, n_groups, w2 != nullptr, act) == 0) return MI_EUNSUPPORTED;
+  if (tile_rows_for(rows, N, K, n_groups, w2 != nullptr, act, false) == 0) return MI_EUNSUPPORTED;
   if (ldy < N || ldy % 4 || !aligned16(xb) || !aligned16(w) || (w2 && !aligned16(w2)) || !aligned16(y) || (bias && !aligned16(bias)) ||
       (bias2 && (!w2 || !aligned16(bias2))))
     return MI_EINVAL;

@@ -73,7 +73,7 @@ def test_soft_capped_products_have_no_256_row_tiles():
 
 def test_expert_feed_forward_takes_the_operands_that_the_two_products_take(recorded):
     """a scale per pair is read as it lies in memory: strided ones are refused by both routes"""
-    G, T, top, W, ff = 4, 10, 2, 256, 256
+    G, T, top, W, ff = 4, 50, 2, 256, 256
     x, gate, down = torch.zeros(T, W), torch.zeros(G, ff, W, dtype=torch.bfloat16), torch.zeros(G, W, ff, dtype=torch.bfloat16)
     i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
     args = (x, i32(T * top), gate, gate, down, _C.ACT_CLAMPED_GLU, i32(G + 1), T * top, i32(T * top), 7.0)
@@ -83,3 +83,12 @@ def test_expert_feed_forward_takes_the_operands_that_the_two_products_take(recor
     with pytest.raises(AssertionError):
         ops.expert_ff(*args, torch.ones(T, 2 * top)[:, :top], i32(T * top))
     assert not recorded
+
+
+def test_few_pairs_of_small_experts_stay_on_the_general_kernels(recorded):
+    """both products or neither: the line is the same whichever of the two a product is"""
+    rows = lambda P, N, K, G, dual=False: _C.lib.mi_gemm_any_tile_rows(P, N, K, G, int(dual), _C.ACT_SILU if dual else _C.ACT_RELU2)
+    for P, ff, width, G in ((16, 256, 256, 8), (96, 256, 512, 16), (32, 256, 512, 32), (24, 192, 512, 128), (32, 512, 1024, 8)):
+        assert not rows(P, ff, width, G, True) and not rows(P, width, ff, G) and not _C.lib.mi_expert_ff_bytes(P, G, ff, width, 1, _C.ACT_SILU)
+    for P, ff, width, G in ((65, 256, 256, 8), (48, 256, 512, 32), (128, 256, 512, 16), (16, 512, 1024, 32), (16, 768, 2048, 64), (96, 512, 1024, 8)):
+        assert rows(P, ff, width, G, True) and rows(P, width, ff, G) and _C.lib.mi_expert_ff_bytes(P, G, ff, width, 1, _C.ACT_SILU)
