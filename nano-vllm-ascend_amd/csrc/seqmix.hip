@@ -91,15 +91,15 @@ __device__ __forceinline__ float vsum(fvec<VEC> v) {
 // One workgroup per row; mean, then the mean of squared deviations.  Bound by the rows' bytes: a thread asks for all of its pieces (the
 // residual's too) before the first sum and keeps them (VEC 4: rows up to 4096 wide; the rest of wider ones is read again), so that a CU
 // has its whole share of requests out at once.  8112 rows of 2048, added to the residual: 37 us with a float per request, each pass over
-// the row again; now 19.
-template <int VEC>
+// the row again; now 19.  KEEP: pieces a thread has; one where it cannot have more (8000 rows of 64: 7.6 us, four 8.4).
+template <int VEC, int KEEP = 4>
 __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ y, int64_t ldy,
                                                             const float* __restrict__ w, const float* __restrict__ b,
                                                             float* __restrict__ out, int64_t ldo, int width, float eps,
                                                             int add) {
   using vec = fvec<VEC>;
   __shared__ float red[4];
-  constexpr int KEEP = 4, STEP = 256 * VEC;
+  constexpr int STEP = 256 * VEC;
   const float* yr = y + (int64_t)blockIdx.x * ldy;
   float* o = out + (int64_t)blockIdx.x * ldo;
   const int c0 = threadIdx.x * VEC;
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
 // + offset, slot < 0: not stored.
 // VEC 4: everything in 16-byte pieces (8-byte ones of a bf16 cache; a piece lies inside one head).  A thread's first KEEP pieces of q and k
 // are kept between the norm and its use.  8112 rows of 8 x 128 + 4 x 128 + 4 x 128: 45 us with a float per request, now 31.
-template <typename TC, int VEC>
+template <typename TC, int VEC, int KEEP = 4>
 __global__ __launch_bounds__(256) void swa_prepare_kernel(float* __restrict__ proj, int64_t ld, int q_off, int k_off,
                                                           int v_off, int nq, int nk, int nv,
                                                           const float* __restrict__ qn_w, const float* __restrict__ kn_w,
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) void swa_prepare_kernel(float* __restrict__ pr
                                                           int G, int D, int Dv, int block_size) {
   using vec = fvec<VEC>;
   __shared__ float red[4];
-  constexpr int KEEP = 4, STEP = 256 * VEC;
+  constexpr int STEP = 256 * VEC;
   float* row = proj + (int64_t)blockIdx.x * ld;
   const int c0 = threadIdx.x * VEC;
   vec q[KEEP], k[KEEP];
@@ -1649,7 +1649,7 @@ __global__ __launch_bounds__(256) void moe_combine_shared_kernel(const float* __
 // w_post; w_next != nullptr: out = res / sqrt(mean(res^2) + eps) * w_next - what the next sublayer reads.  Bound by the rows' bytes: all of
 // a thread's pieces (VEC 4: rows up to 4096 wide; the rest of wider ones is read again) are asked for before the first sum.  8192 rows
 // of 2048 with a gate, 335 MB: 130 us with a float per request; now 57 (5.9 TB/s).
-template <int VEC>
+template <int VEC, int KEEP = 4>
 __global__ __launch_bounds__(256) void gated_norm_add_f32_kernel(float* __restrict__ res, int64_t ldr,
                                                                  const float* __restrict__ y, int64_t ldy,
                                                                  const float* __restrict__ gate_pre, int64_t ldg,
@@ -1658,7 +1658,7 @@ __global__ __launch_bounds__(256) void gated_norm_add_f32_kernel(float* __restri
                                                                  float* __restrict__ out, int64_t ldo, int width) {
   using vec = fvec<VEC>;
   __shared__ float red[4];
-  constexpr int KEEP = 4, STEP = 256 * VEC;
+  constexpr int STEP = 256 * VEC;
   float* r = res + (int64_t)blockIdx.x * ldr;
   const float* yr = y + (int64_t)blockIdx.x * ldy;
   const float* gr = gate_pre ? gate_pre + (int64_t)blockIdx.x * ldg : nullptr;
@@ -2073,7 +2073,8 @@ extern "C" int mi_layernorm_f32(const float* y, int64_t ldy, const float* w, con
   if (rows == 0) return MI_OK;
   // (from 256 wide on: less leaves most of a workgroup without a piece - 8192 rows of 100 9.2 us a float at a time, 10.3 in pieces)
   const bool vec = width >= 256 && width % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(w) && aligned16(b) && aligned16(out);
-  hipLaunchKernelGGL(vec ? layernorm_f32_kernel<4> : layernorm_f32_kernel<1>, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out,
+  const auto kernel = vec ? layernorm_f32_kernel<4> : width <= 256 ? layernorm_f32_kernel<1, 1> : layernorm_f32_kernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out,
                      ldo, width, eps, add_to_out);
   return check_launch();
 }
@@ -2088,14 +2089,15 @@ extern "C" int mi_swa_prepare(float* proj, int64_t ld, int q_off, int k_off, int
   const bool vec = ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 && v_off % 4 == 0 && D % 4 == 0 && Dv % 4 == 0 && aligned16(proj) &&
                    aligned16(qn_w) && aligned16(kn_w) && aligned16(k_cache) && aligned16(v_cache) &&
                    (!v_first || (ld_vf % 4 == 0 && aligned16(v_first)));
+  const bool one = H * D <= 256;   // (a thread has one piece: 8000 rows of 3 + 1 + 1 heads of 30 14.7 us with four, as before them 12.6)
   const auto launch = [&](auto kernel, auto* kc, auto* vc) {
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, S(stream), proj, ld, q_off, k_off, v_off, H * D, G * D, G * Dv, qn_w, kn_w, eps,
                        v_first, ld_vf, lam, kc, vc, slots, G, D, Dv, block_size);
   };
   if (cache_dtype == MI_DTYPE_BF16)
-    launch(vec ? swa_prepare_kernel<uint16_t, 4> : swa_prepare_kernel<uint16_t, 1>, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache));
+    launch(vec ? swa_prepare_kernel<uint16_t, 4> : one ? swa_prepare_kernel<uint16_t, 1, 1> : swa_prepare_kernel<uint16_t, 1>, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache));
   else if (cache_dtype == MI_DTYPE_F32)
-    launch(vec ? swa_prepare_kernel<float, 4> : swa_prepare_kernel<float, 1>, static_cast<float*>(k_cache), static_cast<float*>(v_cache));
+    launch(vec ? swa_prepare_kernel<float, 4> : one ? swa_prepare_kernel<float, 1, 1> : swa_prepare_kernel<float, 1>, static_cast<float*>(k_cache), static_cast<float*>(v_cache));
   else return MI_EINVAL;
   return check_launch();
 }
@@ -2511,7 +2513,8 @@ extern "C" int mi_gated_norm_add_f32(float* res, int64_t ldr, const float* y, in
   // (from 256 wide on, as layernorm: 8192 rows of 100 12.8 / 14.3 us)
   const bool vec = width >= 256 && width % 4 == 0 && ldr % 4 == 0 && ldy % 4 == 0 && aligned16(res) && aligned16(y) && aligned16(w_post) &&
                    (!gate_pre || (ldg % 4 == 0 && aligned16(gate_pre))) && (!w_next || (ldo % 4 == 0 && aligned16(out) && aligned16(w_next)));
-  hipLaunchKernelGGL(vec ? gated_norm_add_f32_kernel<4> : gated_norm_add_f32_kernel<1>, dim3(rows), dim3(256), 0, S(stream), res, ldr, y,
+  const auto kernel = vec ? gated_norm_add_f32_kernel<4> : width <= 256 ? gated_norm_add_f32_kernel<1, 1> : gated_norm_add_f32_kernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, S(stream), res, ldr, y,
                      ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, width);
   return check_launch();
 }
