@@ -502,9 +502,17 @@ struct MidTile {
 constexpr MidTile kMidTiles[3] = {{128, 128, 0.52, 0.62}, {64, 128, 0.36, 0.56}, {64, 64, 0.22, 0.35}};
 constexpr double kLaunchUs = 3.8, kPartialBytesPerUs = 4.0e6;
 
-// fewer 256-tiles than CUs: the 128-tile kernel
-static bool use_mid(int M, int N, int K) {
+// fewer 256-tiles than CUs
+static bool few_tiles(int M, int N) {
   return (int64_t)((M + TILE_T - 1) / TILE_T) * ((N + TILE_F - 1) / TILE_F) < kPersistentGrid;
+}
+// The 128-tile kernel: there, up to two 128-tiles per CU.  More are a second round of its workgroups, and 256-tiles on half of the CUs are
+// done before it (us, small tiles / 256-tiles: 4536 x 2048 x 1024 = 576 of 128, 144 of 256 29.9 / 25.1; 3000 x 4096 x 4096 114.9 / 77.5;
+// 1976 x 6144 x 2048 56.6 / 43.3; K 384: 3256 x 4096 20.2 / 17.3, 256: 256 x 40000 15.3 / 18.5; two per CU: 4024 x 2048 x 1024 21.6 / 25.0,
+// 1976 x 4096 x 4096 68.5 / 74.1).  The second round's time also hung on where the kernel's loop lies in its code (3000 x 4096 x 4096: 113
+// to 125).
+static bool use_mid(int M, int N, int K) {
+  return few_tiles(M, N) && (K < 384 || (int64_t)((M + MID_T - 1) / MID_T) * ((N + MID_F - 1) / MID_F) <= 2 * kPersistentGrid);
 }
 
 struct MidPick {
@@ -637,7 +645,7 @@ extern "C" int mi_gemm_bf16_qkv_store(const mi_bf16* x, int64_t ldx, const mi_bf
   // one wave = one head; whole feature tiles and 16-byte aligned output rows (the whole-line stores of the q heads)
   if (head_dim != 128 || N != (n_q_heads + 2 * n_kv_heads) * 128 || N % TILE_F || ldy % 8 || block_size <= 0 || block_size % 16)
     return MI_EUNSUPPORTED;
-  if (use_mid(M, N, K) || (int64_t)M * ldy * 2 >= ((int64_t)1 << 32)) return MI_EUNSUPPORTED;  // the large-M kernel only
+  if (few_tiles(M, N) || (int64_t)M * ldy * 2 >= ((int64_t)1 << 32)) return MI_EUNSUPPORTED;  // the large-M kernel only
   if (M == 0) return MI_OK;
   TileArgs a{x, w, bias, qkv, ldx, ldy, M, N, K, N / TILE_F, (M + TILE_T - 1) / TILE_T, nullptr,
              {k_w, positions, cos_sin, k_cache, v_cache, slots, eps, n_q_heads, n_kv_heads, block_size}};

@@ -107,6 +107,21 @@ def test_gemm_tile_kernel_choice_boundary(ops, M):
     assert_bf16_close(gu, oracle.silu_and_mul(oracle.linear(x, w)), max_ulp=4, max_frac=3e-2, atol=32 * K * 2.0 ** -22)
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 384), (4097, 2048, 384), (2056, 3964, 448), (2056, 3964, 320), (130, 40000, 384)])
+def test_gemm_tile_two_small_tiles_per_cu(ops, M, N, K):
+    """either side of two 128-tiles per CU, where the 128-tile kernel hands over to the large one before the chip is full of 256-tiles
+    (and of the K up to which it does not): one fp32 chain per element on both, so the same bits, and no K slices"""
+    g, x, w = _case(M, N, K, seed=17)
+    x, w = x.to(DEV), w.to(DEV)
+    y, big, mid = ops.gemm_tile(x, w), ops.gemm_tile(x, w, variant=0), ops.gemm_tile(x, w, variant=65538)
+    assert torch.equal(y.view(torch.int16), big.view(torch.int16)) and torch.equal(y.view(torch.int16), mid.view(torch.int16))
+    b = torch.randn(N, generator=g).bfloat16()
+    assert_bf16_close(ops.gemm_tile(x, w, b.to(DEV))[-200:], oracle.linear(x[-200:].cpu(), w.cpu(), b), max_ulp=1, max_frac=2e-2, atol=K * 2.0 ** -22)
+    if N % 256 == 0:
+        gu = ops.gemm_tile(x, w, silu_mul=True)
+        assert_bf16_close(gu, ops.silu_mul(y).cpu(), max_ulp=2, max_frac=1e-3, atol=32 * K * 2.0 ** -22)
+
+
 def test_gemm_tile_strided_rows(ops):
     """x and y as row-strided views (the q heads of a packed qkv row, a slice of a wider output)"""
     g, xw, w = _case(300, 1024, 2048 + 1024 + 1024, seed=5)
