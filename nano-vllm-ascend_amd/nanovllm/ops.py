@@ -1071,8 +1071,8 @@ def gemm_any_grouped(x, x_rows, w, w2, group_offsets, rows_max: int, y_rows, y_r
 def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_index, limit: float = 0.0, row_scale=None,
               row_scale_rows=None) -> torch.Tensor:
     """Both products of the experts' feed-forwards over expert-sorted pairs: down[e] (act(w[e] x) (* w2[e] x)) of every pair at
-    its place pair_index.  bf16 weights, 16 pairs and more: the inner activations leave the first product as the bf16 rows
-    that the second one multiplies (it would round the same numbers itself)."""
+    its place pair_index.  bf16 weights, 16 pairs and more (of small experts more than few): the inner activations leave the
+    first product as the bf16 rows that the second one multiplies (it would round the same numbers itself)."""
     G, ff, width = w.shape
     n = lib.mi_expert_ff_bytes(pairs, G, ff, width, w2 is not None, int(act)) if w.dtype == _BF16 and down.dtype == _BF16 else 0
     if n and not (w.data_ptr() | down.data_ptr() | (0 if w2 is None else w2.data_ptr())) % 16:
