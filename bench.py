@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Headline benchmark: decode tokens/s (+ p50 TTFT) of Qwen3-0.6B, bs=32, seq=1024, block 16,
-bf16, paged decode under hipGraph on N MI355X.
+bf16, paged decode under hipGraph, on N MI355X.
 
     python bench.py --gpus 1 --steps K --warmup W          # one GPU
     python -m torch.distributed.run --nnodes=1 --nproc-per-node N --master-addr 127.0.0.1 \
@@ -13,7 +13,7 @@ N > 1 measures BOTH ways of using N GPUs, back to back, and reports them in ONE 
                       own 32 sequences (global batch 32 N, weak scaling); `value` is the sum over ranks of
                       tokens / the slowest rank's time (barrier + synchronize on both sides, max over ranks).
   tp   (`tp_run`)     Megatron tensor parallelism over RCCL/xGMI at the fixed batch of 32 (strong scaling):
-                      what a model that does not fit one GPU needs (BASELINE configs[2]); for this 0.6 B
+                      what a model that does not fit one GPU needs; for this 0.6 B
                       model every all-reduce is a 64 KiB latency-bound message, so it does not speed up.
                       Carries its own value, ms_per_step, world_seen, backend, xgmi_selftest and the
                       per-rank kernel rooflines; runs under a watchdog, so a failure there costs the
@@ -21,11 +21,11 @@ N > 1 measures BOTH ways of using N GPUs, back to back, and reports them in ONE 
 
 A "step" is one engine decode step over the batch of 32 sequences (scheduler -> metadata
 -> graph replay incl. sampling -> postprocess), i.e. 32 new tokens.  On one GPU the engine keeps one step queued
-behind the running one (decode_lookahead, DESIGN.md 4.6): the timed region starts - after synchronize - with one
+behind the running one (decode_lookahead): the timed region starts - after synchronize - with one
 step finished and not yet consumed, and ends - after synchronize - with one finished and not consumed, so exactly
 `--steps` steps of device work and of host work lie inside it.  Inputs are synthetic
 (random-init Qwen3-0.6B-shaped weights N(0,0.02^2), random prompt ids in [0,10000],
-random.seed(0); SURVEY.md §8d); the 32 x 1024-token prompts are prefilled through the
+random.seed(0)); the 32 x 1024-token prompts are prefilled through the
 engine first (that is where p50 TTFT comes from), so the KV cache is resident in HBM
 when the timed region starts.
 
@@ -39,7 +39,7 @@ Rank 0 prints ONE JSON line.  Besides the contract fields it carries
                 bytes per launch / average duration vs the 8 TB/s HBM peak; `traffic` = those bytes x
                 the PMC ratio of the newest profiles/r*_attn_traffic.json;
   chain_roofline the six non-attention launches of a layer over all layers' weights;
-  step_roofline the whole decode step against BASELINE.md's bytes(B, ctx) model;
+  step_roofline the whole decode step against its algorithmic bytes(B, ctx);
   cpu_baseline  the CPU oracle (oracle/, a port of the reference's arithmetic) timed on
                 this host on a bounded sample of the same workload;
   prefill_steps_ms  per prefill step: when its launch sequence started, the host's launch time, the device time (HIP
@@ -69,7 +69,7 @@ BATCH, PROMPT_LEN, BLOCK = 32, 1024, 16
 
 
 def step_bytes(batch: int, ctx: int, tp: int = 1) -> float:
-    """algorithmic HBM bytes of one decode step (whole job, all ranks)."""
+    """Algorithmic HBM bytes of one decode step (whole job, all ranks)."""
     return 1_192_099_840 + batch * (114_688 * ctx + 418_560)
 
 
@@ -208,7 +208,7 @@ def _attention_roofline(llm, seqs, iters):
                             "profile (not a counter of this run)",
             "traffic_source": traffic_src,
             # the contexts the counters were collected at, next to this run's: `traffic` is the profile's ratio applied to
-            # this run's bytes - two different ctx_sums here say so at a glance (VERDICT r05 weak 8)
+            # this run's bytes - two different ctx_sums here say so at a glance
             "traffic_ctx_sum": traffic_ctx_sum, "ctx_sum": ctx_sum,
             "bytes_per_launch": algo, "avg_launch_us": dur * 1e6, "launches_timed": iters * len(attn_mods)}
 
@@ -216,7 +216,7 @@ def _attention_roofline(llm, seqs, iters):
 def chain_roofline(llm, batch: int, iters: int = 20):
     """The six launches per layer that are NOT attention (add+RMSNorm x2, qkv / o_proj / gate_up+SwiGLU /
     down_proj GEMMs) replayed as one graph over all layers' real weights, HIP events on the launch stream:
-    algorithmic bytes = the layers' weights (activations excluded, as BASELINE.md §2) / time."""
+    algorithmic bytes = the layers' weights (activations excluded) / time."""
     import torch
 
     from nanovllm import ops
@@ -284,7 +284,7 @@ def prefill_flops(n_seqs: int, seq_len: int, cfg: dict) -> float:
 
 def one_gpu_reference():
     """The newest committed one-GPU line of this bench (profiles/r*bench*.json, n_gpus == 1, the same workload): what
-    north_star's ">= 6x aggregate at 8 GPUs" is a multiple of.  -> (tokens/s, file name) or (None, None)."""
+    the aggregate at 8 GPUs is given as a multiple of.  -> (tokens/s, file name) or (None, None)."""
     import glob
 
     best = (None, None, None)
@@ -294,7 +294,7 @@ def one_gpu_reference():
                 line = json.loads(f.read().strip().splitlines()[-1])
             if line.get("n_gpus") == 1 and line.get("config", {}).get("batch") == BATCH and not line.get("dry_run"):
                 # newest round first; within a round the file the round calls final (then by name) - never the file
-                # time, which is arbitrary after a checkout (ADVICE r05)
+                # time, which is arbitrary after a checkout
                 name = os.path.basename(path)
                 key = (name[:3], "final" in name, name)
                 if best[0] is None or key > best[2]:
@@ -305,9 +305,9 @@ def one_gpu_reference():
 
 
 def self_launch(args) -> int:
-    """`python bench.py --gpus N` with N > 1 and no torchrun around it: start the N ranks ourselves (the same command
-    line the driver uses).  On a box with fewer GPUs than ranks the ranks share devices over gloo - a functional dry
-    run of the N-rank flow, not a measurement (the JSON line says so)."""
+    """`python bench.py --gpus N` with N > 1 and no torchrun around it: start the N ranks ourselves (torch.distributed.run).
+    On a box with fewer GPUs than ranks the ranks share devices over gloo - a functional dry run of the N-rank flow, not a
+    measurement (the JSON line says so)."""
     import socket
     import subprocess
 
@@ -370,10 +370,10 @@ def run_phase(args, mode: str, rank: int, world: int, port: int, model_dir: str)
     t_p_end = time.perf_counter()
     prefill_phase_ms = (t_p_end - t_p) * 1e3
     prefill_trace = [dict(r) for r in llm.prefill_trace]
-    # the phase ends when the LAST prefill step's tokens are on the host (its first-token stamp): since round 5 the engine
+    # the phase ends when the LAST prefill step's tokens are on the host (its first-token stamp): the engine
     # queues the first decode step behind that step, and the synchronize above waits for it as well - a decode step is
     # not prefill time
-    prefill_phase_to_sync_ms = prefill_phase_ms  # (rounds 1-4's definition: reported beside the other)
+    prefill_phase_to_sync_ms = prefill_phase_ms  # (reported beside the other)
     stamps = [r["stamp"] for r in prefill_trace if r["stamp"] is not None]
     if len(stamps) == prefill_steps:
         prefill_phase_ms = (max(stamps) - t_p) * 1e3
@@ -451,8 +451,8 @@ def run_phase(args, mode: str, rank: int, world: int, port: int, model_dir: str)
         "prefill_roofline": {"bound": "mfma", "achieved": pf / (pf_ms * 1e-3) / 1e12, "peak": PREFILL_MFMA_PEAK * tp / 1e12,
                              "unit": "TFLOP/s", "frac": pf / (pf_ms * 1e-3) / (PREFILL_MFMA_PEAK * tp),
                              "flops_per_step": pf, "ms_per_step": pf_ms, "tokens_per_step": per_step * PROMPT_LEN,
-                             # the phase on both clocks: to the last first-token stamp (the definition above, rounds 5+)
-                             # and to the device synchronisation behind it (rounds 1-4; since round 5 that also waits
+                             # the phase on both clocks: to the last first-token stamp (the definition above)
+                             # and to the device synchronisation behind it (that also waits
                              # for the first decode step queued behind the last prefill step)
                              "phase_ms_to_last_stamp": prefill_phase_ms, "phase_ms_to_sync": prefill_phase_to_sync_ms,
                              "what": "the engine's prefill steps (projections + causal attention + head): wall time of the "
@@ -463,7 +463,7 @@ def run_phase(args, mode: str, rank: int, world: int, port: int, model_dir: str)
                           "bytes_per_step": algo / args.steps},
     }
     mr = llm.model_runner
-    if tp > 1:  # what the ranks really ran on: visible to the driver
+    if tp > 1:  # what the ranks really ran on
         result["tp"] = {"world_seen": dist.get_world_size(), "backend": dist.get_backend(),
                         "xgmi_exchange": mr.xgmi is not None, "xgmi_selftest": getattr(mr, "xgmi_selftest", None),
                         "decode_graphs": sorted(mr.graphs), "lookahead": bool(getattr(llm, "lookahead", False))}
@@ -535,7 +535,7 @@ def main():
         torch.cuda.set_device(local)
         os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
         # BENCH_DIST_BACKEND=gloo: functional run of this N > 1 flow with the ranks sharing one GPU
-        # (not a measurement); the driver's runs use RCCL ("nccl"), one GPU per rank
+        # (not a measurement); measurements use RCCL ("nccl"), one GPU per rank
         backend = os.environ.get("BENCH_DIST_BACKEND", "nccl")
         if backend == "nccl":
             dist.init_process_group("nccl", device_id=torch.device("cuda", local))
@@ -583,7 +583,7 @@ def main():
                                                             "roofline", "chain_roofline", "error") if k in tp_run}
                 result["tp_run"].setdefault("n_gpus", world)
         if rank == 0 and result is not None:
-            # north_star: ">= 6x aggregate throughput at TP = 8" - both aggregates as multiples of the one-GPU line
+            # both aggregates as multiples of the one-GPU line
             ref, ref_file = one_gpu_reference()
             if ref:
                 result["speedup_vs_1gpu"] = result["value"] / ref

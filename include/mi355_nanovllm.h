@@ -6,7 +6,7 @@
  * the paged-KV Qwen3 decode path and the prefill that feeds it.
  *
  * The reference has no FFI of its own: its seam is the Python class surface of
- * nanovllm/layers (SURVEY.md §8b).  Every entry point below names the reference
+ * nanovllm/layers.  Every entry point below names the reference
  * call site it stands in for (paths relative to the reference checkout).
  *
  * Conventions (all entry points)
@@ -22,7 +22,7 @@
  *     the reference ops (op_docs/_op_plugin_docs.py:9656-9657, :7123); negative
  *     slots / block ids are skipped.
  *
- * Paged KV cache layout ("fragment-native", DESIGN.md §3)
+ * Paged KV cache layout ("fragment-native")
  *   One layer's K (or V) cache is   [num_blocks][n_kv_heads][block_size/16][2048] bf16,
  *   i.e. one 4 KiB tile per (16 consecutive slots of a block, kv head); head_dim = 128.
  *   Element (t = slot%16, d) of a K tile sits at  (d/32)*512 + (((d%32)/8)*16 + t)*8 + d%8,
@@ -74,7 +74,7 @@ const char* mi_last_launch_error(void);
  * knob or a value outside its range.  (The Python binding maps its MI355_* A/B environment switches onto these at
  * import time: nanovllm/_C.py.) */
 enum mi_tuning_knob {
-  MI_TUNE_ATTN_PIPE = 0,          /* mi_paged_attn_decode: 1 (default) = 8 waves x two chunks in flight, 0 = round-1 16-wave form */
+  MI_TUNE_ATTN_PIPE = 0,          /* mi_paged_attn_decode: 1 (default) = 8 waves x two chunks in flight, 0 = the 16-wave form */
   MI_TUNE_ATTN_RESOLVE = 1,       /* decode attention resolves its block-id run at kernel start (default 0: measured slower)    */
   MI_TUNE_NORM_WPR = 2,           /* mi_add_rmsnorm_splitk: waves per row for <= 64 rows: 4 (default), 2, 1                     */
   MI_TUNE_ROPE_BLOCK64 = 3,       /* mi_qknorm_rope_store: one-wave workgroups for <= 64 tokens (default 1)                     */
@@ -225,12 +225,12 @@ int mi_paged_attn_prefill_fused(const mi_bf16* qkv, int64_t qkv_row_stride, cons
  * as bf16 hi + lo (what MI_TUNE_PREFILL_P_SPLIT selects process-wide; every group size).  Schedule variants, for
  * n_q_heads / n_kv_heads == 2 only (the bench model; MI_EUNSUPPORTED otherwise), same results as variant 0 bit for
  * bit (tests): 1 = the first two K/V chunks requested ahead of the Q preparation; 2 = one workgroup barrier per two
- * chunks; 8 = round 3's V operand reads (ds_read2st64_b64: LDS bank conflicts); 16 = round 3's request path (table
- * read + divisions in front of every chunk request); 24 = 8 + 16; 28 = the round-3 kernel as a whole (4 + 8 + 16);
- * 32 = round 5's softmax (the chunk maximum BEFORE the exponentials; the product tests the lane's sum of exponentials
+ * chunks; 8 = the former V operand reads (ds_read2st64_b64: LDS bank conflicts); 16 = the former request path (table
+ * read + divisions in front of every chunk request); 24 = 8 + 16; 28 = the earliest kernel as a whole (4 + 8 + 16);
+ * 32 = the former softmax (the chunk maximum BEFORE the exponentials; the product tests the lane's sum of exponentials
  * instead and computes a maximum only when the reference point has to move: the same results wherever both rescale in
- * the same chunks); 64 = round 5's request addressing (per-lane 64-bit pointers + global_load_lds; the product keeps the
- * tile address on the scalar unit: buffer_load ... lds); 96 = the round-5 kernel as a whole.  The round-3 forms
+ * the same chunks); 64 = the former request addressing (per-lane 64-bit pointers + global_load_lds; the product keeps the
+ * tile address on the scalar unit: buffer_load ... lds); 96 = 32 + 64.  The earliest forms
  * (8, 16, 24, 28) include 96: they are the kernels that were measured then. */
 int mi_paged_attn_prefill_fused_ex(const mi_bf16* qkv, int64_t qkv_row_stride, const mi_bf16* q_w, float eps,
                                    const int64_t* positions, const float* cos_sin, const mi_bf16* k_cache,
@@ -328,7 +328,7 @@ int mi_gemm_bf16(const mi_bf16* x, int64_t ldx, const mi_bf16* w, const mi_bf16*
 int mi_gemm_bf16_splitk(const mi_bf16* x, int64_t ldx, const mi_bf16* w, float* partials, int M, int N, int K, int ksplit,
                         mi_stream stream);
 /* The packed qkv projection of a prefill step with the K / V side of qwen3.py:79-90 + attention.py:55-58 in its
- * epilogue (round 4): qkv[M][N] = x @ w^T (+ bias) as mi_gemm_bf16, but only the q heads (columns
+ * epilogue: qkv[M][N] = x @ w^T (+ bias) as mi_gemm_bf16, but only the q heads (columns
  * [0, n_q_heads * 128)) are written to `qkv`; every k head is k-normed (k_w, or NULL: none), rotated (positions,
  * cos_sin as mi_qknorm_rope_store) and stored into k_cache, every v head into v_cache, at `slots` (flat int32 [M]:
  * block * block_size + offset; negative = not stored) in the fragment-native tile layout - the same bits
@@ -490,7 +490,7 @@ int mi_gather_last_tokens(const mi_bf16* x, const int32_t* cu_seqlens_q,
 
 /* ---- sampling (reference: layers/sampler.py:9-17) ------------------------- */
 /* Greedy token = lowest index of the row maximum of logits[rows][vocab] (the
- * deterministic path BASELINE config 1 needs; the reference itself only has
+ * deterministic path; the reference itself only has
  * multinomial sampling).  out [rows] int64. */
 int mi_argmax(const mi_bf16* logits, int64_t row_stride, int64_t* out,
               int rows, int vocab, mi_stream stream);
@@ -535,7 +535,7 @@ int mi_logits_pick(const mi_bf16* logits, int M, int N, const float* temperature
 int mi_pick_final(const void* candidates, int n_groups, int rows, int64_t* out,
                   mi_stream stream);
 
-/* ---- fp8 (e4m3) weights, bf16 activations (BASELINE.json configs[4]) --------
+/* ---- fp8 (e4m3) weights, bf16 activations --------
  * No reference semantics exist (the reference is bf16 only): y = x @ (w_q * scale[:, None])^T with
  * w_q OCP e4m3 values and one fp32 scale per weight row (output feature).  Decode GEMMs are bound
  * by the weight stream, not by MFMA rate, so the weights are dequantised to bf16 in registers
@@ -549,7 +549,7 @@ int mi_gemm_fp8w_packed(const mi_bf16* x, const uint8_t* w_packed, const float* 
 int mi_gemm_fp8w_packed_splitk(const mi_bf16* x, const uint8_t* w_packed, const float* scale,
                                float* partials, int M, int N, int K, int ksplit, mi_stream stream);
 
-/* ---- mixture of experts (reference: models/qwen3_moe.py:125-185, BASELINE.json configs[3]) -------------
+/* ---- mixture of experts (reference: models/qwen3_moe.py:125-185) -------------
  * Qwen3MoeSparseMoeBlock.forward as five launches over expert-sorted (token, expert) pairs; P = n_tokens * top_k.
  * The reference loops over the selected experts in Python with three library GEMMs each (:171-184).
  * Expert weights: one fragment-native slab (mi_pack_weight layout) per expert, stacked: gate_up

@@ -9,7 +9,7 @@
 The same random draws in the same order as the reference script (Python's `random`, seed 0), so the token counts are
 the reference's: 133 966 output tokens (README.md:338: "133 966 tok / 75.89 s").  `--max-num-seqs` is the knob the
 reference's table varies (README.md:337-342: 1249 tok/s at 16 ... 3954 tok/s at 256 on an Ascend 910C - other
-hardware, listed in BASELINE.md section 1 for context only).  Synthetic mode: a model directory holding only config.json
+hardware).  Synthetic mode: a model directory holding only config.json
 gets random weights (Config); the prompts are random ids either way, as in the reference.
 
     python bench/throughput_bench.py --model DIR [--max-num-seqs 256] [--num-seqs 256]

@@ -5,7 +5,7 @@
 //     k_cache / v_cache  [num_blocks][n_kv_heads][block_size][head_dim]  bf16
 //
 // (a token's head row is contiguous: 128 or 256 bytes), and kernels written for coverage first:
-//   * mi_kv_store_plain          K1/K2 of SURVEY 2.2: flat slots (prefill) or [block, offset] pairs (decode)
+//   * mi_kv_store_plain          flat slots (prefill) or [block, offset] pairs (decode)
 //   * mi_rope_plain              NeoX rotation with the reference's fp32 roundings (rotary_embedding.py:6-14)
 //   * mi_paged_attn_decode_plain one workgroup per (sequence, kv head, context split): a wave-load is 1 KiB = 4 or 8 whole
 //                                token rows; scores by fp32 dot products (8 dims per lane, shuffle tree over the row's

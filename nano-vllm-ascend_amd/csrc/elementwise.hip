@@ -532,7 +532,7 @@ __global__ __launch_bounds__(128) void qkv_prefill_store_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// head_dim 64 (round 4: Llama-3.2-1B, Qwen2-0.5B on the fragment-native attention kernels): the same tile formulas
+// head_dim 64 (Llama-3.2-1B, Qwen2-0.5B on the fragment-native attention kernels): the same tile formulas
 // (k_tile_off / v_tile_off do not depend on the head width), a 16-token tile is the first 1024 elements = 2 KiB.
 // Pure copies of already rotated K rows and of V rows (the q/k-norm + RoPE fusions above are written for 128-wide
 // heads; models of this width have no q/k norm and take mi_rope_plain first).

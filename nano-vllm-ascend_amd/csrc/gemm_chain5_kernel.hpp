@@ -1,4 +1,4 @@
-// The decode chain in FIVE launches per layer (VERDICT r05 item 1): the row-parallel projections (o_proj, down_proj)
+// The decode chain in FIVE launches per layer: the row-parallel projections (o_proj, down_proj)
 // deliver complete rows, add the residual and emit the RMSNorm statistic; the column-parallel consumers (qkv,
 // gate_up + SwiGLU) normalise their own K-slice on load.  The two add+RMSNorm launches of the seven-launch layer
 // (mi_add_rmsnorm_splitk) disappear.
@@ -10,7 +10,7 @@
 //                                   built in the wave's LDS slab for its K-slice only, under weight loads already in flight
 //   tail      norm_from_stat_kernel the model's final norm from (s, stat)
 //
-// No cross-workgroup hand-off inside a launch (on this part one costs more than a kernel boundary, DESIGN.md section 5):
+// No cross-workgroup hand-off inside a launch (on this part one costs more than a kernel boundary):
 // a workgroup of the producer owns 16 output features of EIGHT activation rows over the whole K, so a tile's weights are
 // read by ceil(M / 8) workgroups (from L2 after the first) and nothing has to be summed across workgroups.
 //

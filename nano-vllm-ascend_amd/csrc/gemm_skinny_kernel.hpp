@@ -633,8 +633,7 @@ __global__ __launch_bounds__(WAVES * 64) void head_stream_kernel(const uint16_t*
 }
 
 // shapes the persistent head kernel takes: bf16 weights, no bias, vocabulary-sized N (>= 2048 tile pairs), and
-//   K = 1024 (Qwen3-0.6B: 8 waves x 128)   up to 64 rows (round 4: bs 64 = BASELINE.json configs[4], VERDICT r03 weak 6 -
-//                                           above 32 rows the head used to fall back to 4748 short-lived workgroups)
+//   K = 1024 (Qwen3-0.6B: 8 waves x 128)   up to 64 rows (the other kernel's head: 4748 short-lived workgroups)
 //   K =  896 (Qwen2-0.5B: 7 waves x 128)   up to 48 rows (one epilogue item per thread: 2 * MT * 64 <= 448)
 //   K = 2048 (Llama-3.2-1B: 8 waves x 256) up to 32 rows (x slices of 64 rows would not fit the register file)
 static bool head_stream_fits(int M, int N, int K) {

@@ -47,7 +47,7 @@ namespace mi {
 
 // Tuning variants of the eight-wave kernel below (mi_gemm_bf16_ex instantiates the combinations it lists - the staggered
 // start V & 1024 and the never-waited DMA V & 256 measured no effect and are not instantiated any more; the timing-only
-// ablations lived in round 4's EXPERIMENTS=1 build flavour, removed in round 5 - their numbers are in
+// ablations lived in an EXPERIMENTS=1 build flavour, since removed - their numbers are in
 // profiles/r04_gemm_ablation.txt; the product entry point uses kDefaultV on the four-wave kernels):
 //   V & 2    both waves of a SIMD in lockstep (no one-barrier stagger)
 //   V & 4    XCD-rectangle tile order instead of the plain one (tile_of_block; measured equal or slower)
@@ -459,8 +459,8 @@ static int tile_ksplit(int M, int N, int K) {
 // The large-M kernel: gemm_w16_kernel (four waves, v_mfma_f32_16x16x32_bf16), with whole-line output stores
 // (kLineStores) wherever the output allows it: full feature tiles, 16-byte aligned rows, 32-bit byte offsets.
 // Tuning / comparison variants: V & kDirectStores keeps the direct stores; V & kMfma32 = the same kernel on
-// v_mfma_f32_32x32x16_bf16 (gemm_w4_kernel: the first form of round 4, still the qkv-store kernel); V & kEightWaves = the
-// eight-wave ping-pong kernel of rounds 2-3.
+// v_mfma_f32_32x32x16_bf16 (gemm_w4_kernel: the first form, still the qkv-store kernel); V & kEightWaves = the
+// eight-wave ping-pong kernel before both.
 constexpr int kEightWaves = 1 << 20, kMfma32 = 1 << 19, kLineStores = 32768, kDirectStores = 1 << 18;
 template <int EPI, bool BIAS, int V = kDefaultV>
 static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
@@ -674,7 +674,7 @@ extern "C" int mi_gemm_bf16_ex(const mi_bf16* x, int64_t ldx, const mi_bf16* w, 
     // the same kernel on 32 x 32 x 16 MFMAs
     case kMfma32: return launch_tile<TEPI_NONE, false, kMfma32>(a, st);
     case kMfma32 + kDirectStores: return launch_tile<TEPI_NONE, false, kMfma32 + kDirectStores>(a, st);
-    // the eight-wave kernel of rounds 2-3 and its variants
+    // the eight-wave kernel and its variants
     case kEightWaves: return launch_tile<TEPI_NONE, false, kEightWaves>(a, st);
     case kEightWaves + 2: return launch_tile<TEPI_NONE, false, kEightWaves + 2>(a, st);
     case kEightWaves + 16: return launch_tile<TEPI_NONE, false, kEightWaves + 16>(a, st);

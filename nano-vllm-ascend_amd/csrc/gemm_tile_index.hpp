@@ -97,7 +97,7 @@ struct MidShape {
 using Mid128 = MidShape<2, 2, 2, 2>;
 static_assert(Mid128::F == MID_F && Mid128::T == MID_T, "the 128 x 128 tile");
 
-// ---- the four-wave 256 x 256 x 64 kernel (gemm_w4_kernel, the product kernel for large M since round 4) ----
+// ---- the four-wave 256 x 256 x 64 kernel (gemm_w4_kernel, the qkv-store kernel) ----
 // One wave per SIMD: fw = wave >> 1 (128 features), tw = wave & 1 (128 tokens), wave tile 128 x 128 = 4 x 4 accumulators.
 // One K step of the tile in LDS is ONE image of 64 PIECES: a piece is what one `buffer_load_dwordx4 ... lds` wave
 // instruction lands - 1 KiB = eight 128-byte row slices (lane l -> slice l >> 3, 16-byte chunk l & 7: the eight lanes

@@ -1,5 +1,5 @@
 // The 256 x 256 x 64 tile GEMM with ONE wave per SIMD (four waves, 512 registers each, wave tile 128 x 128): the
-// product kernel for the compute-bound shapes since round 4.  Included by gemm_tile.hip (TileArgs, TEPI_*, namespace mi).
+// product kernel for the compute-bound shapes before gemm_w16_kernel.  Included by gemm_tile.hip (TileArgs, TEPI_*, namespace mi).
 //
 // Why this shape.  The chip is power-limited under bf16 MFMA load (1.6-1.75 GHz): what a schedule buys is issue
 // cycles per K step, and tools/ubench/gemm_feed.hip measures them for a loop of exactly this form - 2165 cycles per K
@@ -332,8 +332,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const TileArgs a) {
     store_lines(NSLAB - 1);
   };
 
-  // ---- TEPI_QKV: the packed qkv projection whose K and V heads never reach the qkv rows (
-  // qwen3.py:79-90 + attention.py:55-58 of the reference: split, k-norm, RoPE, store_kvcache).  head_dim 128: a wave's
+  // ---- TEPI_QKV: the packed qkv projection whose K and V heads never reach the qkv rows
+  // (qwen3.py:79-90 + attention.py:55-58 of the reference: split, k-norm, RoPE, store_kvcache).  head_dim 128: a wave's
   // 128 features are exactly ONE head (q, k or v - wave-uniform).  Q heads: the ordinary whole-line stores (the
   // attention kernel norms and rotates q in its operand load).  K heads: after the epilogue's half-wave exchange the
   // lane pair (hi = 0 / 1) of a token holds the head as 8-dim groups 2 kk + hi - the distribution of
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const TileArgs a) {
     }
   };
   read_first_groups();
-  // V & 4096 (measurement; round 4 read it with tools/gemm_clock.py, numbers in profiles/r04_gemm_clock.txt): shader cycles and 100 MHz reference ticks of the whole tile loop of
+  // V & 4096 (measurement; read with tools/gemm_clock.py, numbers in profiles/r04_gemm_clock.txt): shader cycles and 100 MHz reference ticks of the whole tile loop of
   // every workgroup, written over the first output bytes when everything else is done
   unsigned long long clk0 = 0, ref0 = 0;
   if (V & 4096) {

@@ -27,8 +27,8 @@
 
 namespace mi {
 
-// DB = head_dim / 32: 4 for the 128-wide heads every kernel here was written around, 2 for head_dim 64 (round 4:
-// Llama-3.2-1B, Qwen2-0.5B - the first DB * 512 elements of the same tile formulas: a 2 KiB tile per 16 tokens)
+// DB = head_dim / 32: 4 for the 128-wide heads every kernel here was written around, 2 for head_dim 64
+// (Llama-3.2-1B, Qwen2-0.5B - the first DB * 512 elements of the same tile formulas: a 2 KiB tile per 16 tokens)
 template <int DB>
 __device__ __forceinline__ void load_tile(const uint16_t* __restrict__ tile, int lane, u32x4 (&f)[DB]) {
 #pragma unroll
@@ -334,7 +334,7 @@ __device__ __forceinline__ void patch_new_token(u32x4 (&K)[4], u32x4 (&V)[4], co
   }
 }
 
-// PIPE = false: the round-1 geometry - 16 waves x 128 VGPRs, one chunk per wave in flight (load all,
+// PIPE = false: the first geometry - 16 waves x 128 VGPRs, one chunk per wave in flight (load all,
 //   attend, load the next), overlap comes from the 16 waves being in different phases.
 // PIPE = true: 8 waves x 256 VGPRs, TWO chunks per wave in flight: chunk i+2 is requested as soon as
 //   chunk i has been consumed, so every wave keeps 16-32 KiB of loads outstanding while it computes
@@ -679,12 +679,12 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(const float* __re
 // ---------------------------------------------------------------------------
 // (f32x16, kDeferMax, xor32_max / xor32_sum, QPrep: prefill_common.hpp)
 
-// Probabilities in the second product.  SPLIT_P = false (the default since round 4): P is ONE bf16 per key, as in
+// Probabilities in the second product.  SPLIT_P = false (the default): P is ONE bf16 per key, as in
 // the reference's own CPU statement of this operator (attention_torch_native.py:80,127,139,188-189 keeps the scale, S
 // and P in bf16; the fp32 running sum l is taken from the un-rounded exponentials): 16 instead of 24 MFMAs and ~50
 // VALU instructions fewer per 32-key chunk in an issue-bound loop.  Bound: |out - fp32 oracle| <= 2^-7 |out| + 1e-4
 // (1 bf16 ulp of the output instead of 1/2; tests/test_kernels_gpu.py).  SPLIT_P = true (tuning knob
-// MI_TUNE_PREFILL_P_SPLIT, the round-1..3 form): P as bf16 hi + lo, two MFMAs per product, <= 1/2 ulp.
+// MI_TUNE_PREFILL_P_SPLIT, the first form): P as bf16 hi + lo, two MFMAs per product, <= 1/2 ulp.
 
 // one hand-issued ds_read_b64 at LDS byte address `addr` + OFF (see PV_READ2 below).  NOT counted by hipcc: the caller
 // waits with its own asm s_waitcnt lgkmcnt naming the destination "+v" before the first use.
@@ -696,24 +696,24 @@ __device__ __forceinline__ void lds_read64_uncounted(uint64_t& dst, uint32_t add
 
 // Variant bits VAR (mi_paged_attn_prefill_fused_ex; the product entry points use 0, or PV_SPLIT_P under the tuning knob):
 //   PV_EARLY   the first two chunks are requested ahead of the Q preparation instead of behind it (stress test)
-//   PV_PAIR    a ring of four buffers and ONE barrier per TWO chunks (measured slower in round 3)
+//   PV_PAIR    a ring of four buffers and ONE barrier per TWO chunks (measured slower)
 //   PV_SPLIT_P P as bf16 hi + lo (see above)
-//   PV_READ2   round 3's V operand reads: the two 8-byte pieces of a fragment through ordinary loads, which hipcc
+//   PV_READ2   the former V operand reads: the two 8-byte pieces of a fragment through ordinary loads, which hipcc
 //              merges into ONE ds_read2st64_b64 - an instruction served in 16-lane groups on 32 banks, where this
 //              layout (16-byte lane stride) is a 2-way conflict: 16 LDS cycles per fragment, 38.6 % of all LDS cycles
 //              of the kernel (profiles/r03_prefill_attention_pmc.txt: SQ_LDS_BANK_CONFLICT 8.65 M = 8 extra cycles x
 //              8 instructions x 16.5 chunks x 8192 waves, to the digit).  Default now: two un-merged ds_read_b64
 //              (32-lane groups on 64 banks: the same addresses are conflict-free, 2 cycles each).
-//   PV_NOPREF  round 3's block-table read: s_load + s_waitcnt right in front of every chunk request.  Default now: the
+//   PV_NOPREF  the former block-table read: s_load + s_waitcnt right in front of every chunk request.  Default now: the
 //              block id of the NEXT request is read one chunk ahead, so the wait finds it landed.
-//   PV_MAXTREE round 5's softmax: the chunk's maximum (a v_max3 tree over the sixteen scores, one v_permlane32_swap) BEFORE
+//   PV_MAXTREE the former softmax: the chunk's maximum (a v_max3 tree over the sixteen scores, one v_permlane32_swap) BEFORE
 //              the exponentials, to decide whether the reference point has to move.  Default now: the exponentials are
 //              taken against the current reference point at once and the lane's sum of them - which the running sum needs
 //              anyway - is the test: a sum <= 2^8 bounds every probability by 2^8, the invariant the deferred rescale
 //              keeps; only when some lane's sum exceeds it (the first chunk, a maximum that ran away) is the maximum
 //              computed, the state rescaled and the chunk's exponentials redone.  ~22 VALU instructions per chunk less
 //              in a loop that is bound by its VALU issue (profiles/r05_prefill_attention_pmc.txt).
-//   PV_VADDR   round 5's request addressing: a per-lane 64-bit pointer (five v_lshl_add_u64 + the block-table index kept
+//   PV_VADDR   the former request addressing: a per-lane 64-bit pointer (five v_lshl_add_u64 + the block-table index kept
 //              in a VGPR: ~13 VALU per chunk) and global_load_lds.  Default now: the tile's address stays on the scalar
 //              unit - a buffer descriptor whose base is the cache block, lane * 16 as the only vector offset - and the
 //              request is buffer_load_dwordx4 ... lds.
@@ -854,7 +854,7 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
     issue(1);
   }
   // (Scores one chunk ahead of the softmax - the eight dependent score MFMAs of chunk c + 1 in the basic block of
-  // chunk c's exponentials, a fourth ring buffer - was built and measured in round 3: 145-147 us against 137-139
+  // chunk c's exponentials, a fourth ring buffer - was built and measured: 145-147 us against 137-139
   // for this form at 16 x 1024 tokens; removed.)
   auto attend = [&](int c, int buf) __attribute__((always_inline)) {  // buf = c % NBUF
     if (c < wave_chunks) {
@@ -1007,7 +1007,7 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
     }
   } else {
     // The same loop with the request side kept as running state - no division, no modulo, no table read in front
-    // of a request (the round-3 form spends ~90 scalar instructions per chunk and wave on them, and the scalar unit
+    // of a request (PV_NOPREF spends ~90 scalar instructions per chunk and wave on them, and the scalar unit
     // is shared by the CU's twelve waves).  Request r (= min(c + 2, wg_chunks - 1), i.e. saturating: past the end
     // the last chunk is requested again into its own slot, which keeps the vmcnt arithmetic uniform) fetches tile
     // rq_t = min(2 r + odd, t_max) = block-table entry rq_bi, tile rq_in of that block, into ring slot rq_slot;
@@ -1328,7 +1328,7 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
     switch (variant) {
       case PV_EARLY: LAUNCH_PRE_AS(2, true, PV_EARLY); break;
       case PV_PAIR: LAUNCH_PRE_AS(2, true, PV_PAIR); break;
-      // the round-3 forms are the round-3 kernels: with the maximum before the exponentials and per-lane request
+      // PV_READ2 and PV_NOPREF are the earliest kernels: with the maximum before the exponentials and per-lane request
       // pointers (PV_MAXTREE | PV_VADDR), as they were measured.  (Merged V reads + P as hi + lo on top of the
       // sum-checked softmax gave wrong, run-to-run different results with this compiler - tools/debug/
       // prefill_variant_determinism.py, variants 12 / 28 of a test build; every form offered here reproduces itself
@@ -1336,12 +1336,12 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
       case PV_READ2: LAUNCH_PRE_AS(2, true, PV_READ2 | PV_MAXTREE | PV_VADDR); break;
       case PV_NOPREF: LAUNCH_PRE_AS(2, true, PV_NOPREF | PV_MAXTREE | PV_VADDR); break;
       case PV_READ2 | PV_NOPREF: LAUNCH_PRE_AS(2, true, PV_READ2 | PV_NOPREF | PV_MAXTREE | PV_VADDR); break;
-      case PV_SPLIT_P | PV_READ2 | PV_NOPREF:  // round 3
+      case PV_SPLIT_P | PV_READ2 | PV_NOPREF:
         LAUNCH_PRE_AS(2, true, PV_SPLIT_P | PV_READ2 | PV_NOPREF | PV_MAXTREE | PV_VADDR);
         break;
       case PV_MAXTREE: LAUNCH_PRE_AS(2, true, PV_MAXTREE); break;
       case PV_VADDR: LAUNCH_PRE_AS(2, true, PV_VADDR); break;
-      case PV_MAXTREE | PV_VADDR: LAUNCH_PRE_AS(2, true, PV_MAXTREE | PV_VADDR); break;  // round 5
+      case PV_MAXTREE | PV_VADDR: LAUNCH_PRE_AS(2, true, PV_MAXTREE | PV_VADDR); break;
       default: return MI_EUNSUPPORTED;
     }
     return check_launch();

@@ -8,7 +8,7 @@ Differences, all forced by the platform:
   * `hccl_port` keeps its name; it is the TCP rendezvous port of the RCCL group.
   * a model directory holding only `config.json` (no *.safetensors) selects
     synthetic random weights N(0, 0.02^2) seeded by `synthetic_seed`
-    (there are no checkpoints on the GPU box).
+    (for machines without checkpoints).
 """
 from __future__ import annotations
 

@@ -55,7 +55,7 @@ def prefill_meta(seqs: list[Sequence], block_size: int, skip_cached: bool = Fals
     """skip_cached=False is the reference: every token of every scheduled sequence is (re)computed -
     cached prefix blocks are not skipped (model_runner.py:248-249) - positions restart at 0.
 
-    skip_cached=True (SURVEY.md 8f.2) feeds only the tokens behind the leading cache hits
+    skip_cached=True feeds only the tokens behind the leading cache hits
     (`num_prefix_tokens`, whole blocks): queries start at that position, their K/V rows go to the
     slots of the non-shared blocks, and attention reaches the shared prefix through the block
     table (kv_lens stays the full length).  A fully cached prompt still computes its last token

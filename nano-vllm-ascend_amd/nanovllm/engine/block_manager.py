@@ -1,5 +1,5 @@
 """Paged-KV block allocator with chained-hash prefix caching
-(reference: nanovllm/engine/block_manager.py:26-118; semantics in SURVEY.md §9).
+(reference: nanovllm/engine/block_manager.py:26-118).
 
 Block tables are part of the parity contract: for the same request stream this
 allocator must hand out the same block ids, in the same order, as the reference's.

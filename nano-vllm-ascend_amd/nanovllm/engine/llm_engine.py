@@ -418,7 +418,7 @@ class LLMEngine:
         if not isinstance(sampling_params, list):
             sampling_params = [sampling_params] * len(prompts)
         # every prompt is checked before any is queued: one over-long prompt must not leave the others behind in the
-        # scheduler as orphans of a call that raised (ADVICE r04)
+        # scheduler as orphans of a call that raised
         if any(isinstance(p, str) for p in prompts):
             if self.tokenizer is None:
                 raise ValueError("this model directory has no tokenizer: pass token ids")

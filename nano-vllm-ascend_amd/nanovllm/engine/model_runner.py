@@ -858,7 +858,7 @@ class ModelRunner(RowSteps):
 
     @torch.inference_mode()
     def run(self, seqs: list[Sequence], is_prefill: bool) -> list[int] | None:
-        if not seqs:  # everything got preempted this step (reference would crash)
+        if not seqs:  # everything got preempted this step (the reference would crash)
             return []
         if self.hybrid:
             return self.run_hybrid(seqs, is_prefill)
@@ -1027,7 +1027,7 @@ class ModelRunner(RowSteps):
                                f"{self.xgmi.timeout_info()}")
 
     def _abort_workers(self):
-        """Rank 0 is about to raise: tell the workers to leave their receive loops (they kept spinning)."""
+        """Rank 0 is about to raise: tell the workers to leave their receive loops (they would keep spinning)."""
         if self.channel is not None and self.rank == 0 and not getattr(self, "_aborted", False):
             self._aborted = True
             self.channel.send("abort")

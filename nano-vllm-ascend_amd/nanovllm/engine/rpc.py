@@ -13,7 +13,7 @@ message:
 one, engine lookahead) the row of the previous step's token buffer each sequence's input id comes from.  The body
 (payload then extra) of a message that does not fit one slot continues in the following slots (`more` = 1 on every
 part but the last): a prefill step ships the token ids behind each sequence's cached prefix, and with prefix-cache
-hits the scheduler's token budget does not bound that sum by one slot (ADVICE r04: 57 sequences sharing a prefix made a
+hits the scheduler's token budget does not bound that sum by one slot (57 sequences sharing a prefix made a
 117 819-word step against a 25 094-word slot) - a slot is the unit of transfer, not a limit on a step.
 
 Messages live in a ring of four slots; a worker consumes them in order and acknowledges each part it has copied out
@@ -52,7 +52,7 @@ class ChannelError(RuntimeError):
 def slot_words(max_num_batched_tokens: int, max_num_seqs: int, max_model_len: int, block_size: int) -> int:
     """int64 words of a slot: what a step message normally needs in ONE part - a prefill step carries the scheduled
     token ids once, every step up to max_num_seqs records of 11 header words + a block table (Sequence.to_wire) - sized
-    from the configuration (ADVICE r03: four fixed 16 MiB slots were just over Docker's default 64 MB /dev/shm, which
+    from the configuration (four fixed 16 MiB slots were just over Docker's default 64 MB /dev/shm, which
     RCCL also uses).  Longer messages (prefix-cache hits, see the module text) travel in several parts."""
     table = -(-(max_model_len + 1) // block_size)
     return _HEADER + max_num_batched_tokens + max_num_seqs * (12 + table + 1) + 1024
@@ -125,7 +125,7 @@ class StepChannel:
             piece = body[k * room:(k + 1) * room]
             gen = self.generation + 1
             # (teardown messages: a worker that is gone never acknowledges - give up on it quickly, the caller goes on
-            # to terminate the ranks, ADVICE r05)
+            # to terminate the ranks)
             self._wait_for_slot(gen, TEARDOWN_ACK_TIMEOUT_S if method in ("exit", "abort") else ACK_TIMEOUT_S)
             b = self.buf[_BASE + (gen % _SLOTS) * self.capacity:]
             b[0] = 0  # the slot is being rewritten

@@ -1,5 +1,5 @@
 """Prefill-first continuous batching with preemption
-(reference: nanovllm/engine/scheduler.py:41-110; semantics in SURVEY.md §9).
+(reference: nanovllm/engine/scheduler.py:41-110).
 
 The schedule determines which block tables / slot mappings reach the device, so it
 is reproduced decision for decision: prefill has absolute priority and admits from
@@ -234,7 +234,7 @@ class Scheduler:
           the prompts' full lengths; the real admission charges only the tokens behind cache hits and may then reach
           the end of the queue after all - such a step is the same for the requests in it, but a request arriving
           meanwhile joins the NEXT step instead of this one: batching under arrivals, not block ids or tokens, may
-          differ from the synchronous engine there - ADVICE r04);
+          differ from the synchronous engine there);
         * the step in flight is long enough (min_inflight_tokens) for the next one's launch sequence to hide behind it -
           queueing a step behind a short one would only delay the short one's tokens.
 

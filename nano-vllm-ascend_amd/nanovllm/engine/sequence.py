@@ -3,7 +3,7 @@
 Text-only (the multimodal fields of the reference are outside the decode path).
 The rank-RPC wire format is a flat int64 array (``to_wire`` / ``from_wire``) rather
 than the reference's pickled dict (sequence.py:116-146), which ships every
-token id each step and drops ``block_size`` (SURVEY.md §3.5).
+token id each step and drops ``block_size``.
 """
 from __future__ import annotations
 

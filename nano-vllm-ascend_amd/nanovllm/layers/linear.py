@@ -17,7 +17,7 @@ from nanovllm.layers.parallel import all_reduce_sum, divide, tp_rank, tp_size
 
 def tile_gemm_takes(rows: int, n: int, k: int) -> bool:
     """mi_gemm_bf16's shape contract (csrc/gemm_tile.hip: K steps of 64, 16-byte output pieces, 32-bit DMA offsets),
-    asked of the library (mi_gemm_bf16_max_rows) instead of restated here (the restatement had drifted).
+    asked of the library (mi_gemm_bf16_max_rows) instead of restated here (a restatement had drifted).
     The row count does not matter as long as one whole tile row fits: ops.gemm_tile walks longer activations through the
     kernel in whole-tile row pieces."""
     return ops.tile_gemm_max_rows(n, k) >= min(max(rows, 1), 256)
@@ -30,7 +30,7 @@ def streaming_gemm_takes(n: int, k: int) -> bool:
 
 def check_linear_shape(name: str, n: int, k: int) -> None:
     """Start-up validation (ModelRunner): a projection no kernel family takes must fail when the model is built, not
-    in the middle of a prefill step (ADVICE r03)."""
+    in the middle of a prefill step."""
     if not (streaming_gemm_takes(n, k) or tile_gemm_takes(1, n, k)):
         raise NotImplementedError(
             f"{name}: a [{n} x {k}] projection fits neither the streaming GEMMs (N % 16, K % 32) nor the tile GEMM "
@@ -62,7 +62,7 @@ def linear_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
         # more rows than one streaming launch takes AND a shape the tile kernel cannot take (K % 64 == 32: e.g. an
         # intermediate size of 11008 over 8 ranks = 1376; an operand of 4 GiB or more): the streaming kernels over the
         # rows in pieces of SKINNY_MAX_M - every piece re-streams the weight, correct and slow, instead of an error in
-        # the middle of a prefill step (the reference's F.linear takes any shape; ADVICE r03)
+        # the middle of a prefill step (the reference's F.linear takes any shape)
         x2 = x.reshape(-1, shape[-1])
         y = torch.empty((rows, n), dtype=x.dtype, device=x.device)
         for r0 in range(0, rows, ops.SKINNY_MAX_M):

@@ -43,7 +43,7 @@ def divide(numerator: int, denominator: int) -> int:
     return numerator // denominator
 
 
-# ---- collectives on a group of ONE rank (a hardware-bring-up hook, VERDICT r03 item 3) -------------------------
+# ---- collectives on a group of ONE rank (a hardware-bring-up hook) -------------------------
 # Every branch that calls RCCL (`dist.get_backend() == "nccl"`) is otherwise reachable only with several GPUs.  With
 # MI355_TP1_COLLECTIVES=1 a tensor_parallel_size == 1 engine creates an RCCL group of world size 1 and takes the
 # collective code paths it would take as one of n ranks whose xGMI exchange is unavailable: RCCL all-reduce behind the
@@ -91,7 +91,7 @@ def group_all_reduce(t, op=None):
 
 
 def all_reduce_sum(t):
-    """C1/C2 of SURVEY.md §2.2: SUM over the TP ranks, in place.  Decode-sized bf16 vectors take
+    """SUM over the TP ranks, in place.  Decode-sized bf16 vectors take
     the one-shot xGMI kernel (mi_allreduce_sum_bf16, hipGraph-capturable, one launch); everything
     else (prefill-sized activations) the RCCL all-reduce."""
     if collectives_on():

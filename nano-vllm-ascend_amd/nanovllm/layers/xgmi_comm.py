@@ -24,7 +24,7 @@ class XgmiComm:
         # What an EAGER launch may put through the region (ModelRunner sets it to the decode-sized rows): the region is
         # also sized for captured prefill steps, whose ranks replay the same graph together; an eager prefill step's ranks
         # arrive at their collectives host-skewed by whole launch sequences, and its prefill-sized all-reduces stay on the
-        # process group (RCCL) as in rounds 1-5.  `large()` lifts the cap while a prefill graph is captured.
+        # process group (RCCL).  `large()` lifts the cap while a prefill graph is captured.
         self.eager_max_bytes = int(max_bytes)
         self._large = 0
         self._peers: list[int] = []

@@ -82,8 +82,8 @@ class Qwen3Attention(nn.Module):
     def _kv_store_in_projection(self, x: torch.Tensor) -> bool:
         """A prefill step whose qkv projection can carry k-norm + RoPE + the K / V cache store in its epilogue
         (mi_gemm_bf16_qkv_store): the large-M tile kernel's shapes, head_dim 128, plain bf16 weights.  OPT-IN
-        (MI355_QKV_STORE=1): bit-identical caches, but measured slower than the two launches it replaces (DESIGN.md
-        section 4.4: 162 vs 147 us per layer at 16 x 1024 tokens) - with one wave per SIMD the epilogue's dependent
+        (MI355_QKV_STORE=1): bit-identical caches, but measured slower than the two launches it replaces (162 vs 147 us
+        per layer at 16 x 1024 tokens) - with one wave per SIMD the epilogue's dependent
         table loads have nothing to hide behind."""
         ctx, proj = get_context(), self.qkv_proj
         return (self.fused and ctx.is_prefill and self.attn.k_cache.numel() > 0 and self.attn.fusable and x.is_cuda
@@ -307,7 +307,7 @@ class Qwen3Model(nn.Module):
     def _forward_streaming(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """<= ops.SKINNY_MAX_M (512) tokens - every decode step, and short prefills - in chunks of 64 rows inside the
         kernels: SEVEN launches per layer (the reference's eager decode layer
-        is ~13, SURVEY.md §3.3):
+        is ~13):
           add+RMSNorm (summing the previous projection's split-K partials)      (mi_add_rmsnorm_splitk)
           -> packed qkv GEMM                                                     (mi_gemm_bf16_packed)
           -> q/k-norm + RoPE + KV store + paged attention in one launch          (mi_paged_attn_decode_fused)

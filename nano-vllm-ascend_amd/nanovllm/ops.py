@@ -463,7 +463,7 @@ def gemm_tile(x, w, bias=None, out=None, silu_mul: bool = False, variant: int | 
     assert out.dim() == 2 and out.shape == (M, n_out) and out.stride(1) == 1
     max_rows = tile_gemm_max_rows(N, K, x.stride(0))
     if M > max_rows >= 256 and variant is None:
-        # more rows than the kernel's 32-bit operand offsets reach (ADVICE r04: 65 536 tokens x K = 25 600): whole-tile
+        # more rows than the kernel's 32-bit operand offsets reach (65 536 tokens x K = 25 600): whole-tile
         # row pieces, each its own launch over the same weight - same bits, every row's K chain is one tile's
         step = max_rows // 256 * 256
         for r0 in range(0, M, step):

@@ -9,7 +9,7 @@ class SamplingParams:
     ignore_eos: bool = False
     # Extension over the reference (which only has multinomial sampling and rejects
     # temperature -> 0): deterministic argmax decoding, needed for parity runs
-    # (BASELINE config 1 "greedy decode").  Default keeps the reference behaviour.
+    # ("greedy decode").  Default keeps the reference behaviour.
     greedy: bool = False
 
     def __post_init__(self):

@@ -2,7 +2,7 @@
 parameters, routing packed projections (q/k/v -> qkv_proj, gate/up -> gate_up_proj)
 through each parameter's `weight_loader` so TP shards land in place.
 
-`init_synthetic_weights` is the documented no-checkpoint mode (SURVEY.md §8d): every
+`init_synthetic_weights` is the documented no-checkpoint mode: every
 rank draws the FULL tensors from one seeded CPU generator and passes them through the
 same weight_loader path, so TP ranks hold consistent shards of one virtual checkpoint.
 """
