@@ -380,6 +380,27 @@ int mi_add_rmsnorm_splitk(const float* partials, int nsplit, const mi_bf16* resi
                           const mi_bf16* w, mi_bf16* y, mi_bf16* residual_out, int rows,
                           int cols, float eps, mi_stream stream);
 
+/* Decode steps of a few rows (csrc/gemm_few.hip), the launch in front of a projection in its operand load; the bits of the two
+ * launches they stand for.  M <= mi_few_rows_max(); bf16 weights (scale NULL) or fp8 ones, packed.
+ * mi_gemm_norm_few: mi_add_rmsnorm_splitk (nsplit 2, 4, 8; K columns: 512, 768, 1024) + mi_gemm_bf16_packed (epilogue 0, 1);
+ * residual_out != residual.
+ * mi_paged_attn_decode_fused_parts: mi_paged_attn_decode_fused whose splits' sums stay in the workspace, one of its own until
+ * mi_gemm_merge_few_splitk has read it; MI_EUNSUPPORTED where contexts are not split (mi_paged_attn_decode_splits == 1).
+ * mi_gemm_merge_few_splitk: the merge + mi_gemm_bf16_packed_splitk (K = heads * 128, K / (64 ksplit) 4, 8, 12 or 16). */
+int mi_few_rows_max(void);
+int mi_gemm_norm_few(const float* partials, int nsplit, const mi_bf16* residual, const mi_bf16* norm_w, float eps,
+                     const void* w_packed, const float* scale, mi_bf16* y, mi_bf16* residual_out, int M, int N, int K,
+                     int epilogue, mi_stream stream);
+int mi_paged_attn_decode_splits(int batch, int n_kv_heads);
+int mi_paged_attn_decode_fused_parts(const mi_bf16* qkv, int64_t qkv_row_stride, const mi_bf16* q_w, const mi_bf16* k_w,
+                                     float eps, const int64_t* positions, const float* cos_sin, const int32_t* slot_2d,
+                                     mi_bf16* k_cache, mi_bf16* v_cache, const int32_t* block_table, int table_stride,
+                                     const int32_t* context_lens, void* workspace, size_t ws_bytes, int batch,
+                                     int n_q_heads, int n_kv_heads, int head_dim, int block_size, float scale,
+                                     mi_stream stream);
+int mi_gemm_merge_few_splitk(const void* workspace, int splits, const void* w_packed, const float* scale, float* partials,
+                             int M, int N, int K, int ksplit, mi_stream stream);
+
 /* Instrumented forms of the decode chain's launches (tools/chain_timeline.py; the same results, separate kernel
  * instantiations): every wave writes s_memrealtime (the chip-wide 100 MHz clock, comparable between launches) at
  * entry / loads issued / data arrived / sums in LDS / barrier passed / stores issued / stores acknowledged into

@@ -1143,7 +1143,7 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
                        const int32_t* block_table, int table_stride, const int32_t* context_lens, mi_bf16* out,
                        void* workspace, size_t ws_bytes, int batch, int n_q_heads, int n_kv_heads, int head_dim,
                        int block_size, float scale, int num_splits, KvStrides kvs, mi_stream stream,
-                       const FusedStep* fused = nullptr, unsigned long long* stamps = nullptr) {
+                       const FusedStep* fused = nullptr, unsigned long long* stamps = nullptr, bool merge = true) {
   int rc = check_attn_common(q, k_cache, v_cache, block_table, n_q_heads, n_kv_heads, head_dim, block_size,
                              q_row_stride);
   if (rc != MI_OK) return rc;
@@ -1159,6 +1159,7 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
   const int waves = pipe ? 8 : decode_waves(G);
   int nsplit = num_splits > 0 ? num_splits : decode_splits(batch, n_kv_heads, pipe ? 16 : waves);
   if (nsplit > 16) nsplit = 16;
+  if (!merge && nsplit == 1) return MI_EUNSUPPORTED;
   float* part_o = static_cast<float*>(workspace);
   float* part_ml = part_o + (size_t)batch * n_q_heads * 16 * 128;
   const float sl2 = scale * 1.4426950408889634f;
@@ -1215,7 +1216,7 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
 #undef LAUNCH_DEC
 #undef LAUNCH_DEC_AS
   rc = check_launch();
-  if (rc != MI_OK || nsplit == 1) return rc;
+  if (rc != MI_OK || nsplit == 1 || !merge) return rc;
   const int rows = batch * n_q_heads;
   if (head_dim == 64)
     hipLaunchKernelGGL(paged_attn_merge_kernel<64>, dim3((rows + 3) / 4), dim3(256), 0, st, part_o, part_ml, out, rows,
@@ -1250,6 +1251,28 @@ extern "C" int mi_paged_attn_decode_fused(const mi_bf16* qkv, int64_t qkv_row_st
   return decode_impl(qkv, qkv_row_stride, k_cache, v_cache, block_table, table_stride, context_lens, out,
                      workspace, ws_bytes, batch, n_q_heads, n_kv_heads, head_dim, block_size, scale, 0,
                      default_strides(n_kv_heads, block_size > 0 ? block_size / 16 : 1), stream, &fs);
+}
+
+// the same without the merge of a split context: the splits' sums stay in `workspace` (mi_gemm_merge_few_splitk)
+extern "C" int mi_paged_attn_decode_splits(int batch, int n_kv_heads) {
+  return batch > 0 && n_kv_heads > 0 ? decode_splits(batch, n_kv_heads, 16) : 0;
+}
+
+extern "C" int mi_paged_attn_decode_fused_parts(const mi_bf16* qkv, int64_t qkv_row_stride, const mi_bf16* q_w,
+                                                const mi_bf16* k_w, float eps, const int64_t* positions,
+                                                const float* cos_sin, const int32_t* slot_2d, mi_bf16* k_cache,
+                                                mi_bf16* v_cache, const int32_t* block_table, int table_stride,
+                                                const int32_t* context_lens, void* workspace, size_t ws_bytes, int batch,
+                                                int n_q_heads, int n_kv_heads, int head_dim, int block_size, float scale,
+                                                mi_stream stream) {
+  if (!positions || !cos_sin || !slot_2d) return MI_EINVAL;
+  if ((q_w == nullptr) != (k_w == nullptr)) return MI_EINVAL;
+  if (!aligned16(cos_sin) || (q_w && (!aligned16(q_w) || !aligned16(k_w)))) return MI_EINVAL;
+  const FusedStep fs{q_w, k_w, positions, cos_sin, slot_2d, eps};
+  return decode_impl(qkv, qkv_row_stride, k_cache, v_cache, block_table, table_stride, context_lens,
+                     static_cast<mi_bf16*>(workspace) /* (no split writes it) */, workspace, ws_bytes, batch, n_q_heads, n_kv_heads,
+                     head_dim, block_size, scale, 0, default_strides(n_kv_heads, block_size > 0 ? block_size / 16 : 1), stream,
+                     &fs, nullptr, false);
 }
 
 // instrumented form of mi_paged_attn_decode_fused (tools/attn_timeline.py): stamps[batch * n_kv_heads * splits][8 waves][8]

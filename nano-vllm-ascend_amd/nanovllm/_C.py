@@ -116,6 +116,15 @@ _SIGNATURES = {
                                        c_int, c_int, c_int, c_int, _p]),
     "mi_pack_weight": (c_int, [_p, _p, c_int, c_int, _p]),
     "mi_gemm_bf16_packed": (c_int, [_p, _p, _p, _p, c_int, c_int, c_int, c_int, _p]),
+    "mi_few_rows_max": (c_int, []),
+    "mi_gemm_norm_few": (c_int, [_p, c_int, _p, _p, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p]),
+    "mi_paged_attn_decode_splits": (c_int, [c_int, c_int]),
+    "mi_paged_attn_decode_fused_parts": (
+        c_int,
+        [_p, c_int64, _p, _p, c_float, _p, _p, _p, _p, _p, _p, c_int, _p, _p, c_size_t, c_int, c_int, c_int, c_int, c_int,
+         c_float, _p],
+    ),
+    "mi_gemm_merge_few_splitk": (c_int, [_p, c_int, _p, _p, _p, c_int, c_int, c_int, c_int, _p]),
     "mi_gemm_bf16_packed_splitk": (c_int, [_p, _p, _p, c_int, c_int, c_int, c_int, _p]),
     "mi_pack_weight_rows4": (c_int, [_p, _p, c_int, c_int, _p]),
     "mi_gemm_bf16_rows4": (c_int, [_p, _p, _p, c_int, c_int, c_int, _p]),

@@ -332,7 +332,8 @@ class Qwen3Model(nn.Module):
         fused_seam = (xgmi is not None and xgmi.fits_rows(rows, h.shape[1])
                       and os.environ.get("MI355_XGMI_FUSED", "1") != "0")
 
-        def attend(attn, qkv):
+        def attend(attn, qkv, o_ksplit=0):
+            """The attention's rows - or, with o_ksplit, o_proj's K-slice sums over them (ops.merge_few_takes)"""
             if not attn.attn.fusable:  # head_dim 64 / groups of 7 / the plain-layout family: one launch per operator
                 return attn._attend_unfused(positions, qkv).flatten(1, -1)
             if not fuse_attn:
@@ -343,6 +344,10 @@ class Qwen3Model(nn.Module):
                 rope.cos_sin_cache = rope.cos_sin_cache.to(qkv.device)
             qw = attn.q_norm.weight if attn.qk_norm else None
             kw = attn.k_norm.weight if attn.qk_norm else None
+            if o_ksplit:
+                return ops.paged_attn_few_proj(qkv, qw, kw, attn.rms_norm_eps, positions, rope.cos_sin_cache, ctx.slot_mapping, a.k_cache,
+                                               a.v_cache, ctx.block_tables, ctx.context_lens, attn.num_heads, attn.num_kv_heads,
+                                               ctx.block_size, a.scale, attn.o_proj.weight_packed, o_ksplit)
             return ops.paged_attn_decode_fused(qkv, qw, kw, attn.rms_norm_eps, positions, rope.cos_sin_cache,
                                                ctx.slot_mapping, a.k_cache, a.v_cache, ctx.block_tables,
                                                ctx.context_lens, attn.num_heads, attn.num_kv_heads, ctx.block_size,
@@ -385,6 +390,8 @@ class Qwen3Model(nn.Module):
 
         def norm_linear(y, is_partials, res, ln, lin, silu_mul=False):
             """linear(rmsnorm(y + res)) -> (out, new residual)"""
+            if is_partials is True and ops.norm_few_takes(rows, y.shape[0], lin.weight_packed, silu_mul):
+                return ops.gemm_norm_few(y, res, ln.weight, ln.eps, lin.weight_packed, silu_mul)
             x, res = add_norm(y, is_partials, res, ln)
             return column_parallel(x, lin, silu_mul), res
 
@@ -416,8 +423,11 @@ class Qwen3Model(nn.Module):
                 qkv = column_parallel(ops.rmsnorm(h, ln1.weight, ln1.eps), attn.qkv_proj)
             else:
                 qkv, residual = norm_linear(parts, is_partials, residual, ln1, attn.qkv_proj)
-            o = attend(attn, qkv)
-            parts, is_partials = row_parallel(o, attn.o_proj)
+            ks = self._ksplit(attn.o_proj.weight)
+            if fuse_attn and not exchange and attn.attn.fusable and ops.merge_few_takes(rows, attn.num_kv_heads, attn.o_proj.weight_packed, ks):
+                parts, is_partials = attend(attn, qkv, ks), True
+            else:
+                parts, is_partials = row_parallel(attend(attn, qkv), attn.o_proj)
             if hasattr(mlp, "experts"):  # sparse block (models/qwen3_moe.py): five launches over expert-sorted pairs
                 x, residual = add_norm(parts, is_partials, residual, ln2)
                 parts, is_partials = mlp(x), False  # summed over the ranks inside the block (before the combine)

@@ -679,6 +679,76 @@ def add_rmsnorm_splitk(partials, residual, w, eps: float, out=None, residual_out
     return out, residual_out
 
 
+# ---- decode steps of a few rows (csrc/gemm_few.hip) ----------------------------------------------------------
+FEW_ROWS_MAX = lib.mi_few_rows_max()
+
+
+def _packed(w_packed):
+    """(weights, scales) of a packed bf16 or fp8 weight"""
+    if isinstance(w_packed, Fp8Weight):
+        return w_packed.data, w_packed.scale
+    require_gpu(w_packed)
+    _bf16(w_packed)
+    assert w_packed.is_contiguous()
+    return w_packed, None
+
+
+def norm_few_takes(rows: int, nsplit: int, w_packed, silu_mul: bool) -> bool:
+    n, k = w_packed.shape
+    unit = 32 if silu_mul else 16
+    return rows <= FEW_ROWS_MAX and nsplit in (2, 4, 8) and k in (512, 768, 1024) and n % unit == 0 and n // unit < 2048
+
+
+def gemm_norm_few(partials, residual, w, eps: float, w_packed, silu_mul: bool = False):
+    """gemm_packed(add_rmsnorm_splitk(partials, residual, w, eps)) in one launch -> (product, new residual)"""
+    require_gpu(partials, residual, w)
+    _bf16(residual, w)
+    assert partials.dtype == torch.float32 and partials.is_contiguous() and residual.is_contiguous()
+    nsplit, cols = partials.shape[0], residual.shape[-1]
+    rows, n = residual.numel() // cols, w_packed.shape[0]
+    assert w_packed.shape[1] == cols and w.numel() == cols and partials.numel() == nsplit * rows * cols
+    data, scale = _packed(w_packed)
+    out = torch.empty((*residual.shape[:-1], n // 2 if silu_mul else n), dtype=_BF16, device=residual.device)
+    residual_out = torch.empty_like(residual)
+    check(lib.mi_gemm_norm_few(ptr(partials), nsplit, ptr(residual), ptr(w), float(eps), ptr(data), ptr(scale), ptr(out), ptr(residual_out),
+                               rows, n, cols, int(silu_mul), stream()), "mi_gemm_norm_few")
+    return out, residual_out
+
+
+def merge_few_takes(rows: int, n_kv_heads: int, w_packed, ksplit: int) -> bool:
+    """Does o_proj weigh the splits of the attention in front of it itself?"""
+    n, k = w_packed.shape
+    return (rows <= FEW_ROWS_MAX and lib.mi_paged_attn_decode_splits(rows, n_kv_heads) > 1 and k % (64 * ksplit) == 0 and k % HEAD_DIM == 0
+            and k // (64 * ksplit) in (4, 8, 12, 16) and n % 16 == 0 and n // 16 * ksplit < 2048)
+
+
+def paged_attn_few_proj(qkv, q_w, k_w, eps: float, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables, context_lens,
+                        n_q_heads: int, n_kv_heads: int, block_size: int, scale: float, w_packed, ksplit: int) -> torch.Tensor:
+    """gemm_packed_splitk(paged_attn_decode_fused(...), w_packed, ksplit), the merge of the splits in the product's operand load"""
+    require_gpu(qkv, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables, context_lens)
+    _bf16(qkv, k_cache, v_cache, q_w, k_w)
+    batch = qkv.shape[0]
+    assert qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] == (n_q_heads + 2 * n_kv_heads) * HEAD_DIM
+    assert positions.dtype == torch.int64 and positions.is_contiguous() and positions.numel() == batch
+    assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous()
+    assert slots_2d.dtype == torch.int32 and slots_2d.is_contiguous() and slots_2d.shape == (batch, 2)
+    assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
+    assert context_lens.dtype == torch.int32 and context_lens.is_contiguous()
+    assert w_packed.shape[1] == n_q_heads * HEAD_DIM
+    data, w_scale = _packed(w_packed)
+    nbytes = lib.mi_paged_attn_decode_workspace(batch, n_q_heads)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=qkv.device)
+    check(lib.mi_paged_attn_decode_fused_parts(ptr(qkv), qkv.stride(0), ptr(q_w), ptr(k_w), float(eps), ptr(positions), ptr(cos_sin),
+                                               ptr(slots_2d), ptr(k_cache), ptr(v_cache), ptr(block_tables), block_tables.stride(0),
+                                               ptr(context_lens), ptr(ws), nbytes, batch, n_q_heads, n_kv_heads, HEAD_DIM, block_size,
+                                               float(scale), stream()), "mi_paged_attn_decode_fused_parts")
+    n, k = w_packed.shape
+    out = torch.empty((ksplit, batch, n), dtype=torch.float32, device=qkv.device)
+    check(lib.mi_gemm_merge_few_splitk(ptr(ws), lib.mi_paged_attn_decode_splits(batch, n_kv_heads), ptr(data), ptr(w_scale), ptr(out), batch,
+                                       n, k, ksplit, stream()), "mi_gemm_merge_few_splitk")
+    return out
+
+
 # ---- the decode chain in five launches per layer (csrc/gemm_chain5_kernel.hpp) ------------------------------
 def chain5_takes(rows: int, hidden: int, ks: tuple) -> bool:
     """Shapes the five-launch chain is built for: a decode-sized batch, consumers (qkv, gate_up; K = hidden) on sixteen
