@@ -796,7 +796,10 @@ int mi_gemm_any_segments(const float* x, int64_t ldx, const void* w, int w_dtype
  * pay or is not taken (bf16 weights, K % 64 == 0, N % 4 == 0, activations of the shapes in use, n_groups <= 1024; n_groups 0:
  * no groups).  mi_gemm_any_table_ints: int32s of the tile table of a grouped operand.  mi_gemm_any_operand: xb[r] = bf16 of
  * x[x_rows ? x_rows[r] : r] for the rows r before group_offsets[n_groups] (all rows without groups), and the table (may be NULL).
- * mi_gemm_any_tile: y[y_rows ? y_rows[r] : r] = epilogue of mi_gemm_any_act / mi_gemm_any_grouped_glu, fp32 or bf16. */
+ * mi_gemm_any_tile: y[y_rows ? y_rows[r] : r] = epilogue of mi_gemm_any_act / mi_gemm_any_grouped_glu, fp32 or bf16.
+ * mi_gemm_any_streams: 1 where mi_gemm_any_act / _grouped_glu over bf16 weights are faster than these (decode batches, experts of a
+ * few rows; x and w on 16 bytes). */
+int mi_gemm_any_streams(int rows, int N, int K, int n_groups);
 int mi_gemm_any_tile_rows(int rows, int N, int K, int n_groups, int dual, int act);
 int64_t mi_gemm_any_table_ints(int rows, int n_groups, int tile_rows);
 int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets, int n_groups,

@@ -2,16 +2,18 @@
 // weights bf16 or fp32 as stored ([N][K] row-major), fp32 accumulation, fp32 output - plain, and grouped over
 // expert-sorted rows (one launch for all experts of a sparse feed-forward, SwiGLU optionally in the epilogue).
 //
-// (bf16 products of more than 8 to 64 rows, by K - a multiple of 64, no segments - go to gemm_any_tile.hip.)
+// (bf16 products of more rows than any_stream_takes says - K a multiple of 64, no segments - go to gemm_any_tile.hip.)
 //
 // These serve the model families whose residual stream, norms and recurrences are kept in 32-bit floats and whose
-// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): six kernels,
+// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): eight kernels,
 //
 //   gemm_any_mfma_kernel   bf16 weights: a 64 x 64 (from 512 rows: 128 x 128, with SwiGLU 128 x 64) output tile per 4-wave
 //                          workgroup, x rounded to bf16 on its way into LDS, v_mfma_f32_16x16x32_bf16, the next K
 //                          step's operands fetched while the current one is multiplied, edges zero-filled
 //   gemm_any_skinny_kernel bf16 weights, up to 64 rows per tile (decode batches, a decode step's experts): 16 features per
 //                          workgroup, the waves split K, fragments straight from memory
+//   gemm_any_stream_kernel bf16 weights, 9 to 64 rows and experts of few rows each, K a multiple of 64: the same work with two 64-deep
+//                          blocks in flight per wave and whole lines through LDS
 //   gemm_any_f32_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, on the fp32 matrix instruction
 //                          - the float32 serving mode, and the routers of sparse feed-forwards in either mode
 //   gemm_any_fma_kernel    the same in plain FMA chains, for operands whose rows are not whole 128-byte lines
@@ -24,7 +26,7 @@
 // on M, on the row's place in the batch or on the tile it falls into (each kernel has ONE fixed order), so the same
 // token gives the same bits whatever it is batched with, within one kernel; between kernels (a row computed in a
 // prompt's portion vs alone) results differ by rounding only.
-#include "mi_common.hpp"
+#include "gemm_any_stream.hpp"
 
 namespace mi {
 
@@ -590,6 +592,148 @@ __global__ __launch_bounds__(256) void gemm_any_skinny_kernel(GemmAnyArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// decode batches (9 to 64 rows), and a decode step's experts: 16 RT output features (DUAL: of both weights) per workgroup, the waves take the
+// 64-deep blocks of K in turn, two blocks in flight each
+// ---------------------------------------------------------------------------------------------------------------
+// These launches are latency-bound: a projection of 2 to 8 MB of weights has a microsecond of bytes and three of round trips.  So: one
+// launch (x is rounded to bf16 on its way into LDS - every workgroup re-reads all rows, 4 bytes per element out of the L2s - instead of
+// an operand pass in front), every wave's loads issued before its first use, no barrier before the waves' sums meet.  A wave asks for
+// whole lines, consecutive lanes consecutive pieces, and turns them into fragments through its own part of LDS: asked for as fragments
+// (16 rows an instruction, as gemm_any_skinny_kernel does) a CU's address path takes four times as long - 32 rows x 2048 x 2048 12.4 us,
+// here 8.5.  Rows beyond the end are the last one again, features beyond N the last one; neither is stored.  K % 64 == 0, rows of x and w
+// on 16 bytes.
+// us, operand pass + tile kernel / here: 24 rows x 1024 x 1024 9.3 / 5.4, 32 x 2048 x 2048 13.0 / 8.5, 9 x 2048 x 2048 12.9 / 5.9, 48 x
+// 4096 x 2048 14.3 / 11.0, 64 x 1024 x 1024 9.5 / 8.2; SwiGLU 32 x 3072 x 2048 20.8 / 11.0; both products of 256 pairs over 64 experts of
+// 768 x 2048 126 / 67 + 37 (402 MB at 6.0 TB/s), of 96 over 32 of 512 x 1024 30 / 17 + 11.
+template <bool DUAL, int MF, int RT, int WAVES, bool EXT>
+__global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_kernel(GemmAnyArgs a) {
+  static_assert(RT == 1 || !DUAL, "several feature tiles: one weight");
+  constexpr int NW = DUAL ? 2 : RT;
+  // per wave: bf16 images [16 NW weight rows | 16 MF x rows][64 k] of the block it multiplies; then its sums
+  constexpr int IMAGE = (NW + MF) * 2048, SUMS = NW * MF * 1024, SLOT = IMAGE > SUMS ? IMAGE : SUMS;
+  __shared__ __attribute__((aligned(16))) char lds[WAVES * SLOT];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  char* const slot = lds + wave * SLOT;
+  auto sums = [&](int i, int t, int f) __attribute__((always_inline)) { return reinterpret_cast<f32x4*>(lds + i * SLOT + ((t * MF + f) * 64 + lane) * 16); };
+  int m_lo, m_hi;
+  const uint16_t *w, *w2;
+  select_group<uint16_t, DUAL>(a, w, w2, m_lo, m_hi);
+  if (m_lo >= m_hi) return;
+  const int n0 = blockIdx.x * 16 * RT;
+  const int fr = lane & 15, g = lane >> 4;
+  const uint16_t* wp[NW][2];  // a request: eight weight rows of 128 bytes / four x rows of 256
+#pragma unroll
+  for (int t = 0; t < NW; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      wp[t][j] = (DUAL && t ? w2 : w) + (int64_t)min(n0 + (DUAL ? 0 : t * 16) + j * 8 + (lane >> 3), a.N - 1) * a.K + wave * 64 + (lane & 7) * 8;
+  const int w_at = (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
+  const int blocks = a.K >> 6, mine = (blocks - wave + WAVES - 1) / WAVES;
+  for (int m0 = m_lo; m0 < m_hi; m0 += 16 * MF) {
+    const float* xp[MF * 4];
+#pragma unroll
+    for (int q = 0; q < MF * 4; ++q) {
+      const int m = min(m0 + q * 4 + g, m_hi - 1);
+      xp[q] = a.x + (int64_t)(a.x_rows ? a.x_rows[m] : m) * a.ldx + wave * 64 + fr * 4;
+    }
+    f32x4 acc[NW][MF];
+#pragma unroll
+    for (int t = 0; t < NW; ++t)
+#pragma unroll
+      for (int f = 0; f < MF; ++f) acc[t][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Block {
+      u32x4 w[NW][2];
+      f32x4 x[MF * 4];
+    };
+    auto issue = [&](Block& b, int i) __attribute__((always_inline)) {
+      const int k = i * (WAVES * 64);
+#pragma unroll
+      for (int t = 0; t < NW; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) b.w[t][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[t][j] + k));
+#pragma unroll
+      for (int q = 0; q < MF * 4; ++q) b.x[q] = *reinterpret_cast<const f32x4*>(xp[q] + k);
+      __builtin_amdgcn_sched_barrier(0);  // (the next block's requests stay in front of this block's waits)
+    };
+    auto consume = [&](const Block& b) __attribute__((always_inline)) {  // (one wave's LDS operations are in order: no barrier)
+#pragma unroll
+      for (int t = 0; t < NW; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<u32x4*>(slot + t * 2048 + j * 1024 + w_at) = b.w[t][j];
+#pragma unroll
+      for (int q = 0; q < MF * 4; ++q) {
+        const int r = (q * 4 + g) & 7;
+        *reinterpret_cast<u32x2*>(slot + NW * 2048 + (q * 4 + g) * 128 + (((fr >> 1) ^ r) << 4) + (fr & 1) * 8) =
+            u32x2{pack_bf(b.x[q][0], b.x[q][1]), pack_bf(b.x[q][2], b.x[q][3])};
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int at = fr * 128 + (((s * 4 + g) ^ (fr & 7)) << 4);
+        bf16x8 wf[NW];
+#pragma unroll
+        for (int t = 0; t < NW; ++t) wf[t] = as_frag(*reinterpret_cast<const u32x4*>(slot + t * 2048 + at));
+#pragma unroll
+        for (int f = 0; f < MF; ++f) {
+          const bf16x8 xf = as_frag(*reinterpret_cast<const u32x4*>(slot + (NW + f) * 2048 + at));
+#pragma unroll
+          for (int t = 0; t < NW; ++t) acc[t][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t], xf, acc[t][f], 0, 0, 0);
+        }
+      }
+    };
+    if (m0 > m_lo) __syncthreads();  // (the sums of the rows before are read)
+    if (mine > 0) {
+      Block A, B;
+      issue(A, 0);
+      int i = 0;
+      for (; i + 2 < mine; i += 2) {
+        issue(B, i + 1);
+        consume(A);
+        issue(A, i + 2);
+        consume(B);
+      }
+      if (i + 1 < mine) {
+        issue(B, i + 1);
+        consume(A);
+        consume(B);
+      } else {
+        consume(A);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NW; ++t)
+#pragma unroll
+      for (int f = 0; f < MF; ++f) *sums(wave, t, f) = acc[t][f];
+    __syncthreads();
+    // a lane's four features n0 + 16 t + 4 g + r of row (lane & 15) of a fragment, the waves' sums in order
+    for (int item = wave; item < (DUAL ? 1 : RT) * MF; item += WAVES) {
+      const int t = item / MF, f = item % MF;
+      const int m = m0 + f * 16 + fr;
+      f32x4 v = *sums(0, t, f), v2 = *sums(0, DUAL ? NW - 1 : t, f);
+#pragma unroll
+      for (int i = 1; i < WAVES; ++i) {
+        v += *sums(i, t, f);
+        if (DUAL) v2 += *sums(i, NW - 1, f);
+      }
+      if (m >= m_hi) continue;
+      const int64_t yrow = a.y_rows ? a.y_rows[m] : m;
+      const int n = n0 + t * 16 + g * 4;
+      float o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = n + r < a.N ? finish<DUAL, EXT>(a, m, yrow, n + r, v[r], v2[r]) : 0.f;
+      float* yp = a.y + yrow * a.ldy + n;
+      if (n + 4 <= a.N && (a.ldy % 4 == 0) && dev_aligned16(a.y)) {
+        *reinterpret_cast<float4*>(yp) = float4{o[0], o[1], o[2], o[3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < a.N) yp[r] = o[r];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // few rows: one wave per FT output features and batch of MT rows (blockIdx.y); the lanes take K in pieces of 8, ascending,
 // 16-byte loads where the operands allow it, then a butterfly over the lanes
 // ---------------------------------------------------------------------------------------------------------------
@@ -705,6 +849,64 @@ __global__ __launch_bounds__(256) void gemm_any_each_row_kernel(GemmAnyArgs a) {
   }
 }
 
+// Where the streaming kernel is the faster one of it and the tile kernels (without groups and batches; us, tile kernels / here): up to 24
+// rows everywhere measured (24 x 32768 x 2048 35.3 / 34.3, 9 rows 35.2 / 28.3); beyond, every workgroup's copy of the rows outweighs its
+// weights from some number of features on: 32 x 16384 x 1024 11.9 / 11.3, x 32768 x 2048 36.2 / 37.0; 48 x 6144 x 2048 15.3 / 13.5, x 16384
+// x 1024 12.3 / 14.2; 64 x 4096 x 1024 9.5 / 8.9, x 16384 x 1024 12.8 / 19.9.  Grouped: up to ten rows a group on average (64 experts of 768 x 2048, 8
+// each 131 / 111, 16 each 131 / 140; 32 of 512 x 1024, 8 each 31.0 / 28.6, 16 each 31.0 / 33.8).
+bool any_stream_takes(int rows, int N, int K, int n_groups) {
+  if (rows <= 8 || K % 64) return false;
+  if (n_groups) return rows <= 10 * (int64_t)n_groups;
+  return rows <= 64 && N <= (rows <= 24 ? INT32_MAX : rows <= 32 ? 16384 : rows <= 48 ? 6144 : 4096);
+}
+
+template <bool DUAL, bool EXT>
+static int launch_stream(const GemmAnyArgs& a, int groups, int rows, hipStream_t st) {
+  auto go = [&](auto kernel, int rt, int waves) {
+    hipLaunchKernelGGL(kernel, dim3((a.N + 16 * rt - 1) / (16 * rt), 1, groups), dim3(64 * waves), 0, st, a);
+    return check_launch();
+  };
+  if (groups > 1 || a.group_offsets) {
+    // workgroups enough: four waves each, so that several share a CU (eight: 256 pairs over 64 experts' second product 55 us, four 37);
+    // groups: 16 rows at a time
+    const int mf = a.group_offsets ? 1 : (rows + 15) / 16;
+    if constexpr (!DUAL) {
+      if (mf == 1 && (int64_t)(a.N / 16) * groups >= 2048) return go(gemm_any_stream_kernel<false, 1, 2, 4, EXT>, 2, 4);
+    }
+    switch (mf) {
+      case 1: return go(gemm_any_stream_kernel<DUAL, 1, 1, 4, EXT>, 1, 4);
+      case 2: return go(gemm_any_stream_kernel<DUAL, 2, 1, 4, EXT>, 1, 4);
+      case 3: return go(gemm_any_stream_kernel<DUAL, 3, 1, 4, EXT>, 1, 4);
+      default: return go(gemm_any_stream_kernel<DUAL, 4, 1, 4, EXT>, 1, 4);
+    }
+  }
+  const int mf = (rows + 15) / 16;
+  if constexpr (DUAL) {
+    switch (mf) {
+      case 1: return go(gemm_any_stream_kernel<true, 1, 1, 4, EXT>, 1, 4);
+      case 2: return go(gemm_any_stream_kernel<true, 2, 1, 4, EXT>, 1, 4);
+      case 3: return go(gemm_any_stream_kernel<true, 3, 1, 4, EXT>, 1, 4);
+      default: return go(gemm_any_stream_kernel<true, 4, 1, 4, EXT>, 1, 4);
+    }
+  } else {
+    // from 384 feature tiles on two per workgroup: half as many copies of x (24 rows x 6144 x 2048 12.8 / 10.5 us, x 4096 8.6 / 9.8)
+    if (a.N >= 6144) {
+      switch (mf) {
+        case 1: return go(gemm_any_stream_kernel<false, 1, 2, 4, EXT>, 2, 4);
+        case 2: return go(gemm_any_stream_kernel<false, 2, 2, 4, EXT>, 2, 4);
+        case 3: return go(gemm_any_stream_kernel<false, 3, 2, 4, EXT>, 2, 4);
+        default: break;
+      }
+    }
+    switch (mf) {
+      case 1: return go(gemm_any_stream_kernel<false, 1, 1, 8, EXT>, 1, 8);
+      case 2: return go(gemm_any_stream_kernel<false, 2, 1, 8, EXT>, 1, 8);
+      case 3: return go(gemm_any_stream_kernel<false, 3, 1, 8, EXT>, 1, 8);
+      default: return go(gemm_any_stream_kernel<false, 4, 1, 4, EXT>, 1, 4);
+    }
+  }
+}
+
 // Exact mode beyond a few rows.  The tile of gemm_any_f32_kernel: the largest of 64 x 64, 32 x 64, 32 x 32 whose grid puts a
 // workgroup on most of the 256 CUs; groups of less than 256 rows (an even share is assumed) in 32-row tiles, whose last one
 // is padded by less.  us, gemm_any_fma_kernel / here: 733 rows, K 1024: N 1024 64 / 17, N 3072 202 / 67, N 32 113 / 12; 32
@@ -786,6 +988,10 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
   }
   const dim3 grid((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups);
   if constexpr (sizeof(TW) == 2) {
+    const bool batches = !a.group_offsets && groups > 1;   // (64 rows a batch at most: the features of a head)
+    if (mode == 0 && (batches ? rows_per_group_max <= 64 && a.K % 64 == 0 : any_stream_takes(rows_per_group_max, a.N, a.K, a.group_offsets ? groups : 0)) &&
+        a.ldx % 4 == 0 && a.x_batch % 4 == 0 && aligned16(a.x) && aligned16(a.w) && (!DUAL || aligned16(a.w2)))
+      return launch_stream<DUAL, EXT>(a, groups, rows_per_group_max, st);
     if (mode == 0 && rows_per_group_max >= 512 && a.N >= 128) {  // prefill-sized: 128-row tiles, 128 (SwiGLU: 64) features
       if (DUAL) {
         hipLaunchKernelGGL((gemm_any_mfma_kernel<DUAL, 4, 2, EXT>), dim3((a.N + 63) / 64, (rows_per_group_max + 127) / 128, groups),
@@ -830,6 +1036,8 @@ static int gemm_any_dispatch(const GemmAnyArgs& a, int w_dtype, int groups, int 
 
 static bool act_ok(int act) { return (act >= MI_ACT_NONE && act <= MI_ACT_SOFTCAP) || act == MI_ACT_RELU2; }
 static bool act_ext_ok(int act) { return (act_ok(act) && act != MI_ACT_SOFTCAP) || act == MI_ACT_TANH || act == MI_ACT_DECAY; }
+
+extern "C" int mi_gemm_any_streams(int rows, int N, int K, int n_groups) { return any_stream_takes(rows, N, K, n_groups) ? 1 : 0; }
 
 extern "C" int mi_gemm_any(const float* x, int64_t ldx, const void* w, int w_dtype, float* y, int64_t ldy, int M, int N,
                            int K, float alpha, int exact, mi_stream stream) {

@@ -10,6 +10,7 @@
 // Measured, 8192 rows: 2048 x 2048 207 -> 75 us + 15 us of operand pass; 64 experts x 8 per row, 2048 -> 2 x 768 with SwiGLU
 // 1192 -> 523 us (790 TFLOP/s), back to 2048 1050 -> 250 us.  Bits: one fp32 chain over k per result, k ascending, from
 // the same rounded operands as gemm_any_mfma_kernel's - the same bits.
+#include "gemm_any_stream.hpp"
 #include "gemm_tile_args.hpp"
 
 namespace mi {
@@ -298,7 +299,8 @@ extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const
   const bool fits = xb && x && w && y && w_dtype == MI_DTYPE_BF16 && M > 0 && ldx >= K && ldy >= N && ldy % 4 == 0 && aligned16(w) &&
                     (!w2 || aligned16(w2)) && aligned16(y) && (!bias || aligned16(bias)) && (!bias2 || (w2 && aligned16(bias2))) &&
                     aligned16(xb) && xb_elems >= (int64_t)M * K && !(act == MI_ACT_SOFTCAP && !(alpha > 0.f));
-  const int t = fits ? tile_rows_for(M, N, K, 0, w2 != nullptr, act) : 0;
+  const bool streams = any_stream_takes(M, N, K, 0) && aligned16(x) && ldx % 4 == 0;
+  const int t = fits && !streams ? tile_rows_for(M, N, K, 0, w2 != nullptr, act) : 0;
   if (!t) return mi_gemm_any_act(x, ldx, w, w2, w_dtype, bias, bias2, act, y, ldy, M, N, K, alpha, 0, stream);
   const int rc = mi_gemm_any_operand(x, ldx, nullptr, nullptr, 0, t, M, K, xb, nullptr, stream);
   return rc != MI_OK ? rc
@@ -306,7 +308,8 @@ extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const
                                         0.f, nullptr, nullptr, 0, y, 0, ldy, nullptr, M, N, K, alpha, stream);
 }
 
-// scratch of mi_expert_ff: the gathered operand, the inner activations, the tile table (each rounded up to 16 bytes)
+// scratch of mi_expert_ff: the gathered operand, the inner activations, the tile table (each rounded up to 16 bytes) - or, streamed, the
+// inner activations in fp32
 static int expert_tile_rows(int pairs, int G, int ff, int width, bool dual, int act) {
   const int a = tile_rows_for(pairs, ff, width, G, dual, act), b = tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE);
   return a < b ? a : b;
@@ -316,7 +319,10 @@ static int64_t round16(int64_t bytes) { return (bytes + 15) & ~(int64_t)15; }
 extern "C" int64_t mi_expert_ff_bytes(int pairs, int G, int ff, int width, int dual, int act) {
   if (pairs < 1 || G < 1) return 0;
   const int t = expert_tile_rows(pairs, G, ff, width, dual != 0, act);
-  return t ? round16((int64_t)pairs * width * 2) + round16((int64_t)pairs * ff * 2) + 4 * mi_gemm_any_table_ints(pairs, G, t) : 0;
+  if (!t) return 0;
+  const int64_t tiles = round16((int64_t)pairs * width * 2) + round16((int64_t)pairs * ff * 2) + 4 * mi_gemm_any_table_ints(pairs, G, t);
+  const int64_t inner = round16((int64_t)pairs * ff * 4);
+  return tiles > inner ? tiles : inner;
 }
 
 extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_token, const mi_bf16* w, const mi_bf16* w2,
@@ -327,6 +333,14 @@ extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_tok
   const int64_t need = mi_expert_ff_bytes(pairs, G, ff, width, w2 != nullptr, act);
   if (need == 0) return MI_EUNSUPPORTED;
   if (scratch_bytes < need) return MI_EWORKSPACE;
+  if (any_stream_takes(pairs, ff, width, G) && any_stream_takes(pairs, width, ff, G) && aligned16(x) && ldx % 4 == 0 && aligned16(w) &&
+      aligned16(down) && (!w2 || aligned16(w2))) {
+    float* inner = static_cast<float*>(scratch);
+    const int rc = mi_gemm_any_grouped_glu(x, ldx, pair_token, w, w2, MI_DTYPE_BF16, act, limit, row_scale, row_scale_rows, offsets, G, pairs,
+                                           inner, ff, nullptr, ff, width, 0, stream);
+    return rc != MI_OK ? rc : mi_gemm_any_grouped(inner, ff, nullptr, down, nullptr, MI_DTYPE_BF16, offsets, G, pairs, y, width, pair_index,
+                                                  width, ff, 0, stream);
+  }
   const int t = expert_tile_rows(pairs, G, ff, width, w2 != nullptr, act);
   char* p = static_cast<char*>(scratch);
   mi_bf16* xb = reinterpret_cast<mi_bf16*>(p);

@@ -209,6 +209,7 @@ _SIGNATURES = {
     "mi_moe_combine_f32": (c_int, [_p, _p, c_int64, _p, _p, c_int, c_int, c_int, c_int, _p, c_int64, _p]),
     "mi_gemm_any_act": (c_int, [_p, c_int64, _p, _p, c_int, _p, _p, c_int, _p, c_int64, c_int, c_int, c_int, c_float,
                                 c_int, _p]),
+    "mi_gemm_any_streams": (c_int, [c_int, c_int, c_int, c_int]),
     "mi_gemm_any_tile_rows": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mi_gemm_any_table_ints": (c_int64, [c_int, c_int, c_int]),
     "mi_gemm_any_fit_elems": (c_int64, [c_int, c_int, c_int, c_int, c_int]),

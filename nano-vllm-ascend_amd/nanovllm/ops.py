@@ -1090,6 +1090,8 @@ def _grouped_tiles(x, x_rows, w, w2, act: int, offsets, rows_max: int, y, y_rows
     """A grouped product through the tile kernels, if it goes there.  Their operand and tile table hold the rows of ALL groups: as many
     as there are places to take one from."""
     total = x.shape[0] if x_rows is None else x_rows.numel()
+    if lib.mi_gemm_any_streams(total, w.shape[1], w.shape[2], w.shape[0]) and not (x.data_ptr() | 4 * x.stride(0) | w.data_ptr()) % 16:
+        return False
     t = _grouped_tile_rows(total, rows_max, w, w2, act, exact, y)
     if t:
         G = w.shape[0]
