@@ -475,20 +475,61 @@ __global__ __launch_bounds__(256) void swa_attention_vec_kernel(const float* __r
   }
 }
 
+// VW consecutive bf16 channels of one value row, and channel c of eight of them (keys) as an MFMA operand
+template <int VW>
+struct VPiece;
+template <>
+struct VPiece<1> {
+  uint16_t w;
+};
+template <>
+struct VPiece<2> {
+  uint32_t w;
+};
+template <>
+struct __attribute__((aligned(16))) VPiece<8> {
+  u32x4 w;
+};
+template <int VW>
+__device__ __forceinline__ u32x4 v_channel(const VPiece<VW> (&v)[8], int c) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (VW == 1) {
+      r[i] = (uint32_t)v[2 * i].w | ((uint32_t)v[2 * i + 1].w << 16);
+    } else {
+      uint32_t a, b;
+      if constexpr (VW == 8) a = v[2 * i].w[c >> 1], b = v[2 * i + 1].w[c >> 1];
+      else a = v[2 * i].w, b = v[2 * i + 1].w;
+      r[i] = __builtin_amdgcn_perm(b, a, (c & 1) ? 0x07060302u : 0x05040100u);
+    }
+  }
+  return r;
+}
+
 // The matrix-core form for DECODE steps (one row per sequence) over a bf16 cache: a workgroup takes one (row, kv head) and
 // up to 16 of the query heads that read it - the heads are the 16 columns of the score tile where the prompt form has 16
 // consecutive rows of one head, so every K and V element the workgroup loads serves all of the group's heads (latent
-// attention: ONE cache row for every head).  Its four waves take the rounds of 32 keys in turn and merge their (max, sum,
+// attention: ONE cache row for every head).  Its waves take the rounds of 32 keys in turn and merge their (max, sum,
 // accumulator) triples through LDS.  Arithmetic as in the prompt form: q and the softmax weights as bf16 hi + lo pairs.
-template <int DKM, int DVM, bool PAIR, bool KEEP>
-__global__ __launch_bounds__(256) void paged_attention_heads_mfma_kernel(
-    const float* __restrict__ q, int64_t ldq, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
-    const int32_t* __restrict__ block_tables, int table_cols, const int32_t* __restrict__ kv_lens, int H, int G, int D,
+//
+// What bounds it: requests in flight.  A round's 16 KiB (heads of 128) leave a wave at once, and eight waves (four of the wider heads,
+// whose registers hold no more) are two per SIMD, one of them computing while the other's rows arrive.  A key's page number is looked
+// up by one lane, a round ahead, and handed to the lanes that read the key's rows: looked up by every lane for each of its ten rows it
+// was a chain of dependent loads per round.  VW channels of V per lane and load: 8 where the value heads are whole 128-channel rows (a
+// key's row in one request), else 2 or 1.  FAST: heads of exactly 32 DKM and 16 DVM channels, pages of a power of two rows, no
+// logarithmic bias and no soft cap - what is left has room for a second round in flight.  Measured, 32 rows x 1024 keys, 8 kv heads of
+// 128 with two query heads each (134 MB): 69 us before, 42 with one round in flight, 34 with two (3.9 TB/s); 24 rows of 30 - 1500 keys,
+// one latent row of 256 for eight heads: 24.5 -> 15.0.
+template <int DKM, int DVM, int VW, bool KEEP, bool FAST, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void paged_attention_heads_mfma_kernel(
+    const float* __restrict__ q, int64_t ldq, const uint16_t* k_cache, const uint16_t* v_cache,
+    const int32_t* block_tables, int table_cols, const int32_t* __restrict__ kv_lens, int H, int G, int D,
     int Dv, int block_size, int window, float scale, AttnBias bias, int64_t ldv, const float* __restrict__ gate,
     int64_t ldg, float* __restrict__ out, int64_t ldo, int n_split, float* __restrict__ ws) {
-  __shared__ __attribute__((aligned(16))) float part_o[3][DVM][64][4];
-  __shared__ float part_ml[3][2][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ __attribute__((aligned(16))) float part_o[WAVES][DVM][64][4];
+  __shared__ float part_ml[WAVES][2][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int row = blockIdx.x, g = blockIdx.y;
   const int Gv = bias.value_heads, gv = g / (G / Gv);
   const int hpg = H / G;
@@ -496,8 +537,8 @@ __global__ __launch_bounds__(256) void paged_attention_heads_mfma_kernel(
   const int h0 = g * hpg + (blockIdx.z / n_split) * 16;   // first head of this workgroup's columns
   const int nh = min(16, g * hpg + hpg - h0);             // valid columns
   const int qi = lane & 15, kg = lane >> 4;
-  const int dk = D / 32, dvt = Dv / 16;
-  const int bs_shift = block_shift(block_size);
+  const int dk = FAST ? DKM : D / 32, dvt = FAST ? DVM : Dv / 16;
+  const int bs_shift = FAST ? __builtin_ctz((unsigned)block_size) : block_shift(block_size);
   const int pos = kv_lens[row] - 1;
   const int32_t* table = block_tables + (int64_t)row * table_cols;
   const HeadBias hb = head_bias(bias, qi < nh ? h0 + qi : h0, H);
@@ -524,48 +565,51 @@ __global__ __launch_bounds__(256) void paged_attention_heads_mfma_kernel(
   }
   const int lo_key = first_key(bias, pos, window), hi_key = pos;
   const int gap = KEEP ? kept_gap(bias, lo_key) : lo_key;
+  // key lane & 31 of the round at j; beyond the last key that key again (masked below, weight 0)
+  auto key_of = [&](int j) { return max(key_at<KEEP>(min(j + (lane & 31), hi_key), lo_key, gap), 0); };
+  auto block_of = [&](int key) { return FAST || bs_shift >= 0 ? key >> bs_shift : key / block_size; };
+  auto page_of = [&](int j) { return (uint32_t)table[block_of(key_of(j))]; };
+  constexpr int NV = DVM / VW;   // a lane's pieces of a value row: channels 16 VW dp + VW qi ..
   float m = -INFINITY, l = 0.f;
   f32x4 oacc[DVM];
 #pragma unroll
   for (int dt = 0; dt < DVM; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int j0 = gap + 32 * (split * 4 + wave); j0 <= hi_key; j0 += 32 * 4 * n_split) {
-    f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    // the round's V words are requested together with its K rows (their addresses do not depend on the scores): one
-    // memory latency per round instead of two behind one another.  The V^T operand: the lane's eight keys (its
-    // contraction slots) at two neighbouring channels per 32-channel pair of tiles (PAIR), else one channel per tile
-    const uint16_t* vrow[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      // (beyond the last key: weight 0)
-      const int key = key_at<KEEP>(min(j0 + (e >> 2) * 16 + kg * 4 + (e & 3), hi_key), lo_key, gap);
-      vrow[e] = v_cache + (int64_t)cache_row(table, key, Gv, gv, block_size, bs_shift) * (int)ldv +
-                (PAIR ? 2 * qi : qi);
-    }
-    uint32_t vw[PAIR ? DVM / 2 : 1][8];
-    if constexpr (PAIR) {
-#pragma unroll
-      for (int dp = 0; dp < DVM / 2; ++dp)
-        if (2 * dp < dvt) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) vw[dp][e] = *reinterpret_cast<const uint32_t*>(vrow[e] + dp * 32);
-        }
-    }
+  struct Round {
+    u32x4 k[2][DKM];
+    VPiece<VW> v[NV][8];
+  };
+  // all of a round's K and V rows are requested before the first is used.  The V^T operand: the lane's eight keys (its contraction
+  // slots) at VW neighbouring channels
+  auto request = [&](Round& b, int j, uint32_t page) __attribute__((always_inline)) {
+    const int key = key_of(j);
+    const uint32_t off = (uint32_t)(key - block_of(key) * block_size);
+    const uint32_t krow = (page * (uint32_t)G + (uint32_t)g) * (uint32_t)block_size + off;
+    const uint32_t vrow = (page * (uint32_t)Gv + (uint32_t)gv) * (uint32_t)block_size + off;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      // this lane's row of the K operand; rows beyond the last key repeat it (their scores are masked below), so
-      // that every load is unconditional and a round's loads are all in flight together
-      const int key = key_at<KEEP>(min(j0 + t * 16 + qi, hi_key), lo_key, gap);
-      const uint16_t* kr =
-          k_cache + (int64_t)cache_row(table, key, G, g, block_size, bs_shift) * D + kg * 8;
+      const uint16_t* kr = k_cache + (int64_t)(uint32_t)__shfl((int)krow, t * 16 + qi) * D + kg * 8;
 #pragma unroll
-      for (int ks = 0; ks < DKM; ++ks) {
-        if (ks < dk) {
-          const bf16x8 kf = as_frag(*reinterpret_cast<const u32x4*>(kr + ks * 32));
-          sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qh[ks], sacc[t], 0, 0, 0);
-          sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, ql[ks], sacc[t], 0, 0, 0);
-        }
-      }
+      for (int ks = 0; ks < DKM; ++ks)
+        if (ks < dk) b.k[t][ks] = *reinterpret_cast<const u32x4*>(kr + ks * 32);
     }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint16_t* vr = v_cache + (int64_t)(uint32_t)__shfl((int)vrow, (e >> 2) * 16 + kg * 4 + (e & 3)) * (int)ldv + VW * qi;
+#pragma unroll
+      for (int dp = 0; dp < NV; ++dp)
+        if (VW * dp < dvt) b.v[dp][e] = *reinterpret_cast<const VPiece<VW>*>(vr + dp * 16 * VW);
+    }
+  };
+  auto attend = [&](const Round& b, int j0) __attribute__((always_inline)) {
+    f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < DKM; ++ks)
+        if (ks < dk) {
+          sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(b.k[t][ks]), qh[ks], sacc[t], 0, 0, 0);
+          sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(b.k[t][ks]), ql[ks], sacc[t], 0, 0, 0);
+        }
     float sc[8];
     bool vis[8];
     int dist[8];
@@ -578,14 +622,14 @@ __global__ __launch_bounds__(256) void paged_attention_heads_mfma_kernel(
       dist[e] = pos - key;
     }
     // (the bias kind is the same for the whole launch: see the prompt form)
-    if (bias.kind == MI_BIAS_LOG) {
+    if (!FAST && bias.kind == MI_BIAS_LOG) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) sc[e] -= hb.a * log1pf(hb.b * (float)max(dist[e], 0));
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) sc[e] -= hb.a * (float)dist[e];
     }
-    if (bias.softcap > 0.f) {
+    if (!FAST && bias.softcap > 0.f) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) sc[e] = bias.softcap * tanhf(sc[e] / bias.softcap);
     }
@@ -611,95 +655,99 @@ __global__ __launch_bounds__(256) void paged_attention_heads_mfma_kernel(
     for (int e = 0; e < 8; ++e) plo[e] = pv[e] - rbf(pv[e]);
     const bf16x8 ph = as_frag(u32x4{pack_bf(pv[0], pv[1]), pack_bf(pv[2], pv[3]), pack_bf(pv[4], pv[5]), pack_bf(pv[6], pv[7])});
     const bf16x8 pl = as_frag(u32x4{pack_bf(plo[0], plo[1]), pack_bf(plo[2], plo[3]), pack_bf(plo[4], plo[5]), pack_bf(plo[6], plo[7])});
-    if constexpr (PAIR) {
 #pragma unroll
-      for (int dp = 0; dp < DVM / 2; ++dp) {
-        if (2 * dp < dvt) {
-          const uint32_t(&w)[8] = vw[dp];
-          const bf16x8 v_even = as_frag(u32x4{(w[0] & 0xffffu) | (w[1] << 16), (w[2] & 0xffffu) | (w[3] << 16),
-                                              (w[4] & 0xffffu) | (w[5] << 16), (w[6] & 0xffffu) | (w[7] << 16)});
-          const bf16x8 v_odd = as_frag(u32x4{(w[0] >> 16) | (w[1] & 0xffff0000u), (w[2] >> 16) | (w[3] & 0xffff0000u),
-                                             (w[4] >> 16) | (w[5] & 0xffff0000u), (w[6] >> 16) | (w[7] & 0xffff0000u)});
-          oacc[2 * dp] *= corr;
-          oacc[2 * dp + 1] *= corr;
-          oacc[2 * dp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_even, ph, oacc[2 * dp], 0, 0, 0);
-          oacc[2 * dp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_even, pl, oacc[2 * dp], 0, 0, 0);
-          oacc[2 * dp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_odd, ph, oacc[2 * dp + 1], 0, 0, 0);
-          oacc[2 * dp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v_odd, pl, oacc[2 * dp + 1], 0, 0, 0);
+    for (int dp = 0; dp < NV; ++dp)
+      if (VW * dp < dvt) {
+#pragma unroll
+        for (int c = 0; c < VW; ++c) {
+          f32x4& o = oacc[VW * dp + c];
+          const bf16x8 vf = as_frag(v_channel<VW>(b.v[dp], c));
+          o *= corr;
+          o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph, o, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, o, 0, 0, 0);
         }
+      }
+  };
+  const int step = 32 * WAVES * n_split;
+  int j0 = gap + 32 * (split * WAVES + wave);
+  if (j0 <= hi_key) {
+    if constexpr (FAST && WAVES == 8) {
+      // two rounds in flight: the next one's requests leave before this one's scores.  Loads return in order: a page number is asked for in
+      // front of the rows of the round before its own, and behind the last round the last key's row is fetched again, so that the number
+      // of requests behind the one that is waited for is known.  (The empty statements, with caches and tables that are not declared unaliased:
+      // loads are otherwise moved behind the branch that follows, to their first use)
+      Round b[2];
+      const uint32_t page0 = page_of(j0);
+      uint32_t page1 = page_of(j0 + step);
+      request(b[0], j0, page0);
+      for (;;) {
+        const uint32_t page2 = page_of(j0 + 2 * step);
+        __builtin_amdgcn_sched_barrier(0);
+        request(b[1], j0 + step, page1);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        attend(b[0], j0);
+        if ((j0 += step) > hi_key) break;
+        page1 = page_of(j0 + 2 * step);
+        __builtin_amdgcn_sched_barrier(0);
+        request(b[0], j0 + step, page2);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        attend(b[1], j0);
+        if ((j0 += step) > hi_key) break;
       }
     } else {
-#pragma unroll
-      for (int dt = 0; dt < DVM; ++dt) {
-        if (dt < dvt) {
-          uint32_t ve[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) ve[e] = (uint32_t)vrow[e][dt * 16];
-          const bf16x8 vf = as_frag(u32x4{ve[0] | (ve[1] << 16), ve[2] | (ve[3] << 16), ve[4] | (ve[5] << 16), ve[6] | (ve[7] << 16)});
-          oacc[dt] *= corr;
-          oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph, oacc[dt], 0, 0, 0);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, oacc[dt], 0, 0, 0);
-        }
+      for (uint32_t page = page_of(j0);;) {
+        Round b;
+        const uint32_t next = page_of(j0 + step);
+        request(b, j0, page);
+        attend(b, j0);
+        if ((j0 += step) > hi_key) break;
+        page = next;
       }
     }
   }
-  // merge the four waves' partial results (same lane layout in every wave); a wave without a round has m = -inf, l = 0
-  if (wave > 0) {
+  // merge the waves' partial results (same lane layout in every wave), each wave DVM / WAVES of the tiles; a wave without a round has
+  // m = -inf, l = 0
 #pragma unroll
-    for (int dt = 0; dt < DVM; ++dt)
-      if (dt < dvt) *reinterpret_cast<f32x4*>(part_o[wave - 1][dt][lane]) = oacc[dt];
-    part_ml[wave - 1][0][lane] = m;
-    part_ml[wave - 1][1][lane] = l;
-  }
+  for (int dt = 0; dt < DVM; ++dt)
+    if (dt < dvt) *reinterpret_cast<f32x4*>(part_o[wave][dt][lane]) = oacc[dt];
+  part_ml[wave][0][lane] = m;
+  part_ml[wave][1][lane] = l;
   __syncthreads();
-  if (wave > 0 || qi >= nh) return;
-  float mm = m;
+  if (qi >= nh) return;
+  float mm = -INFINITY, f[WAVES];
 #pragma unroll
-  for (int w = 0; w < 3; ++w) mm = fmaxf(mm, part_ml[w][0][lane]);
-  const float f0 = m == -INFINITY ? 0.f : expf(m - mm);
-  l *= f0;
+  for (int w = 0; w < WAVES; ++w) mm = fmaxf(mm, f[w] = part_ml[w][0][lane]);
+  l = 0.f;
 #pragma unroll
-  for (int dt = 0; dt < DVM; ++dt) oacc[dt] *= f0;
-#pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    const float mw = part_ml[w][0][lane];
-    const float f = mw == -INFINITY ? 0.f : expf(mw - mm);
-    l = fmaf(part_ml[w][1][lane], f, l);
-#pragma unroll
-    for (int dt = 0; dt < DVM; ++dt)
-      if (dt < dvt) {
-        const f32x4 o = *reinterpret_cast<const f32x4*>(part_o[w][dt][lane]);
-        oacc[dt] += o * f;
-      }
+  for (int w = 0; w < WAVES; ++w) {
+    f[w] = f[w] == -INFINITY ? 0.f : expf(f[w] - mm);
+    l = fmaf(part_ml[w][1][lane], f[w], l);
   }
-  if (n_split > 1) {
-    // several workgroups share this (row, head): leave (max, sum, unnormalised accumulator) for the merge kernel
-    float* p = ws + (((int64_t)row * H + h0 + qi) * n_split + split) * (2 + Dv);
-    if (kg == 0) p[0] = mm, p[1] = l;
-#pragma unroll
-    for (int dt = 0; dt < DVM; ++dt) {
-      if (dt < dvt) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int d = PAIR ? (dt >> 1) * 32 + 2 * (kg * 4 + r) + (dt & 1) : dt * 16 + kg * 4 + r;
-          p[2 + d] = oacc[dt][r];
-        }
-      }
-    }
-    return;
-  }
-  const float inv = 1.f / with_sink(bias, h0 + qi, mm, l);
+  constexpr int ND = DVM / WAVES;
+  // several workgroups that share this (row, head) leave (max, sum, unnormalised accumulator) for the merge kernel
+  float* const p = n_split > 1 ? ws + (((int64_t)row * H + h0 + qi) * n_split + split) * (2 + Dv) : nullptr;
+  if (p && wave == 0 && kg == 0) p[0] = mm, p[1] = l;
+  const float inv = n_split > 1 ? 1.f : 1.f / with_sink(bias, h0 + qi, mm, l);
   const int64_t obase = (int64_t)row * ldo + (int64_t)(h0 + qi) * Dv;
   const int64_t gbase = (int64_t)row * ldg + (int64_t)(h0 + qi) * Dv;
 #pragma unroll
-  for (int dt = 0; dt < DVM; ++dt) {
-    if (dt < dvt) {
+  for (int i = 0; i < ND; ++i) {
+    const int dt = wave * ND + i;
+    if (dt >= dvt) break;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d = PAIR ? (dt >> 1) * 32 + 2 * (kg * 4 + r) + (dt & 1) : dt * 16 + kg * 4 + r;
-        float o = oacc[dt][r] * inv;
-        if (gate) o *= sigmoid_f(gate[gbase + d]);
-        out[obase + d] = o;
+    for (int w = 0; w < WAVES; ++w) o += *reinterpret_cast<const f32x4*>(part_o[w][dt][lane]) * f[w];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = (dt / VW) * 16 * VW + VW * (kg * 4 + r) + dt % VW;
+      if (p) {
+        p[2 + d] = o[r];
+      } else {
+        float y = o[r] * inv;
+        if (gate) y *= sigmoid_f(gate[gbase + d]);
+        out[obase + d] = y;
       }
     }
   }
@@ -2120,28 +2168,36 @@ static int launch_swa(const float* q, int64_t ldq, const void* kc, const void* v
   if constexpr (sizeof(TC) == 2) {
     // decode steps (a row per sequence) over a bf16 cache: the matrix-core form with a kv head's query heads as columns
     if (v16 && rows == n_seqs && D % 32 == 0 && Dv % 16 == 0 && D <= 256 && Dv <= 256 && ldv % 2 == 0 && G <= 65535) {
-      // few (row, kv head) units: up to 16 workgroups share one, each taking every n_split-th batch of four rounds, and
-      // a second launch merges their partial results (workspace: rows * H * n_split * (2 + Dv) floats)
+      // few (row, kv head) units: up to 16 workgroups share one, each taking every n_split-th batch of rounds, and a second launch
+      // merges their partial results (workspace: rows * H * n_split * (2 + Dv) floats).  At most one workgroup per CU: their registers
+      // leave no room for a second, and the rest would wait for the first ones' end
       const int chunks = (H / G + 15) / 16;
       int n_split = 1;
-      while (n_split < 16 && (int64_t)rows * G * chunks * n_split < 256 &&
+      while (n_split < 16 && (int64_t)rows * G * chunks * (2 * n_split) <= 256 &&
              (int64_t)rows * H * (2 * n_split) * (2 + Dv) <= ws_elems)
         n_split *= 2;
       if (!ws) n_split = 1;
       const dim3 grid_h(rows, G, chunks * n_split);
-#define MI_HEADS_MFMA(DKM, DVM, PAIR, KEEP)                                                                           \
-  hipLaunchKernelGGL((paged_attention_heads_mfma_kernel<DKM, DVM, PAIR, KEEP>), grid_h, dim3(256), 0, st, q, ldq, k, v,  \
-                     bt, cols, kv_lens, H, G, D, Dv, block_size, window, scale, bias, ldv, gate, ldg, out, ldo, n_split, ws)
-#define MI_HEADS_MFMA_KEEP(DKM, DVM, PAIR)                    \
-  do {                                                        \
-    if (bias.kept > 0) MI_HEADS_MFMA(DKM, DVM, PAIR, true);   \
-    else MI_HEADS_MFMA(DKM, DVM, PAIR, false);                \
+#define MI_HEADS_MFMA(DKM, DVM, VW, KEEP, FAST)                                                                        \
+  hipLaunchKernelGGL((paged_attention_heads_mfma_kernel<DKM, DVM, VW, KEEP, FAST, DVM <= 8 ? 8 : 4>), grid_h,             \
+                     dim3(DVM <= 8 ? 512 : 256), 0, st, q, ldq, k, v, bt, cols, kv_lens, H, G, D, Dv, block_size, window,    \
+                     scale, bias, ldv, gate, ldg, out, ldo, n_split, ws)
+#define MI_HEADS_MFMA_KEEP(DKM, DVM, VW, FAST)                      \
+  do {                                                               \
+    if (bias.kept > 0) MI_HEADS_MFMA(DKM, DVM, VW, true, FAST);     \
+    else MI_HEADS_MFMA(DKM, DVM, VW, false, FAST);                  \
   } while (0)
-      const bool small = D <= 128 && Dv <= 128, pair = Dv % 32 == 0;
-      if (small && pair) MI_HEADS_MFMA_KEEP(4, 8, true);
-      else if (small) MI_HEADS_MFMA_KEEP(4, 8, false);
-      else if (pair) MI_HEADS_MFMA_KEEP(8, 16, true);
-      else MI_HEADS_MFMA_KEEP(8, 16, false);
+      const bool small = D <= 128 && Dv <= 128;
+      const int vw = Dv % 128 == 0 && ldv % 8 == 0 ? 8 : Dv % 32 == 0 ? 2 : 1;
+      const bool plain = vw == 8 && bias.kind != MI_BIAS_LOG && !(bias.softcap > 0.f) && (block_size & (block_size - 1)) == 0;
+      if (plain && D == 128 && Dv == 128) MI_HEADS_MFMA_KEEP(4, 8, 8, true);
+      else if (plain && D == 256 && Dv == 256) MI_HEADS_MFMA_KEEP(8, 16, 8, true);
+      else if (small && vw == 8) MI_HEADS_MFMA_KEEP(4, 8, 8, false);
+      else if (small && vw == 2) MI_HEADS_MFMA_KEEP(4, 8, 2, false);
+      else if (small) MI_HEADS_MFMA_KEEP(4, 8, 1, false);
+      else if (vw == 8) MI_HEADS_MFMA_KEEP(8, 16, 8, false);
+      else if (vw == 2) MI_HEADS_MFMA_KEEP(8, 16, 2, false);
+      else MI_HEADS_MFMA_KEEP(8, 16, 1, false);
 #undef MI_HEADS_MFMA_KEEP
 #undef MI_HEADS_MFMA
       if (check_launch() != MI_OK) return MI_ELAUNCH;
