@@ -5,7 +5,7 @@
 // (bf16 products of more rows than any_stream_takes says - K a multiple of 64, no segments - go to gemm_any_tile.hip.)
 //
 // These serve the model families whose residual stream, norms and recurrences are kept in 32-bit floats and whose
-// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): eight kernels,
+// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): nine kernels,
 //
 //   gemm_any_mfma_kernel   bf16 weights: a 64 x 64 (from 512 rows: 128 x 128, with SwiGLU 128 x 64) output tile per 4-wave
 //                          workgroup, x rounded to bf16 on its way into LDS, v_mfma_f32_16x16x32_bf16, the next K
@@ -14,6 +14,8 @@
 //                          workgroup, the waves split K, fragments straight from memory
 //   gemm_any_stream_kernel bf16 weights, 9 to 64 rows and experts of few rows each, K a multiple of 64: the same work with two 64-deep
 //                          blocks in flight per wave and whole lines through LDS
+//   gemm_any_heads_kernel  bf16 weights, the batched form over many rows (a head's projection of its own columns): the head's weight in
+//                          LDS, x rows straight into operands
 //   gemm_any_f32_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, on the fp32 matrix instruction
 //                          - the float32 serving mode, and the routers of sparse feed-forwards in either mode
 //   gemm_any_fma_kernel    the same in plain FMA chains, for operands whose rows are not whole 128-byte lines
@@ -1021,6 +1023,83 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
   return launch_exact<TW, DUAL, EXT>(a, groups, rows_per_group_max, st);
 }
 
+// Per-head products of many rows (latent attention's: 8192 rows x 16 heads, 128 -> 256 and back).  What bounds it: memory - x in and y
+// out are 24 KiB per 16 rows of a head, its 64 KiB of weights the only reuse.  So no operand pass and no x tile: a workgroup keeps ONE
+// head's weight in LDS (rows padded by 16 bytes: a lane group's sixteen rows in sixteen bank slots), and its eight waves walk 16-row
+// tiles, x rows from memory into the MFMA operand (rounded to bf16 once, as gemm_any_mfma_kernel does), the next tile's rows requested
+// before this one is multiplied; two workgroups per CU.  gemm_any_mfma_kernel (both operands through LDS for every 64 features, two barriers per K
+// step): 128 -> 256 160 us, 256 -> 128 98 us; here 48 and 43 (4.2 and 4.7 TB/s).  Same summation order (k ascending in one chain), same bits.
+constexpr int kHeadsWeightElems = 32768, kHeadsLds = 2 * kHeadsWeightElems + 16 * 512;
+template <int KF>  // K = 32 KF (256: one workgroup per CU, the next rows' registers)
+__global__ __launch_bounds__(512, KF == 8 ? 2 : 4) void gemm_any_heads_kernel(GemmAnyArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[kHeadsLds];
+  constexpr int K = 32 * KF, ROW = 2 * K + 16;
+  const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int m_lo, m_hi;
+  const uint16_t *w, *w2;
+  select_group<uint16_t, false>(a, w, w2, m_lo, m_hi);
+  for (int i = threadIdx.x; i < a.N * (K / 8); i += 512)
+    *reinterpret_cast<u32x4*>(lds + (i / (K / 8)) * ROW + (i % (K / 8)) * 16) = *reinterpret_cast<const u32x4*>(w + (int64_t)i * 8);
+  f32x4 raw[KF][2];
+  auto request = [&](int m0) __attribute__((always_inline)) {
+    const float* xp = a.x + (int64_t)min(m0 + r16, m_hi - 1) * a.ldx + q * 8;
+#pragma unroll
+    for (int ks = 0; ks < KF; ++ks) {
+      raw[ks][0] = *reinterpret_cast<const f32x4*>(xp + ks * 32);
+      raw[ks][1] = *reinterpret_cast<const f32x4*>(xp + ks * 32 + 4);
+    }
+  };
+  int m0 = (blockIdx.x * 8 + wave) * 16;
+  const int step = gridDim.x * 128;
+  request(m0);
+  __syncthreads();
+  for (; m0 < m_hi; m0 += step) {
+    bf16x8 xf[KF];
+#pragma unroll
+    for (int ks = 0; ks < KF; ++ks)
+      xf[ks] = as_frag(u32x4{pack_bf(raw[ks][0][0], raw[ks][0][1]), pack_bf(raw[ks][0][2], raw[ks][0][3]), pack_bf(raw[ks][1][0], raw[ks][1][1]),
+                             pack_bf(raw[ks][1][2], raw[ks][1][3])});
+    request(m0 + step);   // (past the last tile: the last row again)
+    const int m = m0 + r16;
+    float* yp = a.y + (int64_t)m * a.ldy + q * 4;
+    const float* gp = a.gate ? a.gate + (int64_t)min(m, m_hi - 1) * a.ldgate + q * 4 : nullptr;
+    for (int n = 0; n < a.N; n += 32) {
+      f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int ks = 0; ks < KF; ++ks)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              as_frag(*reinterpret_cast<const u32x4*>(lds + (n + t * 16 + r16) * ROW + ks * 64 + q * 16)), xf[ks], acc[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if (gp) {
+          const f32x4 g = *reinterpret_cast<const f32x4*>(gp + n + t * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[t][e] *= 1.f / (1.f + expf(-g[e]));
+        }
+        if (m < m_hi) *reinterpret_cast<f32x4*>(yp + n + t * 16) = acc[t];
+      }
+    }
+  }
+}
+// x, y and gate rows in 16-byte pieces, whole 32-feature steps, a head's weight in LDS; up to 64 rows the products stream their weights
+static bool heads_takes(const GemmAnyArgs& a, int w_dtype, int n_batch, bool exact) {
+  return !exact && w_dtype == MI_DTYPE_BF16 && n_batch > 1 && a.M > 64 && (a.K == 64 || a.K == 128 || a.K == 256) && a.N > 0 &&
+         a.N % 32 == 0 && a.N <= 512 && a.N * a.K <= kHeadsWeightElems && aligned16(a.x) && aligned16(a.w) && aligned16(a.y) &&
+         a.ldx % 4 == 0 && a.x_batch % 4 == 0 && a.ldy % 4 == 0 && a.y_batch % 4 == 0 &&
+         (!a.gate || (aligned16(a.gate) && a.ldgate % 4 == 0 && a.gate_batch % 4 == 0));
+}
+static int launch_heads(const GemmAnyArgs& a, int n_batch, hipStream_t st) {
+  const int rows = (a.M + 127) / 128, fill = ((a.K == 256 ? 256 : 512) + n_batch - 1) / n_batch;   // (the workgroups that run together)
+  const dim3 grid(rows < fill ? rows : fill, 1, n_batch);
+  if (a.K == 64) hipLaunchKernelGGL((gemm_any_heads_kernel<2>), grid, dim3(512), 0, st, a);
+  else if (a.K == 128) hipLaunchKernelGGL((gemm_any_heads_kernel<4>), grid, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((gemm_any_heads_kernel<8>), grid, dim3(512), 0, st, a);
+  return check_launch();
+}
+
 }  // namespace mi
 
 using namespace mi;
@@ -1069,6 +1148,7 @@ extern "C" int mi_gemm_any_batched(const float* x, int64_t ldx, int64_t x_batch,
   if (n_batch > 65535) return MI_EUNSUPPORTED;
   GemmAnyArgs a{x, ldx, w, nullptr, y, ldy, M, N, K, 1.0f, nullptr, nullptr, nullptr, nullptr, nullptr, MI_ACT_NONE,
                 gate, ldgate, x_batch, y_batch, gate_batch, nullptr, nullptr, 0.f, false, 0, 0, 0};
+  if (heads_takes(a, w_dtype, n_batch, exact != 0)) return launch_heads(a, n_batch, S(stream));
   return gemm_any_dispatch(a, w_dtype, n_batch, M, exact ? 1 : 0, S(stream));
 }
 
