@@ -820,6 +820,11 @@ int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_token, const m
                  int act, float limit, const float* row_scale, const int32_t* row_scale_rows, const int32_t* offsets,
                  const int32_t* pair_index, int pairs, int n_groups, int ff, int width, void* scratch, int64_t scratch_bytes, float* y,
                  mi_stream stream);
+/* ... with the rows of x named (0: not known): every entry of pair_token lies in [0, tokens).  The same results. */
+int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, const int32_t* pair_token, const mi_bf16* w, const mi_bf16* w2,
+                        const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
+                        const int32_t* offsets, const int32_t* pair_index, int pairs, int n_groups, int ff, int width, void* scratch,
+                        int64_t scratch_bytes, float* y, mi_stream stream);
 /* mi_gemm_any_grouped with the activation named: y = act(x w^T) (* (x w2^T) with w2). */
 int mi_gemm_any_grouped_act(const float* x, int64_t ldx, const int32_t* x_rows, const void* w, const void* w2, int w_dtype,
                             int act, const int32_t* group_offsets, int n_groups, int rows_per_group_max, float* y,

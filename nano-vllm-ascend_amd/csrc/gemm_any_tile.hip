@@ -16,10 +16,13 @@
 namespace mi {
 
 // Table of a grouped operand: {row tiles, 0, 0, 0}, then per row tile {group, first row, end of the group's rows, 0}.
-template <int ACT, bool DUAL>
+// GATHER: the (sorted) rows' activations lie at rows x_rows[.] of x, which has x_total rows.
+template <int ACT, bool DUAL, bool GATHER = false>
 struct AnyTileArgs : TileArgs {
   static constexpr int kAct = ACT;
-  static constexpr bool kDual = DUAL;
+  static constexpr bool kDual = DUAL, kGather = GATHER;
+  const int32_t* x_rows;
+  int x_total;
   const uint16_t* w2;
   int groups;
   const int32_t* table;  // nullptr: one group of M rows
@@ -95,18 +98,19 @@ __device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, 
 #include "gemm_w16_kernel.hpp"
 #include "gemm_mid_kernel.hpp"
 
-// x rows -> bf16 rows (eight elements a thread), gathered by x_rows; rows from the groups' end on are left as they are.
-// The grid's last workgroup writes the tile table: `table_tiles` entries at most, of rows before `rows` - whatever the groups' ends say,
-// nothing is written or, by the product that follows the table, read beyond the buffers.
+// x rows -> bf16 rows (eight elements a thread), gathered by x_rows; rows from the groups' end on are left as they are.  sorted == 0: the
+// `rows` rows are those the groups lie in; else the groups lie in `sorted` rows, which the product gathers, and every row is converted.
+// The grid's last workgroup writes the tile table: `table_tiles` entries at most, of rows before `rows` (`sorted`) - whatever the groups'
+// ends say, nothing is written or, by the product that follows the table, read beyond the buffers.
 __global__ __launch_bounds__(256) void any_operand_kernel(const float* __restrict__ x, int64_t ldx,
                                                           const int32_t* __restrict__ x_rows,
                                                           const int32_t* __restrict__ group_offsets, int n_groups,
-                                                          int tile_rows, int rows, int K, uint16_t* __restrict__ xb,
+                                                          int tile_rows, int rows, int sorted, int K, uint16_t* __restrict__ xb,
                                                           int32_t* __restrict__ table, int table_tiles) {
   __shared__ int tiles[1024];
   const int tid = threadIdx.x;
   if (table && blockIdx.x == gridDim.x - 1) {
-    auto end_of = [&](int g) { return min(max(group_offsets[g], 0), rows); };
+    auto end_of = [&](int g) { return min(max(group_offsets[g], 0), sorted ? sorted : rows); };
     for (int g = tid; g < n_groups; g += 256) tiles[g] = (max(end_of(g + 1) - end_of(g), 0) + tile_rows - 1) / tile_rows;
     __syncthreads();
     for (int g = tid; g < n_groups; g += 256) {
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(256) void any_operand_kernel(const float* __restric
   const int per_row = K >> 3;
   const int64_t i = (int64_t)blockIdx.x * 256 + tid;
   const int row = (int)(i / per_row), c = (int)(i - (int64_t)row * per_row) * 8;
-  if (row >= rows || (group_offsets && row >= group_offsets[n_groups])) return;
+  if (row >= rows || (group_offsets && !sorted && row >= group_offsets[n_groups])) return;
   const float* src = x + (int64_t)(x_rows ? x_rows[row] : row) * ldx + c;
   float4 a, b;
   if ((ldx & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
@@ -186,9 +190,9 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   return act != MI_ACT_SOFTCAP && ((rows + 255) / 256) * (int64_t)((N + tf - 1) / tf) >= 160 ? 256 : 128;
 }
 
-template <int ACT, bool DUAL>
-static int launch_any_tile(const AnyTileArgs<ACT, DUAL>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
-  using A = AnyTileArgs<ACT, DUAL>;
+template <int ACT, bool DUAL, bool GATHER>
+static int launch_any_tile(const AnyTileArgs<ACT, DUAL, GATHER>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
+  using A = AnyTileArgs<ACT, DUAL, GATHER>;
   A a = args;
   if (tile_rows == 256) {
     a.tiles_f = (a.N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
@@ -238,9 +242,8 @@ extern "C" int64_t mi_gemm_any_table_ints(int rows, int n_groups, int tile_rows)
   return 4 + 4 * row_tiles(rows, n_groups, tile_rows);
 }
 
-extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets,
-                                   int n_groups, int tile_rows, int rows, int K, mi_bf16* xb, int32_t* table,
-                                   mi_stream stream) {
+static int any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets, int n_groups, int tile_rows,
+                       int rows, int sorted, int K, mi_bf16* xb, int32_t* table, mi_stream stream) {
   if (!x || !xb || rows < 0 || K < 8 || K % 8 || ldx < K || !aligned16(xb)) return MI_EINVAL;
   if (n_groups < 0 || n_groups > 1024 || (n_groups > 0) != (group_offsets != nullptr)) return MI_EINVAL;
   if (table && (!n_groups || !aligned16(table) || !tile_rows_ok(tile_rows))) return MI_EINVAL;
@@ -248,14 +251,21 @@ extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x
   const int64_t blocks = ((int64_t)rows * (K / 8) + 255) / 256 + (table ? 1 : 0);
   if (blocks > 0x7fffffff) return MI_EUNSUPPORTED;
   hipLaunchKernelGGL(any_operand_kernel, dim3((unsigned)blocks), dim3(256), 0, S(stream), x, ldx, x_rows, group_offsets, n_groups,
-                     tile_rows, rows, K, xb, table, table ? (int)row_tiles(rows, n_groups, tile_rows) : 0);
+                     tile_rows, rows, sorted, K, xb, table, table ? (int)row_tiles(sorted ? sorted : rows, n_groups, tile_rows) : 0);
   return check_launch();
 }
 
-extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int tile_rows, const mi_bf16* w, const mi_bf16* w2,
-                                const float* bias, const float* bias2, int act, float limit, const float* row_scale,
-                                const int32_t* row_scale_rows, int n_groups, void* y, int y_is_bf16, int64_t ldy,
-                                const int32_t* y_rows, int rows, int N, int K, float alpha, mi_stream stream) {
+extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets,
+                                   int n_groups, int tile_rows, int rows, int K, mi_bf16* xb, int32_t* table,
+                                   mi_stream stream) {
+  return any_operand(x, ldx, x_rows, group_offsets, n_groups, tile_rows, rows, 0, K, xb, table, stream);
+}
+
+// x_rows (two weights, groups): row m of the groups' rows is row x_rows[m] of xb's x_total
+static int any_tile_product(const mi_bf16* xb, const int32_t* x_rows, int x_total, const int32_t* table, int tile_rows, const mi_bf16* w,
+                            const mi_bf16* w2, const float* bias, const float* bias2, int act, float limit, const float* row_scale,
+                            const int32_t* row_scale_rows, int n_groups, void* y, int y_is_bf16, int64_t ldy, const int32_t* y_rows,
+                            int rows, int N, int K, float alpha, mi_stream stream) {
   if (!xb || !w || !y || rows < 0 || (n_groups > 0) != (table != nullptr) || (row_scale_rows && !row_scale)) return MI_EINVAL;
   if (act == MI_ACT_CLAMPED_GLU && !(limit > 0.f)) return MI_EINVAL;
   if (act == MI_ACT_SOFTCAP && tile_rows == 256) return MI_EUNSUPPORTED;   // (launch_any_tile)
@@ -273,8 +283,15 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
     args.y32 = y_is_bf16 ? nullptr : static_cast<float*>(y), args.y16 = y_is_bf16 ? static_cast<uint16_t*>(y) : nullptr;
     args.y_rows = y_rows, args.bias1 = bias, args.bias2 = bias2, args.alpha = alpha, args.limit = limit;
     args.row_scale = row_scale, args.row_scale_rows = row_scale_rows;
+    args.x_rows = x_rows, args.x_total = x_total;
     return launch_any_tile(args, tile_rows, tiles, S(stream));
   };
+  if (x_rows) {
+    if (!w2 || !table || x_total < 1 || x_total > rows) return MI_EINVAL;   // (xb's rows: at most as many as the limits were taken for)
+    if (act == MI_ACT_SILU) return go(AnyTileArgs<MI_ACT_SILU, true, true>{});
+    if (act == MI_ACT_GELU_TANH) return go(AnyTileArgs<MI_ACT_GELU_TANH, true, true>{});
+    return go(AnyTileArgs<MI_ACT_CLAMPED_GLU, true, true>{});
+  }
   if (w2) {
     if (act == MI_ACT_SILU) return go(AnyTileArgs<MI_ACT_SILU, true>{});
     if (act == MI_ACT_GELU_TANH) return go(AnyTileArgs<MI_ACT_GELU_TANH, true>{});
@@ -284,6 +301,14 @@ extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int til
   if (act == MI_ACT_SOFTCAP) return alpha > 0.f ? go(AnyTileArgs<MI_ACT_SOFTCAP, false>{}) : MI_EINVAL;
   if (act == MI_ACT_GELU_ERF) return go(AnyTileArgs<MI_ACT_GELU_ERF, false>{});
   return go(AnyTileArgs<MI_ACT_RELU2, false>{});
+}
+
+extern "C" int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int tile_rows, const mi_bf16* w, const mi_bf16* w2,
+                                const float* bias, const float* bias2, int act, float limit, const float* row_scale,
+                                const int32_t* row_scale_rows, int n_groups, void* y, int y_is_bf16, int64_t ldy,
+                                const int32_t* y_rows, int rows, int N, int K, float alpha, mi_stream stream) {
+  return any_tile_product(xb, nullptr, 0, table, tile_rows, w, w2, bias, bias2, act, limit, row_scale, row_scale_rows, n_groups, y,
+                          y_is_bf16, ldy, y_rows, rows, N, K, alpha, stream);
 }
 
 // ---- the two launches (operand pass, product) and the choice between these kernels and gemm_any.hip's behind one call: steps that are
@@ -329,6 +354,17 @@ extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_tok
                             const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
                             const int32_t* offsets, const int32_t* pair_index, int pairs, int G, int ff, int width, void* scratch,
                             int64_t scratch_bytes, float* y, mi_stream stream) {
+  return mi_expert_ff_tokens(x, ldx, 0, pair_token, w, w2, down, act, limit, row_scale, row_scale_rows, offsets, pair_index, pairs, G, ff,
+                             width, scratch, scratch_bytes, y, stream);
+}
+
+// tokens: the rows of x (0: not known).  Where the pairs are at least as many, x is rounded to bf16 a token at a time and the first
+// product's feed gathers the pairs' rows; else the operand pass writes them out in the experts' order (65536 pairs of 8192 tokens x 2048,
+// us: pass 112 + product 459, now 15 + 441).
+extern "C" int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, const int32_t* pair_token, const mi_bf16* w,
+                                   const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale,
+                                   const int32_t* row_scale_rows, const int32_t* offsets, const int32_t* pair_index, int pairs, int G,
+                                   int ff, int width, void* scratch, int64_t scratch_bytes, float* y, mi_stream stream) {
   if (!x || !w || !down || !offsets || !scratch || !y || pairs < 1 || G < 1 || !aligned16(scratch)) return MI_EINVAL;
   const int64_t need = mi_expert_ff_bytes(pairs, G, ff, width, w2 != nullptr, act);
   if (need == 0) return MI_EUNSUPPORTED;
@@ -346,10 +382,12 @@ extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_tok
   mi_bf16* xb = reinterpret_cast<mi_bf16*>(p);
   mi_bf16* inner = reinterpret_cast<mi_bf16*>(p += round16((int64_t)pairs * width * 2));
   int32_t* table = reinterpret_cast<int32_t*>(p += round16((int64_t)pairs * ff * 2));
-  int rc = mi_gemm_any_operand(x, ldx, pair_token, offsets, G, t, pairs, width, xb, table, stream);
+  const bool gather = w2 && pair_token && tokens > 0 && tokens <= pairs;
+  int rc = gather ? any_operand(x, ldx, nullptr, offsets, G, t, tokens, pairs, width, xb, table, stream)
+                  : mi_gemm_any_operand(x, ldx, pair_token, offsets, G, t, pairs, width, xb, table, stream);
   if (rc == MI_OK)
-    rc = mi_gemm_any_tile(xb, table, t, w, w2, nullptr, nullptr, act, limit, row_scale, row_scale_rows, G, inner, 1, ff, nullptr, pairs, ff,
-                          width, 1.f, stream);
+    rc = any_tile_product(xb, gather ? pair_token : nullptr, gather ? tokens : 0, table, t, w, w2, nullptr, nullptr, act, limit, row_scale,
+                          row_scale_rows, G, inner, 1, ff, nullptr, pairs, ff, width, 1.f, stream);
   return rc != MI_OK ? rc
                      : mi_gemm_any_tile(inner, table, t, down, nullptr, nullptr, nullptr, MI_ACT_NONE, 0.f, nullptr, nullptr, G, y, 0, width,
                                         pair_index, pairs, width, ff, 1.f, stream);

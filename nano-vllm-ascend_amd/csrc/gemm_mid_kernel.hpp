@@ -63,7 +63,10 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
 #pragma unroll
   for (int i = 0; i < SH::B_PIECES; ++i) {
     const int lr = (wave * SH::B_PIECES + i) * 8 + (lane >> 3), c = (lane & 7) ^ swizzle(lr);
-    srcB[i] = reinterpret_cast<const char*>(a.x) + kbeg_bytes + ((int64_t)min(m0 + lr, m_end - 1) * a.ldx + c * 8) * 2;
+    int64_t rowB = min(m0 + lr, m_end - 1);
+    if constexpr (EPI == TEPI_ANY)
+      if (ARGS::kGather) rowB = a.x_rows[rowB];
+    srcB[i] = reinterpret_cast<const char*>(a.x) + kbeg_bytes + (rowB * a.ldx + c * 8) * 2;
   }
   auto issue = [&](int kt, int p) __attribute__((always_inline)) {
     char* dst = lds + p * SH::STAGE;

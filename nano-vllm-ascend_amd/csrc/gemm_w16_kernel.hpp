@@ -26,6 +26,7 @@
 template <int EPI, bool BIAS, int V, class ARGS = TileArgs>
 __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   constexpr bool LINES = (V & 32768) != 0 && EPI != TEPI_PARTIAL && EPI != TEPI_ANY;
+  constexpr bool GATHER = EPI == TEPI_ANY && ARGS::kGather;  // a tile's activation rows wherever x_rows says
   constexpr bool PAIRED = EPI == TEPI_ANY && ARGS::kDual;  // two weights: half 0 of the A region holds 128 rows of w, half 1 of w2
   __shared__ __attribute__((aligned(1024))) char lds[2 * W16_STEP_BYTES + (LINES ? 4 * W4_STAGE_BYTES : 0)];
   const int lane = threadIdx.x & 63;
@@ -47,6 +48,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   if constexpr (EPI == TEPI_ANY) {
     if (wgt) records *= (uint32_t)a.groups;
     if (PAIRED && wave == 1) src = a.w2;
+    if (GATHER && !wgt) records = (uint32_t)a.x_total * ld2;
   }
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(src), 0, records, 0x00020000);
   // per-lane part of a piece's source offset: the rows of slice lane >> 3 depend on the piece through ONE bit (x3 of the
@@ -59,10 +61,28 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
                (wgt && EPI == TEPI_SILU ? (uint32_t)((rows & 63) + (rows >> 6) * (a.N >> 1)) : (uint32_t)rows) * ld2;
   }
   uint32_t f_row, f_k = kbeg_bytes;
+  uint32_t g_off[EPI == TEPI_ANY && ARGS::kGather ? W4_PIECES : 1];  // GATHER: every piece's source offset (sixteen index loads per tile, in front of some 32 K steps)
   int f_kt = 0, f_blk = (int)blockIdx.x;
   auto fetch_tile = [&](int b) __attribute__((always_inline)) {
     if (b >= ntiles) {  // past the workgroup's last tile: every row beyond the descriptor - the pieces fetch nothing
       f_row = 0xF0000000u;
+      if constexpr (GATHER) {
+#pragma unroll
+        for (int q = 0; q < W4_PIECES; ++q) g_off[q] = f_row;
+      }
+      return;
+    }
+    if constexpr (GATHER) {
+      const AnyTile t = any_tile(a, b, ntiles, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
+      if (wgt) {
+        f_row = (uint32_t)(t.group * a.N + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
+#pragma unroll
+        for (int q = 0; q < W4_PIECES; ++q) g_off[q] = voff[w16_piece_x3(q)] + (f_row + (uint32_t)w16_piece_rows(q) * ld2);
+      } else {
+#pragma unroll
+        for (int q = 0; q < W4_PIECES; ++q)
+          g_off[q] = (uint32_t)(lane & 7) * 16 + (uint32_t)a.x_rows[min(t.m0 + w16_dma_row(wave, q, lane), t.m_end - 1)] * ld2;
+      }
       return;
     }
     if constexpr (EPI == TEPI_ANY) {
@@ -81,8 +101,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   char* const pieces = lds + wave * (W4_PIECES * W16_PIECE_BYTES);
   int wbuf = 0;
   auto piece = [&](int q) __attribute__((always_inline)) {
+    uint32_t off = 0;
+    if constexpr (EPI == TEPI_ANY && ARGS::kGather) off = g_off[q];
+    else off = voff[w16_piece_x3(q)] + (f_row + (uint32_t)w16_piece_rows(q) * ld2);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(pieces + wbuf * W16_STEP_BYTES + q * W16_PIECE_BYTES), 16,
-                                             voff[w16_piece_x3(q)] + (f_row + (uint32_t)w16_piece_rows(q) * ld2), f_k, 0, 0);
+                                             off, f_k, 0, 0);
   };
   auto fetch_advance = [&]() __attribute__((always_inline)) {
     wbuf ^= 1;

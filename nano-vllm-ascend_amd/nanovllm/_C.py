@@ -217,6 +217,8 @@ _SIGNATURES = {
     "mi_expert_ff_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mi_expert_ff": (c_int, [_p, c_int64, _p, _p, _p, _p, c_int, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p, c_int64, _p,
                              _p]),
+    "mi_expert_ff_tokens": (c_int, [_p, c_int64, c_int, _p, _p, _p, _p, c_int, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p,
+                                    c_int64, _p, _p]),
     "mi_gemm_any_operand": (c_int, [_p, c_int64, _p, _p, c_int, c_int, c_int, c_int, _p, _p, _p]),
     "mi_gemm_any_tile": (c_int, [_p, _p, c_int, _p, _p, _p, _p, c_int, c_float, _p, _p, c_int, _p, c_int, c_int64, _p, c_int,
                                  c_int, c_int, c_float, _p]),
