@@ -942,6 +942,15 @@ int mi_linear_attention(const float* proj, int64_t ld, int q_off, int k_off, int
                         int64_t ld_gate, const float* norm_w, int norm_groups, float* state, const int32_t* cu_q,
                         const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows, int H, int D, int Dv,
                         float eps, float* out, int64_t ldo, mi_stream stream);
+/* ... with room for the block form (sixteen rows at a time on the matrix cores): mi_linear_attention_blocks_elems gives the floats of a
+ * 16-byte aligned workspace, 0 where row by row is faster (max_rows: the most rows one sequence brings), -1 where D is not taken.
+ * workspace NULL: row by row.  The two differ by rounding only. */
+int64_t mi_linear_attention_blocks_elems(int n_rows, int n_seqs, int max_rows, int H, int D);
+int mi_linear_attention_ws(const float* proj, int64_t ld, int q_off, int k_off, int v_off, int q_act, int k_act, int v_act, int decay_kind,
+                           const float* decay, const float* f_bias, const float* lower, const float* gate_pre, int64_t ld_gate,
+                           const float* norm_w, int norm_groups, float* state, const int32_t* cu_q, const int32_t* kv_lens,
+                           const int32_t* slot_ids, int n_seqs, int n_rows, int H, int D, int Dv, float eps, float* workspace,
+                           int64_t ws_elems, float* out, int64_t ldo, mi_stream stream);
 
 /* Rotary positions on the projected heads of a step's rows, in place: H query heads [D] at q_off and G key heads [D] at
  * k_off of every proj row.  Position of a row as in mi_paged_attention_f32 (cu_q, kv_lens); angle of pair i =

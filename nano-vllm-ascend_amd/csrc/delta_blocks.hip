@@ -14,10 +14,13 @@
 // are the next block's B operand as they stand) walks a sequence's records.
 //
 // What bounds it: the chain of a sequence's blocks; 104 matrix instructions of 32 cycles each (128 channels) are 1.4 us, the vector
-// work between them brings a block to 2.7 us, against 0.71 us per ROW of the row-by-row walk (LDS reads, cross-lane sums, plain FMAs).
+// work between them brings a block to 2.5 us (2.7 with the accumulators copied to be scaled: the Makefile's flag), against 0.71 us per
+// ROW of the row-by-row walk (LDS reads, cross-lane sums, plain FMAs).
 // 8 sequences of 1024 rows, 8 heads, 128 x 128: 809 us row by row, 294 so (preparation 83, walk 175).  The error against 64 bits is
 // the row-by-row one's or less (rms of the results, 64 .. 1400 rows and decays from 0.05 to 1: 0.87 to 0.98 of it).  A NaN or an
 // infinity in a row must not reach the rows in front of it through the zeros above the diagonals of T and B: see causal() below.
+#include <type_traits>
+
 #include "seqmix_common.hpp"
 
 namespace mi {
@@ -54,15 +57,19 @@ struct BlockArgs {
 };
 
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
-// y = L b of a lower triangular L, operands and result as the walk has them (a lane: rows 4 kg .. + 3 of its column), where the matrix
-// instruction's zeros above L's diagonal met a b that is not finite: rows in front of the column's first such row are taken again with
-// zeros from it on (their sums do not reach that far), the others stay what they are - the row-by-row walk's is not finite either.
-__device__ __forceinline__ f32x4 causal(f32x4 l, f32x4 b, f32x4 y, int kg) {
+// the first of the block's rows whose value in this lane's column is not finite (kB: none)
+__device__ __forceinline__ int first_bad(f32x4 b, int kg) {
   int first = kB;
 #pragma unroll
   for (int r = 3; r >= 0; --r) first = finite(b[r]) ? first : 4 * kg + r;
   first = min(first, __shfl_xor(first, 16));
-  first = min(first, __shfl_xor(first, 32));
+  return min(first, __shfl_xor(first, 32));
+}
+// y = L b of a lower triangular L, operands and result as the walk has them (a lane: rows 4 kg .. + 3 of its column), where the matrix
+// instruction's zeros above L's diagonal met a b that is not finite: rows in front of the column's first such row are taken again with
+// zeros from it on (their sums do not reach that far), the others stay what they are - the row-by-row walk's is not finite either.
+__device__ __forceinline__ f32x4 causal(f32x4 l, f32x4 b, f32x4 y, int kg) {
+  const int first = first_bad(b, kg);
   f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int r = 0; r < 4; ++r) z = __builtin_amdgcn_mfma_f32_16x16x4f32(l[r], 4 * kg + r < first ? b[r] : 0.f, z, 0, 0, 0);
@@ -381,6 +388,339 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Linear attention with a decayed state (mi_linear_attention's recurrence, S <- diag(g_t) S + k_t v_t^T, o_t = S^T q_t) in the same blocks:
+//   O = (q_t P_t)^T S0 + B V,   B_tj = sum_d q_t P_jt k_j  (j <= t),      S <- diag(P_15) S0 + sum_j (k_j P_j15) v_j^T
+// FORGET: g_t per channel from the f rows, k = 1 - g; else one decay per head.  A record: [q P: DP * 16][k P_.15: DP * 16][B: 512][P_15: 2 DP],
+// B and P_15 as high and low parts: a row behind quick decays is little more than its own products, and the state meets the same P_15
+// block after block where a head has one decay.
+//
+// What bounds it: the row-by-row walk reads q, k (and g) of every row for every value column from LDS, 0.38 - 0.42 us a row; here 72 matrix
+// instructions (128 channels) are 1.0 us per sixteen rows, with the LDS reads and sums between them 2.3.  8 sequences of 1024 rows, 16
+// heads of 128 x 128: a decay per head 399 us row by row, 212 so (preparation 68); per channel 458, 253 (109).  rms error against 64
+// bits, row by row = 1 (64 to 1024 rows; D 64, 128, 256): gates around 1/2 0.86 - 0.89, decays of 1 - 2^-5 and slower 0.59 - 0.84,
+// four random decays between 0 and 1 0.94 - 1.06.
+// ---------------------------------------------------------------------------
+constexpr int lin_record_floats(int dp) { return (2 * dp * kB + 512 + 2 * dp + 255) & ~255; }
+
+struct LinearArgs {
+  const float* proj;
+  int64_t ld;
+  int q_off, k_off, v_off;
+  bool q_silu, k_silu, v_silu;
+  const float* decay;     // [H]
+  const float* f_bias;    // [H * D]
+  const float* lower;     // [H * D]
+  const int32_t* cu_q;
+  const int32_t* kv_lens;
+  const int32_t* slot_ids;
+  int n_seqs, H, D, Dv;
+  float* state;
+  float* records;
+  float* out;
+  int64_t ldo;
+};
+
+__device__ __forceinline__ float silu_if(bool on, float z) { return on ? z / (1.f + expf(-z)) : z; }
+
+template <int DT, bool FORGET>
+__global__ __launch_bounds__(256) void linear_prepare_kernel(LinearArgs a) {
+  constexpr int DP = 16 * DT, LD = DP + 4;   // (as blocks_prepare_kernel)
+  __shared__ __attribute__((aligned(16))) float kk[kB][LD], qq[kB][LD], gg[FORGET ? kB : 1][LD];
+  __shared__ float bm[kB][kB + 1], bl[kB][kB + 1], gamma[DP], gamma_low[DP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.y;
+  int s = -1;   // the block's sequence: the last one whose records begin at or before it
+  for (int i0 = 0; i0 < a.n_seqs; i0 += 64) {
+    const int i = i0 + lane;
+    const int found = __popcll(__ballot(i < a.n_seqs && first_record(a.cu_q[min(i, a.n_seqs - 1)], i) <= (int)blockIdx.x));
+    s += found;
+    if (found < 64) break;
+  }
+  s = __builtin_amdgcn_readfirstlane(s);
+  const int r0 = a.cu_q[s] + ((int)blockIdx.x - first_record(a.cu_q[s], s)) * kB, n = min(kB, a.cu_q[s + 1] - r0);
+  if (n <= 0) return;  // (a record that no block uses)
+  // rows beyond the sequence's end and channels beyond D change nothing: q = k = 0, g = 1
+  constexpr int RW = kB / 4, C = DP / 64;
+  float qv[RW][C], kv[RW][C];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {   // (every load first, at clamped places: none waits for another)
+    const float* p = a.proj + (int64_t)(r0 + min(wave * RW + i, n - 1)) * a.ld + h * a.D;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int d = min(lane + 64 * c, a.D - 1);
+      qv[i][c] = p[a.q_off + d];
+      kv[i][c] = p[a.k_off + d];
+    }
+  }
+  const float head_decay = FORGET ? 1.f : a.decay[h];
+  float lo[C], fb[C];
+  if constexpr (FORGET) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int d = h * a.D + min(lane + 64 * c, a.D - 1);
+      lo[c] = a.lower[d], fb[c] = a.f_bias[d];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const int t = wave * RW + i;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const bool ok = t < n && lane + 64 * c < a.D;
+      qq[t][lane + 64 * c] = ok ? silu_if(a.q_silu, qv[i][c]) : 0.f;
+      if constexpr (FORGET) {
+        const float f = lo[c] + (1.f - lo[c]) * sigmoid_f(kv[i][c] + fb[c]);
+        gg[t][lane + 64 * c] = ok ? f : 1.f;
+        kk[t][lane + 64 * c] = ok ? 1.f - f : 0.f;
+      } else {
+        kk[t][lane + 64 * c] = ok ? silu_if(a.k_silu, kv[i][c]) : 0.f;
+      }
+    }
+  }
+  __syncthreads();
+  // ---- B: sixteen lanes per j walk t = 0..15, four channels at a time, with p = k_j P_jt (0 before t = j); one decay per head: with k_j,
+  // and the sum times the decay's power ----
+  {
+    using T = std::conditional_t<FORGET, double, float>;
+    const int j = tid >> 4, c = (tid & 15) * 4;
+    T p[C][4];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const f32x4 k = *reinterpret_cast<const f32x4*>(&kk[j][64 * i + c]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[i][e] = k[e];
+    }
+    double power = 1.;   // of the head's decay, t - j
+#pragma unroll 4
+    for (int t = 0; t < kB; ++t) {
+      T sum[4] = {0, 0, 0, 0};
+      const bool decays = t > j;
+      if (!FORGET && decays) power *= head_decay;
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(&qq[t][64 * i + c]);
+        if constexpr (FORGET) {
+          const f32x4 g = *reinterpret_cast<const f32x4*>(&gg[t][64 * i + c]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) p[i][e] = decays ? p[i][e] * g[e] : p[i][e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += p[i][e] * q[e];
+      }
+      T b = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+      if constexpr (FORGET) {
+#pragma unroll
+        for (int o = 1; o < 16; o *= 2) b += __shfl_xor(b, o);
+      } else {
+        b = xor_sum<8>(xor_sum<4>(xor_sum<2>(xor_sum<1>(b))));
+      }
+      const double bp = t < j ? 0. : FORGET ? (double)b : b * power;
+      if (c == 0) bm[t][j] = (float)bp, bl[t][j] = (float)(bp - (float)bp);
+    }
+  }
+  __syncthreads();
+  // ---- the decayed vectors in place, a thread per channel and direction (products of up to sixteen decays in 64 bits, rounded once: the
+  // walk applies them to what it has summed over all rows) ----
+#pragma unroll
+  for (int i = 0; i < (2 * DP + 255) / 256; ++i) {
+    const int id = tid + 256 * i, d = id < DP ? id : id - DP;
+    if (id >= 2 * DP) break;
+    double p = 1.;
+    if (id < DP) {
+#pragma unroll
+      for (int t = 0; t < kB; ++t) {
+        if (FORGET) p *= gg[FORGET ? t : 0][d];
+        else if (t < n) p *= head_decay;
+        qq[t][d] = (float)(qq[t][d] * p);
+      }
+      gamma[d] = (float)p;
+      gamma_low[d] = (float)(p - gamma[d]);
+    } else {
+#pragma unroll
+      for (int t = kB - 1; t >= 0; --t) {
+        kk[t][d] = (float)(kk[t][d] * p);
+        if (FORGET) p *= gg[FORGET ? t : 0][d];
+        else if (t < n) p *= head_decay;
+      }
+    }
+  }
+  __syncthreads();
+  // ---- the record, 16 bytes a thread: slot (tile m of 16 channels, lane group g, r) ----
+  float* const rec_q = a.records + ((int64_t)blockIdx.x * a.H + h) * lin_record_floats(DP);
+  float* const rec_k = rec_q + DP * kB;
+  float* const rec_b = rec_k + DP * kB;
+  for (int i = tid; i < DT * 64; i += 256) {
+    const int m = i >> 6, kg = (i >> 4) & 3, r = i & 15;
+    *reinterpret_cast<float4*>(rec_q + i * 4) = *reinterpret_cast<const float4*>(&qq[r][16 * m + 4 * kg]);
+    *reinterpret_cast<float4*>(rec_k + i * 4) = float4{kk[4 * kg][16 * m + r], kk[4 * kg + 1][16 * m + r], kk[4 * kg + 2][16 * m + r], kk[4 * kg + 3][16 * m + r]};
+  }
+  if (tid < 64) {
+    const int kg = tid >> 4, r = tid & 15;
+    *reinterpret_cast<float4*>(rec_b + tid * 4) = float4{bm[r][4 * kg], bm[r][4 * kg + 1], bm[r][4 * kg + 2], bm[r][4 * kg + 3]};
+    *reinterpret_cast<float4*>(rec_b + 256 + tid * 4) = float4{bl[r][4 * kg], bl[r][4 * kg + 1], bl[r][4 * kg + 2], bl[r][4 * kg + 3]};
+  }
+  for (int d = tid; d < DP; d += 256) rec_b[512 + d] = gamma[d], rec_b[512 + DP + d] = gamma_low[d];
+}
+
+// grid: (sequences, heads, value columns / 64); a wave takes 16 columns, its S as blocks_walk_kernel's.  Ring of three records by LDS-DMA
+// two blocks ahead (two where three do not fit), with the rows' values behind each.
+template <int DT>
+__global__ __launch_bounds__(256, 1) void linear_walk_kernel(LinearArgs a) {
+  constexpr int DP = 16 * DT, REC = lin_record_floats(DP), PIECES = REC / 256, PP = (PIECES + 3) / 4, IMG = REC * 4 + 4096;
+  constexpr int NST = 3 * IMG <= 163840 ? 3 : 2;
+  __shared__ __attribute__((aligned(1024))) char lds[NST * IMG];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int s = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 64 + wave * 16 + r16;
+  const int r0 = a.cu_q[s], n = a.cu_q[s + 1] - r0;
+  if (n == 0) return;
+  const int nb = (n + kB - 1) / kB;
+  const char* const recs = reinterpret_cast<const char*>(a.records + ((int64_t)first_record(r0, s) * a.H + h) * REC);
+  const int64_t rec_stride = (int64_t)a.H * REC * 4;
+  const float* vp[4];   // the next block's rows 4 kg + r at this lane's column
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    vp[r] = a.proj + (int64_t)(r0 + min(4 * kg + r, n - 1)) * a.ld + a.v_off + (int64_t)h * a.Dv + min(col, a.Dv - 1);
+  // PP + 4 requests, whatever the block (beyond the end: the last one's again; rows beyond the end: the last row's)
+  auto issue = [&](int b, int st) __attribute__((always_inline)) {
+    const int bb = min(b, nb - 1);
+    char* const to = lds + st * IMG;
+#pragma unroll
+    for (int i = 0; i < PP; ++i) {
+      const int p = min(wave * PP + i, PIECES - 1);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(recs + bb * rec_stride + p * 1024 + (uint32_t)(lane * 16)),
+                                       (__attribute__((address_space(3))) void*)(to + p * 1024), 16, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vp[r],
+                                       (__attribute__((address_space(3))) void*)(to + REC * 4 + wave * 1024 + r * 256), 4, 0, 0);
+    const int left = n - 1 - (b + 1) * kB;   // rows behind the next block's first
+    if (left >= kB - 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vp[r] += (int64_t)kB * a.ld;
+    } else if (left >= 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vp[r] += (int64_t)(kB + min(4 * kg + r, left) - (4 * kg + r)) * a.ld;
+    }
+  };
+  // the state: S[m][r] = key channel 16 m + 4 kg + r of this lane's column; in memory four channels of a column together (as the
+  // row-by-row kernel keeps it)
+  const int cb = col / kStateCols, cbs = (a.Dv + kStateCols - 1) / kStateCols, cc = col % kStateCols;
+  const bool has_state = cb < cbs, has_col = col < a.Dv;
+  float* const st = a.state + (((int64_t)a.slot_ids[s] * a.H + h) * cbs + cb) * (DP * kStateCols) + (kg * kStateCols + cc) * 4;
+  f32x4 S[DT];
+#pragma unroll
+  for (int m = 0; m < DT; ++m) {
+    S[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (has_state && a.kv_lens[s] > n) S[m] = *reinterpret_cast<const f32x4*>(st + m * (16 * kStateCols));
+  }
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  float* op = a.out + (int64_t)(r0 + 4 * kg) * a.ldo + (int64_t)h * a.Dv + col;   // (formed beyond the columns, not used there)
+  auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (has_col && b * kB + 4 * kg + r < n) op[r * a.ldo] = o[r];
+    op += (int64_t)kB * a.ldo;
+  };
+#pragma unroll
+  for (int i = 0; i + 1 < NST; ++i) issue(i, i);
+  int cur = 0;
+  for (int b = 0; b < nb; ++b) {
+    // record b has landed (a ring of three: record b + 1's requests may be out); everybody is done with record b - 1: its place is free
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * (PP + 4)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (b > 0) store(b - 1);   // (here, not behind the block: the wait above would have to see them home)
+    issue(b + NST - 1, cur == 0 ? NST - 1 : cur - 1);
+    const char* const img = lds + cur * IMG;
+    cur = cur == NST - 1 ? 0 : cur + 1;
+    const char* const rec_q = img + lane * 16;
+    const char* const rec_k = rec_q + DP * kB * 4;
+    const char* const rec_b = rec_k + DP * kB * 4;
+    const char* const gam = rec_b - lane * 16 + 2048 + kg * 16;   // P_15 of this lane's channels 16 m + 4 kg ..
+    auto vec = [](const char* p) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(p); };
+    f32x4 e[8];   // (eight chains: each is an eighth as long, and so is its rounding)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) e[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 qf[2][2], gf[2][2], gl[2][2], kf[2][2], v, bf = vec(rec_b);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const float*>(img + REC * 4 + wave * 1024 + r * 256 + lane * 4);
+    auto read = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        qf[c & 1][i] = vec(rec_q + (2 * c + i) * 1024);
+        kf[c & 1][i] = vec(rec_k + (2 * c + i) * 1024);
+        gf[c & 1][i] = vec(gam + (2 * c + i) * 64);
+        gl[c & 1][i] = vec(gam + DP * 4 + (2 * c + i) * 64);
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = has_col && b * kB + 4 * kg + r < n ? v[r] : 0.f;
+    if (a.v_silu)   // (silu(0) = 0)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = silu_if(true, v[r]);
+#pragma unroll
+    for (int c = 0; c < DT / 2; ++c) {
+      if (c + 1 < DT / 2) read(c + 1);
+      // a pair of tiles: read with the decayed queries, then decayed and the rows added
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          f32x4& ex = e[4 * i + r];
+          ex = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c & 1][i][r], S[2 * c + i][r], ex, 0, 0, 0);
+        }
+      // (the rows are summed from zero and meet the state once: sixteen roundings of their size, one of the state's)
+      f32x4 rows[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int r = 0; r < 4; ++r)   // (r outside i: a tile's four products wait for each other)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) rows[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c & 1][i][r], v[r], rows[i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[2 * c + i][r] = fmaf(gf[c & 1][i][r], S[2 * c + i][r], fmaf(gl[c & 1][i][r], S[2 * c + i][r], rows[i][r]));
+    }
+    const f32x4 low = vec(rec_b + 1024);
+    f32x4 state4[4], rows4[4];   // (what is left of the sums is added in 64 bits: it rounds once)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) state4[r] = e[r] + e[r + 4];
+    auto add_up = [&](f32x4 b4) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        rows4[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(low[r], b4[r], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        rows4[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[r], b4[r], rows4[r], 0, 0, 0);
+      }
+      f32x4 y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        y[i] = (float)((((double)state4[0][i] + state4[1][i]) + ((double)state4[2][i] + state4[3][i])) +
+                       (((double)rows4[0][i] + rows4[1][i]) + ((double)rows4[2][i] + rows4[3][i])));
+      return y;
+    };
+    o = add_up(v);
+    float zero = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) zero = fmaf(o[r], 0.f, zero);
+    // (the state has what is not finite either way; the whole wave takes the branch)
+    if (__builtin_expect(__any(zero != 0.f), 0)) {   // rows in front of the column's first value that is not finite: see causal()
+      const int first = first_bad(v, kg);
+      f32x4 front;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) front[r] = 4 * kg + r < first ? v[r] : 0.f;
+      const f32x4 y = add_up(front);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = 4 * kg + r < first ? y[r] : o[r];
+    }
+  }
+  store(nb - 1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the requests beyond the end land before the workgroup's LDS is given away)
+  if (!has_state) return;
+#pragma unroll
+  for (int m = 0; m < DT; ++m) *reinterpret_cast<f32x4*>(st + m * (16 * kStateCols)) = S[m];
+}
+
 static int tiles_of(int D) { return D <= 64 ? 4 : D <= 128 ? 8 : D <= 256 ? 16 : 0; }
 
 }  // namespace mi
@@ -425,3 +765,40 @@ extern "C" int mi_channel_delta_blocks(const float* qkv, int64_t ld, int q_off, 
                            : launch(blocks_prepare_kernel<16>, blocks_walk_kernel<16>);
   return rc != MI_OK ? rc : launch_head_norm(out, ldo, gate_pre, ld_gate, norm_w, n_rows, H, Dv, eps, S(stream));
 }
+
+// Where linear attention takes the block form.  us, rows / blocks, a decay per head (per channel), 16 heads of 128 x 128: one sequence of 64 rows
+// 20 / 21 (23 / 23), of 128 38 / 32 (43 / 33), 1024 275 / 185; 8 of 100 49 / 42; 32 of 32 53 / 55 (59 / 62), of 64 109 / 85; 64 rows beside 31
+// single ones 83 / 66; 8 heads: 8 of 100 34 / 35.
+extern "C" int64_t mi_linear_attention_blocks_elems(int n_rows, int n_seqs, int max_rows, int H, int D) {
+  const int dt = tiles_of(D);
+  if (n_rows < 0 || n_seqs < 1 || H < 1 || D < 1 || dt == 0) return -1;
+  if (max_rows < (n_seqs < 16 ? 96 : 48 + n_seqs / 2)) return 0;
+  return ((int64_t)n_rows / kB + n_seqs) * H * lin_record_floats(16 * dt);
+}
+
+namespace mi {
+int launch_linear_blocks(const float* proj, int64_t ld, int q_off, int k_off, int v_off, int q_act, int k_act, int v_act, int decay_kind,
+                         const float* decay, const float* f_bias, const float* lower, float* state, const int32_t* cu_q,
+                         const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows, int H, int D, int Dv, float* workspace,
+                         int64_t ws_elems, float* out, int64_t ldo, hipStream_t st) {
+  const int dt = tiles_of(D);
+  if (dt == 0 || H > 65535 || Dv > 65535 || !aligned16(state)) return MI_EUNSUPPORTED;
+  if (!aligned16(workspace) || ws_elems < ((int64_t)n_rows / kB + n_seqs) * H * lin_record_floats(16 * dt)) return MI_EWORKSPACE;
+  const LinearArgs a{proj, ld, q_off, k_off, v_off, q_act == MI_ACT_SILU, k_act == MI_ACT_SILU, v_act == MI_ACT_SILU, decay, f_bias, lower, cu_q,
+                     kv_lens, slot_ids, n_seqs, H, D, Dv, state, workspace, out, ldo};
+  const dim3 prep(n_rows / kB + n_seqs, H), walk(n_seqs, H, (Dv + 63) / 64);   // (64 columns hold whole blocks of the state's layout)
+  const auto launch = [&](auto prepare, auto walk_kernel) -> int {
+    hipLaunchKernelGGL(prepare, prep, dim3(256), 0, st, a);
+    if (check_launch() != MI_OK) return MI_ELAUNCH;
+    hipLaunchKernelGGL(walk_kernel, walk, dim3(256), 0, st, a);
+    return check_launch();
+  };
+  if (decay_kind == MI_DECAY_FORGET)
+    return dt == 4   ? launch(linear_prepare_kernel<4, true>, linear_walk_kernel<4>)
+           : dt == 8 ? launch(linear_prepare_kernel<8, true>, linear_walk_kernel<8>)
+                     : launch(linear_prepare_kernel<16, true>, linear_walk_kernel<16>);
+  return dt == 4   ? launch(linear_prepare_kernel<4, false>, linear_walk_kernel<4>)
+         : dt == 8 ? launch(linear_prepare_kernel<8, false>, linear_walk_kernel<8>)
+                   : launch(linear_prepare_kernel<16, false>, linear_walk_kernel<16>);
+}
+}  // namespace mi

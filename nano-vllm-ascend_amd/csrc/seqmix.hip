@@ -2609,6 +2609,16 @@ extern "C" int mi_linear_attention(const float* proj, int64_t ld, int q_off, int
                                    float* state, const int32_t* cu_q, const int32_t* kv_lens, const int32_t* slot_ids,
                                    int n_seqs, int n_rows, int H, int D, int Dv, float eps, float* out, int64_t ldo,
                                    mi_stream stream) {
+  return mi_linear_attention_ws(proj, ld, q_off, k_off, v_off, q_act, k_act, v_act, decay_kind, decay, f_bias, lower, gate_pre, ld_gate, norm_w,
+                                norm_groups, state, cu_q, kv_lens, slot_ids, n_seqs, n_rows, H, D, Dv, eps, nullptr, 0, out, ldo, stream);
+}
+
+extern "C" int mi_linear_attention_ws(const float* proj, int64_t ld, int q_off, int k_off, int v_off, int q_act, int k_act, int v_act,
+                                      int decay_kind, const float* decay, const float* f_bias, const float* lower,
+                                      const float* gate_pre, int64_t ld_gate, const float* norm_w, int norm_groups, float* state,
+                                      const int32_t* cu_q, const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows, int H,
+                                      int D, int Dv, float eps, float* workspace, int64_t ws_elems, float* out, int64_t ldo,
+                                      mi_stream stream) {
   if (!proj || !state || !cu_q || !kv_lens || !slot_ids || !out || n_rows < 0 || n_seqs < 1) return MI_EINVAL;
   if (H < 1 || D < 1 || Dv < 1 || ldo < (int64_t)H * Dv) return MI_EINVAL;
   if (decay_kind == MI_DECAY_HEAD ? !decay : decay_kind == MI_DECAY_FORGET ? (!f_bias || !lower) : true) return MI_EINVAL;
@@ -2623,7 +2633,13 @@ extern "C" int mi_linear_attention(const float* proj, int64_t ld, int q_off, int
   hipLaunchKernelGGL((linear_attention_kernel<DR, KIND>), grid, dim3(kLinThreads), 0, S(stream), proj, ld, q_off,    \
                      k_off, v_off, q_act, k_act, v_act, decay, f_bias, lower, state, cu_q, kv_lens, slot_ids, H, D, Dv, \
                      out, ldo)
-  if (decay_kind == MI_DECAY_HEAD) {
+  int rc = MI_EUNSUPPORTED;
+  if (workspace)
+    rc = launch_linear_blocks(proj, ld, q_off, k_off, v_off, q_act, k_act, v_act, decay_kind, decay, f_bias, lower, state, cu_q, kv_lens, slot_ids,
+                              n_seqs, n_rows, H, D, Dv, workspace, ws_elems, out, ldo, S(stream));
+  if (rc != MI_OK && rc != MI_EUNSUPPORTED) return rc;
+  if (rc == MI_OK) {
+  } else if (decay_kind == MI_DECAY_HEAD) {
     if (dr == 64 / kLinLanes) MI_LINATTN(64 / kLinLanes, MI_DECAY_HEAD);
     else if (dr == 128 / kLinLanes) MI_LINATTN(128 / kLinLanes, MI_DECAY_HEAD);
     else MI_LINATTN(256 / kLinLanes, MI_DECAY_HEAD);

@@ -41,4 +41,11 @@ __device__ __forceinline__ int seq_of_row(const int32_t* cu_q, int n_seqs, int r
 int launch_head_norm(float* out, int64_t ldo, const float* gate_pre, int64_t ld_gate, const float* norm_w, int n_rows, int H, int Dv,
                      float eps, hipStream_t st);
 
+// mi_linear_attention's recurrence sixteen rows at a time (delta_blocks.hip): out [rows][H * Dv] before the read-out's norm.  MI_EUNSUPPORTED
+// for what the blocks do not take.
+int launch_linear_blocks(const float* proj, int64_t ld, int q_off, int k_off, int v_off, int q_act, int k_act, int v_act, int decay_kind,
+                         const float* decay, const float* f_bias, const float* lower, float* state, const int32_t* cu_q,
+                         const int32_t* kv_lens, const int32_t* slot_ids, int n_seqs, int n_rows, int H, int D, int Dv, float* workspace,
+                         int64_t ws_elems, float* out, int64_t ldo, hipStream_t st);
+
 }  // namespace mi

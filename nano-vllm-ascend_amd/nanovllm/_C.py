@@ -246,6 +246,9 @@ _SIGNATURES = {
     "mi_linear_attention_state_elems": (c_int64, [c_int, c_int, c_int]),
     "mi_linear_attention": (c_int, [_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _p, _p, _p, _p, c_int64,
                                     _p, c_int, _p, _p, _p, _p, c_int, c_int, c_int, c_int, c_int, c_float, _p, c_int64, _p]),
+    "mi_linear_attention_blocks_elems": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
+    "mi_linear_attention_ws": (c_int, [_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _p, _p, _p, _p, c_int64,
+                                    _p, c_int, _p, _p, _p, _p, c_int, c_int, c_int, c_int, c_int, c_float, _p, c_int64, _p, c_int64, _p]),
     "mi_paged_attention_ext": (c_int, [_p, c_int64, _p, _p, c_int64, c_int, _p, c_int, _p, _p, c_int, c_int, c_int, c_int,
                                        c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _p, _p, _p, c_float, c_int, _p, c_int64,
                                        _p, c_int64, _p, c_int64, _p]),

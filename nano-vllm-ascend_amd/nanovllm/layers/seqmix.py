@@ -479,7 +479,7 @@ class HeadDecayLinearAttention(_LinearAttentionState):
         off = m.offsets
         o = ops.linear_attention(y, off["q"][0], off["k"][0], off["v"][0], (_C.ACT_SILU,) * 3, _C.DECAY_HEAD, self.decay, None,
                                  None, m.cols(y, "g"), self.norm, 1, self.state, ctx.cu_seqlens_q, ctx.kv_lens,
-                                 ctx.state_slots, self.H, self.D, self.Dv, self.eps)
+                                 ctx.state_slots, self.H, self.D, self.Dv, self.eps, max_rows=ctx.max_seqlen_q)
         return ops.gemm_any(o, self.o)
 
 
@@ -502,7 +502,8 @@ class ForgetGateLinearAttention(_LinearAttentionState):
         off = m.offsets
         o = ops.linear_attention(y, off["q"][0], off["f"][0], off["v"][0], (_C.ACT_SILU, _C.ACT_NONE, _C.ACT_NONE),
                                  _C.DECAY_FORGET, None, self.f_bias, self.lower, None, self.norm, self.H, self.state,
-                                 ctx.cu_seqlens_q, ctx.kv_lens, ctx.state_slots, self.H, self.D, self.Dv, self.eps)
+                                 ctx.cu_seqlens_q, ctx.kv_lens, ctx.state_slots, self.H, self.D, self.Dv, self.eps,
+                                 max_rows=ctx.max_seqlen_q)
         return ops.gemm_any(o, self.o)
 
 
@@ -644,7 +645,8 @@ class Retention(nn.Module):
         ops.rotary_store(y, q_off, k_off, v_off, H, H, D, self.rot_dims, _C.ROT_HALVES, self.inv_freq, self.rot_amp, False,
                          self.eps, D ** -0.5, ctx.cu_seqlens_q, ctx.kv_lens)
         ops.linear_attention(y, q_off, k_off, v_off, (_C.ACT_NONE,) * 3, _C.DECAY_HEAD, self.decay, None, None, None, None, H,
-                             self.state[lane], ctx.cu_seqlens_q, ctx.kv_lens, ctx.state_slots, H, D, Dv, self.eps, out=out)
+                             self.state[lane], ctx.cu_seqlens_q, ctx.kv_lens, ctx.state_slots, H, D, Dv, self.eps, out=out,
+                             max_rows=ctx.max_seqlen_q)
         ops.head_norm_gate(out, y[:, g_off:g_off + H * Dv], _C.ACT_SILU, None, H, Dv, self.eps, out_scale)
 
 

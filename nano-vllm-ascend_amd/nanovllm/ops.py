@@ -1607,9 +1607,10 @@ def linear_attention_state_elems(H: int, D: int, Dv: int) -> int:
 
 def linear_attention(proj, q_off: int, k_off: int, v_off: int, acts, decay_kind: int, decay, f_bias, lower, gate_pre, norm_w,
                      norm_groups: int, state, cu_q, kv_lens, slot_ids, H: int, D: int, Dv: int, eps: float,
-                     out=None) -> torch.Tensor:
+                     out=None, max_rows: int = 1) -> torch.Tensor:
     """S <- diag(a) S + k v^T, o = S^T q per head over the step's rows (see mi_linear_attention); acts = the (q, k, v)
-    activations; returns the normed (and gated) read-out [rows, H * Dv]."""
+    activations; returns the normed (and gated) read-out [rows, H * Dv].  max_rows: the most rows that one sequence brings (it only
+    chooses the kernels)."""
     require_gpu(proj, state)
     _f32(proj, decay, f_bias, lower, gate_pre, norm_w, state)
     _i32(cu_q, kv_lens, slot_ids)
@@ -1626,11 +1627,13 @@ def linear_attention(proj, q_off: int, k_off: int, v_off: int, acts, decay_kind:
         out = torch.empty((rows, H * Dv), dtype=_F32, device=proj.device)
     _f32(out)
     assert out.shape[0] == rows and out.shape[1] >= H * Dv   # (a column slice of a wider buffer is fine)
-    check(lib.mi_linear_attention(ptr(proj), proj.stride(0), q_off, k_off, v_off, int(acts[0]), int(acts[1]), int(acts[2]),
-                                  int(decay_kind), ptr(decay), ptr(f_bias), ptr(lower), ptr(gate_pre),
-                                  gate_pre.stride(0) if gate_pre is not None else 0, ptr(norm_w), int(norm_groups),
-                                  ptr(state), ptr(cu_q), ptr(kv_lens), ptr(slot_ids), kv_lens.numel(), rows, H, D, Dv,
-                                  float(eps), ptr(out), out.stride(0), stream()), "mi_linear_attention")
+    n = lib.mi_linear_attention_blocks_elems(rows, kv_lens.numel(), max_rows, H, D)
+    ws = torch.empty(n, dtype=_F32, device=proj.device) if n > 0 else None
+    check(lib.mi_linear_attention_ws(ptr(proj), proj.stride(0), q_off, k_off, v_off, int(acts[0]), int(acts[1]), int(acts[2]),
+                                     int(decay_kind), ptr(decay), ptr(f_bias), ptr(lower), ptr(gate_pre),
+                                     gate_pre.stride(0) if gate_pre is not None else 0, ptr(norm_w), int(norm_groups),
+                                     ptr(state), ptr(cu_q), ptr(kv_lens), ptr(slot_ids), kv_lens.numel(), rows, H, D, Dv,
+                                     float(eps), ptr(ws), max(n, 0), ptr(out), out.stride(0), stream()), "mi_linear_attention_ws")
     return out
 
 
