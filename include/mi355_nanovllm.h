@@ -161,6 +161,20 @@ int mi_paged_attn_decode_fused(const mi_bf16* qkv, int64_t qkv_row_stride,
                                mi_bf16* out, void* workspace, size_t ws_bytes,
                                int batch, int n_q_heads, int n_kv_heads, int head_dim,
                                int block_size, float scale, mi_stream stream);
+/* ... with the order in which the sequences' workgroups start (NULL: by number; used where the units outnumber the CUs): order [batch][2]
+ * from mi_context_order over the same context_lens - {sequence, its context}, the longest first. */
+int mi_paged_attn_decode_fused_ordered(const mi_bf16* qkv, int64_t qkv_row_stride,
+                               const mi_bf16* q_w, const mi_bf16* k_w, float eps,
+                               const int64_t* positions, const float* cos_sin,
+                               const int32_t* slot_2d,
+                               mi_bf16* k_cache, mi_bf16* v_cache,
+                               const int32_t* block_table, int table_stride,
+                               const int32_t* context_lens,
+                               mi_bf16* out, void* workspace, size_t ws_bytes,
+                               int batch, int n_q_heads, int n_kv_heads, int head_dim,
+                               int block_size, float scale, const int32_t* order, mi_stream stream);
+/* n <= 1024; order on 8 bytes. */
+int mi_context_order(const int32_t* context_lens, int n, int32_t* order, mi_stream stream);
 
 /* Instrumented form of mi_paged_attn_decode_fused (tools/attn_timeline.py; n_q_heads / n_kv_heads == 2 only): the same
  * results, and stamps[batch * n_kv_heads * splits][8 waves][8] (uint64, device memory) receives every wave's

@@ -349,35 +349,40 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
     const uint16_t* vc, const int32_t* __restrict__ block_table, int table_stride,
     const int32_t* __restrict__ ctx_lens, float* __restrict__ part_o, float* __restrict__ part_ml,
     uint16_t* __restrict__ out, int n_q_heads, KvStrides kvs, int tpb, int tpb_shift, int resolve_run, float scale_log2e, FusedStep fs,
-    unsigned long long* __restrict__ stamps = nullptr) {
+    const int32_t* __restrict__ order, unsigned long long* __restrict__ stamps = nullptr) {
   static_assert(!FUSE || PIPE, "the fused prologue needs the register room of the 8-wave form");
   static_assert(!FUSE || DB == 4, "the fused step prologue is written for 128-wide heads");
   constexpr int D = 32 * DB;  // head_dim
+  // ORDERED: four waves do the runs of eight, two behind one another, each with sums of its own: the eight-wave form's bits
+  constexpr bool ORDERED = FUSE && WAVES == 4;
+  constexpr int RUNS = ORDERED ? 2 : 1, NR = WAVES * RUNS;  // runs per wave, per workgroup
   unsigned long long ts[8] = {};
 #define MI_STAMP(i)                                        \
   do {                                                     \
     if constexpr (STAMP) ts[i] = __builtin_amdgcn_s_memrealtime(); \
   } while (0)
   MI_STAMP(0);  // entry
-  __shared__ __attribute__((aligned(16))) float sm_o[WAVES][G][D];
-  __shared__ float sm_m[WAVES][16];
-  __shared__ float sm_l[WAVES][16];
+  __shared__ __attribute__((aligned(16))) float sm_o[NR][G][D];
+  __shared__ float sm_m[NR][16];
+  __shared__ float sm_l[NR][16];
   // PIPE: the step's query heads, staged once per workgroup (FUSE: produced by the prologue wave)
   __shared__ __attribute__((aligned(16))) uint16_t sm_q[PIPE ? G : 1][D];
   __shared__ __attribute__((aligned(16))) uint16_t sm_k[FUSE ? 128 : 8], sm_v[FUSE ? 128 : 8];  // the step's new K / V row
 
-  const int split = blockIdx.x, splits = gridDim.x, h = blockIdx.y, b = blockIdx.z;
-  const int ctx = max(ctx_lens[b], 0);
+  const int split = blockIdx.x, splits = gridDim.x, h = blockIdx.y;
+  // order: {sequence, its context} of the z-th workgroups, the long ones first (one scalar load, as the context alone is)
+  const int b = ORDERED ? order[2 * blockIdx.z] : (int)blockIdx.z;
+  const int ctx = max(ORDERED ? order[2 * blockIdx.z + 1] : ctx_lens[b], 0);
   const int n_tiles = (ctx + 15) >> 4;
   // the context is cut into chunks of two 16-token tiles (only the very last chunk may hold one);
   // the chunks are dealt to the WAVES*splits waves as evenly as possible, each wave a contiguous run:
   // run r covers chunks [deal(r), deal(r + 1)), sizes differ by at most one, the longer runs come
   // first (so the last wave of a workgroup - which, when FUSE, also does the step prologue - never has
   // a long one)
-  const int n_chunks = (n_tiles + 1) >> 1, n_waves = WAVES * splits;
+  const int n_chunks = (n_tiles + 1) >> 1, n_waves = NR * splits;
   const int deal_q = n_chunks / n_waves, deal_r = n_chunks % n_waves;
   auto deal = [&](int r) { return r * deal_q + min(r, deal_r); };
-  const int wg_c0 = deal(split * WAVES), wg_c1 = deal((split + 1) * WAVES);
+  const int wg_c0 = deal(split * NR), wg_c1 = deal((split + 1) * NR);
   const int64_t row0 = (int64_t)b * n_q_heads + h * G;  // first q head of this kv head
   if (wg_c0 >= wg_c1) {  // uniform for the workgroup: nothing to attend in this split
     if (splits == 1) {     // empty context (graph padding row): the output row is zero
@@ -395,8 +400,9 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, n = lane & 15;
   const int32_t* table_row = block_table + (int64_t)b * table_stride;
-  const int vw = split * WAVES + wave;
-  const int t0 = 2 * deal(vw), t1 = min(n_tiles, 2 * deal(vw + 1));
+  const int vw = split * NR + wave * RUNS;
+  const int t0 = 2 * deal(vw), t1 = min(n_tiles, 2 * deal(vw + RUNS));
+  const int t_mid = min(n_tiles, 2 * deal(vw + 1));  // (RUNS = 2: the second run's first tile)
   if constexpr (STAMP) asm volatile("" ::"s"(t0), "s"(t1));  // the context length has arrived
   MI_STAMP(1);
 
@@ -432,6 +438,30 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
   f32x4 acc[2 * DB];
 #pragma unroll
   for (int j = 0; j < 2 * DB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto leave = [&](int run) __attribute__((always_inline)) {  // a run's sums, for the merge
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (n < G) {
+#pragma unroll
+      for (int j = 0; j < 2 * DB; ++j) *reinterpret_cast<f32x4*>(&sm_o[run][n][j * 16 + 4 * g]) = acc[j];
+      if (g == 0) {
+        sm_m[run][n] = m;
+        sm_l[run][n] = l;
+      }
+    }
+  };
+  auto first_run_ends = [&](int t) __attribute__((always_inline)) {  // behind the chunk of tile t
+    if constexpr (RUNS == 2) {
+      if (t < t_mid && t + 2 >= t_mid) {
+        leave(wave * RUNS);
+        m = -INFINITY, l = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2 * DB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  if (RUNS == 2 && t0 >= t_mid) leave(wave * RUNS);  // (an empty run; the second one is empty too)
 
   // a single-tile chunk loads its tile twice (a cache hit) and masks the duplicate through the limit
   auto second = [&](int t) { return t + 1 < t1 ? t + 1 : t; };
@@ -500,6 +530,7 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
         }
       }
       attend_chunk<true, DB>(AK0, AK1, AV0, AV1, Q, ta * 16, limit_of(ta), limit_of(ta), scale_log2e, g, m, l, acc);
+      first_run_ends(ta);
     };
     auto attend_b = [&]() __attribute__((always_inline)) {
       if constexpr (FUSE) {
@@ -509,6 +540,7 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
         }
       }
       attend_chunk<true, DB>(BK0, BK1, BV0, BV1, Q, tb * 16, limit_of(tb), limit_of(tb), scale_log2e, g, m, l, acc);
+      first_run_ends(tb);
     };
     if (tb < t1) {  // at least two chunks
       load_a();
@@ -575,17 +607,7 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
   }
   if constexpr (STAMP) asm volatile("" ::"v"(acc[0]), "v"(acc[2 * DB - 1]));
   MI_STAMP(5);  // this wave's run is attended
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-
-  if (n < G) {
-#pragma unroll
-    for (int j = 0; j < 2 * DB; ++j) *reinterpret_cast<f32x4*>(&sm_o[wave][n][j * 16 + 4 * g]) = acc[j];
-    if (g == 0) {
-      sm_m[wave][n] = m;
-      sm_l[wave][n] = l;
-    }
-  }
+  leave(wave * RUNS + RUNS - 1);
   __syncthreads();
   MI_STAMP(6);  // every wave of the workgroup has arrived
   // merge the waves (at least one of them had a chunk, so M is finite; empty ones weigh exp2(-inf) = 0)
@@ -593,10 +615,10 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attn_decode_kernel(
     const int hn = idx / D, d = idx % D;  // (D is a power of two: shifts)
     float M = sm_m[0][hn];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, sm_m[w][hn]);
+    for (int w = 1; w < NR; ++w) M = fmaxf(M, sm_m[w][hn]);
     float o = 0.f, L = 0.f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
+    for (int w = 0; w < NR; ++w) {
       const float e = exp2f(sm_m[w][hn] - M);
       o += e * sm_o[w][hn][d];
       L += e * sm_l[w][hn];
@@ -1104,6 +1126,22 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
   }
 }
 
+// a thread per sequence counts those in front of it
+__global__ __launch_bounds__(1024) void context_order_kernel(const int32_t* __restrict__ lens, int n, int32_t* __restrict__ order) {
+  __shared__ __attribute__((aligned(16))) int len[1024];
+  const int i = threadIdx.x, own = i < n ? lens[i] : -2147483647 - 1;   // (beyond n: behind everything)
+  len[i] = own;
+  __syncthreads();
+  if (i >= n) return;
+  int rank = 0;
+  for (int j = 0; j < (int)blockDim.x; j += 4) {
+    const int4 v = *reinterpret_cast<const int4*>(len + j);
+    rank += (v.x > own || (v.x == own && j < i)) + (v.y > own || (v.y == own && j + 1 < i)) + (v.z > own || (v.z == own && j + 2 < i)) +
+            (v.w > own || (v.w == own && j + 3 < i));
+  }
+  *reinterpret_cast<int2*>(order + 2 * rank) = int2{i, own};
+}
+
 // waves per workgroup: as many as the LDS merge buffer (WAVES * G * 512 B) and the register file allow
 static int decode_waves(int G) { return G <= 4 ? 16 : (G <= 8 ? 8 : 4); }
 
@@ -1143,7 +1181,8 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
                        const int32_t* block_table, int table_stride, const int32_t* context_lens, mi_bf16* out,
                        void* workspace, size_t ws_bytes, int batch, int n_q_heads, int n_kv_heads, int head_dim,
                        int block_size, float scale, int num_splits, KvStrides kvs, mi_stream stream,
-                       const FusedStep* fused = nullptr, unsigned long long* stamps = nullptr, bool merge = true) {
+                       const FusedStep* fused = nullptr, unsigned long long* stamps = nullptr, bool merge = true,
+                       const int32_t* order = nullptr) {
   int rc = check_attn_common(q, k_cache, v_cache, block_table, n_q_heads, n_kv_heads, head_dim, block_size,
                              q_row_stride);
   if (rc != MI_OK) return rc;
@@ -1160,6 +1199,12 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
   int nsplit = num_splits > 0 ? num_splits : decode_splits(batch, n_kv_heads, pipe ? 16 : waves);
   if (nsplit > 16) nsplit = 16;
   if (!merge && nsplit == 1) return MI_EUNSUPPORTED;
+  // More (sequence, kv head) units than CUs: four-wave workgroups, two per CU - one streams while the other starts, merges or stores, which
+  // an eight-wave workgroup has the CU to itself for - and the long contexts first, as the launch ends with its last unit's.  Needs the
+  // order, which the caller makes once per step.  16 / 8 heads, us per launch: 200 sequences of 100 - 1024 keys 89.7 -> 83.7, 64 of
+  // 512 - 1100 40.6 -> 39.7; per step of 28 layers: 200 of 30 - 200 2280 -> 2000, 200 of 500 3654 -> 3406, 36 of 500 1454 -> 1355, 128 of 900
+  // 3542 -> 3514, 100 of 50 - 2000 3340 -> 3243 (by number 3505).
+  if (!fused || nsplit > 1 || (int64_t)batch * n_kv_heads <= 256) order = nullptr;
   float* part_o = static_cast<float*>(workspace);
   float* part_ml = part_o + (size_t)batch * n_q_heads * 16 * 128;
   const float sl2 = scale * 1.4426950408889634f;
@@ -1178,16 +1223,17 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
 #define LAUNCH_DEC_AS(GG, WW, FF, PP, DD)                                                                            \
   hipLaunchKernelGGL((paged_attn_decode_kernel<GG, WW, FF, PP, false, DD>), grid, dim3(WW * 64), 0, st, q,            \
                      q_row_stride, k_cache, v_cache, block_table, table_stride, context_lens, part_o, part_ml, out, \
-                     n_q_heads, kvs, block_size / 16, tpb_shift, resolve_run, sl2, fs)
+                     n_q_heads, kvs, block_size / 16, tpb_shift, resolve_run, sl2, fs, order)
 #define LAUNCH_DEC(GG, WW)                              \
-  if (fused) LAUNCH_DEC_AS(GG, 8, true, true, 4);       \
+  if (order) LAUNCH_DEC_AS(GG, 4, true, true, 4);       \
+  else if (fused) LAUNCH_DEC_AS(GG, 8, true, true, 4);  \
   else if (pipe) LAUNCH_DEC_AS(GG, 8, false, true, 4);  \
   else LAUNCH_DEC_AS(GG, WW, false, false, 4)
   if (stamps != nullptr) {  // the instrumented kernel: the bench model's geometry only
     if (!fused || G != 2) return MI_EUNSUPPORTED;
     hipLaunchKernelGGL((paged_attn_decode_kernel<2, 8, true, true, true>), grid, dim3(8 * 64), 0, st, q, q_row_stride,
                        k_cache, v_cache, block_table, table_stride, context_lens, part_o, part_ml, out, n_q_heads, kvs,
-                       block_size / 16, tpb_shift, resolve_run, sl2, fs, stamps);
+                       block_size / 16, tpb_shift, resolve_run, sl2, fs, nullptr, stamps);
     rc = check_launch();
     if (rc != MI_OK || nsplit == 1) return rc;
     hipLaunchKernelGGL(paged_attn_merge_kernel<128>, dim3((batch * n_q_heads + 3) / 4), dim3(256), 0, st, part_o, part_ml,
@@ -1237,6 +1283,23 @@ extern "C" int mi_paged_attn_decode(const mi_bf16* q, int64_t q_row_stride, cons
                      default_strides(n_kv_heads, block_size > 0 ? block_size / 16 : 1, 16 * head_dim), stream);
 }
 
+extern "C" int mi_paged_attn_decode_fused_ordered(const mi_bf16* qkv, int64_t qkv_row_stride, const mi_bf16* q_w,
+                                          const mi_bf16* k_w, float eps, const int64_t* positions,
+                                          const float* cos_sin, const int32_t* slot_2d, mi_bf16* k_cache,
+                                          mi_bf16* v_cache, const int32_t* block_table, int table_stride,
+                                          const int32_t* context_lens, mi_bf16* out, void* workspace,
+                                          size_t ws_bytes, int batch, int n_q_heads, int n_kv_heads, int head_dim,
+                                          int block_size, float scale, const int32_t* order, mi_stream stream) {
+  if (!positions || !cos_sin || !slot_2d) return MI_EINVAL;
+  if ((q_w == nullptr) != (k_w == nullptr)) return MI_EINVAL;
+  if (!aligned16(cos_sin) || (q_w && (!aligned16(q_w) || !aligned16(k_w)))) return MI_EINVAL;
+  const FusedStep fs{q_w, k_w, positions, cos_sin, slot_2d, eps};
+  return decode_impl(qkv, qkv_row_stride, k_cache, v_cache, block_table, table_stride, context_lens, out,
+                     workspace, ws_bytes, batch, n_q_heads, n_kv_heads, head_dim, block_size, scale, 0,
+                     default_strides(n_kv_heads, block_size > 0 ? block_size / 16 : 1), stream, &fs,
+                     nullptr, true, order);
+}
+
 extern "C" int mi_paged_attn_decode_fused(const mi_bf16* qkv, int64_t qkv_row_stride, const mi_bf16* q_w,
                                           const mi_bf16* k_w, float eps, const int64_t* positions,
                                           const float* cos_sin, const int32_t* slot_2d, mi_bf16* k_cache,
@@ -1244,13 +1307,18 @@ extern "C" int mi_paged_attn_decode_fused(const mi_bf16* qkv, int64_t qkv_row_st
                                           const int32_t* context_lens, mi_bf16* out, void* workspace,
                                           size_t ws_bytes, int batch, int n_q_heads, int n_kv_heads, int head_dim,
                                           int block_size, float scale, mi_stream stream) {
-  if (!positions || !cos_sin || !slot_2d) return MI_EINVAL;
-  if ((q_w == nullptr) != (k_w == nullptr)) return MI_EINVAL;
-  if (!aligned16(cos_sin) || (q_w && (!aligned16(q_w) || !aligned16(k_w)))) return MI_EINVAL;
-  const FusedStep fs{q_w, k_w, positions, cos_sin, slot_2d, eps};
-  return decode_impl(qkv, qkv_row_stride, k_cache, v_cache, block_table, table_stride, context_lens, out,
-                     workspace, ws_bytes, batch, n_q_heads, n_kv_heads, head_dim, block_size, scale, 0,
-                     default_strides(n_kv_heads, block_size > 0 ? block_size / 16 : 1), stream, &fs);
+  return mi_paged_attn_decode_fused_ordered(qkv, qkv_row_stride, q_w, k_w, eps, positions, cos_sin, slot_2d, k_cache, v_cache, block_table,
+                                            table_stride, context_lens, out, workspace, ws_bytes, batch, n_q_heads, n_kv_heads, head_dim, block_size, scale,
+                                            nullptr, stream);
+}
+
+// {sequence, its context} of n <= 1024 sequences in order of falling context (ties: by number)
+extern "C" int mi_context_order(const int32_t* context_lens, int n, int32_t* order, mi_stream stream) {
+  if (!context_lens || !order || n < 0 || (reinterpret_cast<uintptr_t>(order) & 7u)) return MI_EINVAL;
+  if (n > 1024) return MI_EUNSUPPORTED;
+  if (n == 0) return MI_OK;
+  hipLaunchKernelGGL(context_order_kernel, dim3(1), dim3((n + 63) / 64 * 64), 0, S(stream), context_lens, n, order);
+  return check_launch();
 }
 
 // the same without the merge of a split context: the splits' sums stay in `workspace` (mi_gemm_merge_few_splitk)

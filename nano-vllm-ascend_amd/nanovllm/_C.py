@@ -75,6 +75,12 @@ _SIGNATURES = {
         [_p, c_int64, _p, _p, c_float, _p, _p, _p, _p, _p, _p, c_int, _p, _p, _p, c_size_t, c_int, c_int, c_int,
          c_int, c_int, c_float, _p],
     ),
+    "mi_paged_attn_decode_fused_ordered": (
+        c_int,
+        [_p, c_int64, _p, _p, c_float, _p, _p, _p, _p, _p, _p, c_int, _p, _p, _p, c_size_t, c_int, c_int, c_int,
+         c_int, c_int, c_float, _p, _p],
+    ),
+    "mi_context_order": (c_int, [_p, c_int, _p, _p]),
     "mi_paged_attn_decode_fused_ex": (
         c_int,
         [_p, c_int64, _p, _p, c_float, _p, _p, _p, _p, _p, _p, c_int, _p, _p, _p, c_size_t, c_int, c_int, c_int,

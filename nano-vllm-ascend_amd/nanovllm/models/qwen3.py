@@ -327,6 +327,7 @@ class Qwen3Model(nn.Module):
         l0 = self.layers[0]
         rows4 = tp > 1 and l0.self_attn.o_proj.weight_rows4 is not None
         fuse_attn = not ctx.is_prefill and os.environ.get("MI355_ATTN_FUSED", "1") != "0"
+        order = ops.context_order(ctx.context_lens, l0.self_attn.num_kv_heads) if fuse_attn and l0.self_attn.attn.fusable else None
 
         xgmi = get_xgmi_comm() if tp > 1 else None
         fused_seam = (xgmi is not None and xgmi.fits_rows(rows, h.shape[1])
@@ -351,7 +352,7 @@ class Qwen3Model(nn.Module):
             return ops.paged_attn_decode_fused(qkv, qw, kw, attn.rms_norm_eps, positions, rope.cos_sin_cache,
                                                ctx.slot_mapping, a.k_cache, a.v_cache, ctx.block_tables,
                                                ctx.context_lens, attn.num_heads, attn.num_kv_heads, ctx.block_size,
-                                               a.scale)
+                                               a.scale, order=order)
 
         def row_parallel(x, lin):
             """-> (tensor, is_partials): bf16 rows, or fp32 split-K partials for add_rmsnorm_splitk"""

@@ -106,11 +106,25 @@ def paged_attn_decode(q, k_cache, v_cache, block_tables, context_lens, n_q_heads
     return out
 
 
+def context_order(context_lens, n_kv_heads: int):
+    """What paged_attn_decode_fused takes as `order` in every layer of a decode step over these context lengths: {sequence, its context} with
+    the longest first [n, 2] - or None where it makes no difference (no more (sequence, kv head) units than the chip has CUs)."""
+    n = context_lens.numel()
+    if n * n_kv_heads <= 256 or n > 1024:
+        return None
+    require_gpu(context_lens)
+    assert context_lens.dtype == torch.int32 and context_lens.is_contiguous()
+    order = torch.empty((n, 2), dtype=torch.int32, device=context_lens.device)
+    check(lib.mi_context_order(ptr(context_lens), n, ptr(order), stream()), "mi_context_order")
+    return order
+
+
 def paged_attn_decode_fused(qkv, q_w, k_w, eps: float, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables,
                             context_lens, n_q_heads: int, n_kv_heads: int, block_size: int, scale: float,
-                            out=None, workspace=None) -> torch.Tensor:
+                            out=None, workspace=None, order=None) -> torch.Tensor:
     """q/k-norm + RoPE + KV store of the step's token + paged decode attention in ONE launch, straight
-    from the packed qkv rows (bit-identical to qknorm_rope_store followed by paged_attn_decode)."""
+    from the packed qkv rows (bit-identical to qknorm_rope_store followed by paged_attn_decode, with order =
+    context_order(context_lens) too)."""
     require_gpu(qkv, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables, context_lens)
     _bf16(qkv, k_cache, v_cache, q_w, k_w)
     batch = qkv.shape[0]
@@ -120,17 +134,18 @@ def paged_attn_decode_fused(qkv, q_w, k_w, eps: float, positions, cos_sin, slots
     assert slots_2d.dtype == torch.int32 and slots_2d.is_contiguous() and slots_2d.shape == (batch, 2)
     assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
     assert context_lens.dtype == torch.int32 and context_lens.is_contiguous()
+    assert order is None or (order.dtype == torch.int32 and order.is_contiguous() and order.shape == (batch, 2))
     if out is None:
         out = torch.empty((batch, n_q_heads * HEAD_DIM), dtype=_BF16, device=qkv.device)
     if workspace is None:
         workspace = attn_workspace(qkv.device, batch, n_q_heads)
     check(
-        lib.mi_paged_attn_decode_fused(ptr(qkv), qkv.stride(0), ptr(q_w), ptr(k_w), float(eps), ptr(positions),
+        lib.mi_paged_attn_decode_fused_ordered(ptr(qkv), qkv.stride(0), ptr(q_w), ptr(k_w), float(eps), ptr(positions),
                                        ptr(cos_sin), ptr(slots_2d), ptr(k_cache), ptr(v_cache), ptr(block_tables),
                                        block_tables.stride(0), ptr(context_lens), ptr(out), ptr(workspace),
                                        workspace.numel() * workspace.element_size(), batch, n_q_heads, n_kv_heads,
-                                       HEAD_DIM, block_size, float(scale), stream()),
-        "mi_paged_attn_decode_fused",
+                                       HEAD_DIM, block_size, float(scale), ptr(order), stream()),
+        "mi_paged_attn_decode_fused_ordered",
     )
     return out
 
