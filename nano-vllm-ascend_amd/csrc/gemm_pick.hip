@@ -119,7 +119,7 @@ extern "C" int mi_logits_pick(const mi_bf16* logits, int M, int N, const float* 
 // head GEMM with the pick epilogue: the same workgroup geometry as mi_gemm_bf16_packed for this (M, N)
 extern "C" int mi_gemm_pick_groups(int M, int N, int K, int fp8_weights) {
   if (M <= 0 || N <= 0 || N % 16) return 0;
-  if (!fp8_weights && head_stream_fits(M, N, K)) return head_stream_grid(M);
+  if (fp8_weights ? head_stream_fp8_fits(M, N, K) : head_stream_fits(M, N, K)) return head_stream_grid(M);
   return pick_two_tiles(M, N) ? N / 32 : N / 16;
 }
 
@@ -163,6 +163,10 @@ extern "C" int mi_gemm_fp8w_packed_pick(const mi_bf16* x, const uint8_t* w_packe
   GemmArgs a{x, reinterpret_cast<const uint16_t*>(w_packed), nullptr, y, nullptr, M, N, K, 1, S(stream)};
   a.scale = scale;
   a.pick = PickArgs{temperatures, rng, static_cast<uint2*>(candidates), 0};
+  if (head_stream_fp8_fits(M, N, K)) {
+    launch_head_stream<true, 2>(x, a.w, y, M, N, K, a.pick, S(stream), scale);
+    return check_launch();
+  }
   return pick_two_tiles(M, N) ? pick_mt<2, 2, EPI_PICK>(a) : pick_mt<1, 2, EPI_PICK>(a);
 }
 

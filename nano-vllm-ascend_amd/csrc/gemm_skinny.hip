@@ -169,6 +169,10 @@ extern "C" int mi_gemm_fp8w_packed(const mi_bf16* x, const uint8_t* w_packed, co
   GemmArgs a{x, reinterpret_cast<const uint16_t*>(w_packed), nullptr, y, nullptr, M, N, K, 1, S(stream)};
   a.scale = scale;
   if (epilogue == 1) return pick_mt<2, 2, EPI_SILU>(a);
+  if (head_stream_fp8_fits(M, N, K)) {  // as mi_gemm_fp8w_packed_pick: the same logits
+    launch_head_stream<false, 2>(x, a.w, y, M, N, K, PickArgs{nullptr, nullptr, nullptr, 0}, S(stream), scale);
+    return check_launch();
+  }
   if (N / 16 >= 1024 && (N / 16) % 2 == 0 && M <= 32) return pick_mt<2, 2, EPI_NONE>(a);
   return pick_mt<1, 2, EPI_NONE>(a);
 }

@@ -515,11 +515,12 @@ static __global__ __launch_bounds__(256) void pack_weight_kernel(const uint16_t*
 // PICK keep each row's best sampling key in registers - while the others already fetch the next group.
 // Summation order: one MFMA chain per wave over its slice, then the waves in order (deterministic).
 // ---------------------------------------------------------------------------------------------------
-template <int MT, int RT, int WAVES, int STEPS, bool PICK>
+template <int MT, int RT, int WAVES, int STEPS, bool PICK, int WF = 1>
 __global__ __launch_bounds__(WAVES * 64) void head_stream_kernel(const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ w,
-                                                                 uint16_t* __restrict__ y, int M, int N, int K,
-                                                                 int n_groups, PickArgs pk) {
+                                                                 uint16_t* __restrict__ y, int M_all, int N, int K,
+                                                                 int n_groups, PickArgs pk,
+                                                                 const float* __restrict__ scale = nullptr) {
   static_assert(RT * MT * 64 <= WAVES * 64, "one epilogue item per thread");
   __shared__ __attribute__((aligned(16))) float red[2][WAVES][RT * MT][64][4];
   __shared__ float pick_key[PICK ? MT * 16 : 1][RT * 4];
@@ -528,6 +529,8 @@ __global__ __launch_bounds__(WAVES * 64) void head_stream_kernel(const uint16_t*
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
   const int ktiles = K >> 5, kbeg = wave * 32 * STEPS;
+  const int m0 = WF == 2 ? (int)blockIdx.y * kSkinnyRows : 0, M = WF == 2 ? min(M_all - m0, kSkinnyRows) : M_all;
+  if constexpr (WF == 2) x += (int64_t)m0 * K, y += (int64_t)m0 * N;
 
   // this wave's x slice as B fragments: lane (g, c) <- x[16 m + c][kbeg + 32 s + 8 g .. +8]; rows >= M are
   // clamped to row M - 1 (MFMA output columns are independent, the duplicates are never stored)
@@ -549,24 +552,49 @@ __global__ __launch_bounds__(WAVES * 64) void head_stream_kernel(const uint16_t*
   bool noisy = false;
   uint64_t rkey = 0;
   if (PICK && has_item && erow < M) {
-    const float tmp = pk.temperatures ? pk.temperatures[erow] : 0.f;
+    const float tmp = pk.temperatures ? pk.temperatures[m0 + erow] : 0.f;
     noisy = tmp > 0.f;
     inv_t = noisy ? 1.0f / tmp : 1.0f;
-    rkey = sample_row_key(pk.rng[0], pk.rng[1], erow);
+    rkey = sample_row_key(pk.rng[0], pk.rng[1], m0 + erow);
   }
 
   const int first = (int)((int64_t)blockIdx.x * n_groups / gridDim.x);
   const int last = (int)((int64_t)(blockIdx.x + 1) * n_groups / gridDim.x);
   int par = 0;
-  for (int grp = first; grp < last; ++grp, par ^= 1) {
-    // (fetching the next group's fragments before this group's barrier measured slower: 62.3 vs 59.0 us)
-    u32x4 a[RT][STEPS];
+  // WF = 2: half the bytes per group, so two groups' requests are out (a lane's 16 bytes: two k-steps, as gemm_skinny_kernel)
+  u32x4 raw[WF == 2 ? RT : 1][WF == 2 ? STEPS / 2 : 1];
+  auto request = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s)
-        a[t][s] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-            w + ((int64_t)(grp * RT + t) * ktiles + (kbeg >> 5) + s) * 512 + lane * 8));
+      for (int s = 0; s < STEPS / 2; ++s)
+        raw[WF == 2 ? t : 0][WF == 2 ? s : 0] = __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4*>(w + ((int64_t)(grp * RT + t) * (K >> 6) + (kbeg >> 6) + s) * 512 + lane * 8));
+  };
+  if (WF == 2 && first < last) request(first);
+  for (int grp = first; grp < last; ++grp, par ^= 1) {
+    // (bf16: fetching the next group's fragments before this group's barrier measured slower: 62.3 vs 59.0 us)
+    u32x4 a[RT][STEPS];
+    if constexpr (WF == 2) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+          const uint32_t lo = raw[t][s >> 1][2 * (s & 1)], hi = raw[t][s >> 1][2 * (s & 1) + 1];
+          const auto f0 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), f1 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, true);
+          const auto f2 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, false), f3 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, true);
+          a[t][s] = u32x4{pack_bf(f0[0], f0[1]), pack_bf(f1[0], f1[1]), pack_bf(f2[0], f2[1]), pack_bf(f3[0], f3[1])};
+        }
+      request(min(grp + 1, last - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+          a[t][s] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+              w + ((int64_t)(grp * RT + t) * ktiles + (kbeg >> 5) + s) * 512 + lane * 8));
+    }
     f32x4 acc[RT][MT];
 #pragma unroll
     for (int t = 0; t < RT; ++t)
@@ -591,6 +619,7 @@ __global__ __launch_bounds__(WAVES * 64) void head_stream_kernel(const uint16_t*
 #pragma unroll
       for (int wv = 1; wv < WAVES; ++wv) sum += *reinterpret_cast<const f32x4*>(&red[par][wv][et * MT + em][el][0]);
       const int col = (grp * RT + et) * 16 + 4 * (el >> 4);
+      if constexpr (WF == 2) sum *= *reinterpret_cast<const f32x4*>(scale + col);  // per weight row
       u32x2 o;
       o[0] = pack_bf(sum[0], sum[1]);
       o[1] = pack_bf(sum[2], sum[3]);
@@ -627,7 +656,7 @@ __global__ __launch_bounds__(WAVES * 64) void head_stream_kernel(const uint16_t*
           c2 = c3;
         }
       }
-      pk.cand[(int64_t)row * gridDim.x + blockIdx.x] = uint2{__float_as_uint(b2), (uint32_t)c2};
+      pk.cand[(int64_t)(m0 + row) * gridDim.x + blockIdx.x] = uint2{__float_as_uint(b2), (uint32_t)c2};
     }
   }
 }
@@ -646,16 +675,23 @@ static bool head_stream_fits(int M, int N, int K) {
 constexpr int kHeadStreamGrid = 1024;
 static int head_stream_grid(int M) { return M <= 32 ? kHeadStreamGrid : kHeadStreamGrid / 2; }
 
-template <bool PICK>
+// fp8 weights, more than 64 rows in chunks of 64, each a pass over the weights.  us at 151936 x 1024, pick, gemm_skinny_kernel's workgroups
+// (which fetch all of x again for every 16 or 32 KiB of weights) / these: 16 rows 39.9 / 39.4 (without pick 31.0 / 32.6), 32 rows 51 / 46, 64 rows
+// 105 / 55, 65 rows 176 / 93, 200 rows 356 / 181; 896 deep: 32 rows 44 / 41 (35.8 / 37.0), 48 rows 80 / 46; 2048 deep: 32 rows 83 / 83.
+static bool head_stream_fp8_fits(int M, int N, int K) {
+  return (K == 1024 && M > 16 && head_stream_fits(32, N, K)) || (K == 896 && M > 32 && head_stream_fits(M, N, K));
+}
+
+template <bool PICK, int WF = 1>
 static void launch_head_stream(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int K, PickArgs pk,
-                               hipStream_t st) {
-  const int grid = head_stream_grid(M);
-#define MI_HEAD_LAUNCH(MT, WAVES, STEPS)                                                                          \
-  hipLaunchKernelGGL((head_stream_kernel<MT, 2, WAVES, STEPS, PICK>), dim3(grid), dim3(WAVES * 64), 0, st, x, w, y, \
-                     M, N, K, N / 32, pk)
-  const int mt = (M + 15) / 16;
+                               hipStream_t st, const float* scale = nullptr) {
+  const dim3 grid(head_stream_grid(M), WF == 2 ? (M + kSkinnyRows - 1) / kSkinnyRows : 1);
+#define MI_HEAD_LAUNCH(MT, WAVES, STEPS)                                                                         \
+  hipLaunchKernelGGL((head_stream_kernel<MT, 2, WAVES, STEPS, PICK, WF>), grid, dim3(WAVES * 64), 0, st, x, w, y, \
+                     M, N, K, N / 32, pk, scale)
+  const int mt = (min(M, kSkinnyRows) + 15) / 16;
   if (K == 1024) {
-    if (mt == 1) MI_HEAD_LAUNCH(1, 8, 4);
+    if (WF == 1 && mt == 1) MI_HEAD_LAUNCH(1, 8, 4);
     else if (mt == 2) MI_HEAD_LAUNCH(2, 8, 4);
     else if (mt == 3) MI_HEAD_LAUNCH(3, 8, 4);
     else MI_HEAD_LAUNCH(4, 8, 4);
@@ -663,7 +699,7 @@ static void launch_head_stream(const uint16_t* x, const uint16_t* w, uint16_t* y
     if (mt == 1) MI_HEAD_LAUNCH(1, 7, 4);
     else if (mt == 2) MI_HEAD_LAUNCH(2, 7, 4);
     else MI_HEAD_LAUNCH(3, 7, 4);
-  } else {  // 2048
+  } else if constexpr (WF == 1) {  // 2048
     if (mt == 1) MI_HEAD_LAUNCH(1, 8, 8);
     else MI_HEAD_LAUNCH(2, 8, 8);
   }
