@@ -28,6 +28,8 @@
 // on M, on the row's place in the batch or on the tile it falls into (each kernel has ONE fixed order), so the same
 // token gives the same bits whatever it is batched with, within one kernel; between kernels (a row computed in a
 // prompt's portion vs alone) results differ by rounding only.
+#include <algorithm>
+
 #include "gemm_any_stream.hpp"
 
 namespace mi {
@@ -63,6 +65,7 @@ struct GemmAnyArgs {
   // several projections of one input, each with an activation of its own, as one product
   bool ext;
   int act_from, act2, act2_from;
+  int n_groups;  // gemm_any_f32_kernel's grouped form
 };
 
 template <typename TW>
@@ -236,7 +239,33 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
 // Rows beyond the group's end and features beyond N are read from the last valid one and not stored.
 // Needs K % 32 == 0, 16-byte aligned rows of x and w; anything else: gemm_any_fma_kernel.
 // Measured against gemm_any_fma_kernel (64 x 64 tiles, element-wise loads, plain FMA chains), us: see launch_exact.
-template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT>
+// The tile-th row tile of BM rows over all groups (group by group): its group and rows, or false beyond the last.  Every wave for itself.
+template <int BM>
+__device__ __forceinline__ bool group_tile(const int32_t* __restrict__ offsets, int groups, int tile, int& g, int& m0, int& m_hi) {
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < groups; base += 64) {
+    const int i = min(base + lane, groups - 1), lo = offsets[i], hi = offsets[i + 1];
+    const int mine = base + lane < groups ? (max(hi - lo, 0) + BM - 1) / BM : 0;
+    int upto = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+      const int v = __shfl_up(upto, o);
+      upto += lane >= o ? v : 0;
+    }
+    const uint64_t behind = __ballot(upto > tile);
+    if (behind) {
+      const int l = __builtin_ctzll(behind);
+      g = base + l;
+      m0 = __builtin_amdgcn_readlane(lo, l) + (tile - (__builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(mine, l))) * BM;
+      m_hi = __builtin_amdgcn_readlane(hi, l);
+      return true;
+    }
+    tile -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return false;
+}
+
+template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT, bool GROUPED>
 __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
   constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN, BK = 32, NST = 4, ND = DUAL ? 2 : 1;
   constexpr bool WF = sizeof(TW) == 4;
@@ -247,115 +276,131 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int m_lo, m_hi;
-  const TW *w, *w2;
-  select_group<TW, DUAL>(a, w, w2, m_lo, m_hi);
-  const int m0 = m_lo + blockIdx.y * BM;
-  if (m0 >= m_hi) return;
-  const int n0 = blockIdx.x * BN;
-  const char* src[PP];
-  int dst[PP];
-#pragma unroll
-  for (int i = 0; i < PP; ++i) {
-    const int p = min(wave * PP + i, PIECES - 1);
-    dst[i] = p * 1024;
-    if (p < XB / 1024) {
-      const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-      const int m = min(m0 + r, m_hi - 1);
-      const int64_t row = a.x_rows ? a.x_rows[m] : m;
-      src[i] = reinterpret_cast<const char*>(a.x + row * a.ldx) + c * 16;
-    } else {
-      const int q = p - XB / 1024, d = q / (WB / 1024);
-      constexpr int CH = WROW / 16;
-      const int r = (q - d * (WB / 1024)) * WRP + lane / CH;
-      const int c = (lane % CH) ^ (WF ? (r >> 1) & 7 : (r >> 2) & 3);
-      src[i] = reinterpret_cast<const char*>((DUAL && d ? w2 : w) + (int64_t)min(n0 + r, a.N - 1) * a.K) + c * 16;
-    }
-  }
-  const int KT = a.K / BK;
-  auto issue = [&](int kt) __attribute__((always_inline)) {
-    char* base = lds + (kt & (NST - 1)) * STAGE;
-#pragma unroll
-    for (int i = 0; i < PP; ++i) {
-      const bool x = dst[i] < XB;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)kt * (x ? 128 : WROW)),
-                                       (__attribute__((address_space(3))) void*)(base + dst[i]), 16, 0, 0);
-    }
-  };
+  const int n0 = blockIdx.x * BN, KT = a.K / BK;
   const int wm = (wave / WN) * 16 * FM, wn = (wave % WN) * 16 * FN;
   const int r16 = lane & 15, kg = lane >> 4;
-  f32x4 acc[ND][FM][FN];
+  const bool y_vec = (a.ldy % 4 == 0) && dev_aligned16(a.y);
+  // without groups the workgroup's one tile; with them every gridDim.y-th row tile of all groups
+  for (int tile = blockIdx.y;; tile += gridDim.y) {
+    int m0 = tile * BM, m_hi = a.M;
+    const float* x = a.x;
+    const TW *w = static_cast<const TW*>(a.w), *w2 = static_cast<const TW*>(a.w2);
+    float* y = a.y;
+    if constexpr (GROUPED) {
+      int g;
+      if (!group_tile<BM>(a.group_offsets, a.n_groups, tile, g, m0, m_hi)) return;
+      w += (int64_t)g * a.N * a.K;
+      if (DUAL) w2 += (int64_t)g * a.N * a.K;
+      if (tile != (int)blockIdx.y) __syncthreads();  // (the tile before is read)
+    } else {
+      if (m0 >= m_hi) return;
+      x += (int64_t)blockIdx.z * a.x_batch;
+      y += (int64_t)blockIdx.z * a.y_batch;
+      if (a.gate) a.gate += (int64_t)blockIdx.z * a.gate_batch;
+      w += (int64_t)blockIdx.z * a.N * a.K;
+      if (DUAL) w2 += (int64_t)blockIdx.z * a.N * a.K;
+    }
+    const char* src[PP];
+    int dst[PP];
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[d][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < KT) issue(s);
-  for (int kt = 0; kt < KT; ++kt) {
-    const int behind = min(KT - 1 - kt, NST - 2);  // steps requested behind this one: their pieces may still fly
-    if (behind == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PP) : "memory");
-    else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PP) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    if (kt + NST - 1 < KT) issue(kt + NST - 1);  // (into the image everybody finished reading before the barrier)
-    const char* sx = lds + (kt & (NST - 1)) * STAGE;
-    const char* sw = sx + XB;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      f32x4 xf[FM], wf[ND][FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int r = wm + i * 16 + r16;
-        xf[i] = *reinterpret_cast<const f32x4*>(sx + r * 128 + (((ks * 4 + kg) ^ ((r >> 1) & 7)) << 4));
+    for (int i = 0; i < PP; ++i) {
+      const int p = min(wave * PP + i, PIECES - 1);
+      dst[i] = p * 1024;
+      if (p < XB / 1024) {
+        const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        const int m = min(m0 + r, m_hi - 1);
+        const int64_t row = a.x_rows ? a.x_rows[m] : m;
+        src[i] = reinterpret_cast<const char*>(x + row * a.ldx) + c * 16;
+      } else {
+        const int q = p - XB / 1024, d = q / (WB / 1024);
+        constexpr int CH = WROW / 16;
+        const int r = (q - d * (WB / 1024)) * WRP + lane / CH;
+        const int c = (lane % CH) ^ (WF ? (r >> 1) & 7 : (r >> 2) & 3);
+        src[i] = reinterpret_cast<const char*>((DUAL && d ? w2 : w) + (int64_t)min(n0 + r, a.N - 1) * a.K) + c * 16;
       }
+    }
+    auto issue = [&](int kt) __attribute__((always_inline)) {
+      char* base = lds + (kt & (NST - 1)) * STAGE;
 #pragma unroll
-      for (int d = 0; d < ND; ++d)
+      for (int i = 0; i < PP; ++i) {
+        const bool is_x = dst[i] < XB;
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)kt * (is_x ? 128 : WROW)),
+                                         (__attribute__((address_space(3))) void*)(base + dst[i]), 16, 0, 0);
+      }
+    };
+    f32x4 acc[ND][FM][FN];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int r = wn + j * 16 + r16;
-          if constexpr (WF) {
-            wf[d][j] = *reinterpret_cast<const f32x4*>(sw + d * WB + r * 128 + (((ks * 4 + kg) ^ ((r >> 1) & 7)) << 4));
-          } else {
-            const u32x2 v = *reinterpret_cast<const u32x2*>(sw + d * WB + r * 64 + (((ks * 2 + (kg >> 1)) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8);
-            wf[d][j] = f32x4{lo_bf(v[0]), hi_bf(v[0]), lo_bf(v[1]), hi_bf(v[1])};
-          }
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[d][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+      if (s < KT) issue(s);
+    for (int kt = 0; kt < KT; ++kt) {
+      const int behind = min(KT - 1 - kt, NST - 2);  // steps requested behind this one: their pieces may still fly
+      if (behind == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PP) : "memory");
+      else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PP) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (kt + NST - 1 < KT) issue(kt + NST - 1);  // (into the image everybody finished reading before the barrier)
+      const char* sx = lds + (kt & (NST - 1)) * STAGE;
+      const char* sw = sx + XB;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        f32x4 xf[FM], wf[ND][FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          const int r = wm + i * 16 + r16;
+          xf[i] = *reinterpret_cast<const f32x4*>(sx + r * 128 + (((ks * 4 + kg) ^ ((r >> 1) & 7)) << 4));
         }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int d = 0; d < ND; ++d)
 #pragma unroll
-          for (int i = 0; i < FM; ++i)
+          for (int j = 0; j < FN; ++j) {
+            const int r = wn + j * 16 + r16;
+            if constexpr (WF) {
+              wf[d][j] = *reinterpret_cast<const f32x4*>(sw + d * WB + r * 128 + (((ks * 4 + kg) ^ ((r >> 1) & 7)) << 4));
+            } else {
+              const u32x2 v = *reinterpret_cast<const u32x2*>(sw + d * WB + r * 64 + (((ks * 2 + (kg >> 1)) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8);
+              wf[d][j] = f32x4{lo_bf(v[0]), hi_bf(v[0]), lo_bf(v[1]), hi_bf(v[1])};
+            }
+          }
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-              acc[d][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[d][j][e], xf[i][e], acc[d][i][j], 0, 0, 0);
-    }
-  }
-  const bool y_vec = (a.ldy % 4 == 0) && dev_aligned16(a.y);
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int m = m0 + wm + i * 16 + r16;
-    if (m >= m_hi) continue;
-    const int64_t yrow = a.y_rows ? a.y_rows[m] : m;
+          for (int d = 0; d < ND; ++d)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int n = n0 + wn + j * 16 + kg * 4;
-      float v[4];
+            for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        v[r] = n + r < a.N ? finish<DUAL, EXT>(a, m, yrow, n + r, acc[0][i][j][r], acc[ND - 1][i][j][r]) : 0.f;
-      float* yp = a.y + yrow * a.ldy + n;
-      if (n + 4 <= a.N && y_vec) {
-        *reinterpret_cast<float4*>(yp) = float4{v[0], v[1], v[2], v[3]};
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < a.N) yp[r] = v[r];
+              for (int j = 0; j < FN; ++j)
+                acc[d][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[d][j][e], xf[i][e], acc[d][i][j], 0, 0, 0);
       }
     }
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int m = m0 + wm + i * 16 + r16;
+      if (m >= m_hi) continue;
+      const int64_t yrow = a.y_rows ? a.y_rows[m] : m;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int n = n0 + wn + j * 16 + kg * 4;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] = n + r < a.N ? finish<DUAL, EXT>(a, m, yrow, n + r, acc[0][i][j][r], acc[ND - 1][i][j][r]) : 0.f;
+        float* yp = y + yrow * a.ldy + n;
+        if (n + 4 <= a.N && y_vec) {
+          *reinterpret_cast<float4*>(yp) = float4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < a.N) yp[r] = v[r];
+        }
+      }
+    }
+    if constexpr (!GROUPED) return;
   }
 }
 
@@ -909,28 +954,47 @@ static int launch_stream(const GemmAnyArgs& a, int groups, int rows, hipStream_t
   }
 }
 
-// Exact mode beyond a few rows.  The tile of gemm_any_f32_kernel: the largest of 64 x 64, 32 x 64, 32 x 32 whose grid puts a
-// workgroup on most of the 256 CUs; groups of less than 256 rows (an even share is assumed) in 32-row tiles, whose last one
-// is padded by less.  us, gemm_any_fma_kernel / here: 733 rows, K 1024: N 1024 64 / 17, N 3072 202 / 67, N 32 113 / 12; 32
-// experts of 92 rows, 1024 -> 2 x 512 with SwiGLU 351 / 96 (64-row tiles: 141), back to 1024 216 / 55 (66); a router, 8192
-// rows, K 2048, 64 bf16 rows 235 / 36.
+// Exact mode beyond a few rows.  The tile of gemm_any_f32_kernel: a launch takes some 6 us and, per 1024 of K, 18.7 us for every 256 tiles of
+// 64 x 64, 9.6 of 32 x 64, 5.05 of 32 x 32 or part of them (the matrix rate, shared by a CU's tiles): the least of the three.  us, the
+// largest tile that fills 180 workgroups / this: 721 rows x 1024 x 1024 25.3 / 20.7, x 2048 42.2 / 35.1, x 3072 62.7 / 51.7, 400 rows x 3072
+// 42.0 / 32.3; 1000 rows x 4096 keep 64 x 64 (81.1, 83.0, 87.1).  Groups: a last tile each that is half empty on average, and no workgroup for
+// a tile that is not there: 32 experts, 1024 -> 2 x 512 / back: 256 pairs 79 / 29 -> 28 / 18, 1600 pairs 69 / 37 -> 53 / 34, 6000 pairs 176 / 92 ->
+// 147 / 78; 64 experts, 2048 -> 2 x 768 / back, 512 pairs 304 / 88 -> 162 / 81.
 template <typename TW, bool DUAL, bool EXT>
-static int launch_exact(const GemmAnyArgs& a, int groups, int rows_per_group_max, hipStream_t st) {
+static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_max, hipStream_t st) {
+  GemmAnyArgs a = args;
+  a.n_groups = groups;
   constexpr int W16 = 16 / (int)sizeof(TW);
   const bool grouped = a.group_offsets != nullptr;
   const bool vec = a.K % 32 == 0 && a.ldx % 4 == 0 && aligned16(a.x) && aligned16(a.w) && (!DUAL || aligned16(a.w2)) && a.K % W16 == 0 &&
                    a.x_batch % 4 == 0;
   if (vec) {
-    const int rows = grouped ? (rows_per_group_max + groups - 1) / groups : rows_per_group_max;
-    auto tiles = [&](int bm, int bn) { return (int64_t)((rows + bm - 1) / bm) * ((a.N + bn - 1) / bn) * groups; };
-    auto grid = [&](int bm, int bn) { return dim3((a.N + bn - 1) / bn, (rows_per_group_max + bm - 1) / bm, groups); };
-    if (rows > 32 && a.N > 32 && tiles(64, 64) >= 180 && !(grouped && rows < 256)) {
-      hipLaunchKernelGGL((gemm_any_f32_kernel<TW, DUAL, 2, 2, 2, 2, EXT>), grid(64, 64), dim3(256), 0, st, a);
-    } else if (a.N > 32 && tiles(32, 64) >= 180) {
-      hipLaunchKernelGGL((gemm_any_f32_kernel<TW, DUAL, 2, 1, 1, 4, EXT>), grid(32, 64), dim3(256), 0, st, a);
-    } else {
-      hipLaunchKernelGGL((gemm_any_f32_kernel<TW, DUAL, 1, 1, 2, 2, EXT>), grid(32, 32), dim3(256), 0, st, a);
-    }
+    const auto nx = [&](int bn) { return (a.N + bn - 1) / bn; };
+    // groups: as many row tiles as rows_per_group_max rows in all of them have at most, and no fewer than four workgroups per CU; what
+    // there is beyond (the bound is one group's) the workgroups take behind their first.  (A tile per group and row tile of the bound were
+    // 23296 workgroups for 768 tiles: 2900 pairs over 32 experts.)
+    auto grid = [&](int bm, int bn) {
+      const int ny = (rows_per_group_max + bm - 1) / bm;
+      if (!grouped) return dim3(nx(bn), ny, groups);
+      const int64_t most = (int64_t)ny * groups, total = rows_per_group_max / bm + groups, fill = (1024 + nx(bn) - 1) / nx(bn);
+      return dim3(nx(bn), (unsigned)std::min(most, std::max(total, fill)), 1);
+    };
+    const auto cost = [&](int bm, int bn, double us) {
+      const int64_t row_tiles = grouped ? rows_per_group_max / bm + (groups + 1) / 2 : (int64_t)((rows_per_group_max + bm - 1) / bm) * groups;
+      const int64_t per_cu = (row_tiles * nx(bn) + 255) / 256;
+      return per_cu == 1 ? 1.07 * us : (double)per_cu * us;   // (alone on its CU a tile waits out its own starts)
+    };
+    // (two weights: 64 x 64 has a CU to itself; the small tiles read their operands most often: beyond two per CU only where it is clear)
+    const double large = cost(64, 64, DUAL ? 21.0 : 18.7), medium = cost(32, 64, 9.6), one = cost(32, 32, 5.05), small = one > 11. ? 1.06 * one : one;
+    const auto go = [&](auto plain, auto of_groups, dim3 g) {   // (no group has the extended epilogue)
+      if (grouped) hipLaunchKernelGGL(of_groups, g, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL(plain, g, dim3(256), 0, st, a);
+    };
+#define MI_F32_TILE(FM, FN, WM, WN) gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, false>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, !EXT>
+    if (a.N > 32 && large <= medium && large <= small) go(MI_F32_TILE(2, 2, 2, 2), grid(64, 64));
+    else if (a.N > 32 && medium <= small) go(MI_F32_TILE(2, 1, 1, 4), grid(32, 64));
+    else go(MI_F32_TILE(1, 1, 2, 2), grid(32, 32));
+#undef MI_F32_TILE
     return check_launch();
   }
   // a router over a prompt: one column of tiles - short tiles, more of them (us, 64 / 16 rows: 1024 rows x 64 features x 1000 93 / 75,
