@@ -80,6 +80,8 @@ template <int VEC>
 using fvec = float __attribute__((ext_vector_type(VEC)));
 template <int VEC>
 __device__ __forceinline__ fvec<VEC> vat(const float* p) { return *reinterpret_cast<const fvec<VEC>*>(p); }
+template <int VEC>   // what is read once and is not in the caches
+__device__ __forceinline__ fvec<VEC> vat_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const fvec<VEC>*>(p)); }
 template <int VEC>
 __device__ __forceinline__ float vsum(fvec<VEC> v) {
   float s = 0.f;
@@ -1313,8 +1315,9 @@ __global__ __launch_bounds__(256) void route_grouped_kernel(const float* __restr
 }
 
 // grid (token, 256 * VEC channels); the parts' pieces are asked for CH at a time (beyond top_k: the last one again, not added).  Bound by
-// the experts' outputs: 8192 tokens of 8 x 2048 floats, 191 us with a float per request and one part after the other; now 134 (4.8 TB/s).
-template <int VEC, int CH>
+// the experts' outputs: 8192 tokens of 8 x 2048 floats, 191 us with a float per request and one part after the other, 128 in pieces, with ONCE
+// 94 (6.4 TB/s).  ONCE: outputs beyond what the caches hold of them are fetched past them (133 MB stay: 25.3 us, so 25.8).
+template <int VEC, int CH, bool ONCE = false>
 __global__ __launch_bounds__(256) void moe_combine_f32_kernel(const float* __restrict__ y, const float* __restrict__ h,
                                                               int64_t ldh, const int32_t* __restrict__ ids,
                                                               const float* __restrict__ wts, int top_k, int n_experts,
@@ -1329,7 +1332,8 @@ __global__ __launch_bounds__(256) void moe_combine_f32_kernel(const float* __res
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int k = min(k0 + j, top_k - 1);
-      v[j] = vat<VEC>((ids[t * top_k + k] >= n_experts ? h + t * ldh : y + (t * top_k + k) * width) + c);
+      const float* p = (ids[t * top_k + k] >= n_experts ? h + t * ldh : y + (t * top_k + k) * width) + c;
+      v[j] = ONCE ? vat_once<VEC>(p) : vat<VEC>(p);
     }
 #pragma unroll
     for (int j = 0; j < CH; ++j)
@@ -2426,9 +2430,10 @@ extern "C" int mi_moe_combine_f32(const float* y, const float* h, int64_t ldh, c
   if (n_tokens == 0) return MI_OK;
   const bool vec = width % 4 == 0 && ldh % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(h) && aligned16(out);
   // (no more requests than parts, about: 8192 tokens of one part of 250 6.7 us, four requests 9.5)
-  const auto kernel = vec ? (top_k <= 2   ? moe_combine_f32_kernel<4, 2>
-                             : top_k <= 4 ? moe_combine_f32_kernel<4, 4>
-                                          : moe_combine_f32_kernel<4, 8>)
+  const bool once = (int64_t)n_tokens * top_k * width > (int64_t)64 << 20;   // (the Infinity Cache: 256 MB)
+  const auto kernel = vec ? (top_k <= 2   ? (once ? moe_combine_f32_kernel<4, 2, true> : moe_combine_f32_kernel<4, 2>)
+                             : top_k <= 4 ? (once ? moe_combine_f32_kernel<4, 4, true> : moe_combine_f32_kernel<4, 4>)
+                                          : (once ? moe_combine_f32_kernel<4, 8, true> : moe_combine_f32_kernel<4, 8>))
                           : (top_k <= 2 ? moe_combine_f32_kernel<1, 1> : moe_combine_f32_kernel<1, 4>);
   const int cols = vec ? 1024 : 256;
   hipLaunchKernelGGL(kernel, dim3(n_tokens, (width + cols - 1) / cols), dim3(256), 0, S(stream), y, h, ldh, ids, weights, top_k,
