@@ -22,6 +22,7 @@
 //   gemm_any_rows_kernel   M <= 8 rows, and the exact mode up to 64: one wave per (one or four output features, batch of rows)
 //                          streams its weight row once, lanes split K in 16-byte pieces, butterfly reduction; both
 //                          dtypes, x not rounded
+//   gemm_any_rows_lds_kernel  the same sums for 2 to 8 rows and many features of bf16 weights: the rows in LDS
 //   gemm_any_each_row_kernel  the same for groups that have a row or none each
 //
 // A row of the result is a function of its own x row and the weights only: the summation order over k does not depend
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_kernel(GemmAnyArgs
 // Bound by what is asked for at a time: the rows' pieces are loaded without a branch (rows beyond the end: the last one again, not
 // stored), so that a K piece is one round trip and not one per row - a router's 32 rows x 64 features x 2048 10.7 -> 6.7 us - and
 // four features share the rows' pieces where there are enough features for the chip (N 32768, K 2048: 8 rows 110 us with one feature
-// and a branch per row, now 76, 4 rows 62 / 40; a single row 31 with one feature, 36 with four).
+// and a branch per row, 76 so, 4 rows 62 / 40; a single row 31 with one feature, 36 with four).
 // UNROLL: K pieces that are asked for together; more than one only where all lanes have as many pieces - the last ones, which some lanes
 // lack, would be a pass of their own (64 rows x 1024 features x 1000 18.5 us, one at a time 13.2).
 template <typename TW, int MT, int FT, bool DUAL, bool EXT, int UNROLL = (FT == 1 ? 2 : 1)>
@@ -847,6 +848,82 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(GemmAnyArgs a) {
         a.y[yrow * a.ldy + n + f] = finish<DUAL, EXT>(a, m0 + r, yrow, n + f, v, v2);
       }
     }
+}
+
+// butterfly steps OFF, OFF / 2, ... over 2 HALF sums: after a step a lane goes on with the half of them that its side keeps
+template <int HALF, int OFF, int C>
+__device__ __forceinline__ void halve_sums(float (&v)[C], int lane) {
+  const bool up = lane & OFF;
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) {
+    if constexpr (OFF >= 16) {   // (the swap of the one's upper lanes with the other's lower ones is the exchange)
+      const uint32_t lo = __float_as_uint(v[i]), hi = __float_as_uint(v[i + HALF]);
+      const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(lo, hi, false, false) : __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
+      v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+      const float keep = up ? v[i + HALF] : v[i], give = up ? v[i] : v[i + HALF];
+      v[i] = keep + xor_get<OFF>(give);
+    }
+  }
+  if constexpr (HALF > 1) halve_sums<HALF / 2, OFF / 2>(v, lane);
+}
+
+// The same for 2 to 8 rows of wide products (the heads of a few sequences): the rows lie in LDS, so that a wave's only requests are its
+// weights, the next piece's ahead of the arithmetic; persistent workgroups of eight waves, two per CU, so that the rows are laid out
+// once.  The sums are gemm_any_rows_kernel's, in its order: a lane's pieces ascending, then the butterfly - of which a lane continues only the
+// half of the sums that its side of the step keeps (32 exchanges instead of 192).  A row's pieces of eight lie as their first and
+// their second halves: 16-byte reads of neighbouring lanes on neighbouring banks.
+// Bound by the weights (us, weights beyond the caches, gemm_any_rows_kernel / here, TB/s here): 8 rows x 32768 x 2048 76.7 / 32.5 (4.1), x 151936
+// x 1024 211 / 62.9 (4.9); 4 rows 41.7 / 28.5 (4.7) and 113 / 54.9 (5.7).
+template <int MT, bool EXT>
+__global__ __launch_bounds__(512, 4) void gemm_any_rows_lds_kernel(GemmAnyArgs a) {
+  constexpr int FT = 4, C = FT * MT;
+  extern __shared__ __attribute__((aligned(16))) f32x4 xs[];  // [MT][2][K / 8]
+  const int lane = threadIdx.x & 63, np = a.K / 8, pieces = a.K / 512;
+  for (int i = threadIdx.x; i < MT * 2 * np; i += 512) {
+    const int r = i / (2 * np), c = i - r * 2 * np, m = min(r, a.M - 1);
+    xs[r * 2 * np + (c & 1) * np + (c >> 1)] = *reinterpret_cast<const f32x4*>(a.x + (int64_t)(a.x_rows ? a.x_rows[m] : m) * a.ldx + c * 4);
+  }
+  __syncthreads();
+  const int quads = (a.N + FT - 1) / FT, step = gridDim.x * 8;
+  const uint16_t* const w = static_cast<const uint16_t*>(a.w) + lane * 8;
+  u32x4 next[FT];
+  auto ask = [&](int q, int p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+      next[f] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(w + (int64_t)min(q * FT + f, a.N - 1) * a.K + p * 512));
+  };
+  int q = blockIdx.x * 8 + (threadIdx.x >> 6);
+  if (q >= quads) return;  // (whole waves, behind the only barrier)
+  ask(q, 0);
+  for (; q < quads; q += step) {
+    float acc[C] = {};
+    for (int p = 0; p < pieces; ++p) {
+      u32x4 now[FT];
+#pragma unroll
+      for (int f = 0; f < FT; ++f) now[f] = next[f];
+      const bool last = p + 1 == pieces;
+      ask(last ? min(q + step, quads - 1) : q, last ? 0 : p + 1);
+#pragma unroll
+      for (int r = 0; r < MT; ++r) {
+        const f32x4 x0 = xs[r * 2 * np + p * 64 + lane], x1 = xs[r * 2 * np + np + p * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int f = 0; f < FT; ++f)
+            acc[f * MT + r] = fmaf(i < 4 ? x0[i & 3] : x1[i & 3], i & 1 ? hi_bf(now[f][i >> 1]) : lo_bf(now[f][i >> 1]), acc[f * MT + r]);
+      }
+    }
+    halve_sums<C / 2, 32>(acc, lane);
+    float v = acc[0];
+    if constexpr (C == 16) v = xor_sum<2>(v);
+    v = xor_sum<1>(v);
+    const int idx = lane / (64 / C), m = idx % MT, n = q * FT + idx / MT;
+    if (lane % (64 / C) == 0 && m < a.M && n < a.N) {
+      const int64_t yrow = a.y_rows ? a.y_rows[m] : m;
+      a.y[yrow * a.ldy + n] = finish<false, EXT>(a, m, yrow, n, v, 0.f);
+    }
+  }
 }
 
 // The same one row after the other, for groups that have one or none each (the experts of a token or two): a batch would multiply its
@@ -1021,6 +1098,17 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
     }
     const int ft = !DUAL && mt > 1 && a.N >= 8192 ? 4 : 1;   // (a wave per four features: from two workgroups per CU on)
     const dim3 grid((a.N + 4 * ft - 1) / (4 * ft), (rows_per_group_max + mt - 1) / mt, groups);
+    // From 4096 features on and 12288 sums, in which the layout of the rows and the wide waves pay (us, gemm_any_rows_kernel / here: 2 rows x 4096 x
+    // 2048 7.6 / 8.2, 3 rows 9.0 / 8.1, 8 rows 16.4 / 10.7; 2 x 6144 x 2048 9.8 / 9.0; 5 x 3072 x 2048 9.8 / 10.2); 64 KB of rows at most: two
+    // workgroups on a CU.
+    if constexpr (!DUAL && sizeof(TW) == 2)
+      if (mt > 1 && rows_per_group_max <= 8 && a.N >= 4096 && (int64_t)a.N * rows_per_group_max >= 12288 && groups == 1 && !a.group_offsets && a.K % 512 == 0 && mt * a.K * 4 <= 65536 && a.ldx % 4 == 0 &&
+          aligned16(a.x) && aligned16(a.w)) {
+        const dim3 persistent(std::min(512, (a.N + 31) / 32));
+        if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_lds_kernel<4, EXT>), persistent, dim3(512), mt * a.K * 4, st, a);
+        else hipLaunchKernelGGL((gemm_any_rows_lds_kernel<8, EXT>), persistent, dim3(512), mt * a.K * 4, st, a);
+        return check_launch();
+      }
     if constexpr (!DUAL)
       if (ft == 4) {
         if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_kernel<TW, 4, 4, DUAL, EXT>), grid, dim3(256), 0, st, a);
