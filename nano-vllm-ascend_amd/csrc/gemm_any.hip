@@ -66,7 +66,7 @@ struct GemmAnyArgs {
   // several projections of one input, each with an activation of its own, as one product
   bool ext;
   int act_from, act2, act2_from;
-  int n_groups;  // gemm_any_f32_kernel's grouped form
+  int n_groups;  // the grouped forms of gemm_any_f32_kernel and the streaming kernel
 };
 
 template <typename TW>
@@ -240,12 +240,13 @@ __global__ __launch_bounds__(256) void gemm_any_fma_kernel(GemmAnyArgs a) {
 // Rows beyond the group's end and features beyond N are read from the last valid one and not stored.
 // Needs K % 32 == 0, 16-byte aligned rows of x and w; anything else: gemm_any_fma_kernel.
 // Measured against gemm_any_fma_kernel (64 x 64 tiles, element-wise loads, plain FMA chains), us: see launch_exact.
-// The tile-th row tile of BM rows over all groups (group by group): its group and rows, or false beyond the last.  Every wave for itself.
-template <int BM>
+// The tile-th row tile of BM rows over all groups (group by group, a group's first SKIP rows left out): its group, its first row and the end
+// of the group's rows, or false beyond the last.  Every wave for itself.
+template <int BM, int SKIP = 0>
 __device__ __forceinline__ bool group_tile(const int32_t* __restrict__ offsets, int groups, int tile, int& g, int& m0, int& m_hi) {
   const int lane = threadIdx.x & 63;
   for (int base = 0; base < groups; base += 64) {
-    const int i = min(base + lane, groups - 1), lo = offsets[i], hi = offsets[i + 1];
+    const int i = min(base + lane, groups - 1), lo = offsets[i] + SKIP, hi = offsets[i + 1];
     const int mine = base + lane < groups ? (max(hi - lo, 0) + BM - 1) / BM : 0;
     int upto = mine;
 #pragma unroll
@@ -653,21 +654,18 @@ __global__ __launch_bounds__(256) void gemm_any_skinny_kernel(GemmAnyArgs a) {
 // us, operand pass + tile kernel / here: 24 rows x 1024 x 1024 9.3 / 5.4, 32 x 2048 x 2048 13.0 / 8.5, 9 x 2048 x 2048 12.9 / 5.9, 48 x
 // 4096 x 2048 14.3 / 11.0, 64 x 1024 x 1024 9.5 / 8.2; SwiGLU 32 x 3072 x 2048 20.8 / 11.0; both products of 256 pairs over 64 experts of
 // 768 x 2048 126 / 67 + 37 (402 MB at 6.0 TB/s), of 96 over 32 of 512 x 1024 30 / 17 + 11.
+constexpr int stream_slot(int nw, int mf) {  // per wave: bf16 images [16 nw weight rows | 16 mf x rows][64 k] of the block it multiplies; then its sums
+  return (nw + mf) * 2048 > nw * mf * 1024 ? (nw + mf) * 2048 : nw * mf * 1024;
+}
+// the workgroup's features of rows m_lo .. m_hi - 1, 16 MF at a time
 template <bool DUAL, int MF, int RT, int WAVES, bool EXT>
-__global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_kernel(GemmAnyArgs a) {
+__device__ __forceinline__ void stream_rows(const GemmAnyArgs& a, char* lds, const uint16_t* w, const uint16_t* w2, int m_lo, int m_hi) {
   static_assert(RT == 1 || !DUAL, "several feature tiles: one weight");
-  constexpr int NW = DUAL ? 2 : RT;
-  // per wave: bf16 images [16 NW weight rows | 16 MF x rows][64 k] of the block it multiplies; then its sums
-  constexpr int IMAGE = (NW + MF) * 2048, SUMS = NW * MF * 1024, SLOT = IMAGE > SUMS ? IMAGE : SUMS;
-  __shared__ __attribute__((aligned(16))) char lds[WAVES * SLOT];
+  constexpr int NW = DUAL ? 2 : RT, SLOT = stream_slot(NW, MF);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   char* const slot = lds + wave * SLOT;
   auto sums = [&](int i, int t, int f) __attribute__((always_inline)) { return reinterpret_cast<f32x4*>(lds + i * SLOT + ((t * MF + f) * 64 + lane) * 16); };
-  int m_lo, m_hi;
-  const uint16_t *w, *w2;
-  select_group<uint16_t, DUAL>(a, w, w2, m_lo, m_hi);
-  if (m_lo >= m_hi) return;
   const int n0 = blockIdx.x * 16 * RT;
   const int fr = lane & 15, g = lane >> 4;
   const uint16_t* wp[NW][2];  // a request: eight weight rows of 128 bytes / four x rows of 256
@@ -778,6 +776,40 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_kernel(GemmAnyArgs
           if (n + r < a.N) yp[r] = o[r];
       }
     }
+  }
+}
+
+template <bool DUAL, int MF, int RT, int WAVES, bool EXT>
+__global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_kernel(GemmAnyArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[WAVES * stream_slot(DUAL ? 2 : RT, MF)];
+  int m_lo, m_hi;
+  const uint16_t *w, *w2;
+  select_group<uint16_t, DUAL>(a, w, w2, m_lo, m_hi);
+  stream_rows<DUAL, MF, RT, WAVES, EXT>(a, lds, w, w2, m_lo, m_hi);
+}
+
+// Groups, sixteen rows per workgroup: the first n_groups (blockIdx.z) take their group's first ones, those behind share what is left - of the few
+// groups that have more than the others, or of a step whose pairs go to one expert.  A group as one workgroup's walk, whatever it has: 757
+// pairs on one of 128 experts of 512 x 512 212 us, so 24 (tile kernels 19); 512 on two of 64 of 768 x 2048 230 / 52 (30); shared as a router
+// does, 256 pairs of those 108 / 105 (125).  32 or 64 rows at a time for what is left hold registers and LDS that the first rows then lack (126
+// and 160 us for 512 pairs, eight each; so 112).
+template <bool DUAL, int RT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_groups_kernel(GemmAnyArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[WAVES * stream_slot(DUAL ? 2 : RT, 1)];
+  int m_lo, m_hi;
+  const uint16_t *w, *w2;
+  const int share = (int)gridDim.z - a.n_groups;
+  if ((int)blockIdx.z < a.n_groups) {
+    select_group<uint16_t, DUAL>(a, w, w2, m_lo, m_hi);
+    stream_rows<DUAL, 1, RT, WAVES, false>(a, lds, w, w2, m_lo, share ? min(m_hi, m_lo + 16) : m_hi);
+    return;
+  }
+  int g;
+  for (int piece = (int)blockIdx.z - a.n_groups; group_tile<16, 16>(a.group_offsets, a.n_groups, piece, g, m_lo, m_hi); piece += share) {
+    w = static_cast<const uint16_t*>(a.w) + (int64_t)g * a.N * a.K;
+    w2 = DUAL ? static_cast<const uint16_t*>(a.w2) + (int64_t)g * a.N * a.K : nullptr;
+    stream_rows<DUAL, 1, RT, WAVES, false>(a, lds, w, w2, m_lo, min(m_hi, m_lo + 16));
+    __syncthreads();  // (the sums are read)
   }
 }
 
@@ -985,26 +1017,36 @@ bool any_stream_takes(int rows, int N, int K, int n_groups) {
 }
 
 template <bool DUAL, bool EXT>
-static int launch_stream(const GemmAnyArgs& a, int groups, int rows, hipStream_t st) {
+static int launch_stream(const GemmAnyArgs& args, int groups, int rows, hipStream_t st) {
+  GemmAnyArgs a = args;
+  a.n_groups = groups;
+  int z = groups;
   auto go = [&](auto kernel, int rt, int waves) {
-    hipLaunchKernelGGL(kernel, dim3((a.N + 16 * rt - 1) / (16 * rt), 1, groups), dim3(64 * waves), 0, st, a);
+    hipLaunchKernelGGL(kernel, dim3((a.N + 16 * rt - 1) / (16 * rt), 1, z), dim3(64 * waves), 0, st, a);
     return check_launch();
   };
-  if (groups > 1 || a.group_offsets) {
-    // workgroups enough: four waves each, so that several share a CU (eight: 256 pairs over 64 experts' second product 55 us, four 37);
-    // groups: 16 rows at a time
-    const int mf = a.group_offsets ? 1 : (rows + 15) / 16;
-    if constexpr (!DUAL) {
-      if (mf == 1 && (int64_t)(a.N / 16) * groups >= 2048) return go(gemm_any_stream_kernel<false, 1, 2, 4, EXT>, 2, 4);
-    }
-    switch (mf) {
-      case 1: return go(gemm_any_stream_kernel<DUAL, 1, 1, 4, EXT>, 1, 4);
-      case 2: return go(gemm_any_stream_kernel<DUAL, 2, 1, 4, EXT>, 1, 4);
-      case 3: return go(gemm_any_stream_kernel<DUAL, 3, 1, 4, EXT>, 1, 4);
-      default: return go(gemm_any_stream_kernel<DUAL, 4, 1, 4, EXT>, 1, 4);
-    }
+  // groups and batches: workgroups enough, four waves each, so that several share a CU (eight: 256 pairs over 64 experts' second product 55
+  // us, four 37)
+  if (a.group_offsets) {
+    if constexpr (EXT) return MI_EUNSUPPORTED;   // (no group has the extended epilogue)
+    z = groups + std::min(rows / 16, 65535 - groups);   // (`rows` rows in all have no more sixteens beyond a group's first)
+    if constexpr (!DUAL && !EXT)
+      if ((int64_t)(a.N / 16) * groups >= 2048) return go(gemm_any_stream_groups_kernel<false, 2, 4>, 2, 4);
+    if constexpr (!EXT) return go(gemm_any_stream_groups_kernel<DUAL, 1, 4>, 1, 4);
   }
   const int mf = (rows + 15) / 16;
+  if constexpr (!DUAL && !EXT) {   // (no batch has two weights or the extended epilogue)
+    if (groups > 1) {
+      switch (mf) {
+        case 1:
+          return (int64_t)(a.N / 16) * groups >= 2048 ? go(gemm_any_stream_kernel<false, 1, 2, 4, false>, 2, 4)
+                                                      : go(gemm_any_stream_kernel<false, 1, 1, 4, false>, 1, 4);
+        case 2: return go(gemm_any_stream_kernel<false, 2, 1, 4, false>, 1, 4);
+        case 3: return go(gemm_any_stream_kernel<false, 3, 1, 4, false>, 1, 4);
+        default: return go(gemm_any_stream_kernel<false, 4, 1, 4, false>, 1, 4);
+      }
+    }
+  }
   if constexpr (DUAL) {
     switch (mf) {
       case 1: return go(gemm_any_stream_kernel<true, 1, 1, 4, EXT>, 1, 4);
