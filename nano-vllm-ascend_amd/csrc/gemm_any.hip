@@ -1016,6 +1016,10 @@ bool any_stream_takes(int rows, int N, int K, int n_groups) {
   return rows <= 64 && N <= (rows <= 24 ? INT32_MAX : rows <= 32 ? 16384 : rows <= 48 ? 6144 : 4096);
 }
 
+// Batches (64 rows a batch at most: the features of a head); many of one 64-deep block each are slower so (32 of 64 rows x 512 x 64: 6.9 us on
+// gemm_any_skinny_kernel, 7.9)
+static bool batches_stream(int rows, int N, int K, int n_batch) { return rows <= 64 && K % 64 == 0 && !(K == 64 && (int64_t)n_batch * N > 8192); }
+
 template <bool DUAL, bool EXT>
 static int launch_stream(const GemmAnyArgs& args, int groups, int rows, hipStream_t st) {
   GemmAnyArgs a = args;
@@ -1184,8 +1188,8 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
   }
   const dim3 grid((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups);
   if constexpr (sizeof(TW) == 2) {
-    const bool batches = !a.group_offsets && groups > 1;   // (64 rows a batch at most: the features of a head)
-    if (mode == 0 && (batches ? rows_per_group_max <= 64 && a.K % 64 == 0 : any_stream_takes(rows_per_group_max, a.N, a.K, a.group_offsets ? groups : 0)) &&
+    const bool batches = !a.group_offsets && groups > 1;
+    if (mode == 0 && (batches ? batches_stream(rows_per_group_max, a.N, a.K, groups) : any_stream_takes(rows_per_group_max, a.N, a.K, a.group_offsets ? groups : 0)) &&
         a.ldx % 4 == 0 && a.x_batch % 4 == 0 && aligned16(a.x) && aligned16(a.w) && (!DUAL || aligned16(a.w2)))
       return launch_stream<DUAL, EXT>(a, groups, rows_per_group_max, st);
     if (mode == 0 && rows_per_group_max >= 512 && a.N >= 128) {  // prefill-sized: 128-row tiles, 128 (SwiGLU: 64) features
@@ -1223,9 +1227,11 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
 // tiles, x rows from memory into the MFMA operand (rounded to bf16 once, as gemm_any_mfma_kernel does), the next tile's rows requested
 // before this one is multiplied; two workgroups per CU.  gemm_any_mfma_kernel (both operands through LDS for every 64 features, two barriers per K
 // step): 128 -> 256 160 us, 256 -> 128 98 us; here 48 and 43 (4.2 and 4.7 TB/s).  Same summation order (k ascending in one chain), same bits.
+// Fewer rows and heads than CUs: a head's features are shared by several workgroups (blockIdx.y, n_share features each): 4 heads of 185 rows, 64 -> 512
+// 5.5 us on gemm_any_mfma_kernel, 10.3 with a workgroup per 128 rows, 3.4 so; 16 of 318, 128 -> 256 8.0 / 10.4 / 6.0.
 constexpr int kHeadsWeightElems = 32768, kHeadsLds = 2 * kHeadsWeightElems + 16 * 512;
 template <int KF>  // K = 32 KF (256: one workgroup per CU, the next rows' registers)
-__global__ __launch_bounds__(512, KF == 8 ? 2 : 4) void gemm_any_heads_kernel(GemmAnyArgs a) {
+__global__ __launch_bounds__(512, KF == 8 ? 2 : 4) void gemm_any_heads_kernel(GemmAnyArgs a, int n_share) {
   __shared__ __attribute__((aligned(16))) char lds[kHeadsLds];
   constexpr int K = 32 * KF, ROW = 2 * K + 16;
   const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
@@ -1233,8 +1239,9 @@ __global__ __launch_bounds__(512, KF == 8 ? 2 : 4) void gemm_any_heads_kernel(Ge
   int m_lo, m_hi;
   const uint16_t *w, *w2;
   select_group<uint16_t, false>(a, w, w2, m_lo, m_hi);
-  for (int i = threadIdx.x; i < a.N * (K / 8); i += 512)
-    *reinterpret_cast<u32x4*>(lds + (i / (K / 8)) * ROW + (i % (K / 8)) * 16) = *reinterpret_cast<const u32x4*>(w + (int64_t)i * 8);
+  const int n_lo = blockIdx.y * n_share, n_count = min(a.N - n_lo, n_share);
+  for (int i = threadIdx.x; i < n_count * (K / 8); i += 512)
+    *reinterpret_cast<u32x4*>(lds + (i / (K / 8)) * ROW + (i % (K / 8)) * 16) = *reinterpret_cast<const u32x4*>(w + (int64_t)n_lo * K + (int64_t)i * 8);
   f32x4 raw[KF][2];
   auto request = [&](int m0) __attribute__((always_inline)) {
     const float* xp = a.x + (int64_t)min(m0 + r16, m_hi - 1) * a.ldx + q * 8;
@@ -1256,9 +1263,9 @@ __global__ __launch_bounds__(512, KF == 8 ? 2 : 4) void gemm_any_heads_kernel(Ge
                              pack_bf(raw[ks][1][2], raw[ks][1][3])});
     request(m0 + step);   // (past the last tile: the last row again)
     const int m = m0 + r16;
-    float* yp = a.y + (int64_t)m * a.ldy + q * 4;
-    const float* gp = a.gate ? a.gate + (int64_t)min(m, m_hi - 1) * a.ldgate + q * 4 : nullptr;
-    for (int n = 0; n < a.N; n += 32) {
+    float* yp = a.y + (int64_t)m * a.ldy + n_lo + q * 4;
+    const float* gp = a.gate ? a.gate + (int64_t)min(m, m_hi - 1) * a.ldgate + n_lo + q * 4 : nullptr;
+    for (int n = 0; n < n_count; n += 32) {
       f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int ks = 0; ks < KF; ++ks)
@@ -1278,19 +1285,22 @@ __global__ __launch_bounds__(512, KF == 8 ? 2 : 4) void gemm_any_heads_kernel(Ge
     }
   }
 }
-// x, y and gate rows in 16-byte pieces, whole 32-feature steps, a head's weight in LDS; up to 64 rows the products stream their weights
+// x, y and gate rows in 16-byte pieces, whole 32-feature steps, a head's weight in LDS; up to 64 rows the products stream their weights, and many heads of
+// up to 128 rows stay where they were at K 256 (16 of 128 rows, 64 features: 1.20 times as long here; 8 heads 0.86)
 static bool heads_takes(const GemmAnyArgs& a, int w_dtype, int n_batch, bool exact) {
   return !exact && w_dtype == MI_DTYPE_BF16 && n_batch > 1 && a.M > 64 && (a.K == 64 || a.K == 128 || a.K == 256) && a.N > 0 &&
-         a.N % 32 == 0 && a.N <= 512 && a.N * a.K <= kHeadsWeightElems && aligned16(a.x) && aligned16(a.w) && aligned16(a.y) &&
+         !(a.K == 256 && a.M <= 128 && n_batch >= 16) && a.N % 32 == 0 && a.N <= 512 && a.N * a.K <= kHeadsWeightElems && aligned16(a.x) && aligned16(a.w) && aligned16(a.y) &&
          a.ldx % 4 == 0 && a.x_batch % 4 == 0 && a.ldy % 4 == 0 && a.y_batch % 4 == 0 &&
          (!a.gate || (aligned16(a.gate) && a.ldgate % 4 == 0 && a.gate_batch % 4 == 0));
 }
 static int launch_heads(const GemmAnyArgs& a, int n_batch, hipStream_t st) {
   const int rows = (a.M + 127) / 128, fill = ((a.K == 256 ? 256 : 512) + n_batch - 1) / n_batch;   // (the workgroups that run together)
-  const dim3 grid(rows < fill ? rows : fill, 1, n_batch);
-  if (a.K == 64) hipLaunchKernelGGL((gemm_any_heads_kernel<2>), grid, dim3(512), 0, st, a);
-  else if (a.K == 128) hipLaunchKernelGGL((gemm_any_heads_kernel<4>), grid, dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((gemm_any_heads_kernel<8>), grid, dim3(512), 0, st, a);
+  const int gx = rows < fill ? rows : fill, steps = a.N / 32;
+  const int slices = std::min(steps, std::max(1, 256 / (gx * n_batch))), n_share = (steps + slices - 1) / slices * 32;
+  const dim3 grid(gx, (a.N + n_share - 1) / n_share, n_batch);
+  if (a.K == 64) hipLaunchKernelGGL((gemm_any_heads_kernel<2>), grid, dim3(512), 0, st, a, n_share);
+  else if (a.K == 128) hipLaunchKernelGGL((gemm_any_heads_kernel<4>), grid, dim3(512), 0, st, a, n_share);
+  else hipLaunchKernelGGL((gemm_any_heads_kernel<8>), grid, dim3(512), 0, st, a, n_share);
   return check_launch();
 }
 
