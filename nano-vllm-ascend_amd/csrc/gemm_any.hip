@@ -1005,15 +1005,23 @@ __global__ __launch_bounds__(256) void gemm_any_each_row_kernel(GemmAnyArgs a) {
   }
 }
 
-// Where the streaming kernel is the faster one of it and the tile kernels (without groups and batches; us, tile kernels / here): up to 24
-// rows everywhere measured (24 x 32768 x 2048 35.3 / 34.3, 9 rows 35.2 / 28.3); beyond, every workgroup's copy of the rows outweighs its
-// weights from some number of features on: 32 x 16384 x 1024 11.9 / 11.3, x 32768 x 2048 36.2 / 37.0; 48 x 6144 x 2048 15.3 / 13.5, x 16384
-// x 1024 12.3 / 14.2; 64 x 4096 x 1024 9.5 / 8.9, x 16384 x 1024 12.8 / 19.9.  Grouped: up to ten rows a group on average (64 experts of 768 x 2048, 8
-// each 131 / 111, 16 each 131 / 140; 32 of 512 x 1024, 8 each 31.0 / 28.6, 16 each 31.0 / 33.8).
-bool any_stream_takes(int rows, int N, int K, int n_groups) {
+// Where the streaming kernel is the faster one of it and the tile kernels (us, tile kernels / here).  Without groups and batches every workgroup's
+// copy of the rows outweighs its weights from some number of features on: 24 rows x 32768 x 2048 35.3 / 34.3, 32 x 16384 x 1024 11.9 / 11.3,
+// x 32768 x 2048 36.2 / 37.0; 48 x 6144 x 2048 15.3 / 13.5, x 16384 x 1024 12.3 / 14.2; 64 x 4096 x 1024 9.5 / 8.9, x 16384 x 1024 12.8 / 19.9.
+// Beyond 16384 features and 16 rows a short K is too little work per workgroup (24 x 18432: K 64 1.09 times the tile kernels' time, 256 1.04,
+// 512 0.94); between 8192 and 16384 features a long one leaves a part round of long workgroups (24 x 12288: K 1024 0.95, 2048 1.02, 4096 1.15; 16
+// rows: 2048 0.90, 4096 1.03; 24 x 16384 x 8192 1.07).  Two weights: 17 rows x 12288 and 16384, K to 1024 1.00 to 1.20, from 2048 on 0.78 to 0.87;
+// 9 rows x 16384, K 128 1.09, 256 0.96.
+// Grouped: up to ten rows a group on average, eight where K is below 1024 (64 experts of 768 x 2048, 8 each 128 / 107, 10 each 120 / 111; 128 of 256
+// x 512, 10 each 31.8 / 34.6) and none of many short products (944 pairs, 128 experts of 768 x 256: 41 / 54).
+bool any_stream_takes(int rows, int N, int K, int n_groups, bool dual) {
   if (rows <= 8 || K % 64) return false;
-  if (n_groups) return rows <= 10 * (int64_t)n_groups;
-  return rows <= 64 && N <= (rows <= 24 ? INT32_MAX : rows <= 32 ? 16384 : rows <= 48 ? 6144 : 4096);
+  if (n_groups) return rows <= (K < 1024 ? 8 : 10) * (int64_t)n_groups && !(K <= 256 && (int64_t)n_groups * N >= 65536);
+  if (rows > 64) return false;
+  const int most = rows <= 24 ? INT32_MAX : rows <= 32 ? 16384 : rows <= 48 ? 6144 : 4096;
+  if (dual) return N <= std::min(most, rows <= 16 ? (K <= 128 ? 12288 : most) : K <= 1024 ? 8192 : most);
+  if (rows > 16 && ((N > 16384 && K < 512) || (N > 8192 && K >= 8192))) return false;
+  return N <= most && !(N > 8192 && N < 16384 && K >= (rows > 16 ? 2048 : 4096));
 }
 
 // Batches (64 rows a batch at most: the features of a head); many of one 64-deep block each are slower so (32 of 64 rows x 512 x 64: 6.9 us on
@@ -1059,8 +1067,9 @@ static int launch_stream(const GemmAnyArgs& args, int groups, int rows, hipStrea
       default: return go(gemm_any_stream_kernel<true, 4, 1, 4, EXT>, 1, 4);
     }
   } else {
-    // from 384 feature tiles on two per workgroup: half as many copies of x (24 rows x 6144 x 2048 12.8 / 10.5 us, x 4096 8.6 / 9.8)
-    if (a.N >= 6144) {
+    // more feature tiles than CUs: two per workgroup, half as many copies of x and no part round (24 rows x 6144 x 2048 12.8 / 10.5 us, x 4096 8.6
+    // / 9.8; of the tile kernels' time: 48 x 4224 x 2048 1.30 / 0.92, 24 x 5120 x 1024 0.96 / 0.72)
+    if (a.N > 4096) {
       switch (mf) {
         case 1: return go(gemm_any_stream_kernel<false, 1, 2, 4, EXT>, 2, 4);
         case 2: return go(gemm_any_stream_kernel<false, 2, 2, 4, EXT>, 2, 4);
@@ -1189,7 +1198,7 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
   const dim3 grid((a.N + 63) / 64, (rows_per_group_max + 63) / 64, groups);
   if constexpr (sizeof(TW) == 2) {
     const bool batches = !a.group_offsets && groups > 1;
-    if (mode == 0 && (batches ? batches_stream(rows_per_group_max, a.N, a.K, groups) : any_stream_takes(rows_per_group_max, a.N, a.K, a.group_offsets ? groups : 0)) &&
+    if (mode == 0 && (batches ? batches_stream(rows_per_group_max, a.N, a.K, groups) : any_stream_takes(rows_per_group_max, a.N, a.K, a.group_offsets ? groups : 0, DUAL)) &&
         a.ldx % 4 == 0 && a.x_batch % 4 == 0 && aligned16(a.x) && aligned16(a.w) && (!DUAL || aligned16(a.w2)))
       return launch_stream<DUAL, EXT>(a, groups, rows_per_group_max, st);
     if (mode == 0 && rows_per_group_max >= 512 && a.N >= 128) {  // prefill-sized: 128-row tiles, 128 (SwiGLU: 64) features
@@ -1320,7 +1329,7 @@ static int gemm_any_dispatch(const GemmAnyArgs& a, int w_dtype, int groups, int 
 static bool act_ok(int act) { return (act >= MI_ACT_NONE && act <= MI_ACT_SOFTCAP) || act == MI_ACT_RELU2; }
 static bool act_ext_ok(int act) { return (act_ok(act) && act != MI_ACT_SOFTCAP) || act == MI_ACT_TANH || act == MI_ACT_DECAY; }
 
-extern "C" int mi_gemm_any_streams(int rows, int N, int K, int n_groups) { return any_stream_takes(rows, N, K, n_groups) ? 1 : 0; }
+extern "C" int mi_gemm_any_streams(int rows, int N, int K, int n_groups) { return any_stream_takes(rows, N, K, n_groups, false) ? 1 : 0; }
 
 extern "C" int mi_gemm_any(const float* x, int64_t ldx, const void* w, int w_dtype, float* y, int64_t ldy, int M, int N,
                            int K, float alpha, int exact, mi_stream stream) {

@@ -324,7 +324,7 @@ extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const
   const bool fits = xb && x && w && y && w_dtype == MI_DTYPE_BF16 && M > 0 && ldx >= K && ldy >= N && ldy % 4 == 0 && aligned16(w) &&
                     (!w2 || aligned16(w2)) && aligned16(y) && (!bias || aligned16(bias)) && (!bias2 || (w2 && aligned16(bias2))) &&
                     aligned16(xb) && xb_elems >= (int64_t)M * K && !(act == MI_ACT_SOFTCAP && !(alpha > 0.f));
-  const bool streams = any_stream_takes(M, N, K, 0) && aligned16(x) && ldx % 4 == 0;
+  const bool streams = any_stream_takes(M, N, K, 0, w2 != nullptr) && aligned16(x) && ldx % 4 == 0;
   const int t = fits && !streams ? tile_rows_for(M, N, K, 0, w2 != nullptr, act) : 0;
   if (!t) return mi_gemm_any_act(x, ldx, w, w2, w_dtype, bias, bias2, act, y, ldy, M, N, K, alpha, 0, stream);
   const int rc = mi_gemm_any_operand(x, ldx, nullptr, nullptr, 0, t, M, K, xb, nullptr, stream);
@@ -369,7 +369,7 @@ extern "C" int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, cons
   const int64_t need = mi_expert_ff_bytes(pairs, G, ff, width, w2 != nullptr, act);
   if (need == 0) return MI_EUNSUPPORTED;
   if (scratch_bytes < need) return MI_EWORKSPACE;
-  if (any_stream_takes(pairs, ff, width, G) && any_stream_takes(pairs, width, ff, G) && aligned16(x) && ldx % 4 == 0 && aligned16(w) &&
+  if (any_stream_takes(pairs, ff, width, G, false) && any_stream_takes(pairs, width, ff, G, false) && aligned16(x) && ldx % 4 == 0 && aligned16(w) &&
       aligned16(down) && (!w2 || aligned16(w2))) {
     float* inner = static_cast<float*>(scratch);
     const int rc = mi_gemm_any_grouped_glu(x, ldx, pair_token, w, w2, MI_DTYPE_BF16, act, limit, row_scale, row_scale_rows, offsets, G, pairs,
