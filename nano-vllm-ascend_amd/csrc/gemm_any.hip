@@ -267,7 +267,9 @@ __device__ __forceinline__ bool group_tile(const int32_t* __restrict__ offsets, 
   return false;
 }
 
-template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT, bool GROUPED>
+// GROUPS: 0 none; 1 a workgroup for every row tile that a group can have; 2 as many as all groups' rows need, each every gridDim.y-th row tile of all
+// groups, which it has to find (0.8 us)
+template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT, int GROUPS>
 __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
   constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN, BK = 32, NST = 4, ND = DUAL ? 2 : 1;
   constexpr bool WF = sizeof(TW) == 4;
@@ -282,20 +284,26 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
   const int wm = (wave / WN) * 16 * FM, wn = (wave % WN) * 16 * FN;
   const int r16 = lane & 15, kg = lane >> 4;
   const bool y_vec = (a.ldy % 4 == 0) && dev_aligned16(a.y);
-  // without groups the workgroup's one tile; with them every gridDim.y-th row tile of all groups
+  if constexpr (GROUPS == 1)   // (asked for here: behind the way out below they would be a round trip of their own)
+    asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.y), "s"(a.x_rows), "s"(a.y_rows), "s"(a.ldx), "s"(a.ldy), "s"(a.row_scale), "s"(a.bias));
   for (int tile = blockIdx.y;; tile += gridDim.y) {
     int m0 = tile * BM, m_hi = a.M;
     const float* x = a.x;
     const TW *w = static_cast<const TW*>(a.w), *w2 = static_cast<const TW*>(a.w2);
     float* y = a.y;
-    if constexpr (GROUPED) {
-      int g;
-      if (!group_tile<BM>(a.group_offsets, a.n_groups, tile, g, m0, m_hi)) return;
+    if constexpr (GROUPS != 0) {
+      int g = blockIdx.z;
+      if constexpr (GROUPS == 1) {
+        m0 = a.group_offsets[g] + tile * BM, m_hi = a.group_offsets[g + 1];
+        if (m0 >= m_hi) return;
+      } else {
+        if (!group_tile<BM>(a.group_offsets, a.n_groups, tile, g, m0, m_hi)) return;
+      }
       w += (int64_t)g * a.N * a.K;
       if (DUAL) w2 += (int64_t)g * a.N * a.K;
       if (tile != (int)blockIdx.y) __syncthreads();  // (the tile before is read)
     } else {
-      if (m0 >= m_hi) return;
+      // (the launch has no tile beyond the rows: a way out here would put the other arguments' loads behind it, 0.3 us)
       x += (int64_t)blockIdx.z * a.x_batch;
       y += (int64_t)blockIdx.z * a.y_batch;
       if (a.gate) a.gate += (int64_t)blockIdx.z * a.gate_batch;
@@ -402,7 +410,7 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
         }
       }
     }
-    if constexpr (!GROUPED) return;
+    if constexpr (GROUPS != 2) return;
   }
 }
 
@@ -1102,14 +1110,17 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
                    a.x_batch % 4 == 0;
   if (vec) {
     const auto nx = [&](int bn) { return (a.N + bn - 1) / bn; };
-    // groups: as many row tiles as rows_per_group_max rows in all of them have at most, and no fewer than four workgroups per CU; what
-    // there is beyond (the bound is one group's) the workgroups take behind their first.  (A tile per group and row tile of the bound were
-    // 23296 workgroups for 768 tiles: 2900 pairs over 32 experts.)
+    // groups: a workgroup for every row tile that a group can have while they are few (32 pairs of 16 experts of 512 x 256: 14.1 us so, 16.9 where each
+    // looks for its tile); else as many row tiles as rows_per_group_max rows in all groups have at most, and no fewer than four workgroups per
+    // CU; what there is beyond (the bound is one group's) the workgroups take behind their first.  (A tile per group and row tile of the bound
+    // were 23296 workgroups for 768 tiles: 2900 pairs over 32 experts.)
     auto grid = [&](int bm, int bn) {
       const int ny = (rows_per_group_max + bm - 1) / bm;
       if (!grouped) return dim3(nx(bn), ny, groups);
-      const int64_t most = (int64_t)ny * groups, total = rows_per_group_max / bm + groups, fill = (1024 + nx(bn) - 1) / nx(bn);
-      return dim3(nx(bn), (unsigned)std::min(most, std::max(total, fill)), 1);
+      const int64_t most = (int64_t)ny * groups;
+      if (most * nx(bn) <= 1024) return dim3(nx(bn), ny, groups);
+      const int64_t total = rows_per_group_max / bm + groups, fill = (1024 + nx(bn) - 1) / nx(bn);
+      return dim3(nx(bn), (unsigned)std::min<int64_t>(std::min(most, std::max(total, fill)), 65535), 1);
     };
     const auto cost = [&](int bm, int bn, double us) {
       const int64_t row_tiles = grouped ? rows_per_group_max / bm + (groups + 1) / 2 : (int64_t)((rows_per_group_max + bm - 1) / bm) * groups;
@@ -1118,11 +1129,14 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
     };
     // (two weights: 64 x 64 has a CU to itself; the small tiles read their operands most often: beyond two per CU only where it is clear)
     const double large = cost(64, 64, DUAL ? 21.0 : 18.7), medium = cost(32, 64, 9.6), one = cost(32, 32, 5.05), small = one > 11. ? 1.06 * one : one;
-    const auto go = [&](auto plain, auto of_groups, dim3 g) {   // (no group has the extended epilogue)
-      if (grouped) hipLaunchKernelGGL(of_groups, g, dim3(256), 0, st, a);
-      else hipLaunchKernelGGL(plain, g, dim3(256), 0, st, a);
+    const auto go = [&](auto plain, auto direct, auto found, dim3 g) {   // (no group has the extended epilogue)
+      if (!grouped) hipLaunchKernelGGL(plain, g, dim3(256), 0, st, a);
+      else if ((int)g.z == groups && groups > 1) hipLaunchKernelGGL(direct, g, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL(found, g, dim3(256), 0, st, a);
     };
-#define MI_F32_TILE(FM, FN, WM, WN) gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, false>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, !EXT>
+#define MI_F32_TILE(FM, FN, WM, WN)                                                                                          \
+  gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, 0>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 1>, \
+      gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 2>
     if (a.N > 32 && large <= medium && large <= small) go(MI_F32_TILE(2, 2, 2, 2), grid(64, 64));
     else if (a.N > 32 && medium <= small) go(MI_F32_TILE(2, 1, 1, 4), grid(32, 64));
     else go(MI_F32_TILE(1, 1, 2, 2), grid(32, 32));
