@@ -283,7 +283,6 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
   const int n0 = blockIdx.x * BN, KT = a.K / BK;
   const int wm = (wave / WN) * 16 * FM, wn = (wave % WN) * 16 * FN;
   const int r16 = lane & 15, kg = lane >> 4;
-  const bool y_vec = (a.ldy % 4 == 0) && dev_aligned16(a.y);
   if constexpr (GROUPS == 1)   // (asked for here: behind the way out below they would be a round trip of their own)
     asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.y), "s"(a.x_rows), "s"(a.y_rows), "s"(a.ldx), "s"(a.ldy), "s"(a.row_scale), "s"(a.bias));
   for (int tile = blockIdx.y;; tile += gridDim.y) {
@@ -310,6 +309,7 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
       w += (int64_t)blockIdx.z * a.N * a.K;
       if (DUAL) w2 += (int64_t)blockIdx.z * a.N * a.K;
     }
+    const bool y_vec = (a.ldy % 4 == 0) && dev_aligned16(y);   // (a batch's rows begin where its stride says)
     const char* src[PP];
     int dst[PP];
 #pragma unroll

@@ -35,3 +35,20 @@ def test_groups(counts, bound, dual):
             z, size = torch.nn.functional.silu(z) * (xr[s] * b).sum(-1), 4 * size * ((xr[s] * b).abs().sum(-1) + 1)
         ok &= bool(((y[s] - z).abs() <= (K + 16) * 2.0 ** -24 * size + 1e-6).all())
     assert ok
+
+
+@pytest.mark.parametrize("M,N,shift", [(70, 36, 0), (100, 33, 1), (65, 64, 2)])
+def test_batches_off_16_bytes(M, N, shift):
+    """each batch's rows of the result begin where they begin, whatever the first one's do"""
+    from nanovllm import ops
+
+    B, K = 3, 64
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w = torch.randn(M, B * K, device="cuda", generator=g), torch.randn(B, N, K, device="cuda", generator=g)
+    out = torch.full((M, 4 * (B * (N + shift) // 4 + 2)), 7.0, device="cuda")
+    ops.gemm_any_batched(x, K, w, out, N + shift)
+    for b in range(B):
+        xr = x[:, b * K:(b + 1) * K].double()
+        got = out[:, b * (N + shift):b * (N + shift) + N].double()
+        assert bool(((got - xr @ w[b].double().T).abs() <= (K + 16) * 2.0 ** -24 * (xr.abs() @ w[b].double().abs().T)).all())
+        assert bool((out[:, b * (N + shift) + N:(b + 1) * (N + shift)] == 7.0).all())
