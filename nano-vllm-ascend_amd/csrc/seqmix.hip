@@ -671,7 +671,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_heads_mfma_kernel(
       }
   };
   const int step = 32 * WAVES * n_split;
-  int j0 = gap + 32 * (wave * n_split + split);   // (a context's first rounds go to different workgroups, that is, CUs)
+  int j0 = gap + 32 * (wave * n_split + split);   // (a context's first rounds go to different CUs: 1000 keys, 2 heads of 128 / 16, 10.8 -> 9.5 us)
   if (j0 <= hi_key) {
     if constexpr (FAST && WAVES == 8) {
       // two rounds in flight: the next one's requests leave before this one's scores.  Loads return in order: a page number is asked for in

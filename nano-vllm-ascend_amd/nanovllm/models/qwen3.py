@@ -327,7 +327,9 @@ class Qwen3Model(nn.Module):
         l0 = self.layers[0]
         rows4 = tp > 1 and l0.self_attn.o_proj.weight_rows4 is not None
         fuse_attn = not ctx.is_prefill and os.environ.get("MI355_ATTN_FUSED", "1") != "0"
-        order = ops.context_order(ctx.context_lens, l0.self_attn.num_kv_heads) if fuse_attn and l0.self_attn.attn.fusable else None
+        order = None
+        if fuse_attn and l0.self_attn.attn.fusable:
+            order = ops.context_order(ctx.context_lens, l0.self_attn.num_kv_heads, len(self.layers))
 
         xgmi = get_xgmi_comm() if tp > 1 else None
         fused_seam = (xgmi is not None and xgmi.fits_rows(rows, h.shape[1])

@@ -106,11 +106,15 @@ def paged_attn_decode(q, k_cache, v_cache, block_tables, context_lens, n_q_heads
     return out
 
 
-def context_order(context_lens, n_kv_heads: int):
+CONTEXT_ORDER_LAYERS = 4   # an order takes 2.8 to 4.6 us, and saves one to nine a layer
+
+
+def context_order(context_lens, n_kv_heads: int, layers: int | None = None):
     """What paged_attn_decode_fused takes as `order` in every layer of a decode step over these context lengths: {sequence, its context} with
-    the longest first [n, 2] - or None where it makes no difference (no more (sequence, kv head) units than the chip has CUs)."""
+    the longest first [n, 2] - or None where it makes no difference (no more (sequence, kv head) units than the chip has CUs) or would not
+    pay (layers, where it is told: fewer than CONTEXT_ORDER_LAYERS)."""
     n = context_lens.numel()
-    if n * n_kv_heads <= 256 or n > 1024:
+    if n * n_kv_heads <= 256 or n > 1024 or (layers is not None and layers < CONTEXT_ORDER_LAYERS):
         return None
     require_gpu(context_lens)
     assert context_lens.dtype == torch.int32 and context_lens.is_contiguous()

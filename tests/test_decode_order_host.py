@@ -1,0 +1,31 @@
+"""What the order of a decode step's contexts is made for, and what takes it.  The library is not called."""
+import pytest
+import torch
+
+from nanovllm import _C, ops
+
+
+class _Recorder:
+    def __init__(self, lib):
+        self.lib, self.calls = lib, []
+
+    def __getattr__(self, name):
+        if name not in ("mi_context_order", "mi_paged_attn_decode_fused_ordered"):
+            return getattr(self.lib, name)
+        return lambda *a: self.calls.append((name, a)) or 0
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    rec = _Recorder(_C.lib)
+    monkeypatch.setattr(ops, "lib", rec)
+    monkeypatch.setattr(ops, "require_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "stream", lambda: 0)
+    return rec.calls
+
+
+def test_shallow_models_make_no_order(calls):
+    lens = torch.full((64,), 500, dtype=torch.int32)
+    assert ops.context_order(lens, 8, 1) is None and ops.context_order(lens, 8, ops.CONTEXT_ORDER_LAYERS - 1) is None and not calls
+    assert ops.context_order(lens, 8, ops.CONTEXT_ORDER_LAYERS) is not None and ops.context_order(lens, 8) is not None and len(calls) == 2
+    assert ops.context_order(lens, 4, 28) is None and len(calls) == 2
