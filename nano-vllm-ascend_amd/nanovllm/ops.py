@@ -129,7 +129,7 @@ def paged_attn_decode_fused(qkv, q_w, k_w, eps: float, positions, cos_sin, slots
     """q/k-norm + RoPE + KV store of the step's token + paged decode attention in ONE launch, straight
     from the packed qkv rows (bit-identical to qknorm_rope_store followed by paged_attn_decode, with order =
     context_order(context_lens) too)."""
-    require_gpu(qkv, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables, context_lens)
+    require_gpu(qkv, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables, context_lens, order)
     _bf16(qkv, k_cache, v_cache, q_w, k_w)
     batch = qkv.shape[0]
     assert qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] == (n_q_heads + 2 * n_kv_heads) * HEAD_DIM
