@@ -677,9 +677,11 @@ static int head_stream_grid(int M) { return M <= 32 ? kHeadStreamGrid : kHeadStr
 
 // fp8 weights, more than 64 rows in chunks of 64, each a pass over the weights.  us at 151936 x 1024, pick, gemm_skinny_kernel's workgroups
 // (which fetch all of x again for every 16 or 32 KiB of weights) / these: 16 rows 39.9 / 39.4 (without pick 31.0 / 32.6), 32 rows 51 / 46, 64 rows
-// 105 / 55, 65 rows 176 / 93, 200 rows 356 / 181; 896 deep: 32 rows 44 / 41 (35.8 / 37.0), 48 rows 80 / 46; 2048 deep: 32 rows 83 / 83.
+// 105 / 55, 65 rows 176 / 93, 200 rows 356 / 181; 896 deep: 32 rows 44 / 41 (35.8 / 37.0), 48 rows 80 / 46; 2048 deep: 32 rows 83 / 83.  17 to 32 rows
+// of fewer features leave these workgroups too short a share (their time of gemm_skinny_kernel's, 24 rows, without pick / with: 65536 features 1.08 /
+// 1.05, 114688 1.03 / 1.03, 131072 0.95 / 0.95, 151936 0.98 / 0.96).
 static bool head_stream_fp8_fits(int M, int N, int K) {
-  return (K == 1024 && M > 16 && head_stream_fits(32, N, K)) || (K == 896 && M > 32 && head_stream_fits(M, N, K));
+  return (K == 1024 && M > (N >= 131072 ? 16 : 32) && head_stream_fits(32, N, K)) || (K == 896 && M > 32 && head_stream_fits(M, N, K));
 }
 
 template <bool PICK, int WF = 1>
@@ -690,19 +692,18 @@ static void launch_head_stream(const uint16_t* x, const uint16_t* w, uint16_t* y
   hipLaunchKernelGGL((head_stream_kernel<MT, 2, WAVES, STEPS, PICK, WF>), grid, dim3(WAVES * 64), 0, st, x, w, y, \
                      M, N, K, N / 32, pk, scale)
   const int mt = (min(M, kSkinnyRows) + 15) / 16;
-  if (K == 1024) {
-    if (WF == 1 && mt == 1) MI_HEAD_LAUNCH(1, 8, 4);
-    else if (mt == 2) MI_HEAD_LAUNCH(2, 8, 4);
-    else if (mt == 3) MI_HEAD_LAUNCH(3, 8, 4);
-    else MI_HEAD_LAUNCH(4, 8, 4);
-  } else if (K == 896) {
-    if (mt == 1) MI_HEAD_LAUNCH(1, 7, 4);
-    else if (mt == 2) MI_HEAD_LAUNCH(2, 7, 4);
-    else MI_HEAD_LAUNCH(3, 7, 4);
-  } else if constexpr (WF == 1) {  // 2048
-    if (mt == 1) MI_HEAD_LAUNCH(1, 8, 8);
-    else MI_HEAD_LAUNCH(2, 8, 8);
+  if constexpr (WF == 1) {   // (fp8: from 17 rows on, and from 33 at K 896)
+    if (K == 1024 && mt == 1) MI_HEAD_LAUNCH(1, 8, 4);
+    else if (K == 896 && mt == 1) MI_HEAD_LAUNCH(1, 7, 4);
+    else if (K == 896 && mt == 2) MI_HEAD_LAUNCH(2, 7, 4);
+    else if (K == 2048 && mt == 1) MI_HEAD_LAUNCH(1, 8, 8);
+    else if (K == 2048) MI_HEAD_LAUNCH(2, 8, 8);
+    if (K == 2048 || mt == 1 || (K == 896 && mt == 2)) return;
   }
+  if (K == 896) MI_HEAD_LAUNCH(3, 7, 4);
+  else if (mt == 2) MI_HEAD_LAUNCH(2, 8, 4);
+  else if (mt == 3) MI_HEAD_LAUNCH(3, 8, 4);
+  else MI_HEAD_LAUNCH(4, 8, 4);
 #undef MI_HEAD_LAUNCH
 }
 
