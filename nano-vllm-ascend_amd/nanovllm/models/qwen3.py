@@ -306,13 +306,14 @@ class Qwen3Model(nn.Module):
 
     def _forward_streaming(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """<= ops.SKINNY_MAX_M (512) tokens - every decode step, and short prefills - in chunks of 64 rows inside the
-        kernels: SEVEN launches per layer (the reference's eager decode layer
+        kernels: SEVEN launches per layer, FIVE in decode steps of up to four rows (the reference's eager decode layer
         is ~13):
           add+RMSNorm (summing the previous projection's split-K partials)      (mi_add_rmsnorm_splitk)
           -> packed qkv GEMM                                                     (mi_gemm_bf16_packed)
           -> q/k-norm + RoPE + KV store + paged attention in one launch          (mi_paged_attn_decode_fused)
           -> split-K o_proj -> add+RMSNorm -> gate_up GEMM + SwiGLU epilogue -> split-K down_proj
-        (above 64 rows the bf16 projections are tile GEMMs on the weights as stored: ops.gemm_tile, ops.gemm_tile_splitk).
+        (up to four rows the norms and the merge of the attention's splits are in the next projection's operand load, where that pays:
+        ops.norm_few_pays, ops.merge_few_pays; above 64 rows the bf16 projections are tile GEMMs on the weights as stored: ops.gemm_tile, ops.gemm_tile_splitk).
         MI355_ATTN_FUSED=0 keeps q/k-norm+RoPE+store as its own launch (mi_qknorm_rope_store).
         With tensor parallelism the two row-parallel projections produce bf16 partial sums as complete
         rows (mi_gemm_bf16_rows4); the all-reduce over the ranks (linear.py:149-153) and the following
@@ -336,7 +337,7 @@ class Qwen3Model(nn.Module):
                       and os.environ.get("MI355_XGMI_FUSED", "1") != "0")
 
         def attend(attn, qkv, o_ksplit=0):
-            """The attention's rows - or, with o_ksplit, o_proj's K-slice sums over them (ops.merge_few_takes)"""
+            """The attention's rows - or, with o_ksplit, o_proj's K-slice sums over them (ops.merge_few_pays)"""
             if not attn.attn.fusable:  # head_dim 64 / groups of 7 / the plain-layout family: one launch per operator
                 return attn._attend_unfused(positions, qkv).flatten(1, -1)
             if not fuse_attn:
@@ -393,7 +394,7 @@ class Qwen3Model(nn.Module):
 
         def norm_linear(y, is_partials, res, ln, lin, silu_mul=False):
             """linear(rmsnorm(y + res)) -> (out, new residual)"""
-            if is_partials is True and ops.norm_few_takes(rows, y.shape[0], lin.weight_packed, silu_mul):
+            if is_partials is True and ops.norm_few_pays(rows, y.shape[0], lin.weight_packed, silu_mul):
                 return ops.gemm_norm_few(y, res, ln.weight, ln.eps, lin.weight_packed, silu_mul)
             x, res = add_norm(y, is_partials, res, ln)
             return column_parallel(x, lin, silu_mul), res
@@ -427,7 +428,7 @@ class Qwen3Model(nn.Module):
             else:
                 qkv, residual = norm_linear(parts, is_partials, residual, ln1, attn.qkv_proj)
             ks = self._ksplit(attn.o_proj.weight)
-            if fuse_attn and not exchange and attn.attn.fusable and ops.merge_few_takes(rows, attn.num_kv_heads, attn.o_proj.weight_packed, ks):
+            if fuse_attn and not exchange and attn.attn.fusable and ops.merge_few_pays(rows, attn.num_kv_heads, attn.o_proj.weight_packed, ks):
                 parts, is_partials = attend(attn, qkv, ks), True
             else:
                 parts, is_partials = row_parallel(attend(attn, qkv), attn.o_proj)

@@ -713,9 +713,25 @@ def _packed(w_packed):
 
 
 def norm_few_takes(rows: int, nsplit: int, w_packed, silu_mul: bool) -> bool:
+    """What gemm_norm_few takes (K / 64 waves are one workgroup: at most 1024 columns)"""
     n, k = w_packed.shape
     unit = 32 if silu_mul else 16
     return rows <= FEW_ROWS_MAX and nsplit in (2, 4, 8) and k in (512, 768, 1024) and n % unit == 0 and n // unit < 2048
+
+
+def norm_few_pays(rows: int, nsplit: int, w_packed, silu_mul: bool) -> bool:
+    """... and is not slower than the two launches.  Each workgroup reads the norm's whole operand, 4 nsplit + 2 bytes per element and row: of the two
+    launches' time, whatever the rows, K 1024 with four sums 0.83 to 0.87 for up to 4096 features, 0.91 to 1.0 for 8192 (38 MB), 1.04 for 12288,
+    1.2 to 1.3 for 16384; eight sums 0.94 for 4096, 1.15 for 8192; K 768 with four 0.87 for 8192, 1.01 for 12288; K 512 with eight 0.87 and
+    0.95 to 1.03.  With SwiGLU at K 1024 the waves' sums of both weights weigh more: four sums 0.90 to 0.95 for up to 8192 features (19 MB), 1.01 for
+    12288; eight 1.0 to 1.15, and fp8 weights, half the bytes to hide the norm under, 0.98 to 1.01 with two sums, 1.0 to 1.08 with four."""
+    if not norm_few_takes(rows, nsplit, w_packed, silu_mul):
+        return False
+    n, k = w_packed.shape
+    reads = n // (32 if silu_mul else 16) * FEW_ROWS_MAX * k * (4 * nsplit + 2)
+    if silu_mul and k == 1024:
+        return not isinstance(w_packed, Fp8Weight) and nsplit <= 4 and reads <= 24 << 20
+    return reads <= 38 << 20
 
 
 def gemm_norm_few(partials, residual, w, eps: float, w_packed, silu_mul: bool = False):
@@ -735,10 +751,17 @@ def gemm_norm_few(partials, residual, w, eps: float, w_packed, silu_mul: bool = 
 
 
 def merge_few_takes(rows: int, n_kv_heads: int, w_packed, ksplit: int) -> bool:
-    """Does o_proj weigh the splits of the attention in front of it itself?"""
+    """Can o_proj weigh the splits of the attention in front of it itself?"""
     n, k = w_packed.shape
     return (rows <= FEW_ROWS_MAX and lib.mi_paged_attn_decode_splits(rows, n_kv_heads) > 1 and k % (64 * ksplit) == 0 and k % HEAD_DIM == 0
             and k // (64 * ksplit) in (4, 8, 12, 16) and n % 16 == 0 and n // 16 * ksplit < 2048)
+
+
+def merge_few_pays(rows: int, n_kv_heads: int, w_packed, ksplit: int) -> bool:
+    """... and is not slower than the merge's launch: sixteen waves (1024 columns a workgroup) of three or four rows read more than it saves (of the two
+    launches' time, contexts of 20 / 128 / 600 / 1500 keys, 16 heads, 2048 features: three rows 1.08 / 1.08 / 1.03 / 0.97, two 0.86 / 0.87 / 0.84 /
+    0.81; eight waves, 1024 features: three rows 0.95 / 0.96 / 0.92 / 0.86, four 0.88 / 0.90 / 0.87 / 0.82)"""
+    return merge_few_takes(rows, n_kv_heads, w_packed, ksplit) and (rows <= 2 or w_packed.shape[1] // (64 * ksplit) < 16)
 
 
 def paged_attn_few_proj(qkv, q_w, k_w, eps: float, positions, cos_sin, slots_2d, k_cache, v_cache, block_tables, context_lens,

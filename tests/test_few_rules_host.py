@@ -1,0 +1,26 @@
+"""Where a decode step of a few rows has its norms and the merge of its contexts' splits in the next projection's operand load."""
+import pytest
+import torch
+
+from nanovllm import ops
+
+
+def _w(n, k, fp8=False):
+    return ops.Fp8Weight(torch.empty(0), torch.empty(0), (n, k)) if fp8 else torch.empty(n, k, dtype=torch.bfloat16, device="meta")
+
+
+@pytest.mark.parametrize("nsplit,n,k,silu,fp8,pays", [(4, 4096, 1024, False, False, True), (4, 8192, 1024, False, True, True), (4, 12288, 1024, False, False, False),
+                                                      (8, 4096, 1024, False, False, True), (8, 6144, 1024, False, False, False), (4, 6144, 1024, True, False, True),
+                                                      (4, 6144, 1024, True, True, False), (4, 12288, 1024, True, False, False), (8, 6144, 1024, True, False, False),
+                                                      (8, 8192, 512, False, False, True), (8, 16384, 512, False, False, False), (4, 8192, 768, False, False, True),
+                                                      (8, 16384, 512, True, True, True), (4, 4096, 2048, False, False, False)])
+def test_norm(nsplit, n, k, silu, fp8, pays):
+    for rows in (1, 2, 3, 4):
+        assert ops.norm_few_pays(rows, nsplit, _w(n, k, fp8), silu) == pays
+    assert not ops.norm_few_pays(ops.FEW_ROWS_MAX + 1, nsplit, _w(n, k, fp8), silu)
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,n,ksplit,pays", [(1, 16, 8, 2048, 2, True), (2, 16, 8, 2048, 2, True), (3, 16, 8, 2048, 2, False), (4, 32, 8, 1024, 4, False),
+                                                               (4, 16, 8, 1024, 4, True), (3, 12, 4, 768, 2, True), (4, 8, 8, 1024, 4, True), (5, 8, 8, 1024, 4, False)])
+def test_merge(rows, heads, kv_heads, n, ksplit, pays):
+    assert ops.merge_few_pays(rows, kv_heads, _w(n, heads * 128), ksplit) == pays
