@@ -43,7 +43,8 @@ def test_norm_few_refuses():
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("heads,kv_heads,ksplit", [(16, 8, 4), (8, 2, 2), (16, 8, 1)])
+# 8, 8, 4, 12, 16 and 8 waves; the last with four splits at four rows
+@pytest.mark.parametrize("heads,kv_heads,ksplit", [(16, 8, 4), (8, 2, 2), (8, 8, 4), (12, 3, 2), (16, 8, 2), (16, 16, 4)])
 @pytest.mark.parametrize("lens", [[1], [16], [33, 0], [300, 17, 1], [128, 2047, 64, 1], [5, 700, 31, 32]])
 def test_merge_few(lens, heads, kv_heads, ksplit, fp8):
     """Contexts of no, one and many splits with keys; a length of 0 (a padding row of a captured batch) gives a zero row"""
@@ -72,7 +73,16 @@ def test_merge_few(lens, heads, kv_heads, ksplit, fp8):
     rest = (table, ctx, heads, kv_heads, block, D ** -0.5)
     k2, v2 = kc.clone(), vc.clone()
     want = ops.gemm_packed_splitk(ops.paged_attn_decode_fused(qkv, *args, k2, v2, *rest), w, ksplit)
-    if not ops.merge_few_takes(B, kv_heads, w, ksplit):
-        pytest.skip("not split, or slices no wave count takes")
+    assert ops.merge_few_takes(B, kv_heads, w, ksplit)
     got = ops.paged_attn_few_proj(qkv, *args, kc, vc, *rest, w, ksplit)
     assert torch.equal(kc, k2) and torch.equal(vc, v2) and torch.equal(got, want)
+
+
+def test_merge_few_refuses():
+    from nanovllm import ops
+
+    w = _pack(_rand(256, 2048), False)
+    assert not ops.merge_few_takes(1, 8, w, 1)     # 32 waves
+    assert not ops.merge_few_takes(1, 8, w, 16)    # 2 waves
+    assert not ops.merge_few_takes(ops.FEW_ROWS_MAX + 1, 8, w, 4)
+    assert not ops.merge_few_takes(4, 64, w, 4)    # contexts in one piece
