@@ -360,7 +360,7 @@ extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_tok
 
 // tokens: the rows of x (0: not known).  Where the pairs are at least as many, x is rounded to bf16 a token at a time and the first
 // product's feed gathers the pairs' rows; else the operand pass writes them out in the experts' order (65536 pairs of 8192 tokens x 2048,
-// us: pass 112 + product 459, now 15 + 441).
+// us: pass 112 + product 459, now 15 + 441; 48 to 2000 pairs of 2 to 16 experts, both products: 0.97 to 1.01 of the time, 0.99 on average).
 extern "C" int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, const int32_t* pair_token, const mi_bf16* w,
                                    const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale,
                                    const int32_t* row_scale_rows, const int32_t* offsets, const int32_t* pair_index, int pairs, int G,

@@ -1198,13 +1198,9 @@ def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_in
         assert w.is_contiguous() and down.is_contiguous() and (w2 is None or (w2.shape == w.shape and w2.is_contiguous() and w2.dtype == _BF16))
         scratch = torch.empty(n, dtype=torch.uint8, device=x.device)
         y = torch.empty((pairs, width), dtype=_F32, device=x.device)
-        args = (ptr(w), ptr(w2), ptr(down), int(act), float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets), ptr(pair_index),
-                pairs, G, ff, width, ptr(scratch), n, ptr(y), stream())
-        ldx = x.stride(0) if x.shape[0] > 1 else width
-        if pairs <= 256:   # (its operand pass costs a launch and no more: 400 pairs of 1024 columns 24.8 us, gathered by the product 24.6)
-            check(lib.mi_expert_ff(ptr(x), ldx, ptr(pair_token), *args), "mi_expert_ff")
-        else:
-            check(lib.mi_expert_ff_tokens(ptr(x), ldx, x.shape[0], ptr(pair_token), *args), "mi_expert_ff_tokens")
+        check(lib.mi_expert_ff_tokens(ptr(x), x.stride(0) if x.shape[0] > 1 else width, x.shape[0], ptr(pair_token), ptr(w), ptr(w2),
+                                      ptr(down), int(act), float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets),
+                                      ptr(pair_index), pairs, G, ff, width, ptr(scratch), n, ptr(y), stream()), "mi_expert_ff_tokens")
         return y
     a = gemm_any_grouped_glu(x, pair_token, w, w2, act, limit, row_scale, row_scale_rows, offsets, pairs, None, pairs)
     return gemm_any_grouped(a, None, down, None, offsets, pairs, pair_index, pairs)

@@ -7,13 +7,13 @@ from nanovllm import _C, ops
 
 
 class _Recorder:
-    """mi_gemm_any_operand / mi_gemm_any_tile recorded, everything else the library's own"""
+    """mi_gemm_any_operand / mi_gemm_any_tile / mi_expert_ff_tokens recorded, everything else the library's own"""
 
     def __init__(self, lib):
         self.lib, self.calls = lib, {}
 
     def __getattr__(self, name):
-        if name not in ("mi_gemm_any_operand", "mi_gemm_any_tile", "mi_expert_ff"):
+        if name not in ("mi_gemm_any_operand", "mi_gemm_any_tile", "mi_expert_ff_tokens"):
             return getattr(self.lib, name)
         return lambda *a: self.calls.__setitem__(name, a) or 0
 
@@ -78,7 +78,7 @@ def test_expert_feed_forward_takes_the_operands_that_the_two_products_take(recor
     i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
     args = (x, i32(T * top), gate, gate, down, _C.ACT_CLAMPED_GLU, i32(G + 1), T * top, i32(T * top), 7.0)
     ops.expert_ff(*args, torch.ones(T, top), i32(T * top))
-    assert "mi_expert_ff" in recorded
+    assert "mi_expert_ff_tokens" in recorded
     recorded.clear()
     with pytest.raises(AssertionError):
         ops.expert_ff(*args, torch.ones(T, 2 * top)[:, :top], i32(T * top))
