@@ -563,12 +563,12 @@ __global__ __launch_bounds__(256) void linear_prepare_kernel(LinearArgs a) {
 }
 
 // grid: (sequences, heads, value columns / 64); a wave takes 16 columns, its S as blocks_walk_kernel's.  Ring of three records by LDS-DMA
-// two blocks ahead (two where three do not fit), with the rows' values behind each.
+// two blocks ahead, with the rows' values behind each.
 template <int DT>
 __global__ __launch_bounds__(256, 1) void linear_walk_kernel(LinearArgs a) {
   constexpr int DP = 16 * DT, REC = lin_record_floats(DP), PIECES = REC / 256, PP = (PIECES + 3) / 4, IMG = REC * 4 + 4096;
-  constexpr int NST = 3 * IMG <= 163840 ? 3 : 2;
-  __shared__ __attribute__((aligned(1024))) char lds[NST * IMG];
+  static_assert(3 * IMG <= 163840, "three records");
+  __shared__ __attribute__((aligned(1024))) char lds[3 * IMG];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
   const int s = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 64 + wave * 16 + r16;
@@ -624,16 +624,16 @@ __global__ __launch_bounds__(256, 1) void linear_walk_kernel(LinearArgs a) {
     op += (int64_t)kB * a.ldo;
   };
 #pragma unroll
-  for (int i = 0; i + 1 < NST; ++i) issue(i, i);
+  for (int i = 0; i < 2; ++i) issue(i, i);
   int cur = 0;
   for (int b = 0; b < nb; ++b) {
-    // record b has landed (a ring of three: record b + 1's requests may be out); everybody is done with record b - 1: its place is free
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * (PP + 4)) : "memory");
+    // record b has landed (record b + 1's requests may be out); everybody is done with record b - 1: its place is free
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PP + 4) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     if (b > 0) store(b - 1);   // (here, not behind the block: the wait above would have to see them home)
-    issue(b + NST - 1, cur == 0 ? NST - 1 : cur - 1);
+    issue(b + 2, cur == 0 ? 2 : cur - 1);
     const char* const img = lds + cur * IMG;
-    cur = cur == NST - 1 ? 0 : cur + 1;
+    cur = cur == 2 ? 0 : cur + 1;
     const char* const rec_q = img + lane * 16;
     const char* const rec_k = rec_q + DP * kB * 4;
     const char* const rec_b = rec_k + DP * kB * 4;
