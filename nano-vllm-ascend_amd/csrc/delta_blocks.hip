@@ -397,9 +397,10 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
 //
 // What bounds it: the row-by-row walk reads q, k (and g) of every row for every value column from LDS, 0.38 - 0.42 us a row; here 72 matrix
 // instructions (128 channels) are 1.0 us per sixteen rows, with the LDS reads and sums between them 2.3.  8 sequences of 1024 rows, 16
-// heads of 128 x 128: a decay per head 399 us row by row, 212 so (preparation 68); per channel 458, 253 (109).  rms error against 64
-// bits, row by row = 1 (64 to 1024 rows; D 64, 128, 256): gates around 1/2 0.86 - 0.89, decays of 1 - 2^-5 and slower 0.59 - 0.84,
-// four random decays between 0 and 1 0.94 - 1.06.
+// heads of 128 x 128: a decay per head 399 us row by row, 205 so (preparation 68); per channel 458, 235 (109).  rms error against 64
+// bits, row by row = 1 (128 and 300 rows; D 64, 128, 256; means of six inputs): forget gates 0.82 - 0.86, decays of 1 - 2^-5 and slower 0.64 - 0.87,
+// one decay of 0.3 to 0.8 0.81 - 0.87, of 0.95 0.79 - 0.90.  (B's products of q and k summed over the lanes in 32 bits: 1.01 - 1.08 for decays up to
+// 0.7, whose rows are little else, and 1 to 4 % less time; the lanes' few products each are.)
 // ---------------------------------------------------------------------------
 constexpr int lin_record_floats(int dp) { return (2 * dp * kB + 512 + 2 * dp + 255) & ~255; }
 
@@ -420,6 +421,11 @@ struct LinearArgs {
   float* out;
   int64_t ldo;
 };
+
+template <int O>   // v + the value of lane ^ O, without the LDS crossbar
+__device__ __forceinline__ double xor_sum64(double v) {
+  return v + __hiloint2double(__float_as_int(xor_get<O>(__int_as_float(__double2hiint(v)))), __float_as_int(xor_get<O>(__int_as_float(__double2loint(v)))));
+}
 
 __device__ __forceinline__ float silu_if(bool on, float z) { return on ? z / (1.f + expf(-z)) : z; }
 
@@ -481,8 +487,8 @@ __global__ __launch_bounds__(256) void linear_prepare_kernel(LinearArgs a) {
   // ---- B: sixteen lanes per j walk t = 0..15, four channels at a time, with p = k_j P_jt (0 before t = j); one decay per head: with k_j,
   // and the sum times the decay's power ----
   {
-    using T = std::conditional_t<FORGET, double, float>;
     const int j = tid >> 4, c = (tid & 15) * 4;
+    using T = std::conditional_t<FORGET, double, float>;
     T p[C][4];
 #pragma unroll
     for (int i = 0; i < C; ++i) {
@@ -507,14 +513,8 @@ __global__ __launch_bounds__(256) void linear_prepare_kernel(LinearArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] += p[i][e] * q[e];
       }
-      T b = (sum[0] + sum[1]) + (sum[2] + sum[3]);
-      if constexpr (FORGET) {
-#pragma unroll
-        for (int o = 1; o < 16; o *= 2) b += __shfl_xor(b, o);
-      } else {
-        b = xor_sum<8>(xor_sum<4>(xor_sum<2>(xor_sum<1>(b))));
-      }
-      const double bp = t < j ? 0. : FORGET ? (double)b : b * power;
+      const double b = xor_sum64<8>(xor_sum64<4>(xor_sum64<2>(xor_sum64<1>(((double)sum[0] + sum[1]) + ((double)sum[2] + sum[3])))));
+      const double bp = t < j ? 0. : FORGET ? b : b * power;
       if (c == 0) bm[t][j] = (float)bp, bl[t][j] = (float)(bp - (float)bp);
     }
   }
