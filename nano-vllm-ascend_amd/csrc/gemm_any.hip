@@ -5,7 +5,7 @@
 // (bf16 products of more rows than any_stream_takes says - K a multiple of 64, no segments - go to gemm_any_tile.hip.)
 //
 // These serve the model families whose residual stream, norms and recurrences are kept in 32-bit floats and whose
-// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): nine kernels,
+// widths are not the fragment-native kernels' (csrc/gemm_skinny*.hpp, gemm_tile.hip): ten kernels,
 //
 //   gemm_any_mfma_kernel   bf16 weights: a 64 x 64 (from 512 rows: 128 x 128, with SwiGLU 128 x 64) output tile per 4-wave
 //                          workgroup, x rounded to bf16 on its way into LDS, v_mfma_f32_16x16x32_bf16, the next K
@@ -14,6 +14,7 @@
 //                          workgroup, the waves split K, fragments straight from memory
 //   gemm_any_stream_kernel bf16 weights, 9 to 64 rows and experts of few rows each, K a multiple of 64: the same work with two 64-deep
 //                          blocks in flight per wave and whole lines through LDS
+//   gemm_any_stream_groups_kernel  the same for more than 96 rows of experts, whose shares may be uneven
 //   gemm_any_heads_kernel  bf16 weights, the batched form over many rows (a head's projection of its own columns): the head's weight in
 //                          LDS, x rows straight into operands
 //   gemm_any_f32_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, on the fp32 matrix instruction
@@ -796,27 +797,25 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_kernel(GemmAnyArgs
   stream_rows<DUAL, MF, RT, WAVES, EXT>(a, lds, w, w2, m_lo, m_hi);
 }
 
-// Groups, sixteen rows per workgroup: the first n_groups (blockIdx.z) take their group's first ones, those behind share what is left - of the few
-// groups that have more than the others, or of a step whose pairs go to one expert.  A group as one workgroup's walk, whatever it has: 757
-// pairs on one of 128 experts of 512 x 512 212 us, so 24 (tile kernels 19); 512 on two of 64 of 768 x 2048 230 / 52 (30); shared as a router
-// does, 256 pairs of those 108 / 105 (125).  32 or 64 rows at a time for what is left hold registers and LDS that the first rows then lack (126
-// and 160 us for 512 pairs, eight each; so 112).
+// Groups, sixteen rows per workgroup: the last n_groups (blockIdx.z) take their group's first ones, the a.M in front of them share what is left - of the
+// few groups that have more than the others, or of a step whose pairs go to one expert (in front: behind them it was 0.3 to 0.5 us at the
+// launch's end, where there is nothing left).  us, both products, a group as one workgroup's walk | so | tile kernels: 757 pairs on one of 128 experts
+// of 512 x 512 212 | 22 | 19; 512 on two of 64 of 768 x 2048 153 | 55 | 30; 32 equal tokens' 256 on eight of those 37 | 34 | 29; shared as a
+// router does, 256 pairs of those 104 | 104 | 125.  32 or 64 rows at a time for what is left hold registers and LDS that the first rows then lack (512
+// pairs, eight each: 126 and 160 us, so 113).
 template <bool DUAL, int RT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void gemm_any_stream_groups_kernel(GemmAnyArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[WAVES * stream_slot(DUAL ? 2 : RT, 1)];
-  int m_lo, m_hi;
-  const uint16_t *w, *w2;
-  const int share = (int)gridDim.z - a.n_groups;
-  if ((int)blockIdx.z < a.n_groups) {
-    select_group<uint16_t, DUAL>(a, w, w2, m_lo, m_hi);
-    stream_rows<DUAL, 1, RT, WAVES, false>(a, lds, w, w2, m_lo, share ? min(m_hi, m_lo + 16) : m_hi);
+  const int share = a.M, own = (int)blockIdx.z - share;   // (among the first arguments: the grid's size is a line of its own)
+  auto weights = [&](const void* w, int g) { return static_cast<const uint16_t*>(w) + (int64_t)g * a.N * a.K; };
+  int g, m_lo, m_hi;
+  if (own >= 0) {
+    m_lo = a.group_offsets[own], m_hi = a.group_offsets[own + 1];
+    stream_rows<DUAL, 1, RT, WAVES, false>(a, lds, weights(a.w, own), DUAL ? weights(a.w2, own) : nullptr, m_lo, share ? min(m_hi, m_lo + 16) : m_hi);
     return;
   }
-  int g;
-  for (int piece = (int)blockIdx.z - a.n_groups; group_tile<16, 16>(a.group_offsets, a.n_groups, piece, g, m_lo, m_hi); piece += share) {
-    w = static_cast<const uint16_t*>(a.w) + (int64_t)g * a.N * a.K;
-    w2 = DUAL ? static_cast<const uint16_t*>(a.w2) + (int64_t)g * a.N * a.K : nullptr;
-    stream_rows<DUAL, 1, RT, WAVES, false>(a, lds, w, w2, m_lo, min(m_hi, m_lo + 16));
+  for (int piece = blockIdx.z; group_tile<16, 16>(a.group_offsets, a.n_groups, piece, g, m_lo, m_hi); piece += share) {
+    stream_rows<DUAL, 1, RT, WAVES, false>(a, lds, weights(a.w, g), DUAL ? weights(a.w2, g) : nullptr, m_lo, min(m_hi, m_lo + 16));
     __syncthreads();  // (the sums are read)
   }
 }
@@ -1047,12 +1046,24 @@ static int launch_stream(const GemmAnyArgs& args, int groups, int rows, hipStrea
   };
   // groups and batches: workgroups enough, four waves each, so that several share a CU (eight: 256 pairs over 64 experts' second product 55
   // us, four 37)
-  if (a.group_offsets) {
-    if constexpr (EXT) return MI_EUNSUPPORTED;   // (no group has the extended epilogue)
-    z = groups + std::min(rows / 16, 65535 - groups);   // (`rows` rows in all have no more sixteens beyond a group's first)
-    if constexpr (!DUAL && !EXT)
-      if ((int64_t)(a.N / 16) * groups >= 2048) return go(gemm_any_stream_groups_kernel<false, 2, 4>, 2, 4);
-    if constexpr (!EXT) return go(gemm_any_stream_groups_kernel<DUAL, 1, 4>, 1, 4);
+  if (a.group_offsets) {   // (no group has the extended epilogue)
+    // up to 96 rows a group's own workgroups walk them all, six times sixteen at most: the choice costs every launch 0.3 us (96 pairs, 32 experts of
+    // 512 x 1024: 24.0 us so, 24.6)
+    const bool wide = !DUAL && (int64_t)(a.N / 16) * groups >= 2048;
+    if constexpr (!EXT) {
+      if (rows <= 96) {
+        if constexpr (!DUAL)
+          if (wide) return go(gemm_any_stream_kernel<false, 1, 2, 4, false>, 2, 4);
+        return go(gemm_any_stream_kernel<DUAL, 1, 1, 4, false>, 1, 4);
+      }
+      // (`rows` rows in all have at most twice as many sixteens beyond a group's first, and seldom as many: few stay without one)
+      a.M = std::min((rows + 31) / 32, 65535 - groups);
+      z = groups + a.M;
+      if constexpr (!DUAL)
+        if (wide) return go(gemm_any_stream_groups_kernel<false, 2, 4>, 2, 4);
+      return go(gemm_any_stream_groups_kernel<DUAL, 1, 4>, 1, 4);
+    }
+    return MI_EUNSUPPORTED;
   }
   const int mf = (rows + 15) / 16;
   if constexpr (!DUAL && !EXT) {   // (no batch has two weights or the extended epilogue)

@@ -143,6 +143,8 @@ static bool tile_rows_ok(int t) { return t == 64 || t == 128 || t == 256; }
 // the row tiles of `rows` rows in at most n_groups groups (0: one, its tiles known)
 static int64_t row_tiles(int rows, int n_groups, int t) { return n_groups ? rows / t + n_groups : (rows + t - 1) / t; }
 
+// (Reached by operands that the streaming kernel does not take - x off 16 bytes -, and by mi_expert_ff_bytes, which is 0 here: these products are
+// two calls.)
 // Few pairs over small experts: the operand pass and the rings' first round trips are longer than the general kernels' whole walk (us with
 // weights not in the L2s, both products, general / tile kernels: 8 experts of 256 x 1024, 64 pairs 15.8 / 18.2; 16 of 256 x 512, 96 pairs
 // 12.0 / 14.8; 32 of 256 x 512, 32 pairs 13.3 / 14.7, 48 pairs 16.6 / 14.6; 128 of 256 x 256, 24 pairs 12.4 / 13.3; 8 of 512 x 1024,
