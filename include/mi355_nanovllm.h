@@ -812,7 +812,7 @@ int mi_gemm_any_segments(const float* x, int64_t ldx, const void* w, int w_dtype
  * x[x_rows ? x_rows[r] : r] for the rows r before group_offsets[n_groups] (all rows without groups), and the table (may be NULL).
  * mi_gemm_any_tile: y[y_rows ? y_rows[r] : r] = epilogue of mi_gemm_any_act / mi_gemm_any_grouped_glu, fp32 or bf16.
  * mi_gemm_any_streams: 1 where mi_gemm_any_act / _grouped_glu over bf16 weights are faster than these (decode batches, experts of a
- * few rows; x and w on 16 bytes). */
+ * few rows; x and w on 16 bytes; without groups: one weight). */
 int mi_gemm_any_streams(int rows, int N, int K, int n_groups);
 int mi_gemm_any_tile_rows(int rows, int N, int K, int n_groups, int dual, int act);
 int64_t mi_gemm_any_table_ints(int rows, int n_groups, int tile_rows);
