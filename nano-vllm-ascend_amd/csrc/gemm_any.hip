@@ -1179,10 +1179,10 @@ static int launch_any(const GemmAnyArgs& a, int groups, int rows_per_group_max, 
     const int ft = !DUAL && mt > 1 && a.N >= 8192 ? 4 : 1;   // (a wave per four features: from two workgroups per CU on)
     const dim3 grid((a.N + 4 * ft - 1) / (4 * ft), (rows_per_group_max + mt - 1) / mt, groups);
     // From 4096 features on and 12288 sums, in which the layout of the rows and the wide waves pay (us, gemm_any_rows_kernel / here: 2 rows x 4096 x
-    // 2048 7.6 / 8.2, 3 rows 9.0 / 8.1, 8 rows 16.4 / 10.7; 2 x 6144 x 2048 9.8 / 9.0; 5 x 3072 x 2048 9.8 / 10.2); 64 KB of rows at most: two
-    // workgroups on a CU.
+    // 2048 7.6 / 8.2, 3 rows 9.0 / 8.1, 8 rows 16.4 / 10.7; 2 x 6144 x 2048 9.8 / 9.0; 5 x 3072 x 2048 9.8 / 10.2), 16384 where a row of K is one piece (2 x
+    // 6261 x 512 4.4 / 5.0, x 8192 x 512 0.70 of the time); 64 KB of rows at most: two workgroups on a CU.
     if constexpr (!DUAL && sizeof(TW) == 2)
-      if (mt > 1 && rows_per_group_max <= 8 && a.N >= 4096 && (int64_t)a.N * rows_per_group_max >= 12288 && groups == 1 && !a.group_offsets && a.K % 512 == 0 && mt * a.K * 4 <= 65536 && a.ldx % 4 == 0 &&
+      if (mt > 1 && rows_per_group_max <= 8 && a.N >= 4096 && (int64_t)a.N * rows_per_group_max >= (a.K > 512 ? 12288 : 16384) && groups == 1 && !a.group_offsets && a.K % 512 == 0 && mt * a.K * 4 <= 65536 && a.ldx % 4 == 0 &&
           aligned16(a.x) && aligned16(a.w)) {
         const dim3 persistent(std::min(512, (a.N + 31) / 32));
         if (mt == 4) hipLaunchKernelGGL((gemm_any_rows_lds_kernel<4, EXT>), persistent, dim3(512), mt * a.K * 4, st, a);

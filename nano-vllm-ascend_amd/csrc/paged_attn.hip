@@ -1213,7 +1213,8 @@ static int decode_impl(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_
   // 512 - 1100 40.6 -> 39.7; per step of 28 layers: 200 of 30 - 200 2280 -> 2000, 200 of 500 3654 -> 3406, 36 of 500 1454 -> 1355, 128 of 900
   // 3542 -> 3514, 100 of 50 - 2000 3340 -> 3243 (by number 3505).
   // Not where all contexts are long and equal and the units are no multiple of 512: 160 of 2000 keys 204.4 -> 207.4 us a launch (the last round of 512
-  // is a part one more often than one of 256).
+  // is a part one more often than one of 256), nor always for few long and ragged ones, whose longest then has four waves (33 of 100 - 2000 keys, 64 heads,
+  // 28.1 -> 29.5; of 100 - 200 14.1 -> 11.9, 33 of 1000 36.3 -> 32.8).
   if (!fused || nsplit > 1 || (int64_t)batch * n_kv_heads <= 256) order = nullptr;
   float* part_o = static_cast<float*>(workspace);
   float* part_ml = part_o + (size_t)batch * n_q_heads * 16 * 128;
