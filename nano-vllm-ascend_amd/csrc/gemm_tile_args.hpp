@@ -1,6 +1,7 @@
 // What the MFMA tile GEMM kernels (gemm_w16_kernel.hpp, gemm_mid_kernel.hpp, ...) share: arguments and tile order.
 #pragma once
 #include <type_traits>
+#include <utility>
 
 #include "mi_common.hpp"
 #include "gemm_tile_index.hpp"

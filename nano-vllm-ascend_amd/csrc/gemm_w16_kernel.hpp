@@ -8,8 +8,19 @@
 // 1.243 vs 1.313 us per K step, the whole loop with the qkv GEMM's fetch pattern 1.356 vs 1.422).
 //   * wave tile 128 x 128 = 8 x 8 accumulators of 16 x 16 (f32x4 each: 256 registers); a K step is two k halves of 64
 //     MFMAs; the fragments of the next half are read during the current one (two register sets of 8 + 8 fragments,
-//     128 registers - the same lead of ~1000 cycles as "two k groups ahead" above); ONE wait + barrier per K step
-//     behind the first half; the sixteen pieces one behind every fourth MFMA of the second half;
+//     128 registers);
+//   * the K loop is bound by the matrix pipe (2350 cycles a step) only as long as a piece has landed when its step comes,
+//     and what misses the L2 takes 2200 cycles (Infinity Cache) to 3400 (HBM: a weight's first use).  With two images the
+//     time a piece has is what lies between the last read of the image it replaces and the first read of its own, so the
+//     reads stand close together, as far apart from each other as the registers allow: the sixteen of k half 1 in the
+//     first quarter of a step, then a barrier (the image is free), its sixteen pieces one behind every fourth MFMA, the
+//     wait for the NEXT image - issued a whole step ago: a counted wait, this step's pieces stay in flight - and a second
+//     barrier, and the sixteen reads of its k half 0 in the last quarter.  A piece has 0.95 of a step; with one barrier in
+//     the middle and the reads spread over both halves it had 0.5, and a step took 3450 cycles (4600 with cold weights).
+//     us per launch, weights and activations not in the L2s, before -> now: 16384 x 1024 x 2048 88 -> 70, x 3072 121 -> 89,
+//     16384 x 4096 x 1024 139 -> 118, fp32 results 8192 x 2048 x 2048 74 -> 67, 8192 x 8192 x 2048 252 -> 238.  Pieces one
+//     behind every 2 / 3 / 5 MFMAs: 94 / 83 / 100 us where every fourth takes 89 (the L1 feeds 64 bytes a cycle: 8 MFMAs
+//     for the four waves' pieces);
 //   * the MFMAs are inline assembly, in place (`v_mfma ... %0, %1, %2, %0`): with the builtin hipcc gives the result
 //     another register quad than the addend and copies 64 quads around at the loop's back edge.  What the compiler
 //     then no longer knows is handled here: a tile's first MFMA into an accumulator takes the constant 0 as addend
@@ -22,6 +33,11 @@
 // Summation order: one fp32 MFMA chain over K per output element, k ascending - the same bits as every other GEMM here
 // (tests/test_gemm_tile_gpu.py holds the two MFMA shapes against each other and against the library).
 #pragma once
+
+template <class F, int... I>
+__device__ __forceinline__ void w16_slots(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
 
 template <int EPI, bool BIAS, int V, class ARGS = TileArgs>
 __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
@@ -147,45 +163,42 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[f][t]) : "v"(Ra[kh][f]), "v"(Rb[kh][t]));
   };
 
+  // the slots (MFMAs) of a K step: see the head of this file
+  constexpr int kFreed = 38, kPiece0 = 40, kPieceEvery = 4, kLanded = 95, kRead0 = 96;
+  constexpr int kYoung = (kLanded - kPiece0) / kPieceEvery + 1;  // this step's pieces that are in flight at kLanded
+  static_assert(kPiece0 > kFreed && kPiece0 + 15 * kPieceEvery < 128 && kRead0 + 2 * 15 < 128 && kYoung < 16, "the slots of a K step");
   auto kstep = [&](auto first) __attribute__((always_inline)) {
     using First = decltype(first);
-    // first half: MFMAs of k half 0, reads of k half 1 of the same image
-#pragma unroll
-    for (int g = 0; g < 16; ++g) {
-      if constexpr (First::value) {
-        mma_first(0, 4 * g);
-        mma_first(0, 4 * g + 1);
-        read1(1, g);
-        mma_first(0, 4 * g + 2);
-        mma_first(0, 4 * g + 3);
-      } else {
-        mma_acc(0, 4 * g);
-        mma_acc(0, 4 * g + 1);
-        read1(1, g);
-        mma_acc(0, 4 * g + 2);
-        mma_acc(0, 4 * g + 3);
+    w16_slots([&](auto slot) __attribute__((always_inline)) {
+      constexpr int m = decltype(slot)::value;
+      if constexpr (m >= 64) mma_acc(1, m - 64);
+      else if constexpr (First::value) mma_first(0, m);
+      else mma_acc(0, m);
+      if constexpr (m < 32 && m % 2 == 1) {
+        read1(1, m / 2);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // my reads of this image are back, my pieces of the next step have landed (and a previous tile's stores are out)
-    if (V & 128) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    offa += flip;
-    offb += flip;
-    flip = -flip;
-    // second half: k half 1; reads of k half 0 of the NEXT step; the pieces of the step after it
-#pragma unroll
-    for (int g = 0; g < 16; ++g) {
-      mma_acc(1, 4 * g);
-      mma_acc(1, 4 * g + 1);
-      if (!(V & 64)) read1(0, g);
-      __builtin_amdgcn_sched_barrier(0);
-      mma_acc(1, 4 * g + 2);
-      mma_acc(1, 4 * g + 3);
-      if (!(V & 32)) piece(g);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      if constexpr (m == kFreed) {  // my reads of this image are back: everybody's are, behind the barrier
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        offa += flip;
+        offb += flip;
+        flip = -flip;
+      }
+      if constexpr (m >= kPiece0 && (m - kPiece0) % kPieceEvery == 0 && (m - kPiece0) / kPieceEvery < 16) {
+        piece((m - kPiece0) / kPieceEvery);  // of the step after the next
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (m == kLanded) {  // the next step's pieces (and a previous tile's stores) are older than this step's
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kYoung) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (m >= kRead0 && m % 2 == 0) {
+        read1(0, (m - kRead0) / 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }, std::make_integer_sequence<int, 128>{});
     fetch_advance();
   };
 
@@ -206,13 +219,6 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   constexpr int NF = EPI == TEPI_SILU ? 4 : 8;  // output feature fragments of a wave
   // direct form (edge shapes, split-K partials): four features per lane and store
   auto epilogue = [&](int m0, int n0) __attribute__((always_inline)) {
-    if (V & 512) {  // ablation: no output (the accumulators are kept alive by an empty asm)
-#pragma unroll
-      for (int f = 0; f < 8; ++f)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) asm volatile("" ::"a"(acc[f][t]));
-      return;
-    }
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       const int tok = m0 + w16_acc_token(tw, t, n16);
