@@ -7,9 +7,9 @@
 // (gemm_any_mfma_kernel: x converted by every feature tile again, operands through registers into LDS, two barriers per K
 // step) reached 200-350 TFLOP/s; the tile kernels fetch both operands with LDS-DMA, which needs them in bf16 - hence the
 // pass over x, which reads and writes 6 bytes per element once and is paid back from the second feature tile on.
-// Measured, 8192 rows: 2048 x 2048 207 -> 75 us + 15 us of operand pass; 64 experts x 8 per row, 2048 -> 2 x 768 with SwiGLU
-// 1192 -> 523 us (790 TFLOP/s), back to 2048 1050 -> 250 us.  Bits: one fp32 chain over k per result, k ascending, from
-// the same rounded operands as gemm_any_mfma_kernel's - the same bits.
+// Measured, 8192 rows: 2048 x 2048 207 -> 63 us + 15 us of operand pass; 64 experts x 8 per row, 2048 -> 2 x 768 with SwiGLU
+// 1192 -> 410 us (1.0 PFLOP/s), back to 2048 1050 -> 280 us.  Bits: one fp32 chain over k per result, k ascending, from
+// the same rounded operands as gemm_any_mfma_kernel's - the same bits (silu, a form of its own, to an ulp).
 #include "gemm_any_stream.hpp"
 #include "gemm_tile_args.hpp"
 
@@ -63,16 +63,10 @@ __device__ __forceinline__ AnyRow any_row(const A& a, int m, int m_end) {
   if (a.row_scale) r.scale = a.row_scale[a.row_scale_rows ? a.row_scale_rows[m] : m];
   return r;
 }
-// four consecutive features of one row: the epilogue of gemm_any.hip's finish(), operation for operation
+// four consecutive features of one row: the epilogue of gemm_any.hip's finish(), operation for operation but for silu's form (b1, b2:
+// their biases, where the operand has any)
 template <class A>
-__device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, f32x4 v, f32x4 v2) {
-  if (row.y < 0 || n >= a.N) return;
-  if (a.row_scale) {
-    v *= row.scale;
-    if (A::kDual) v2 *= row.scale;
-  }
-  if (a.bias1) v += *reinterpret_cast<const f32x4*>(a.bias1 + n);
-  if (A::kDual && a.bias2) v2 += *reinterpret_cast<const f32x4*>(a.bias2 + n);
+__device__ __forceinline__ f32x4 any_act(const A& a, f32x4 v, f32x4 v2) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float z = v[e];
@@ -81,19 +75,36 @@ __device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, 
       const float g = fminf(z, a.limit), u = fminf(fmaxf(v2[e], -a.limit), a.limit);
       o = g / (1.f + expf(-1.702f * g)) * (u + 1.f);
     } else {
-      if constexpr (A::kAct == MI_ACT_SILU) o = z / (1.f + expf(-z));
+      if constexpr (A::kAct == MI_ACT_SILU) o = silu_f32(z);
       if constexpr (A::kAct == MI_ACT_GELU_TANH) o = 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
       if constexpr (A::kAct == MI_ACT_GELU_ERF) o = 0.5f * z * (1.f + erff(z * 0.7071067811865476f));
-      if constexpr (A::kAct == MI_ACT_SOFTCAP) o = tanhf(z / a.alpha);   // (times alpha below: alpha tanh(z / alpha))
+      if constexpr (A::kAct == MI_ACT_SOFTCAP) o = tanhf(z / a.alpha);   // (times alpha behind: alpha tanh(z / alpha))
       if constexpr (A::kAct == MI_ACT_RELU2) o = fmaxf(z, 0.f) * fmaxf(z, 0.f);
       if (A::kDual) o *= v2[e];
     }
-    v[e] = o * a.alpha;
+    v[e] = o;
   }
+  return v;
+}
+template <class A>
+__device__ __forceinline__ f32x4 any_value(const A& a, float scale, f32x4 v, f32x4 v2, f32x4 b1, f32x4 b2) {
+  if (a.row_scale) {
+    v *= scale;
+    if (A::kDual) v2 *= scale;
+  }
+  if (a.bias1) v += b1;
+  if (A::kDual && a.bias2) v2 += b2;
+  return any_act(a, v, v2) * a.alpha;
+}
+template <class A>
+__device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, f32x4 v, f32x4 v2) {
+  if (row.y < 0 || n >= a.N) return;
+  const f32x4 none = {};
+  v = any_value(a, row.scale, v, v2, a.bias1 ? *reinterpret_cast<const f32x4*>(a.bias1 + n) : none,
+                A::kDual && a.bias2 ? *reinterpret_cast<const f32x4*>(a.bias2 + n) : none);
   if (a.y16) *reinterpret_cast<u32x2*>(a.y16 + row.y * a.ldy + n) = u32x2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
   else *reinterpret_cast<f32x4*>(a.y32 + row.y * a.ldy + n) = v;
 }
-
 
 #include "gemm_w16_kernel.hpp"
 #include "gemm_mid_kernel.hpp"
@@ -200,9 +211,18 @@ static int launch_any_tile(const AnyTileArgs<ACT, DUAL, GATHER>& args, int tile_
     a.tiles_f = (a.N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
     a.tiles_t = (a.M + 255) / 256;
     const int64_t tiles = row_tiles_max * a.tiles_f;
-    if constexpr (ACT != MI_ACT_SOFTCAP)   // (a head's product: never that many rows; it would not fit the persistent kernel's registers)
-      hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 0, A>), dim3((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid)),
-                         dim3(256), 0, st, a);
+    const dim3 grid((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid));
+    // the epilogue's short form takes what the models' projections and experts ask for
+    [[maybe_unused]] const bool lean = !a.row_scale && a.alpha == 1.f && a.N % (DUAL ? 128 : 256) == 0 &&
+                                       (DUAL ? a.y16 && !a.bias1 && !a.bias2 && a.ldy % 8 == 0 : !a.y16);
+    if constexpr (ACT != MI_ACT_SOFTCAP) {  // (a head's product: never that many rows; it would not fit the persistent kernel's registers)
+      if constexpr (DUAL ? ACT == MI_ACT_SILU : ACT == MI_ACT_NONE)
+        if (lean) {
+          hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 32768, A>), grid, dim3(256), 0, st, a);
+          return check_launch();
+        }
+      hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 0, A>), grid, dim3(256), 0, st, a);
+    }
   } else if (tile_rows == 64) {
     // two weights: 128 feature rows (64 outputs); one: 64, or 128 where that leaves at least four tiles per CU (the experts' second
     // product, us, 64 / 128 features: 32 experts of 1024 x 512 8.9 / 9.6, 64 of 2048 x 768 41 / 39.5)

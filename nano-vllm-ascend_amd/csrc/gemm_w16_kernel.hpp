@@ -43,8 +43,10 @@ template <int EPI, bool BIAS, int V, class ARGS = TileArgs>
 __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   constexpr bool LINES = (V & 32768) != 0 && EPI != TEPI_PARTIAL && EPI != TEPI_ANY;
   constexpr bool GATHER = EPI == TEPI_ANY && ARGS::kGather;  // a tile's activation rows wherever x_rows says
+  constexpr bool LEAN = (V & 32768) != 0 && EPI == TEPI_ANY;  // the epilogue's short form: see any_begin
   constexpr bool PAIRED = EPI == TEPI_ANY && ARGS::kDual;  // two weights: half 0 of the A region holds 128 rows of w, half 1 of w2
-  __shared__ __attribute__((aligned(1024))) char lds[2 * W16_STEP_BYTES + (LINES ? 4 * W4_STAGE_BYTES : 0)];
+  constexpr bool WIDE = LEAN && !PAIRED;
+  __shared__ __attribute__((aligned(1024))) char lds[2 * W16_STEP_BYTES + (LINES || WIDE ? 4 * W4_STAGE_BYTES : 0)];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fw = wave >> 1, tw = wave & 1, q4 = lane >> 4, n16 = lane & 15;
@@ -242,14 +244,96 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     }
   };
 
+  // TEPI_ANY.  What the epilogue needs besides the accumulators - the output rows of the lane's tokens with their factors, the features'
+  // biases - is asked for in front of the tile's K steps: a load behind them waits for the pieces and the stores before it, once per
+  // token fragment (an index) or per store (a bias).
+  // What bounds it is issue: one wave per SIMD, no matrix instruction beside it.  LEAN (whole feature tiles; no factor on rows or
+  // results; one weight: fp32 results, no activation; two: bf16 results, no bias) knows at compile time what the rest selects per value
+  // and branches on per store.  us per tile from the last K step to the end, before -> LEAN: one weight 8.0 -> 6.2 (rows by an index
+  // 11.0 -> 6.2), two 14.0 -> 6.3.
+  constexpr int NV = EPI == TEPI_ANY ? (PAIRED ? 4 : 8) : 1, NT = EPI == TEPI_ANY ? (WIDE ? 16 : 8) : 1;
+  int any_y[NT];  // of token fragment t's row n16; WIDE: of the wave's row 8 t + lane / 8
+  float any_scale[NT];
+  f32x4 any_b1[NV], any_b2[PAIRED ? NV : 1];
+  auto any_begin = [&](int m0, int n0, int m_end) __attribute__((always_inline)) {
+    if constexpr (EPI == TEPI_ANY) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int m = m0 + (WIDE ? tw * 128 + 8 * t + (lane >> 3) : w16_acc_token(tw, t, n16)), at = min(m, m_end - 1);
+        const int y = a.y_rows ? a.y_rows[at] : at;
+        any_y[t] = m < m_end ? y : -1;
+        if constexpr (!LEAN) any_scale[t] = a.row_scale ? a.row_scale[a.row_scale_rows ? a.row_scale_rows[at] : at] : 1.f;
+      }
+      if constexpr (!LEAN || !PAIRED) {
+        const int n = n0 + fw * (PAIRED ? 64 : 128) + 4 * q4;
+#pragma unroll
+        for (int f = 0; f < NV; ++f) {
+          const int c = min(n + 16 * f, a.N - 4);
+          any_b1[f] = a.bias1 ? *reinterpret_cast<const f32x4*>(a.bias1 + c) : f32x4{-0.f, -0.f, -0.f, -0.f};  // (x + -0 is x)
+          if constexpr (PAIRED)
+            if (a.bias2) any_b2[f] = *reinterpret_cast<const f32x4*>(a.bias2 + c);
+        }
+      }
+    }
+  };
+  auto any_out = [&](int f, int t) __attribute__((always_inline)) -> f32x4 {
+    if constexpr (EPI == TEPI_ANY) {
+      // (the next tile's first fragments are live here: accumulators copied out early would spill them)
+      if constexpr (PAIRED) asm volatile("" : "+a"(acc[f][t]), "+a"(acc[f + 4][t]));
+      if constexpr (WIDE) return acc[f][t] + any_b1[f];
+      else if constexpr (LEAN) return any_act(a, acc[f][t], acc[f + 4][t]);
+      else return any_value(a, any_scale[t], acc[f][t], acc[PAIRED ? f + 4 : f][t], any_b1[f], any_b2[PAIRED ? f : 0]);
+    }
+    return f32x4{};
+  };
+  auto epilogue_any = [&](int n0) __attribute__((always_inline)) {
+    if constexpr (EPI == TEPI_ANY) {
+      const int n = n0 + fw * (PAIRED ? 64 : 128) + 4 * q4;
+      const bool whole = n0 + (PAIRED ? 128 : 256) <= a.N;
+      if constexpr (LEAN) {
+        // bf16: two fragments' lanes exchanged so that a lane stores eight consecutive features of one of them (through LDS, in whole
+        // lines: 7.3 us)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          uint16_t* const p = a.y16 + any_y[t] * a.ldy + (n - 4 * q4) + 16 * (q4 & 1) + 8 * (q4 >> 1);
+#pragma unroll
+          for (int f = 0; f < NV; f += 2) {
+            const f32x4 u = any_out(f, t), v = any_out(f + 1, t);
+            const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf(u[0], u[1]), pack_bf(v[0], v[1]), false, false);
+            const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf(u[2], u[3]), pack_bf(v[2], v[3]), false, false);
+            if (any_y[t] >= 0) *reinterpret_cast<u32x4*>(p + 16 * f) = u32x4{s0[0], s1[0], s0[1], s1[1]};
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        return;
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int64_t at = any_y[t] * a.ldy + n;
+#pragma unroll
+        for (int f = 0; f < NV; ++f) {
+          const f32x4 v = any_out(f, t);
+          if (any_y[t] >= 0 && (whole || n + 16 * f < a.N)) {
+            if (a.y16) *reinterpret_cast<u32x2*>(a.y16 + at + 16 * f) = u32x2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+            else *reinterpret_cast<f32x4*>(a.y32 + at + 16 * f) = v;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+
   // whole-line form (V & 32768; the host guarantees full feature tiles and 16-byte aligned rows): a slab = 32 tokens
   // (token fragments 2 tt, 2 tt + 1) x 64 output features (fragments 4 u .. 4 u + 3) through the wave's 4 KiB stage
   // (128-byte rows, 16-byte chunks XOR-swizzled by the row), written and read with inline assembly (for a C++ access to
   // LDS the compiler drains the VMEM queue first), the reads of one slab in flight while the next one is converted.
-  constexpr int NU = NF / 4, NSLAB = 4 * NU;
+  // WIDE (LEAN with one weight): a slab is 32 tokens x 32 features of fp32 - the same bytes, a fragment's four features a chunk.  (Stored straight
+  // from the fragments, 64-byte pieces and lanes that are neighbours in different rows, a CU's store path takes 62 cycles for a wave's
+  // 1 KiB, and 18 for whole lines: 6.8 us per tile, whatever the other CUs do.)
+  constexpr int NU = WIDE ? 4 : NF / 4, NSLAB = 4 * NU;
   const uint32_t stg_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + 2 * W16_STEP_BYTES) + wave * W4_STAGE_BYTES;
   // after the exchange lane (n16, q4) holds chunk 2 * (2 pr + (q4 & 1)) + (q4 >> 1) of row 16 ts + n16 (pr: fragment pair)
-  const uint32_t stg_w = stg_base + (uint32_t)n16 * 128 + (uint32_t)(((2 * (q4 & 1) + (q4 >> 1)) ^ (n16 & 7)) << 4);
+  const uint32_t stg_w = stg_base + (uint32_t)n16 * 128 + (uint32_t)(((WIDE ? q4 : 2 * (q4 & 1) + (q4 >> 1)) ^ (n16 & 7)) << 4);
   const uint32_t stg_r = stg_base + (uint32_t)(lane >> 3) * 128 + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
   const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (uint32_t)a.M * (uint32_t)a.ldy * 2, 0x00020000);
   const uint32_t y_lane = (uint32_t)(lane >> 3) * (uint32_t)a.ldy * 2 + (uint32_t)(lane & 7) * 16;
@@ -263,6 +347,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
       for (int ts = 0; ts < 2; ++ts)
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {
+          if constexpr (WIDE) {
+            out[2 * ts + pr] = __builtin_bit_cast(u32x4, any_out(2 * u + pr, 2 * tt + ts));
+            continue;
+          }
           const int t = 2 * tt + ts, f = 4 * u + 2 * pr;
           uint32_t x0 = pack_bf(out_value(f, t, 0, n0), out_value(f, t, 1, n0)), x1 = pack_bf(out_value(f, t, 2, n0), out_value(f, t, 3, n0));
           uint32_t y0 = pack_bf(out_value(f + 1, t, 0, n0), out_value(f + 1, t, 1, n0)), y1 = pack_bf(out_value(f + 1, t, 2, n0), out_value(f + 1, t, 3, n0));
@@ -271,6 +359,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
           const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
           const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
           out[2 * ts + pr] = u32x4{s0[0], s1[0], s0[1], s1[1]};
+          __builtin_amdgcn_sched_barrier(0);  // (accumulators copied out early would spill the next tile's first fragments)
         }
     };
     auto stage_in = [&]() __attribute__((always_inline)) {
@@ -288,6 +377,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     auto store_lines = [&](int slab) __attribute__((always_inline)) {
       const int tt = slab / NU, u = slab % NU;
       asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(back[0]), "+v"(back[1]), "+v"(back[2]), "+v"(back[3])::"memory");
+      if constexpr (WIDE) {
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const int row = any_y[4 * tt + it];
+          if (row >= 0) *reinterpret_cast<u32x4*>(a.y32 + row * a.ldy + (n0 + fw * 128 + (lane & 7) * 4) + u * 32) = back[it];
+        }
+        return;
+      }
       const uint32_t colb = (uint32_t)(EPI == TEPI_SILU ? (n0 >> 1) + fw * 64 : n0 + fw * 128 + u * 64) * 2;
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
@@ -334,6 +431,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     if constexpr (EPI == TEPI_ANY) {
       const AnyTile t = any_tile(a, blk, ntiles, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
       m0 = t.m0, n0 = t.n0, m_end = t.m_end;
+      any_begin(m0, n0, m_end);
     }
     kstep(std::true_type{});
     for (int kt = 1; kt < KT; ++kt) kstep(std::false_type{});
@@ -348,19 +446,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     asm volatile("" : "+a"(acc[5][3]), "+a"(acc[5][4]), "+a"(acc[5][5]), "+a"(acc[5][6]), "+a"(acc[5][7]), "+a"(acc[6][0]), "+a"(acc[6][1]), "+a"(acc[6][2]), "+a"(acc[6][3]), "+a"(acc[6][4]), "+a"(acc[6][5]), "+a"(acc[6][6]), "+a"(acc[6][7]), "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]), "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7]));
     // A workgroup's last tile: its (empty) past-the-end pieces must not outlive the workgroup's LDS
     if (blk + stride >= ntiles) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (EPI == TEPI_ANY) {
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const AnyRow row = any_row(a, m0 + w16_acc_token(tw, t, n16), m_end);
-#pragma unroll
-        for (int f = 0; f < (PAIRED ? 4 : 8); ++f) {
-          // (the next tile's first fragments are live here: accumulators copied out early would spill them)
-          if constexpr (PAIRED) asm volatile("" : "+a"(acc[f][t]), "+a"(acc[f + 4][t]));
-          any_store(a, row, n0 + fw * (PAIRED ? 64 : 128) + 16 * f + 4 * q4, acc[f][t], acc[PAIRED ? f + 4 : f][t]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    } else if constexpr (LINES) {
+    if constexpr (EPI == TEPI_ANY && !WIDE) {
+      epilogue_any(n0);
+    } else if constexpr (LINES || WIDE) {
       epilogue_lines(m0, n0);
     } else {
       epilogue(m0, n0);

@@ -167,3 +167,45 @@ def test_more_tiles_than_the_chip_holds(tile, G, N, K, dual, rows):
                                                   (256, 2048, 768, 64, False, 64), (8192, 2048, 2048, 0, False, 256), (2048, 768, 2048, 32, True, 128)])
 def test_rule_reaches_the_large_forms(rows, N, K, G, dual, want):
     assert _C.lib.mi_gemm_any_tile_rows(rows, N, K, G, int(dual), _C.ACT_SILU if dual else _C.ACT_NONE) == want
+
+
+@pytest.mark.parametrize("rows,N,K", [(130, 256, 64), (255, 512, 128), (257, 768, 64), (700, 256, 320)])
+@pytest.mark.parametrize("form", ["plain", "bias", "groups", "pair"])
+def test_whole_feature_tiles_of_the_persistent_kernel(form, rows, N, K):
+    """The 256-row kernel's short epilogue (whole feature tiles, nothing on rows or results; two weights: bf16 results): the same bits as
+    the 128-row kernel's, row for row, scattered and bounded by the groups; nothing written beside them."""
+    g = torch.Generator(device="cuda").manual_seed(rows + N + K)
+    G = 3 if form in ("groups", "pair") else 0
+    x = torch.randn(rows, K, device="cuda", generator=g)
+    w, w2 = (torch.randn(max(G, 1), N, K, device="cuda", generator=g).mul(K ** -0.5).bfloat16() for _ in range(2))
+    w, w2 = (w, w2) if G else (w[0], w2[0])
+    bias = torch.randn(N, device="cuda", generator=g) if form == "bias" else None
+    cut = rows // 3
+    off = torch.tensor([0, cut, cut, rows - rows // 7], dtype=torch.int32, device="cuda") if G else None
+    place = torch.randperm(rows, device="cuda", generator=g).to(torch.int32) if G else None
+    outs = []
+    for tile in (256, 128):
+        out = torch.full((rows + 1, N), 7.0, device="cuda", dtype=torch.bfloat16 if form == "pair" else torch.float32)
+        operand = ops._tile_operand(x, tile, None, off, G, rows) if G else ops._tile_operand(x, tile)
+        ops._tile_gemm(operand, tile, w, w2 if form == "pair" else None, out[:rows], _C.ACT_SILU if form == "pair" else _C.ACT_NONE, G,
+                       place, bias=bias)
+        outs.append(out)
+    assert torch.equal(*outs)
+    done = rows - rows // 7 if G else rows
+    assert int((outs[0] != 7.0).any(1).sum()) == done and bool((outs[0][rows] == 7.0).all())
+    if form in ("plain", "bias"):
+        xr, b = x.bfloat16().double(), 0.0 if bias is None else bias
+        size = xr.abs() @ w.double().abs().T + (0.0 if bias is None else bias.abs())
+        _close(outs[0][:rows], xr @ w.double().T + b, size, K)
+
+
+@pytest.mark.parametrize("tile", [64, 256])
+def test_silu_of_large_arguments(tile):
+    """0 and z to an ulp where the exponential is out of range, finite everywhere"""
+    z = torch.tensor([0.0, -0.0, 80.0, -80.0, 87.0, 88.0, -88.0, 104.5, -104.5, 1e30, -1e30, 3e38, -3e38], device="cuda").bfloat16().float().repeat(6)
+    x, w, w2 = torch.zeros(z.numel(), 64, device="cuda"), torch.zeros(128, 64, device="cuda"), torch.zeros(128, 64, device="cuda")
+    x[:, 0], x[:, 1], w[:, 0], w2[:, 1] = z, 1.0, 1.0, 1.0
+    out = torch.empty(z.numel(), 128, device="cuda")
+    ops._tile_gemm(ops._tile_operand(x, tile), tile, w.bfloat16(), w2.bfloat16(), out, _C.ACT_SILU)
+    want = torch.nn.functional.silu(z.double()).unsqueeze(1)
+    assert bool(((out.double() - want).abs() <= 4 * 2.0 ** -24 * want.abs() + 1e-35).all())
