@@ -23,9 +23,8 @@ __device__ __forceinline__ u32x4 pack16(const float (&f)[8]) {
   return o;
 }
 
-// rms-normalise the 128 values held by 8 lanes (16 each) with weight w
-__device__ __forceinline__ void head_rmsnorm(float (&a)[8], float (&b)[8], const uint16_t* w, int j,
-                                             float eps) {
+// rms-normalise the 128 values held by 8 lanes (16 each) with weights wa, wb
+__device__ __forceinline__ void head_rmsnorm(float (&a)[8], float (&b)[8], const float (&wa)[8], const float (&wb)[8], float eps) {
 #pragma clang fp contract(off)
   float ss = 0.f;
 #pragma unroll
@@ -36,25 +35,31 @@ __device__ __forceinline__ void head_rmsnorm(float (&a)[8], float (&b)[8], const
   ss = xor_sum<2>(ss);
   ss = xor_sum<4>(ss);
   const float rs = 1.0f / sqrtf(ss / 128.0f + eps);
-  float wa[8], wb[8];
-  load16(w + 8 * j, wa);
-  load16(w + 64 + 8 * j, wb);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     a[i] = rbf(rbf(a[i] * rs) * wa[i]);
     b[i] = rbf(rbf(b[i] * rs) * wb[i]);
   }
 }
+__device__ __forceinline__ void head_rmsnorm(float (&a)[8], float (&b)[8], const uint16_t* w, int j, float eps) {
+  float wa[8], wb[8];
+  load16(w + 8 * j, wa);
+  load16(w + 64 + 8 * j, wb);
+  head_rmsnorm(a, b, wa, wb, eps);
+}
 
 // NeoX rotation in fp32 (rotary_embedding.py:6-14): separate mul / sub / add
-__device__ __forceinline__ void head_rope(float (&a)[8], float (&b)[8], const float* cs, int j) {
+struct HeadRope {  // the cosines and sines of lane j's eight pairs
+  float4 c0, c1, s0, s1;
+};
+__device__ __forceinline__ HeadRope head_rope_load(const float* cs, int j) {
+  return HeadRope{*reinterpret_cast<const float4*>(cs + 8 * j), *reinterpret_cast<const float4*>(cs + 8 * j + 4),
+                  *reinterpret_cast<const float4*>(cs + 64 + 8 * j), *reinterpret_cast<const float4*>(cs + 64 + 8 * j + 4)};
+}
+__device__ __forceinline__ void head_rope(float (&a)[8], float (&b)[8], const HeadRope& r) {
 #pragma clang fp contract(off)
-  const float4 c0 = *reinterpret_cast<const float4*>(cs + 8 * j);
-  const float4 c1 = *reinterpret_cast<const float4*>(cs + 8 * j + 4);
-  const float4 s0 = *reinterpret_cast<const float4*>(cs + 64 + 8 * j);
-  const float4 s1 = *reinterpret_cast<const float4*>(cs + 64 + 8 * j + 4);
-  const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-  const float s[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  const float c[8] = {r.c0.x, r.c0.y, r.c0.z, r.c0.w, r.c1.x, r.c1.y, r.c1.z, r.c1.w};
+  const float s[8] = {r.s0.x, r.s0.y, r.s0.z, r.s0.w, r.s1.x, r.s1.y, r.s1.z, r.s1.w};
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float x1 = a[i], x2 = b[i];
@@ -62,6 +67,7 @@ __device__ __forceinline__ void head_rope(float (&a)[8], float (&b)[8], const fl
     b[i] = rbf(x2 * c[i] + x1 * s[i]);
   }
 }
+__device__ __forceinline__ void head_rope(float (&a)[8], float (&b)[8], const float* cs, int j) { head_rope(a, b, head_rope_load(cs, j)); }
 
 // ---- the same arithmetic on the MFMA-operand distribution of a head --------------------------
 // Four lanes g = 0..3 (lane ids n, n+16, n+32, n+48 of a wavefront) hold one head: lane g owns

@@ -1127,6 +1127,207 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same attention for steps with few query rows (a short prompt, the new rows behind a cached prefix), where the kernel above has a
+// workgroup on a tenth of the CUs and each walks its chunks one after another: 137 tokens x 16 heads (8 kv) are 24 workgroups, whose
+// longest takes 9.4 us - 2.9 the query rows' preparation, 2.5 the first chunk behind it, 0.75 every further one, 1.1 the transposed store.
+// Here a workgroup is 32 columns (32 / G query tokens x G heads), and its waves share the KEYS: wave w takes the chunks w, w + W, ..,
+// cache -> registers in operand order (a wave's chunks are its own: no ring, no barrier), the first of them requested behind the query
+// rows' loads and landing under their preparation, the next one under the running one; the waves' sums meet in LDS.  Per column the same
+// operations, chunks summed per wave: fp32 rounding apart the same rows. 
+// Measured: at few_query_rows.
+// ---------------------------------------------------------------------------
+template <int G, bool FUSE_Q, bool SPLIT_P, int W>
+__global__ __launch_bounds__(64 * W) void paged_attn_prefill_few_kernel(
+    const uint16_t* __restrict__ q, int64_t q_stride, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ kv_lens,
+    uint16_t* __restrict__ out, int n_q_heads, int n_kv_heads, int tpb, int tpb_shift, float scale_log2e, int n_qblocks, int n_pairs,
+    QPrep qp) {
+  constexpr int D = 128, TQ = 32 / G;
+  __shared__ __attribute__((aligned(16))) float sums[W][32][D];  // 16-byte pieces XOR-swizzled by the column
+  __shared__ float maxes[W][32], dens[W][32];
+  // (query blocks of one (sequence, kv head) on one XCD, the latest first: as above)
+  const int pair = ((int)blockIdx.x / (8 * n_qblocks)) * 8 + ((int)blockIdx.x & 7);
+  const int qblock = ((int)blockIdx.x >> 3) % n_qblocks;
+  if (pair >= n_pairs) return;
+  const int seq = pair / n_kv_heads, h = pair % n_kv_heads;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hi = lane >> 5, n = lane & 31;
+  const int q_start = cu_q[seq], q_len = cu_q[seq + 1] - q_start, kv_len = kv_lens[seq];
+  const int qt0 = (n_qblocks - 1 - qblock) * TQ;
+  if (qt0 >= q_len) return;  // uniform for the workgroup
+  const int shift = kv_len - q_len, last_pos = shift + min(qt0 + TQ, q_len) - 1;
+  const int chunks = (last_pos + 32) >> 5, tiles = (last_pos + 16) >> 4;
+  const int limit = shift + min(qt0 + n / G, q_len - 1) + 1;      // keys [0, limit) are visible to this lane's column
+  const int limit_all = shift + qt0 + 1;                           // ... to all of them
+
+  // the loads in the order they are needed (they come back in order): what the query rows take - eight lanes a column, the columns
+  // shared by the waves -, then the wave's first chunk
+  const int qc = (int)threadIdx.x >> 3, j = threadIdx.x & 7;  // (W waves: 8 W columns at a time)
+  constexpr int QN = 4 / W;
+  static_assert(QN * W == 4, "the 32 columns in whole passes");
+  u32x4 qa[QN], qb[QN];
+  HeadRope rope[QN];
+  float wa[8], wb[8];
+#pragma unroll
+  for (int i = 0; i < QN; ++i) {
+    const int col = i * 8 * W + qc, row = q_start + min(qt0 + col / G, q_len - 1);  // (columns beyond the last row: copies, not stored)
+    const uint16_t* const src = q + (int64_t)row * q_stride + (int64_t)(h * G + col % G) * D + 8 * j;
+    if constexpr (FUSE_Q) rope[i] = head_rope_load(qp.cos_sin + qp.positions[row] * 128, j);
+    qa[i] = *reinterpret_cast<const u32x4*>(src), qb[i] = *reinterpret_cast<const u32x4*>(src + 64);
+  }
+  if (FUSE_Q && qp.q_w) load16(qp.q_w + 8 * j, wa), load16(qp.q_w + 64 + 8 * j, wb);
+  __builtin_amdgcn_sched_barrier(0);
+
+  const int32_t* const table_row = block_table + (int64_t)seq * table_stride;
+  const KvStrides st = default_strides(n_kv_heads, tpb, 16 * D);
+  auto tile_at = [&](int tile) -> int64_t {  // element offset of a tile of the sequence at this kv head
+    const int blk = table_row[tpb_shift >= 0 ? tile >> tpb_shift : tile / tpb];
+    return (int64_t)blk * st.block + (int64_t)h * st.head + (int64_t)(tpb_shift >= 0 ? tile & (tpb - 1) : tile % tpb) * st.tile;
+  };
+  // K: key n = token n % 16 of tile n / 16, dims 16 kk + 8 hi .. + 7;  V: the 16 bytes of piece n / 16 of dim block db, tile s - dims
+  // 32 db + n % 16 and + 16 at four keys, the halves of which lanes n and n ^ 16 exchange
+  const int k_off = (hi * 16 + (n & 15)) * 8, v_off = k_off + (n >> 4) * 256;
+  struct Chunk {
+    u32x4 k[8], v[2][4];
+  };
+  auto request = [&](Chunk& x, int c) __attribute__((always_inline)) {
+    const int64_t t0 = tile_at(2 * c), t1 = tile_at(min(2 * c + 1, tiles - 1));
+    const uint16_t* const kp = kc + (n >> 4 ? t1 : t0) + k_off;
+    const uint16_t* const vp[2] = {vc + t0 + v_off, vc + t1 + v_off};
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) x.k[kk] = *reinterpret_cast<const u32x4*>(kp + (kk >> 1) * 512 + (kk & 1) * 256);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int db = 0; db < 4; ++db) x.v[s][db] = *reinterpret_cast<const u32x4*>(vp[s] + db * 512);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  Chunk a, b;
+  if (wave < chunks) request(a, wave);
+
+  uint16_t* const qs = reinterpret_cast<uint16_t*>(&sums[0][0][0]);  // [32 columns][128 dims], 16-byte pieces XOR-swizzled by the column
+#pragma unroll
+  for (int i = 0; i < QN; ++i) {
+    const int col = i * 8 * W + qc;
+    if constexpr (FUSE_Q) {
+      float x[8], y[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[2 * e] = lo_bf(qa[i][e]), x[2 * e + 1] = hi_bf(qa[i][e]);
+        y[2 * e] = lo_bf(qb[i][e]), y[2 * e + 1] = hi_bf(qb[i][e]);
+      }
+      if (qp.q_w) head_rmsnorm(x, y, wa, wb, qp.eps);
+      head_rope(x, y, rope[i]);
+      qa[i] = pack16(x), qb[i] = pack16(y);
+    }
+    *reinterpret_cast<u32x4*>(qs + col * D + ((j ^ col) & 15) * 8) = qa[i];
+    *reinterpret_cast<u32x4*>(qs + col * D + (((j + 8) ^ col) & 15) * 8) = qb[i];
+  }
+  __syncthreads();
+  bf16x8 Q[8];  // B operand of S^T = K . Q^T: column n, dims 16 kk + 8 hi .. + 7
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) Q[kk] = as_frag(*reinterpret_cast<const u32x4*>(qs + n * D + (((2 * kk + hi) ^ n) & 15) * 8));
+
+  float m = -INFINITY, l = 0.f;  // reference point (log2 domain) and this lane's share of the sum
+  f32x16 acc[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[j][i] = 0.f;
+  auto attend = [&](const Chunk& x, int c) __attribute__((always_inline)) {
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(x.k[kk]), Q[kk], s, 0, 0, 0);
+    // register i of this lane: key c * 32 + (i & 3) + 8 (i >> 2) + 4 hi
+    if (c * 32 + 32 > limit_all) {  // wave-uniform: some column does not see the whole chunk
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (c * 32 + 4 * hi + (i & 3) + 8 * (i >> 2) >= limit) s[i] = -INFINITY;
+    }
+    float mc = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mc = fmaxf(mc, s[i]);
+    mc = xor32_max(mc) * scale_log2e;  // scale > 0: the max commutes with it
+    if (__any(mc > m + kDeferMax)) {
+      // (a column may see none of this wave's keys so far: its reference point stays -inf and its sums 0)
+      const float mn = fmaxf(m, mc), alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[j][i] *= alpha;
+      m = mn;
+    }
+    const float ref = m == -INFINITY ? 0.f : m;
+    float p[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], scale_log2e, -ref));
+    l += ((p[0] + p[4]) + (p[8] + p[12])) + ((p[1] + p[5]) + (p[9] + p[13])) +
+         (((p[2] + p[6]) + (p[10] + p[14])) + ((p[3] + p[7]) + (p[11] + p[15])));
+    u32x4 ph[2], pl[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t hw = pack_bf(p[2 * i], p[2 * i + 1]);
+      ph[i >> 2][i & 3] = hw;
+      if (SPLIT_P) pl[i >> 2][i & 3] = pack_bf(p[2 * i] - lo_bf(hw), p[2 * i + 1] - hi_bf(hw));
+    }
+#pragma unroll
+    for (int sg = 0; sg < 2; ++sg)
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const u32x4 v = x.v[sg][db];
+        const auto v0 = __builtin_amdgcn_permlane16_swap(v[0], v[2], false, false);
+        const auto v1 = __builtin_amdgcn_permlane16_swap(v[1], v[3], false, false);
+        const bf16x8 va = as_frag(u32x4{v0[0], v1[0], v0[1], v1[1]});
+        acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, as_frag(ph[sg]), acc[db], 0, 0, 0);
+        if (SPLIT_P) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, as_frag(pl[sg]), acc[db], 0, 0, 0);
+      }
+  };
+  for (int c = wave; c < chunks; c += 2 * W) {
+    if (c + W < chunks) request(b, c + W);
+    attend(a, c);
+    if (c + W >= chunks) break;
+    if (c + 2 * W < chunks) request(a, c + 2 * W);
+    attend(b, c + W);
+  }
+
+  // the waves' sums (over the queries' image: every wave has read it in front of the barrier below): each scaled to the columns' common reference point, added in the waves' order
+  l = xor32_sum(l);
+  if (hi == 0) maxes[wave][n] = m, dens[wave][n] = l;
+  __syncthreads();
+  float top = maxes[0][n];
+#pragma unroll
+  for (int w = 1; w < W; ++w) top = fmaxf(top, maxes[w][n]);  // (finite: key 0 is visible to every column)
+  float den = 0.f;
+#pragma unroll
+  for (int w = 0; w < W; ++w) den += maxes[w][n] == -INFINITY ? 0.f : dens[w][n] * __builtin_amdgcn_exp2f(maxes[w][n] - top);
+  const float own = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top) / den;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4)  // dims 32 db + 8 i4 + 4 hi .. + 3
+      *reinterpret_cast<f32x4*>(&sums[wave][n][((db * 8 + i4 * 2 + hi) ^ n) * 4]) =
+          f32x4{acc[db][4 * i4] * own, acc[db][4 * i4 + 1] * own, acc[db][4 * i4 + 2] * own, acc[db][4 * i4 + 3] * own};
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < 8 / W; ++it) {  // a wave: four columns of 256 bytes at a time
+    const int col = (it * W + wave) * 4 + (lane >> 4), piece = (lane & 15) * 2;
+    f32x4 x = {}, y = {};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      x += *reinterpret_cast<const f32x4*>(&sums[w][col][(piece ^ col) * 4]);
+      y += *reinterpret_cast<const f32x4*>(&sums[w][col][((piece + 1) ^ col) * 4]);
+    }
+    const int qt = qt0 + col / G;
+    if (qt < q_len)
+      *reinterpret_cast<u32x4*>(out + ((int64_t)(q_start + qt) * n_q_heads + h * G + col % G) * D + (lane & 15) * 8) =
+          u32x4{pack_bf(x[0], x[1]), pack_bf(x[2], x[3]), pack_bf(y[0], y[1]), pack_bf(y[2], y[3])};
+  }
+}
+
 // A workgroup places 64 sequences, a lane each: its waves count those in front of it among 64 of the sequences each.  (One workgroup that counted all for
 // all of them: 4.4 us for 64 sequences, 14 for 560; so 2.8 and 3.8.)
 __global__ __launch_bounds__(1024) void context_order_kernel(const int32_t* __restrict__ lens, int n, int32_t* __restrict__ order) {
@@ -1386,6 +1587,18 @@ extern "C" int mi_paged_attn_decode_ex(const mi_bf16* q, int64_t q_row_stride, c
                      KvStrides{stride_block, stride_head, stride_tile}, stream);
 }
 
+// Which steps take paged_attn_prefill_few_kernel, by its workgroups (sequences x kv heads x blocks of 32 columns): about one per CU; two
+// while the last query block's chunks are many; four where one sequence's alone make more of them.  us per step of 28 layers, 8 kv heads,
+// the kernel for many rows / this one: 1 x 64 rows 1284 / 1204, 1 x 137 1537 / 1435, behind 320 cached 1759 / 1523, 1 x 400 2056 / 1887,
+// 1 x 1024 3061 / 2759, 1 x 2047 (1024 workgroups) 4908 / 4627, 2 x 300 2462 / 2329, 2 x 512 (512) 2763 / 2659, 3 x 200 behind 600 2638 / 2477,
+// 4 x 137 (288) 2028 / 1919, 4 x 256 (512) 2422 / 2402; beyond the lines 6 x 128 (384) 2444 / 2461, 3 x 400 (600) 3086 / 3130, 2 x 1024 (1024)
+// 4117 / 4224, 4 x 512 (1024) 3951 / 4161.
+constexpr int kFewWaves = 4;
+static bool few_query_rows(int n_pairs, int max_q, int G) {
+  const int64_t groups = (int64_t)n_pairs * ((max_q + 32 / G - 1) / (32 / G));
+  return groups <= 320 || (groups <= 512 && max_q >= 256) || (groups <= 1024 && groups < max_q);
+}
+
 static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* prep, const mi_bf16* k_cache,
                         const mi_bf16* v_cache, const int32_t* block_table, int table_stride,
                         const int32_t* cu_seqlens_q, const int32_t* kv_lens, int n_seqs, int max_seqlen_q,
@@ -1413,6 +1626,27 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
     if ((1 << sft) == block_size / 16) tpb_shift = sft;
   hipStream_t st = S(stream);
   const QPrep qp = prep ? *prep : QPrep{nullptr, nullptr, nullptr, 0.f};
+  if (head_dim == MI_HEAD_DIM && (variant & ~PV_SPLIT_P) == 0 && few_query_rows(n_pairs, max_seqlen_q, G)) {
+    const int blocks = (max_seqlen_q + 32 / G - 1) / (32 / G);
+    const dim3 few((unsigned)((n_pairs + 7) / 8 * 8 * blocks));
+    auto go = [&](auto group) {
+      constexpr int GG = decltype(group)::value;
+      auto with = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, few, dim3(64 * kFewWaves), 0, st, q, q_row_stride, k_cache, v_cache, block_table, table_stride,
+                           cu_seqlens_q, kv_lens, out, n_q_heads, n_kv_heads, block_size / 16, tpb_shift, sl2, blocks, n_pairs, qp);
+        return check_launch();
+      };
+      if (prep) return split_p ? with(paged_attn_prefill_few_kernel<GG, true, true, kFewWaves>) : with(paged_attn_prefill_few_kernel<GG, true, false, kFewWaves>);
+      return split_p ? with(paged_attn_prefill_few_kernel<GG, false, true, kFewWaves>) : with(paged_attn_prefill_few_kernel<GG, false, false, kFewWaves>);
+    };
+    switch (G) {
+      case 1: return go(std::integral_constant<int, 1>{});
+      case 2: return go(std::integral_constant<int, 2>{});
+      case 4: return go(std::integral_constant<int, 4>{});
+      case 8: return go(std::integral_constant<int, 8>{});
+      case 16: return go(std::integral_constant<int, 16>{});
+    }
+  }
 #define LAUNCH_PRE_AS(GG, FQ, VV)                                                                                  \
   hipLaunchKernelGGL((paged_attn_prefill_kernel<GG, FQ, VV>), grid, dim3(256), 0, st, q, q_row_stride, k_cache,   \
                      v_cache, block_table, table_stride, cu_seqlens_q, kv_lens, out, n_q_heads, n_kv_heads,       \

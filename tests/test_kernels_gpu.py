@@ -753,6 +753,29 @@ def test_prefill_attention_random(ops, hq, hkv, block_size, prefill_p):
     assert bool((err <= tol).all()), (err - tol).max().item()
 
 
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (8, 8), (32, 8), (64, 8), (16, 1)])
+@pytest.mark.parametrize("block_size", [16, 48, 256])
+def test_prefill_attention_of_few_rows(ops, hq, hkv, block_size, prefill_p):
+    """The waves share the keys: fewer chunks than waves, one more, a whole round and a part; columns that see none of a wave's keys;
+    query blocks of one row and of a part; a cached prefix of whole chunks, of a part and none."""
+    gen = torch.Generator().manual_seed(hq * 5 + hkv + block_size)
+    q_lens = [1, 7, 16, 33, 2, 30]
+    kv_lens = [1, 33, 16, 129 + 33, 257, 128]
+    T = sum(q_lens)
+    _, kc_l, vc_l, bt = _random_paged_case(gen, hq, hkv, block_size, kv_lens)
+    q = torch.randn(T, hq, 128, generator=gen).bfloat16()
+    cu = torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32)
+    kvl = torch.tensor(kv_lens, dtype=torch.int32)
+    want = oracle.paged_attention_prefill(q, kc_l, vc_l, bt, cu, kvl, keep_fp32=True)
+    want_absv = oracle.paged_attention_prefill(q, kc_l, vc_l.abs(), bt, cu, kvl, keep_fp32=True)
+    out = ops.paged_attn_prefill(q.to(DEV), to_fragment(kc_l, False).to(DEV), to_fragment(vc_l, True).to(DEV),
+                                 bt.to(DEV), cu.to(DEV), kvl.to(DEV), max(q_lens), hq, hkv, block_size,
+                                 1.0 / math.sqrt(128)).cpu()
+    err = (out.float() - want).abs()
+    tol = _prefill_bound(want, want_absv, prefill_p)
+    assert bool((err <= tol).all()), (err - tol).max().item()
+
+
 def test_prefill_attention_chunk_pipeline_stress(ops):
     """Kernel-level guard of the prefill attention's LDS-DMA ring (the counted `s_waitcnt vmcnt(4)` of its chunk
     loop): the bench's prefill step - 16 sequences x 1024 tokens, Qwen3-0.6B heads, block 16 - with SCRAMBLED block
