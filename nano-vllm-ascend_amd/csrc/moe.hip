@@ -206,6 +206,9 @@ __global__ __launch_bounds__(WAVES * 64) void moe_gemm_kernel(const uint16_t* __
   const int ktiles = K >> 5, kbeg = wave * 32 * STEPS;
   const int n_rows = GATE_UP ? 2 * N : N;  // weight rows per expert
   const uint16_t* we = w + (int64_t)e * n_rows * K;
+  // (loads come back in order: the first pairs' rows are asked for ahead of the weights, so that their x is asked for under them)
+  int pair = pair_token[p0 + min(r, n_e - 1)];
+  __builtin_amdgcn_sched_barrier(0);
   u32x4 a[RT][STEPS];
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
@@ -215,10 +218,12 @@ __global__ __launch_bounds__(WAVES * 64) void moe_gemm_kernel(const uint16_t* __
       a[t][s] = __builtin_nontemporal_load(
           reinterpret_cast<const u32x4*>(we + ((int64_t)tile * ktiles + (kbeg >> 5) + s) * 512 + lane * 8));
   }
+  __builtin_amdgcn_sched_barrier(0);
   for (int m0 = 0; m0 < n_e; m0 += 16) {
     const int pr = p0 + min(m0 + r, n_e - 1);  // pairs past the end shadow the last one (results unused)
-    const int64_t row = GATE_UP ? (int64_t)pair_token[pr] : (int64_t)pr;
-    const int64_t out_row = GATE_UP ? (int64_t)(p0 + m0 + r) : (int64_t)pair_token[pr];
+    const int64_t row = GATE_UP ? (int64_t)pair : (int64_t)pr;
+    const int64_t out_row = GATE_UP ? (int64_t)(p0 + m0 + r) : (int64_t)pair;
+    const int next = pair_token[p0 + min(m0 + 16 + r, n_e - 1)];
     f32x4 acc[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -230,6 +235,7 @@ __global__ __launch_bounds__(WAVES * 64) void moe_gemm_kernel(const uint16_t* __
 #pragma unroll
       for (int t = 0; t < RT; ++t)
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[t][s]), as_frag(b[s]), acc[t], 0, 0, 0);
+    pair = next;
     if (m0 > 0) __syncthreads();  // the previous pass has read red[]
 #pragma unroll
     for (int t = 0; t < RT; ++t) *reinterpret_cast<f32x4*>(&red[wave][t][lane][0]) = acc[t];
