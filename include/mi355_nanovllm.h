@@ -617,6 +617,15 @@ int mi_moe_gate_up(const mi_bf16* x, const mi_bf16* w_gate_up_packed, const int3
 int mi_moe_down(const mi_bf16* act, const mi_bf16* w_down_packed, const int32_t* expert_offsets,
                 const int32_t* pair_index, mi_bf16* y, int n_experts, int hidden, int inter,
                 mi_stream stream);
+/* Both products for steps of many pairs, from the weights as they are stored (row-major gate_up [E][2 * inter][hidden], down
+ * [E][hidden][inter]) on the tile kernels: same rows, same rounding points, sums over K in one fp32 chain.  mi_moe_tiles_bytes: its
+ * scratch for that many pairs, or 0 where mi_moe_gate_up / mi_moe_down are faster or the sizes are not taken.  act [P][inter] and
+ * scratch are overwritten; MI_EWORKSPACE if scratch is short. */
+int64_t mi_moe_tiles_bytes(int pairs, int n_experts, int inter, int hidden);
+int mi_moe_tiles(const mi_bf16* x, int n_tokens, const mi_bf16* gate_up, const mi_bf16* down,
+                 const int32_t* expert_offsets, const int32_t* pair_token, const int32_t* pair_index, mi_bf16* act,
+                 mi_bf16* y, int pairs, int n_experts, int hidden, int inter, void* scratch, int64_t scratch_bytes,
+                 mi_stream stream);
 /* out[t] = sum over the token's pairs j (ascending expert id) of bf16(y[t * top_k + j] * topk_w[t][j]), every
  * partial sum rounded to bf16 - `index_add_` into a bf16 tensor (:178-184). */
 int mi_moe_combine(const mi_bf16* y, const mi_bf16* topk_w, mi_bf16* out,

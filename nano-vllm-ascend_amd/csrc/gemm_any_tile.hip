@@ -17,10 +17,12 @@ namespace mi {
 
 // Table of a grouped operand: {row tiles, 0, 0, 0}, then per row tile {group, first row, end of the group's rows, 0}.
 // GATHER: the (sorted) rows' activations lie at rows x_rows[.] of x, which has x_total rows.
-template <int ACT, bool DUAL, bool GATHER = false>
+// HALF: the results are bf16 (y16), one weight's persistent products (two weights': always, in their short epilogue).
+template <int ACT, bool DUAL, bool GATHER = false, bool HALF = false>
 struct AnyTileArgs : TileArgs {
   static constexpr int kAct = ACT;
-  static constexpr bool kDual = DUAL, kGather = GATHER;
+  static constexpr bool kDual = DUAL, kGather = GATHER, kHalf = HALF;
+  int w_rows;  // weight rows from one group's to the next (N, or 2 N where w and w2 are the halves of one matrix)
   const int32_t* x_rows;
   int x_total;
   const uint16_t* w2;
@@ -35,6 +37,9 @@ struct AnyTileArgs : TileArgs {
   const float* row_scale;
   const int32_t* row_scale_rows;
 };
+
+// SiluAndMul with the roundings of a bf16 product in front of it (moe.hip): two weights only
+constexpr int kActMoeGlu = 100;
 
 // the operand's table is read through the scalar cache: it was written by an earlier launch and is the same for a whole wave
 typedef const __attribute__((address_space(4))) int32_t* ConstInts;
@@ -71,7 +76,9 @@ __device__ __forceinline__ f32x4 any_act(const A& a, f32x4 v, f32x4 v2) {
   for (int e = 0; e < 4; ++e) {
     const float z = v[e];
     float o = z;
-    if constexpr (A::kAct == MI_ACT_CLAMPED_GLU) {
+    if constexpr (A::kAct == kActMoeGlu) {
+      o = rbf(silu_f32(rbf(z))) * rbf(v2[e]);
+    } else if constexpr (A::kAct == MI_ACT_CLAMPED_GLU) {
       const float g = fminf(z, a.limit), u = fminf(fmaxf(v2[e], -a.limit), a.limit);
       o = g / (1.f + expf(-1.702f * g)) * (u + 1.f);
     } else {
@@ -188,24 +195,24 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
     return 0;
   const int tf = dual ? 128 : 256;
   if (n_groups && act == MI_ACT_SOFTCAP) return 0;   // (no group has one)
+  // 64-row tiles, or 256-row ones (the persistent kernel) where those are enough for the chip and not mostly padding; 128-row ones lie
+  // between the two nearly everywhere (two long-K weights of some 64 rows a group alone 99 / 103 / 119) and are left to softcap.
   if (n_groups) {
-    // 64-row tiles while a group's rows are fewer than its last tile's padding would be: 32 rows of 64 experts each 129 / 147 us with
-    // 128-row tiles (32 experts 28 / 36), 64 rows 163 / 156 (37 / 38)
-    if (rows < 48 * (int64_t)n_groups) return 64;
-    // 256-row tiles from 128 rows and some 350 tiles on, where the groups' last, part-filled tiles no longer weigh (64 experts: 128
-    // rows each 246 / 253; 32 experts of 512 rows = 320 tiles: 142 / 131)
-    return rows >= 128 * n_groups && (rows / 256 + n_groups / 2) * (int64_t)((N + tf - 1) / tf) >= 350 ? 256 : 128;
+    // us of both products, 64- / 128- / 256-row tiles: 32 experts of 512 x 1024, 48 rows each 37 / 57 / 49, 64 43 / 58 / 48, 96 55 / 59 / 49,
+    // 128 66 / 64 / 49, 512 118 / 114 / 91; 64 of 768 x 2048, 64 154 / 157 / 172, 96 173 / 165 / 173, 128 224 / 219 / 186, 512 647 / 554 / 400;
+    // 128 of 256 x 1024, 48 70 / 71 / 62, 128 94 / 93 / 68; 8 of 512 x 1024 (48 and 80 tiles of 256) 256 rows 40 / 53 / 47, 512 63 / 63 / 48
+    if (dual && K >= 2048 && rows >= 48 * (int64_t)n_groups && rows < 80 * (int64_t)n_groups) return 128;
+    return rows >= 80 * (int64_t)n_groups && (rows / 256 + n_groups / 2) * (int64_t)((N + tf - 1) / tf) >= 80 ? 256 : 64;
   }
-  // 64-row tiles while they are at most two per CU (N 2048, K 2048, 512 rows: 13.0, with 128-row tiles 24.7; N 6144: 256 rows 16.7 /
-  // 25.1, 512 rows 29.5 / 26.7); 256-row tiles from about 160 of them on (N 3072, K 1024, 4096 rows: 40, with 128-row tiles 48;
-  // N 2048, K 2048, 4096 rows = 128 tiles: 57 / 53)
-  if ((int64_t)((rows + 63) / 64) * ((N + 63) / 64) <= 512) return 64;
-  return act != MI_ACT_SOFTCAP && ((rows + 255) / 256) * (int64_t)((N + tf - 1) / tf) >= 160 ? 256 : 128;
+  // us, 64- / 128- / 256-row tiles: 2000 x 2048 x 1024 (1024 tiles of 64 x 64) 24 / 32 / 29, 3000 (1504) 39 / 36 / 30; 4000 x 1024 x 1024 (1008)
+  // 22 / 32 / 29, 6000 39 / 36 / 30; 2000 x 2048 x 2048 39 / 40 / 45, 3000 55 / 50 / 46; 500 x 6144 x 2048 (768) 36 / 37 / 44, 700 (1056) 59 / 49 / 45
+  if ((int64_t)((rows + 63) / 64) * ((N + 63) / 64) <= 1024) return 64;
+  return act != MI_ACT_SOFTCAP ? 256 : 128;
 }
 
-template <int ACT, bool DUAL, bool GATHER>
-static int launch_any_tile(const AnyTileArgs<ACT, DUAL, GATHER>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
-  using A = AnyTileArgs<ACT, DUAL, GATHER>;
+template <int ACT, bool DUAL, bool GATHER, bool HALF>
+static int launch_any_tile(const AnyTileArgs<ACT, DUAL, GATHER, HALF>& args, int tile_rows, int64_t row_tiles_max, hipStream_t st) {
+  using A = AnyTileArgs<ACT, DUAL, GATHER, HALF>;
   A a = args;
   if (tile_rows == 256) {
     a.tiles_f = (a.N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
@@ -214,9 +221,9 @@ static int launch_any_tile(const AnyTileArgs<ACT, DUAL, GATHER>& args, int tile_
     const dim3 grid((unsigned)(tiles < kPersistentGrid ? tiles : kPersistentGrid));
     // the epilogue's short form takes what the models' projections and experts ask for
     [[maybe_unused]] const bool lean = !a.row_scale && a.alpha == 1.f && a.N % (DUAL ? 128 : 256) == 0 &&
-                                       (DUAL ? a.y16 && !a.bias1 && !a.bias2 && a.ldy % 8 == 0 : !a.y16);
+                                       (DUAL || HALF ? a.y16 && !a.bias1 && !a.bias2 && a.ldy % 8 == 0 : !a.y16);
     if constexpr (ACT != MI_ACT_SOFTCAP) {  // (a head's product: never that many rows; it would not fit the persistent kernel's registers)
-      if constexpr (DUAL ? ACT == MI_ACT_SILU : ACT == MI_ACT_NONE)
+      if constexpr (DUAL ? ACT == MI_ACT_SILU || ACT == kActMoeGlu : ACT == MI_ACT_NONE)
         if (lean) {
           hipLaunchKernelGGL((gemm_w16_kernel<TEPI_ANY, false, 32768, A>), grid, dim3(256), 0, st, a);
           return check_launch();
@@ -301,7 +308,7 @@ static int any_tile_product(const mi_bf16* xb, const int32_t* x_rows, int x_tota
   auto go = [&](auto args) {
     args.x = xb, args.w = w, args.w2 = w2, args.bias = nullptr, args.y = nullptr, args.part = nullptr;
     args.ldx = K, args.ldy = ldy, args.M = rows, args.N = N, args.K = K;
-    args.groups = n_groups ? n_groups : 1, args.table = table;
+    args.groups = n_groups ? n_groups : 1, args.table = table, args.w_rows = N;
     args.y32 = y_is_bf16 ? nullptr : static_cast<float*>(y), args.y16 = y_is_bf16 ? static_cast<uint16_t*>(y) : nullptr;
     args.y_rows = y_rows, args.bias1 = bias, args.bias2 = bias2, args.alpha = alpha, args.limit = limit;
     args.row_scale = row_scale, args.row_scale_rows = row_scale_rows;
@@ -353,6 +360,50 @@ extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const
   return rc != MI_OK ? rc
                      : mi_gemm_any_tile(xb, nullptr, t, static_cast<const mi_bf16*>(w), static_cast<const mi_bf16*>(w2), bias, bias2, act,
                                         0.f, nullptr, nullptr, 0, y, 0, ldy, nullptr, M, N, K, alpha, stream);
+}
+
+// ---- the experts of moe.hip (bf16 activations and weights as they are stored, row-major) on the tile kernels: steps that bring prompts ----
+// moe.hip's kernels keep 16 features' weights in registers and walk an expert's pairs 16 at a time, a round trip and two barriers each:
+// made for the few pairs of a decode step.  us of a block (route to combine) with them / here on 64-row / on 256-row tiles:
+//   64 experts of 768 x 2048     16 pairs each 155 / 161 / 190   24 182 / 162 / 190   64 306 / 192 / 199   128 523 / 249 / 215   512 1834 / 648 / 392
+//   32 of 512 x 1024             24 47 / 48 / 57   32 53 / 48 / 58   64 72 / 55 / 58   128 111 / 80 / 61   512 358 / 142 / 109
+//   8 of 512 x 1024              64 42 / 45 / 53   256 69 / 52 / 57   512 114 / 75 / 60;  8 of 1536 x 4096  32 97 / 83 / 130   128 237 / 145 / 140
+// (128-row tiles are between the two nearly everywhere.)  A step of 8 x 1024 tokens, four layers of 64 experts: 15.7 -> 3.9 ms.
+static int moe_tile_rows(int pairs, int G, int ff, int width) {
+  if (pairs < 1 || G < 1 || width % BK || ff % BK || width % 8 || ff % 8) return 0;
+  if (2 * (int64_t)ff > INT32_MAX || ((int64_t)G * 2 * ff + 256) * width * 2 >= (int64_t)1 << 31) return 0;   // (32-bit offsets into gate_up)
+  if (pairs < 24 * (int64_t)G || (int64_t)pairs * (ff + width) < 1600000) return 0;
+  const int a = tile_rows_for(pairs, ff, width, G, true, MI_ACT_SILU, false), b = tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE, false);
+  return a < b ? a : b;
+}
+extern "C" int64_t mi_moe_tiles_bytes(int pairs, int n_experts, int inter, int hidden) {
+  const int t = moe_tile_rows(pairs, n_experts, inter, hidden);
+  return t ? 4 * mi_gemm_any_table_ints(pairs, n_experts, t) : 0;
+}
+extern "C" int mi_moe_tiles(const mi_bf16* x, int n_tokens, const mi_bf16* gate_up, const mi_bf16* down, const int32_t* expert_offsets,
+                            const int32_t* pair_token, const int32_t* pair_index, mi_bf16* act, mi_bf16* y, int pairs, int n_experts,
+                            int hidden, int inter, void* scratch, int64_t scratch_bytes, mi_stream stream) {
+  if (!x || !gate_up || !down || !expert_offsets || !pair_token || !pair_index || !act || !y || !scratch) return MI_EINVAL;
+  if (!aligned16(x) || !aligned16(gate_up) || !aligned16(down) || !aligned16(act) || !aligned16(y) || !aligned16(scratch)) return MI_EINVAL;
+  if (n_tokens < 1 || n_tokens > pairs) return MI_EINVAL;
+  const int t = moe_tile_rows(pairs, n_experts, inter, hidden);
+  if (!t) return MI_EUNSUPPORTED;
+  if (scratch_bytes < mi_moe_tiles_bytes(pairs, n_experts, inter, hidden)) return MI_EWORKSPACE;
+  int32_t* table = static_cast<int32_t*>(scratch);
+  const int64_t tiles = row_tiles(pairs, n_experts, t);
+  hipLaunchKernelGGL(any_operand_kernel, dim3(1), dim3(256), 0, S(stream), nullptr, 0, nullptr, expert_offsets, n_experts, t, 0, pairs, 8, nullptr,
+                     table, (int)tiles);   // (no rows: the table only)
+  int rc = check_launch();
+  if (rc != MI_OK) return rc;
+  AnyTileArgs<kActMoeGlu, true, true> g{};
+  g.x = x, g.w = gate_up, g.w2 = gate_up + (int64_t)inter * hidden, g.ldx = hidden, g.ldy = inter, g.M = pairs, g.N = inter, g.K = hidden;
+  g.w_rows = 2 * inter, g.x_rows = pair_token, g.x_total = n_tokens, g.groups = n_experts, g.table = table, g.y16 = act, g.alpha = 1.f;
+  rc = launch_any_tile(g, t, tiles, S(stream));
+  if (rc != MI_OK) return rc;
+  AnyTileArgs<MI_ACT_NONE, false, false, true> d{};
+  d.x = act, d.w = down, d.ldx = inter, d.ldy = hidden, d.M = pairs, d.N = hidden, d.K = inter;
+  d.w_rows = hidden, d.groups = n_experts, d.table = table, d.y16 = y, d.y_rows = pair_index, d.alpha = 1.f;
+  return launch_any_tile(d, t, tiles, S(stream));
 }
 
 // scratch of mi_expert_ff: the gathered operand, the inner activations, the tile table (each rounded up to 16 bytes) - or, streamed, the

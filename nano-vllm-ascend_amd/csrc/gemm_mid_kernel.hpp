@@ -41,7 +41,7 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
     const int ntiles = any_tiles(a);
     if ((int)blockIdx.x >= ntiles) return;  // (the grid is the host's bound on the grouped tiles)
     const AnyTile t = any_tile(a, (int)blockIdx.x, ntiles, SH::T, ARGS::kDual ? SH::F / 2 : SH::F);
-    n0 = t.n0, m0 = t.m0, m_end = t.m_end, wrow0 = (int64_t)t.group * a.N;
+    n0 = t.n0, m0 = t.m0, m_end = t.m_end, wrow0 = (int64_t)t.group * a.w_rows;
   }
 
   // LDS-DMA: wave w moves its share of the 1 KiB pieces (8 local rows each) of the feature rows and of the token rows

@@ -15,7 +15,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 enum { TEPI_NONE = 0, TEPI_SILU = 1, TEPI_PARTIAL = 2, TEPI_QKV = 3, TEPI_ANY = 4 };
 
 struct TileArgs {
-  static constexpr bool kDual = false, kGather = false;
+  static constexpr bool kDual = false, kGather = false, kHalf = false;
   const uint16_t* x;
   const uint16_t* w;
   const uint16_t* bias;

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   constexpr bool GATHER = EPI == TEPI_ANY && ARGS::kGather;  // a tile's activation rows wherever x_rows says
   constexpr bool LEAN = (V & 32768) != 0 && EPI == TEPI_ANY;  // the epilogue's short form: see any_begin
   constexpr bool PAIRED = EPI == TEPI_ANY && ARGS::kDual;  // two weights: half 0 of the A region holds 128 rows of w, half 1 of w2
-  constexpr bool WIDE = LEAN && !PAIRED;
+  constexpr bool WIDE = LEAN && !PAIRED, F32 = WIDE && !ARGS::kHalf;
   __shared__ __attribute__((aligned(1024))) char lds[2 * W16_STEP_BYTES + (LINES || WIDE ? 4 * W4_STAGE_BYTES : 0)];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   uint32_t records = (uint32_t)(wgt ? a.N : a.M) * ld2;
   const uint16_t* src = wgt ? a.w : a.x;
   if constexpr (EPI == TEPI_ANY) {
-    if (wgt) records *= (uint32_t)a.groups;
+    if (wgt) records += (uint32_t)(a.groups - 1) * (uint32_t)a.w_rows * ld2;
     if (PAIRED && wave == 1) src = a.w2;
     if (GATHER && !wgt) records = (uint32_t)a.x_total * ld2;
   }
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     if constexpr (GATHER) {
       const AnyTile t = any_tile(a, b, ntiles, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
       if (wgt) {
-        f_row = (uint32_t)(t.group * a.N + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
+        f_row = (uint32_t)(t.group * a.w_rows + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
 #pragma unroll
         for (int q = 0; q < W4_PIECES; ++q) g_off[q] = voff[w16_piece_x3(q)] + (f_row + (uint32_t)w16_piece_rows(q) * ld2);
       } else {
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
     if constexpr (EPI == TEPI_ANY) {
       const AnyTile t = any_tile(a, b, ntiles, TILE_T, PAIRED ? TILE_F / 2 : TILE_F);
       if (!wgt) f_row = (uint32_t)(t.m0 + (wave & 1) * 128) * ld2;
-      else f_row = (uint32_t)(t.group * a.N + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
+      else f_row = (uint32_t)(t.group * a.w_rows + t.n0 + (PAIRED ? 0 : (wave & 1) * 128)) * ld2;
       return;
     }
     const int tid = tile_of_block(b, a.tiles_t, a.tiles_f, (V & 4) != 0);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   // biases - is asked for in front of the tile's K steps: a load behind them waits for the pieces and the stores before it, once per
   // token fragment (an index) or per store (a bias).
   // What bounds it is issue: one wave per SIMD, no matrix instruction beside it.  LEAN (whole feature tiles; no factor on rows or
-  // results; one weight: fp32 results, no activation; two: bf16 results, no bias) knows at compile time what the rest selects per value
+  // results; one weight: no activation; two, or one with bf16 results: bf16 results, no bias) knows at compile time what the rest selects per value
   // and branches on per store.  us per tile from the last K step to the end, before -> LEAN: one weight 8.0 -> 6.2 (rows by an index
   // 11.0 -> 6.2), two 14.0 -> 6.3.
   constexpr int NV = EPI == TEPI_ANY ? (PAIRED ? 4 : 8) : 1, NT = EPI == TEPI_ANY ? (WIDE ? 16 : 8) : 1;
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
         any_y[t] = m < m_end ? y : -1;
         if constexpr (!LEAN) any_scale[t] = a.row_scale ? a.row_scale[a.row_scale_rows ? a.row_scale_rows[at] : at] : 1.f;
       }
-      if constexpr (!LEAN || !PAIRED) {
+      if constexpr (!LEAN || F32) {
         const int n = n0 + fw * (PAIRED ? 64 : 128) + 4 * q4;
 #pragma unroll
         for (int f = 0; f < NV; ++f) {
@@ -327,13 +327,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   // (token fragments 2 tt, 2 tt + 1) x 64 output features (fragments 4 u .. 4 u + 3) through the wave's 4 KiB stage
   // (128-byte rows, 16-byte chunks XOR-swizzled by the row), written and read with inline assembly (for a C++ access to
   // LDS the compiler drains the VMEM queue first), the reads of one slab in flight while the next one is converted.
-  // WIDE (LEAN with one weight): a slab is 32 tokens x 32 features of fp32 - the same bytes, a fragment's four features a chunk.  (Stored straight
+  // F32 (LEAN with one weight, fp32 results): a slab is 32 tokens x 32 features of fp32 - the same bytes, a fragment's four features a chunk.  (Stored straight
   // from the fragments, 64-byte pieces and lanes that are neighbours in different rows, a CU's store path takes 62 cycles for a wave's
   // 1 KiB, and 18 for whole lines: 6.8 us per tile, whatever the other CUs do.)
-  constexpr int NU = WIDE ? 4 : NF / 4, NSLAB = 4 * NU;
+  constexpr int NU = F32 ? 4 : NF / 4, NSLAB = 4 * NU;
   const uint32_t stg_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + 2 * W16_STEP_BYTES) + wave * W4_STAGE_BYTES;
   // after the exchange lane (n16, q4) holds chunk 2 * (2 pr + (q4 & 1)) + (q4 >> 1) of row 16 ts + n16 (pr: fragment pair)
-  const uint32_t stg_w = stg_base + (uint32_t)n16 * 128 + (uint32_t)(((WIDE ? q4 : 2 * (q4 & 1) + (q4 >> 1)) ^ (n16 & 7)) << 4);
+  const uint32_t stg_w = stg_base + (uint32_t)n16 * 128 + (uint32_t)(((F32 ? q4 : 2 * (q4 & 1) + (q4 >> 1)) ^ (n16 & 7)) << 4);
   const uint32_t stg_r = stg_base + (uint32_t)(lane >> 3) * 128 + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
   const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (uint32_t)a.M * (uint32_t)a.ldy * 2, 0x00020000);
   const uint32_t y_lane = (uint32_t)(lane >> 3) * (uint32_t)a.ldy * 2 + (uint32_t)(lane & 7) * 16;
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
       for (int ts = 0; ts < 2; ++ts)
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {
-          if constexpr (WIDE) {
+          if constexpr (F32) {
             out[2 * ts + pr] = __builtin_bit_cast(u32x4, any_out(2 * u + pr, 2 * tt + ts));
             continue;
           }
@@ -381,7 +381,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
           const int row = any_y[4 * tt + it];
-          if (row >= 0) *reinterpret_cast<u32x4*>(a.y32 + row * a.ldy + (n0 + fw * 128 + (lane & 7) * 4) + u * 32) = back[it];
+          if constexpr (F32) {
+            if (row >= 0) *reinterpret_cast<u32x4*>(a.y32 + row * a.ldy + (n0 + fw * 128 + (lane & 7) * 4) + u * 32) = back[it];
+          } else {
+            if (row >= 0) *reinterpret_cast<u32x4*>(a.y16 + row * a.ldy + (n0 + fw * 128 + (lane & 7) * 8) + u * 64) = back[it];
+          }
         }
         return;
       }

@@ -175,6 +175,8 @@ _SIGNATURES = {
     "mi_moe_route": (c_int, [_p, c_int, c_int, c_int, _p, _p, _p]),
     "mi_moe_sort": (c_int, [_p, c_int, c_int, c_int, _p, _p, _p, _p]),
     "mi_moe_gate_up": (c_int, [_p, _p, _p, _p, _p, c_int, c_int, c_int, _p]),
+    "mi_moe_tiles_bytes": (c_int64, [c_int, c_int, c_int, c_int]),
+    "mi_moe_tiles": (c_int, [_p, c_int, _p, _p, _p, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p, c_int64, _p]),
     "mi_moe_down": (c_int, [_p, _p, _p, _p, _p, c_int, c_int, c_int, _p]),
     "mi_moe_combine": (c_int, [_p, _p, _p, c_int, c_int, c_int, _p]),
     "mi_comm_region_bytes": (c_size_t, [c_int, c_size_t]),

@@ -80,7 +80,8 @@ class Qwen3MoeSparseMoeBlock(nn.Module):
         x = x.reshape(-1, shape[-1])
         logits = linear_forward(x, self.gate.weight, None, self.gate_packed)  # bf16 router logits (:151)
         out, _, _ = ops.moe_forward(x.contiguous(), logits, self.gate_up_packed, self.down_packed, self.top_k,
-                                    all_reduce=all_reduce_sum if collectives_on() else None)
+                                    all_reduce=all_reduce_sum if collectives_on() else None,
+                                    gate_up=self.gate_up_stacked, down=self.down_stacked)
         return out.view(shape)
 
 

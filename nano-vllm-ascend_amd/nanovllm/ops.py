@@ -993,10 +993,11 @@ def pack_expert_weights(w, out=None) -> torch.Tensor:
     return out
 
 
-def moe_forward(x, router_logits, gate_up_packed, down_packed, top_k: int, all_reduce=None):
+def moe_forward(x, router_logits, gate_up_packed, down_packed, top_k: int, all_reduce=None, gate_up=None, down=None):
     """Qwen3MoeSparseMoeBlock.forward (qwen3_moe.py:150-185) behind the router GEMM: route -> group the pairs by
     expert -> grouped gate_up+SwiGLU -> grouped down (-> all-reduce of the ranks' partial sums) -> combine.
-    x [T, H], router_logits [T, E] bf16; returns [T, H] bf16."""
+    x [T, H], router_logits [T, E] bf16; returns [T, H] bf16.  gate_up, down: the weights as they are stored, which steps of many
+    pairs are multiplied from (mi_moe_tiles)."""
     require_gpu(x, router_logits, gate_up_packed, down_packed)
     _bf16(x, router_logits, gate_up_packed, down_packed)
     assert x.is_contiguous() and router_logits.is_contiguous()
@@ -1014,11 +1015,20 @@ def moe_forward(x, router_logits, gate_up_packed, down_packed, top_k: int, all_r
     check(lib.mi_moe_sort(ptr(ids), T, top_k, E, ptr(offsets), ptr(pair_token), ptr(pair_index), stream()),
           "mi_moe_sort")
     act = torch.empty((T * top_k, inter), dtype=_BF16, device=dev)
-    check(lib.mi_moe_gate_up(ptr(x), ptr(gate_up_packed), ptr(offsets), ptr(pair_token), ptr(act), E, H, inter,
-                             stream()), "mi_moe_gate_up")
     y = torch.empty((T * top_k, H), dtype=_BF16, device=dev)  # row t * top_k + j: the same on every TP rank
-    check(lib.mi_moe_down(ptr(act), ptr(down_packed), ptr(offsets), ptr(pair_index), ptr(y), E, H, inter, stream()),
-          "mi_moe_down")
+    n = lib.mi_moe_tiles_bytes(T * top_k, E, inter, H) if gate_up is not None and down is not None and T else 0
+    if n and not (x.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16:
+        require_gpu(gate_up, down)
+        _bf16(gate_up, down)
+        assert gate_up.shape == gate_up_packed.shape and down.shape == down_packed.shape and gate_up.is_contiguous() and down.is_contiguous()
+        table = torch.empty(n, dtype=torch.uint8, device=dev)
+        check(lib.mi_moe_tiles(ptr(x), T, ptr(gate_up), ptr(down), ptr(offsets), ptr(pair_token), ptr(pair_index), ptr(act), ptr(y),
+                               T * top_k, E, H, inter, ptr(table), n, stream()), "mi_moe_tiles")
+    else:
+        check(lib.mi_moe_gate_up(ptr(x), ptr(gate_up_packed), ptr(offsets), ptr(pair_token), ptr(act), E, H, inter,
+                                 stream()), "mi_moe_gate_up")
+        check(lib.mi_moe_down(ptr(act), ptr(down_packed), ptr(offsets), ptr(pair_index), ptr(y), E, H, inter, stream()),
+              "mi_moe_down")
     if all_reduce is not None:
         y = all_reduce(y)
     out = torch.empty((T, H), dtype=_BF16, device=dev)

@@ -1093,6 +1093,28 @@ def test_moe_block_golden(ops, golden_moe_block):
         _assert_moe_close(got, bf(g[f"{tag}_y"]))
 
 
+@pytest.mark.parametrize("T,H,E,K,I,tile", [(700, 1024, 8, 2, 512, 64), (2600, 1024, 8, 2, 512, 256), (1100, 512, 32, 4, 384, 256), (500, 640, 16, 8, 192, 64)])
+@pytest.mark.parametrize("uneven", [False, True])
+def test_moe_block_from_the_stored_weights(ops, T, H, E, K, I, tile, uneven):
+    """Steps of many pairs on the tile kernels (mi_moe_tiles): the same routing, an output each row's sums over K in another order apart
+    - half an ulp of the two products, which the chain of bf16 additions carries as _assert_moe_close says - and no other expert's rows
+    where the shares are uneven (experts without a pair, one with nearly half of them)."""
+    gen = torch.Generator().manual_seed(T + E)
+    x = torch.randn(T, H, generator=gen).bfloat16().to(DEV)
+    logits = torch.randn(T, E, generator=gen)
+    if uneven:
+        logits[:, 1] += 6.0
+        logits[:, 2::5] -= 12.0
+    logits = logits.bfloat16().to(DEV)
+    gu, dn = ((torch.randn(E, *s, generator=gen) * s[1] ** -0.5).bfloat16().to(DEV) for s in ((2 * I, H), (H, I)))
+    packed = ops.pack_expert_weights(gu), ops.pack_expert_weights(dn)
+    assert ops.lib.mi_moe_tiles_bytes(T * K, E, I, H) > 0 and ops.lib.mi_gemm_any_tile_rows(T * K, I, H, E, 1, 1) == tile
+    want, wid, ww = ops.moe_forward(x, logits, *packed, K)
+    got, ids, w = ops.moe_forward(x, logits, *packed, K, gate_up=gu, down=dn)
+    assert torch.equal(ids, wid) and torch.equal(w, ww)
+    _assert_moe_close(got.cpu(), want.cpu())
+
+
 @pytest.mark.parametrize("T", [1, 32, 64, 100])
 @pytest.mark.parametrize("inter", [768, 192])
 def test_moe_block_qwen3_30b_a3b_shapes(ops, T, inter):
