@@ -1131,21 +1131,24 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
 // The same attention for steps with few query rows (a short prompt, the new rows behind a cached prefix), where the kernel above has a
 // workgroup on a tenth of the CUs and each walks its chunks one after another: 137 tokens x 16 heads (8 kv) are 24 workgroups, whose
 // longest takes 9.4 us - 2.9 the query rows' preparation, 2.5 the first chunk behind it, 0.75 every further one, 1.1 the transposed store.
-// Here a workgroup is 32 columns (32 / G query tokens x G heads), and its waves share the KEYS: wave w takes the chunks w, w + W, ..,
-// cache -> registers in operand order (a wave's chunks are its own: no ring, no barrier), the first of them requested behind the query
-// rows' loads and landing under their preparation, the next one under the running one; the waves' sums meet in LDS.  Per column the same
-// operations, chunks summed per wave: fp32 rounding apart the same rows. 
+// Here a workgroup is 32 columns (32 / G query tokens x G heads; one wave of the kernel above) and takes four chunks at a time: wave w the
+// scores and exponentials of the w-th, which the waves exchange through LDS, and the four chunks' products with ITS 32 of the 128 dims,
+// chunk after chunk - every sum has the order it has above, and a row the same bits.  Keys and values go from the cache into registers
+// in operand order (nobody shares them: no ring), the first round's asked for behind the query rows' loads and landing under their
+// preparation, which eight lanes a column do once per workgroup, the next round's under the running one.
 // Measured: at few_query_rows.
 // ---------------------------------------------------------------------------
-template <int G, bool FUSE_Q, bool SPLIT_P, int W>
-__global__ __launch_bounds__(64 * W) void paged_attn_prefill_few_kernel(
+template <int G, bool FUSE_Q, bool SPLIT_P>
+__global__ __launch_bounds__(256) void paged_attn_prefill_few_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ kv_lens,
     uint16_t* __restrict__ out, int n_q_heads, int n_kv_heads, int tpb, int tpb_shift, float scale_log2e, int n_qblocks, int n_pairs,
     QPrep qp) {
-  constexpr int D = 128, TQ = 32 / G;
-  __shared__ __attribute__((aligned(16))) float sums[W][32][D];  // 16-byte pieces XOR-swizzled by the column
-  __shared__ float maxes[W][32], dens[W][32];
+  constexpr int D = 128, TQ = 32 / G, W = 4, PN = SPLIT_P ? 4 : 2;
+  __shared__ __attribute__((aligned(16))) uint16_t rows[32][D];          // the queries, then the results; 16-byte pieces XOR-swizzled by the column
+  __shared__ __attribute__((aligned(16))) uint32_t probs[2][W][PN][64][4];  // [round][chunk]: a lane's operand of the second product
+  __shared__ float chunk_sums[2][W][64], first[32], points[W][32], alphas[W][32];
+  __shared__ int ahead[2][W];
   // (query blocks of one (sequence, kv head) on one XCD, the latest first: as above)
   const int pair = ((int)blockIdx.x / (8 * n_qblocks)) * 8 + ((int)blockIdx.x & 7);
   const int qblock = ((int)blockIdx.x >> 3) % n_qblocks;
@@ -1158,173 +1161,193 @@ __global__ __launch_bounds__(64 * W) void paged_attn_prefill_few_kernel(
   if (qt0 >= q_len) return;  // uniform for the workgroup
   const int shift = kv_len - q_len, last_pos = shift + min(qt0 + TQ, q_len) - 1;
   const int chunks = (last_pos + 32) >> 5, tiles = (last_pos + 16) >> 4;
-  const int limit = shift + min(qt0 + n / G, q_len - 1) + 1;      // keys [0, limit) are visible to this lane's column
-  const int limit_all = shift + qt0 + 1;                           // ... to all of them
+  const int limit = shift + min(qt0 + n / G, q_len - 1) + 1;  // keys [0, limit) are visible to this lane's column
+  const int limit_all = shift + qt0 + 1;                      // ... to all of them
 
-  // the loads in the order they are needed (they come back in order): what the query rows take - eight lanes a column, the columns
-  // shared by the waves -, then the wave's first chunk
-  const int qc = (int)threadIdx.x >> 3, j = threadIdx.x & 7;  // (W waves: 8 W columns at a time)
-  constexpr int QN = 4 / W;
-  static_assert(QN * W == 4, "the 32 columns in whole passes");
-  u32x4 qa[QN], qb[QN];
-  HeadRope rope[QN];
+  // the loads in the order they are needed (they come back in order): what the query rows take, then the first round's keys and values
+  const int col = (int)threadIdx.x >> 3, j = threadIdx.x & 7;
+  u32x4 qa, qb;
+  HeadRope rope;
   float wa[8], wb[8];
-#pragma unroll
-  for (int i = 0; i < QN; ++i) {
-    const int col = i * 8 * W + qc, row = q_start + min(qt0 + col / G, q_len - 1);  // (columns beyond the last row: copies, not stored)
+  {
+    const int row = q_start + min(qt0 + col / G, q_len - 1);  // (columns beyond the last row: copies, not stored)
     const uint16_t* const src = q + (int64_t)row * q_stride + (int64_t)(h * G + col % G) * D + 8 * j;
-    if constexpr (FUSE_Q) rope[i] = head_rope_load(qp.cos_sin + qp.positions[row] * 128, j);
-    qa[i] = *reinterpret_cast<const u32x4*>(src), qb[i] = *reinterpret_cast<const u32x4*>(src + 64);
+    if constexpr (FUSE_Q) rope = head_rope_load(qp.cos_sin + qp.positions[row] * 128, j);
+    qa = *reinterpret_cast<const u32x4*>(src), qb = *reinterpret_cast<const u32x4*>(src + 64);
+    if (FUSE_Q && qp.q_w) load16(qp.q_w + 8 * j, wa), load16(qp.q_w + 64 + 8 * j, wb);
   }
-  if (FUSE_Q && qp.q_w) load16(qp.q_w + 8 * j, wa), load16(qp.q_w + 64 + 8 * j, wb);
   __builtin_amdgcn_sched_barrier(0);
 
   const int32_t* const table_row = block_table + (int64_t)seq * table_stride;
   const KvStrides st = default_strides(n_kv_heads, tpb, 16 * D);
-  auto tile_at = [&](int tile) -> int64_t {  // element offset of a tile of the sequence at this kv head
-    const int blk = table_row[tpb_shift >= 0 ? tile >> tpb_shift : tile / tpb];
-    return (int64_t)blk * st.block + (int64_t)h * st.head + (int64_t)(tpb_shift >= 0 ? tile & (tpb - 1) : tile % tpb) * st.tile;
+  auto tile_at = [&](int tile) -> int64_t {  // element offset of a tile of the sequence (past its end: the last one) at this kv head
+    const int t = min(tile, tiles - 1);
+    const int blk = table_row[tpb_shift >= 0 ? t >> tpb_shift : t / tpb];
+    return (int64_t)blk * st.block + (int64_t)h * st.head + (int64_t)(tpb_shift >= 0 ? t & (tpb - 1) : t % tpb) * st.tile;
   };
-  // K: key n = token n % 16 of tile n / 16, dims 16 kk + 8 hi .. + 7;  V: the 16 bytes of piece n / 16 of dim block db, tile s - dims
-  // 32 db + n % 16 and + 16 at four keys, the halves of which lanes n and n ^ 16 exchange
-  const int k_off = (hi * 16 + (n & 15)) * 8, v_off = k_off + (n >> 4) * 256;
-  struct Chunk {
-    u32x4 k[8], v[2][4];
+  // K: key n = token n % 16 of tile n / 16, dims 16 kk + 8 hi .. + 7;  V: the 16 bytes of piece n / 16 of the wave's dim block, tile s - dims
+  // n % 16 and + 16 of it at four keys, the halves of which lanes n and n ^ 16 exchange
+  const int k_off = (hi * 16 + (n & 15)) * 8, v_off = k_off + (n >> 4) * 256 + wave * 512;
+  struct Round {
+    u32x4 k[8], v[W][2];
   };
-  auto request = [&](Chunk& x, int c) __attribute__((always_inline)) {
-    const int64_t t0 = tile_at(2 * c), t1 = tile_at(min(2 * c + 1, tiles - 1));
+  auto request = [&](Round& x, int c0) __attribute__((always_inline)) {
+    const int64_t t0 = tile_at(2 * (c0 + wave)), t1 = tile_at(2 * (c0 + wave) + 1);
     const uint16_t* const kp = kc + (n >> 4 ? t1 : t0) + k_off;
-    const uint16_t* const vp[2] = {vc + t0 + v_off, vc + t1 + v_off};
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) x.k[kk] = *reinterpret_cast<const u32x4*>(kp + (kk >> 1) * 512 + (kk & 1) * 256);
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int c = 0; c < W; ++c)
 #pragma unroll
-      for (int db = 0; db < 4; ++db) x.v[s][db] = *reinterpret_cast<const u32x4*>(vp[s] + db * 512);
+      for (int s = 0; s < 2; ++s) x.v[c][s] = *reinterpret_cast<const u32x4*>(vc + tile_at(2 * (c0 + c) + s) + v_off);
     __builtin_amdgcn_sched_barrier(0);
   };
-  Chunk a, b;
-  if (wave < chunks) request(a, wave);
+  Round a, b;
+  request(a, 0);
 
-  uint16_t* const qs = reinterpret_cast<uint16_t*>(&sums[0][0][0]);  // [32 columns][128 dims], 16-byte pieces XOR-swizzled by the column
+  if constexpr (FUSE_Q) {
+    float x[8], y[8];
 #pragma unroll
-  for (int i = 0; i < QN; ++i) {
-    const int col = i * 8 * W + qc;
-    if constexpr (FUSE_Q) {
-      float x[8], y[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[2 * e] = lo_bf(qa[i][e]), x[2 * e + 1] = hi_bf(qa[i][e]);
-        y[2 * e] = lo_bf(qb[i][e]), y[2 * e + 1] = hi_bf(qb[i][e]);
-      }
-      if (qp.q_w) head_rmsnorm(x, y, wa, wb, qp.eps);
-      head_rope(x, y, rope[i]);
-      qa[i] = pack16(x), qb[i] = pack16(y);
+    for (int e = 0; e < 4; ++e) {
+      x[2 * e] = lo_bf(qa[e]), x[2 * e + 1] = hi_bf(qa[e]);
+      y[2 * e] = lo_bf(qb[e]), y[2 * e + 1] = hi_bf(qb[e]);
     }
-    *reinterpret_cast<u32x4*>(qs + col * D + ((j ^ col) & 15) * 8) = qa[i];
-    *reinterpret_cast<u32x4*>(qs + col * D + (((j + 8) ^ col) & 15) * 8) = qb[i];
+    if (qp.q_w) head_rmsnorm(x, y, wa, wb, qp.eps);
+    head_rope(x, y, rope);
+    qa = pack16(x), qb = pack16(y);
   }
+  *reinterpret_cast<u32x4*>(&rows[col][((j ^ col) & 15) * 8]) = qa;
+  *reinterpret_cast<u32x4*>(&rows[col][(((j + 8) ^ col) & 15) * 8]) = qb;
   __syncthreads();
   bf16x8 Q[8];  // B operand of S^T = K . Q^T: column n, dims 16 kk + 8 hi .. + 7
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) Q[kk] = as_frag(*reinterpret_cast<const u32x4*>(qs + n * D + (((2 * kk + hi) ^ n) & 15) * 8));
+  for (int kk = 0; kk < 8; ++kk) Q[kk] = as_frag(*reinterpret_cast<const u32x4*>(&rows[n][(((2 * kk + hi) ^ n) & 15) * 8]));
 
-  float m = -INFINITY, l = 0.f;  // reference point (log2 domain) and this lane's share of the sum
-  f32x16 acc[4];
+  f32x16 s, acc;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[j][i] = 0.f;
-  auto attend = [&](const Chunk& x, int c) __attribute__((always_inline)) {
-    f32x16 s;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(x.k[kk]), Q[kk], s, 0, 0, 0);
-    // register i of this lane: key c * 32 + (i & 3) + 8 (i >> 2) + 4 hi
-    if (c * 32 + 32 > limit_all) {  // wave-uniform: some column does not see the whole chunk
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (c * 32 + 4 * hi + (i & 3) + 8 * (i >> 2) >= limit) s[i] = -INFINITY;
-    }
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  float m = 0.f, l = 0.f;  // reference point (log2 domain) and this lane's share of the sum: the same in every wave
+  auto chunk_max = [&]() __attribute__((always_inline)) {
     float mc = s[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mc = fmaxf(mc, s[i]);
-    mc = xor32_max(mc) * scale_log2e;  // scale > 0: the max commutes with it
-    if (__any(mc > m + kDeferMax)) {
-      // (a column may see none of this wave's keys so far: its reference point stays -inf and its sums 0)
-      const float mn = fmaxf(m, mc), alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
-      l *= alpha;
+    return xor32_max(mc) * scale_log2e;  // scale > 0: the max commutes with it
+  };
+  float p[16];
+  auto exps = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[j][i] *= alpha;
-      m = mn;
-    }
-    const float ref = m == -INFINITY ? 0.f : m;
-    float p[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], scale_log2e, -ref));
-    l += ((p[0] + p[4]) + (p[8] + p[12])) + ((p[1] + p[5]) + (p[9] + p[13])) +
-         (((p[2] + p[6]) + (p[10] + p[14])) + ((p[3] + p[7]) + (p[11] + p[15])));
-    u32x4 ph[2], pl[2];
+    for (int i = 0; i < 16; ++i) p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], scale_log2e, -m));
+    return ((p[0] + p[4]) + (p[8] + p[12])) + ((p[1] + p[5]) + (p[9] + p[13])) +
+           (((p[2] + p[6]) + (p[10] + p[14])) + ((p[3] + p[7]) + (p[11] + p[15])));
+  };
+  auto publish = [&](int buf, float lc) __attribute__((always_inline)) {
+    uint32_t ph[8], pl[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const uint32_t hw = pack_bf(p[2 * i], p[2 * i + 1]);
-      ph[i >> 2][i & 3] = hw;
-      if (SPLIT_P) pl[i >> 2][i & 3] = pack_bf(p[2 * i] - lo_bf(hw), p[2 * i + 1] - hi_bf(hw));
+      ph[i] = pack_bf(p[2 * i], p[2 * i + 1]);
+      if (SPLIT_P) pl[i] = pack_bf(p[2 * i] - lo_bf(ph[i]), p[2 * i + 1] - hi_bf(ph[i]));
     }
 #pragma unroll
-    for (int sg = 0; sg < 2; ++sg)
+    for (int x = 0; x < 2; ++x) {
+      *reinterpret_cast<u32x4*>(probs[buf][wave][x][lane]) = u32x4{ph[4 * x], ph[4 * x + 1], ph[4 * x + 2], ph[4 * x + 3]};
+      if constexpr (SPLIT_P) *reinterpret_cast<u32x4*>(probs[buf][wave][2 + x][lane]) = u32x4{pl[4 * x], pl[4 * x + 1], pl[4 * x + 2], pl[4 * x + 3]};
+    }
+    chunk_sums[buf][wave][lane] = lc;
+  };
+  auto round = [&](const Round& x, int c0, int buf) __attribute__((always_inline)) {
+    const int c = c0 + wave;
+    if (c < chunks) {
 #pragma unroll
-      for (int db = 0; db < 4; ++db) {
-        const u32x4 v = x.v[sg][db];
-        const auto v0 = __builtin_amdgcn_permlane16_swap(v[0], v[2], false, false);
-        const auto v1 = __builtin_amdgcn_permlane16_swap(v[1], v[3], false, false);
-        const bf16x8 va = as_frag(u32x4{v0[0], v1[0], v0[1], v1[1]});
-        acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, as_frag(ph[sg]), acc[db], 0, 0, 0);
-        if (SPLIT_P) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, as_frag(pl[sg]), acc[db], 0, 0, 0);
+      for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(x.k[kk]), Q[kk], s, 0, 0, 0);
+      // register i of this lane: key c * 32 + (i & 3) + 8 (i >> 2) + 4 hi
+      if (c * 32 + 32 > limit_all) {  // wave-uniform: some column does not see the whole chunk
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (c * 32 + 4 * hi + (i & 3) + 8 * (i >> 2) >= limit) s[i] = -INFINITY;
+      }
+    }
+    if (c0 == 0) {  // the reference point: the first chunk's maximum (finite: key 0 is visible to every column)
+      if (wave == 0) {
+        const float mc = chunk_max();
+        if (hi == 0) first[n] = mc;
+      }
+      __syncthreads();
+      m = first[n];
+    }
+    bool runs_ahead = false;
+    if (c < chunks) {
+      const float lc = exps();
+      runs_ahead = __any(!(lc <= 256.0f));  // (kDeferMax: see the kernel above)
+      publish(buf, lc);
+    }
+    if (lane == 0) ahead[buf][wave] = runs_ahead;
+    __syncthreads();
+    const bool moved = ahead[buf][0] | ahead[buf][1] | ahead[buf][2] | ahead[buf][3];
+    if (moved) {
+      // a score ran ahead of the reference point (rare): the round's chunks again, one after another, each from the point its
+      // predecessor left
+      for (int w = 0; w < W && c0 + w < chunks; ++w) {
+        if (wave == w) {
+          float alpha = 1.f, lc = exps();
+          if (__any(!(lc <= 256.0f))) {
+            const float mn = fmaxf(m, chunk_max());
+            alpha = __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            lc = exps();
+          }
+          publish(buf, lc);
+          if (hi == 0) points[w][n] = m, alphas[w][n] = alpha;
+        }
+        __syncthreads();
+        m = points[w][n];
+      }
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+      if (c0 + w < chunks) {
+        if (moved) {
+          const float alpha = alphas[w][n];
+          l *= alpha;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[i] *= alpha;
+        }
+        l += chunk_sums[buf][w][lane];
+#pragma unroll
+        for (int sg = 0; sg < 2; ++sg) {
+          const u32x4 v = x.v[w][sg];
+          const auto v0 = __builtin_amdgcn_permlane16_swap(v[0], v[2], false, false);
+          const auto v1 = __builtin_amdgcn_permlane16_swap(v[1], v[3], false, false);
+          const bf16x8 va = as_frag(u32x4{v0[0], v1[0], v0[1], v1[1]});
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, as_frag(*reinterpret_cast<const u32x4*>(probs[buf][w][sg][lane])), acc, 0, 0, 0);
+          if constexpr (SPLIT_P)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, as_frag(*reinterpret_cast<const u32x4*>(probs[buf][w][2 + sg][lane])), acc, 0, 0, 0);
+        }
       }
   };
-  for (int c = wave; c < chunks; c += 2 * W) {
-    if (c + W < chunks) request(b, c + W);
-    attend(a, c);
-    if (c + W >= chunks) break;
-    if (c + 2 * W < chunks) request(a, c + 2 * W);
-    attend(b, c + W);
+  // (two copies of what the waves exchange: a wave is at most one barrier ahead of the one that still reads the round before)
+  for (int c0 = 0; c0 < chunks; c0 += 2 * W) {
+    if (c0 + W < chunks) request(b, c0 + W);
+    round(a, c0, 0);
+    if (c0 + W >= chunks) break;
+    if (c0 + 2 * W < chunks) request(a, c0 + 2 * W);
+    round(b, c0 + W, 1);
   }
 
-  // the waves' sums (over the queries' image: every wave has read it in front of the barrier below): each scaled to the columns' common reference point, added in the waves' order
   l = xor32_sum(l);
-  if (hi == 0) maxes[wave][n] = m, dens[wave][n] = l;
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  // (the queries' image: read by every wave in front of the rounds' barriers)
+#pragma unroll
+  for (int i4 = 0; i4 < 4; ++i4)  // dims 32 wave + 8 i4 + 4 hi .. + 3: half of 16-byte piece 4 wave + i4
+    *reinterpret_cast<u32x2*>(&rows[n][(((wave * 4 + i4) ^ n) & 15) * 8 + 4 * hi]) =
+        u32x2{pack_bf(acc[4 * i4] * inv, acc[4 * i4 + 1] * inv), pack_bf(acc[4 * i4 + 2] * inv, acc[4 * i4 + 3] * inv)};
   __syncthreads();
-  float top = maxes[0][n];
-#pragma unroll
-  for (int w = 1; w < W; ++w) top = fmaxf(top, maxes[w][n]);  // (finite: key 0 is visible to every column)
-  float den = 0.f;
-#pragma unroll
-  for (int w = 0; w < W; ++w) den += maxes[w][n] == -INFINITY ? 0.f : dens[w][n] * __builtin_amdgcn_exp2f(maxes[w][n] - top);
-  const float own = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top) / den;
-#pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4)  // dims 32 db + 8 i4 + 4 hi .. + 3
-      *reinterpret_cast<f32x4*>(&sums[wave][n][((db * 8 + i4 * 2 + hi) ^ n) * 4]) =
-          f32x4{acc[db][4 * i4] * own, acc[db][4 * i4 + 1] * own, acc[db][4 * i4 + 2] * own, acc[db][4 * i4 + 3] * own};
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < 8 / W; ++it) {  // a wave: four columns of 256 bytes at a time
-    const int col = (it * W + wave) * 4 + (lane >> 4), piece = (lane & 15) * 2;
-    f32x4 x = {}, y = {};
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      x += *reinterpret_cast<const f32x4*>(&sums[w][col][(piece ^ col) * 4]);
-      y += *reinterpret_cast<const f32x4*>(&sums[w][col][((piece + 1) ^ col) * 4]);
-    }
-    const int qt = qt0 + col / G;
-    if (qt < q_len)
-      *reinterpret_cast<u32x4*>(out + ((int64_t)(q_start + qt) * n_q_heads + h * G + col % G) * D + (lane & 15) * 8) =
-          u32x4{pack_bf(x[0], x[1]), pack_bf(x[2], x[3]), pack_bf(y[0], y[1]), pack_bf(y[2], y[3])};
+  const int qt = qt0 + col / G;
+  if (qt < q_len) {
+    uint16_t* const op = out + ((int64_t)(q_start + qt) * n_q_heads + h * G + col % G) * D;
+    *reinterpret_cast<u32x4*>(op + j * 8) = *reinterpret_cast<const u32x4*>(&rows[col][((j ^ col) & 15) * 8]);
+    *reinterpret_cast<u32x4*>(op + 64 + j * 8) = *reinterpret_cast<const u32x4*>(&rows[col][(((j + 8) ^ col) & 15) * 8]);
   }
 }
 
@@ -1587,16 +1610,15 @@ extern "C" int mi_paged_attn_decode_ex(const mi_bf16* q, int64_t q_row_stride, c
                      KvStrides{stride_block, stride_head, stride_tile}, stream);
 }
 
-// Which steps take paged_attn_prefill_few_kernel, by its workgroups (sequences x kv heads x blocks of 32 columns): about one per CU; two
-// while the last query block's chunks are many; four where one sequence's alone make more of them.  us per step of 28 layers, 8 kv heads,
-// the kernel for many rows / this one: 1 x 64 rows 1284 / 1204, 1 x 137 1537 / 1435, behind 320 cached 1759 / 1523, 1 x 400 2056 / 1887,
-// 1 x 1024 3061 / 2759, 1 x 2047 (1024 workgroups) 4908 / 4627, 2 x 300 2462 / 2329, 2 x 512 (512) 2763 / 2659, 3 x 200 behind 600 2638 / 2477,
-// 4 x 137 (288) 2028 / 1919, 4 x 256 (512) 2422 / 2402; beyond the lines 6 x 128 (384) 2444 / 2461, 3 x 400 (600) 3086 / 3130, 2 x 1024 (1024)
-// 4117 / 4224, 4 x 512 (1024) 3951 / 4161.
-constexpr int kFewWaves = 4;
+// Which steps take paged_attn_prefill_few_kernel (same bits), by its workgroups (sequences x kv heads x blocks of 32 columns): three per CU,
+// or four where a query block's chunks are as many as there are workgroups.  us per step of 28 layers, 8 kv heads, the kernel for many rows / this
+// one: 1 x 64 rows 1277 / 1189, 1 x 137 1533 / 1451, behind 320 cached 1754 / 1576, 1 x 400 2041 / 1933, 1 x 1024 (512 workgroups) 3033 / 2806,
+// 1 x 2047 (1024) 4949 / 4666, 2 x 512 (512) 2742 / 2605, 2 x 700 (704) 3585 / 3393, 2 x 1024 (1024) 4164 / 4111, 3 x 200 behind 600 2644 / 2443,
+// 4 x 256 (512) 2419 / 2291, 16 x 48 (384) 2287 / 2212, 8 x 128 behind 600 (512) 2911 / 2784; beyond the lines 4 x 512 (1024) 3871 / 3921,
+// 1 x 3000 (1504) 6752 / 7031.
 static bool few_query_rows(int n_pairs, int max_q, int G) {
   const int64_t groups = (int64_t)n_pairs * ((max_q + 32 / G - 1) / (32 / G));
-  return groups <= 320 || (groups <= 512 && max_q >= 256) || (groups <= 1024 && groups < max_q);
+  return groups <= 768 || (groups <= 1024 && groups <= max_q);
 }
 
 static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* prep, const mi_bf16* k_cache,
@@ -1632,12 +1654,12 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
     auto go = [&](auto group) {
       constexpr int GG = decltype(group)::value;
       auto with = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, few, dim3(64 * kFewWaves), 0, st, q, q_row_stride, k_cache, v_cache, block_table, table_stride,
+        hipLaunchKernelGGL(kernel, few, dim3(256), 0, st, q, q_row_stride, k_cache, v_cache, block_table, table_stride,
                            cu_seqlens_q, kv_lens, out, n_q_heads, n_kv_heads, block_size / 16, tpb_shift, sl2, blocks, n_pairs, qp);
         return check_launch();
       };
-      if (prep) return split_p ? with(paged_attn_prefill_few_kernel<GG, true, true, kFewWaves>) : with(paged_attn_prefill_few_kernel<GG, true, false, kFewWaves>);
-      return split_p ? with(paged_attn_prefill_few_kernel<GG, false, true, kFewWaves>) : with(paged_attn_prefill_few_kernel<GG, false, false, kFewWaves>);
+      if (prep) return split_p ? with(paged_attn_prefill_few_kernel<GG, true, true>) : with(paged_attn_prefill_few_kernel<GG, true, false>);
+      return split_p ? with(paged_attn_prefill_few_kernel<GG, false, true>) : with(paged_attn_prefill_few_kernel<GG, false, false>);
     };
     switch (G) {
       case 1: return go(std::integral_constant<int, 1>{});

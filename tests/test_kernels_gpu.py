@@ -776,6 +776,33 @@ def test_prefill_attention_of_few_rows(ops, hq, hkv, block_size, prefill_p):
     assert bool((err <= tol).all()), (err - tol).max().item()
 
 
+@pytest.mark.parametrize("sharpness", [1.0, 9.0])
+def test_prefill_attention_of_few_rows_takes_the_bits_of_many(ops, sharpness):
+    """Every sum in the order of the kernel for many rows (asked for by its request order, variant 1): the same bits, also where scores
+    run ahead of the first chunk's maximum (keys of norm 9: some 40 log2 units between a row's scores)."""
+    gen = torch.Generator().manual_seed(int(sharpness))
+    hq, hkv, bs = 16, 8, 16
+    q_lens, prefix = [137, 1, 64, 33, 100], [0, 300, 0, 129, 31]
+    kv_lens = [a + b for a, b in zip(q_lens, prefix)]
+    T, nb = sum(q_lens), [-(-n // bs) for n in kv_lens]
+    perm = torch.randperm(sum(nb), generator=gen).to(torch.int32)
+    bt = torch.full((len(nb), max(nb)), -1, dtype=torch.int32)
+    o = 0
+    for i, k in enumerate(nb):
+        bt[i, :k] = perm[o:o + k]
+        o += k
+    pos = torch.cat([torch.arange(p, p + k) for p, k in zip(prefix, q_lens)]).to(torch.int64).to(DEV)
+    qkv = torch.randn(T, (hq + 2 * hkv) * 128, generator=gen).bfloat16().to(DEV)
+    qw = torch.full((128,), sharpness, dtype=torch.bfloat16, device=DEV)
+    table = oracle.build_cos_sin_cache(128, 4096, 1e6).to(DEV)
+    kc, vc = (torch.randn(ops.kv_cache_shape(sum(nb), hkv, bs), generator=gen).bfloat16().to(DEV) for _ in range(2))
+    cu = torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32).to(DEV)
+    kvl = torch.tensor(kv_lens, dtype=torch.int32).to(DEV)
+    few, many = (ops.paged_attn_prefill_fused(qkv, qw, 1e-6, pos, table, kc, vc, bt.to(DEV), cu, kvl, max(q_lens), hq, hkv, bs,
+                                              128 ** -0.5, variant=v) for v in (0, 1))
+    assert float(few.float().abs().max()) > 0.1 and torch.equal(few.view(torch.int16), many.view(torch.int16))
+
+
 def test_prefill_attention_chunk_pipeline_stress(ops):
     """Kernel-level guard of the prefill attention's LDS-DMA ring (the counted `s_waitcnt vmcnt(4)` of its chunk
     loop): the bench's prefill step - 16 sequences x 1024 tokens, Qwen3-0.6B heads, block 16 - with SCRAMBLED block
