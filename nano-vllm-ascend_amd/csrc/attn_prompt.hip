@@ -8,7 +8,7 @@
 //   scores   S^T = K Q^T: keys on the MFMA's row axis, the columns on its column axis.
 //            bf16 cache: v_mfma_f32_16x16x32_bf16 with q as bf16 hi + lo (products exact, 16 mantissa bits of q);
 //            fp32 cache: v_mfma_f32_16x16x4_f32.
-//   softmax  scale, bias, cap, mask, running maximum and sum per column in fp32 on the accumulators; a lane holds the keys
+//   softmax  scale, bias, cap, mask, running reference point and sum per column in fp32 on the accumulators; a lane holds the keys
 //            4 kg + {0..3} of the step's two 16-key tiles for its column.
 //   output   O^T += V^T P^T with the contraction slots in the order the scores lie in the registers, so a weight never leaves
 //            its lane.  bf16 cache: weights as hi + lo pairs, V^T by the transposing LDS read (four keys at a lane's channel); fp32
@@ -75,6 +75,62 @@ __device__ __forceinline__ void attend_column(const float* q, const TC* k_cache,
   }
 }
 
+// The rank-th tile (of R rows) in the order of the positions their last rows have, the largest first - the longest walks first, whatever
+// sequences they belong to: workgroups are dispatched in this order, and where there are more than the chip holds the short ones fill
+// the gaps (with sequence after sequence the last sequence's longest walks began when half of the chip was idle).  By one wave for itself, a
+// lane a sequence: bisection for the position that rank tiles lie behind.  us, sequence after sequence / this order: 8 x 1024 rows, 16
+// heads over one 256-channel row (1024 workgroups on 512 places) 271 / 210; 11 prompts, 8112 rows, 8 / 4 heads x 128, window 512: 95 / 89.
+__device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* kv_lens, int n_seqs, int R, int rank, int& s, int& first) {
+  const int lane = threadIdx.x & 63;
+  int q0 = 0, n = 0, past = 0;
+  auto look = [&](int i) __attribute__((always_inline)) {
+    q0 = i < n_seqs ? cu_q[i] : 0, n = i < n_seqs ? cu_q[i + 1] - q0 : 0;
+    past = i < n_seqs ? kv_lens[i] - n : 0;
+  };
+  // tiles whose last row's position is at least p, among the lane's sequence
+  auto from = [&](int p) __attribute__((always_inline)) {
+    const int nt = (n + R - 1) / R;
+    return nt - (past + n - 1 < p ? nt : min(max(p - past, 0) / R, max(nt - 1, 0)));
+  };
+  auto over_all = [&](auto&& f) __attribute__((always_inline)) {  // (sums below 2^24: exact)
+    int c = 0;
+    for (int i = lane; i < n_seqs + lane; i += 64) {
+      if (n_seqs > 64) look(i);
+      c += f();
+    }
+    return (int)wave_sum((float)c);
+  };
+  look(lane);
+  int top = -1;
+  for (int i = lane; i < n_seqs + lane; i += 64) {
+    if (n_seqs > 64) look(i);
+    if (n > 0) top = max(top, past + n - 1);
+  }
+  int lo = 0, hi = (int)wave_max((float)top) + 1, behind = 0;
+  if (rank >= over_all([&] { return from(0); })) return false;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, c = over_all([&] { return from(mid); });
+    if (c > rank) lo = mid;
+    else hi = mid, behind = c;
+  }
+  int k = rank - behind;
+  for (int i0 = 0; i0 < n_seqs; i0 += 64) {
+    look(i0 + lane);
+    const int end = past + n - 1;
+    uint64_t has = __ballot(n > 0 && (lo == end || (lo >= past && lo < end && (lo - past + 1) % R == 0)));
+    const int c = __builtin_popcountll(has);
+    if (k < c) {
+      for (; k > 0; --k) has &= has - 1;
+      const int at = __builtin_ctzll(has);
+      s = i0 + at;
+      first = __builtin_amdgcn_readlane(q0, at) + (lo - __builtin_amdgcn_readlane(past, at)) / R * R;
+      return true;
+    }
+    k -= c;
+  }
+  return false;
+}
+
 // up to 32 DKM key and 16 DVM value channels; smaller heads are zero-padded to that in the images: a branch per fragment would put
 // every fragment's LDS latency behind the one before.  VIK: the values are the leading channels of the key rows.  PAGED16: pages
 // of a multiple of 16 rows.  V4: value rows that start on 4 bytes only (bf16, an even stride), requested in 4-byte pieces.
@@ -83,7 +139,7 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
     const float* __restrict__ q, int64_t ldq, const TC* __restrict__ k_cache, const TC* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, int table_cols, const int32_t* __restrict__ cu_q,
     const int32_t* __restrict__ kv_lens, int n_seqs, int H, int G, int D, int Dv, int block_size, int window, float scale,
-    AttnBias bias, int64_t ldv, const float* __restrict__ gate, int64_t ldg, float* __restrict__ out, int64_t ldo) {
+    AttnBias bias, int64_t ldv, const float* __restrict__ gate, int64_t ldg, float* __restrict__ out, int64_t ldo, bool longest_first) {
   constexpr bool BF = sizeof(TC) == 2;
   constexpr int VEC = 16 / (int)sizeof(TC);                 // channels of a 16-byte chunk
   constexpr int KROW = DKM * 32 * (int)sizeof(TC);          // bytes of a row in the image
@@ -106,15 +162,21 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
   const int Gv = bias.value_heads, gv = g / (G / Gv);
   const int h0 = blockIdx.z * kCols, nh = min(hpg - h0, kCols);   // heads of this kv head that the workgroup takes
   const int R = kCols / nh;                                       // rows of a tile
-  // ---- the tile: sequences in order, a sequence's last rows (the longest walks) first ----
-  int s = 0, t = blockIdx.x, nt = 0;
-  for (; s < n_seqs; ++s) {
-    nt = (cu_q[s + 1] - cu_q[s] + R - 1) / R;
-    if (t < nt) break;
-    t -= nt;
+  int s = 0, first, nr;
+  if (longest_first) {
+    if (!tile_by_end(cu_q, kv_lens, n_seqs, R, (int)blockIdx.x, s, first)) return;  // (the grid is the host's bound)
+    nr = min(R, cu_q[s + 1] - first);
+  } else {
+    // ---- the tile: sequences in order, a sequence's last rows (the longest walks) first ----
+    int t = blockIdx.x, nt = 0;
+    for (; s < n_seqs; ++s) {
+      nt = (cu_q[s + 1] - cu_q[s] + R - 1) / R;
+      if (t < nt) break;
+      t -= nt;
+    }
+    if (s == n_seqs) return;  // (the grid is the host's bound)
+    first = cu_q[s] + (nt - 1 - t) * R, nr = min(R, cu_q[s + 1] - first);
   }
-  if (s == n_seqs) return;  // (the grid is the host's bound)
-  const int first = cu_q[s] + (nt - 1 - t) * R, nr = min(R, cu_q[s + 1] - first);
   const int pos0 = kv_lens[s] - (cu_q[s + 1] - cu_q[s]) + (first - cu_q[s]);
   const int32_t* table = block_tables + (int64_t)s * table_cols;
   const int bs_shift = block_shift(block_size);
@@ -316,24 +378,29 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
         sc[e] = vis ? sc[e] : -INFINITY;
       }
     }
-    float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-    mx = xor_max<32>(xor_max<16>(mx));
-    const float m_new = fmaxf(m, mx);
-    const float mref = m_new == -INFINITY ? 0.f : m_new;   // (a column that has seen nothing yet: its weights are 2^-inf = 0)
-    const float corr = __builtin_amdgcn_exp2f(m - mref);
-    float pv[8], psum = 0.f;
+    // No maximum in the common case: a lane's eight weights against the current reference point add up to at most 2^8 while none of them is
+    // larger (at the first step the point is -inf, the sum is not finite and the comparison fails).  Weights of up to 2^8 are held as
+    // hi + lo, and in fp32, as those below 1 are.  (The maximum, its exchange and the rescaling were a third of a step's vector instructions.)
+    float pv[8];
+    auto weigh = [&](float ref) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      pv[e] = __builtin_amdgcn_exp2f(sc[e] - mref);
-      psum += pv[e];
-    }
-    psum = xor_sum<32>(xor_sum<16>(psum));
-    l = l * corr + psum;
-    m = m_new;
-    if (__any(corr != 1.f)) {  // (a maximum that stays: nothing to rescale)
+      for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(sc[e] - ref);
+      return ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+    };
+    float psum = weigh(m);
+    if (__any(!(psum <= 256.f))) {
+      float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+      mx = xor_max<32>(xor_max<16>(mx));
+      const float m_new = fmaxf(m, mx);
+      const float mref = m_new == -INFINITY ? 0.f : m_new;   // (a column that has seen nothing yet: its weights are 2^-inf = 0)
+      const float corr = __builtin_amdgcn_exp2f(m - mref);
+      psum = weigh(mref);
+      l *= corr;
+      m = m_new;
 #pragma unroll
       for (int f = 0; f < DVM; ++f) oacc[f] *= corr;
     }
+    l += psum;   // (the lane's share)
     if constexpr (BF) {
       u32x4 hi, lo;
 #pragma unroll
@@ -364,6 +431,7 @@ __global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
   }
 
   // the lane holds channels 16 f + 4 kg + {0..3} of its column
+  l = xor_sum<32>(xor_sum<16>(l));
   const float inv = 1.f / (bias.sink ? l + __builtin_amdgcn_exp2f(bias.sink[ch] * kLog2e - m) : l);
   const int64_t row = first + crow;
   float* op = out + row * ldo + (int64_t)ch * Dv + kg * 4;
@@ -415,6 +483,7 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   const int64_t tiles = rows / R + n_seqs;
   if (tiles > 0x7fffffff || (hpg + kCols - 1) / kCols > 65535) return MI_EUNSUPPORTED;
   const dim3 grid((unsigned)tiles, G, (hpg + kCols - 1) / kCols);
+  const bool longest_first = tiles * G * grid.z > 512;   // (two workgroups per CU: with no more than that all begin at once)
   // us, the kernels before / this one: 8 x 1024 rows, 16 heads over one 256-channel row (values inside it) 917 / 271; 11 prompts,
   // 8112 rows, 8 / 4 heads x 128, window 512: 189 / 96; fp32 pages, 733 rows of 16 sequences behind up to 700: 760 / 83.  With K
   // and V through registers into the image (V transposed on the way): 345, 104, 86.
@@ -431,7 +500,7 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
 #define MI_PROMPT(TC, DKM, DVM, NST, ...)                                                                                  \
   hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
                      static_cast<const TC*>(k_cache), static_cast<const TC*>(v_cache), bt, cols, cu_q, kv_lens, n_seqs, H, G, D, Dv, \
-                     block_size, window, scale, bias, ldv, gate, ldg, out, ldo)
+                     block_size, window, scale, bias, ldv, gate, ldg, out, ldo, longest_first)
   // (WIDE: stages of the ring at 256 channels of keys and of values.  Pages of 24 rows, 400 rows of 4 sequences, 8 / 4 heads, us, the kernels
   // before / 256 channels for every head / by head size: fp32 x 64 72 / 177 / 43, x 128 144 / 183 / 79; bf16 x 64 46 / 46 / 21.)
 #define MI_PROMPT_SIZES(TC, PAGED16, WIDE)                                   \

@@ -110,6 +110,36 @@ def test_masks_and_biases(dtype, form):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,G,seqs", [(6, 6, [(i * 37 % 90, (i * 53) % 48) for i in range(100)]), (12, 6, [(40, 700), (0, 0), (3, 257), (0, 1000)] * 3),
+                                      (24, 1, [(0, 300)] * 10 + [(500, 61)] * 9), (8, 8, [(i % 3, 64 + i % 2) for i in range(64)]),
+                                      (130, 5, [(0, 0)] * 63 + [(7, 129), (0, 127)] * 2 + [(i, 1) for i in range(60)])])
+def test_more_tiles_than_the_chip_holds(dtype, H, G, seqs):
+    """the longest walks first, over all sequences: every tile once, whatever ends, equal ends, empty sequences and numbers of sequences"""
+    _case(dtype, H, G, 32, 32, 16, seqs)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("step", [2.0, 7.9, 8.1, 40.0])
+def test_scores_that_grow_along_the_keys(dtype, step):
+    """maxima that the reference point follows at once, later or never: keys whose scores rise by `step` powers of two per 32 keys"""
+    n, D, block = 160, 32, 16
+    k = torch.zeros(10, 1, block, D, device="cuda")
+    p = torch.arange(n, device="cuda").view(10, 1, block)
+    k[..., 0] = (p // 32) * step            # (integers and tenths: bf16 rounds them as the oracle reads them)
+    k, v = k.to(dtype), torch.randn(10, 1, block, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)).to(dtype)
+    q = torch.zeros(n, D, device="cuda")
+    q[:, 0] = torch.linspace(-1, 1, n, device="cuda")
+    table = torch.arange(10, device="cuda").int().view(1, 10)
+    cu, kv = torch.tensor([0, n], dtype=torch.int32, device="cuda"), torch.tensor([n], dtype=torch.int32, device="cuda")
+    got = ops.paged_attention_f32(q, k, v, D, table, cu, kv, 1, 1, D, D, block, 2 ** 31 - 1, math.log(2))
+    s = (q.double() @ k.double().view(n, D).T * math.log(2)).masked_fill(torch.ones(n, n, device="cuda").triu(1).bool(), -math.inf)
+    want = torch.softmax(s, 1) @ v.double().view(n, D)
+    # (scores of up to 160: 2^-17 of their size in a weight's exponent on bf16 pages, 2^-22 on fp32 pages, as the module's bounds say)
+    tol = (2e-5 if dtype == torch.bfloat16 else 1e-5) * max(1.0, 4 * step / 30) * float(want.abs().max())
+    assert float((got.double() - want).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("D,Dv", [(256, 256), (224, 160)])
 def test_values_inside_the_key_rows(dtype, D, Dv):
     _case(dtype, 16, 1, D, Dv, 64, SEQS, vik=True, sink=True)
