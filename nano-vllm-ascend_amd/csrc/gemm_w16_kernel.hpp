@@ -332,15 +332,17 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   // 1 KiB, and 18 for whole lines: 6.8 us per tile, whatever the other CUs do.)
   constexpr int NU = F32 ? 4 : NF / 4, NSLAB = 4 * NU;
   const uint32_t stg_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + 2 * W16_STEP_BYTES) + wave * W4_STAGE_BYTES;
-  // after the exchange lane (n16, q4) holds chunk 2 * (2 pr + (q4 & 1)) + (q4 >> 1) of row 16 ts + n16 (pr: fragment pair)
-  const uint32_t stg_w = stg_base + (uint32_t)n16 * 128 + (uint32_t)(((F32 ? q4 : 2 * (q4 & 1) + (q4 >> 1)) ^ (n16 & 7)) << 4);
-  const uint32_t stg_r = stg_base + (uint32_t)(lane >> 3) * 128 + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
   const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (uint32_t)a.M * (uint32_t)a.ldy * 2, 0x00020000);
-  const uint32_t y_lane = (uint32_t)(lane >> 3) * (uint32_t)a.ldy * 2 + (uint32_t)(lane & 7) * 16;
   auto epilogue_lines = [&](int m0, int n0) __attribute__((always_inline)) {
     u32x4 out[4], back[4];
-    uint32_t w_addr = stg_w;  // (opaque per tile: otherwise the chunk addresses are hoisted out of the tile loop and spilled)
-    asm volatile("" : "+v"(w_addr));
+    // (opaque per tile: otherwise the addresses are hoisted out of the tile loop and spilled, and a reload waits for every piece and store in
+    // flight - 0.9 us per tile)
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    // after the exchange lane (n16, q4) holds chunk 2 * (2 pr + (q4 & 1)) + (q4 >> 1) of row 16 ts + n16 (pr: fragment pair)
+    const uint32_t w_addr = stg_base + (uint32_t)(l & 15) * 128 + (uint32_t)(((F32 ? l >> 4 : 2 * ((l >> 4) & 1) + (l >> 5)) ^ (l & 7)) << 4);
+    const uint32_t stg_r = stg_base + (uint32_t)(l >> 3) * 128 + (uint32_t)(((l & 7) ^ (l >> 3)) << 4);
+    const uint32_t y_lane = (uint32_t)(l >> 3) * (uint32_t)a.ldy * 2 + (uint32_t)(l & 7) * 16;
     auto convert = [&](int slab) __attribute__((always_inline)) {
       const int tt = slab / NU, u = slab % NU;
 #pragma unroll
