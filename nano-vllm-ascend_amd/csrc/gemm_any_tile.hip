@@ -101,14 +101,24 @@ __device__ __forceinline__ f32x4 any_value(const A& a, float scale, f32x4 v, f32
   }
   if (a.bias1) v += b1;
   if (A::kDual && a.bias2) v2 += b2;
-  return any_act(a, v, v2) * a.alpha;
+  v = any_act(a, v, v2);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] *= a.alpha;
+  return v;
 }
+// (a bias is added in the branch that loads it: joined behind it, every store of the lane before is waited for, 2 us of a 64-row tile each)
 template <class A>
 __device__ __forceinline__ void any_store(const A& a, const AnyRow& row, int n, f32x4 v, f32x4 v2) {
   if (row.y < 0 || n >= a.N) return;
-  const f32x4 none = {};
-  v = any_value(a, row.scale, v, v2, a.bias1 ? *reinterpret_cast<const f32x4*>(a.bias1 + n) : none,
-                A::kDual && a.bias2 ? *reinterpret_cast<const f32x4*>(a.bias2 + n) : none);
+  if (a.row_scale) {
+    v *= row.scale;
+    if (A::kDual) v2 *= row.scale;
+  }
+  if (a.bias1) v += *reinterpret_cast<const f32x4*>(a.bias1 + n);
+  if (A::kDual && a.bias2) v2 += *reinterpret_cast<const f32x4*>(a.bias2 + n);
+  v = any_act(a, v, v2);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] *= a.alpha;
   if (a.y16) *reinterpret_cast<u32x2*>(a.y16 + row.y * a.ldy + n) = u32x2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
   else *reinterpret_cast<f32x4*>(a.y32 + row.y * a.ldy + n) = v;
 }
@@ -193,21 +203,24 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
                : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) ||
                    (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
     return 0;
-  const int tf = dual ? 128 : 256;
   if (n_groups && act == MI_ACT_SOFTCAP) return 0;   // (no group has one)
-  // 64-row tiles, or 256-row ones (the persistent kernel) where those are enough for the chip and not mostly padding; 128-row ones lie
-  // between the two nearly everywhere (two long-K weights of some 64 rows a group alone 99 / 103 / 119) and are left to softcap.
+  // 64-row tiles while they are few or a group's rows fewer than a larger tile's padding would be; the persistent kernel's 256-row ones where
+  // 128-row ones are more than the chip holds (two workgroups per CU) and not mostly padding.
+  const auto tiles = [=](int t, int f) { return (int64_t)((n_groups ? rows / t + n_groups / 2 : (rows + t - 1) / t)) * ((N + f - 1) / f); };
   if (n_groups) {
-    // us of both products, 64- / 128- / 256-row tiles: 32 experts of 512 x 1024, 48 rows each 37 / 57 / 49, 64 43 / 58 / 48, 96 55 / 59 / 49,
-    // 128 66 / 64 / 49, 512 118 / 114 / 91; 64 of 768 x 2048, 64 154 / 157 / 172, 96 173 / 165 / 173, 128 224 / 219 / 186, 512 647 / 554 / 400;
-    // 128 of 256 x 1024, 48 70 / 71 / 62, 128 94 / 93 / 68; 8 of 512 x 1024 (48 and 80 tiles of 256) 256 rows 40 / 53 / 47, 512 63 / 63 / 48
-    if (dual && K >= 2048 && rows >= 48 * (int64_t)n_groups && rows < 80 * (int64_t)n_groups) return 128;
-    return rows >= 80 * (int64_t)n_groups && (rows / 256 + n_groups / 2) * (int64_t)((N + tf - 1) / tf) >= 80 ? 256 : 64;
+    // us of both products from cold weights, 64- / 128- / 256-row tiles, uneven groups of this mean: 32 experts of 512 x 1024, 48 rows 33 / 35 / 50,
+    // 96 43 / 40 / 50, 192 52 / 43 / 52, 256 62 / 67 / 52, 512 105 / 103 / 97; 64 of 768 x 2048, 48 134 / 150 / 170, 64 149 / 156 / 172, 96 179 / 161 /
+    // 192, 128 213 / 194 / 199, 192 272 / 257 / 209, 512 607 / 506 / 377; 8 of 512 x 1024, 96 18 / 27 / 47, 256 27 / 28 / 49, 512 41 / 38 / 50;
+    // 128 of 256 x 1024, 48 56 / 70 / 67, 96 68 / 77 / 100, 160 97 / 93 / 103, 192 110 / 105 / 105, 256 138 / 132 / 108
+    // (K below 512 was not measured: no more than the padding's rule there)
+    if (rows < (dual ? K >= 2048 ? 64 : 88 : 72) * (int64_t)n_groups || (K >= 512 && tiles(64, 64) < 512)) return 64;
+    return rows >= 160 * (int64_t)n_groups && tiles(128, dual ? 64 : 128) > 512 ? 256 : 128;
   }
-  // us, 64- / 128- / 256-row tiles: 2000 x 2048 x 1024 (1024 tiles of 64 x 64) 24 / 32 / 29, 3000 (1504) 39 / 36 / 30; 4000 x 1024 x 1024 (1008)
-  // 22 / 32 / 29, 6000 39 / 36 / 30; 2000 x 2048 x 2048 39 / 40 / 45, 3000 55 / 50 / 46; 500 x 6144 x 2048 (768) 36 / 37 / 44, 700 (1056) 59 / 49 / 45
-  if ((int64_t)((rows + 63) / 64) * ((N + 63) / 64) <= 1024) return 64;
-  return act != MI_ACT_SOFTCAP ? 256 : 128;
+  // us, cold weights, 64- / 128- / 256-row tiles: 2000 x 1024 x 1024 (512 / 128 / 32 tiles) 12 / 16 / 26, 2000 x 2048 x 1024 (1024 / 256 / 64) 23 / 18 / 28,
+  // 4000 x 2048 x 1024 (2016 / 512 / 128) 33 / 27 / 30, 3000 x 3072 x 1024 (2256 / 576 / 144) 41 / 37 / 31; 1000 x 2048 x 2048 (512 / 128 / 32) 22 / 26 / 47,
+  // 1300 (672 / 176 / 48) 29 / 27 / 44, 4000 (2016 / 512 / 128) 53 / 42 / 48, 1300 x 6144 x 2048 (2016 / 528 / 144) 76 / 61 / 46
+  if (tiles(64, 64) <= 512) return 64;
+  return act != MI_ACT_SOFTCAP && tiles(128, dual ? 64 : 128) > 512 ? 256 : 128;
 }
 
 template <int ACT, bool DUAL, bool GATHER, bool HALF>
@@ -364,15 +377,17 @@ extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const
 
 // ---- the experts of moe.hip (bf16 activations and weights as they are stored, row-major) on the tile kernels: steps that bring prompts ----
 // moe.hip's kernels keep 16 features' weights in registers and walk an expert's pairs 16 at a time, a round trip and two barriers each:
-// made for the few pairs of a decode step.  us of a block (route to combine) with them / here on 64-row / on 256-row tiles:
-//   64 experts of 768 x 2048     16 pairs each 155 / 161 / 190   24 182 / 162 / 190   64 306 / 192 / 199   128 523 / 249 / 215   512 1834 / 648 / 392
-//   32 of 512 x 1024             24 47 / 48 / 57   32 53 / 48 / 58   64 72 / 55 / 58   128 111 / 80 / 61   512 358 / 142 / 109
-//   8 of 512 x 1024              64 42 / 45 / 53   256 69 / 52 / 57   512 114 / 75 / 60;  8 of 1536 x 4096  32 97 / 83 / 130   128 237 / 145 / 140
-// (128-row tiles are between the two nearly everywhere.)  A step of 8 x 1024 tokens, four layers of 64 experts: 15.7 -> 3.9 ms.
+// made for the few pairs of a decode step.  us of a block (route to combine) with them / here on 64- / 128- / 256-row tiles:
+//   64 experts of 768 x 2048     8 pairs each 127 / 146 / 162 / 185   16 153 / 148 / 164 / 188   64 306 / 173 / 183 / 197   128 530 / 229 / 236 / 212
+//                                512 1843 / 620 / 524 / 385
+//   32 of 512 x 1024             8 34 / 34 / 38 / 56   16 40 / 35 / 38 / 56   64 72 / 44 / 44 / 57   192 155 / 62 / 56 / 63   512 360 / 115 / 110 / 106
+//   8 of 512 x 1024              32 22 / 27 / 36 / 51   64 28 / 28 / 36 / 52   256 67 / 38 / 40 / 55   512 114 / 53 / 51 / 58
+//   8 of 1536 x 4096             16 71 / 71 / 82 / 126   64 145 / 110 / 107 / 131;   128 of 768 x 2048   8 242 / 237 / 250 / 281   128 1017 / 417 / 401 / 335
+// A step of 8 x 1024 tokens, four layers of 64 experts: 15.7 -> 3.9 ms.
 static int moe_tile_rows(int pairs, int G, int ff, int width) {
   if (pairs < 1 || G < 1 || width % BK || ff % BK || width % 8 || ff % 8) return 0;
   if (2 * (int64_t)ff > INT32_MAX || ((int64_t)G * 2 * ff + 256) * width * 2 >= (int64_t)1 << 31) return 0;   // (32-bit offsets into gate_up)
-  if (pairs < 24 * (int64_t)G || (int64_t)pairs * (ff + width) < 1600000) return 0;
+  if (pairs < 16 * (int64_t)G || (int64_t)pairs * (ff + width) < 800000) return 0;
   const int a = tile_rows_for(pairs, ff, width, G, true, MI_ACT_SILU, false), b = tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE, false);
   return a < b ? a : b;
 }

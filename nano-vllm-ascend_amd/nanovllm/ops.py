@@ -1009,30 +1009,28 @@ def moe_forward(x, router_logits, gate_up_packed, down_packed, top_k: int, all_r
     ids = torch.empty((T, top_k), dtype=torch.int32, device=dev)
     w = torch.empty((T, top_k), dtype=_BF16, device=dev)
     check(lib.mi_moe_route(ptr(router_logits), T, E, top_k, ptr(ids), ptr(w), stream()), "mi_moe_route")
-    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    pair_token = torch.empty(T * top_k, dtype=torch.int32, device=dev)
-    pair_index = torch.empty(T * top_k, dtype=torch.int32, device=dev)
-    check(lib.mi_moe_sort(ptr(ids), T, top_k, E, ptr(offsets), ptr(pair_token), ptr(pair_index), stream()),
-          "mi_moe_sort")
-    act = torch.empty((T * top_k, inter), dtype=_BF16, device=dev)
-    y = torch.empty((T * top_k, H), dtype=_BF16, device=dev)  # row t * top_k + j: the same on every TP rank
-    n = lib.mi_moe_tiles_bytes(T * top_k, E, inter, H) if gate_up is not None and down is not None and T else 0
+    pairs, st = T * top_k, stream()
+    plan = torch.empty(E + 1 + 2 * pairs, dtype=torch.int32, device=dev)   # the experts' offsets, the pairs' tokens, their places
+    offsets = ptr(plan)
+    pair_token = offsets + 4 * (E + 1)
+    pair_index = pair_token + 4 * pairs
+    check(lib.mi_moe_sort(ptr(ids), T, top_k, E, offsets, pair_token, pair_index, st), "mi_moe_sort")
+    n = lib.mi_moe_tiles_bytes(pairs, E, inter, H) if gate_up is not None and down is not None and T else 0
+    act = torch.empty(pairs * inter + n // 2, dtype=_BF16, device=dev)   # (behind the pairs' activations: the tiles' table)
+    y = torch.empty((pairs, H), dtype=_BF16, device=dev)  # row t * top_k + j: the same on every TP rank
     if n and not (x.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16:
         require_gpu(gate_up, down)
         _bf16(gate_up, down)
         assert gate_up.shape == gate_up_packed.shape and down.shape == down_packed.shape and gate_up.is_contiguous() and down.is_contiguous()
-        table = torch.empty(n, dtype=torch.uint8, device=dev)
-        check(lib.mi_moe_tiles(ptr(x), T, ptr(gate_up), ptr(down), ptr(offsets), ptr(pair_token), ptr(pair_index), ptr(act), ptr(y),
-                               T * top_k, E, H, inter, ptr(table), n, stream()), "mi_moe_tiles")
+        check(lib.mi_moe_tiles(ptr(x), T, ptr(gate_up), ptr(down), offsets, pair_token, pair_index, ptr(act), ptr(y), pairs, E, H, inter,
+                               ptr(act) + pairs * inter * 2, n, st), "mi_moe_tiles")
     else:
-        check(lib.mi_moe_gate_up(ptr(x), ptr(gate_up_packed), ptr(offsets), ptr(pair_token), ptr(act), E, H, inter,
-                                 stream()), "mi_moe_gate_up")
-        check(lib.mi_moe_down(ptr(act), ptr(down_packed), ptr(offsets), ptr(pair_index), ptr(y), E, H, inter, stream()),
-              "mi_moe_down")
+        check(lib.mi_moe_gate_up(ptr(x), ptr(gate_up_packed), offsets, pair_token, ptr(act), E, H, inter, st), "mi_moe_gate_up")
+        check(lib.mi_moe_down(ptr(act), ptr(down_packed), offsets, pair_index, ptr(y), E, H, inter, st), "mi_moe_down")
     if all_reduce is not None:
         y = all_reduce(y)
     out = torch.empty((T, H), dtype=_BF16, device=dev)
-    check(lib.mi_moe_combine(ptr(y), ptr(w), ptr(out), T, top_k, H, stream()), "mi_moe_combine")
+    check(lib.mi_moe_combine(ptr(y), ptr(w), ptr(out), T, top_k, H, st), "mi_moe_combine")
     return out, ids, w
 
 

@@ -1120,7 +1120,8 @@ def test_moe_block_golden(ops, golden_moe_block):
         _assert_moe_close(got, bf(g[f"{tag}_y"]))
 
 
-@pytest.mark.parametrize("T,H,E,K,I,tile", [(700, 1024, 8, 2, 512, 64), (2600, 1024, 8, 2, 512, 256), (1100, 512, 32, 4, 384, 256), (500, 640, 16, 8, 192, 64)])
+@pytest.mark.parametrize("T,H,E,K,I,tile", [(700, 1024, 8, 2, 512, 64), (2600, 1024, 8, 2, 512, 128), (5000, 1024, 8, 2, 512, 256), (1300, 512, 32, 4, 384, 128),
+                                            (500, 640, 16, 8, 192, 64)])
 @pytest.mark.parametrize("uneven", [False, True])
 def test_moe_block_from_the_stored_weights(ops, T, H, E, K, I, tile, uneven):
     """Steps of many pairs on the tile kernels (mi_moe_tiles): the same routing, an output each row's sums over K in another order apart
