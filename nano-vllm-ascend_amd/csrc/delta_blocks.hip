@@ -10,13 +10,13 @@
 //   u_t = beta_t (v_t - D_t - sum_j A_tj u_j)   =>   U = T (V - D),  T = (1 + diag(beta) A)^-1 diag(beta)   (16 x 16, lower triangular)
 //   O = E + B U,      S <- diag(P_15) S0 + sum_j (k_j P_j15) u_j^T
 // blocks_prepare_kernel (a workgroup per block and head, all blocks at once) leaves (k P), (q P), (k P_.15), P_15, B and T of a block as
-// one record in MFMA operand order; blocks_walk_kernel (a wave per 16 value columns, S in its registers as MFMA accumulators, which
+// one record in MFMA operand order; blocks_walk_kernel (two waves per 16 value columns, S in their registers as MFMA accumulators, which
 // are the next block's B operand as they stand) walks a sequence's records.
 //
-// What bounds it: the chain of a sequence's blocks; 104 matrix instructions of 32 cycles each (128 channels) are 1.4 us, the vector
-// work between them brings a block to 2.5 us (2.7 with the accumulators copied to be scaled: the Makefile's flag), against 0.71 us per
-// ROW of the row-by-row walk (LDS reads, cross-lane sums, plain FMAs).
-// 8 sequences of 1024 rows, 8 heads, 128 x 128: 809 us row by row, 294 so (preparation 83, walk 175).  The error against 64 bits is
+// What bounds it: the longest sequence's chain of blocks - 56 matrix instructions of 32 cycles a wave (128 channels), the LDS reads, sums and
+// barriers between them -, and the matrix pipe where two workgroups share a CU, against 0.71 us per ROW of the row-by-row walk (LDS reads,
+// cross-lane sums, plain FMAs).
+// 8 sequences of 1024 rows, 8 heads, 128 x 128: 809 us row by row, 294 so with one wave for all channels (preparation 83, walk 175).  The error against 64 bits is
 // the row-by-row one's or less (rms of the results, 64 .. 1400 rows and decays from 0.05 to 1: 0.87 to 0.98 of it).  A NaN or an
 // infinity in a row must not reach the rows in front of it through the zeros above the diagonals of T and B: see causal() below.
 #include <type_traits>
@@ -227,62 +227,97 @@ __global__ __launch_bounds__(256) void blocks_prepare_kernel(BlockArgs a) {
   for (int d = tid; d < DP; d += 256) rec_b[512 + d] = gamma[d];
 }
 
-// grid: (sequences, heads, value columns / 64); a wave takes 16 columns.  Ring of three records (two where three do not fit: 256 channels) (with the rows' values behind each, a
-// wave's own 16 columns) by LDS-DMA two blocks ahead; in front of a group's matrix instructions stand the LDS reads of the next one.
+// The rank-th sequence in the order of the rows it brings, the most first: the longest chains begin first and alone.  By one wave for itself.
+__device__ __forceinline__ int by_length(const int32_t* cu_q, int n_seqs, int rank) {
+  const int lane = threadIdx.x & 63;
+  auto rows = [&](int i) __attribute__((always_inline)) { return i < n_seqs ? cu_q[i + 1] - cu_q[i] : -1; };
+  const int mine = rows(lane);
+  auto count = [&](auto&& f) __attribute__((always_inline)) {
+    int c = __popcll(__ballot(f(mine)));
+    for (int i0 = 64; i0 < n_seqs; i0 += 64) c += __popcll(__ballot(f(rows(i0 + lane))));
+    return c;
+  };
+  int lo = 0, hi = cu_q[n_seqs] + 1, behind = 0;   // count(n >= lo) > rank >= count(n >= hi) = behind
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, c = count([&](int n) { return n >= mid; });
+    if (c > rank) lo = mid;
+    else hi = mid, behind = c;
+  }
+  for (int i0 = 0, k = rank - behind; i0 < n_seqs; i0 += 64) {
+    uint64_t has = __ballot(rows(i0 + lane) == lo);
+    const int c = __popcll(has);
+    if (k < c) {
+      for (; k > 0; --k) has &= has - 1;
+      return i0 + __builtin_ctzll(has);
+    }
+    k -= c;
+  }
+  return 0;   // (not reached: ranks are below n_seqs)
+}
+
+// grid: (heads, value columns / 32, sequences) in one, the longest sequences first; two waves take 16 columns, each half of the key channels: what
+// one has read of the state meets the other's in LDS, both then have the block's u; the rows' results, which nothing waits for, are put together
+// beside the next block's products.  Rings (three records, two where three do not leave room for two workgroups per CU), with the rows' values
+// behind each, by LDS-DMA a block or two ahead, its pieces between the products; in front of a group's matrix instructions stand the LDS reads of
+// the next one.  us, before (one wave for all channels, 64 columns a workgroup, sequences in order) / so: 11 sequences, 8112 rows, 8 heads of 128 x
+// 128 219 / 158 (sequences in order 201; 64 columns, eight waves in step 215); 728 rows of 16 sequences 58 / 39.
 template <int DT>
-__global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
-  constexpr int DP = 16 * DT, REC = record_floats(DP), PIECES = REC / 256, PP = (PIECES + 3) / 4, IMG = REC * 4 + 4096;
-  constexpr int NST = 3 * IMG <= 163840 ? 3 : 2;
-  __shared__ __attribute__((aligned(1024))) char lds[NST * IMG];
+__global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
+  constexpr int DP = 16 * DT, HT = DT / 2, KT = HT < 4 ? HT : 4, REC = record_floats(DP), PIECES = REC / 256, PP = (PIECES + 3) / 4, IMG = REC * 4 + 2048;
+  constexpr int NST = 3 * IMG + 6144 <= 81920 ? 3 : 2;
+  __shared__ __attribute__((aligned(1024))) char lds[NST * IMG + 6144];   // (behind the ring: four waves' D, two waves' E)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
-  const int s = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 64 + wave * 16 + r16;
+  const int cg = wave & 1, half = wave >> 1;   // 16 columns, HT tiles of 16 key channels
+  // heads, their columns (one XCD's, where the heads are a multiple of eight: they share the records), sequences
+  const int zs = (a.Dv + 31) / 32, hz = (int)blockIdx.x % (a.H * zs), h = hz % a.H, col = hz / a.H * 32 + cg * 16 + r16;
+  const int s = by_length(a.cu_q, a.n_seqs, (int)blockIdx.x / (a.H * zs));
   const int r0 = a.cu_q[s], n = a.cu_q[s + 1] - r0;
   if (n == 0) return;
   const int nb = (n + kB - 1) / kB;
   const char* const recs = reinterpret_cast<const char*>(a.records + ((int64_t)first_record(r0, s) * a.H + h) * REC);
   const int64_t rec_stride = (int64_t)a.H * REC * 4;
-  const float* vp[4];   // the next block's rows 4 kg + r at this lane's column
+  const float* vp[2];   // the next block's rows 4 kg + 2 half + i at this lane's column
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    vp[r] = a.qkv + (int64_t)(r0 + min(4 * kg + r, n - 1)) * a.ld + a.v_off + (int64_t)h * a.Dv + min(col, a.Dv - 1);
-  // PP + 4 requests, whatever the block (beyond the end: the last one's again; rows beyond the end: the last row's)
-  auto issue = [&](int b, int st) __attribute__((always_inline)) {
-    const int bb = min(b, nb - 1);
+  for (int i = 0; i < 2; ++i)
+    vp[i] = a.qkv + (int64_t)(r0 + min(4 * kg + 2 * half + i, n - 1)) * a.ld + a.v_off + (int64_t)h * a.Dv + min(col, a.Dv - 1);
+  // PP + 2 requests, whatever the block (beyond the end: the last one's again; rows beyond the end: the last row's)
+  auto piece = [&](int b, int st, int i) __attribute__((always_inline)) {
+    const int p = min(wave * PP + i, PIECES - 1);
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(recs + min(b, nb - 1) * rec_stride + p * 1024 + (uint32_t)(lane * 16)),
+                                     (__attribute__((address_space(3))) void*)(lds + st * IMG + p * 1024), 16, 0, 0);
+  };
+  auto values = [&](int b, int st) __attribute__((always_inline)) {
     char* const to = lds + st * IMG;
 #pragma unroll
-    for (int i = 0; i < PP; ++i) {
-      const int p = min(wave * PP + i, PIECES - 1);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(recs + bb * rec_stride + p * 1024 + (uint32_t)(lane * 16)),
-                                       (__attribute__((address_space(3))) void*)(to + p * 1024), 16, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vp[r],
-                                       (__attribute__((address_space(3))) void*)(to + REC * 4 + wave * 1024 + r * 256), 4, 0, 0);
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vp[i],
+                                       (__attribute__((address_space(3))) void*)(to + REC * 4 + cg * 1024 + (2 * half + i) * 256), 4, 0, 0);
     const int left = n - 1 - (b + 1) * kB;   // rows behind the next block's first
     if (left >= kB - 1) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vp[r] += (int64_t)kB * a.ld;
+      for (int i = 0; i < 2; ++i) vp[i] += (int64_t)kB * a.ld;
     } else if (left >= 0) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vp[r] += (int64_t)(kB + min(4 * kg + r, left) - (4 * kg + r)) * a.ld;
+      for (int i = 0; i < 2; ++i) vp[i] += (int64_t)(kB + min(4 * kg + 2 * half + i, left) - (4 * kg + 2 * half + i)) * a.ld;
     }
   };
-  // the state: S[m][r] = key channel 16 m + 4 kg + r of this lane's column; in memory as the row-by-row kernels keep it
+  // the state: S[m][r] = key channel 16 (half HT + m) + 4 kg + r of this lane's column; in memory as the row-by-row kernels keep it
   const int cb = col / kStateCols, cbs = (a.Dv + kStateCols - 1) / kStateCols, cc = col % kStateCols;
   const bool has_state = cb < cbs, has_col = col < a.Dv;
-  float* const st = a.state + (((int64_t)a.slot_ids[s] * a.H + h) * cbs + cb) * (DP * kStateCols);
-  f32x4 S[DT];
+  float* const st = a.state + (((int64_t)a.slot_ids[s] * a.H + h) * cbs + cb) * (DP * kStateCols) + half * HT * (16 * kStateCols);
+  f32x4 S[HT];
 #pragma unroll
-  for (int m = 0; m < DT; ++m) S[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < HT; ++m) S[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (has_state && a.kv_lens[s] > n) {
 #pragma unroll
-    for (int m = 0; m < DT; ++m) {
+    for (int m = 0; m < HT; ++m) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[m][r] = st[(4 * m + r) * (4 * kStateCols) + cc * 4 + kg];
     }
   }
+  const uint32_t x_mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + NST * IMG) + wave * 1024 + lane * 16;
+  const uint32_t x_other = half ? x_mine - 2048 : x_mine + 2048, x_e = x_mine + (half ? 2048 : 4096);
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   float* op = a.out + (int64_t)(r0 + 4 * kg) * a.ldo + (int64_t)h * a.Dv + col;   // (formed beyond the columns, not used there)
   auto store = [&](int b) __attribute__((always_inline)) {
@@ -298,28 +333,50 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
     op += (int64_t)kB * a.ldo;
   };
 #pragma unroll
-  for (int i = 0; i + 1 < NST; ++i) issue(i, i);
+  for (int i = 0; i + 1 < NST; ++i) {
+#pragma unroll
+    for (int q = 0; q < PP; ++q) piece(i, i, q);
+    values(i, i);
+  }
+  f32x4 e_own = {}, x = {}, w = {}, u = {};
+  // block b's rows, when the halves' sums of E have met (in the next block, beside its products)
+  auto finish = [&](int b) __attribute__((always_inline)) {
+    f32x4 e_other;
+    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(e_other) : "v"(x_e) : "memory");
+    e_other += e_own;
+    o = e_other + x;
+    float zero = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) zero = fmaf(o[r], 0.f, zero);
+    // (the state has what is not finite either way; the whole wave takes the branch)
+    if (__builtin_expect(__any(zero != 0.f), 0)) {
+      const char* const at = recs + b * rec_stride + 3 * DP * kB * 4 + lane * 16;
+      const f32x4 x2 = causal(*reinterpret_cast<const f32x4*>(at), causal(*reinterpret_cast<const f32x4*>(at + 1024), w, u, kg), x, kg);
+      o = e_other + x2;
+    }
+    store(b);
+  };
   int cur = 0;
   for (int b = 0; b < nb; ++b) {
     // record b has landed (a ring of three: record b + 1's requests may be out); everybody is done with record b - 1: its place is free
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * (PP + 4)) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * (PP + 2)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
-    if (b > 0) store(b - 1);   // (here, not behind the block: the wait above would have to see them home)
-    issue(b + NST - 1, cur == 0 ? NST - 1 : cur - 1);
+    if (b > 0 && half == 0) finish(b - 1);   // (the other half's products keep the matrix pipe busy)
+    const int next = cur == 0 ? NST - 1 : cur - 1;
     const char* const img = lds + cur * IMG;
     cur = cur == NST - 1 ? 0 : cur + 1;
-    const char* const rec = img + lane * 16;
+    const char* const rec = img + lane * 16 + half * HT * 1024;
     const char* const rec_q = rec + DP * kB * 4;
     const char* const rec_k = rec_q + DP * kB * 4;
-    const char* const rec_b = rec_k + DP * kB * 4;
-    const char* const gam = rec_b - lane * 16 + 2048 + kg * 16;   // P_15 of this lane's channels 16 m + 4 kg ..
+    const char* const rec_b = img + lane * 16 + 3 * DP * kB * 4;
+    const char* const gam = rec_b - lane * 16 + 2048 + kg * 16 + half * HT * 64;   // P_15 of this lane's channels 16 m + 4 kg ..
     auto vec = [](const char* p) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(p); };
     f32x4 d[8], e[8];   // (eight chains: each is an eighth as long, and so is its rounding)
 #pragma unroll
     for (int r = 0; r < 8; ++r) d[r] = e[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    f32x4 pf[2][2], qf[2][2], gf[2][2], kf[2][4], u, tf = vec(rec_b + 1024), bf = vec(rec_b);
+    f32x4 pf[2][2], qf[2][2], gf[2][2], kf[2][4], tf = vec(rec_b + 1024), bf = vec(rec_b);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = *reinterpret_cast<const float*>(img + REC * 4 + wave * 1024 + r * 256 + lane * 4);
+    for (int r = 0; r < 4; ++r) u[r] = *reinterpret_cast<const float*>(img + REC * 4 + cg * 1024 + r * 256 + lane * 4);
     auto read_q = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -330,12 +387,12 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
     };
     auto read_k = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) kf[c & 1][i] = vec(rec_k + (4 * c + i) * 1024);
+      for (int i = 0; i < KT; ++i) kf[c & 1][i] = vec(rec_k + (KT * c + i) * 1024);
     };
     read_q(0);
 #pragma unroll
-    for (int c = 0; c < DT / 2; ++c) {
-      if (c + 1 < DT / 2) read_q(c + 1);
+    for (int c = 0; c < HT / 2; ++c) {
+      if (c + 1 < HT / 2) read_q(c + 1);
       else read_k(0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -345,6 +402,18 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
           f32x4 &dx = d[4 * i + r], &ex = e[4 * i + r];
           dx = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[c & 1][i][r], S[2 * c + i][r], dx, 0, 0, 0);
           ex = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c & 1][i][r], S[2 * c + i][r], ex, 0, 0, 0);
+          // the record after the next, a piece behind every few products (in front of them all the CU's requests took 700 cycles)
+          constexpr int EVERY = HT * 4 / PP;
+          static_assert(EVERY > 0, "every piece has its place");
+          const int at = (c * 2 + i) * 4 + r;
+          if (at % EVERY == EVERY - 1 && at / EVERY < PP) {
+            piece(b + NST - 1, next, at / EVERY);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (at == HT * 4 - 1) {
+            values(b + NST - 1, next);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
 #pragma unroll
       for (int i = 0; i < 2; ++i) S[2 * c + i] *= gf[c & 1][i];
@@ -352,37 +421,39 @@ __global__ __launch_bounds__(256, 1) void blocks_walk_kernel(BlockArgs a) {
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) u[r] = has_col && b * kB + 4 * kg + r < n ? u[r] : 0.f;
-    const f32x4 w = u - sum8(d);
+    const f32x4 mine = sum8(d);
+    f32x4 other;
+    asm volatile("ds_write_b128 %0, %1" ::"v"(x_mine), "v"(mine) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (read below, and written again only behind the next block's barrier)
+    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(other) : "v"(x_other) : "memory");
+    w = u - (mine + other);
     u = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 4; ++r) u = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[r], w[r], u, 0, 0, 0);
 #pragma unroll
-    for (int c = 0; c < DT / 4; ++c) {
-      if (c + 1 < DT / 4) read_k(c + 1);
+    for (int c = 0; c < HT / KT; ++c) {
+      if (c + 1 < HT / KT) read_k(c + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = 0; r < 4; ++r)   // (r outside i: a tile's four products wait for each other)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c & 1][i][r], u[r], S[4 * c + i], 0, 0, 0);
+        for (int i = 0; i < KT; ++i) S[KT * c + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c & 1][i][r], u[r], S[KT * c + i], 0, 0, 0);
     }
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+    e_own = sum8(e);
+    if (half) {   // (read behind the next block's barrier, and written again behind its second)
+      asm volatile("ds_write_b128 %0, %1" ::"v"(x_e), "v"(e_own) : "memory");
+    } else {
+      x = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[r], u[r], x, 0, 0, 0);
-    o = sum8(e) + x;
-    float zero = 0.f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) zero = fmaf(o[r], 0.f, zero);
-    // (the state has what is not finite either way; the whole wave takes the branch)
-    if (__builtin_expect(__any(zero != 0.f), 0)) {
-      const f32x4 x2 = causal(vec(rec_b), causal(vec(rec_b + 1024), w, u, kg), x, kg);
-      o = sum8(e) + x2;
+      for (int r = 0; r < 4; ++r) x = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[r], u[r], x, 0, 0, 0);
     }
   }
-  store(nb - 1);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the requests beyond the end land before the workgroup's LDS is given away)
+  // (the requests beyond the end land before the workgroup's LDS is given away)
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if (half == 0) finish(nb - 1);
   if (!has_state) return;
 #pragma unroll
-  for (int m = 0; m < DT; ++m) {
+  for (int m = 0; m < HT; ++m) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) st[(4 * m + r) * (4 * kStateCols) + cc * 4 + kg] = S[m][r];
   }
@@ -753,7 +824,9 @@ extern "C" int mi_channel_delta_blocks(const float* qkv, int64_t ld, int q_off, 
   if (!aligned16(workspace) || ws_elems < ((int64_t)n_rows / kB + n_seqs) * H * record_floats(16 * dt)) return MI_EWORKSPACE;
   const BlockArgs a{qkv, ld, q_off, k_off, v_off, beta_pre, ld_beta, decay_pre, ld_decay, dt_bias, a_log, cu_q, kv_lens, slot_ids,
                     n_seqs, H, G, D, Dv, state, workspace, out, ldo};
-  const dim3 prep(n_rows / kB + n_seqs, H), walk(n_seqs, H, (Dv + 63) / 64);   // (64 columns hold whole blocks of the state's layout)
+  const int64_t walks = (int64_t)n_seqs * H * ((Dv + 31) / 32);   // (a block of the state's layout each)
+  if (walks > 0x7fffffff) return MI_EUNSUPPORTED;
+  const dim3 prep(n_rows / kB + n_seqs, H), walk((unsigned)walks);
   const auto launch = [&](auto prepare, auto walk_kernel) -> int {
     hipLaunchKernelGGL(prepare, prep, dim3(256), 0, S(stream), a);
     if (check_launch() != MI_OK) return MI_ELAUNCH;

@@ -91,6 +91,14 @@ def test_channel_delta_by_blocks(ops, lens, H, G, D, Dv):
     assert all((s_blocks[len(lens) - 1 - i] == 7.0).all() for i, n in enumerate(lens) if n == 0)
 
 
+@pytest.mark.parametrize("lens", [tuple(i * 37 % 23 for i in range(70)), (40,) * 65, (0,) * 64 + (33, 0, 34), (1,) * 3 + (90,)])
+@pytest.mark.parametrize("H,G,D,Dv", [(3, 1, 64, 40), (2, 2, 128, 96)])
+def test_sequences_in_the_order_of_their_rows(ops, lens, H, G, D, Dv):
+    """every sequence walked once: more than a wave looks at, equal ones, empty ones"""
+    test_channel_delta_by_blocks(ops, lens, H, G, D, Dv)
+
+
+
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 @pytest.mark.parametrize("where", ["q", "k", "v", "decay", "beta"])
 @pytest.mark.parametrize("at", [0, 5, 21, 32, 66])
