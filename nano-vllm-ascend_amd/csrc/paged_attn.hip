@@ -764,9 +764,11 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
   // Workgroups are dealt to the 8 XCDs round-robin by linear id.  All query blocks of one
   // (sequence, kv head) re-read the same K/V tiles, so they are given ids that are equal mod 8:
   // the pair's K/V (2 x 256 KiB per 1024 tokens) is then served by ONE XCD's L2 instead of being
-  // pulled into all eight.  id = ((pair / 8) * n_qblocks + qblock) * 8 + pair % 8.
-  const int pair = ((int)blockIdx.x / (8 * n_qblocks)) * 8 + ((int)blockIdx.x & 7);
-  const int qblock = ((int)blockIdx.x >> 3) % n_qblocks;
+  // pulled into all eight.  id = (qblock * (pairs / 8) + pair / 8) * 8 + pair % 8: the heaviest query blocks of ALL
+  // pairs first - pair after pair, the last pairs' heaviest blocks begin when the chip is running empty.
+  // us a launch, 16 sequences of 1024 rows, 16 / 8 heads: 118 -> 101.
+  const int pair8s = (n_pairs + 7) >> 3, qblock = ((int)blockIdx.x >> 3) / pair8s;
+  const int pair = (((int)blockIdx.x >> 3) % pair8s) * 8 + ((int)blockIdx.x & 7);
   if (pair >= n_pairs) return;
   const int seq = pair / n_kv_heads, h = pair % n_kv_heads;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
