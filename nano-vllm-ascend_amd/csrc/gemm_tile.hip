@@ -457,7 +457,8 @@ static int tile_ksplit(int M, int N, int K) {
 }
 
 // The large-M kernel: gemm_w16_kernel (four waves, v_mfma_f32_16x16x32_bf16), with whole-line output stores
-// (kLineStores) wherever the output allows it: full feature tiles, 16-byte aligned rows, 32-bit byte offsets.
+// (kLineStores) wherever the output allows it: full feature tiles (plain results: full halves, a wave's 128 features - a head of 151936 rows, us,
+// 200 tokens 104 -> 97, 256 112 -> 102, 400 173 -> 163), 16-byte aligned rows, 32-bit byte offsets.
 // Tuning / comparison variants: V & kDirectStores keeps the direct stores; V & kMfma32 = the same kernel on
 // v_mfma_f32_32x32x16_bf16 (gemm_w4_kernel: the first form, still the qkv-store kernel); V & kEightWaves = the
 // eight-wave ping-pong kernel before both.
@@ -469,7 +470,7 @@ static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
   const bool persistent = !(V & 16) && ntiles > kPersistentGrid;
   const dim3 grid(persistent ? kPersistentGrid : ntiles, ksplit);
   constexpr int VK = V & ~(kDirectStores | kMfma32 | kEightWaves);  // the kernel's own flags
-  const bool lines = EPI != TEPI_PARTIAL && !(V & (kDirectStores | 8 | 512)) && a.N % TILE_F == 0 && a.ldy % 8 == 0 &&
+  const bool lines = EPI != TEPI_PARTIAL && !(V & (kDirectStores | 8 | 512)) && a.N % (EPI == TEPI_SILU || (V & kMfma32) ? TILE_F : TILE_F / 2) == 0 && a.ldy % 8 == 0 &&
                      (int64_t)a.M * a.ldy * 2 < ((int64_t)1 << 32) && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
   if constexpr ((V & kEightWaves) != 0) {
     hipLaunchKernelGGL((gemm_tile_kernel<EPI, BIAS, VK>), grid, dim3(512), 0, st, a);

@@ -334,6 +334,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   const uint32_t stg_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + 2 * W16_STEP_BYTES) + wave * W4_STAGE_BYTES;
   const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (uint32_t)a.M * (uint32_t)a.ldy * 2, 0x00020000);
   auto epilogue_lines = [&](int m0, int n0) __attribute__((always_inline)) {
+    if (LINES && EPI == TEPI_NONE && n0 + fw * 128 >= a.N) return;  // (half a feature tile beyond the last: the whole wave's)
     u32x4 out[4], back[4];
     // (opaque per tile: otherwise the addresses are hoisted out of the tile loop and spilled, and a reload waits for every piece and store in
     // flight - 0.9 us per tile)

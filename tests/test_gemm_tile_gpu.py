@@ -229,3 +229,17 @@ def test_more_rows_than_one_launch_addresses_go_through_in_row_pieces(ops):
     want = ops.gemm_tile(x.to(DEV), wd)  # contiguous rows: one launch
     assert torch.equal(y.view(torch.int16), want.view(torch.int16))
     assert_bf16_close(y, oracle.linear(x, w, None), max_ulp=1, max_frac=2e-2, atol=K * 2.0 ** -22)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 128, 64), (257, 384, 128), (255, 640, 64), (300, 4992, 192), (513, 33152, 128)])
+def test_half_a_feature_tile_in_whole_lines(ops, M, N, K):
+    """N an odd multiple of 128: the last tile's second half stores nothing (the next row's first features stay), the rest the bits of the
+    128-tile kernel."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = (torch.randn(*s, device="cuda", generator=gen).bfloat16() for s in ((M, K), (N, K)))
+    want = ops.gemm_tile(x, w, variant=65536)
+    out = torch.full((M, N + 136), 7.0, dtype=torch.bfloat16, device="cuda")
+    for y in (ops.gemm_tile(x, w, variant=0), ops.gemm_tile(x, w, out=out[:, :N], variant=0)):
+        assert torch.equal(y, want)
+    assert bool((out[:, N:] == 7.0).all())
+
