@@ -72,3 +72,25 @@ def test_few_features_over_rows_that_are_no_whole_lines(dtype, M, N, K, odd):
     got, want = ops.gemm_any(x, w, exact=True), x.double() @ w.double().T
     size = x.double().abs() @ w.double().abs().T
     assert bool(((got.double() - want).abs() <= K * 2.0 ** -23 * size + 1e-12).all())
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192])
+@pytest.mark.parametrize("M,N,dtype,dual", [(130, 40, torch.float32, False), (300, 200, torch.float32, True), (700, 512, torch.bfloat16, False),
+                                            (1300, 900, torch.float32, False), (1300, 900, torch.bfloat16, True)])
+def test_fragments_read_a_step_ahead(M, N, dtype, dual, K):
+    """one to six K steps (fewer than the ring holds, odd and even) of every tile size: K roundings of the terms' sum"""
+    from nanovllm import _C, ops
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda", generator=g)
+    w, w2 = (torch.randn(N, K, device="cuda", generator=g).to(dtype) for _ in range(2))
+    got = ops.gemm_any_act(x, w, None, _C.ACT_SILU, w2=w2, exact=True) if dual else ops.gemm_any(x, w, exact=True)
+    z, size = x.double() @ w.double().T, x.abs().double() @ w.abs().double().T
+    tol = (K + 4) * 2.0 ** -24 * size
+    if dual:   # |silu'| < 1.1, |silu(z)| <= |z|; its own form adds a few roundings of the result
+        u, usize = x.double() @ w2.double().T, x.abs().double() @ w2.abs().double().T
+        want = torch.nn.functional.silu(z) * u
+        tol = 1.1 * tol * u.abs() + z.abs() * (K + 4) * 2.0 ** -24 * usize + 16 * 2.0 ** -24 * want.abs() + tol * (K + 4) * 2.0 ** -24 * usize
+    else:
+        want = z
+    assert bool(((got.double() - want).abs() <= tol).all())
+
