@@ -8,7 +8,7 @@
 // step) reached 200-350 TFLOP/s; the tile kernels fetch both operands with LDS-DMA, which needs them in bf16 - hence the
 // pass over x, which reads and writes 6 bytes per element once and is paid back from the second feature tile on.
 // Measured, 8192 rows: 2048 x 2048 207 -> 63 us + 15 us of operand pass; 64 experts x 8 per row, 2048 -> 2 x 768 with SwiGLU
-// 1192 -> 410 us (1.0 PFLOP/s), back to 2048 1050 -> 280 us.  Bits: one fp32 chain over k per result, k ascending, from
+// 1192 -> 355 us (1.16 PFLOP/s), back to 2048 1050 -> 280 us.  Bits: one fp32 chain over k per result, k ascending, from
 // the same rounded operands as gemm_any_mfma_kernel's - the same bits (silu, a form of its own, to an ulp).
 #include "gemm_any_stream.hpp"
 #include "gemm_tile_args.hpp"
