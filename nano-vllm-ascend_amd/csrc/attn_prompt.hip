@@ -106,7 +106,8 @@ __device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* 
     if (n_seqs > 64) look(i);
     if (n > 0) top = max(top, past + n - 1);
   }
-  int lo = 0, hi = (int)wave_max((float)top) + 1, behind = 0;
+  const int last = (int)wave_max((float)top);   // (rounded beyond 2^24: hi only has to lie behind every position)
+  int lo = 0, hi = last + 1 + (last >> 23), behind = 0;
   if (rank >= over_all([&] { return from(0); })) return false;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1, c = over_all([&] { return from(mid); });
@@ -483,7 +484,8 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   const int64_t tiles = rows / R + n_seqs;
   if (tiles > 0x7fffffff || (hpg + kCols - 1) / kCols > 65535) return MI_EUNSUPPORTED;
   const dim3 grid((unsigned)tiles, G, (hpg + kCols - 1) / kCols);
-  const bool longest_first = tiles * G * grid.z > 512;   // (two workgroups per CU: with no more than that all begin at once)
+  // (two workgroups per CU: with no more than that all begin at once; the order's sums are exact below 2^24)
+  const bool longest_first = tiles * G * grid.z > 512 && tiles < 1 << 24;
   // us, the kernels before / this one: 8 x 1024 rows, 16 heads over one 256-channel row (values inside it) 917 / 271; 11 prompts,
   // 8112 rows, 8 / 4 heads x 128, window 512: 189 / 96; fp32 pages, 733 rows of 16 sequences behind up to 700: 760 / 83.  With K
   // and V through registers into the image (V transposed on the way): 345, 104, 86.
