@@ -21,6 +21,8 @@
 // geometry is static and hipGraph-capturable; a second kernel merges the splits.
 #include <limits.h>
 
+#include <algorithm>
+
 #include "mi_common.hpp"
 #include "kv_store.hpp"
 #include "prefill_common.hpp"
@@ -749,7 +751,8 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, const int32_t* __restrict__ block_table, int table_stride,
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ kv_lens, uint16_t* __restrict__ out,
-    int n_q_heads, int n_kv_heads, int tpb, int tpb_shift, float scale_log2e, int n_qblocks, int n_pairs, QPrep qp) {
+    int n_q_heads, int n_kv_heads, int tpb, int tpb_shift, float scale_log2e, int n_qblocks, int n_pairs, QPrep qp,
+    const int32_t* __restrict__ n_rows, int even_rows) {
   constexpr bool EARLY = (VAR & PV_EARLY) != 0, PAIR = (VAR & PV_PAIR) != 0, SPLIT_P = (VAR & PV_SPLIT_P) != 0;
   constexpr bool READ2 = (VAR & PV_READ2) != 0, PREF = !(VAR & PV_NOPREF) && !PAIR;
   constexpr bool MAXTREE = (VAR & PV_MAXTREE) != 0, VADDR = (VAR & PV_VADDR) != 0;
@@ -764,17 +767,24 @@ __global__ __launch_bounds__(256) void paged_attn_prefill_kernel(
   // Workgroups are dealt to the 8 XCDs round-robin by linear id.  All query blocks of one
   // (sequence, kv head) re-read the same K/V tiles, so they are given ids that are equal mod 8:
   // the pair's K/V (2 x 256 KiB per 1024 tokens) is then served by ONE XCD's L2 instead of being
-  // pulled into all eight.  id = (qblock * (pairs / 8) + pair / 8) * 8 + pair % 8: the heaviest query blocks of ALL
-  // pairs first - pair after pair, the last pairs' heaviest blocks begin when the chip is running empty.
-  // us a launch, 16 sequences of 1024 rows, 16 / 8 heads: 118 -> 101.
-  const int pair8s = (n_pairs + 7) >> 3, qblock = ((int)blockIdx.x >> 3) / pair8s;
-  const int pair = (((int)blockIdx.x >> 3) % pair8s) * 8 + ((int)blockIdx.x & 7);
+  // pulled into all eight.  id = ((pair / 8) * n_qblocks + qblock) * 8 + pair % 8: pair after pair; or, where the step brings
+  // even_rows rows and more (all_pairs_first): id = (qblock * (pairs / 8) + pair / 8) * 8 + pair % 8, the heaviest query
+  // blocks of ALL pairs first - pair after pair, the last pairs' heaviest blocks begin when the chip is running empty.
+  const int pair8s = (n_pairs + 7) >> 3, id8 = (int)blockIdx.x >> 3;
+  int qblock = id8 % n_qblocks, pair = (id8 / n_qblocks) * 8 + ((int)blockIdx.x & 7);
+  // (asked for beside n_rows: most workgroups of uneven prompts lie beyond their sequence's end and only look that up)
+  const int at = min(pair, n_pairs - 1) / n_kv_heads;
+  int q_start = cu_q[at], q_end = cu_q[at + 1];
+  if (even_rows == 0 || *n_rows >= even_rows) {
+    qblock = id8 / pair8s, pair = (id8 % pair8s) * 8 + ((int)blockIdx.x & 7);
+    const int seq = min(pair, n_pairs - 1) / n_kv_heads;
+    q_start = cu_q[seq], q_end = cu_q[seq + 1];
+  }
   if (pair >= n_pairs) return;
   const int seq = pair / n_kv_heads, h = pair % n_kv_heads;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hi = lane >> 5, n = lane & 31;
-  const int q_start = cu_q[seq];
-  const int q_len = cu_q[seq + 1] - q_start;
+  const int q_len = q_end - q_start;
   const int kv_len = kv_lens[seq];
   // heaviest (latest) query blocks are dispatched first
   const int wg_qt0 = (n_qblocks - 1 - qblock) * TQ_WG;
@@ -1623,6 +1633,25 @@ static bool few_query_rows(int n_pairs, int max_q, int G) {
   return groups <= 768 || (groups <= 1024 && groups <= max_q);
 }
 
+// From how many rows of a step on paged_attn_prefill_kernel's workgroups begin with the heaviest query blocks of all pairs (0: always, INT_MAX:
+// never), each measured against pair after pair, us a launch, that / this:
+//  - not where the prompts differ in length: a short one's blocks beyond its end lie BETWEEN the long ones' blocks, in a period that
+//    deals the long ones to a few of an XCD's CUs (heads; rows as a share of prompts x longest): 8 up to 1728 rows (32 / 8; 0.21) 75 / 150,
+//    31 up to 1935 (8 / 1; 0.22) 189 / 474.  This by that, one head on a kv head: at 0.57 0.91 .. 0.99, at 0.75 0.90 .. 0.94; two: at 0.57
+//    0.98 .. 1.09, at 0.66 0.89 .. 1.07, at 0.73 0.90 .. 1.05, at 0.75 0.90 .. 0.94; more: at 0.75 1.00 .. 1.12, at 0.9 0.94 .. 1.05, at 1 as below;
+//  - not where the keys and values of an XCD's pairs are several times its L2's 4 MiB: 16 x 2048 (16 / 8; 16 MiB) 355 / 334, 16 x 4000
+//    (31) 1085 / 1109, 40 x 2000 (39) 794 / 904, 40 x 4000 (8 / 8; 78) 1436 / 2011, 40 x 500 behind 2000 (32 / 8; 49) 773 / 1006;
+//  - not where several heads on a kv head make the workgroups many rounds of an XCD's 64 places: four heads, 8 x 1000 (256 of them) 0.88,
+//    16 x 1024 (512) 0.97, 24 x 1000 (768) 1.05, 40 x 1000 (1280) 1.09; eight, 4 x 700 (176) 0.89, 27 x 1072 (268) 0.96, 8 x 1000 (504) 1.02, 24 x 1000
+//    (1512) 1.06; sixteen, 16 x 500 behind 2000 (126) 0.95, 8 x 2000 (500) 1.08.
+// keys: what the block table holds for a sequence, at most so many for any.
+static int all_pairs_first(int n_seqs, int n_pairs, int max_q, int n_qblocks, int G, int64_t keys, int head_dim) {
+  const int64_t pair8s = (n_pairs + 7) / 8, bytes = pair8s * keys * head_dim * 4;
+  if (G <= 2 ? bytes > (24 << 20) : bytes > (16 << 20) || pair8s * n_qblocks * G > 2048) return INT_MAX;
+  const int64_t rows = (int64_t)n_seqs * max_q;
+  return n_seqs == 1 ? 0 : (int)std::min<int64_t>(rows - rows / (G == 1 ? 2 : G == 2 ? 4 : 32), INT_MAX);
+}
+
 static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* prep, const mi_bf16* k_cache,
                         const mi_bf16* v_cache, const int32_t* block_table, int table_stride,
                         const int32_t* cu_seqlens_q, const int32_t* kv_lens, int n_seqs, int max_seqlen_q,
@@ -1644,6 +1673,8 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
   const int tq_wg = 4 * (32 / (G == 7 ? 8 : G));  // query tokens per workgroup
   const int n_qblocks = (max_seqlen_q + tq_wg - 1) / tq_wg, n_pairs = n_seqs * n_kv_heads;
   const dim3 grid((unsigned)((n_pairs + 7) / 8 * 8 * n_qblocks));
+  const int32_t* const n_rows = cu_seqlens_q + n_seqs;
+  const int even_rows = all_pairs_first(n_seqs, n_pairs, max_seqlen_q, n_qblocks, G, (int64_t)table_stride * block_size, head_dim);
   const float sl2 = scale * 1.4426950408889634f;
   int tpb_shift = -1;
   for (int sft = 0; sft < 12; ++sft)
@@ -1674,7 +1705,7 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
 #define LAUNCH_PRE_AS(GG, FQ, VV)                                                                                  \
   hipLaunchKernelGGL((paged_attn_prefill_kernel<GG, FQ, VV>), grid, dim3(256), 0, st, q, q_row_stride, k_cache,   \
                      v_cache, block_table, table_stride, cu_seqlens_q, kv_lens, out, n_q_heads, n_kv_heads,       \
-                     block_size / 16, tpb_shift, sl2, n_qblocks, n_pairs, qp)
+                     block_size / 16, tpb_shift, sl2, n_qblocks, n_pairs, qp, n_rows, even_rows)
   // every group size: {raw q rows, q prepared in the kernel} x {P as one bf16, P as hi + lo}
 #define LAUNCH_PRE(GG)                                                       \
   do {                                                                       \
@@ -1711,11 +1742,11 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
     if (split_p)                                                                                                  \
       hipLaunchKernelGGL((paged_attn_prefill_kernel<GG, false, PV_SPLIT_P * (DD == 4), DD>), grid, dim3(256), 0, st, q, \
                          q_row_stride, k_cache, v_cache, block_table, table_stride, cu_seqlens_q, kv_lens, out,   \
-                         n_q_heads, n_kv_heads, block_size / 16, tpb_shift, sl2, n_qblocks, n_pairs, qp);         \
+                         n_q_heads, n_kv_heads, block_size / 16, tpb_shift, sl2, n_qblocks, n_pairs, qp, n_rows, even_rows);   \
     else                                                                                                          \
       hipLaunchKernelGGL((paged_attn_prefill_kernel<GG, false, 0, DD>), grid, dim3(256), 0, st, q, q_row_stride,   \
                          k_cache, v_cache, block_table, table_stride, cu_seqlens_q, kv_lens, out, n_q_heads,      \
-                         n_kv_heads, block_size / 16, tpb_shift, sl2, n_qblocks, n_pairs, qp);                    \
+                         n_kv_heads, block_size / 16, tpb_shift, sl2, n_qblocks, n_pairs, qp, n_rows, even_rows); \
   } while (0)
   if (head_dim == 64) {  // 2 KiB tiles, prepared q rows; P as one bf16 (the hi + lo form exists for 128-wide heads)
     switch (G) {

@@ -803,6 +803,48 @@ def test_prefill_attention_of_few_rows_takes_the_bits_of_many(ops, sharpness):
     assert float(few.float().abs().max()) > 0.1 and torch.equal(few.view(torch.int16), many.view(torch.int16))
 
 
+def _prefill_step(ops, gen, hq, hkv, bs, q_lens, prefix, sharpness=1.0):
+    """-> call(max_q, only=None): the fused attention of a step with `max_q` as its bound on the sequences' rows (one sequence's rows alone
+    with `only`), and plain(max_q): the same step from prepared queries."""
+    kv_lens = [a + b for a, b in zip(q_lens, prefix)]
+    T, nb = sum(q_lens), [-(-n // bs) for n in kv_lens]
+    perm = torch.randperm(sum(nb), generator=gen).to(torch.int32)
+    bt = torch.full((len(nb), max(nb)), -1, dtype=torch.int32)
+    o = 0
+    for i, k in enumerate(nb):
+        bt[i, :k] = perm[o:o + k]
+        o += k
+    pos = torch.cat([torch.arange(p, p + k) for p, k in zip(prefix, q_lens)]).to(torch.int64).to(DEV)
+    qkv = torch.randn(T, (hq + 2 * hkv) * 128, generator=gen).bfloat16().to(DEV)
+    qw = torch.full((128,), sharpness, dtype=torch.bfloat16, device=DEV)
+    table = oracle.build_cos_sin_cache(128, 4096, 1e6).to(DEV)
+    kc, vc = (torch.randn(ops.kv_cache_shape(sum(nb), hkv, bs), generator=gen).bfloat16().to(DEV) for _ in range(2))
+    cu, kvl, bt = torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32).to(DEV), torch.tensor(kv_lens, dtype=torch.int32).to(DEV), bt.to(DEV)
+
+    def call(max_q, only=None):
+        if only is None:
+            return ops.paged_attn_prefill_fused(qkv, qw, 1e-6, pos, table, kc, vc, bt, cu, kvl, max_q, hq, hkv, bs, 128 ** -0.5)
+        r, one = slice(int(cu[only]), int(cu[only + 1])), torch.tensor([0, q_lens[only]], dtype=torch.int32).to(DEV)
+        return ops.paged_attn_prefill_fused(qkv[r], qw, 1e-6, pos[r], table, kc, vc, bt[only:only + 1], one, kvl[only:only + 1], max_q, hq, hkv,
+                                            bs, 128 ** -0.5)
+
+    def plain(max_q):
+        return ops.paged_attn_prefill(qkv[:, :hq * 128].contiguous(), kc, vc, bt, cu, kvl, max_q, hq, hkv, bs, 128 ** -0.5)
+    return call, plain
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (10, 5), (32, 8), (16, 2), (16, 1)])
+@pytest.mark.parametrize("q_lens", [(200, 200, 200), (200, 195, 200), (200, 3, 71), (1, 160, 0, 260)])
+def test_prefill_attention_orders_of_the_workgroups(ops, hq, hkv, q_lens):
+    """Prompts of one length, of nearly one and of very different ones (and a bound on the rows above them all: many blocks beyond every
+    sequence's end), pairs of sequence and kv head that are no multiple of eight: every sequence has the bits that it has alone."""
+    gen = torch.Generator().manual_seed(hq * 3 + hkv + sum(q_lens))
+    call, _ = _prefill_step(ops, gen, hq, hkv, 16, list(q_lens), [(37 * i) % 50 for i in range(len(q_lens))])
+    alone = torch.cat([call(n, i) for i, n in enumerate(q_lens) if n])
+    for max_q in (max(q_lens), 8192):
+        assert torch.equal(call(max_q).view(torch.int16), alone.view(torch.int16)), max_q
+
+
 def test_prefill_attention_chunk_pipeline_stress(ops):
     """Kernel-level guard of the prefill attention's LDS-DMA ring (the counted `s_waitcnt vmcnt(4)` of its chunk
     loop): the bench's prefill step - 16 sequences x 1024 tokens, Qwen3-0.6B heads, block 16 - with SCRAMBLED block
