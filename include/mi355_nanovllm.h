@@ -224,6 +224,10 @@ int mi_paged_attn_prefill(const mi_bf16* q, int64_t q_row_stride,
                           int n_q_heads, int n_kv_heads, int head_dim,
                           int block_size, float scale, mi_stream stream);
 
+/* 1 if a step of n_seqs sequences takes the kernel for few query rows (the same bits; group = n_q_heads / n_kv_heads, head_dim 128;
+ * keys: table_stride * block_size).  No launch. */
+int mi_paged_attn_prefill_takes_few(int n_seqs, int n_kv_heads, int group, int max_seqlen_q, int64_t keys);
+
 /* The same with the query side of qwen3.py:79-88 folded into the Q-operand load: q points at the RAW packed qkv
  * rows (linear.py:117-126); per-head RMSNorm with q_w (NULL: no norm) and NeoX RoPE at positions[token] are
  * applied in registers, bit-identical to what mi_qknorm_rope_store writes to q_out.  K and V must already be in

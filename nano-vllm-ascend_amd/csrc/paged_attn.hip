@@ -1622,15 +1622,21 @@ extern "C" int mi_paged_attn_decode_ex(const mi_bf16* q, int64_t q_row_stride, c
                      KvStrides{stride_block, stride_head, stride_tile}, stream);
 }
 
-// Which steps take paged_attn_prefill_few_kernel (same bits), by its workgroups (sequences x kv heads x blocks of 32 columns): three per CU,
-// or four where a query block's chunks are as many as there are workgroups.  us per step of 28 layers, 8 kv heads, the kernel for many rows / this
-// one: 1 x 64 rows 1277 / 1189, 1 x 137 1533 / 1451, behind 320 cached 1754 / 1576, 1 x 400 2041 / 1933, 1 x 1024 (512 workgroups) 3033 / 2806,
-// 1 x 2047 (1024) 4949 / 4666, 2 x 512 (512) 2742 / 2605, 2 x 700 (704) 3585 / 3393, 2 x 1024 (1024) 4164 / 4111, 3 x 200 behind 600 2644 / 2443,
-// 4 x 256 (512) 2419 / 2291, 16 x 48 (384) 2287 / 2212, 8 x 128 behind 600 (512) 2911 / 2784; beyond the lines 4 x 512 (1024) 3871 / 3921,
-// 1 x 3000 (1504) 6752 / 7031.
-static bool few_query_rows(int n_pairs, int max_q, int G) {
-  const int64_t groups = (int64_t)n_pairs * ((max_q + 32 / G - 1) / (32 / G));
-  return groups <= 768 || (groups <= 1024 && groups <= max_q);
+// Which steps take paged_attn_prefill_few_kernel (same bits): by the workgroups (blocks of 32 columns of a pair) that an XCD has - a pair's are
+// all on one, so fewer pairs than XCDs leave the others idle - of which its 32 CUs hold 64.  us a launch, the kernel for many rows / this one, per
+// heads, prompts and [workgroups of an XCD]:
+//   up to 64: 0.55 .. 0.87 of that one, 0.99 at worst behind 2000 cached rows (40 x 32 rows, 8 / 8 heads [40] 72 / 71)
+//   more are a second round: 40 x 14 rows (32 / 2) [70] 9.1 / 11, 16 x 96 (16 / 8) [96] 10 / 11, 1 x 144 behind 2000 (16 / 1) [72] 53 / 73,
+//   1 x 2561 (8 / 1) [641] 114 / 299, 1 x 923 (16 / 1) [462] 42 / 92
+//   but longer prompts without much in front of them, whose walks differ, fill the gaps with their short ones: 4 x 288 (16 / 8) [72] 14 / 11, 4 x 576
+//   (8 / 8) [72] 20 / 16, behind 300 28 / 24, 4 x 144 (32 / 8) [72] 11.3 / 10.2; and few pairs' long after: 1 x 576 (32 / 8) [72] 20 / 16, 2 x 384 [96] 17 / 15, behind
+//   300 2 x 768 (16 / 8) [96] 32 / 31 (2 x 384, 32 / 8: 24 / 26), 1 x 1536 [96] 48 / 41; 1 x 2048 (16 / 8) [128] 53 / 49, behind 300 61 / 61, 2 x 1024 [128] 31 / 30,
+//   1 x 256 (16 / 1) [128] 13.0 / 13.6, four prompts of 1024 (8 / 8) [128] 32 / 38.
+// keys: what the block table holds for a sequence, at most so many for any.
+static bool few_query_rows(int n_pairs, int max_q, int G, int64_t keys) {
+  const int64_t blocks = ((int64_t)max_q * G + 31) / 32, groups = (n_pairs + 7) / 8 * blocks;
+  if (groups <= 64 || (groups <= 80 && max_q >= 128 && 5 * keys <= 8 * (int64_t)max_q)) return true;
+  return n_pairs <= 16 && (groups <= 96 ? 2 * keys <= 3 * (int64_t)max_q : groups <= 128 && max_q >= 1024 && 8 * keys <= 9 * (int64_t)max_q);
 }
 
 // From how many rows of a step on paged_attn_prefill_kernel's workgroups begin with the heaviest query blocks of all pairs (0: always, INT_MAX:
@@ -1681,7 +1687,7 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
     if ((1 << sft) == block_size / 16) tpb_shift = sft;
   hipStream_t st = S(stream);
   const QPrep qp = prep ? *prep : QPrep{nullptr, nullptr, nullptr, 0.f};
-  if (head_dim == MI_HEAD_DIM && (variant & ~PV_SPLIT_P) == 0 && few_query_rows(n_pairs, max_seqlen_q, G)) {
+  if (head_dim == MI_HEAD_DIM && (variant & ~PV_SPLIT_P) == 0 && few_query_rows(n_pairs, max_seqlen_q, G, (int64_t)table_stride * block_size)) {
     const int blocks = (max_seqlen_q + 32 / G - 1) / (32 / G);
     const dim3 few((unsigned)((n_pairs + 7) / 8 * 8 * blocks));
     auto go = [&](auto group) {
@@ -1771,6 +1777,11 @@ static int prefill_impl(const mi_bf16* q, int64_t q_row_stride, const QPrep* pre
 #undef LAUNCH_PRE
 #undef LAUNCH_PRE_AS
   return check_launch();
+}
+
+extern "C" int mi_paged_attn_prefill_takes_few(int n_seqs, int n_kv_heads, int group, int max_seqlen_q, int64_t keys) {
+  return n_seqs > 0 && n_kv_heads > 0 && max_seqlen_q > 0 && (group == 1 || group == 2 || group == 4 || group == 8 || group == 16) &&
+         few_query_rows(n_seqs * n_kv_heads, max_seqlen_q, group, keys);
 }
 
 extern "C" int mi_paged_attn_prefill(const mi_bf16* q, int64_t q_row_stride, const mi_bf16* k_cache,

@@ -100,6 +100,7 @@ _SIGNATURES = {
         [_p, c_int64, _p, c_float, _p, _p, _p, _p, _p, c_int, _p, _p, c_int, c_int, _p, c_int, c_int, c_int, c_int,
          c_float, _p],
     ),
+    "mi_paged_attn_prefill_takes_few": (c_int, [c_int, c_int, c_int, c_int, c_int64]),
     "mi_paged_attn_prefill_fused_ex": (
         c_int,
         [_p, c_int64, _p, c_float, _p, _p, _p, _p, _p, c_int, _p, _p, c_int, c_int, _p, c_int, c_int, c_int, c_int,

@@ -24,3 +24,16 @@ def test_norm(nsplit, n, k, silu, fp8, pays):
                                                                (4, 16, 8, 1024, 4, True), (3, 12, 4, 768, 2, True), (4, 8, 8, 1024, 4, True), (5, 8, 8, 1024, 4, False)])
 def test_merge(rows, heads, kv_heads, n, ksplit, pays):
     assert ops.merge_few_pays(rows, kv_heads, _w(n, heads * 128), ksplit) == pays
+
+
+def test_prefill_attention_of_few_rows_rule():
+    """The rule counts an XCD's workgroups (fewer pairs than XCDs leave the others idle) and, beyond its places, asks whether the walks
+    differ.  Steps measured on both sides of the line."""
+    from nanovllm import _C
+
+    takes = lambda seqs, hq, hkv, q, keys: bool(_C.lib.mi_paged_attn_prefill_takes_few(seqs, hkv, hq // hkv, q, keys))  # noqa: E731
+    assert takes(1, 16, 8, 137, 144) and takes(16, 32, 8, 16, 2048) and takes(1, 8, 1, 256, 2304) and takes(40, 8, 8, 32, 2048)
+    assert takes(1, 16, 8, 2048, 2048) and takes(2, 16, 8, 768, 1072) and takes(1, 32, 8, 576, 576) and takes(4, 16, 8, 288, 288) and takes(4, 8, 8, 576, 880)
+    assert not takes(1, 8, 1, 2561, 2768) and not takes(1, 16, 1, 923, 928) and not takes(1, 32, 2, 914, 928) and not takes(1, 8, 1, 340, 2560)
+    assert not takes(40, 32, 2, 14, 16) and not takes(2, 32, 8, 384, 688) and not takes(4, 8, 8, 1024, 1024) and not takes(1, 16, 8, 2049, 2064)
+    assert not takes(1, 16, 8, 2048, 8192)   # (a table wider than the prompt: a prefix may lie in front of it)

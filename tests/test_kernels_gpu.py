@@ -845,6 +845,19 @@ def test_prefill_attention_orders_of_the_workgroups(ops, hq, hkv, q_lens):
         assert torch.equal(call(max_q).view(torch.int16), alone.view(torch.int16)), max_q
 
 
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (10, 5), (12, 3), (16, 2), (16, 1)])
+@pytest.mark.parametrize("block_size", [16, 48])
+@pytest.mark.parametrize("sharpness", [1.0, 9.0])
+def test_prefill_attention_of_few_rows_and_of_many(ops, hq, hkv, block_size, sharpness, prefill_p):
+    """Both kernels at every group size, from prepared and from raw queries, P as one bf16 and as hi + lo, pages that are no power of two:
+    the same bits.  (The bound on the sequences' rows chooses: the exact one takes the kernel for few rows, 8192 the one for many.)"""
+    gen = torch.Generator().manual_seed(hq + hkv + block_size)
+    call, plain = _prefill_step(ops, gen, hq, hkv, block_size, [70, 1, 64, 33, 0, 90], [0, 300, 0, 129, 5, 31], sharpness)
+    for f in (call, plain):
+        few, many = f(90), f(8192)
+        assert float(few.float().abs().max()) > 0.1 and torch.equal(few.view(torch.int16), many.view(torch.int16))
+
+
 def test_prefill_attention_chunk_pipeline_stress(ops):
     """Kernel-level guard of the prefill attention's LDS-DMA ring (the counted `s_waitcnt vmcnt(4)` of its chunk
     loop): the bench's prefill step - 16 sequences x 1024 tokens, Qwen3-0.6B heads, block 16 - with SCRAMBLED block
