@@ -135,8 +135,9 @@ __device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* 
 // up to 32 DKM key and 16 DVM value channels; smaller heads are zero-padded to that in the images: a branch per fragment would put
 // every fragment's LDS latency behind the one before.  VIK: the values are the leading channels of the key rows.  PAGED16: pages
 // of a multiple of 16 rows.  V4: value rows that start on 4 bytes only (bf16, an even stride), requested in 4-byte pieces.
-template <typename TC, int DKM, int DVM, int NST, bool VIK, bool PAGED16, bool V4 = false>
-__global__ __launch_bounds__(kPromptThreads, 2) void prompt_attention_kernel(
+// TWO: registers for two workgroups per CU (128; four of them spilled).
+template <typename TC, int DKM, int DVM, int NST, bool VIK, bool PAGED16, bool V4 = false, bool TWO = false>
+__global__ __launch_bounds__(kPromptThreads, TWO ? 4 : 2) void prompt_attention_kernel(
     const float* __restrict__ q, int64_t ldq, const TC* __restrict__ k_cache, const TC* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, int table_cols, const int32_t* __restrict__ cu_q,
     const int32_t* __restrict__ kv_lens, int n_seqs, int H, int G, int D, int Dv, int block_size, int window, float scale,
@@ -499,6 +500,14 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   // ... and of at most 32 channels, padded to 64, where there are too few tiles for the chip (8 / 4 heads x 32: 1 x 400 rows 36 / 40, 1 x 1600 140 /
   // 151; 4 x 1000 rows 171 / 115; x 16: 4 x 400 31 / 40, 4 x 1600 217 / 242)
   if (!bf16 && D <= 32 && Dv <= 32 && keys > 32 && tiles * G * grid.z <= (D <= 16 && Dv <= 16 ? 420 : 108)) return MI_EUNSUPPORTED;
+  // fp32 heads of up to 64 channels: two workgroups per CU where the matrix pipe would wait for the one, but not where a few hundred uneven
+  // walks would meet on some CUs and leave others idle, and not where one per CU is all there is (us, one / two, the rule's numbers in
+  // brackets: 60 x 3 rows behind 500, 16 / 8 heads [496, alike] 86 / 57, 100 x 1 behind 600 and 300 rows, 8 / 4 [428, alike] 103 / 79, 1 x 4539
+  // (16 / 8) [568] 762 / 670, 16 x 1600 (16 / 8) [3328] 995 / 920; 12 x 481 (6 / 1) [286] 60 / 84, 1 x 7500 (6 / 1) [358] 690 / 819,
+  // (8 / 4) [472] 900 / 1000, 14 up to 1370 (6 / 1) [537] 138 / 167; 30 x 30 behind 100 (32 / 4) [344, at least 224] 27 / 36; up to 256: 3 to 6 % more)
+  const int64_t wgs = tiles * G * grid.z, least = std::max<int64_t>(rows / R, n_seqs) * G * grid.z;
+  const bool alike = rows <= (int64_t)n_seqs * R || keys >= 2 * (int64_t)window;   // (a tile per sequence, or walks of the window's length)
+  const bool two = !bf16 && (wgs > 540 || (least > 256 && alike));
 #define MI_PROMPT(TC, DKM, DVM, NST, ...)                                                                                  \
   hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
                      static_cast<const TC*>(k_cache), static_cast<const TC*>(v_cache), bt, cols, cu_q, kv_lens, n_seqs, H, G, D, Dv, \
@@ -507,7 +516,8 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   // before / 256 channels for every head / by head size: fp32 x 64 72 / 177 / 43, x 128 144 / 183 / 79; bf16 x 64 46 / 46 / 21.)
 #define MI_PROMPT_SIZES(TC, PAGED16, WIDE)                                   \
   do {                                                                       \
-    if (D <= 64 && Dv <= 64) MI_PROMPT(TC, 2, 4, 4, false, PAGED16);         \
+    if (two && D <= 64 && Dv <= 64) MI_PROMPT(TC, 2, 4, 4, false, PAGED16, false, sizeof(TC) == 4); \
+    else if (D <= 64 && Dv <= 64) MI_PROMPT(TC, 2, 4, 4, false, PAGED16);    \
     else if (D <= 64 && Dv <= 128) MI_PROMPT(TC, 2, 8, 4, false, PAGED16);   \
     else if (D <= 128 && Dv <= 128) MI_PROMPT(TC, 4, 8, 4, false, PAGED16);  \
     else if (vik) MI_PROMPT(TC, 8, 16, 4, true, PAGED16);                    \

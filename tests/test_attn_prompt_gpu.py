@@ -118,6 +118,15 @@ def test_more_tiles_than_the_chip_holds(dtype, H, G, seqs):
     _case(dtype, H, G, 32, 32, 16, seqs)
 
 
+@pytest.mark.parametrize("block", [16, 24])
+@pytest.mark.parametrize("D,Dv", [(64, 64), (48, 32)])
+@pytest.mark.parametrize("seqs,window", [([(90, 3)] * 40, 2 ** 31 - 1), ([(0, 700), (30, 600)], 64), ([(0, 700), (30, 600)], 2 ** 31 - 1),
+                                         ([(i, 40 + 7 * i) for i in range(30)], 2 ** 31 - 1)])
+def test_small_fp32_heads_with_one_workgroup_per_cu_and_with_two(block, D, Dv, seqs, window):
+    """both sides of the line: a few hundred like walks, a few hundred unlike ones, and many"""
+    _case(torch.float32, 14, 7, D, Dv, block, seqs, window=window)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("step", [2.0, 7.9, 8.1, 40.0])
 def test_scores_that_grow_along_the_keys(dtype, step):
