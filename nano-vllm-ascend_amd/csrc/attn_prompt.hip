@@ -78,24 +78,36 @@ __device__ __forceinline__ void attend_column(const float* q, const TC* k_cache,
 // The rank-th tile (of R rows) in the order of the positions their last rows have, the largest first - the longest walks first, whatever
 // sequences they belong to: workgroups are dispatched in this order, and where there are more than the chip holds the short ones fill
 // the gaps (with sequence after sequence the last sequence's longest walks began when half of the chip was idle).  By one wave for itself, a
-// lane a sequence: bisection for the position that rank tiles lie behind.  us, sequence after sequence / this order: 8 x 1024 rows, 16
-// heads over one 256-channel row (1024 workgroups on 512 places) 271 / 210; 11 prompts, 8112 rows, 8 / 4 heads x 128, window 512: 95 / 89.
-__device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* kv_lens, int n_seqs, int R, int rank, int& s, int& first) {
+// lane a sequence: bisection for the position that rank tiles lie behind.  table: {rows, rows in front of them} of more than 64 sequences in
+// LDS (from memory in every round of the bisection, 3 loads per 64 sequences: us, sequence after sequence / so / now: 100 sequences of 1 row behind 600
+// and one of 300, 16 heads of 64 on fp32 pages 215 / 262 / 219, 300 and one of 600 752 / 897 / 770).  us, sequence after sequence / this order:
+// 8 x 1024 rows, 16 heads over one 256-channel row (1024 workgroups, one per CU) 271 / 210; 11 prompts, 8112 rows, 8 / 4 heads x 128, window
+// 512: 95 / 89.
+constexpr int kOrderedSeqs = 4096;   // (the smallest ring's 32 KiB)
+__device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* kv_lens, const int2* table, int n_seqs, int R, int rank, int& s,
+                                            int& first) {
   const int lane = threadIdx.x & 63;
-  int q0 = 0, n = 0, past = 0;
+  int n = 0, past = 0;
   auto look = [&](int i) __attribute__((always_inline)) {
-    q0 = i < n_seqs ? cu_q[i] : 0, n = i < n_seqs ? cu_q[i + 1] - q0 : 0;
-    past = i < n_seqs ? kv_lens[i] - n : 0;
+    n = past = 0;
+    if (i >= n_seqs) return;
+    if (table) {
+      n = table[i].x, past = table[i].y;
+    } else {
+      n = cu_q[i + 1] - cu_q[i], past = kv_lens[i] - n;
+    }
   };
+  const int r_shift = block_shift(R);   // (a division is half of a round of the bisection)
+  auto by_rows = [&](int rows) __attribute__((always_inline)) { return r_shift >= 0 ? rows >> r_shift : rows / R; };
   // tiles whose last row's position is at least p, among the lane's sequence
   auto from = [&](int p) __attribute__((always_inline)) {
-    const int nt = (n + R - 1) / R;
-    return nt - (past + n - 1 < p ? nt : min(max(p - past, 0) / R, max(nt - 1, 0)));
+    const int nt = by_rows(n + R - 1);
+    return nt - (past + n - 1 < p ? nt : min(by_rows(max(p - past, 0)), max(nt - 1, 0)));
   };
   auto over_all = [&](auto&& f) __attribute__((always_inline)) {  // (sums below 2^24: exact)
     int c = 0;
     for (int i = lane; i < n_seqs + lane; i += 64) {
-      if (n_seqs > 64) look(i);
+      if (table) look(i);
       c += f();
     }
     return (int)wave_sum((float)c);
@@ -103,7 +115,7 @@ __device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* 
   look(lane);
   int top = -1;
   for (int i = lane; i < n_seqs + lane; i += 64) {
-    if (n_seqs > 64) look(i);
+    if (table) look(i);
     if (n > 0) top = max(top, past + n - 1);
   }
   const int last = (int)wave_max((float)top);   // (rounded beyond 2^24: hi only has to lie behind every position)
@@ -124,7 +136,7 @@ __device__ __forceinline__ bool tile_by_end(const int32_t* cu_q, const int32_t* 
       for (; k > 0; --k) has &= has - 1;
       const int at = __builtin_ctzll(has);
       s = i0 + at;
-      first = __builtin_amdgcn_readlane(q0, at) + (lo - __builtin_amdgcn_readlane(past, at)) / R * R;
+      first = cu_q[s] + (lo - __builtin_amdgcn_readlane(past, at)) / R * R;
       return true;
     }
     k -= c;
@@ -152,6 +164,7 @@ __global__ __launch_bounds__(kPromptThreads, TWO ? 4 : 2) void prompt_attention_
                                                      : (KP + VP <= 32 ? 4 : 8);
   static_assert(!V4 || (BF && !VIK), "see above");
   static_assert(KP / 2 % PP == 0 && VP / 2 % PP == 0 && KP + VP <= PP * kWaves && (NST & (NST - 1)) == 0, "see above");
+  static_assert(NST * STAGE >= kOrderedSeqs * 8, "the order's table");
   __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE];
   // the chunk that lies at position p of row r is p ^ swizzle(r): sixteen rows at one chunk (a K fragment) and four or eight
   // rows at neighbouring chunks (a V fragment) fall into different banks
@@ -166,7 +179,17 @@ __global__ __launch_bounds__(kPromptThreads, TWO ? 4 : 2) void prompt_attention_
   const int R = kCols / nh;                                       // rows of a tile
   int s = 0, first, nr;
   if (longest_first) {
-    if (!tile_by_end(cu_q, kv_lens, n_seqs, R, (int)blockIdx.x, s, first)) return;  // (the grid is the host's bound)
+    int2* const table = n_seqs > 64 ? reinterpret_cast<int2*>(lds) : nullptr;
+    if (table) {
+      for (int i = tid; i < n_seqs; i += kPromptThreads) {
+        const int n = cu_q[i + 1] - cu_q[i];
+        table[i] = int2{n, kv_lens[i] - n};
+      }
+      __syncthreads();
+    }
+    const bool found = tile_by_end(cu_q, kv_lens, table, n_seqs, R, (int)blockIdx.x, s, first);
+    if (table) __syncthreads();   // (the ring's images lie there next)
+    if (!found) return;  // (the grid is the host's bound)
     nr = min(R, cu_q[s + 1] - first);
   } else {
     // ---- the tile: sequences in order, a sequence's last rows (the longest walks) first ----
@@ -485,8 +508,10 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   const int64_t tiles = rows / R + n_seqs;
   if (tiles > 0x7fffffff || (hpg + kCols - 1) / kCols > 65535) return MI_EUNSUPPORTED;
   const dim3 grid((unsigned)tiles, G, (hpg + kCols - 1) / kCols);
-  // (two workgroups per CU: with no more than that all begin at once; the order's sums are exact below 2^24)
-  const bool longest_first = tiles * G * grid.z > 512 && tiles < 1 << 24;
+  // Where there are more workgroups than the chip holds.  (Looking for the order takes 1 to 2 us of a workgroup, which like walks do not give back; unlike
+  // ones do, also of sequences of a tile or less: us, sequence after sequence / longest first, 8 / 4 heads of 128, 361 sequences of 1 .. 63 rows behind 16
+  // .. 1498 317 / 264, 16 / 8 heads of 64 on fp32 pages, 241 of 1 .. 339 574 / 466; 24 x 72 rows, 16 heads on as many 27.6 / 28.3.)
+  const bool longest_first = tiles * G * grid.z > 512 && tiles < 1 << 24 && n_seqs <= kOrderedSeqs;   // (its sums are exact below 2^24)
   // us, the kernels before / this one: 8 x 1024 rows, 16 heads over one 256-channel row (values inside it) 917 / 271; 11 prompts,
   // 8112 rows, 8 / 4 heads x 128, window 512: 189 / 96; fp32 pages, 733 rows of 16 sequences behind up to 700: 760 / 83.  With K
   // and V through registers into the image (V transposed on the way): 345, 104, 86.
@@ -502,11 +527,13 @@ int launch_prompt_attention(const float* q, int64_t ldq, const void* k_cache, co
   if (!bf16 && D <= 32 && Dv <= 32 && keys > 32 && tiles * G * grid.z <= (D <= 16 && Dv <= 16 ? 420 : 108)) return MI_EUNSUPPORTED;
   // fp32 heads of up to 64 channels: two workgroups per CU where the matrix pipe would wait for the one, but not where a few hundred uneven
   // walks would meet on some CUs and leave others idle, and not where one per CU is all there is (us, one / two, the rule's numbers in
-  // brackets: 60 x 3 rows behind 500, 16 / 8 heads [496, alike] 86 / 57, 100 x 1 behind 600 and 300 rows, 8 / 4 [428, alike] 103 / 79, 1 x 4539
+  // brackets: 60 x 3 rows behind 500, 16 / 8 heads [496, alike] 86 / 57, 100 x 1 behind 600 and 300 rows, 8 / 4 [428, alike] 103 / 79, 13 x 225
+  // (16 / 8) [464, alike] 56 / 42, 1 x 4539
   // (16 / 8) [568] 762 / 670, 16 x 1600 (16 / 8) [3328] 995 / 920; 12 x 481 (6 / 1) [286] 60 / 84, 1 x 7500 (6 / 1) [358] 690 / 819,
   // (8 / 4) [472] 900 / 1000, 14 up to 1370 (6 / 1) [537] 138 / 167; 30 x 30 behind 100 (32 / 4) [344, at least 224] 27 / 36; up to 256: 3 to 6 % more)
   const int64_t wgs = tiles * G * grid.z, least = std::max<int64_t>(rows / R, n_seqs) * G * grid.z;
-  const bool alike = rows <= (int64_t)n_seqs * R || keys >= 2 * (int64_t)window;   // (a tile per sequence, or walks of the window's length)
+  // (a tile per sequence, short prompts, or walks of the window's length)
+  const bool alike = rows <= (int64_t)n_seqs * std::max(R, 256) || keys >= 2 * (int64_t)window;
   const bool two = !bf16 && (wgs > 540 || (least > 256 && alike));
 #define MI_PROMPT(TC, DKM, DVM, NST, ...)                                                                                  \
   hipLaunchKernelGGL((prompt_attention_kernel<TC, DKM, DVM, NST, __VA_ARGS__>), grid, dim3(kPromptThreads), 0, st, q, ldq,    \
