@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kPromptThreads, TWO ? 4 : 2) void prompt_attention_
     for (int e = 0; e < 4; ++e)
       vslot[e] = (VIK ? 0 : KB) + (4 * kg + e) * VROW + (((r16 >> 2) ^ swizzle(4 * kg + e, VROW)) << 4) + (r16 & 3) * 4;
   }
-  float m = -INFINITY, l = 0.f;
+  float m = live ? -INFINITY : 0.f, l = 0.f;   // (a column without a row: all its weights are 0, and none of them asks for another point)
   f32x4 oacc[DVM];
 #pragma unroll
   for (int f = 0; f < DVM; ++f) oacc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(kPromptThreads, TWO ? 4 : 2) void prompt_attention_
       }
     }
     // No maximum in the common case: a lane's eight weights against the current reference point add up to at most 2^8 while none of them is
-    // larger (at the first step the point is -inf, the sum is not finite and the comparison fails).  Weights of up to 2^8 are held as
+    // larger (until a column has seen a key its point is -inf, the sum is not finite and the comparison fails).  Weights of up to 2^8 are held as
     // hi + lo, and in fp32, as those below 1 are.  (The maximum, its exchange and the rescaling were a third of a step's vector instructions.)
     float pv[8];
     auto weigh = [&](float ref) __attribute__((always_inline)) {
