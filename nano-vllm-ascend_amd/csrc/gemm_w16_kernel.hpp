@@ -206,6 +206,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
 
   // ---- epilogues.  acc[f][t][e] of lane (n16, q4): feature 16 f + 4 q4 + e, token 16 t + n16 of the wave tile ----
   const int n_out = EPI == TEPI_SILU ? a.N >> 1 : a.N;
+  // A bias is asked for in front of the tile's K steps: a load behind them waits for the pieces and the stores before it, once per use.
+  u32x2 bias[BIAS ? 8 : 1];   // the lane's four features of fragment f
+  auto bias_begin = [&](int n0) __attribute__((always_inline)) {
+    if constexpr (BIAS) {
+#pragma unroll
+      for (int f = 0; f < 8; ++f)
+        bias[f] = *reinterpret_cast<const u32x2*>(a.bias + min(n0 + fw * 128 + 16 * f + 4 * q4, a.N - 4));   // (beyond the features: not stored)
+    }
+  };
   // the output value of (fragment f, token fragment t, e): SwiGLU pairs the gate fragment f with the up fragment f + 4
   // (the reference's three roundings, silu on v_exp_f32 / v_rcp_f32 as gemm_tile_kernel's epilogue)
   auto out_value = [&](int f, int t, int e, int n0) __attribute__((always_inline)) -> float {
@@ -215,7 +224,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
       return sb * rbf(acc[f + 4][t][e]);
     }
     float o = acc[f][t][e];
-    if (BIAS) o += bf2f(a.bias[n0 + fw * 128 + 16 * f + 4 * q4 + e]);
+    if constexpr (BIAS) o += e & 1 ? hi_bf(bias[f][e >> 1]) : lo_bf(bias[f][e >> 1]);
     return o;
   };
   constexpr int NF = EPI == TEPI_SILU ? 4 : 8;  // output feature fragments of a wave
@@ -336,10 +345,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   auto epilogue_lines = [&](int m0, int n0) __attribute__((always_inline)) {
     if (LINES && EPI == TEPI_NONE && n0 + fw * 128 >= a.N) return;  // (half a feature tile beyond the last: the whole wave's)
     u32x4 out[4], back[4];
-    // (opaque per tile: otherwise the addresses are hoisted out of the tile loop and spilled, and a reload waits for every piece and store in
-    // flight - 0.9 us per tile)
-    int l = lane;
+    // (from the lane's number, made here per tile: otherwise the addresses - or, with a bias in registers, the number - are kept over the K loop
+    // and spilled, and a reload waits for every piece and store in flight - 0.9 us per tile)
+    int l = 0;
     asm volatile("" : "+v"(l));
+    l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, l));
     // after the exchange lane (n16, q4) holds chunk 2 * (2 pr + (q4 & 1)) + (q4 >> 1) of row 16 ts + n16 (pr: fragment pair)
     const uint32_t w_addr = stg_base + (uint32_t)(l & 15) * 128 + (uint32_t)(((F32 ? l >> 4 : 2 * ((l >> 4) & 1) + (l >> 5)) ^ (l & 7)) << 4);
     const uint32_t stg_r = stg_base + (uint32_t)(l >> 3) * 128 + (uint32_t)(((l & 7) ^ (l >> 3)) << 4);
@@ -440,6 +450,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
       m0 = t.m0, n0 = t.n0, m_end = t.m_end;
       any_begin(m0, n0, m_end);
     }
+    bias_begin(n0);
     kstep(std::true_type{});
     for (int kt = 1; kt < KT; ++kt) kstep(std::false_type{});
     __builtin_amdgcn_sched_barrier(0);

@@ -243,3 +243,18 @@ def test_half_a_feature_tile_in_whole_lines(ops, M, N, K):
         assert torch.equal(y, want)
     assert bool((out[:, N:] == 7.0).all())
 
+
+@pytest.mark.parametrize("M,N,K", [(8300, 2176, 64), (4100, 2196, 384), (8200, 2304, 128), (16600, 1156, 192)])
+def test_biased_products_of_the_persistent_kernel(ops, M, N, K):
+    """Part-filled row and feature tiles (half a feature tile, whole ones, neither), several tiles per workgroup, one K step: row for row the
+    bits of the 128-tile kernel (1024 rows at a time), and nothing written beside them."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w, b = (torch.randn(*s, device="cuda", generator=gen).bfloat16() for s in ((M, K), (N, K), (N,)))
+    assert all(ops.lib.mi_gemm_bf16_workspace(m, N, K, 0) == 0 for m in (M, 1024, M % 1024))   # (no K slices)
+    want = torch.cat([ops.gemm_tile(x[r:r + 1024], w, b) for r in range(0, M, 1024)])
+    size = (N + 15) // 8 * 8
+    out = torch.full((M + 1, size), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.gemm_tile(x, w, b, out=out[:M, :N])
+    assert torch.equal(out[:M, :N], want) and bool((out[:, N:] == 7.0).all()) and bool((out[M] == 7.0).all())
+    exact = x.double() @ w.double().T + b.double()
+    assert bool(((want.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + (K + 1) * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T + b.abs())).all())
