@@ -270,7 +270,7 @@ __device__ __forceinline__ bool group_tile(const int32_t* __restrict__ offsets, 
 
 // GROUPS: 0 none; 1 a workgroup for every row tile that a group can have; 2 as many as all groups' rows need, each every gridDim.y-th row tile of all
 // groups, which it has to find (0.8 us)
-template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT, int GROUPS>
+template <typename TW, bool DUAL, int FM, int FN, int WM, int WN, bool EXT, int GROUPS, bool AHEAD>
 __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
   constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN, BK = 32, NST = 4, ND = DUAL ? 2 : 1;
   constexpr bool WF = sizeof(TW) == 4;
@@ -349,9 +349,11 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s)
       if (s < KT) issue(s);
-    // a step's fragments are read during the matrix instructions of the step before: with one or two waves on a SIMD nothing else stands beside
-    // the barrier and the reads' latency.  us, before / so: 728 rows of fp32 steps, the wide products 45.2 / 43.7, the narrow ones 12.3 / 11.8; 8192
-    // rows x 64 x 2048 31.5 / 30.2; experts 82 / 81.5 (three workgroups per CU there); steps of 13 to 15 sequences 2.5 % less.
+    // AHEAD: a step's fragments are read during the matrix instructions of the step before: with one or two waves on a SIMD nothing else stands
+    // beside the barrier and the reads' latency.  Of the time without: 32 x 32 tiles, one weight in fp32 0.91 .. 0.97 (200 x 1024 x 1024 11.7 / 10.8 us, 728 x
+    // 1024 x 1024 21.4 / 20.6), in bf16 0.94 .. 0.98 and two weights 0.95 .. 0.98 up to a tile per CU, 0.98 .. 1.03 from two on.  Larger tiles keep a SIMD's
+    // matrix pipe busy with the waves of a CU's other tiles: 32 x 64 0.97 .. 1.07, 64 x 64 1.00, and where these ran in step, a CU was given two of
+    // the last tiles and its neighbour none (two weights, 1500 x 1024 x 1024 64 / 78 us; one, 2100 x 1408 x 1088 65 / 80).
     struct Frags {
       f32x4 x[2][FM];
       std::conditional_t<WF, f32x4, u32x2> w[2][ND][FN];
@@ -381,7 +383,7 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
             else f.w[ks][d][j] = *reinterpret_cast<const u32x2*>(sw + d * WB + r * 64 + (((ks * 2 + (kg >> 1)) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8);
           }
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
     };
     auto multiply = [&](const Frags& f) __attribute__((always_inline)) {
 #pragma unroll
@@ -405,20 +407,27 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
                 acc[d][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[d][j][e], f.x[ks][i][e], acc[d][i][j], 0, 0, 0);
       }
     };
-    read(0, fa);
-    int kt = 1;
-    for (; kt + 1 < KT; kt += 2) {
-      read(kt, fb);
-      multiply(fa);
-      read(kt + 1, fa);
-      multiply(fb);
-    }
-    if (kt < KT) {
-      read(kt, fb);
-      multiply(fa);
-      multiply(fb);
+    if constexpr (AHEAD) {
+      read(0, fa);
+      int kt = 1;
+      for (; kt + 1 < KT; kt += 2) {
+        read(kt, fb);
+        multiply(fa);
+        read(kt + 1, fa);
+        multiply(fb);
+      }
+      if (kt < KT) {
+        read(kt, fb);
+        multiply(fa);
+        multiply(fb);
+      } else {
+        multiply(fa);
+      }
     } else {
-      multiply(fa);
+      for (int kt = 0; kt < KT; ++kt) {
+        read(kt, fa);
+        multiply(fa);
+      }
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
@@ -1164,10 +1173,12 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
       const int64_t total = rows_per_group_max / bm + groups, fill = (1024 + nx(bn) - 1) / nx(bn);
       return dim3(nx(bn), (unsigned)std::min<int64_t>(std::min(most, std::max(total, fill)), 65535), 1);
     };
-    const auto cost = [&](int bm, int bn, double us) {
+    const auto per_cu = [&](int bm, int bn) {
       const int64_t row_tiles = grouped ? rows_per_group_max / bm + (groups + 1) / 2 : (int64_t)((rows_per_group_max + bm - 1) / bm) * groups;
-      const int64_t per_cu = (row_tiles * nx(bn) + 255) / 256;
-      return per_cu == 1 ? 1.07 * us : (double)per_cu * us;   // (alone on its CU a tile waits out its own starts)
+      return (row_tiles * nx(bn) + 255) / 256;
+    };
+    const auto cost = [&](int bm, int bn, double us) {
+      return per_cu(bm, bn) == 1 ? 1.07 * us : (double)per_cu(bm, bn) * us;   // (alone on its CU a tile waits out its own starts)
     };
     // (two weights: 64 x 64 has a CU to itself; the small tiles read their operands most often: beyond two per CU only where it is clear)
     const double large = cost(64, 64, DUAL ? 21.0 : 18.7), medium = cost(32, 64, 9.6), one = cost(32, 32, 5.05), small = one > 11. ? 1.06 * one : one;
@@ -1176,12 +1187,15 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
       else if ((int)g.z == groups && groups > 1) hipLaunchKernelGGL(direct, g, dim3(256), 0, st, a);
       else hipLaunchKernelGGL(found, g, dim3(256), 0, st, a);
     };
-#define MI_F32_TILE(FM, FN, WM, WN)                                                                                          \
-  gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, 0>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 1>, \
-      gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 2>
-    if (a.N > 32 && large <= medium && large <= small) go(MI_F32_TILE(2, 2, 2, 2), grid(64, 64));
-    else if (a.N > 32 && medium <= small) go(MI_F32_TILE(2, 1, 1, 4), grid(32, 64));
-    else go(MI_F32_TILE(1, 1, 2, 2), grid(32, 32));
+#define MI_F32_TILE(FM, FN, WM, WN, AHEAD)                                                                                          \
+  gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, 0, AHEAD>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 1, AHEAD>, \
+      gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 2, AHEAD>
+    // (fragments a step ahead: see the kernel)
+    constexpr bool always_ahead = !DUAL && sizeof(TW) == 4;
+    if (a.N > 32 && large <= medium && large <= small) go(MI_F32_TILE(2, 2, 2, 2, false), grid(64, 64));
+    else if (a.N > 32 && medium <= small) go(MI_F32_TILE(2, 1, 1, 4, false), grid(32, 64));
+    else if (always_ahead || per_cu(32, 32) <= 2) go(MI_F32_TILE(1, 1, 2, 2, true), grid(32, 32));
+    else go(MI_F32_TILE(1, 1, 2, 2, always_ahead), grid(32, 32));
 #undef MI_F32_TILE
     return check_launch();
   }

@@ -76,7 +76,7 @@ def test_few_features_over_rows_that_are_no_whole_lines(dtype, M, N, K, odd):
 
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192])
 @pytest.mark.parametrize("M,N,dtype,dual", [(130, 40, torch.float32, False), (300, 200, torch.float32, True), (700, 512, torch.bfloat16, False),
-                                            (1300, 900, torch.float32, False), (1300, 900, torch.bfloat16, True)])
+                                            (1300, 900, torch.float32, False), (1300, 900, torch.bfloat16, True), (400, 1408, torch.bfloat16, True)])
 def test_fragments_read_a_step_ahead(M, N, dtype, dual, K):
     """one to six K steps (fewer than the ring holds, odd and even) of every tile size: K roundings of the terms' sum"""
     from nanovllm import _C, ops
