@@ -227,51 +227,69 @@ __global__ __launch_bounds__(256) void blocks_prepare_kernel(BlockArgs a) {
   for (int d = tid; d < DP; d += 256) rec_b[512 + d] = gamma[d];
 }
 
-// The rank-th sequence in the order of the rows it brings, the most first: the longest chains begin first and alone.  By one wave for itself.
+// The rank-th sequence in the order of the rows it brings, the most first: the longest chains begin first and alone.  By one wave for itself, a
+// lane for every 64th sequence (up to kOrderedSeqs: read again in every round of the bisection, the numbers of 233 sequences, all but 29 of one row,
+// 16 heads of 64 x 128, took a third of the whole call: 679 us, so 455).
+constexpr int kOrderedSeqs = 512;
 __device__ __forceinline__ int by_length(const int32_t* cu_q, int n_seqs, int rank) {
   const int lane = threadIdx.x & 63;
-  auto rows = [&](int i) __attribute__((always_inline)) { return i < n_seqs ? cu_q[i + 1] - cu_q[i] : -1; };
-  const int mine = rows(lane);
-  auto count = [&](auto&& f) __attribute__((always_inline)) {
-    int c = __popcll(__ballot(f(mine)));
-    for (int i0 = 64; i0 < n_seqs; i0 += 64) c += __popcll(__ballot(f(rows(i0 + lane))));
-    return c;
-  };
-  int lo = 0, hi = cu_q[n_seqs] + 1, behind = 0;   // count(n >= lo) > rank >= count(n >= hi) = behind
+  int n[kOrderedSeqs / 64], top = 0;
+#pragma unroll
+  for (int j = 0; j < kOrderedSeqs / 64; ++j) {
+    const int i = j * 64 + lane;
+    n[j] = i < n_seqs ? cu_q[i + 1] - cu_q[i] : -1;
+  }
+#pragma unroll
+  for (int j = 0; j < kOrderedSeqs / 64; ++j) top = max(top, n[j]);
+#pragma unroll
+  for (int o = 1; o < 64; o *= 2) top = max(top, __shfl_xor(top, o));
+  int lo = 0, hi = __builtin_amdgcn_readfirstlane(top) + 1, behind = 0;   // count(n >= lo) > rank >= count(n >= hi) = behind
   while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1, c = count([&](int n) { return n >= mid; });
+    const int mid = (lo + hi) >> 1;
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < kOrderedSeqs / 64; ++j)
+      if (j * 64 < n_seqs) c += __popcll(__ballot(n[j] >= mid));
     if (c > rank) lo = mid;
     else hi = mid, behind = c;
   }
-  for (int i0 = 0, k = rank - behind; i0 < n_seqs; i0 += 64) {
-    uint64_t has = __ballot(rows(i0 + lane) == lo);
+  int k = rank - behind, found = 0;
+#pragma unroll
+  for (int j = 0; j < kOrderedSeqs / 64; ++j) {
+    uint64_t has = __ballot(n[j] == lo);
     const int c = __popcll(has);
-    if (k < c) {
-      for (; k > 0; --k) has &= has - 1;
-      return i0 + __builtin_ctzll(has);
+    if (k >= 0 && k < c) {
+      for (int l = 0; l < k; ++l) has &= has - 1;
+      found = j * 64 + __builtin_ctzll(has);
     }
     k -= c;
   }
-  return 0;   // (not reached: ranks are below n_seqs)
+  return found;
 }
 
-// grid: (heads, value columns / 32, sequences) in one, the longest sequences first; two waves take 16 columns, each half of the key channels: what
+// grid: (heads, value columns / (16 CG), sequences) in one, the longest sequences first; two waves take 16 columns, each half of the key channels: what
 // one has read of the state meets the other's in LDS, both then have the block's u; the rows' results, which nothing waits for, are put together
-// beside the next block's products.  Rings (three records, two where three do not leave room for two workgroups per CU), with the rows' values
-// behind each, by LDS-DMA a block or two ahead, its pieces between the products; in front of a group's matrix instructions stand the LDS reads of
-// the next one.  us, before (one wave for all channels, 64 columns a workgroup, sequences in order) / so: 11 sequences, 8112 rows, 8 heads of 128 x
-// 128 219 / 158 (sequences in order 201; 64 columns, eight waves in step 215); 728 rows of 16 sequences 58 / 39.
-template <int DT>
-__global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
-  constexpr int DP = 16 * DT, HT = DT / 2, KT = HT < 4 ? HT : 4, REC = record_floats(DP), PIECES = REC / 256, PP = (PIECES + 3) / 4, IMG = REC * 4 + 2048;
-  constexpr int NST = 3 * IMG + 6144 <= 81920 ? 3 : 2;
-  __shared__ __attribute__((aligned(1024))) char lds[NST * IMG + 6144];   // (behind the ring: four waves' D, two waves' E)
+// beside the next block's products.  Two records with the rows' values behind each, by LDS-DMA a block ahead, its pieces between the products; in
+// front of a group's matrix instructions stand the LDS reads of the next one.  us, before (one wave for all channels, 64 columns a workgroup,
+// sequences in order) / so: 11 sequences, 8112 rows, 8 heads of 128 x 128 219 / 158 (sequences in order 201; 64 columns, eight waves in step 215); 728
+// rows of 16 sequences 58 / 39.  Of the whole call's time before, drawn steps of 1 .. 500 sequences: 128 channels 0.68 .. 1.02, 64 0.67 .. 1.06 (the most
+// where equal sequences filled the CUs once with 64 columns each and now do twice, with 32), 200 and 256 0.61 .. 1.00.
+// 64 channels: four workgroups per CU (with a ring of three records and two per CU, 13 sequences of 1752 rows, 16 heads of 64 x 128 677 / 767 us,
+// 26 of 840, 8 heads 322 / 363; so 718 and 338) - 128 registers, hence E's products behind D's sum.
+// CG: groups of 16 columns of a workgroup.  256 channels leave room for one workgroup per CU: 32 columns were twice the records for
+// sequences of a row or two (69 sequences of up to 130 rows, 16 heads of 256 x 256 421 / 520 us; so 414), 64 where there are more than the chip holds.
+template <int DT, int CG = 2>
+__global__ __launch_bounds__(128 * CG, DT == 4 ? 4 : CG == 4 || DT == 8 ? 2 : 1) void blocks_walk_kernel(BlockArgs a) {
+  constexpr int DP = 16 * DT, HT = DT / 2, KT = HT < 4 ? HT : 4, REC = record_floats(DP), PIECES = REC / 256, PP = (PIECES + 2 * CG - 1) / (2 * CG);
+  constexpr int IMG = REC * 4 + CG * 1024;
+  constexpr bool FOUR = DT == 4;   // workgroups per CU
+  __shared__ __attribute__((aligned(1024))) char lds[2 * IMG + 3 * CG * 1024];   // (behind the ring: all waves' D, half of the waves' E)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
-  const int cg = wave & 1, half = wave >> 1;   // 16 columns, HT tiles of 16 key channels
+  const int cg = wave % CG, half = wave / CG;   // 16 columns, HT tiles of 16 key channels
   // heads, their columns (one XCD's, where the heads are a multiple of eight: they share the records), sequences
-  const int zs = (a.Dv + 31) / 32, hz = (int)blockIdx.x % (a.H * zs), h = hz % a.H, col = hz / a.H * 32 + cg * 16 + r16;
-  const int s = by_length(a.cu_q, a.n_seqs, (int)blockIdx.x / (a.H * zs));
+  const int zs = (a.Dv + 16 * CG - 1) / (16 * CG), hz = (int)blockIdx.x % (a.H * zs), h = hz % a.H, col = hz / a.H * (16 * CG) + cg * 16 + r16;
+  const int rank = (int)blockIdx.x / (a.H * zs), s = a.n_seqs <= kOrderedSeqs ? by_length(a.cu_q, a.n_seqs, rank) : rank;
   const int r0 = a.cu_q[s], n = a.cu_q[s + 1] - r0;
   if (n == 0) return;
   const int nb = (n + kB - 1) / kB;
@@ -316,8 +334,8 @@ __global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
       for (int r = 0; r < 4; ++r) S[m][r] = st[(4 * m + r) * (4 * kStateCols) + cc * 4 + kg];
     }
   }
-  const uint32_t x_mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + NST * IMG) + wave * 1024 + lane * 16;
-  const uint32_t x_other = half ? x_mine - 2048 : x_mine + 2048, x_e = x_mine + (half ? 2048 : 4096);
+  const uint32_t x_mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(lds + 2 * IMG) + wave * 1024 + lane * 16;
+  const uint32_t x_other = half ? x_mine - CG * 1024 : x_mine + CG * 1024, x_e = x_mine + (half ? CG : 2 * CG) * 1024;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   float* op = a.out + (int64_t)(r0 + 4 * kg) * a.ldo + (int64_t)h * a.Dv + col;   // (formed beyond the columns, not used there)
   auto store = [&](int b) __attribute__((always_inline)) {
@@ -333,11 +351,8 @@ __global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
     op += (int64_t)kB * a.ldo;
   };
 #pragma unroll
-  for (int i = 0; i + 1 < NST; ++i) {
-#pragma unroll
-    for (int q = 0; q < PP; ++q) piece(i, i, q);
-    values(i, i);
-  }
+  for (int q = 0; q < PP; ++q) piece(0, 0, q);
+  values(0, 0);
   f32x4 e_own = {}, x = {}, w = {}, u = {};
   // block b's rows, when the halves' sums of E have met (in the next block, beside its products)
   auto finish = [&](int b) __attribute__((always_inline)) {
@@ -358,13 +373,12 @@ __global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
   };
   int cur = 0;
   for (int b = 0; b < nb; ++b) {
-    // record b has landed (a ring of three: record b + 1's requests may be out); everybody is done with record b - 1: its place is free
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * (PP + 2)) : "memory");
+    // record b has landed; everybody is done with record b - 1: its place is free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     if (b > 0 && half == 0) finish(b - 1);   // (the other half's products keep the matrix pipe busy)
-    const int next = cur == 0 ? NST - 1 : cur - 1;
     const char* const img = lds + cur * IMG;
-    cur = cur == NST - 1 ? 0 : cur + 1;
+    cur ^= 1;
     const char* const rec = img + lane * 16 + half * HT * 1024;
     const char* const rec_q = rec + DP * kB * 4;
     const char* const rec_k = rec_q + DP * kB * 4;
@@ -374,7 +388,7 @@ __global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
     f32x4 d[8], e[8];   // (eight chains: each is an eighth as long, and so is its rounding)
 #pragma unroll
     for (int r = 0; r < 8; ++r) d[r] = e[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    f32x4 pf[2][2], qf[2][2], gf[2][2], kf[2][4], tf = vec(rec_b + 1024), bf = vec(rec_b);
+    f32x4 mine, pf[2][2], qf[2][2], gf[2][2], kf[2][4], tf = vec(rec_b + 1024), bf = vec(rec_b);
 #pragma unroll
     for (int r = 0; r < 4; ++r) u[r] = *reinterpret_cast<const float*>(img + REC * 4 + cg * 1024 + r * 256 + lane * 4);
     auto read_q = [&](int c) __attribute__((always_inline)) {
@@ -401,27 +415,35 @@ __global__ __launch_bounds__(256, 2) void blocks_walk_kernel(BlockArgs a) {
         for (int r = 0; r < 4; ++r) {
           f32x4 &dx = d[4 * i + r], &ex = e[4 * i + r];
           dx = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[c & 1][i][r], S[2 * c + i][r], dx, 0, 0, 0);
-          ex = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c & 1][i][r], S[2 * c + i][r], ex, 0, 0, 0);
-          // the record after the next, a piece behind every few products (in front of them all the CU's requests took 700 cycles)
+          if constexpr (!FOUR) ex = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c & 1][i][r], S[2 * c + i][r], ex, 0, 0, 0);
+          // the next record, a piece behind every few products (in front of them all the CU's requests took 700 cycles)
           constexpr int EVERY = HT * 4 / PP;
           static_assert(EVERY > 0, "every piece has its place");
           const int at = (c * 2 + i) * 4 + r;
           if (at % EVERY == EVERY - 1 && at / EVERY < PP) {
-            piece(b + NST - 1, next, at / EVERY);
+            piece(b + 1, cur, at / EVERY);
             __builtin_amdgcn_sched_barrier(0);
           }
           if (at == HT * 4 - 1) {
-            values(b + NST - 1, next);
+            values(b + 1, cur);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
+      if constexpr (FOUR) {   // (E behind D: a set of chains less in registers)
+        mine = sum8(d);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) e[4 * i + r] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[0][i][r], S[i][r], e[4 * i + r], 0, 0, 0);
+      }
 #pragma unroll
       for (int i = 0; i < 2; ++i) S[2 * c + i] *= gf[c & 1][i];
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) u[r] = has_col && b * kB + 4 * kg + r < n ? u[r] : 0.f;
-    const f32x4 mine = sum8(d);
+    if constexpr (!FOUR) mine = sum8(d);
     f32x4 other;
     asm volatile("ds_write_b128 %0, %1" ::"v"(x_mine), "v"(mine) : "memory");
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (read below, and written again only behind the next block's barrier)
@@ -824,18 +846,20 @@ extern "C" int mi_channel_delta_blocks(const float* qkv, int64_t ld, int q_off, 
   if (!aligned16(workspace) || ws_elems < ((int64_t)n_rows / kB + n_seqs) * H * record_floats(16 * dt)) return MI_EWORKSPACE;
   const BlockArgs a{qkv, ld, q_off, k_off, v_off, beta_pre, ld_beta, decay_pre, ld_decay, dt_bias, a_log, cu_q, kv_lens, slot_ids,
                     n_seqs, H, G, D, Dv, state, workspace, out, ldo};
-  const int64_t walks = (int64_t)n_seqs * H * ((Dv + 31) / 32);   // (a block of the state's layout each)
-  if (walks > 0x7fffffff) return MI_EUNSUPPORTED;
-  const dim3 prep(n_rows / kB + n_seqs, H), walk((unsigned)walks);
-  const auto launch = [&](auto prepare, auto walk_kernel) -> int {
+  const auto walks = [&](int cg) { return (int64_t)n_seqs * H * ((Dv + 16 * cg - 1) / (16 * cg)); };   // (32 columns: a block of the state's layout)
+  if (walks(2) > 0x7fffffff) return MI_EUNSUPPORTED;
+  const dim3 prep(n_rows / kB + n_seqs, H);
+  const auto launch = [&](auto prepare, auto walk_kernel, int cg) -> int {
     hipLaunchKernelGGL(prepare, prep, dim3(256), 0, S(stream), a);
     if (check_launch() != MI_OK) return MI_ELAUNCH;
-    hipLaunchKernelGGL(walk_kernel, walk, dim3(256), 0, S(stream), a);
+    hipLaunchKernelGGL(walk_kernel, dim3((unsigned)walks(cg)), dim3(128 * cg), 0, S(stream), a);
     return check_launch();
   };
-  const int rc = dt == 4   ? launch(blocks_prepare_kernel<4>, blocks_walk_kernel<4>)
-                 : dt == 8 ? launch(blocks_prepare_kernel<8>, blocks_walk_kernel<8>)
-                           : launch(blocks_prepare_kernel<16>, blocks_walk_kernel<16>);
+  // (256 channels: a CU holds one workgroup; where 32 columns each would be more than that, 64)
+  const int rc = dt == 4             ? launch(blocks_prepare_kernel<4>, blocks_walk_kernel<4>, 2)
+                 : dt == 8           ? launch(blocks_prepare_kernel<8>, blocks_walk_kernel<8>, 2)
+                 : walks(2) <= 256   ? launch(blocks_prepare_kernel<16>, blocks_walk_kernel<16>, 2)
+                                     : launch(blocks_prepare_kernel<16>, blocks_walk_kernel<16, 4>, 4);
   return rc != MI_OK ? rc : launch_head_norm(out, ldo, gate_pre, ld_gate, norm_w, n_rows, H, Dv, eps, S(stream));
 }
 

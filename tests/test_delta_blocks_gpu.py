@@ -91,10 +91,12 @@ def test_channel_delta_by_blocks(ops, lens, H, G, D, Dv):
     assert all((s_blocks[len(lens) - 1 - i] == 7.0).all() for i, n in enumerate(lens) if n == 0)
 
 
-@pytest.mark.parametrize("lens", [tuple(i * 37 % 23 for i in range(70)), (40,) * 65, (0,) * 64 + (33, 0, 34), (1,) * 3 + (90,)])
-@pytest.mark.parametrize("H,G,D,Dv", [(3, 1, 64, 40), (2, 2, 128, 96)])
+@pytest.mark.parametrize("lens", [tuple(i * 37 % 23 for i in range(70)), (40,) * 65, (0,) * 64 + (33, 0, 34), (1,) * 3 + (90,),
+                                  tuple(i % 3 for i in range(511)) + (35,), tuple(i % 3 for i in range(512)) + (35,)])
+@pytest.mark.parametrize("H,G,D,Dv", [(3, 1, 64, 40), (2, 2, 128, 96), (4, 2, 200, 72)])
 def test_sequences_in_the_order_of_their_rows(ops, lens, H, G, D, Dv):
-    """every sequence walked once: more than a wave looks at, equal ones, empty ones"""
+    """every sequence walked once: more than a wave looks at, as many as are put in order and one more, equal ones, empty ones; 256 channels
+    with 32 columns a workgroup and (more of them than CUs) 64, which are beyond the state's columns here"""
     test_channel_delta_by_blocks(ops, lens, H, G, D, Dv)
 
 
