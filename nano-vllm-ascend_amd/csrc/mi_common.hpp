@@ -31,17 +31,19 @@ __device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
 __device__ __forceinline__ float rbf(float f) { return bf2f(f2bf(f)); }
 
 // z / (1 + exp(-z)) in half the instructions of expf and a division (a tile product's epilogue has 128 of them a lane, with no matrix
-// instruction beside them): exp2 of the fraction of -z log2(e), which two fused steps leave exact to the last bit, times the power of
-// two; one Newton step on the quotient.  med3 clamps the argument to where the exponential is 0 or infinity anyhow, and takes a NaN
-// for its lower bound, so that an infinite z or denominator keeps its quotient.  Error against 64 bits, relative 2-norm over normal z
-// of deviation 0.5 / 2 / 6: 3.92 / 4.17 / 3.39e-8, as the two calls'.
+// instruction beside them).  The exponential by two-part argument reduction: -z log2(e) less the nearest whole number n, log2(e) as a float
+// and the rounded rest of it, leaves a fraction exact to the last bit; exp2 of that times 2^n.  The quotient by one Newton step on z / 4 and a
+// quarter of the denominator, whose reciprocal is a normal number wherever the exponential is finite (v_rcp_f32 gives 0 for 1 / d below 2^-126: z from
+// -88.7 to -87.4 were 0 instead of some -5e-37).  med3 clamps the argument to where the exponential is 0 or infinity anyhow, and takes a NaN for
+// its lower bound, so that an infinite z or denominator keeps its quotient.  Error against 64 bits, relative 2-norm over normal z of deviation
+// 0.5 / 2 / 6: 3.92 / 4.17 / 3.39e-8, as the two calls'.
 __device__ __forceinline__ float silu_f32(float z) {
-  const float c = __builtin_amdgcn_fmed3f(z, -104.f, 104.f);
+  const float c = __builtin_amdgcn_fmed3f(z, -104.f, 104.f), z4 = 0.25f * z;
   const float n = __builtin_rintf(c * -1.44269502162933349609375f);
   const float f = fmaf(c, -1.925963033500011e-8f, fmaf(c, -1.44269502162933349609375f, -n));
-  const float d = 1.f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
-  const float r = __builtin_amdgcn_rcpf(d), q = z * r;
-  return fmaf(__builtin_amdgcn_fmed3f(fmaf(-q, d, z), -3e38f, 3e38f), r, q);
+  const float d4 = fmaf(__builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n), 0.25f, 0.25f);
+  const float r = __builtin_amdgcn_rcpf(d4), q = z4 * r;
+  return fmaf(__builtin_amdgcn_fmed3f(fmaf(-q, d4, z4), -3e38f, 3e38f), r, q);
 }
 __device__ __forceinline__ bf16x8 as_frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 

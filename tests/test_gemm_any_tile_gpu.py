@@ -201,11 +201,13 @@ def test_whole_feature_tiles_of_the_persistent_kernel(form, rows, N, K):
 
 @pytest.mark.parametrize("tile", [64, 256])
 def test_silu_of_large_arguments(tile):
-    """0 and z to an ulp where the exponential is out of range, finite everywhere"""
-    z = torch.tensor([0.0, -0.0, 80.0, -80.0, 87.0, 88.0, -88.0, 104.5, -104.5, 1e30, -1e30, 3e38, -3e38], device="cuda").bfloat16().float().repeat(6)
+    """0 and z to an ulp where the exponential is out of range, finite everywhere; to an ulp also where the quotient's reciprocal is no normal
+    number (-88.5 .. -87.5); below that the exponential overflows, as expf's did"""
+    z = torch.tensor([0.0, -0.0, 80.0, -80.0, 87.0, 88.0, -87.0, -87.5, -88.0, -88.5, 104.5, -104.5, 1e30, -1e30, 3e38, -3e38], device="cuda").bfloat16().float().repeat(5)
     x, w, w2 = torch.zeros(z.numel(), 64, device="cuda"), torch.zeros(128, 64, device="cuda"), torch.zeros(128, 64, device="cuda")
     x[:, 0], x[:, 1], w[:, 0], w2[:, 1] = z, 1.0, 1.0, 1.0
     out = torch.empty(z.numel(), 128, device="cuda")
     ops._tile_gemm(ops._tile_operand(x, tile), tile, w.bfloat16(), w2.bfloat16(), out, _C.ACT_SILU)
     want = torch.nn.functional.silu(z.double()).unsqueeze(1)
-    assert bool(((out.double() - want).abs() <= 4 * 2.0 ** -24 * want.abs() + 1e-35).all())
+    low = torch.where((z < -88.72) & (z > -120), 3e-37, 0.0).unsqueeze(1)   # (z / inf)
+    assert bool(((out.double() - want).abs() <= 4 * 2.0 ** -24 * want.abs() + low).all())
