@@ -37,3 +37,24 @@ def test_prefill_attention_of_few_rows_rule():
     assert not takes(1, 8, 1, 2561, 2768) and not takes(1, 16, 1, 923, 928) and not takes(1, 32, 2, 914, 928) and not takes(1, 8, 1, 340, 2560)
     assert not takes(40, 32, 2, 14, 16) and not takes(2, 32, 8, 384, 688) and not takes(4, 8, 8, 1024, 1024) and not takes(1, 16, 8, 2049, 2064)
     assert not takes(1, 16, 8, 2048, 8192)   # (a table wider than the prompt: a prefix may lie in front of it)
+
+
+def test_moe_tiles_refusals():
+    """What mi_moe_tiles refuses before any launch: missing and misaligned operands, more tokens than pairs, sizes it does not take, and
+    scratch that is a byte short."""
+    from nanovllm import _C
+
+    lib, EINVAL, EUNSUPPORTED, EWORKSPACE = _C.lib, -1, -2, -3
+    pairs, E, H, I = 2400, 8, 1024, 512
+    n = lib.mi_moe_tiles_bytes(pairs, E, I, H)
+    assert n > 0 and lib.mi_moe_tiles_bytes(120, E, I, H) == 0 and lib.mi_moe_tiles_bytes(pairs, E, I + 8, H) == 0
+    good = dict(x=4096, n_tokens=1200, gate_up=4096, down=4096, offsets=4096, pair_token=4096, pair_index=4096, act=4096, y=4096, pairs=pairs, n_experts=E,
+                hidden=H, inter=I, scratch=4096, scratch_bytes=n - 1)   # (never read: the last refusal is the scratch's)
+    call = lambda **k: lib.mi_moe_tiles(*{**good, **k}.values(), 0)  # noqa: E731
+    codes = [call()]
+    for name in ("x", "gate_up", "down", "act", "y", "scratch"):
+        codes += [call(**{name: 0}), call(**{name: 4098})]
+    for name in ("offsets", "pair_token", "pair_index"):
+        codes.append(call(**{name: 0}))
+    codes += [call(n_tokens=0), call(n_tokens=pairs + 1), call(pairs=120, n_tokens=60), call(inter=I + 8), call(scratch_bytes=0)]
+    assert codes == [EWORKSPACE] + [EINVAL] * 15 + [EINVAL] * 2 + [EUNSUPPORTED] * 2 + [EWORKSPACE], codes

@@ -1198,6 +1198,57 @@ def test_moe_block_from_the_stored_weights(ops, T, H, E, K, I, tile, uneven):
     _assert_moe_close(got.cpu(), want.cpu())
 
 
+@pytest.mark.parametrize("H,I", [(640, 192), (640, 256), (1024, 192)])
+@pytest.mark.parametrize("uneven", [False, True])
+def test_moe_products_of_part_feature_tiles(ops, H, I, uneven):
+    """mi_moe_tiles on 256-row tiles whose last feature tile is part-filled in the first product, the second or both (the persistent kernel's
+    general epilogue): its activations and results row by row against both products in 64 bits, one bf16 rounding of each side of the
+    SwiGLU and of the result apart, no row beside them written."""
+    E, K, T = 8, 2, 12000
+    P = T * K
+    g = torch.Generator(device=DEV).manual_seed(H + I + uneven)
+    x = torch.randn(T, H, device=DEV, generator=g).bfloat16()
+    gu, dn = ((torch.randn(E, *s, device=DEV, generator=g) * s[1] ** -0.5).bfloat16() for s in ((2 * I, H), (H, I)))
+    counts = torch.tensor([P // 2 - 700, 0, 700] + [P // 10] * 5 if uneven else [P // E] * E)
+    off = torch.tensor([0] + counts.cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    assert int(off[-1]) == P and all(ops.lib.mi_gemm_any_tile_rows(P, n, k, E, d, d) == 256 for n, k, d in ((I, H, 1), (H, I, 0)))
+    token = (torch.randperm(P, device=DEV, generator=g) // K).to(torch.int32)
+    place = torch.randperm(P, device=DEV, generator=g).to(torch.int32)
+    n = ops.lib.mi_moe_tiles_bytes(P, E, I, H)
+    scratch = torch.empty(n, dtype=torch.uint8, device=DEV)
+    act, y = torch.full((P + 1, I), 7.0, dtype=torch.bfloat16, device=DEV), torch.full((P + 1, H), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert ops.lib.mi_moe_tiles(ops.ptr(x), T, ops.ptr(gu), ops.ptr(dn), ops.ptr(off), ops.ptr(token), ops.ptr(place), ops.ptr(act), ops.ptr(y),
+                                P, E, H, I, ops.ptr(scratch), n, ops.stream()) == 0
+    assert bool((act[P] == 7.0).all()) and bool((y[P] == 7.0).all())
+    for e in range(E):
+        r = slice(int(off[e]), int(off[e + 1]))
+        xe, at = x[token[r].long()].float(), place[r].long()
+        z, u = xe @ gu[e, :I].float().T, xe @ gu[e, I:].float().T
+        want = torch.nn.functional.silu(z) * u
+        # (z and u are rounded to bf16 each, silu(z) and the product too: 2^-8 each, silu's slope is at most 1.1; fp32 sums behind that)
+        tol = 2.0 ** -8 * (3 * want.abs() + 1.1 * z.abs() * u.abs()) * 1.02 + 1e-4
+        assert bool(((act[r].float() - want).abs() <= tol).all()), e
+        want = act[r].float() @ dn[e].float().T
+        size = act[r].float().abs() @ dn[e].float().abs().T
+        assert bool(((y[at].float() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 2 * I * 2.0 ** -24 * size).all()), e
+
+
+def test_moe_block_in_one_step_and_in_small_ones(ops):
+    """The same tokens in one step of many pairs (the stored weights on the tile kernels) and in steps below the line (the packed ones): the
+    same picks, and rows that differ by the order of the sums over K alone."""
+    T, H, E, K, I = 1200, 1024, 8, 2, 512
+    gen = torch.Generator().manual_seed(11)
+    x, logits = torch.randn(T, H, generator=gen).bfloat16().to(DEV), torch.randn(T, E, generator=gen).bfloat16().to(DEV)
+    gu, dn = ((torch.randn(E, *s, generator=gen) * s[1] ** -0.5).bfloat16().to(DEV) for s in ((2 * I, H), (H, I)))
+    packed = ops.pack_expert_weights(gu), ops.pack_expert_weights(dn)
+    step = 60
+    assert ops.lib.mi_moe_tiles_bytes(T * K, E, I, H) > 0 and ops.lib.mi_moe_tiles_bytes(step * K, E, I, H) == 0
+    whole, ids, w = ops.moe_forward(x, logits, *packed, K, gate_up=gu, down=dn)
+    parts = [ops.moe_forward(x[i:i + step], logits[i:i + step], *packed, K, gate_up=gu, down=dn) for i in range(0, T, step)]
+    assert torch.equal(ids, torch.cat([p[1] for p in parts])) and torch.equal(w, torch.cat([p[2] for p in parts]))
+    _assert_moe_close(torch.cat([p[0] for p in parts]).cpu(), whole.cpu())
+
+
 @pytest.mark.parametrize("T", [1, 32, 64, 100])
 @pytest.mark.parametrize("inter", [768, 192])
 def test_moe_block_qwen3_30b_a3b_shapes(ops, T, inter):
