@@ -212,8 +212,15 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
     // 96 43 / 40 / 50, 192 52 / 43 / 52, 256 62 / 67 / 52, 512 105 / 103 / 97; 64 of 768 x 2048, 48 134 / 150 / 170, 64 149 / 156 / 172, 96 179 / 161 /
     // 192, 128 213 / 194 / 199, 192 272 / 257 / 209, 512 607 / 506 / 377; 8 of 512 x 1024, 96 18 / 27 / 47, 256 27 / 28 / 49, 512 41 / 38 / 50;
     // 128 of 256 x 1024, 48 56 / 70 / 67, 96 68 / 77 / 100, 160 97 / 93 / 103, 192 110 / 105 / 105, 256 138 / 132 / 108
+    // One product, K 512 to 4096, time of 128- by 64-row tiles at 64 to 88 rows: two weights 128 of 384 0.97 .. 1.06, 64 of 768 0.92 .. 1.07 (below 1 from
+    // K 3072 on), 64 of 512 1.11 .. 1.28, 96 of 640 0.88 .. 1.14, 48 of 1024 0.95 .. 1.05; one weight 0.82 .. 1.05, 64 of 512 0.93 .. 1.16, 96 of 640 with 88 rows 1.16 ..
+    // 1.25: within a tenth of the line either is right, for how the tiles fill the CUs.  Few of two weights: 128-row tiles where they are one per CU and
+    // groups of more than 64 rows make 64-row ones more than that (32 of 512 x 4096, 48 rows 118 / 99; 16 of 1024 x 2048 76 / 67, 24 of 640 x 1024 0.93 of the time).
     // (K below 512 was not measured: no more than the padding's rule there)
-    if (rows < (dual ? K >= 2048 ? 64 : 88 : 72) * (int64_t)n_groups || (K >= 512 && tiles(64, 64) < 512)) return 64;
+    if (rows < (dual ? K >= 2048 ? 64 : 88 : 72) * (int64_t)n_groups || (K >= 512 && tiles(64, 64) < 512)) {
+      const bool one_per_cu = dual && K >= 512 && n_groups * (int64_t)((N + 63) / 64) <= 256 && tiles(64, 64) > 256 && tiles(64, 64) <= 360;
+      return one_per_cu ? 128 : 64;
+    }
     return rows >= 160 * (int64_t)n_groups && tiles(128, dual ? 64 : 128) > 512 ? 256 : 128;
   }
   // us, cold weights, 64- / 128- / 256-row tiles: 2000 x 1024 x 1024 (512 / 128 / 32 tiles) 12 / 16 / 26, 2000 x 2048 x 1024 (1024 / 256 / 64) 23 / 18 / 28,
