@@ -508,12 +508,11 @@ static bool few_tiles(int M, int N) {
   return (int64_t)((M + TILE_T - 1) / TILE_T) * ((N + TILE_F - 1) / TILE_F) < kPersistentGrid;
 }
 // The 128-tile kernel: there, up to two 128-tiles per CU.  More are a second round of its workgroups, and 256-tiles on half of the CUs are
-// done before it (us, small tiles / 256-tiles: 4536 x 2048 x 1024 = 576 of 128, 144 of 256 29.9 / 25.1; 3000 x 4096 x 4096 114.9 / 77.5;
-// 1976 x 6144 x 2048 56.6 / 43.3; K 384: 3256 x 4096 20.2 / 17.3, 256: 256 x 40000 15.3 / 18.5; two per CU: 4024 x 2048 x 1024 21.6 / 25.0,
-// 1976 x 4096 x 4096 68.5 / 74.1).  The second round's time also hung on where the kernel's loop lies in its code (3000 x 4096 x 4096: 113
-// to 125).
+// done before it (us with cold weights, small tiles / 256-tiles, two per CU: 4024 x 2048 x 1024 26.2 / 31.2, 2000 x 4096 x 4096 76 / 93, 8000 x 1024 x 3072
+// 67 / 71; beyond, before a K step of the 256-tiles was shortened: 4536 x 2048 x 1024 29.9 / 25.1, 3000 x 4096 x 4096 115 / 78); of short K up to three
+// (10240 features x 256: 640 tiles 16.2 / 16.6, 880 19.5 / 16.8; 4096 x 128: 768 14.1 / 14.2, 896 15.5 / 14.6; 1024 x 320: 632 19.1 / 17.9, 816 22.6 / 19.2).
 static bool use_mid(int M, int N, int K) {
-  return few_tiles(M, N) && (K < 384 || (int64_t)((M + MID_T - 1) / MID_T) * ((N + MID_F - 1) / MID_F) <= 2 * kPersistentGrid);
+  return few_tiles(M, N) && (int64_t)((M + MID_T - 1) / MID_T) * ((N + MID_F - 1) / MID_F) <= (K < 384 ? 3 : 2) * kPersistentGrid;
 }
 
 struct MidPick {

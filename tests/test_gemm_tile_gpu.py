@@ -107,7 +107,7 @@ def test_gemm_tile_kernel_choice_boundary(ops, M):
     assert_bf16_close(gu, oracle.silu_and_mul(oracle.linear(x, w)), max_ulp=4, max_frac=3e-2, atol=32 * K * 2.0 ** -22)
 
 
-@pytest.mark.parametrize("M,N,K", [(4096, 2048, 384), (4097, 2048, 384), (2056, 3964, 448), (2056, 3964, 320), (130, 40000, 384)])
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 384), (4097, 2048, 384), (2056, 3964, 448), (2056, 3964, 320), (130, 40000, 384), (3072, 4096, 320), (3073, 4096, 320)])
 def test_gemm_tile_two_small_tiles_per_cu(ops, M, N, K):
     """either side of two 128-tiles per CU, where the 128-tile kernel hands over to the large one before the chip is full of 256-tiles
     (and of the K up to which it does not): one fp32 chain per element on both, so the same bits, and no K slices"""
