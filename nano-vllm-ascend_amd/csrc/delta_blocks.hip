@@ -16,7 +16,7 @@
 // What bounds it: the longest sequence's chain of blocks - 56 matrix instructions of 32 cycles a wave (128 channels), the LDS reads, sums and
 // barriers between them -, and the matrix pipe where two workgroups share a CU, against 0.71 us per ROW of the row-by-row walk (LDS reads,
 // cross-lane sums, plain FMAs).
-// 8 sequences of 1024 rows, 8 heads, 128 x 128: 809 us row by row, 294 so with one wave for all channels (preparation 83, walk 175).  The error against 64 bits is
+// 8 sequences of 1024 rows, 8 heads, 128 x 128: 809 us row by row, 206 so (one wave for all channels 263).  The error against 64 bits is
 // the row-by-row one's or less (rms of the results, 64 .. 1400 rows and decays from 0.05 to 1: 0.87 to 0.98 of it).  A NaN or an
 // infinity in a row must not reach the rows in front of it through the zeros above the diagonals of T and B: see causal() below.
 #include <type_traits>
@@ -820,14 +820,15 @@ static int tiles_of(int D) { return D <= 64 ? 4 : D <= 128 ? 8 : D <= 256 ? 16 :
 
 using namespace mi;
 
-// Where the block form is used: a sequence's chain of blocks is 2.7 us per 16 rows against 0.71 us a row, but every sequence, also one
-// that brings a single row, costs a record.  us, rows / blocks, 8 heads of 128 x 128: one sequence of 16 rows 24 / 30, of 64 58 / 38;
-// 32 sequences of 16 rows 32 / 45, of 64 86 / 76; 64 rows beside 31 single ones 63 / 59, 256 beside 255 281 / 274, 1024 beside 255
-// 986 / 606; 256 sequences of 2 rows 64 / 179.
+// Where the block form is used: a sequence's chain of blocks is 1.9 us per 16 rows against 0.71 us a row, but every sequence, also one
+// that brings a single row, costs a record and a workgroup per 32 columns.  us from cold inputs, rows / blocks, 8 heads of 128 x 128: one sequence of 16 rows
+// 35 / 35, of 32 46 / 37; 32 sequences of 16 rows 46 / 52, of 32 64 / 62; 64 of 16 69 / 75; 32 rows beside 31 single ones 50 / 46, 64 beside 127 96 / 107, 96
+// beside 127 124 / 108, 128 beside 255 174 / 193, 160 beside 255 201 / 193; 256 sequences of 2 rows 69 / 186 (4 heads of 64 x 128, 16 of 128 x 128
+// and 8 of 256 x 256: none slower beyond the line).
 extern "C" int64_t mi_channel_delta_blocks_elems(int n_rows, int n_seqs, int max_rows, int H, int D) {
   const int dt = tiles_of(D);
   if (n_rows < 0 || n_seqs < 1 || H < 1 || D < 1 || dt == 0) return -1;
-  if (max_rows < 64 + n_seqs / 2) return 0;
+  if (max_rows < 32 + n_seqs / 2) return 0;
   return ((int64_t)n_rows / kB + n_seqs) * H * record_floats(16 * dt);
 }
 

@@ -58,3 +58,12 @@ def test_moe_tiles_refusals():
         codes.append(call(**{name: 0}))
     codes += [call(n_tokens=0), call(n_tokens=pairs + 1), call(pairs=120, n_tokens=60), call(inter=I + 8), call(scratch_bytes=0)]
     assert codes == [EWORKSPACE] + [EINVAL] * 15 + [EINVAL] * 2 + [EUNSUPPORTED] * 2 + [EWORKSPACE], codes
+
+
+def test_delta_rule_by_blocks_rule():
+    """From 32 rows of a sequence on, and half a row more for every sequence of the step; 0 floats of workspace elsewhere."""
+    from nanovllm import _C
+
+    blocks = lambda rows, seqs, most: _C.lib.mi_channel_delta_blocks_elems(rows, seqs, most, 8, 128) > 0  # noqa: E731
+    assert blocks(33, 1, 33) and blocks(64 * 64, 64, 64) and blocks(160 + 255, 256, 160)
+    assert not blocks(31, 1, 31) and not blocks(63 * 64, 64, 63) and not blocks(512, 256, 2) and not blocks(1, 1, 1)
