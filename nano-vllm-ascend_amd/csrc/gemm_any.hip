@@ -351,8 +351,8 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
       if (s < KT) issue(s);
     // AHEAD: a step's fragments are read during the matrix instructions of the step before: with one or two waves on a SIMD nothing else stands
     // beside the barrier and the reads' latency.  Of the time without: 32 x 32 tiles, one weight in fp32 0.91 .. 0.97 (200 x 1024 x 1024 11.7 / 10.8 us, 728 x
-    // 1024 x 1024 21.4 / 20.6), in bf16 0.94 .. 0.98 and two weights 0.95 .. 0.98 up to a tile per CU, 0.98 .. 1.03 from two on (two in fp32 from K 1024 on
-    // 0.966 .. 1.00: experts of 512 x 1024, 90 rows each, 86 / 83).  Larger tiles keep a SIMD's
+    // 1024 x 1024 21.4 / 20.6), in bf16 0.94 .. 0.98 and two weights 0.95 .. 0.98 up to a tile per CU, 0.98 .. 1.03 from two on; two weights in fp32 with two tiles
+    // on some CUs 0.98 .. 1.06 (400 rows of 32 experts of 512 x 1024 29.0 / 30.7), with more from K 1024 on 0.97 .. 1.00.  Larger tiles keep a SIMD's
     // matrix pipe busy with the waves of a CU's other tiles: 32 x 64 one weight in fp32 0.955 .. 0.99 from K 1024 on and up to five tiles per CU, else
     // 0.98 .. 1.10 (K 512 1.00 .. 1.02, 160 1.00 .. 1.07; nine tiles 1.02), 64 x 64 1.00; and where these ran in step, a CU was given two of
     // the last tiles and its neighbour none (two weights, 1500 x 1024 x 1024 64 / 78 us; one, 2100 x 1408 x 1088 65 / 80).
@@ -1197,7 +1197,7 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
     if (a.N > 32 && large <= medium && large <= small) go(MI_F32_TILE(2, 2, 2, 2, false), grid(64, 64));
     else if (a.N > 32 && medium <= small && one_fp32 && a.K >= 1024 && per_cu(32, 64) <= 5) go(MI_F32_TILE(2, 1, 1, 4, one_fp32), grid(32, 64));
     else if (a.N > 32 && medium <= small) go(MI_F32_TILE(2, 1, 1, 4, false), grid(32, 64));
-    else if (one_fp32 || per_cu(32, 32) <= 2 || (sizeof(TW) == 4 && a.K >= 1024)) go(MI_F32_TILE(1, 1, 2, 2, true), grid(32, 32));
+    else if (one_fp32 || (sizeof(TW) == 2 ? per_cu(32, 32) <= 2 : per_cu(32, 32) == 1 || (per_cu(32, 32) > 2 && a.K >= 1024))) go(MI_F32_TILE(1, 1, 2, 2, true), grid(32, 32));
     else go(MI_F32_TILE(1, 1, 2, 2, one_fp32), grid(32, 32));
 #undef MI_F32_TILE
     return check_launch();
