@@ -1,6 +1,6 @@
 // The 256 x 256 x 64 tile GEMM with one wave per SIMD on v_mfma_f32_16x16x32_bf16: the product kernel for the
-// compute-bound shapes.  Included by gemm_tile.hip (TileArgs, TEPI_*, namespace mi).  Schedule, feed and persistence
-// are those of gemm_w4_kernel.hpp (read its header first); what differs is the MFMA shape and what follows from it.
+// compute-bound shapes.  Included by gemm_tile.hip and gemm_any_tile.hip (TileArgs, TEPI_*, namespace mi).  Feed (LDS-DMA pieces from 32-bit
+// offsets) and persistence are those of gemm_w4_kernel.hpp (read its header first); the MFMA shape and the schedule of a K step are its own.
 //
 // Why 16 x 16 x 32.  The chip is power-limited under this load, and the accumulator traffic of a 32 x 32 x 16 MFMA is
 // twice that of a 16 x 16 x 32 per flop (16 + 16 instead of 4 + 4 registers per 32 768 / 16 384 flops): the same loop
@@ -17,6 +17,10 @@
 //     wait for the NEXT image - issued a whole step ago: a counted wait, this step's pieces stay in flight - and a second
 //     barrier, and the sixteen reads of its k half 0 in the last quarter.  A piece has 0.95 of a step; with one barrier in
 //     the middle and the reads spread over both halves it had 0.5, and a step took 3450 cycles (4600 with cold weights).
+//     Whole launches, cycles a step with the epilogue and clock (profiles/gemm_clock.txt): cold weights 16384 x 4096 x 1024 3080 at 1894 MHz -> 2949 at
+//     1853, x 1024 x 3072 5185 at 2279 -> 4065 at 2141, 8192 x 8192 x 8192 3331 at 2172 -> 2683 at 1920: fewer stalls at a lower clock.  Where everything
+//     comes from the caches - one product over and over - nothing stalled before either, and 16384 x 2048 x 2048 takes 110 us for 106, 8192 x 4608 x 3584 229
+//     for 222; with cold weights 117 for 123 and 241 for 242.
 //     us per launch, weights and activations not in the L2s, before -> now: 16384 x 1024 x 2048 88 -> 70, x 3072 121 -> 89,
 //     16384 x 4096 x 1024 139 -> 118, fp32 results 8192 x 2048 x 2048 74 -> 67, 8192 x 8192 x 2048 252 -> 238.  Pieces one
 //     behind every 2 / 3 / 5 MFMAs: 94 / 83 / 100 us where every fourth takes 89 (the L1 feeds 64 bytes a cycle: 8 MFMAs
@@ -434,7 +438,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w16_kernel(const ARGS a) {
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < 16; ++q) read1(0, q);
-  // V & 4096 (measurement; read with tools/gemm_clock.py, numbers in profiles/r04_gemm_clock.txt): shader cycles and 100 MHz reference ticks of the whole tile loop of
+  // V & 4096 (measurement; numbers in profiles/gemm_clock.txt): shader cycles and 100 MHz reference ticks of the whole tile loop of
   // every workgroup, written over the first output bytes when everything else is done
   unsigned long long clk0 = 0, ref0 = 0;
   if (V & 4096) {

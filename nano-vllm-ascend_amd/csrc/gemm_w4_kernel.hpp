@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const TileArgs a) {
     }
   };
   read_first_groups();
-  // V & 4096 (measurement; read with tools/gemm_clock.py, numbers in profiles/r04_gemm_clock.txt): shader cycles and 100 MHz reference ticks of the whole tile loop of
+  // V & 4096 (measurement; numbers in profiles/r04_gemm_clock.txt): shader cycles and 100 MHz reference ticks of the whole tile loop of
   // every workgroup, written over the first output bytes when everything else is done
   unsigned long long clk0 = 0, ref0 = 0;
   if (V & 4096) {

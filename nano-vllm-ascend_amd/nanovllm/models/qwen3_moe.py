@@ -65,6 +65,7 @@ class Qwen3MoeSparseMoeBlock(nn.Module):
         return self.gate_up_stacked
 
     def pack(self) -> None:
+        # (after every change of a weight, as for the linear layers: small steps read the packed copies, large ones the stored weights)
         # nn.Module.to() may have re-created the buffers: the experts' parameters must alias them again
         for e, ex in enumerate(self.experts):
             if ex.gate_up_proj.weight.data_ptr() != self.gate_up_stacked[e].data_ptr():

@@ -997,7 +997,8 @@ def moe_forward(x, router_logits, gate_up_packed, down_packed, top_k: int, all_r
     """Qwen3MoeSparseMoeBlock.forward (qwen3_moe.py:150-185) behind the router GEMM: route -> group the pairs by
     expert -> grouped gate_up+SwiGLU -> grouped down (-> all-reduce of the ranks' partial sums) -> combine.
     x [T, H], router_logits [T, E] bf16; returns [T, H] bf16.  gate_up, down: the weights as they are stored, which steps of many
-    pairs are multiplied from (mi_moe_tiles)."""
+    pairs are multiplied from (mi_moe_tiles: from 16 pairs an expert on; one chain of sums over K, where the packed form adds up its waves'
+    chains, so a row's last bits depend on which of the two its step takes)."""
     require_gpu(x, router_logits, gate_up_packed, down_packed)
     _bf16(x, router_logits, gate_up_packed, down_packed)
     assert x.is_contiguous() and router_logits.is_contiguous()
@@ -1015,13 +1016,14 @@ def moe_forward(x, router_logits, gate_up_packed, down_packed, top_k: int, all_r
     pair_token = offsets + 4 * (E + 1)
     pair_index = pair_token + 4 * pairs
     check(lib.mi_moe_sort(ptr(ids), T, top_k, E, offsets, pair_token, pair_index, st), "mi_moe_sort")
-    n = lib.mi_moe_tiles_bytes(pairs, E, inter, H) if gate_up is not None and down is not None and T else 0
+    stored = gate_up is not None and down is not None and T > 0 and gate_up.is_contiguous() and down.is_contiguous()
+    n = lib.mi_moe_tiles_bytes(pairs, E, inter, H) if stored else 0
     act = torch.empty(pairs * inter + n // 2, dtype=_BF16, device=dev)   # (behind the pairs' activations: the tiles' table)
     y = torch.empty((pairs, H), dtype=_BF16, device=dev)  # row t * top_k + j: the same on every TP rank
     if n and not (x.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16:
         require_gpu(gate_up, down)
         _bf16(gate_up, down)
-        assert gate_up.shape == gate_up_packed.shape and down.shape == down_packed.shape and gate_up.is_contiguous() and down.is_contiguous()
+        assert gate_up.shape == gate_up_packed.shape and down.shape == down_packed.shape
         check(lib.mi_moe_tiles(ptr(x), T, ptr(gate_up), ptr(down), offsets, pair_token, pair_index, ptr(act), ptr(y), pairs, E, H, inter,
                                ptr(act) + pairs * inter * 2, n, st), "mi_moe_tiles")
     else:
