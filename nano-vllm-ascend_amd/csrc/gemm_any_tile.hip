@@ -184,6 +184,30 @@ static bool few_pairs(int64_t pairs, int N, int K, int64_t G) {
   return G * pairs * (N + K) <= (narrow ? 22000 : (int64_t)N * K <= (256 << 10) ? 12800 : 10240) * (G + pairs);
 }
 
+// us of a grouped product on tiles of t rows (64, 128, 256): a CU's share of the tiles, each its K steps and what lies around them, for one tile
+// alone on a CU and for several (up to 64 outputs a tile of 64 rows and, of two weights, of 128; else as many as rows, of two weights half).  Fitted to 300
+// drawn products from cold weights - 4 to 128 groups of 90 to 2200 rows, shares uneven by a third, 64 to 2112 outputs, K 64 to 4224 - which the choice by it
+// misses the best tile's time of by 1.3 % in the mean (26 at worst, two products); by lines in rows per group and tiles, before, 5.2 % (60): 64 groups of 276
+// rows, two weights of 320 x 192 35 us for 22, 16 of 1974, 256 x 384 and back 67 for 52, 32 of 145, 1664 x 3456 and back 442 for 367.  1.1: over another 1588
+// products of 24 to 112 rows the larger tile was the better one where the two are near (1.6 % missed in the mean with it, 1.8 without, 2.5 by the lines).
+static double grouped_us(int t, int rows, int N, int K, int G, bool dual) {
+  const int f = t == 64 || !dual ? t : t / 2;
+  const int64_t row_tiles = rows / t + G / 2, tiles = (row_tiles < G ? G : row_tiles) * ((N + f - 1) / f), c = (tiles + 255) / 256;
+  const double kt = K / BK;
+  if (t == 64) return 1.1 * (dual ? (c == 1 ? 0.63 * kt + 2.5 : c * (0.49 * kt + 1.25)) : (c == 1 ? 0.38 * kt + 2.6 : c * (0.28 * kt + 1.3)));
+  if (t == 128) return dual ? (c == 1 ? 0.83 * kt + 4.7 : c * (0.75 * kt + 2.35)) : (c == 1 ? 0.77 * kt + 6.6 : c * (0.77 * kt + 3.3));
+  return c * (dual ? 1.67 * kt + 10.2 : 1.6 * kt + 11.3);
+}
+// the cheapest tile by us(t); 256-row ones not for groups of less than half a tile, whose cold weights they wait for (128 of 256 x 1024, 96 rows: 100 us, 68 and 77
+// with the smaller ones)
+template <class F>
+static int cheapest_tile(int rows, int n_groups, F us) {
+  int best = 64;
+  if (us(128) < us(best)) best = 128;
+  if (rows >= 128 * (int64_t)n_groups && us(256) < us(best)) best = 256;
+  return best;
+}
+
 // 0: not taken; else the rows of a tile (256: the persistent kernel, 128 and 64: the small-tile kernel).  pays: only where it is not slower
 // than the general kernels
 static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int act, bool pays = true) {
@@ -204,30 +228,20 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
                    (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
     return 0;
   if (n_groups && act == MI_ACT_SOFTCAP) return 0;   // (no group has one)
-  // 64-row tiles while they are few or a group's rows fewer than a larger tile's padding would be; the persistent kernel's 256-row ones where
-  // 128-row ones are more than the chip holds (two workgroups per CU) and not mostly padding.
-  const auto tiles = [=](int t, int f) { return (int64_t)((n_groups ? rows / t + n_groups / 2 : (rows + t - 1) / t)) * ((N + f - 1) / f); };
-  if (n_groups) {
-    // us of both products from cold weights, 64- / 128- / 256-row tiles, uneven groups of this mean: 32 experts of 512 x 1024, 48 rows 33 / 35 / 50,
-    // 96 43 / 40 / 50, 192 52 / 43 / 52, 256 62 / 67 / 52, 512 105 / 103 / 97; 64 of 768 x 2048, 48 134 / 150 / 170, 64 149 / 156 / 172, 96 179 / 161 /
-    // 192, 128 213 / 194 / 199, 192 272 / 257 / 209, 512 607 / 506 / 377; 8 of 512 x 1024, 96 18 / 27 / 47, 256 27 / 28 / 49, 512 41 / 38 / 50;
-    // 128 of 256 x 1024, 48 56 / 70 / 67, 96 68 / 77 / 100, 160 97 / 93 / 103, 192 110 / 105 / 105, 256 138 / 132 / 108
-    // One product, K 512 to 4096, time of 128- by 64-row tiles at 64 to 88 rows: two weights 128 of 384 0.97 .. 1.06, 64 of 768 0.92 .. 1.07 (below 1 from
-    // K 3072 on), 64 of 512 1.11 .. 1.28, 96 of 640 0.88 .. 1.14, 48 of 1024 0.95 .. 1.05; one weight 0.82 .. 1.05, 64 of 512 0.93 .. 1.16, 96 of 640 with 88 rows 1.16 ..
-    // 1.25: within a tenth of the line either is right, for how the tiles fill the CUs.  Few of two weights: 128-row tiles where they are one per CU and
-    // groups of more than 64 rows make 64-row ones more than that (32 of 512 x 4096, 48 rows 118 / 99; 16 of 1024 x 2048 76 / 67, 24 of 640 x 1024 0.93 of the time).
-    // (K below 512 was not measured: no more than the padding's rule there)
-    if (rows < (dual ? K >= 2048 ? 64 : 88 : 72) * (int64_t)n_groups || (K >= 512 && tiles(64, 64) < 512)) {
-      const bool one_per_cu = dual && K >= 512 && n_groups * (int64_t)((N + 63) / 64) <= 256 && tiles(64, 64) > 256 && tiles(64, 64) <= 360;
-      return one_per_cu ? 128 : 64;
-    }
-    return rows >= 160 * (int64_t)n_groups && tiles(128, dual ? 64 : 128) > 512 ? 256 : 128;
-  }
+  if (n_groups) return cheapest_tile(rows, n_groups, [=](int t) { return grouped_us(t, rows, N, K, n_groups, dual); });
+  // 64-row tiles while they are few; the persistent kernel's 256-row ones where 128-row ones are more than the chip holds (two workgroups per CU).
+  const auto tiles = [=](int t, int f) { return (int64_t)((rows + t - 1) / t) * ((N + f - 1) / f); };
   // us, cold weights, 64- / 128- / 256-row tiles: 2000 x 1024 x 1024 (512 / 128 / 32 tiles) 12 / 16 / 26, 2000 x 2048 x 1024 (1024 / 256 / 64) 23 / 18 / 28,
   // 4000 x 2048 x 1024 (2016 / 512 / 128) 33 / 27 / 30, 3000 x 3072 x 1024 (2256 / 576 / 144) 41 / 37 / 31; 1000 x 2048 x 2048 (512 / 128 / 32) 22 / 26 / 47,
   // 1300 (672 / 176 / 48) 29 / 27 / 44, 4000 (2016 / 512 / 128) 53 / 42 / 48, 1300 x 6144 x 2048 (2016 / 528 / 144) 76 / 61 / 46
   if (tiles(64, 64) <= 512) return 64;
   return act != MI_ACT_SOFTCAP && tiles(128, dual ? 64 : 128) > 512 ? 256 : 128;
+}
+
+// ... of experts' two products, which share one table of tiles
+static int pair_tile_rows(int pairs, int G, int ff, int width, bool dual, int act, bool pays) {
+  if (!tile_rows_for(pairs, ff, width, G, dual, act, pays) || !tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE, pays)) return 0;
+  return cheapest_tile(pairs, G, [=](int t) { return grouped_us(t, pairs, ff, width, G, dual) + grouped_us(t, pairs, width, ff, G, false); });
 }
 
 template <int ACT, bool DUAL, bool GATHER, bool HALF>
@@ -395,8 +409,7 @@ static int moe_tile_rows(int pairs, int G, int ff, int width) {
   if (pairs < 1 || G < 1 || width % BK || ff % BK || width % 8 || ff % 8) return 0;
   if (2 * (int64_t)ff > INT32_MAX || ((int64_t)G * 2 * ff + 256) * width * 2 >= (int64_t)1 << 31) return 0;   // (32-bit offsets into gate_up)
   if (pairs < 16 * (int64_t)G || (int64_t)pairs * (ff + width) < 800000) return 0;
-  const int a = tile_rows_for(pairs, ff, width, G, true, MI_ACT_SILU, false), b = tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE, false);
-  return a < b ? a : b;
+  return pair_tile_rows(pairs, G, ff, width, true, MI_ACT_SILU, false);
 }
 extern "C" int64_t mi_moe_tiles_bytes(int pairs, int n_experts, int inter, int hidden) {
   const int t = moe_tile_rows(pairs, n_experts, inter, hidden);
@@ -431,8 +444,7 @@ extern "C" int mi_moe_tiles(const mi_bf16* x, int n_tokens, const mi_bf16* gate_
 // scratch of mi_expert_ff: the gathered operand, the inner activations, the tile table (each rounded up to 16 bytes) - or, streamed, the
 // inner activations in fp32
 static int expert_tile_rows(int pairs, int G, int ff, int width, bool dual, int act) {
-  const int a = tile_rows_for(pairs, ff, width, G, dual, act), b = tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE);
-  return a < b ? a : b;
+  return pair_tile_rows(pairs, G, ff, width, dual, act, true);
 }
 static int64_t round16(int64_t bytes) { return (bytes + 15) & ~(int64_t)15; }
 

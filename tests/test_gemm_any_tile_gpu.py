@@ -165,7 +165,8 @@ def test_more_tiles_than_the_chip_holds(tile, G, N, K, dual, rows):
 
 @pytest.mark.parametrize("rows,N,K,G,dual,want", [(65536, 768, 2048, 64, True, 256), (65536, 2048, 768, 64, False, 256), (1024, 2048, 768, 64, False, 64),
                                                   (256, 2048, 768, 64, False, 64), (8192, 2048, 2048, 0, False, 256), (2048, 768, 2048, 32, True, 128),
-                                                  (1536, 512, 4096, 32, True, 128), (1536, 512, 4096, 32, False, 64), (1280, 512, 2048, 20, True, 64)])
+                                                  (1536, 512, 4096, 32, True, 128), (1536, 512, 4096, 32, False, 64), (1280, 512, 2048, 20, True, 64),
+                                                  (31580, 384, 256, 16, False, 128), (4660, 1664, 3456, 32, True, 256), (17664, 320, 192, 64, True, 128)])
 def test_rule_reaches_the_large_forms(rows, N, K, G, dual, want):
     assert _C.lib.mi_gemm_any_tile_rows(rows, N, K, G, int(dual), _C.ACT_SILU if dual else _C.ACT_NONE) == want
 
