@@ -187,7 +187,7 @@ static bool few_pairs(int64_t pairs, int N, int K, int64_t G) {
 // us of a grouped product on tiles of t rows (64, 128, 256): a CU's share of the tiles, each its K steps and what lies around them, for one tile
 // alone on a CU and for several (up to 64 outputs a tile of 64 rows and, of two weights, of 128; else as many as rows, of two weights half).  Fitted to 300
 // drawn products from cold weights - 4 to 128 groups of 90 to 2200 rows, shares uneven by a third, 64 to 2112 outputs, K 64 to 4224 - which the choice by it
-// misses the best tile's time of by 1.3 % in the mean (26 at worst, two products); by lines in rows per group and tiles, before, 5.2 % (60): 64 groups of 276
+// misses the best tile's time of by 1.2 % in the mean from K 512 on, 3.7 over all with the line below; by lines in rows per group and tiles, before, 5.2: 64 groups of 276
 // rows, two weights of 320 x 192 35 us for 22, 16 of 1974, 256 x 384 and back 67 for 52, 32 of 145, 1664 x 3456 and back 442 for 367.  1.1: over another 1588
 // products of 24 to 112 rows the larger tile was the better one where the two are near (1.6 % missed in the mean with it, 1.8 without, 2.5 by the lines).
 static double grouped_us(int t, int rows, int N, int K, int G, bool dual) {
@@ -198,12 +198,15 @@ static double grouped_us(int t, int rows, int N, int K, int G, bool dual) {
   if (t == 128) return dual ? (c == 1 ? 0.83 * kt + 4.7 : c * (0.75 * kt + 2.35)) : (c == 1 ? 0.77 * kt + 6.6 : c * (0.77 * kt + 3.3));
   return c * (dual ? 1.67 * kt + 10.2 : 1.6 * kt + 11.3);
 }
+// K below 512, -1, 0, 1 (not, by the cost, yes): 64-row tiles where a larger one would be mostly padding, and only there.  A line that leaves time: 8 groups of 122
+// rows, 384 x 256 11.6 us for 7.6, 8 of 397, 448 x 256 11.8 for 9.2.
+static int short_k_64(int rows, int K, int G, bool dual) { return K >= 512 ? 0 : rows < (dual ? 88 : 72) * (int64_t)G ? 1 : -1; }
 // the cheapest tile by us(t); 256-row ones not for groups of less than half a tile, whose cold weights they wait for (128 of 256 x 1024, 96 rows: 100 us, 68 and 77
 // with the smaller ones)
 template <class F>
-static int cheapest_tile(int rows, int n_groups, F us) {
-  int best = 64;
-  if (us(128) < us(best)) best = 128;
+static int cheapest_tile(int rows, int n_groups, int take_64, F us) {
+  if (take_64 > 0) return 64;
+  int best = take_64 < 0 || us(128) < us(64) ? 128 : 64;
   if (rows >= 128 * (int64_t)n_groups && us(256) < us(best)) best = 256;
   return best;
 }
@@ -228,7 +231,8 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
                    (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
     return 0;
   if (n_groups && act == MI_ACT_SOFTCAP) return 0;   // (no group has one)
-  if (n_groups) return cheapest_tile(rows, n_groups, [=](int t) { return grouped_us(t, rows, N, K, n_groups, dual); });
+  if (n_groups)
+    return cheapest_tile(rows, n_groups, short_k_64(rows, K, n_groups, dual), [=](int t) { return grouped_us(t, rows, N, K, n_groups, dual); });
   // 64-row tiles while they are few; the persistent kernel's 256-row ones where 128-row ones are more than the chip holds (two workgroups per CU).
   const auto tiles = [=](int t, int f) { return (int64_t)((rows + t - 1) / t) * ((N + f - 1) / f); };
   // us, cold weights, 64- / 128- / 256-row tiles: 2000 x 1024 x 1024 (512 / 128 / 32 tiles) 12 / 16 / 26, 2000 x 2048 x 1024 (1024 / 256 / 64) 23 / 18 / 28,
@@ -241,7 +245,9 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
 // ... of experts' two products, which share one table of tiles
 static int pair_tile_rows(int pairs, int G, int ff, int width, bool dual, int act, bool pays) {
   if (!tile_rows_for(pairs, ff, width, G, dual, act, pays) || !tile_rows_for(pairs, width, ff, G, false, MI_ACT_NONE, pays)) return 0;
-  return cheapest_tile(pairs, G, [=](int t) { return grouped_us(t, pairs, ff, width, G, dual) + grouped_us(t, pairs, width, ff, G, false); });
+  const int a = short_k_64(pairs, width, G, dual), b = short_k_64(pairs, ff, G, false);
+  return cheapest_tile(pairs, G, a > 0 || b > 0 ? 1 : a < b ? a : b,
+                       [=](int t) { return grouped_us(t, pairs, ff, width, G, dual) + grouped_us(t, pairs, width, ff, G, false); });
 }
 
 template <int ACT, bool DUAL, bool GATHER, bool HALF>
