@@ -3,12 +3,17 @@
 // The same GEMM on 128 x 128 tiles, for shapes whose 256 x 256 tiles cannot fill the chip (64 < M <= ~2048 rows:
 // large decode batches, short prompts).  Four waves, each 64 features x 64 tokens (2 x 2 accumulators); one K step of
 // the tile is two 16 KiB half-tiles in the layout of gemm_tile_index.hpp (A: local row = tile feature row, B: local
-// row = tile token row) in a ring of NST stages.  One barrier per K step: "my pieces of step t have landed" (a COUNTED
-// wait: the pieces of the NST - 2 steps behind it may still fly) -> barrier (everybody's have, and everybody is done
-// reading step t - 1) -> request step t + NST - 1 into the buffer step t - 1 used -> fragments of step t -> sixteen
-// MFMAs.  These shapes have at most a workgroup or two per CU and a K loop of 16-80 steps: with one step of
-// prefetch (NST = 2, two workgroups per CU) every step waits out most of a DMA round trip (0.75 us per step
-// measured); NST = 4 (128 KiB, one workgroup per CU) keeps three steps in flight.
+// row = tile token row) in a ring of NST stages.  One barrier per K step: "my pieces of step t + 1 have landed" (a COUNTED wait: the
+// pieces of the NST - 2 steps behind it may still fly) and "I have read step t" -> barrier -> step t's matrix instructions, and behind each of
+// them two fragment reads of step t + 1 and one request of step t + NST, into the slot of step t.
+// What bounds it: with a tile or two per CU nothing else stands beside a wave's own waits, so a step must not have its requests, its reads
+// and its matrix instructions one after the other (the reads of a 128 x 128 tile's step take a CU's LDS 512 cycles, its requests the
+// address path about as long, its matrix instructions 512).  us per step of 64, 128 x 128 tiles, ring of four: two tiles 0.53 with the three one
+// after the other, 0.45 with the reads a step ahead, 0.28 so; 224 tiles 0.54 / 0.46 / 0.40: now the L2s' rate, 32 KiB per tile and step = 17.5
+// TB/s (64 x 64: 256 tiles 0.25 -> 0.16, 25 TB/s).  Launches (cold weights): 137 x 4096 x 1024 7.0 -> 6.3 us, 500 x 1024 x 2048 10.3 -> 7.7, 886 x 4096
+// x 1024 15.0 -> 13.4, 2450 x 1024 x 3072 31.9 -> 25.5, with SwiGLU 500 x 6144 x 1024 14.7 -> 13.2.
+// A ring of two steps still leaves a step's pieces one step's time to arrive (two tiles share the CU then); four (128 KiB, one tile per CU)
+// keep three steps in flight.
 // Same summation order and epilogues as the large kernel: results are bit-identical.
 // SwiGLU: the tile's 128 weight rows are, per wave, 32 gate rows (fragment 0) and the 32 up rows that pair with them.
 // ---------------------------------------------------------------------------
@@ -17,13 +22,17 @@
 template <int N, int PER_STEP>
 __device__ __forceinline__ void mid_wait(int behind) {  // all but the pieces of the `behind` (<= N) newest K steps have landed
   if constexpr (N == 0) {
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   } else {
-    if (behind >= N) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N * PER_STEP) : "memory");
+    if (behind >= N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N * PER_STEP) : "memory");
     else mid_wait<N - 1, PER_STEP>(behind);
   }
 }
 
+// one piece: a lane's 16 bytes at byte `off` (its own) + k (the wave's) of the operand to dst + 16 lane
+__device__ __forceinline__ void mid_piece(const __amdgpu_buffer_rsrc_t r, char* dst, uint32_t off, uint32_t k) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, k, 0, 0);
+}
 template <int EPI, bool BIAS, int NST, class ARGS = TileArgs, class SH = Mid128>
 __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void gemm_mid_kernel(const ARGS a) {
   constexpr int WF = SH::WF, WT = SH::WT;
@@ -34,7 +43,7 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
   const int fw = wave / SH::TW, tw = wave % SH::TW, hi = lane >> 5, l31 = lane & 31;
   const int KT_all = a.K / BK;
   const int KT = EPI == TEPI_PARTIAL ? KT_all / (int)gridDim.y : KT_all;
-  const int64_t kbeg_bytes = EPI == TEPI_PARTIAL ? (int64_t)blockIdx.y * KT * (BK * 2) : 0;
+  const uint32_t k0 = EPI == TEPI_PARTIAL ? blockIdx.y * (uint32_t)KT * (BK * 2) : 0;  // bytes of a row in front of this slice of K
   int n0 = ((int)blockIdx.x % a.tiles_f) * SH::F, m0 = ((int)blockIdx.x / a.tiles_f) * SH::T, m_end = a.M;
   int64_t wrow0 = 0;
   if constexpr (EPI == TEPI_ANY) {
@@ -44,21 +53,24 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
     n0 = t.n0, m0 = t.m0, m_end = t.m_end, wrow0 = (int64_t)t.group * a.w_rows;
   }
 
-  // LDS-DMA: wave w moves its share of the 1 KiB pieces (8 local rows each) of the feature rows and of the token rows
-  const char* srcA[SH::A_PIECES];
-  const char* srcB[SH::B_PIECES];
+  // LDS-DMA: wave w moves its share of the 1 KiB pieces (8 local rows each) of the feature rows and of the token rows.  A piece's source is a 32-bit
+  // offset per lane from the operand's base (the entry points refuse operands beyond 2 GiB) and the K step on the scalar unit.
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.w), 0, 0x80000000u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.x), 0, 0x80000000u, 0x00020000);
+  const uint16_t* w2 = a.w;
+  if constexpr (ARGS::kDual) w2 = a.w2;
+  const __amdgpu_buffer_rsrc_t w2_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w2), 0, 0x80000000u, 0x00020000);
+  uint32_t offA[SH::A_PIECES], offB[SH::B_PIECES];
 #pragma unroll
   for (int i = 0; i < SH::A_PIECES; ++i) {
     const int lr = (wave * SH::A_PIECES + i) * 8 + (lane >> 3), c = (lane & 7) ^ swizzle(lr);
-    if constexpr (EPI == TEPI_ANY) {
+    int64_t rowA = 0;
+    if constexpr (EPI == TEPI_ANY)
       // two weights: every wave's first fragment holds 32 rows of w, its second the rows of w2 that pair with them
-      const bool second = ARGS::kDual && ((lr >> 5) & 1);
-      const int rowA = ARGS::kDual ? n0 + (lr >> 6) * 32 + (lr & 31) : n0 + lr;
-      srcA[i] = reinterpret_cast<const char*>(second ? a.w2 : a.w) + ((wrow0 + min(rowA, a.N - 1)) * a.K + c * 8) * 2;
-    } else {
-      const int rowA = mid_weight_row(lr, n0, a.N, EPI == TEPI_SILU);
-      srcA[i] = reinterpret_cast<const char*>(a.w) + kbeg_bytes + ((int64_t)min(rowA, a.N - 1) * a.K + c * 8) * 2;
-    }
+      rowA = wrow0 + min(ARGS::kDual ? n0 + (lr >> 6) * 32 + (lr & 31) : n0 + lr, a.N - 1);
+    else
+      rowA = min(mid_weight_row(lr, n0, a.N, EPI == TEPI_SILU), a.N - 1);
+    offA[i] = (uint32_t)((rowA * a.K + c * 8) * 2);
   }
 #pragma unroll
   for (int i = 0; i < SH::B_PIECES; ++i) {
@@ -66,19 +78,29 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
     int64_t rowB = min(m0 + lr, m_end - 1);
     if constexpr (EPI == TEPI_ANY)
       if (ARGS::kGather) rowB = a.x_rows[rowB];
-    srcB[i] = reinterpret_cast<const char*>(a.x) + kbeg_bytes + (rowB * a.ldx + c * 8) * 2;
+    offB[i] = (uint32_t)((rowB * a.ldx + c * 8) * 2);
   }
-  auto issue = [&](int kt, int p) __attribute__((always_inline)) {
-    char* dst = lds + p * SH::STAGE;
-#pragma unroll
-    for (int i = 0; i < (SH::A_PIECES > SH::B_PIECES ? SH::A_PIECES : SH::B_PIECES); ++i) {
-      if (i < SH::A_PIECES)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcA[i < SH::A_PIECES ? i : 0] + (int64_t)kt * (BK * 2)),
-                                         (__attribute__((address_space(3))) void*)(dst + (wave * SH::A_PIECES + i) * 1024), 16, 0, 0);
-      if (i < SH::B_PIECES)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(srcB[i < SH::B_PIECES ? i : 0] + (int64_t)kt * (BK * 2)),
-                                         (__attribute__((address_space(3))) void*)(dst + SH::F * 128 + (wave * SH::B_PIECES + i) * 1024), 16, 0, 0);
+  constexpr int PIECES = SH::A_PIECES + SH::B_PIECES;
+  auto piece = [&](int kt, int p, int i) __attribute__((always_inline)) {  // the i-th of this wave's pieces of step kt, into ring slot p
+    const uint32_t k = k0 + (uint32_t)kt * (BK * 2);
+    char* const image = lds + p * SH::STAGE;
+    if (i < SH::A_PIECES) {
+      const int q = wave * SH::A_PIECES + i;
+      const uint32_t off = offA[i < SH::A_PIECES ? i : 0];
+      if constexpr (EPI == TEPI_ANY && ARGS::kDual)
+        if ((q >> 2) & 1) {
+          mid_piece(w2_rsrc, image + q * 1024, off, k);
+          return;
+        }
+      mid_piece(w_rsrc, image + q * 1024, off, k);
+    } else {
+      const int q = wave * SH::B_PIECES + i - SH::A_PIECES;
+      mid_piece(x_rsrc, image + SH::F * 128 + q * 1024, offB[i < SH::A_PIECES ? 0 : i - SH::A_PIECES], k);
     }
+  };
+  auto issue = [&](int kt, int p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) piece(kt, p, i);
   };
   int kx[4];
 #pragma unroll
@@ -94,33 +116,74 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
       for (int r = 0; r < 16; ++r) acc[f][b][r] = 0.f;
 
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
+  for (int s = 0; s < NST; ++s)
     if (s < KT) issue(s, s);
-  int p = 0, pn = NST - 1;  // ring slots of step kt and of step kt + NST - 1
-  for (int kt = 0; kt < KT; ++kt) {
-    // requested so far: steps <= kt + NST - 2; the same number of pieces per step and wave, completing in order
-    mid_wait<NST - 2, SH::A_PIECES + SH::B_PIECES>(min(KT - 1 - kt, NST - 2));
-    __builtin_amdgcn_sched_barrier(0);
-    if (kt + NST - 1 < KT) issue(kt + NST - 1, pn);
-    const char* sa = lds + p * SH::STAGE + fw * WF * 4096;
-    const char* sb = lds + p * SH::STAGE + SH::F * 128 + tw * WT * 4096;
+  struct Frags {
     u32x4 A[WF][4], B[WT][4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-#pragma unroll
-      for (int f = 0; f < WF; ++f) A[f][kk] = *reinterpret_cast<const u32x4*>(sa + f * 4096 + kx[kk]);
-#pragma unroll
-      for (int b = 0; b < WT; ++b) B[b][kk] = *reinterpret_cast<const u32x4*>(sb + b * 4096 + kx[kk]);
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int f = 0; f < WF; ++f)
-#pragma unroll
-        for (int b = 0; b < WT; ++b)
-          acc[f][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(A[f][kk]), as_frag(B[b][kk]), acc[f][b], 0, 0, 0);
+  } fa, fb;
+  constexpr int READS = 4 * (WF + WT), MULS = 4 * WF * WT;
+  auto read = [&](int p, int i, Frags& f) __attribute__((always_inline)) {  // the i-th fragment of the step in ring slot p, k ascending
+    const int kk = i / (WF + WT), r = i % (WF + WT);
+    if (r < WF) f.A[r < WF ? r : 0][kk] = *reinterpret_cast<const u32x4*>(lds + p * SH::STAGE + (fw * WF + r) * 4096 + kx[kk]);
+    else f.B[r < WF ? 0 : r - WF][kk] = *reinterpret_cast<const u32x4*>(lds + p * SH::STAGE + SH::F * 128 + (tw * WT + r - WF) * 4096 + kx[kk]);
+  };
+  auto multiply = [&](int i, const Frags& f) __attribute__((always_inline)) {  // the i-th matrix instruction of a step, k ascending
+    const int kk = i / (WF * WT), u = i / WT % WF, b = i % WT;
+    acc[u][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(f.A[u][kk]), as_frag(f.B[b][kk]), acc[u][b], 0, 0, 0);
+  };
+  int p = 0;  // ring slot of step kt
+  // Step kt, which is not the last one: its fragments are in `cur`; behind its matrix instructions the reads of step kt + 1 into `next` (two each: in
+  // front of the first one it would wait for them) and the requests of step kt + NST, one each (all at once they hold the wave up for as long as its
+  // matrix instructions take) - REST: near the end, where there may be none.
+  auto step = [&](auto rest, int kt, const Frags& cur, Frags& next) __attribute__((always_inline)) {
+    constexpr bool REST = decltype(rest)::value;
+    // requested so far: steps <= kt + NST - 1; the same number of pieces per step and wave, completing in order
+    mid_wait<NST - 2, PIECES>(REST ? min(KT - 2 - kt, NST - 2) : NST - 2);
+    __builtin_amdgcn_sched_barrier(0);
+    const int free = p;  // (everybody has read step kt)
     p = p + 1 == NST ? 0 : p + 1;
-    pn = pn + 1 == NST ? 0 : pn + 1;
+    if (REST && kt + NST < KT) issue(kt + NST, free);
+    constexpr int RD = MULS < READS ? (READS + MULS / 2 - 1) / (MULS / 2) : 2, DM = (PIECES + MULS - 1) / MULS;
+#pragma unroll
+    for (int i = 0; i < MULS; ++i) {
+      multiply(i, cur);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+      for (int j = 0; j < RD; ++j)
+        if (i * RD + j < READS) {
+          read(p, i * RD + j, next);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+      if constexpr (!REST)
+#pragma unroll
+        for (int j = 0; j < DM; ++j)
+          if (i * DM + j < PIECES) {
+            piece(kt + NST, free, i * DM + j);
+            __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+          }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  mid_wait<NST - 1, PIECES>(min(KT - 1, NST - 1));
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < READS; ++i) read(0, i, fa);
+  int kt = 0;
+  for (; kt + 1 + NST < KT; kt += 2) {
+    step(std::false_type{}, kt, fa, fb);
+    step(std::false_type{}, kt + 1, fb, fa);
+  }
+  for (; kt + 2 < KT; kt += 2) {
+    step(std::true_type{}, kt, fa, fb);
+    step(std::true_type{}, kt + 1, fb, fa);
+  }
+  if (kt + 1 < KT) {
+    step(std::true_type{}, kt, fa, fb);
+#pragma unroll
+    for (int i = 0; i < MULS; ++i) multiply(i, fb);
+  } else {
+#pragma unroll
+    for (int i = 0; i < MULS; ++i) multiply(i, fa);
   }
 
   // epilogue: lane (hi, l31) holds token (tw WT + b) 32 + l31, features 8 rq + 4 hi + {0..3} of each 32-row fragment
