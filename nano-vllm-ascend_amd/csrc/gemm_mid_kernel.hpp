@@ -33,6 +33,15 @@ __device__ __forceinline__ void mid_wait(int behind) {  // all but the pieces of
 __device__ __forceinline__ void mid_piece(const __amdgpu_buffer_rsrc_t r, char* dst, uint32_t off, uint32_t k) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, k, 0, 0);
 }
+// Block b's tile (its feature tile and its token tile; false: none).  The dispatcher places block b on XCD b % 8 (a speed assumption only): XCD x works on
+// feature run x % 2^lf and token run x >> lf, features fastest, so that its L2 fetches 1 / 2^lf of the weights and 2^lf / 8 of the activations.
+__device__ __forceinline__ bool mid_tile(uint32_t b, uint32_t tiles_f, uint32_t tiles_t, int lf, uint32_t& f, uint32_t& t) {
+  const uint32_t run_f = tiles_f >> lf, n = run_f * tiles_t, each = ((n << lf) + 7) >> 3;
+  const uint32_t i = ((b & 7) >> lf) * each + (b >> 3);
+  t = i / run_f;  // (one division: each is some 40 dependent instructions in front of the first request)
+  f = i - t * run_f + (b & ((1u << lf) - 1)) * run_f;
+  return (b >> 3) < each && i < n;
+}
 template <int EPI, bool BIAS, int NST, class ARGS = TileArgs, class SH = Mid128>
 __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void gemm_mid_kernel(const ARGS a) {
   constexpr int WF = SH::WF, WT = SH::WT;
@@ -44,13 +53,17 @@ __global__ __launch_bounds__(64 * SH::NW, NST * SH::STAGE <= 81920 ? 2 : 1) void
   const int KT_all = a.K / BK;
   const int KT = EPI == TEPI_PARTIAL ? KT_all / (int)gridDim.y : KT_all;
   const uint32_t k0 = EPI == TEPI_PARTIAL ? blockIdx.y * (uint32_t)KT * (BK * 2) : 0;  // bytes of a row in front of this slice of K
-  int n0 = ((int)blockIdx.x % a.tiles_f) * SH::F, m0 = ((int)blockIdx.x / a.tiles_f) * SH::T, m_end = a.M;
+  int n0 = 0, m0 = 0, m_end = a.M;
   int64_t wrow0 = 0;
   if constexpr (EPI == TEPI_ANY) {
     const int ntiles = any_tiles(a);
     if ((int)blockIdx.x >= ntiles) return;  // (the grid is the host's bound on the grouped tiles)
     const AnyTile t = any_tile(a, (int)blockIdx.x, ntiles, SH::T, ARGS::kDual ? SH::F / 2 : SH::F);
     n0 = t.n0, m0 = t.m0, m_end = t.m_end, wrow0 = (int64_t)t.group * a.w_rows;
+  } else {
+    uint32_t f, t;
+    if (!mid_tile(blockIdx.x, a.tiles_f, a.tiles_t, a.xcd_lf, f, t)) return;
+    n0 = f * SH::F, m0 = t * SH::T;
   }
 
   // LDS-DMA: wave w moves its share of the 1 KiB pieces (8 local rows each) of the feature rows and of the token rows.  A piece's source is a 32-bit

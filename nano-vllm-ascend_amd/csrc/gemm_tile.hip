@@ -485,81 +485,99 @@ static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
 }
 
 // ---- which kernel, how many K slices ----
-// The 128-tile kernel takes the shapes whose 256-tiles are too few for the chip; both kernels give the same bits,
-// the choice is a matter of time only.  Modelled time of a launch: rounds of workgroups x K steps x time per step
-// (measured: tools/gemm_bench.py), plus - with K slices - the fp32 partial sums out and back and the second launch.
-// gemm_mid_kernel's shapes (features x tokens): its time per K step with one workgroup on a CU (what the ring's requests take), and for
-// two sharing it.  us, one launch: 200 rows x 4096 features x 1024 with 128 x 128 / 64 x 128 / 64 x 64 tiles 12.5 / 9.3 / 7.1
-// (64 / 128 / 256 workgroups; the weight-streaming kernel 18.6), 400 rows 12.5 / 9.3 / 9.6; 200 x 5120 x 2048 21.2 / 15.8 / 14.5;
-// SwiGLU of 6144 rows x 1024 at 200 tokens 12.7 / 9.4, at 400 12.9 / 12.5; 1024 rows x 1024 features x 3072: 128 x 128 in four K
-// slices 19.8, 64 x 64 14.1.  Beyond 2048 rows the smaller tiles only read the operands more often (4096 rows x 1024 x 2048:
-// 26.4 / 31.2).
-using Mid64x128 = MidShape<1, 4, 2, 1>;   // (a wave holds a gate and an up fragment: SwiGLU too)
-using Mid64 = MidShape<2, 2, 1, 1>;
+// Where the 256-tiles are fewer than the CUs: the shape of tile (gemm_mid_kernel's, or still the large one's) and the number of K slices whose
+// modelled time is the least; all give the same bits but for the slices.  Modelled: a launch, the rounds of its tiles, the K steps of a round - which take
+// the longer the more of the chip's places are in use (the L2s' rate: (F + T) 128 bytes per tile and step) - and with K slices the fp32 partial sums out
+// and back and the second launch.  The constants are fitted to 400 random products with cold weights (65 .. 6000 rows, K from 512 on; 7 to 14 % off
+// in the mean), those of 64 x 64 and 128 x 64 corrected by whole prompt steps, whose activations another kernel has just written (1260 rows, 28 layers, us a
+// step with o on 128 x 64 / 64 x 64 3131 / 3084, down 3131 / 3045); over 380 random products within 1 % of the best shape.  Two-place shapes: rings of which two fit
+// a CU; 128 x 64 and 128 x 128 have a deeper one too, a tile per CU, whose requests reach further ahead.  us, 64 x 64 / 128 x 64 / 128 x 128 / 128 x 192
+// / 256 x 256 (the better ring of each): 137 x 4096 x 1024 6.2 / 8.8 / 10.3 / 13.6 / 24, 500 rows 10.7 / 9.8 / 12.2 / 13.8 / 26, 886 rows
+// 16.2 / 12.9 / 12.8 / 14.4 / 25, 1260 rows 19.1 / 18.8 / 17.9 / 15.8 / 26, 2048 rows 30 / 25 / 22.1 / 28 / 29; 886 x 5120 x 2048 35 / 33 / 32 / 24.8 / 43;
+// 1260 x 1024 x 2048 14.4 / 11.9 / 14.8 / 19.6 / 40, 2450 rows 21.7 / 20.7 / 16.6 / 20.2 / 40.  Against the choice among 64 x 64, 64 x 128, 128 x 128 and
+// 256 x 256 by one time per step each (and that kernel's longer steps), 300 products: 0.85 of the time in the geometric mean.
 struct MidTile {
-  int f, t;
-  double step_us, pair_us;
+  int f, t, places;  // features, tokens; tiles that share a CU
+  double launch_us, round_us, step_us, step_load_us, pair_us, pair_load_us;
 };
-constexpr MidTile kMidTiles[3] = {{128, 128, 0.52, 0.62}, {64, 128, 0.36, 0.56}, {64, 64, 0.22, 0.35}};
+// (a tile's two fragments of features are a gate's and an up's with SwiGLU: 64 x 64 has one only)
+enum { kMid128, kMid128Pairs, kMid128x64Pairs, kMid128x64, kMid128x192, kMid64, kMidTileCount };
+constexpr MidTile kMidTiles[kMidTileCount] = {{128, 128, 1, 2.2, 1.8, 0.32, 0.24, 0., 0.},     {128, 128, 2, 0.7, 1.8, 0.57, 0.27, 0.89, 0.10},
+                                              {128, 64, 2, 3.3, 0., 0.29, 0.18, 0.60, 0.18},  {128, 64, 1, 2.8, 1.4, 0.21, 0.21, 0., 0.},
+                                              {128, 192, 1, 1.7, 3.1, 0.43, 0.29, 0., 0.},     {64, 64, 2, 3.1, 0., 0.14, 0.08, 0.32, 0.12}};
+constexpr MidTile kLargeTile = {256, 256, 1, 3.1, 3.7, 1.04, 0.48, 0., 0.};
 constexpr double kLaunchUs = 3.8, kPartialBytesPerUs = 4.0e6;
 
 // fewer 256-tiles than CUs
 static bool few_tiles(int M, int N) {
   return (int64_t)((M + TILE_T - 1) / TILE_T) * ((N + TILE_F - 1) / TILE_F) < kPersistentGrid;
 }
-// The 128-tile kernel: there, up to two 128-tiles per CU.  More are a second round of its workgroups, and 256-tiles on half of the CUs are
-// done before it (us with cold weights, small tiles / 256-tiles, two per CU: 4024 x 2048 x 1024 26.2 / 31.2, 2000 x 4096 x 4096 76 / 93, 8000 x 1024 x 3072
-// 67 / 71; beyond, before a K step of the 256-tiles was shortened: 4536 x 2048 x 1024 29.9 / 25.1, 3000 x 4096 x 4096 115 / 78); of short K up to three
-// (10240 features x 256: 640 tiles 16.2 / 16.6, 880 19.5 / 16.8; 4096 x 128: 768 14.1 / 14.2, 896 15.5 / 14.6; 1024 x 320: 632 19.1 / 17.9, 816 22.6 / 19.2).
-static bool use_mid(int M, int N, int K) {
-  return few_tiles(M, N) && (int64_t)((M + MID_T - 1) / MID_T) * ((N + MID_F - 1) / MID_F) <= (K < 384 ? 3 : 2) * kPersistentGrid;
-}
-
 struct MidPick {
-  int tile, ksplit;
+  int tile, ksplit;  // tile -1: the large kernel
 };
+// modelled time of `tiles` tiles of kt K steps: whole rounds of all CUs, then what is left, whose steps take the less the fewer they are
+static double tiles_us(const MidTile& s, int64_t tiles, int kt) {
+  const int64_t round = (int64_t)s.places * kPersistentGrid, rest = tiles % round;
+  const auto step = [&](int64_t n) {
+    return s.places == 2 && n > kPersistentGrid ? s.pair_us + s.pair_load_us * (n - kPersistentGrid) / kPersistentGrid
+                                                : s.step_us + s.step_load_us * n / kPersistentGrid;
+  };
+  return s.launch_us + (double)(tiles / round) * (s.round_us + kt * step(round)) + (rest ? s.round_us + kt * step(rest) : 0.);
+}
 // fixed_ks: the caller wants that many slices' sums; 0: whatever is fastest, the sum of the slices included
 static MidPick pick_mid(int M, int N, int K, bool silu, int fixed_ks = 0) {
   const int kt = K / BK;
-  const int shapes = M > 2048 ? 1 : silu ? 2 : 3;
-  double best = 1e30;
-  MidPick pick{0, 1};
-  for (int i = 0; i < shapes; ++i) {
-    const MidTile& s = kMidTiles[i];
-    const int64_t tiles = (int64_t)((M + s.t - 1) / s.t) * ((N + s.f - 1) / s.f);
+  const auto tiles = [&](const MidTile& s) { return (int64_t)((M + s.t - 1) / s.t) * ((N + s.f - 1) / s.f); };
+  MidPick pick{-1, 1};
+  double best = fixed_ks ? 1e30 : tiles_us(kLargeTile, tiles(kLargeTile), kt);
+  for (int i = 0; i < (silu ? kMid64 : kMidTileCount); ++i)
     for (int ks = fixed_ks ? fixed_ks : 1; ks <= (fixed_ks ? fixed_ks : silu ? 1 : 16); ks *= 2) {
       if (!fixed_ks && (kt % ks || (ks > 1 && kt / ks < 2))) break;
-      const int64_t per_cu = (tiles * ks + kPersistentGrid - 1) / kPersistentGrid;
-      double t = (per_cu == 1 ? s.step_us : (per_cu + 1) / 2 * s.pair_us) * (kt / ks) + kLaunchUs;
+      double t = tiles_us(kMidTiles[i], tiles(kMidTiles[i]) * ks, kt / ks);
       if (!fixed_ks && ks > 1) t += 2.0 * ks * (double)M * N * sizeof(float) / kPartialBytesPerUs + kLaunchUs;
       if (t < best) best = t, pick = MidPick{i, ks};
     }
-  }
   return pick;
 }
 
-// NST = 0: by shape and workgroup count.  128 x 128: at most one workgroup per CU - the deep ring (nothing else hides the DMA round
-// trip); more: the two-stage ring, two workgroups per CU (22 vs 27 us on 1024 x 6144 x 1024, 31 vs 34 the other way round on
-// 1024 x 1024 x 3072).  The smaller shapes: rings of which two fit a CU (64 x 64, five stages: 7.1 us above, nine 7.7).
-template <int EPI, bool BIAS, int NST = 0>
-static int launch_mid(TileArgs a, hipStream_t st, MidPick pick = {0, 1}) {
+// mi_gemm_bf16's plan
+static MidPick tile_plan(int M, int N, int K, bool silu) {
+  if (few_tiles(M, N)) return pick_mid(M, N, K, silu);
+  return MidPick{-1, silu ? 1 : tile_ksplit(M, N, K)};
+}
+
+// (log2 of the) runs of features that the XCDs share the tiles in: the fewest rows of both operands into all L2s.  us within a prompt step, eight runs / this:
+// 1842 rows x 1024 features x 2048 and x 3072 21.1 / 19.9 on average, 2450 rows 22.7 / 21.7, 886 rows 13.8 / 13.2; few rows and many features keep
+// eight (137 x 4096 x 1024: eight 7.0, four 6.9, two 7.4, one 7.3; 886 x 6144 x 1024 16.2 / 16.0, one 18.0).
+static int xcd_features(int M, int N, int tiles_f) {
+  const auto rows = [&](int lf) { return ((int64_t)M << lf) + ((int64_t)N << (3 - lf)); };
+  int best = 0;
+  for (int lf = 1; lf <= 3 && tiles_f % (1 << lf) == 0; ++lf)
+    if (rows(lf) < rows(best)) best = lf;
+  return best;
+}
+
+template <int EPI, bool BIAS>
+static int launch_mid(TileArgs a, hipStream_t st, MidPick pick) {
   const MidTile& s = kMidTiles[pick.tile];
   a.tiles_f = (a.N + s.f - 1) / s.f;
   a.tiles_t = (a.M + s.t - 1) / s.t;
-  const dim3 grid(a.tiles_f * a.tiles_t, pick.ksplit);
-  if constexpr (NST != 0) {
-    hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, NST>), grid, dim3(256), 0, st, a);
-  } else {
-    if constexpr (EPI != TEPI_SILU)
-      if (pick.tile == 2) {
-        hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 5, TileArgs, Mid64>), grid, dim3(256), 0, st, a);
-        return check_launch();
-      }
-    if (pick.tile == 1) hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 3, TileArgs, Mid64x128>), grid, dim3(256), 0, st, a);
-    else if ((int64_t)grid.x * grid.y > kPersistentGrid) hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 2>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_mid_kernel<EPI, BIAS, 4>), grid, dim3(256), 0, st, a);
+  a.xcd_lf = xcd_features(a.M, a.N, a.tiles_f);
+  const dim3 grid((a.tiles_f * a.tiles_t + 7) / 8 * 8, pick.ksplit);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a);
+    return check_launch();
+  };
+  switch (pick.tile) {
+    case kMid128: return go(gemm_mid_kernel<EPI, BIAS, 4, TileArgs, Mid128>);
+    case kMid128Pairs: return go(gemm_mid_kernel<EPI, BIAS, 2, TileArgs, Mid128>);
+    case kMid128x64Pairs: return go(gemm_mid_kernel<EPI, BIAS, 3, TileArgs, MidShape<2, 2, 2, 1>>);
+    case kMid128x64: return go(gemm_mid_kernel<EPI, BIAS, 6, TileArgs, MidShape<2, 2, 2, 1>>);
+    case kMid128x192: return go(gemm_mid_kernel<EPI, BIAS, 3, TileArgs, MidShape<2, 2, 2, 3>>);
+    default: break;
   }
-  return check_launch();
+  if constexpr (EPI != TEPI_SILU) return go(gemm_mid_kernel<EPI, BIAS, 5, TileArgs, MidShape<2, 2, 1, 1>>);
+  return MI_EUNSUPPORTED;  // (never picked)
 }
 
 static int check_tile_gemm(const void* x, int64_t ldx, const void* w, const void* bias, const void* y, int64_t ldy,
@@ -591,7 +609,7 @@ extern "C" int64_t mi_gemm_bf16_max_rows(int N, int K, int64_t ldx) {
 
 extern "C" size_t mi_gemm_bf16_workspace(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK || epilogue != 0) return 0;
-  const int ks = use_mid(M, N, K) ? pick_mid(M, N, K, false).ksplit : tile_ksplit(M, N, K);   // (mi_gemm_bf16's own plan)
+  const int ks = tile_plan(M, N, K, false).ksplit;
   return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
 }
 
@@ -602,10 +620,10 @@ extern "C" int mi_gemm_bf16(const mi_bf16* x, int64_t ldx, const mi_bf16* w, con
   if (rc != MI_OK || M == 0) return rc;
   TileArgs a{x, w, bias, y, ldx, ldy, M, N, K, (N + TILE_F - 1) / TILE_F, (M + TILE_T - 1) / TILE_T, nullptr};
   hipStream_t st = S(stream);
-  const bool mid = use_mid(M, N, K);
-  const MidPick pick = mid ? pick_mid(M, N, K, epilogue == 1) : MidPick{0, 1};
+  const MidPick pick = tile_plan(M, N, K, epilogue == 1);
+  const bool mid = pick.tile >= 0;
   if (epilogue == 1) return mid ? launch_mid<TEPI_SILU, false>(a, st, pick) : launch_tile<TEPI_SILU, false>(a, st);
-  const int ks = mid ? pick.ksplit : tile_ksplit(M, N, K);
+  const int ks = pick.ksplit;
   if (ks > 1) {  // two launches: K slices as fp32 partial sums, then their sum (+ bias) rounded once
     if (!workspace || !aligned16(workspace) || ws_bytes < (size_t)ks * M * N * sizeof(float)) return MI_EWORKSPACE;
     a.part = static_cast<float*>(workspace);
@@ -679,9 +697,13 @@ extern "C" int mi_gemm_bf16_ex(const mi_bf16* x, int64_t ldx, const mi_bf16* w, 
     case kEightWaves + 2: return launch_tile<TEPI_NONE, false, kEightWaves + 2>(a, st);
     case kEightWaves + 16: return launch_tile<TEPI_NONE, false, kEightWaves + 16>(a, st);
     case kEightWaves + 8192: return launch_tile<TEPI_NONE, false, kEightWaves + 8192>(a, st);
-    case 65536: return launch_mid<TEPI_NONE, false, 4>(a, st);  // the 128-tile kernel, no K slices, four-stage ring
-    case 65538: return launch_mid<TEPI_NONE, false, 2>(a, st);  // ... with a two-stage ring, two workgroups per CU
-    case 65539: return launch_mid<TEPI_NONE, false, 3>(a, st);
+    // gemm_mid_kernel's shapes, no K slices
+    case 65536: return launch_mid<TEPI_NONE, false>(a, st, {kMid128, 1});
+    case 65538: return launch_mid<TEPI_NONE, false>(a, st, {kMid128Pairs, 1});
+    case 65539: return launch_mid<TEPI_NONE, false>(a, st, {kMid128x192, 1});
+    case 65540: return launch_mid<TEPI_NONE, false>(a, st, {kMid128x64Pairs, 1});
+    case 65541: return launch_mid<TEPI_NONE, false>(a, st, {kMid128x64, 1});
+    case 65542: return launch_mid<TEPI_NONE, false>(a, st, {kMid64, 1});
     default: return MI_EUNSUPPORTED;
   }
 }

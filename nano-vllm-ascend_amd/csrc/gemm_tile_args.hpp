@@ -35,6 +35,7 @@ struct TileArgs {
     float eps;
     int n_q_heads, n_kv_heads, block_size;
   } qkv;
+  int xcd_lf;  // gemm_mid_kernel: the XCDs share the tiles as 2^xcd_lf runs of features times 2^(3 - xcd_lf) runs of tokens (mid_tile)
 };
 
 constexpr int kPersistentGrid = 256;  // one workgroup per CU

@@ -258,3 +258,36 @@ def test_biased_products_of_the_persistent_kernel(ops, M, N, K):
     assert torch.equal(out[:M, :N], want) and bool((out[:, N:] == 7.0).all()) and bool((out[M] == 7.0).all())
     exact = x.double() @ w.double().T + b.double()
     assert bool(((want.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + (K + 1) * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T + b.abs())).all())
+
+
+@pytest.mark.parametrize("M", [65, 191, 192, 193, 385])
+@pytest.mark.parametrize("N,K", [(132, 64), (256, 128), (640, 448), (1000, 1600)])
+def test_gemm_tile_small_shapes_one_chain(ops, M, N, K):
+    """every small-tile shape (65536 ..: 128 x 128 with either ring, 128 x 192, 128 x 64 with either ring, 64 x 64) at part-filled tiles of rows
+    and features and at K loops shorter than, as long as and longer than its ring: the large kernel's bits"""
+    g, x, w = _case(M, N, K, seed=23)
+    x, w = x.to(DEV), w.to(DEV)
+    big = ops.gemm_tile(x, w, variant=0)
+    assert_bf16_close(big, oracle.linear(x.cpu(), w.cpu()), max_ulp=1, max_frac=2e-2, atol=K * 2.0 ** -22)
+    for variant in (65536, 65538, 65539, 65540, 65541, 65542):
+        y = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.gemm_tile(x, w, out=y[:M], variant=variant)
+        assert torch.equal(y[:M].view(torch.int16), big.view(torch.int16)), variant
+        assert bool((y[M] == 7.0).all()), variant
+
+
+# the shapes the choice of tile sends to 128 x 192, 128 x 64 (either ring) and 128 x 128 tiles, with SwiGLU, a bias and in K slices
+@pytest.mark.parametrize("M,N,K", [(1255, 4096, 1024), (886, 6144, 1024), (320, 6144, 1024), (500, 4096, 1024), (1025, 1024, 2048), (640, 6144, 1024)])
+def test_gemm_tile_small_shapes_epilogues(ops, M, N, K):
+    g, x, w = _case(M, N, K, seed=29)
+    b = torch.randn(N, generator=g).bfloat16()
+    xd, wd = x.to(DEV), w.to(DEV)
+    atol = K * 2.0 ** -22
+    plain = ops.gemm_tile(xd, wd, variant=0)
+    assert torch.equal(ops.gemm_tile(xd, wd).view(torch.int16), plain.view(torch.int16))
+    rows = torch.cat([torch.arange(0, 70), torch.arange(M - 70, M)])
+    assert_bf16_close(ops.gemm_tile(xd, wd, b.to(DEV))[rows], oracle.linear(x[rows], w, b), max_ulp=1, max_frac=2e-2, atol=atol)
+    assert_bf16_close(ops.gemm_tile(xd, wd, silu_mul=True), ops.silu_mul(plain).cpu(), max_ulp=2, max_frac=1e-3, atol=32 * atol)
+    part = ops.gemm_tile_splitk(xd, wd, 4)
+    want = torch.stack([x[rows, i * K // 4:(i + 1) * K // 4].double() @ w[:, i * K // 4:(i + 1) * K // 4].double().T for i in range(4)])
+    assert float((part.cpu().double()[:, rows] - want).abs().max()) <= K // 4 * 2.0 ** -24 * float((x.abs().double() @ w.abs().double().T).max())

@@ -48,8 +48,8 @@ def main():
     variants = {"tile": 0, "xcd_rect": 4, "direct_stores": 1 << 18, "mfma_32x32x16": 1 << 19, "eight_wave_r03": E8}
     if os.environ.get("GEMM_QUICK"):  # the four prefill projections only
         shapes = shapes[:4]
-    if os.environ.get("GEMM_MID"):  # the two kernels side by side over the mid-size shapes
-        variants = {"tile": 0, "mid128": 65536, "mid128_2stage": 65538, "mid128_3stage": 65539}
+    if os.environ.get("GEMM_MID"):  # the kernels and small-tile shapes side by side over the mid-size shapes
+        variants = {"tile": 0, "mid128": 65536, "mid128_2stage": 65538, "mid128x192": 65539, "mid128x64_3stage": 65540, "mid128x64": 65541, "mid64": 65542}
         shapes = [(M, N, K, f"{name}@{M}") for M in ((16384,) if os.environ.get("GEMM_MID") == "big" else (128, 256, 512, 1024, 2048, 4096))
                   for N, K, name in ((4096, 1024, "qkv"), (1024, 2048, "o_proj"), (6144, 1024, "gate_up"), (1024, 3072, "down"))]
     rows = []
