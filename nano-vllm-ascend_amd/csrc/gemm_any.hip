@@ -19,6 +19,7 @@
 //                          LDS, x rows straight into operands
 //   gemm_any_f32_kernel    true 32-bit: fp32 (or bf16, widened exactly) weights, x NOT rounded, on the fp32 matrix instruction
 //                          - the float32 serving mode, and the routers of sparse feed-forwards in either mode
+//   gemm_any_split_kernel  true 32-bit for fp32 weights and larger launches: both operands in three bf16 parts, on the bf16 instruction
 //   gemm_any_fma_kernel    the same in plain FMA chains, for operands whose rows are not whole 128-byte lines
 //   gemm_any_rows_kernel   M <= 8 rows, and the exact mode up to 64: one wave per (one or four output features, batch of rows)
 //                          streams its weight row once, lanes split K in 16-byte pieces, butterfly reduction; both
@@ -31,6 +32,7 @@
 // token gives the same bits whatever it is batched with, within one kernel; between kernels (a row computed in a
 // prompt's portion vs alone) results differ by rounding only.
 #include <algorithm>
+#include <cmath>
 
 #include "gemm_any_stream.hpp"
 
@@ -456,6 +458,10 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(GemmAnyArgs a) {
     if constexpr (GROUPS != 2) return;
   }
 }
+
+}  // namespace mi
+#include "gemm_any_split.hpp"
+namespace mi {
 
 // ---------------------------------------------------------------------------------------------------------------
 // MFMA kernel (bf16 weights): 4 waves as 2 x 2, each FM x FN fragments of 16 x 16 - a 64 x 64 tile, or 128 x 128
@@ -1192,6 +1198,23 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
 #define MI_F32_TILE(FM, FN, WM, WN, AHEAD)                                                                                          \
   gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, 0, AHEAD>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 1, AHEAD>, \
       gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 2, AHEAD>
+    // fp32 weights of larger launches: gemm_any_split_kernel, by the same model.  It has some 6 us more to begin with (32 with two weights: a step alone on its
+    // CU is a chain of read, split, write and multiply) and then, per 1024 of K, 13 us for every 256 tiles of 64 x 64; two weights above: ragged groups and
+    // the tile each looks for take 1.2 of the model's time.  Without groups from two tiles per CU on, one weight of groups from four tiles a group on: below
+    // it gains nothing or, groups, loses.  us, above / split: 721 rows x 1024 x 1024 24 / 28, x 2048 41 / 40, x 3072 60 / 50; 32 experts, 1024 -> 2 x 512: 400 pairs 56 / 65,
+    // 1200 66 / 69, 2884 90 / 79.  Steps of four layers, neither / products without groups / experts' first / experts' second: width 1024, 721 rows (90 pairs an
+    // expert) 1356 / 1338 / 1339 / 1400, 2831 rows (354) 3271 / 3010 / 3003 / 3236; width 2048, 381 rows (48) 2706 / 2724 (from two tiles per CU on 2672) / 2546 / 2776,
+    // 2461 rows (307) 11032 / 10415 / 9670 / 10745, all three 8690.  (431 rows of width 1024, 54 pairs an expert: experts' first 1024 / 1041, and not taken.)
+    if constexpr (sizeof(TW) == 4) {
+      const double row_tiles = grouped ? std::max(rows_per_group_max / 64. + groups / 2., (double)groups) : (double)((rows_per_group_max + 63) / 64) * groups;
+      const double n = row_tiles * nx(64) / 256., k = a.K / 1024.;
+      const double split_us = DUAL ? 32. + 26. * k * (grouped ? std::max(n, 1.) : std::ceil(n)) : 6. + 13. * k * (grouped ? std::max(n, 1.) : std::ceil(n));
+      const bool fills = grouped ? DUAL || rows_per_group_max >= 256 * (int64_t)groups : rows_per_group_max / 64. * groups * nx(64) / 256. >= 2.;
+      if (a.N > 32 && fills && split_us < std::min(large, std::min(medium, small)) * (DUAL ? grouped ? 2.4 : 2. : 1.) * k) {
+        go(gemm_any_split_kernel<DUAL, EXT, 0>, gemm_any_split_kernel<DUAL, EXT, EXT ? 0 : 1>, gemm_any_split_kernel<DUAL, EXT, EXT ? 0 : 2>, grid(64, 64));
+        return check_launch();
+      }
+    }
     // (fragments a step ahead: see the kernel)
     constexpr bool one_fp32 = !DUAL && sizeof(TW) == 4;
     if (a.N > 32 && large <= medium && large <= small) go(MI_F32_TILE(2, 2, 2, 2, false), grid(64, 64));
