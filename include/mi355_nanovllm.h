@@ -726,6 +726,9 @@ int mi_embedding_sinusoid_f32(const int64_t* ids, const void* table, int table_d
  * add_to_out != 0: out += LN(y) (a residual stream whose norm sits on the sublayer's output). */
 int mi_layernorm_f32(const float* y, int64_t ldy, const float* w, const float* b, float* out, int64_t ldo, int rows,
                      int width, float eps, int add_to_out, mi_stream stream);
+/* ... and out's rows rounded to bf16 beside them: rounded [rows][width], 16-byte aligned. */
+int mi_layernorm_f32_rounded(const float* y, int64_t ldy, const float* w, const float* b, float* out, int64_t ldo, int rows, int width,
+                             float eps, int add_to_out, mi_bf16* rounded, mi_stream stream);
 /* Sliding-window attention, per-row preparation.  proj rows hold q [H*D] at q_off, k [G*D] at k_off, v [G*Dv] at
  * v_off.  q <- q / rms(q over ALL H*D) * qn_w in place; k likewise with kn_w, stored to k_cache; v_first != NULL:
  * v <- (1 - *lam) v + *lam * v_first (in place), stored to v_cache.  Caches [blocks][G][block_size][D | Dv],
@@ -840,6 +843,10 @@ int mi_gemm_any_tile(const mi_bf16* xb, const int32_t* table, int tile_rows, con
 int64_t mi_gemm_any_fit_elems(int M, int N, int K, int dual, int act);
 int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias, const float* bias2,
                     int act, float* y, int64_t ldy, int M, int N, int K, float alpha, mi_bf16* xb, int64_t xb_elems, mi_stream stream);
+/* ... with x rounded to bf16 in xb [M][K] already: the tile kernels read xb, the general ones x.  The same results. */
+int mi_gemm_any_fit_rounded(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias, const float* bias2,
+                            int act, float* y, int64_t ldy, int M, int N, int K, float alpha, const mi_bf16* xb, int64_t xb_elems,
+                            mi_stream stream);
 /* Both products of the experts' feed-forwards over expert-sorted pairs on the tile kernels: y[pair_index] = down[e] act(w[e] x) (* w2[e] x).
  * mi_expert_ff_bytes: 16-byte aligned scratch, 0 where the shapes are not taken. */
 int64_t mi_expert_ff_bytes(int pairs, int n_groups, int ff, int width, int dual, int act);
@@ -852,6 +859,11 @@ int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, const int32_t* 
                         const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
                         const int32_t* offsets, const int32_t* pair_index, int pairs, int n_groups, int ff, int width, void* scratch,
                         int64_t scratch_bytes, float* y, mi_stream stream);
+/* ... with the tokens' rows rounded to bf16 in rounded [tokens][width] already (or NULL).  The same results. */
+int mi_expert_ff_rounded(const float* x, int64_t ldx, const mi_bf16* rounded, int tokens, const int32_t* pair_token, const mi_bf16* w,
+                         const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
+                         const int32_t* offsets, const int32_t* pair_index, int pairs, int n_groups, int ff, int width, void* scratch,
+                         int64_t scratch_bytes, float* y, mi_stream stream);
 /* mi_gemm_any_grouped with the activation named: y = act(x w^T) (* (x w2^T) with w2). */
 int mi_gemm_any_grouped_act(const float* x, int64_t ldx, const int32_t* x_rows, const void* w, const void* w2, int w_dtype,
                             int act, const int32_t* group_offsets, int n_groups, int rows_per_group_max, float* y,
@@ -947,6 +959,10 @@ int mi_moe_combine_shared(const float* y, const int32_t* ids, const float* weigh
 int mi_gated_norm_add_f32(float* res, int64_t ldr, const float* y, int64_t ldy, const float* gate_pre, int64_t ldg,
                           const float* w_post, float eps, const float* w_next, float* out, int64_t ldo, int rows, int width,
                           mi_stream stream);
+/* ... with w_next, and out's rows rounded to bf16 beside them: rounded [rows][width], 16-byte aligned. */
+int mi_gated_norm_add_f32_rounded(float* res, int64_t ldr, const float* y, int64_t ldy, const float* gate_pre, int64_t ldg,
+                                  const float* w_post, float eps, const float* w_next, float* out, int64_t ldo, int rows, int width,
+                                  mi_bf16* rounded, mi_stream stream);
 /* The same without a gate for an output still in parts: v = sum_k weights[row][k] * y[row * parts + k] + shared[row]
  * (y [rows * parts][width]; weights may be NULL: ones; shared may be NULL), res += v / sqrt(mean(v^2) + eps) * w_post;
  * w_next != NULL: out = res / sqrt(mean(res^2) + eps) * w_next. */

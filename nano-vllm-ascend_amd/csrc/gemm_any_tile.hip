@@ -324,6 +324,13 @@ static int any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const
   return check_launch();
 }
 
+// the table alone
+static int tile_table(const int32_t* group_offsets, int n_groups, int tile_rows, int sorted, int32_t* table, mi_stream stream) {
+  hipLaunchKernelGGL(any_operand_kernel, dim3(1), dim3(256), 0, S(stream), nullptr, 0, nullptr, group_offsets, n_groups, tile_rows, 0, sorted, 8, nullptr,
+                     table, (int)row_tiles(sorted, n_groups, tile_rows));
+  return check_launch();
+}
+
 extern "C" int mi_gemm_any_operand(const float* x, int64_t ldx, const int32_t* x_rows, const int32_t* group_offsets,
                                    int n_groups, int tile_rows, int rows, int K, mi_bf16* xb, int32_t* table,
                                    mi_stream stream) {
@@ -387,19 +394,29 @@ extern "C" int64_t mi_gemm_any_fit_elems(int M, int N, int K, int dual, int act)
   return tile_rows_for(M, N, K, 0, dual != 0, act) ? (int64_t)M * K : 0;
 }
 
-extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias,
-                               const float* bias2, int act, float* y, int64_t ldy, int M, int N, int K, float alpha, mi_bf16* xb,
-                               int64_t xb_elems, mi_stream stream) {
+// ready: xb holds x rounded to bf16 already (it is written here where not)
+static int any_fit(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias, const float* bias2, int act, float* y,
+                   int64_t ldy, int M, int N, int K, float alpha, const mi_bf16* xb, int64_t xb_elems, bool ready, mi_stream stream) {
   const bool fits = xb && x && w && y && w_dtype == MI_DTYPE_BF16 && M > 0 && ldx >= K && ldy >= N && ldy % 4 == 0 && aligned16(w) &&
                     (!w2 || aligned16(w2)) && aligned16(y) && (!bias || aligned16(bias)) && (!bias2 || (w2 && aligned16(bias2))) &&
                     aligned16(xb) && xb_elems >= (int64_t)M * K && !(act == MI_ACT_SOFTCAP && !(alpha > 0.f));
   const bool streams = any_stream_takes(M, N, K, 0, w2 != nullptr) && aligned16(x) && ldx % 4 == 0;
   const int t = fits && !streams ? tile_rows_for(M, N, K, 0, w2 != nullptr, act) : 0;
   if (!t) return mi_gemm_any_act(x, ldx, w, w2, w_dtype, bias, bias2, act, y, ldy, M, N, K, alpha, 0, stream);
-  const int rc = mi_gemm_any_operand(x, ldx, nullptr, nullptr, 0, t, M, K, xb, nullptr, stream);
+  const int rc = ready ? MI_OK : mi_gemm_any_operand(x, ldx, nullptr, nullptr, 0, t, M, K, const_cast<mi_bf16*>(xb), nullptr, stream);
   return rc != MI_OK ? rc
                      : mi_gemm_any_tile(xb, nullptr, t, static_cast<const mi_bf16*>(w), static_cast<const mi_bf16*>(w2), bias, bias2, act,
                                         0.f, nullptr, nullptr, 0, y, 0, ldy, nullptr, M, N, K, alpha, stream);
+}
+extern "C" int mi_gemm_any_fit(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias,
+                               const float* bias2, int act, float* y, int64_t ldy, int M, int N, int K, float alpha, mi_bf16* xb,
+                               int64_t xb_elems, mi_stream stream) {
+  return any_fit(x, ldx, w, w2, w_dtype, bias, bias2, act, y, ldy, M, N, K, alpha, xb, xb_elems, false, stream);
+}
+extern "C" int mi_gemm_any_fit_rounded(const float* x, int64_t ldx, const void* w, const void* w2, int w_dtype, const float* bias, const float* bias2,
+                                       int act, float* y, int64_t ldy, int M, int N, int K, float alpha, const mi_bf16* xb, int64_t xb_elems,
+                                       mi_stream stream) {
+  return any_fit(x, ldx, w, w2, w_dtype, bias, bias2, act, y, ldy, M, N, K, alpha, xb, xb_elems, true, stream);
 }
 
 // ---- the experts of moe.hip (bf16 activations and weights as they are stored, row-major) on the tile kernels: steps that bring prompts ----
@@ -432,9 +449,7 @@ extern "C" int mi_moe_tiles(const mi_bf16* x, int n_tokens, const mi_bf16* gate_
   if (scratch_bytes < mi_moe_tiles_bytes(pairs, n_experts, inter, hidden)) return MI_EWORKSPACE;
   int32_t* table = static_cast<int32_t*>(scratch);
   const int64_t tiles = row_tiles(pairs, n_experts, t);
-  hipLaunchKernelGGL(any_operand_kernel, dim3(1), dim3(256), 0, S(stream), nullptr, 0, nullptr, expert_offsets, n_experts, t, 0, pairs, 8, nullptr,
-                     table, (int)tiles);   // (no rows: the table only)
-  int rc = check_launch();
+  int rc = tile_table(expert_offsets, n_experts, t, pairs, table, stream);
   if (rc != MI_OK) return rc;
   AnyTileArgs<kActMoeGlu, true, true> g{};
   g.x = x, g.w = gate_up, g.w2 = gate_up + (int64_t)inter * hidden, g.ldx = hidden, g.ldy = inter, g.M = pairs, g.N = inter, g.K = hidden;
@@ -463,21 +478,14 @@ extern "C" int64_t mi_expert_ff_bytes(int pairs, int G, int ff, int width, int d
   return tiles > inner ? tiles : inner;
 }
 
-extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_token, const mi_bf16* w, const mi_bf16* w2,
-                            const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
-                            const int32_t* offsets, const int32_t* pair_index, int pairs, int G, int ff, int width, void* scratch,
-                            int64_t scratch_bytes, float* y, mi_stream stream) {
-  return mi_expert_ff_tokens(x, ldx, 0, pair_token, w, w2, down, act, limit, row_scale, row_scale_rows, offsets, pair_index, pairs, G, ff,
-                             width, scratch, scratch_bytes, y, stream);
-}
-
 // tokens: the rows of x (0: not known).  Where the pairs are at least as many, x is rounded to bf16 a token at a time and the first
 // product's feed gathers the pairs' rows; else the operand pass writes them out in the experts' order (65536 pairs of 8192 tokens x 2048,
 // us: pass 112 + product 459, now 15 + 441; 48 to 2000 pairs of 2 to 16 experts, both products: 0.97 to 1.01 of the time, 0.99 on average).
-extern "C" int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, const int32_t* pair_token, const mi_bf16* w,
-                                   const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale,
-                                   const int32_t* row_scale_rows, const int32_t* offsets, const int32_t* pair_index, int pairs, int G,
-                                   int ff, int width, void* scratch, int64_t scratch_bytes, float* y, mi_stream stream) {
+// rounded: the tokens' rows in bf16 already, or nullptr.
+static int expert_ff(const float* x, int64_t ldx, const mi_bf16* rounded, int tokens, const int32_t* pair_token, const mi_bf16* w,
+                     const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale,
+                     const int32_t* row_scale_rows, const int32_t* offsets, const int32_t* pair_index, int pairs, int G,
+                     int ff, int width, void* scratch, int64_t scratch_bytes, float* y, mi_stream stream) {
   if (!x || !w || !down || !offsets || !scratch || !y || pairs < 1 || G < 1 || !aligned16(scratch)) return MI_EINVAL;
   const int64_t need = mi_expert_ff_bytes(pairs, G, ff, width, w2 != nullptr, act);
   if (need == 0) return MI_EUNSUPPORTED;
@@ -496,12 +504,36 @@ extern "C" int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, cons
   mi_bf16* inner = reinterpret_cast<mi_bf16*>(p += round16((int64_t)pairs * width * 2));
   int32_t* table = reinterpret_cast<int32_t*>(p += round16((int64_t)pairs * ff * 2));
   const bool gather = w2 && pair_token && tokens > 0 && tokens <= pairs;
-  int rc = gather ? any_operand(x, ldx, nullptr, offsets, G, t, tokens, pairs, width, xb, table, stream)
-                  : mi_gemm_any_operand(x, ldx, pair_token, offsets, G, t, pairs, width, xb, table, stream);
+  const bool ready = gather && rounded && aligned16(rounded);
+  int rc = ready  ? tile_table(offsets, G, t, pairs, table, stream)
+           : gather ? any_operand(x, ldx, nullptr, offsets, G, t, tokens, pairs, width, xb, table, stream)
+                    : mi_gemm_any_operand(x, ldx, pair_token, offsets, G, t, pairs, width, xb, table, stream);
   if (rc == MI_OK)
-    rc = any_tile_product(xb, gather ? pair_token : nullptr, gather ? tokens : 0, table, t, w, w2, nullptr, nullptr, act, limit, row_scale,
+    rc = any_tile_product(ready ? rounded : xb, gather ? pair_token : nullptr, gather ? tokens : 0, table, t, w, w2, nullptr, nullptr, act, limit, row_scale,
                           row_scale_rows, G, inner, 1, ff, nullptr, pairs, ff, width, 1.f, stream);
   return rc != MI_OK ? rc
                      : mi_gemm_any_tile(inner, table, t, down, nullptr, nullptr, nullptr, MI_ACT_NONE, 0.f, nullptr, nullptr, G, y, 0, width,
                                         pair_index, pairs, width, ff, 1.f, stream);
+}
+
+extern "C" int mi_expert_ff_tokens(const float* x, int64_t ldx, int tokens, const int32_t* pair_token, const mi_bf16* w,
+                                   const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale,
+                                   const int32_t* row_scale_rows, const int32_t* offsets, const int32_t* pair_index, int pairs, int G,
+                                   int ff, int width, void* scratch, int64_t scratch_bytes, float* y, mi_stream stream) {
+  return expert_ff(x, ldx, nullptr, tokens, pair_token, w, w2, down, act, limit, row_scale, row_scale_rows, offsets, pair_index, pairs, G, ff,
+                   width, scratch, scratch_bytes, y, stream);
+}
+extern "C" int mi_expert_ff_rounded(const float* x, int64_t ldx, const mi_bf16* rounded, int tokens, const int32_t* pair_token, const mi_bf16* w,
+                                    const mi_bf16* w2, const mi_bf16* down, int act, float limit, const float* row_scale,
+                                    const int32_t* row_scale_rows, const int32_t* offsets, const int32_t* pair_index, int pairs, int G,
+                                    int ff, int width, void* scratch, int64_t scratch_bytes, float* y, mi_stream stream) {
+  return expert_ff(x, ldx, rounded, tokens, pair_token, w, w2, down, act, limit, row_scale, row_scale_rows, offsets, pair_index, pairs, G, ff,
+                   width, scratch, scratch_bytes, y, stream);
+}
+extern "C" int mi_expert_ff(const float* x, int64_t ldx, const int32_t* pair_token, const mi_bf16* w, const mi_bf16* w2,
+                            const mi_bf16* down, int act, float limit, const float* row_scale, const int32_t* row_scale_rows,
+                            const int32_t* offsets, const int32_t* pair_index, int pairs, int G, int ff, int width, void* scratch,
+                            int64_t scratch_bytes, float* y, mi_stream stream) {
+  return mi_expert_ff_tokens(x, ldx, 0, pair_token, w, w2, down, act, limit, row_scale, row_scale_rows, offsets, pair_index, pairs, G, ff,
+                             width, scratch, scratch_bytes, y, stream);
 }

@@ -90,15 +90,22 @@ __device__ __forceinline__ float vsum(fvec<VEC> v) {
   return s;
 }
 
+template <int VEC>
+__device__ __forceinline__ void store_rounded(uint16_t* to, const fvec<VEC>& v) {
+  if constexpr (VEC == 4) *reinterpret_cast<u32x2*>(to) = u32x2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+  else *to = f2bf(*reinterpret_cast<const float*>(&v));
+}
+
 // One workgroup per row; mean, then the mean of squared deviations.  Bound by the rows' bytes: a thread asks for all of its pieces (the
 // residual's too) before the first sum and keeps them (VEC 4: rows up to 4096 wide; the rest of wider ones is read again), so that a CU
-// has its whole share of requests out at once.  8112 rows of 2048, added to the residual: 37 us with a float per request, each pass over
+// has its whole share of requests out at once.  ROUND: a second output, the rows rounded to bf16 - the operand of the tile products that read them next, which
+// would each read the fp32 rows for it (8192 rows of 2048: 15.4 us a product).  8112 rows of 2048, added to the residual: 37 us with a float per request, each pass over
 // the row again; now 19.  KEEP: pieces a thread has; one where it cannot have more (8000 rows of 64: 7.6 us, four 8.4).
-template <int VEC, int KEEP = 4>
+template <int VEC, int KEEP = 4, bool ROUND = false>
 __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ y, int64_t ldy,
                                                             const float* __restrict__ w, const float* __restrict__ b,
                                                             float* __restrict__ out, int64_t ldo, int width, float eps,
-                                                            int add) {
+                                                            int add, uint16_t* __restrict__ rounded) {
   using vec = fvec<VEC>;
   __shared__ float red[4];
   constexpr int STEP = 256 * VEC;
@@ -136,13 +143,15 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
   for (int i = 0; i < KEEP; ++i) {
     const int c = c0 + i * STEP;
     if (c < width) {
-      const vec v = (kept[i] - mean) * rstd * vat<VEC>(w + c) + vat<VEC>(b + c);
-      *reinterpret_cast<vec*>(o + c) = add ? base[i] + v : v;
+      const vec v = (kept[i] - mean) * rstd * vat<VEC>(w + c) + vat<VEC>(b + c), sum = add ? base[i] + v : v;
+      *reinterpret_cast<vec*>(o + c) = sum;
+      if constexpr (ROUND) store_rounded<VEC>(rounded + (int64_t)blockIdx.x * width + c, sum);
     }
   }
   for (int c = c0 + KEEP * STEP; c < width; c += STEP) {
-    const vec v = (vat<VEC>(yr + c) - mean) * rstd * vat<VEC>(w + c) + vat<VEC>(b + c);
-    *reinterpret_cast<vec*>(o + c) = add ? vat<VEC>(o + c) + v : v;
+    const vec v = (vat<VEC>(yr + c) - mean) * rstd * vat<VEC>(w + c) + vat<VEC>(b + c), sum = add ? vat<VEC>(o + c) + v : v;
+    *reinterpret_cast<vec*>(o + c) = sum;
+    if constexpr (ROUND) store_rounded<VEC>(rounded + (int64_t)blockIdx.x * width + c, sum);
   }
 }
 
@@ -1698,16 +1707,17 @@ __global__ __launch_bounds__(256) void moe_combine_shared_kernel(const float* __
 // gated sublayer output behind its own norm, added to the residual: res += rms(y * sigmoid(gate)) * w_post
 // ---------------------------------------------------------------------------------------------------------------
 // One workgroup per row.  v = y * sigmoid(gate_pre) (gate_pre may be nullptr: v = y); res += v / sqrt(mean(v^2) + eps) *
-// w_post; w_next != nullptr: out = res / sqrt(mean(res^2) + eps) * w_next - what the next sublayer reads.  Bound by the rows' bytes: all of
+// w_post; w_next != nullptr: out = res / sqrt(mean(res^2) + eps) * w_next - what the next sublayer reads, with ROUND in bf16 beside it.  Bound by the rows' bytes: all of
 // a thread's pieces (VEC 4: rows up to 4096 wide; the rest of wider ones is read again) are asked for before the first sum.  8192 rows
 // of 2048 with a gate, 335 MB: 130 us with a float per request; now 57 (5.9 TB/s).
-template <int VEC, int KEEP = 4>
+template <int VEC, int KEEP = 4, bool ROUND = false>
 __global__ __launch_bounds__(256) void gated_norm_add_f32_kernel(float* __restrict__ res, int64_t ldr,
                                                                  const float* __restrict__ y, int64_t ldy,
                                                                  const float* __restrict__ gate_pre, int64_t ldg,
                                                                  const float* __restrict__ w_post, float eps,
                                                                  const float* __restrict__ w_next,
-                                                                 float* __restrict__ out, int64_t ldo, int width) {
+                                                                 float* __restrict__ out, int64_t ldo, int width,
+                                                                 uint16_t* __restrict__ rounded) {
   using vec = fvec<VEC>;
   __shared__ float red[4];
   constexpr int STEP = 256 * VEC;
@@ -1774,10 +1784,17 @@ __global__ __launch_bounds__(256) void gated_norm_add_f32_kernel(float* __restri
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
     const int c = c0 + i * STEP;
-    if (c < width) *reinterpret_cast<vec*>(o + c) = kept[i] * rstd2 * vat<VEC>(w_next + c);
+    if (c < width) {
+      const vec h = kept[i] * rstd2 * vat<VEC>(w_next + c);
+      *reinterpret_cast<vec*>(o + c) = h;
+      if constexpr (ROUND) store_rounded<VEC>(rounded + (int64_t)blockIdx.x * width + c, h);
+    }
   }
-  for (int c = c0 + KEEP * STEP; c < width; c += STEP)  // (a thread re-reads its own writes)
-    *reinterpret_cast<vec*>(o + c) = vat<VEC>(r + c) * rstd2 * vat<VEC>(w_next + c);
+  for (int c = c0 + KEEP * STEP; c < width; c += STEP) {  // (a thread re-reads its own writes)
+    const vec h = vat<VEC>(r + c) * rstd2 * vat<VEC>(w_next + c);
+    *reinterpret_cast<vec*>(o + c) = h;
+    if constexpr (ROUND) store_rounded<VEC>(rounded + (int64_t)blockIdx.x * width + c, h);
+  }
 }
 
 // The same without a gate, for a sublayer output that is still in parts: v = sum_k wts[row][k] y[row * parts + k] +
@@ -2119,16 +2136,25 @@ extern "C" int mi_embedding_sinusoid_f32(const int64_t* ids, const void* table, 
   return check_launch();
 }
 
-extern "C" int mi_layernorm_f32(const float* y, int64_t ldy, const float* w, const float* b, float* out, int64_t ldo,
-                                int rows, int width, float eps, int add_to_out, mi_stream stream) {
+static int layernorm_f32(const float* y, int64_t ldy, const float* w, const float* b, float* out, int64_t ldo, int rows, int width, float eps,
+                         int add_to_out, uint16_t* rounded, mi_stream stream) {
   if (!y || !w || !b || !out || rows < 0 || width < 1 || ldy < width || ldo < width) return MI_EINVAL;
   if (rows == 0) return MI_OK;
   // (from 256 wide on: less leaves most of a workgroup without a piece - 8192 rows of 100 9.2 us a float at a time, 10.3 in pieces)
   const bool vec = width >= 256 && width % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned16(y) && aligned16(w) && aligned16(b) && aligned16(out);
-  const auto kernel = vec ? layernorm_f32_kernel<4> : width <= 256 ? layernorm_f32_kernel<1, 1> : layernorm_f32_kernel<1>;
-  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out,
-                     ldo, width, eps, add_to_out);
+  const auto plain = vec ? layernorm_f32_kernel<4> : width <= 256 ? layernorm_f32_kernel<1, 1> : layernorm_f32_kernel<1>;
+  const auto both = vec ? layernorm_f32_kernel<4, 4, true> : width <= 256 ? layernorm_f32_kernel<1, 1, true> : layernorm_f32_kernel<1, 4, true>;
+  hipLaunchKernelGGL(rounded ? both : plain, dim3(rows), dim3(256), 0, S(stream), y, ldy, w, b, out, ldo, width, eps, add_to_out, rounded);
   return check_launch();
+}
+extern "C" int mi_layernorm_f32(const float* y, int64_t ldy, const float* w, const float* b, float* out, int64_t ldo,
+                                int rows, int width, float eps, int add_to_out, mi_stream stream) {
+  return layernorm_f32(y, ldy, w, b, out, ldo, rows, width, eps, add_to_out, nullptr, stream);
+}
+extern "C" int mi_layernorm_f32_rounded(const float* y, int64_t ldy, const float* w, const float* b, float* out, int64_t ldo, int rows, int width,
+                                        float eps, int add_to_out, mi_bf16* rounded, mi_stream stream) {
+  if (!rounded || !aligned16(rounded)) return MI_EINVAL;
+  return layernorm_f32(y, ldy, w, b, out, ldo, rows, width, eps, add_to_out, rounded, stream);
 }
 
 extern "C" int mi_swa_prepare(float* proj, int64_t ld, int q_off, int k_off, int v_off, const float* qn_w,
@@ -2566,18 +2592,29 @@ extern "C" int mi_moe_combine_shared(const float* y, const int32_t* ids, const f
   return check_launch();
 }
 
-extern "C" int mi_gated_norm_add_f32(float* res, int64_t ldr, const float* y, int64_t ldy, const float* gate_pre,
-                                     int64_t ldg, const float* w_post, float eps, const float* w_next, float* out,
-                                     int64_t ldo, int rows, int width, mi_stream stream) {
+static int gated_norm_add_f32(float* res, int64_t ldr, const float* y, int64_t ldy, const float* gate_pre, int64_t ldg, const float* w_post, float eps,
+                              const float* w_next, float* out, int64_t ldo, int rows, int width, uint16_t* rounded, mi_stream stream) {
   if (!res || !y || !w_post || rows < 0 || width < 1 || (w_next && !out)) return MI_EINVAL;
   if (rows == 0) return MI_OK;
   // (from 256 wide on, as layernorm: 8192 rows of 100 12.8 / 14.3 us)
   const bool vec = width >= 256 && width % 4 == 0 && ldr % 4 == 0 && ldy % 4 == 0 && aligned16(res) && aligned16(y) && aligned16(w_post) &&
                    (!gate_pre || (ldg % 4 == 0 && aligned16(gate_pre))) && (!w_next || (ldo % 4 == 0 && aligned16(out) && aligned16(w_next)));
-  const auto kernel = vec ? gated_norm_add_f32_kernel<4> : width <= 256 ? gated_norm_add_f32_kernel<1, 1> : gated_norm_add_f32_kernel<1>;
-  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, S(stream), res, ldr, y,
-                     ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, width);
+  const auto plain = vec ? gated_norm_add_f32_kernel<4> : width <= 256 ? gated_norm_add_f32_kernel<1, 1> : gated_norm_add_f32_kernel<1>;
+  const auto both = vec ? gated_norm_add_f32_kernel<4, 4, true> : width <= 256 ? gated_norm_add_f32_kernel<1, 1, true> : gated_norm_add_f32_kernel<1, 4, true>;
+  hipLaunchKernelGGL(rounded ? both : plain, dim3(rows), dim3(256), 0, S(stream), res, ldr, y,
+                     ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, width, rounded);
   return check_launch();
+}
+extern "C" int mi_gated_norm_add_f32(float* res, int64_t ldr, const float* y, int64_t ldy, const float* gate_pre,
+                                     int64_t ldg, const float* w_post, float eps, const float* w_next, float* out,
+                                     int64_t ldo, int rows, int width, mi_stream stream) {
+  return gated_norm_add_f32(res, ldr, y, ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, rows, width, nullptr, stream);
+}
+extern "C" int mi_gated_norm_add_f32_rounded(float* res, int64_t ldr, const float* y, int64_t ldy, const float* gate_pre, int64_t ldg,
+                                             const float* w_post, float eps, const float* w_next, float* out, int64_t ldo, int rows, int width,
+                                             mi_bf16* rounded, mi_stream stream) {
+  if (!rounded || !aligned16(rounded) || !w_next) return MI_EINVAL;
+  return gated_norm_add_f32(res, ldr, y, ldy, gate_pre, ldg, w_post, eps, w_next, out, ldo, rows, width, rounded, stream);
 }
 
 extern "C" int mi_parts_norm_add_f32(float* res, int64_t ldr, const float* y, int parts, const float* weights,

@@ -198,6 +198,7 @@ _SIGNATURES = {
     "mi_embedding_f32": (c_int, [_p, _p, c_int, _p, c_int, c_int, c_int, c_float, _p]),
     "mi_embedding_sinusoid_f32": (c_int, [_p, _p, c_int, _p, c_int, c_int, c_int, c_float, _p, _p, _p, c_int, _p]),
     "mi_layernorm_f32": (c_int, [_p, c_int64, _p, _p, _p, c_int64, c_int, c_int, c_float, c_int, _p]),
+    "mi_layernorm_f32_rounded": (c_int, [_p, c_int64, _p, _p, _p, c_int64, c_int, c_int, c_float, c_int, _p, _p]),
     "mi_swa_prepare": (c_int, [_p, c_int64, c_int, c_int, c_int, _p, _p, c_float, _p, c_int64, _p, _p, _p, c_int, _p,
                                c_int, c_int, c_int, c_int, c_int, c_int, _p]),
     "mi_swa_attention": (c_int, [_p, c_int64, _p, _p, c_int, _p, c_int, _p, _p, c_int, c_int, c_int, c_int, c_int,
@@ -223,11 +224,14 @@ _SIGNATURES = {
     "mi_gemm_any_table_ints": (c_int64, [c_int, c_int, c_int]),
     "mi_gemm_any_fit_elems": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
     "mi_gemm_any_fit": (c_int, [_p, c_int64, _p, _p, c_int, _p, _p, c_int, _p, c_int64, c_int, c_int, c_int, c_float, _p, c_int64, _p]),
+    "mi_gemm_any_fit_rounded": (c_int, [_p, c_int64, _p, _p, c_int, _p, _p, c_int, _p, c_int64, c_int, c_int, c_int, c_float, _p, c_int64, _p]),
     "mi_expert_ff_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mi_expert_ff": (c_int, [_p, c_int64, _p, _p, _p, _p, c_int, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p, c_int64, _p,
                              _p]),
     "mi_expert_ff_tokens": (c_int, [_p, c_int64, c_int, _p, _p, _p, _p, c_int, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p,
                                     c_int64, _p, _p]),
+    "mi_expert_ff_rounded": (c_int, [_p, c_int64, _p, c_int, _p, _p, _p, _p, c_int, c_float, _p, _p, _p, _p, c_int, c_int, c_int, c_int, _p,
+                                     c_int64, _p, _p]),
     "mi_gemm_any_operand": (c_int, [_p, c_int64, _p, _p, c_int, c_int, c_int, c_int, _p, _p, _p]),
     "mi_gemm_any_tile": (c_int, [_p, _p, c_int, _p, _p, _p, _p, c_int, c_float, _p, _p, c_int, _p, c_int, c_int64, _p, c_int,
                                  c_int, c_int, c_float, _p]),
@@ -251,6 +255,7 @@ _SIGNATURES = {
     "mi_route_topk": (c_int, [_p, c_int64, c_int, c_int, c_int, c_float, _p, _p, _p]),
     "mi_moe_combine_shared": (c_int, [_p, _p, _p, c_int, c_int, c_int, _p, c_int64, _p, c_int64, _p, c_int64, _p]),
     "mi_gated_norm_add_f32": (c_int, [_p, c_int64, _p, c_int64, _p, c_int64, _p, c_float, _p, _p, c_int64, c_int, c_int, _p]),
+    "mi_gated_norm_add_f32_rounded": (c_int, [_p, c_int64, _p, c_int64, _p, c_int64, _p, c_float, _p, _p, c_int64, c_int, c_int, _p, _p]),
     "mi_parts_norm_add_f32": (c_int, [_p, c_int64, _p, c_int, _p, _p, c_int64, _p, c_float, _p, _p, c_int64, c_int, c_int, _p]),
     "mi_linear_attention_state_elems": (c_int64, [c_int, c_int, c_int]),
     "mi_linear_attention": (c_int, [_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _p, _p, _p, _p, c_int64,

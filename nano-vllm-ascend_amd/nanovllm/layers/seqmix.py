@@ -102,10 +102,10 @@ class MergedRows(nn.Module):
         off, n = self.offsets[name]
         return y[:, off:off + n]
 
-    def forward(self, x: torch.Tensor, exact: bool = False) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, exact: bool = False, rounded=None) -> torch.Tensor:
         if self.bias is not None:
-            return ops.gemm_any_act(x, self.weight, bias=self.bias, exact=exact)
-        return ops.gemm_any(x, self.weight, exact=exact)
+            return ops.gemm_any_act(x, self.weight, bias=self.bias, exact=exact, rounded=rounded)
+        return ops.gemm_any(x, self.weight, exact=exact, rounded=rounded)
 
 
 class OutputLayerNorm(nn.Module):
@@ -114,9 +114,9 @@ class OutputLayerNorm(nn.Module):
         self.eps = eps
         self.weight, self.bias = _vector(width, 1.0), _vector(width)
 
-    def add_to(self, residual: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
-        """residual += LN(y), in place."""
-        return ops.layernorm_f32(y, self.weight, self.bias, self.eps, add_to=residual)
+    def add_to(self, residual: torch.Tensor, y: torch.Tensor, rounded=None) -> torch.Tensor:
+        """residual += LN(y), in place (rounded: gets it in bf16 too)."""
+        return ops.layernorm_f32(y, self.weight, self.bias, self.eps, add_to=residual, rounded=rounded)
 
     def forward(self, y: torch.Tensor) -> torch.Tensor:
         return ops.layernorm_f32(y, self.weight, self.bias, self.eps)
@@ -141,9 +141,9 @@ class SlidingWindowAttention(nn.Module):
     def cache_shapes(self, num_blocks: int, block_size: int):
         return (num_blocks, self.G, block_size, self.D), (num_blocks, self.G, block_size, self.Dv)
 
-    def forward(self, x: torch.Tensor, v_first: torch.Tensor | None):
+    def forward(self, x: torch.Tensor, v_first: torch.Tensor | None, rounded=None):
         ctx, m = get_context(), self.qkvg
-        y = m(x)
+        y = m(x, rounded=rounded)
         (qo, _), (ko, _), (vo, nv), (go, _) = m.offsets["q"], m.offsets["k"], m.offsets["v"], m.offsets["g"]
         mix_in = v_first if self.mixes_values == "later" else None
         ops.swa_prepare(y, qo, ko, vo, self.q_norm, self.k_norm, self.eps, mix_in, self.vmix if mix_in is not None else None,
@@ -173,12 +173,12 @@ class ChannelDeltaMixer(nn.Module):
         return ((n_slots, ops.channel_delta_state_elems(self.H, self.D, self.Dv)),
                 (n_slots, max(self.taps - 1, 1), self.qkv.weight.shape[0]))
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, rounded=None) -> torch.Tensor:
         ctx = get_context()
         cu, kv, slots = ctx.cu_seqlens_q, ctx.kv_lens, ctx.state_slots
-        pre = self.qkv(x)
+        pre = self.qkv(x, rounded=rounded)
         qkv = ops.causal_conv_advance(pre, self.conv.weight, self.conv_state, cu, kv, slots, ctx.max_seqlen_q, silu=True)
-        low = self.low(x)
+        low = self.low(x, rounded=rounded)
         decay_pre = ops.gemm_any(self.low.cols(low, "a1"), self.a2)
         gate_pre = ops.gemm_any(self.low.cols(low, "g1"), self.g2)
         off = self.qkv.offsets
@@ -205,13 +205,13 @@ class GroupedSparseMLP(nn.Module):
         for p in (self.gate, self.up, self.down):
             p.weight_loader = lambda param, tensor, expert: param.data[expert].copy_(tensor)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, rounded=None) -> torch.Tensor:
         z = ops.gemm_any(x, self.router, exact=True)  # router logits in true 32-bit in every serving mode
         ids, wts = ops.route_grouped(z, self.correction, self.top_k, self.groups, self.keep, self.score_kind,
                                      self.group_kind)
         offsets, pair_token, pair_index = ops.moe_sort(ids, self.n_out)
         P = ids.numel()
-        y = ops.expert_ff(x, pair_token, self.gate, self.up, self.down, _C.ACT_SILU, offsets, P, pair_index)
+        y = ops.expert_ff(x, pair_token, self.gate, self.up, self.down, _C.ACT_SILU, offsets, P, pair_index, rounded=rounded)
         return ops.moe_combine_f32(y, x, ids, wts, self.E)
 
 
@@ -444,13 +444,13 @@ class GatedOutputNorm(nn.Module):
         self.eps = eps
         self.gate, self.gate_b, self.weight = _matrix(width, width), _vector(width), _vector(width, 1.0)
 
-    def gate_of(self, h: torch.Tensor) -> torch.Tensor:
+    def gate_of(self, h: torch.Tensor, rounded=None) -> torch.Tensor:
         """-> W_g h + b_g (the sigmoid is taken where the gate is applied)"""
-        return ops.gemm_any_act(h, self.gate, bias=self.gate_b)
+        return ops.gemm_any_act(h, self.gate, bias=self.gate_b, rounded=rounded)
 
-    def add_to(self, residual: torch.Tensor, y: torch.Tensor, gate_pre: torch.Tensor, next_norm: torch.Tensor | None):
-        """residual += rms(y * sigmoid(gate_pre)) * w in place; -> rms(residual) * next_norm (None without one)"""
-        return ops.gated_norm_add_f32(residual, y, gate_pre, self.weight, self.eps, next_norm)
+    def add_to(self, residual: torch.Tensor, y: torch.Tensor, gate_pre: torch.Tensor, next_norm: torch.Tensor | None, rounded=None):
+        """residual += rms(y * sigmoid(gate_pre)) * w in place; -> rms(residual) * next_norm (None without one; rounded: gets it in bf16)"""
+        return ops.gated_norm_add_f32(residual, y, gate_pre, self.weight, self.eps, next_norm, rounded)
 
 
 class _LinearAttentionState(nn.Module):

@@ -224,14 +224,19 @@ class FelolornForCausalLM(nn.Module):
         cfg, n = self.config, len(self.layers)
         x = ops.embedding_f32(input_ids, self.embed, scale=cfg.embedding_scale)
         h = ops.add_rmsnorm_f32(x, None, 0.0, self.layers[0].norm1, cfg.norm_eps)
+        operand, hb = ops.product_operand(x, self.embed.dtype), None   # hb: h in bf16, once a norm has written it
         for i, layer in enumerate(self.layers):
             after = self.layers[i + 1].norm1 if i + 1 < n else None   # (the output's norm is taken of the wanted rows only)
-            gate = layer.out1.gate_of(h)
+            gate = layer.out1.gate_of(h, hb)
             y = layer.mix(layer.conv(h))
-            h = layer.out1.add_to(x, y, gate, layer.norm2 if layer.mlp is not None else after)
+            then = layer.norm2 if layer.mlp is not None else after
+            hb = operand if then is not None else None
+            h = layer.out1.add_to(x, y, gate, then, hb)
             if layer.mlp is not None:
-                gate = layer.out2.gate_of(h)
-                h = layer.out2.add_to(x, layer.mlp(h), gate, after)
+                gate = layer.out2.gate_of(h, hb)
+                y = layer.mlp(h, hb)
+                hb = operand if after is not None else None
+                h = layer.out2.add_to(x, y, gate, after, hb)
             if self.trace_layers is not None:
                 self.trace_layers.append(x.clone())
         return x

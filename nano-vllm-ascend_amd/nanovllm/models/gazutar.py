@@ -211,15 +211,19 @@ class GazutarForCausalLM(nn.Module):
     # ---- one step over the rows the context describes ----------------------------------------------------------------
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor | None = None) -> torch.Tensor:
         x = ops.embedding_f32(input_ids, self.embed)
-        v_first = None
-        for layer in self.layers:
+        v_first, operand, n = None, ops.product_operand(x, self.embed.dtype), len(self.layers)
+        xb = None   # x in bf16, once a norm has written it
+        for i, layer in enumerate(self.layers):
             if layer.kind == "attention":
-                y, v_first = layer.mix(x, v_first)
+                y, v_first = layer.mix(x, v_first, rounded=xb)
             else:
-                y = layer.mix(x)
-            layer.norm1.add_to(x, y)
+                y = layer.mix(x, rounded=xb)
+            xb = operand if i + 1 < n or layer.mlp is not None else None
+            layer.norm1.add_to(x, y, rounded=xb)
             if layer.mlp is not None:
-                layer.norm2.add_to(x, layer.mlp(x))
+                y = layer.mlp(x, rounded=xb)
+                xb = operand if i + 1 < n else None
+                layer.norm2.add_to(x, y, rounded=xb)
             if self.trace_layers is not None:
                 self.trace_layers.append(x.clone())
         return x

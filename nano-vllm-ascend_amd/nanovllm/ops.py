@@ -1151,15 +1151,35 @@ def _grouped_tiles(x, x_rows, w, w2, act: int, offsets, rows_max: int, y, y_rows
     return t > 0
 
 
-def _gemm_any_fit(x, w, w2, bias, bias2, act: int, out, M: int, N: int, K: int, alpha: float) -> None:
+def product_operand(x, dtype) -> torch.Tensor | None:
+    """Where a norm puts its rows rounded to bf16 beside x, its fp32 rows, for the products over weights of `dtype` that read them next (their
+    `rounded`), or None.  From 512 rows on: those go to the tile kernels, each of which would otherwise round the rows in a pass of its own
+    (fewer are left as they are: a decode step's products read fp32 rows)."""
+    return torch.empty(x.shape, dtype=_BF16, device=x.device) if dtype == _BF16 and x.shape[0] >= 512 and x.shape[1] % 64 == 0 else None
+
+
+def _rounded(x, rounded) -> None:
+    if rounded is not None:
+        require_gpu(rounded)
+        _bf16(rounded)
+        assert rounded.shape == x.shape and rounded.is_contiguous()
+
+
+def _gemm_any_fit(x, w, w2, bias, bias2, act: int, out, M: int, N: int, K: int, alpha: float, rounded=None) -> None:
+    if rounded is not None:
+        _rounded(x, rounded)
+        check(lib.mi_gemm_any_fit_rounded(ptr(x), x.stride(0), ptr(w), ptr(w2), _C.DTYPE_BF16, ptr(bias), ptr(bias2), act, ptr(out),
+                                          out.stride(0), M, N, K, alpha, ptr(rounded), M * K, stream()), "mi_gemm_any_fit_rounded")
+        return
     n = lib.mi_gemm_any_fit_elems(M, N, K, w2 is not None, act)
     xb = torch.empty(n, dtype=_BF16, device=x.device) if n else None
     check(lib.mi_gemm_any_fit(ptr(x), x.stride(0), ptr(w), ptr(w2), _C.DTYPE_BF16, ptr(bias), ptr(bias2), act, ptr(out), out.stride(0),
                               M, N, K, alpha, ptr(xb), n, stream()), "mi_gemm_any_fit")
 
 
-def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None) -> torch.Tensor:
-    """alpha * x @ w.T for any shapes; x may be a column slice of a wider buffer (unit inner stride)."""
+def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None, rounded=None) -> torch.Tensor:
+    """alpha * x @ w.T for any shapes; x may be a column slice of a wider buffer (unit inner stride).  rounded: x in bf16
+    (product_operand)."""
     require_gpu(x, w)
     _f32(x, out)
     assert x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1], (x.shape, w.shape)
@@ -1169,7 +1189,7 @@ def gemm_any(x, w, alpha: float = 1.0, exact: bool = False, out=None) -> torch.T
         out = torch.empty((M, N), dtype=_F32, device=x.device)
     assert out.shape == (M, N)
     if M > 8 and not exact and w.dtype == _BF16:
-        _gemm_any_fit(x, w, None, None, None, _C.ACT_NONE, out, M, N, K, alpha)
+        _gemm_any_fit(x, w, None, None, None, _C.ACT_NONE, out, M, N, K, alpha, rounded)
         return out
     check(lib.mi_gemm_any(ptr(x), x.stride(0) if M > 1 else K, ptr(w), _dt(w), ptr(out), out.stride(0) if M > 1 else N,
                           M, N, K, float(alpha), int(exact), stream()), "mi_gemm_any")
@@ -1193,10 +1213,11 @@ def gemm_any_grouped(x, x_rows, w, w2, group_offsets, rows_max: int, y_rows, y_r
 
 
 def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_index, limit: float = 0.0, row_scale=None,
-              row_scale_rows=None) -> torch.Tensor:
+              row_scale_rows=None, rounded=None) -> torch.Tensor:
     """Both products of the experts' feed-forwards over expert-sorted pairs: down[e] (act(w[e] x) (* w2[e] x)) of every pair at
     its place pair_index.  bf16 weights, 16 pairs and more (of small experts more than few): the inner activations leave the
-    first product as the bf16 rows that the second one multiplies (it would round the same numbers itself)."""
+    first product as the bf16 rows that the second one multiplies (it would round the same numbers itself).  rounded: x in bf16
+    (product_operand)."""
     G, ff, width = w.shape
     n = lib.mi_expert_ff_bytes(pairs, G, ff, width, w2 is not None, int(act)) if w.dtype == _BF16 and down.dtype == _BF16 else 0
     if n and not (w.data_ptr() | down.data_ptr() | (0 if w2 is None else w2.data_ptr())) % 16:
@@ -1208,9 +1229,10 @@ def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_in
         assert w.is_contiguous() and down.is_contiguous() and (w2 is None or (w2.shape == w.shape and w2.is_contiguous() and w2.dtype == _BF16))
         scratch = torch.empty(n, dtype=torch.uint8, device=x.device)
         y = torch.empty((pairs, width), dtype=_F32, device=x.device)
-        check(lib.mi_expert_ff_tokens(ptr(x), x.stride(0) if x.shape[0] > 1 else width, x.shape[0], ptr(pair_token), ptr(w), ptr(w2),
-                                      ptr(down), int(act), float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets),
-                                      ptr(pair_index), pairs, G, ff, width, ptr(scratch), n, ptr(y), stream()), "mi_expert_ff_tokens")
+        _rounded(x, rounded)
+        check(lib.mi_expert_ff_rounded(ptr(x), x.stride(0) if x.shape[0] > 1 else width, ptr(rounded), x.shape[0], ptr(pair_token), ptr(w),
+                                       ptr(w2), ptr(down), int(act), float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets),
+                                       ptr(pair_index), pairs, G, ff, width, ptr(scratch), n, ptr(y), stream()), "mi_expert_ff_rounded")
         return y
     a = gemm_any_grouped_glu(x, pair_token, w, w2, act, limit, row_scale, row_scale_rows, offsets, pairs, None, pairs)
     return gemm_any_grouped(a, None, down, None, offsets, pairs, pair_index, pairs)
@@ -1242,13 +1264,18 @@ def embedding_sinusoid_f32(ids, table, scale: float, inv_freq, cu_q, kv_lens) ->
     return out
 
 
-def layernorm_f32(y, w, b, eps: float, add_to=None) -> torch.Tensor:
-    """LN(y) * w + b per row; add_to: the residual it is added to IN PLACE (returned)."""
+def layernorm_f32(y, w, b, eps: float, add_to=None, rounded=None) -> torch.Tensor:
+    """LN(y) * w + b per row; add_to: the residual it is added to IN PLACE (returned).  rounded: gets the result in bf16."""
     require_gpu(y, w, b)
     _f32(y, w, b, add_to)
     rows, width = y.shape
     out = add_to if add_to is not None else torch.empty((rows, width), dtype=_F32, device=y.device)
     assert out.shape == y.shape and w.numel() == width and b.numel() == width
+    if rounded is not None:
+        _rounded(out, rounded)
+        check(lib.mi_layernorm_f32_rounded(ptr(y), y.stride(0), ptr(w), ptr(b), ptr(out), out.stride(0), rows, width, float(eps),
+                                           int(add_to is not None), ptr(rounded), stream()), "mi_layernorm_f32_rounded")
+        return out
     check(lib.mi_layernorm_f32(ptr(y), y.stride(0), ptr(w), ptr(b), ptr(out), out.stride(0), rows, width, float(eps),
                                int(add_to is not None), stream()), "mi_layernorm_f32")
     return out
@@ -1407,8 +1434,8 @@ def moe_combine_f32(y, h, ids, wts, n_experts: int) -> torch.Tensor:
 # ---- pre-norm 32-bit families: epilogue / batched projections, residual stack, minimal gated recurrence, latent and
 # log-distance-biased attention, plain top-k routing (csrc/gemm_any.hip, csrc/seqmix.hip)
 def gemm_any_act(x, w, bias=None, act: int = _C.ACT_NONE, w2=None, bias2=None, alpha: float = 1.0, exact: bool = False,
-                 out=None) -> torch.Tensor:
-    """alpha * act(x w^T + bias), or with w2: alpha * act(x w^T + bias) * (x w2^T + bias2)."""
+                 out=None, rounded=None) -> torch.Tensor:
+    """alpha * act(x w^T + bias), or with w2: alpha * act(x w^T + bias) * (x w2^T + bias2).  rounded: x in bf16 (product_operand)."""
     require_gpu(x, w)
     _f32(x, out, bias, bias2)
     assert x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1], (x.shape, w.shape)
@@ -1420,7 +1447,7 @@ def gemm_any_act(x, w, bias=None, act: int = _C.ACT_NONE, w2=None, bias2=None, a
         out = torch.empty((M, N), dtype=_F32, device=x.device)
     assert out.shape == (M, N)
     if M > 8 and not exact and w.dtype == _BF16:
-        _gemm_any_fit(x, w, w2, bias, bias2, int(act), out, M, N, K, alpha)
+        _gemm_any_fit(x, w, w2, bias, bias2, int(act), out, M, N, K, alpha, rounded)
         return out
     check(lib.mi_gemm_any_act(ptr(x), x.stride(0) if M > 1 else K, ptr(w), ptr(w2), _dt(w), ptr(bias), ptr(bias2), int(act),
                               ptr(out), out.stride(0) if M > 1 else N, M, N, K, float(alpha), int(exact), stream()),
@@ -1608,9 +1635,9 @@ def moe_combine_shared(y, ids, wts, width: int, shared=None, shared_gate=None) -
 
 
 # ---- sandwich-normed families with gated residual branches, decayed linear attention (csrc/seqmix.hip)
-def gated_norm_add_f32(res, y, gate_pre, w_post, eps: float, w_next=None):
+def gated_norm_add_f32(res, y, gate_pre, w_post, eps: float, w_next=None, rounded=None):
     """res += rms(y * sigmoid(gate_pre)) * w_post in place (gate_pre None: no gate); w_next given: returns
-    rms(res) * w_next, else None."""
+    rms(res) * w_next (rounded: gets it in bf16), else None."""
     require_gpu(res, y, w_post)
     _f32(res, y, gate_pre, w_post, w_next)
     rows, width = res.shape
@@ -1619,6 +1646,12 @@ def gated_norm_add_f32(res, y, gate_pre, w_post, eps: float, w_next=None):
     if w_next is not None:
         assert w_next.numel() == width
         out = torch.empty((rows, width), dtype=_F32, device=res.device)
+    if rounded is not None:
+        _rounded(res, rounded)
+        check(lib.mi_gated_norm_add_f32_rounded(ptr(res), res.stride(0), ptr(y), y.stride(0), ptr(gate_pre),
+                                                gate_pre.stride(0) if gate_pre is not None else 0, ptr(w_post), float(eps), ptr(w_next),
+                                                ptr(out), width, rows, width, ptr(rounded), stream()), "mi_gated_norm_add_f32_rounded")
+        return out
     check(lib.mi_gated_norm_add_f32(ptr(res), res.stride(0), ptr(y), y.stride(0), ptr(gate_pre),
                                     gate_pre.stride(0) if gate_pre is not None else 0, ptr(w_post), float(eps), ptr(w_next),
                                     ptr(out), width, rows, width, stream()), "mi_gated_norm_add_f32")
