@@ -506,7 +506,9 @@ constexpr MidTile kMidTiles[kMidTileCount] = {{128, 128, 1, 2.2, 1.8, 0.32, 0.24
                                               {128, 64, 2, 3.3, 0., 0.29, 0.18, 0.60, 0.18},  {128, 64, 1, 2.8, 1.4, 0.21, 0.21, 0., 0.},
                                               {128, 192, 1, 1.7, 3.1, 0.43, 0.29, 0., 0.},     {64, 64, 2, 3.1, 0., 0.14, 0.08, 0.32, 0.12}};
 constexpr MidTile kLargeTile = {256, 256, 1, 3.1, 3.7, 1.04, 0.48, 0., 0.};
-constexpr double kLaunchUs = 3.8, kPartialBytesPerUs = 4.0e6;
+// the sum of K slices: its launch and its bytes (us, four or eight slices / none: 200 x 1024 x 3072 9.3 / 9.7, 137 8.7 / 9.5, 100 x 1024 x 4096 9.6 / 11.7; 300 x 1024 x
+// 3072 and 200 x 1024 x 2048 are not cut)
+constexpr double kLaunchUs = 3.2, kPartialBytesPerUs = 4.0e6;
 
 // fewer 256-tiles than CUs
 static bool few_tiles(int M, int N) {
