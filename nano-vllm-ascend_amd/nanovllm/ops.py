@@ -1230,9 +1230,13 @@ def expert_ff(x, pair_token, w, w2, down, act: int, offsets, pairs: int, pair_in
         scratch = torch.empty(n, dtype=torch.uint8, device=x.device)
         y = torch.empty((pairs, width), dtype=_F32, device=x.device)
         _rounded(x, rounded)
-        check(lib.mi_expert_ff_rounded(ptr(x), x.stride(0) if x.shape[0] > 1 else width, ptr(rounded), x.shape[0], ptr(pair_token), ptr(w),
-                                       ptr(w2), ptr(down), int(act), float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets),
-                                       ptr(pair_index), pairs, G, ff, width, ptr(scratch), n, ptr(y), stream()), "mi_expert_ff_rounded")
+        rest = (ptr(pair_token), ptr(w), ptr(w2), ptr(down), int(act), float(limit), ptr(row_scale), ptr(row_scale_rows), ptr(offsets),
+                ptr(pair_index), pairs, G, ff, width, ptr(scratch), n, ptr(y), stream())
+        ldx = x.stride(0) if x.shape[0] > 1 else width
+        if rounded is not None:
+            check(lib.mi_expert_ff_rounded(ptr(x), ldx, ptr(rounded), x.shape[0], *rest), "mi_expert_ff_rounded")
+        else:
+            check(lib.mi_expert_ff_tokens(ptr(x), ldx, x.shape[0], *rest), "mi_expert_ff_tokens")
         return y
     a = gemm_any_grouped_glu(x, pair_token, w, w2, act, limit, row_scale, row_scale_rows, offsets, pairs, None, pairs)
     return gemm_any_grouped(a, None, down, None, offsets, pairs, pair_index, pairs)
