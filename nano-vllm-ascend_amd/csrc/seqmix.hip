@@ -99,7 +99,7 @@ __device__ __forceinline__ void store_rounded(uint16_t* to, const fvec<VEC>& v) 
 // One workgroup per row; mean, then the mean of squared deviations.  Bound by the rows' bytes: a thread asks for all of its pieces (the
 // residual's too) before the first sum and keeps them (VEC 4: rows up to 4096 wide; the rest of wider ones is read again), so that a CU
 // has its whole share of requests out at once.  ROUND: a second output, the rows rounded to bf16 - the operand of the tile products that read them next, which
-// would each read the fp32 rows for it (8192 rows of 2048: 15.4 us a product).  8112 rows of 2048, added to the residual: 37 us with a float per request, each pass over
+// would each read the fp32 rows for it (8112 rows of 1024: 8.9 us a product; 18.6 -> 20.7 here).  8112 rows of 2048, added to the residual: 37 us with a float per request, each pass over
 // the row again; now 19.  KEEP: pieces a thread has; one where it cannot have more (8000 rows of 64: 7.6 us, four 8.4).
 template <int VEC, int KEEP = 4, bool ROUND = false>
 __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ y, int64_t ldy,
