@@ -6,8 +6,12 @@ namespace mi {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
-// Eight numbers as three bf16 parts, each the nearest to what the parts before it leave: x = h + m + l exactly (8 + 8 + 8 bits; the rests are
-// floats).  (The rests by the two-term dot product, one instruction in place of two: the same time.)
+// Operands are split times 2^24, and sums leave times 2^-48: the last bit of the smallest number, 2^-149, is then above the smallest normal number, so
+// that no part of any operand is lost or subnormal, and a sum reaches below what fp32 holds.
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
+
+// Eight numbers, times kSplitScale, as three bf16 parts, each the nearest to what the parts before it leave: h + m + l exactly (8 + 8 + 8 bits; the
+// rests are floats).  (The rests by the two-term dot product, one instruction in place of two: the same time.)
 struct SplitParts {
   u32x4 part[3];
 };
@@ -15,7 +19,7 @@ __device__ __forceinline__ SplitParts split_parts(const f32x4& a, const f32x4& b
   SplitParts p;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float u = i < 2 ? a[2 * i] : b[2 * i - 4], v = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+    float u = kSplitScale * (i < 2 ? a[2 * i] : b[2 * i - 4]), v = kSplitScale * (i < 2 ? a[2 * i + 1] : b[2 * i - 3]);
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
       p.part[s][i] = pack_bf(u, v);
@@ -30,14 +34,14 @@ __device__ __forceinline__ SplitParts split_parts(const f32x4& a, const f32x4& b
 // m m, h l and l h on v_mfma_f32_16x16x32_bf16, those with a rest in a sum of their own.  The products left out are below 2^-25 of |x w|; a step of
 // 32 k is rounded once into each sum where the fp32 matrix instruction rounds eight times: error against 64 bits (2-norm) 1.9e-7 at K =
 // 1024 and 4.0e-7 at 4096, the fp32 instruction's (gemm_any_f32_kernel) 5.7e-7 and 1.15e-6.
-// What bounds it: the fp32 matrix rate is 1/16 of the bf16 one, so six products are 3/8 of its time; the split (eleven vector instructions for
+// What bounds it: the fp32 matrix rate is 1/16 of the bf16 one, so six products are 3/8 of its time; the split (thirteen vector instructions for
 // two numbers) and the LDS (24 KB written and 48 KB read per step) take about as long as the products beside them, and the clock falls with the matrix
 // pipe's load.  The matrix instructions stand among the next step's split (one tile alone on its CU 34.7 -> 27.9 us, 721 x 1024 x 1024).
 // us with cold weights, gemm_any_f32_kernel / here: 4096 x 4096 x 4096 1129 / 827, 1500 x 4096 x 2048 241 / 180, 721 x 3072 x 1024 60 / 50; 5768 pairs
 // of 64 experts, 2048 -> 2 x 768 477 / 408, back 241 / 237.  128-row tiles are 8 % faster at 4096 x 4096 x 4096 and lose with their fewer
 // tiles below it and with uneven groups (a step of 721 rows 1311 us, 1337 with 128 x 32 of two weights, 1347 with 48 x 64).
-// An infinity has no finite rest, the first part of a number next to the largest may be one, and the last part of one below 2^-110 may fall
-// under bf16's smallest: outputs that come out infinite, not a number or below 2^-90 are summed once more in plain fp32 by their lane.
+// An infinity has no finite rest, a number of 2^104 and more times 2^24 is one, and so may a sum of 2^80 and more be: outputs that come out
+// infinite or not a number are summed once more in plain fp32 by their lane.
 // Rows beyond the group's end and features beyond N are read from the last valid one and not stored.  Needs what gemm_any_f32_kernel needs.
 template <bool DUAL, bool EXT, int GROUPS>
 __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
@@ -154,7 +158,7 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
       if (INSIDE || kt + 3 < KT) request(kt + 3, next);
       multiply(p);
       // reads, some of the split in their shadow, then its rest and its LDS writes among the matrix instructions
-      constexpr int MULS = 6 * ND * FM * FN, VALU = U * 44, EACH = MULS / (3 * U);
+      constexpr int MULS = 6 * ND * FM * FN, VALU = U * 52, EACH = MULS / (3 * U);
       __builtin_amdgcn_sched_group_barrier(0x100, 3 * (FM + ND * FN), 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
 #pragma unroll
@@ -185,8 +189,8 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
           acc[d][i][j] += low[d][i][j];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float v = fabsf(acc[d][i][j][r]);
-            redo |= !(v <= FLT_MAX) || (v < 0x1p-90f && v != 0.f);
+            redo |= !(fabsf(acc[d][i][j][r]) <= FLT_MAX);
+            acc[d][i][j][r] *= kSplitUnscale;
           }
         }
 #pragma unroll

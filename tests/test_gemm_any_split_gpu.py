@@ -83,3 +83,15 @@ def test_split_products_of_numbers_without_parts(ops):
     tiny = want[40, 12:]
     assert float((y[40, 12:].double() - tiny).norm() / tiny.norm()) <= K * 2.0 ** -24
     assert bool((y[42, 12:] == 0).all())
+
+
+# x of 2^a, weights of 2^b: operands below what three bf16 parts hold, against large ones (outputs that are ordinary numbers), either way round
+@pytest.mark.parametrize("a,b", [(-116, 36), (-120, 79), (-124, 40), (-130, 60), (-138, 79), (36, -116), (60, -130), (-60, -60)])
+def test_split_products_of_small_operands(ops, a, b):
+    M, N, K = 2000, 1100, 1024
+    g = torch.Generator().manual_seed(5 - a)
+    x, w = (torch.randn(M, K, generator=g) * 2.0 ** a).to(DEV), (torch.randn(N, K, generator=g) * 2.0 ** b).to(DEV)
+    y = ops.gemm_any(x, w, exact=True)
+    want = x.double() @ w.double().T
+    # as of ordinary operands: 2^-24 a rounding; a bf16 part less is 3.5e-6
+    assert float((y.double() - want).norm() / want.norm()) <= 4e-7
