@@ -40,8 +40,10 @@ __device__ __forceinline__ SplitParts split_parts(const f32x4& a, const f32x4& b
 // us with cold weights, gemm_any_f32_kernel / here: 4096 x 4096 x 4096 1129 / 827, 1500 x 4096 x 2048 241 / 180, 721 x 3072 x 1024 60 / 50; 5768 pairs
 // of 64 experts, 2048 -> 2 x 768 477 / 408, back 241 / 237.  128-row tiles are 8 % faster at 4096 x 4096 x 4096 and lose with their fewer
 // tiles below it and with uneven groups (a step of 721 rows 1311 us, 1337 with 128 x 32 of two weights, 1347 with 48 x 64).
-// An infinity has no finite rest, a number of 2^104 and more times 2^24 is one, and so may a sum of 2^80 and more be: outputs that come out
-// infinite or not a number are summed once more in plain fp32 by their lane.
+// An infinity has no finite rest, a number of 2^104 and more times 2^24 is one, and so may a sum of 2^80 and more be: a wave with an output
+// that is not finite sums its outputs once more on the fp32 matrix instruction, and takes from there those that were not finite and no other (an output is a
+// function of its own row of x and of the weights).  us, no / one / forty rows with a NaN: 2831 x 1024 x 1024 52 / 64 / 77, 2048 x 2048 x 2048 with two
+// weights 212 / 252 / 329 (gemm_any_f32_kernel 69 and 321 whatever the numbers are).
 // Rows beyond the group's end and features beyond N are read from the last valid one and not stored.  Needs what gemm_any_f32_kernel needs.
 template <bool DUAL, bool EXT, int GROUPS>
 __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
@@ -179,20 +181,67 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
       step(std::false_type{}, kt + 1, ra);
     }
     if (kt < KT) step(std::false_type{}, kt, rb);
-    bool redo = false;
+    bool finite = true;
 #pragma unroll
     for (int d = 0; d < ND; ++d)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          acc[d][i][j] += low[d][i][j];
+          acc[d][i][j] = (acc[d][i][j] + low[d][i][j]) * kSplitUnscale;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            redo |= !(fabsf(acc[d][i][j][r]) <= FLT_MAX);
-            acc[d][i][j][r] *= kSplitUnscale;
-          }
+          for (int r = 0; r < 4; ++r) finite &= fabsf(acc[d][i][j][r]) <= FLT_MAX;
         }
+    if (__builtin_expect(__any(!finite), 0)) {
+      // the wave's outputs on the fp32 matrix instruction, k in gemm_any_f32_kernel's order; each that was not finite, and only those, from here
+      const float *xr[FM], *wr[ND][FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int m = min(m0 + (wm + i) * 16 + r16, m_hi - 1);
+        xr[i] = x + (a.x_rows ? a.x_rows[m] : m) * a.ldx + kg * 4;
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) wr[d][j] = (DUAL && d ? w2 : w) + (int64_t)min(n0 + (wn + j) * 16 + r16, a.N - 1) * a.K + kg * 4;
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) low[d][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int k = 0; k < a.K; k += BK) {
+        f32x4 xf[2][FM], wf[2][ND][FN];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+          for (int i = 0; i < FM; ++i) xf[h][i] = *reinterpret_cast<const f32x4*>(xr[i] + k + h * 16);
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) wf[h][d][j] = *reinterpret_cast<const f32x4*>(wr[d][j] + k + h * 16);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+#pragma unroll
+              for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                  low[d][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[h][d][j][e], xf[h][i][e], low[d][i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[d][i][j][r] = fabsf(acc[d][i][j][r]) <= FLT_MAX ? acc[d][i][j][r] : low[d][i][j][r];
+    }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       const int m = m0 + (wm + i) * 16 + r16;
@@ -201,22 +250,6 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         const int n = n0 + (wn + j) * 16 + kg * 4;
-        if (__builtin_expect(redo, 0)) {
-          const float* xr = x + (a.x_rows ? a.x_rows[m] : m) * a.ldx;
-#pragma unroll
-          for (int d = 0; d < ND; ++d)
-            for (int r = 0; r < 4; ++r) {
-              const float* wr = (DUAL && d ? w2 : w) + (int64_t)min(n + r, a.N - 1) * a.K;
-              float v = 0.f;
-              for (int k = 0; k < a.K; k += 4) {
-                const f32x4 xv = *reinterpret_cast<const f32x4*>(xr + k), wv = *reinterpret_cast<const f32x4*>(wr + k);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v = fmaf(xv[e], wv[e], v);
-              }
-#pragma unroll
-              for (int q = 0; q < 4; ++q) acc[d][i][j][q] = q == r ? v : acc[d][i][j][q];
-            }
-        }
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r)

@@ -95,3 +95,29 @@ def test_split_products_of_small_operands(ops, a, b):
     want = x.double() @ w.double().T
     # as of ordinary operands: 2^-24 a rounding; a bf16 part less is 3.5e-6
     assert float((y.double() - want).norm() / want.norm()) <= 4e-7
+
+
+# rows that have no finite parts (NaN, infinities, numbers from 2^104 on) in a batch: every other row's bits, those 16 rows on among them, are its own, and
+# a row whose outputs are finite all the same has the fp32 kernel's accuracy
+@pytest.mark.parametrize("dual", [False, True])
+def test_split_products_rows_keep_their_bits(ops, dual):
+    from nanovllm import _C
+
+    M, N, K = 2049, 2050, 1024
+    g = torch.Generator().manual_seed(11)
+    x, w, w2 = (torch.randn(n, K, generator=g).to(DEV) for n in (M, N, N))
+    product = lambda rows: ops.gemm_any_act(rows, w, act=_C.ACT_SILU if dual else _C.ACT_NONE, w2=w2 if dual else None, exact=True)
+    want = product(x)
+    odd = x.clone()
+    bad = {5: float("nan"), 70: float("inf"), 83: 2.0 ** 105, 1000: 3.4e38, 2032: float("-inf"), 2048: 2.0 ** 120}
+    for r, v in bad.items():
+        odd[r, r % K] = v
+    odd[86] *= 2.0 ** 100   # (sums beyond 2^80)
+    got = product(odd)
+    same = torch.ones(M, dtype=torch.bool, device=DEV)
+    same[list(bad) + [86]] = False
+    assert torch.equal(got[same].view(torch.int32), want[same].view(torch.int32))
+    if not dual:
+        big = odd[[83, 86]].double() @ w.double().T
+        assert bool(((got[[83, 86]].double() - big).abs() <= _bound(odd[[83, 86]], w, K)).all())
+    assert bool(got[5].isnan().all()) and not bool(got[70].isfinite().any())
