@@ -1198,20 +1198,23 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
 #define MI_F32_TILE(FM, FN, WM, WN, AHEAD)                                                                                          \
   gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, 0, AHEAD>, gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 1, AHEAD>, \
       gemm_any_f32_kernel<TW, DUAL, FM, FN, WM, WN, EXT, EXT ? 0 : 2, AHEAD>
-    // fp32 weights of larger launches: gemm_any_split_kernel, by the same model.  It has some 6 us more to begin with (32 with two weights: a step alone on its
-    // CU is a chain of read, split, write and multiply) and then, per 1024 of K, 13 us for every 256 tiles of 64 x 64; two weights above: ragged groups and
-    // the tile each looks for take 1.2 of the model's time.  Without groups from two tiles per CU on, one weight of groups from four tiles a group on: below
-    // it gains nothing or, groups, loses.  us, above / split: 721 rows x 1024 x 1024 24 / 28, x 2048 41 / 40, x 3072 60 / 50; 32 experts, 1024 -> 2 x 512: 400 pairs 56 / 65,
-    // 1200 66 / 69, 2884 90 / 79.  Steps of four layers, neither / products without groups / experts' first / experts' second: width 1024, 721 rows (90 pairs an
-    // expert) 1356 / 1338 / 1339 / 1400, 2831 rows (354) 3271 / 3010 / 3003 / 3236; width 2048, 381 rows (48) 2706 / 2724 (from two tiles per CU on 2672) / 2546 / 2776,
-    // 2461 rows (307) 11032 / 10415 / 9670 / 10745, all three 8690.  (431 rows of width 1024, 54 pairs an expert: experts' first 1024 / 1041, and not taken.)
+    // fp32 weights of larger launches: gemm_any_split_kernel, by a model of its own against that of the tiles above (times two for two weights).  Per 1024 of K
+    // it takes some 13 us for every 256 tiles of 64 x 64 and 26 for two weights; alone on its CU a tile is a chain of read, split, write and multiply: 6 us more
+    // and, two weights, 32.  Without groups from two tiles per CU on.  Two weights of groups, whose last tiles are half empty and which look for their tiles: 30
+    // us a round and one round more.  One weight of groups is not taken: launches by themselves were 0.92 of the time, a step of four layers with 2831 rows (354
+    // an expert) 3068 us with them and 3003 without.  Over 5600 drawn products (64 to 9000 rows, 64 to 6200 features, K 64 to 4096; batches; 2 to 128
+    // groups of up to 45000 pairs in all, even and uneven), one at a time and back to back, those taken: 0.83 of the time above without groups (450 of 2091; two
+    // weights 0.77, 104 of 756), batches 0.84 (128 of 380), groups 0.79 (644 of 2115); 7 of them slower by more than 1 % (6 % at most).  us, above / split: 721 rows
+    // x 1024 x 1024 25 and not taken, x 3072 61 / 57, 2831 x 1024 x 1024 69 / 58, 4096 x 4096 x 4096 1127 / 991; 32 experts, 1024 -> 2 x 512, 11324 pairs 276 / 241; 64
+    // experts, 2048 -> 2 x 768, 5768 pairs 449 / 486 and not taken, 19688 pairs 1169 / 1067.
     if constexpr (sizeof(TW) == 4) {
       const double row_tiles = grouped ? std::max(rows_per_group_max / 64. + groups / 2., (double)groups) : (double)((rows_per_group_max + 63) / 64) * groups;
       const double n = row_tiles * nx(64) / 256., k = a.K / 1024.;
-      const double split_us = DUAL ? 32. + 26. * k * (grouped ? std::max(n, 1.) : std::ceil(n)) : 6. + 13. * k * (grouped ? std::max(n, 1.) : std::ceil(n));
-      const bool fills = grouped ? DUAL || rows_per_group_max >= 256 * (int64_t)groups : rows_per_group_max / 64. * groups * nx(64) / 256. >= 2.;
-      if (a.N > 32 && fills && split_us < std::min(large, std::min(medium, small)) * (DUAL ? grouped ? 2.4 : 2. : 1.) * k) {
-        go(gemm_any_split_kernel<DUAL, EXT, 0>, gemm_any_split_kernel<DUAL, EXT, EXT ? 0 : 1>, gemm_any_split_kernel<DUAL, EXT, EXT ? 0 : 2>, grid(64, 64));
+      const double split_us = grouped ? 30. * k * (n + 1.) : DUAL ? 32. + 26. * k * std::ceil(n) : 6. + 13. * k * std::ceil(n);
+      const bool fills = grouped ? DUAL : rows_per_group_max / 64. * groups * nx(64) / 256. >= 2.;
+      if (a.N > 32 && fills && split_us < std::min(large, std::min(medium, small)) * (DUAL ? 2. : 1.) * k) {
+        constexpr int GROUPS = DUAL && !EXT;   // (the forms that are taken)
+        go(gemm_any_split_kernel<DUAL, EXT, 0>, gemm_any_split_kernel<DUAL, EXT, GROUPS>, gemm_any_split_kernel<DUAL, EXT, 2 * GROUPS>, grid(64, 64));
         return check_launch();
       }
     }

@@ -30,21 +30,24 @@ __device__ __forceinline__ SplitParts split_parts(const f32x4& a, const f32x4& b
 }
 
 // 64 x 64 tiles, four waves with 2 x 2 fragments of 16 x 16 each (two weights: of each), K in steps of 32.  A step's operands travel memory -> registers (two
-// steps ahead) -> three bf16 parts -> LDS (two images, one barrier a step), each number split once per workgroup; the products h h, h m, m h,
-// m m, h l and l h on v_mfma_f32_16x16x32_bf16, those with a rest in a sum of their own.  The products left out are below 2^-25 of |x w|; a step of
-// 32 k is rounded once into each sum where the fp32 matrix instruction rounds eight times: error against 64 bits (2-norm) 1.9e-7 at K =
-// 1024 and 4.0e-7 at 4096, the fp32 instruction's (gemm_any_f32_kernel) 5.7e-7 and 1.15e-6.
-// What bounds it: the fp32 matrix rate is 1/16 of the bf16 one, so six products are 3/8 of its time; the split (thirteen vector instructions for
+// steps ahead) -> three bf16 parts -> LDS (two images, one barrier a step), each number split once per workgroup; all products of parts but l l on
+// v_mfma_f32_16x16x32_bf16, h h in one sum and the seven others, smallest first, in another.  Left out: below 2^-34 of |x w|, so that a sum of one product is
+// rounded as fp32 arithmetic rounds it (without m l and l m, which reach 2^-24 together, up to 0.95 of a last bit).  A step of 32 k is rounded
+// once into each sum where the fp32 matrix instruction rounds eight times: error against 64 bits (2-norm) 1.9e-7 at K = 1024 and 4.0e-7 at 4096, the fp32
+// instruction's (gemm_any_f32_kernel) 5.7e-7 and 1.15e-6.
+// What bounds it: the fp32 matrix rate is 1/16 of the bf16 one, so eight products are half of its time; the split (thirteen vector instructions for
 // two numbers) and the LDS (24 KB written and 48 KB read per step) take about as long as the products beside them, and the clock falls with the matrix
-// pipe's load.  The matrix instructions stand among the next step's split (one tile alone on its CU 34.7 -> 27.9 us, 721 x 1024 x 1024).
-// us with cold weights, gemm_any_f32_kernel / here: 4096 x 4096 x 4096 1129 / 827, 1500 x 4096 x 2048 241 / 180, 721 x 3072 x 1024 60 / 50; 5768 pairs
-// of 64 experts, 2048 -> 2 x 768 477 / 408, back 241 / 237.  128-row tiles are 8 % faster at 4096 x 4096 x 4096 and lose with their fewer
-// tiles below it and with uneven groups (a step of 721 rows 1311 us, 1337 with 128 x 32 of two weights, 1347 with 48 x 64).
+// pipe's load.  The matrix instructions stand among the next step's split (one tile alone on its CU, of six products, 34.7 -> 27.9 us, 721 x 1024 x 1024).
+// us with cold weights, gemm_any_f32_kernel / here: 4096 x 4096 x 4096 1127 / 970-1010, 1500 x 4096 x 2048 237 / 200, 721 x 3072 x 1024 61 / 57; 11324 pairs of
+// 32 experts, 1024 -> 2 x 512, 276 / 241.  Steps of four layers without / with it: width 1024, 1327 rows 1840 / 1760, 2831 rows 3237 / 2890; width 2048, 2831 rows
+// 12400 / 11210.  128-row tiles were 8 % faster at 4096 x 4096 x 4096 and lose with their fewer tiles below it and with uneven groups (a step of 721
+// rows 1311 us, 1337 with 128 x 32 of two weights, 1347 with 48 x 64; all with six products).
 // An infinity has no finite rest, a number of 2^104 and more times 2^24 is one, and so may a sum of 2^80 and more be: a wave with an output
 // that is not finite sums its outputs once more on the fp32 matrix instruction, and takes from there those that were not finite and no other (an output is a
 // function of its own row of x and of the weights).  us, no / one / forty rows with a NaN: 2831 x 1024 x 1024 52 / 64 / 77, 2048 x 2048 x 2048 with two
 // weights 212 / 252 / 329 (gemm_any_f32_kernel 69 and 321 whatever the numbers are).
 // Rows beyond the group's end and features beyond N are read from the last valid one and not stored.  Needs what gemm_any_f32_kernel needs.
+// GROUPS: as in gemm_any_f32_kernel.
 template <bool DUAL, bool EXT, int GROUPS>
 __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
   constexpr int FM = 2, FN = 2, WM = 2, WN = 2, BM = 16 * FM * WM, BN = 16 * FN * WN, BK = 32, ND = DUAL ? 2 : 1;
@@ -144,7 +147,7 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
               sum[d][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, p.w[sw][d][j]), __builtin_bit_cast(bf16x8, p.x[sx][i]),
                                                                      sum[d][i][j], 0, 0, 0);
       };
-      all(2, 0, low), all(0, 2, low), all(1, 1, low), all(1, 0, low), all(0, 1, low), all(0, 0, acc);
+      all(2, 1, low), all(1, 2, low), all(2, 0, low), all(0, 2, low), all(1, 1, low), all(1, 0, low), all(0, 1, low), all(0, 0, acc);
     };
     request(0, ra);
     if (1 < KT) request(1, rb);
@@ -160,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
       if (INSIDE || kt + 3 < KT) request(kt + 3, next);
       multiply(p);
       // reads, some of the split in their shadow, then its rest and its LDS writes among the matrix instructions
-      constexpr int MULS = 6 * ND * FM * FN, VALU = U * 52, EACH = MULS / (3 * U);
+      constexpr int MULS = 8 * ND * FM * FN, VALU = U * 52, EACH = MULS / (3 * U);
       __builtin_amdgcn_sched_group_barrier(0x100, 3 * (FM + ND * FN), 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
 #pragma unroll

@@ -121,3 +121,16 @@ def test_split_products_rows_keep_their_bits(ops, dual):
         big = odd[[83, 86]].double() @ w.double().T
         assert bool(((got[[83, 86]].double() - big).abs() <= _bound(odd[[83, 86]], w, K)).all())
     assert bool(got[5].isnan().all()) and not bool(got[70].isfinite().any())
+
+
+def test_split_products_of_single_terms(ops):
+    """sums of one nonzero product, which fp32 arithmetic rounds once: what is left out (l l, below 2^-34 of it) and the rounding of the low sum (below
+    2^-31) are some 0.01 of a last bit"""
+    M, N, K = 2049, 2050, 1024
+    g = torch.Generator().manual_seed(17)
+    at = torch.randint(0, K, (M,), generator=g).to(DEV)
+    x, w, v = torch.zeros(M, K, device=DEV), torch.randn(N, K, generator=g).to(DEV), torch.randn(M, generator=g).to(DEV)
+    x[torch.arange(M, device=DEV), at] = v
+    want = v.double()[:, None] * w.double().T[at]
+    ulp = torch.exp2(torch.floor(torch.log2(want.abs())) - 23)
+    assert float(((ops.gemm_any(x, w, exact=True).double() - want).abs() / ulp).max()) <= 0.52
