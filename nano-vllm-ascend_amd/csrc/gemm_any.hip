@@ -1201,20 +1201,23 @@ static int launch_exact(const GemmAnyArgs& args, int groups, int rows_per_group_
     // fp32 weights of larger launches: gemm_any_split_kernel, by a model of its own against that of the tiles above (times two for two weights).  Per 1024 of K
     // it takes some 13 us for every 256 tiles of 64 x 64 and 26 for two weights; alone on its CU a tile is a chain of read, split, write and multiply: 6 us more
     // and, two weights, 32.  Without groups from two tiles per CU on.  Two weights of groups, whose last tiles are half empty and which look for their tiles: 30
-    // us a round and one round more.  One weight of groups is not taken: launches by themselves were 0.92 of the time, a step of four layers with 2831 rows (354
-    // an expert) 3068 us with them and 3003 without.  Over 5600 drawn products (64 to 9000 rows, 64 to 6200 features, K 64 to 4096; batches; 2 to 128
-    // groups of up to 45000 pairs in all, even and uneven), one at a time and back to back, those taken: 0.83 of the time above without groups (450 of 2091; two
-    // weights 0.77, 104 of 756), batches 0.84 (128 of 380), groups 0.79 (644 of 2115); 7 of them slower by more than 1 % (6 % at most).  us, above / split: 721 rows
-    // x 1024 x 1024 25 and not taken, x 3072 61 / 57, 2831 x 1024 x 1024 69 / 58, 4096 x 4096 x 4096 1127 / 991; 32 experts, 1024 -> 2 x 512, 11324 pairs 276 / 241; 64
-    // experts, 2048 -> 2 x 768, 5768 pairs 449 / 486 and not taken, 19688 pairs 1169 / 1067.
+    // us a round and one round more (launches with a workgroup for every tile of a group are smaller).  One weight of groups is not taken: launches by themselves
+    // were 0.92 of the time, a step of four layers with 2831 rows (354 an expert) 3068 us with them and 3003 without.  Over 5600 drawn products (64 to 9000
+    // rows, 64 to 6200 features, K 64 to 4096; batches; 2 to 128 groups of up to 45000 pairs in all, even and uneven), one at a time and back to back, those
+    // taken: 0.83 of the time above without groups (450 of 2091; two weights 0.77, 104 of 756), batches 0.84 (128 of 380), groups 0.79 (644 of 2115); 7 of
+    // them slower by more than 1 % (6 % at most).  us, above / split: 721 rows x 1024 x 1024 25 and not taken, x 3072 61 / 57, 2831 x 1024 x 1024 69 / 58,
+    // 4096 x 4096 x 4096 1127 / 991; 32 experts, 1024 -> 2 x 512, 11324 pairs 276 / 241; 64 experts, 2048 -> 2 x 768, 5768 pairs 449 / 486 and not
+    // taken, 19688 pairs 1169 / 1067.
     if constexpr (sizeof(TW) == 4) {
       const double row_tiles = grouped ? std::max(rows_per_group_max / 64. + groups / 2., (double)groups) : (double)((rows_per_group_max + 63) / 64) * groups;
       const double n = row_tiles * nx(64) / 256., k = a.K / 1024.;
       const double split_us = grouped ? 30. * k * (n + 1.) : DUAL ? 32. + 26. * k * std::ceil(n) : 6. + 13. * k * std::ceil(n);
-      const bool fills = grouped ? DUAL : rows_per_group_max / 64. * groups * nx(64) / 256. >= 2.;
+      const bool fills = grouped ? DUAL && grid(64, 64).z == 1 : rows_per_group_max / 64. * groups * nx(64) / 256. >= 2.;
       if (a.N > 32 && fills && split_us < std::min(large, std::min(medium, small)) * (DUAL ? 2. : 1.) * k) {
-        constexpr int GROUPS = DUAL && !EXT;   // (the forms that are taken)
-        go(gemm_any_split_kernel<DUAL, EXT, 0>, gemm_any_split_kernel<DUAL, EXT, GROUPS>, gemm_any_split_kernel<DUAL, EXT, 2 * GROUPS>, grid(64, 64));
+        constexpr bool GROUPS = DUAL && !EXT;   // (the forms that are taken)
+        const dim3 g = grid(64, 64);
+        if (grouped) hipLaunchKernelGGL((gemm_any_split_kernel<DUAL, EXT, GROUPS>), g, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((gemm_any_split_kernel<DUAL, EXT, false>), g, dim3(256), 0, st, a);
         return check_launch();
       }
     }

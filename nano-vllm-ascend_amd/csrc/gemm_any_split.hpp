@@ -44,11 +44,11 @@ __device__ __forceinline__ SplitParts split_parts(const f32x4& a, const f32x4& b
 // rows 1311 us, 1337 with 128 x 32 of two weights, 1347 with 48 x 64; all with six products).
 // An infinity has no finite rest, a number of 2^104 and more times 2^24 is one, and so may a sum of 2^80 and more be: a wave with an output
 // that is not finite sums its outputs once more on the fp32 matrix instruction, and takes from there those that were not finite and no other (an output is a
-// function of its own row of x and of the weights).  us, no / one / forty rows with a NaN: 2831 x 1024 x 1024 52 / 64 / 77, 2048 x 2048 x 2048 with two
-// weights 212 / 252 / 329 (gemm_any_f32_kernel 69 and 321 whatever the numbers are).
+// function of its own row of x and of the weights).  us, no / one / forty rows with a NaN: 2831 x 1024 x 1024 56 / 69 / 78, 2048 x 2048 x 2048 with two
+// weights 233 / 273 / 343 (gemm_any_f32_kernel 69 and 321 whatever the numbers are).
 // Rows beyond the group's end and features beyond N are read from the last valid one and not stored.  Needs what gemm_any_f32_kernel needs.
-// GROUPS: as in gemm_any_f32_kernel.
-template <bool DUAL, bool EXT, int GROUPS>
+// GROUPS: a workgroup finds its tiles, every gridDim.y-th row tile of all groups.
+template <bool DUAL, bool EXT, bool GROUPS>
 __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
   constexpr int FM = 2, FN = 2, WM = 2, WN = 2, BM = 16 * FM * WM, BN = 16 * FN * WN, BK = 32, ND = DUAL ? 2 : 1;
   constexpr int FRAGS = BM / 16 + ND * BN / 16, PLANE = FRAGS * 1024, STAGE = 3 * PLANE, U = FRAGS / 4;
@@ -62,14 +62,9 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
     int m0 = tile * BM, m_hi = a.M;
     const float *x = a.x, *w = static_cast<const float*>(a.w), *w2 = static_cast<const float*>(a.w2);
     float* y = a.y;
-    if constexpr (GROUPS != 0) {
-      int g = blockIdx.z;
-      if constexpr (GROUPS == 1) {
-        m0 = a.group_offsets[g] + tile * BM, m_hi = a.group_offsets[g + 1];
-        if (m0 >= m_hi) return;
-      } else {
-        if (!group_tile<BM>(a.group_offsets, a.n_groups, tile, g, m0, m_hi)) return;
-      }
+    if constexpr (GROUPS) {
+      int g;
+      if (!group_tile<BM>(a.group_offsets, a.n_groups, tile, g, m0, m_hi)) return;
       w += (int64_t)g * a.N * a.K;
       if (DUAL) w2 += (int64_t)g * a.N * a.K;
     } else {
@@ -267,7 +262,7 @@ __global__ __launch_bounds__(256, 2) void gemm_any_split_kernel(GemmAnyArgs a) {
         }
       }
     }
-    if constexpr (GROUPS != 2) return;
+    if constexpr (!GROUPS) return;
   }
 }
 
