@@ -1,4 +1,4 @@
-"""The tile GEMM's small shapes (csrc/gemm_mid_kernel.hpp: 64 x 128 and 64 x 64 tiles; 65 .. some hundred rows), its K slices, and the
+"""The tile GEMM's small shapes (csrc/gemm_mid_kernel.hpp; 65 .. some hundred rows), its K slices, and the
 sampler's candidates from logits in memory (csrc/gemm_pick.hip).
 
 Tolerance: fp32 accumulation of K bf16 products (exact), K * 2^-24 of the sum of magnitudes, then the roundings to bf16 (2^-9 each; SwiGLU
