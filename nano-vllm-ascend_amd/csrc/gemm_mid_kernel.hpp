@@ -1,7 +1,7 @@
 #pragma once
 // ---------------------------------------------------------------------------
-// The same GEMM on 128 x 128 tiles, for shapes whose 256 x 256 tiles cannot fill the chip (64 < M <= ~2048 rows:
-// large decode batches, short prompts).  Four waves, each 64 features x 64 tokens (2 x 2 accumulators); one K step of
+// The same GEMM on smaller tiles, for shapes whose 256 x 256 tiles cannot fill the chip (large decode batches, prompts of
+// some thousand rows).  128 x 128: four waves, each 64 features x 64 tokens (2 x 2 accumulators); one K step of
 // the tile is two 16 KiB half-tiles in the layout of gemm_tile_index.hpp (A: local row = tile feature row, B: local
 // row = tile token row) in a ring of NST stages.  One barrier per K step: "my pieces of step t + 1 have landed" (a COUNTED wait: the
 // pieces of the NST - 2 steps behind it may still fly) and "I have read step t" -> barrier -> step t's matrix instructions, and behind each of

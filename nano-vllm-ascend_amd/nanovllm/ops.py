@@ -464,8 +464,8 @@ def tile_gemm_max_rows(n: int, k: int, ldx: int | None = None) -> int:
 
 
 def gemm_tile(x, w, bias=None, out=None, silu_mul: bool = False, variant: int | None = None) -> torch.Tensor:
-    """y = x @ w.T (+ bias) for any number of rows on the MFMA tile kernels (mi_gemm_bf16: 256 x 256 tiles, 128 x 128
-    for shapes with few of those); silu_mul:
+    """y = x @ w.T (+ bias) for any number of rows on the MFMA tile kernels (mi_gemm_bf16: 256 x 256 tiles, smaller
+    ones for shapes with few of those); silu_mul:
     w stacks gate | up rows and y = SiluAndMul(x @ w.T).  x may be a row-strided 2-D view."""
     require_gpu(x, w, bias)
     _bf16(x, w, bias)
