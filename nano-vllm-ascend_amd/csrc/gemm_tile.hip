@@ -489,10 +489,10 @@ static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
 // modelled time is the least; all give the same bits but for the slices.  Modelled: a launch, the rounds of its tiles, the K steps of a round - which take
 // the longer the more of the chip's places are in use (the L2s' rate: (F + T) 128 bytes per tile and step) - and with K slices the fp32 partial sums out
 // and back and the second launch.  The constants are fitted to random products (65 .. 6000 rows, K from 512 on; 64 x 128: 677 of them, 6 % off in the mean,
-// the others 7 to 14 %), those of 64 x 64 and 128 x 64 corrected by whole prompt steps, whose activations another kernel has just written (1260 rows, 28
+// the others 7 to 14 %; a launch of the two-place shapes by 500 of K 64 to 512), those of 64 x 64 and 128 x 64 corrected by whole prompt steps, whose activations another kernel has just written (1260 rows, 28
 // layers, us a step with o on 128 x 64 / 64 x 64 3131 / 3084, down 3131 / 3045).  Over another 674 (K from 256 on, every launch's weights from memory) the
-// choice is 1.1 % above the best shape and number of slices in the mean, SwiGLU 0.7 %; without 64 x 128, the best shape of half of the latter, 2.5 % and
-// 2.8 %.  Two-place shapes: rings of which two fit a CU; 128 x 64 and 128 x 128 have a deeper one too, a tile per CU, whose requests reach further
+// choice is 1.0 % above the best shape and number of slices in the mean, SwiGLU 0.7 %, over the 500 of short K 0.8 and 0.9; without 64 x 128, the best shape
+// of half of the former with SwiGLU, 2.5 % and 2.8 %.  Two-place shapes: rings of which two fit a CU; 128 x 64 and 128 x 128 have a deeper one too, a tile per CU, whose requests reach further
 // ahead.  us, 64 x 64 / 128 x 64 / 128 x 128 / 128 x 192 / 256 x 256 (the better ring of each): 137 x 4096 x 1024 6.2 / 8.8 / 10.3 / 13.6 / 24, 500
 // rows 10.7 / 9.8 / 12.2 / 13.8 / 26, 886 rows 16.2 / 12.9 / 12.8 / 14.4 / 25, 1260 rows 19.1 / 18.8 / 17.9 / 15.8 / 26, 2048 rows 30 / 25 / 22.1 / 28 /
 // 29; 886 x 5120 x 2048 35 / 33 / 32 / 24.8 / 43; 1260 x 1024 x 2048 14.4 / 11.9 / 14.8 / 19.6 / 40, 2450 rows 21.7 / 20.7 / 16.6 / 20.2 / 40; 128 x 64 / 64 x
@@ -505,13 +505,13 @@ struct MidTile {
 };
 // (a tile's two fragments of features are a gate's and an up's with SwiGLU: 64 x 64 has one only)
 enum { kMid128, kMid128Pairs, kMid128x64Pairs, kMid128x64, kMid128x192, kMid64x128, kMid64, kMidTileCount };
-constexpr MidTile kMidTiles[kMidTileCount] = {{128, 128, 1, 2.2, 1.8, 0.32, 0.24, 0., 0.},     {128, 128, 2, 0.7, 1.8, 0.57, 0.27, 0.89, 0.10},
+constexpr MidTile kMidTiles[kMidTileCount] = {{128, 128, 1, 2.2, 1.8, 0.32, 0.24, 0., 0.},     {128, 128, 2, 1.5, 1.8, 0.57, 0.27, 0.89, 0.10},
                                               {128, 64, 2, 3.3, 0., 0.29, 0.18, 0.60, 0.18},  {128, 64, 1, 2.8, 1.4, 0.21, 0.21, 0., 0.},
-                                              {128, 192, 1, 1.7, 3.1, 0.43, 0.29, 0., 0.},     {64, 128, 2, 2.9, 0., 0.25, 0.10, 0.52, 0.15},
-                                              {64, 64, 2, 3.1, 0., 0.14, 0.08, 0.32, 0.12}};
+                                              {128, 192, 1, 1.7, 3.1, 0.43, 0.29, 0., 0.},     {64, 128, 2, 2.8, 0., 0.25, 0.10, 0.52, 0.15},
+                                              {64, 64, 2, 2.75, 0., 0.14, 0.08, 0.32, 0.12}};
 constexpr MidTile kLargeTile = {256, 256, 1, 3.1, 3.7, 1.04, 0.48, 0., 0.};
-// the sum of K slices: its launch and its bytes (a launch of 2 us misses the best of all shapes and numbers of slices by 1.1 % over the 674 products, one of 3.2 by
-// 1.4 and of 1 by 1.1; us, best with / without: 361 x 384 x 2560 9.4 / 13.2, 127 x 1984 x 3456 13.4 / 17.4, 166 x 2048 x 3456 13.1 / 15.7)
+// the sum of K slices: its launch and its bytes (a launch of 2 us misses the best of all shapes and numbers of slices by 1.0 % over the 674 products, one of 3.2 by
+// 1.3; us, best with / without: 361 x 384 x 2560 9.4 / 13.2, 127 x 1984 x 3456 13.4 / 17.4, 166 x 2048 x 3456 13.1 / 15.7)
 constexpr double kLaunchUs = 2.0, kPartialBytesPerUs = 4.0e6;
 
 // fewer 256-tiles than CUs

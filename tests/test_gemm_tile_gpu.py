@@ -282,18 +282,18 @@ def test_gemm_tile_small_shapes_one_chain(ops, M, N, K):
                                    (886, 6144, 1024),     # 128 x 192, 128 x 192, 64 x 128
                                    (320, 6144, 1024),     # 64 x 64, 128 x 64/2, 128 x 64/2
                                    (500, 4096, 1024),     # 64 x 128, 64 x 128, 128 x 128/2
-                                   (1025, 1024, 2048),    # 64 x 128, 64 x 128, 128 x 128/2
+                                   (1025, 1024, 2048),    # 64 x 128, 64 x 128, 128 x 192
                                    (640, 6144, 1024),     # 128 x 128, 128 x 128, 128 x 128/2
-                                   (65, 256, 64),         # 128 x 128/2, 128 x 128/2, -
-                                   (257, 11020, 320),     # 128 x 64/2, -, -
-                                   (1100, 10100, 64),     # 64 x 128, -, -
-                                   (100, 256, 2176),      # 64 x 64 in 2 slices, 128 x 64, -
-                                   (65, 700, 512),        # 64 x 64, -, 64 x 128
-                                   (129, 5392, 2048),     # 64 x 64, -, 128 x 192
-                                   (129, 10420, 512),     # 64 x 64, -, 128 x 64/2
+                                   (65, 256, 64),         # 64 x 64, 64 x 128, -
+                                   (65, 11712, 64),       # 64 x 128, -, -
+                                   (257, 16924, 128),     # 128 x 128/2, -, -
+                                   (385, 13056, 128),     # 128 x 128/2, 128 x 128/2, -
+                                   (129, 18492, 448),     # 128 x 64/2, -, -
+                                   (137, 8448, 1664),     # 64 x 64, 128 x 64, -
+                                   (65, 2888, 256),       # 64 x 64, -, 64 x 128
+                                   (129, 5712, 1536),     # 64 x 128, -, 128 x 192
                                    (65, 68, 512),         # 64 x 64, -, 64 x 64
-                                   (65, 80, 2304),        # 64 x 64 in 4 slices, -, 64 x 64
-                                   (65, 136, 2048)])      # 64 x 128 in 16 slices, -, 64 x 64
+                                   (65, 80, 2304)])       # 64 x 64 in 4 slices, -, 64 x 64
 def test_gemm_tile_small_shapes_epilogues(ops, M, N, K):
     g, x, w = _case(M, N, K, seed=29)
     b = torch.randn(N, generator=g).bfloat16()
