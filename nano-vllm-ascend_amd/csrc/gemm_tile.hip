@@ -625,7 +625,7 @@ extern "C" int mi_gemm_bf16(const mi_bf16* x, int64_t ldx, const mi_bf16* w, con
                             mi_stream stream) {
   const int rc = check_tile_gemm(x, ldx, w, bias, y, ldy, M, N, K, epilogue);
   if (rc != MI_OK || M == 0) return rc;
-  TileArgs a{x, w, bias, y, ldx, ldy, M, N, K, (N + TILE_F - 1) / TILE_F, (M + TILE_T - 1) / TILE_T, nullptr};
+  TileArgs a{x, w, bias, y, ldx, ldy, M, N, K, (N + TILE_F - 1) / TILE_F, (M + TILE_T - 1) / TILE_T, 0, nullptr};
   hipStream_t st = S(stream);
   const MidPick pick = tile_plan(M, N, K, epilogue == 1);
   const bool mid = pick.tile >= 0;
@@ -653,7 +653,7 @@ extern "C" int mi_gemm_bf16_splitk(const mi_bf16* x, int64_t ldx, const mi_bf16*
   if (rc != MI_OK) return rc;
   if (ksplit < 1 || ksplit > 65535 || K % ((int64_t)BK * ksplit)) return MI_EUNSUPPORTED;
   if (M == 0) return MI_OK;
-  TileArgs a{x, w, nullptr, nullptr, ldx, N, M, N, K, 0, 0, partials};
+  TileArgs a{x, w, nullptr, nullptr, ldx, N, M, N, K, 0, 0, 0, partials};
   return launch_mid<TEPI_PARTIAL, false>(a, S(stream), pick_mid(M, N, K, false, ksplit));
 }
 
@@ -672,7 +672,7 @@ extern "C" int mi_gemm_bf16_qkv_store(const mi_bf16* x, int64_t ldx, const mi_bf
     return MI_EUNSUPPORTED;
   if (few_tiles(M, N) || (int64_t)M * ldy * 2 >= ((int64_t)1 << 32)) return MI_EUNSUPPORTED;  // the large-M kernel only
   if (M == 0) return MI_OK;
-  TileArgs a{x, w, bias, qkv, ldx, ldy, M, N, K, N / TILE_F, (M + TILE_T - 1) / TILE_T, nullptr,
+  TileArgs a{x, w, bias, qkv, ldx, ldy, M, N, K, N / TILE_F, (M + TILE_T - 1) / TILE_T, 0, nullptr,
              {k_w, positions, cos_sin, k_cache, v_cache, slots, eps, n_q_heads, n_kv_heads, block_size}};
   const int ntiles = a.tiles_f * a.tiles_t;
   const dim3 grid(ntiles > kPersistentGrid ? kPersistentGrid : ntiles);
@@ -687,7 +687,7 @@ extern "C" int mi_gemm_bf16_ex(const mi_bf16* x, int64_t ldx, const mi_bf16* w, 
                                int K, int variant, mi_stream stream) {
   const int rc = check_tile_gemm(x, ldx, w, nullptr, y, ldy, M, N, K, 0);
   if (rc != MI_OK || M == 0) return rc;
-  const TileArgs a{x, w, nullptr, y, ldx, ldy, M, N, K, (N + TILE_F - 1) / TILE_F, (M + TILE_T - 1) / TILE_T, nullptr};
+  const TileArgs a{x, w, nullptr, y, ldx, ldy, M, N, K, (N + TILE_F - 1) / TILE_F, (M + TILE_T - 1) / TILE_T, 0, nullptr};
   hipStream_t st = S(stream);
   switch (variant) {
     // the product kernel (four waves, 16 x 16 x 32 MFMAs) and its variants

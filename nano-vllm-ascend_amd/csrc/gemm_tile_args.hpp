@@ -23,6 +23,10 @@ struct TileArgs {
   int64_t ldx, ldy;
   int M, N, K;
   int tiles_f, tiles_t;
+  // gemm_mid_kernel: the XCDs share the tiles as 2^xcd_lf runs of features times 2^(3 - xcd_lf) runs of tokens (mid_tile).  (Here, in what would be padding:
+  // at the end it moved AnyTileArgs' own arguments across a 64-byte line, one more to fetch at a launch's start: 0.46 us where other kernels run between, 95 x
+  // 576 x 64 3.4 / 3.9.)
+  int xcd_lf;
   float* part;  // split-K (gridDim.y > 1): fp32 partial sums [gridDim.y][M][N] instead of y
   // TEPI_QKV (mi_gemm_bf16_qkv_store): the K and V heads of the packed qkv projection go straight to the paged cache
   struct QkvStore {
@@ -35,7 +39,6 @@ struct TileArgs {
     float eps;
     int n_q_heads, n_kv_heads, block_size;
   } qkv;
-  int xcd_lf;  // gemm_mid_kernel: the XCDs share the tiles as 2^xcd_lf runs of features times 2^(3 - xcd_lf) runs of tokens (mid_tile)
 };
 
 constexpr int kPersistentGrid = 256;  // one workgroup per CU
