@@ -1061,13 +1061,14 @@ __global__ __launch_bounds__(256) void gemm_any_each_row_kernel(GemmAnyArgs a) {
 }
 
 // Where the streaming kernel is the faster one of it and the tile kernels (us, tile kernels / here).  Without groups and batches every workgroup's
-// copy of the rows outweighs its weights from some number of features on: 24 rows x 32768 x 2048 35.3 / 34.3, 32 x 16384 x 1024 11.9 / 11.3,
-// x 32768 x 2048 36.2 / 37.0; 48 x 6144 x 2048 15.3 / 13.5, x 16384 x 1024 12.3 / 14.2; 64 x 4096 x 1024 9.5 / 8.9, x 16384 x 1024 12.8 / 19.9.
+// copy of the rows outweighs its weights from some number of features on: 24 rows x 32768 x 2048 34.4 / 34.1, 32 x 16384 x 1024 12.0 / 11.5,
+// 48 x 6144 x 2048 14.8 / 13.7, 64 x 4096 x 1024 10.3 / 8.8, 33 x 2048 x 1024 9.3 / 6.4; and, against tile kernels with a longer K loop than now, 32 x 32768 x
+// 2048 36.2 / 37.0, 48 x 16384 x 1024 12.3 / 14.2, 64 x 16384 x 1024 12.8 / 19.9 (the tile kernels now 34.6, 12.1, 12.8).  So are the ratios that follow.
 // Beyond 16384 features and 16 rows a short K is too little work per workgroup (24 x 18432: K 64 1.09 times the tile kernels' time, 256 1.04,
-// 512 0.94); between 8192 and 16384 features a long one leaves a part round of long workgroups (24 x 12288: K 1024 0.95, 2048 1.02, 4096 1.15; 16
+// 512 0.94, now 10.4 / 9.9 us); between 8192 and 16384 features a long one leaves a part round of long workgroups (24 x 12288: K 1024 0.95, 2048 1.02, 4096 1.15; 16
 // rows: 2048 0.90, 4096 1.03; 24 x 16384 x 8192 1.07).  Two weights: 17 rows x 12288 and 16384, K to 1024 1.00 to 1.20, from 2048 on 0.78 to 0.87;
 // 9 rows x 16384, K 128 1.09, 256 0.96.
-// Grouped: up to ten rows a group on average, eight where K is below 1024 (64 experts of 768 x 2048, 8 each 128 / 107, 10 each 120 / 111; 128 of 256
+// Grouped: up to ten rows a group on average, eight where K is below 1024 (64 experts of 768 x 2048, 8 each 128 / 107, now 136 / 118, 10 each 120 / 111; 128 of 256
 // x 512, 10 each 31.8 / 34.6) and none of many short products (944 pairs, 128 experts of 768 x 256: 41 / 54).
 bool any_stream_takes(int rows, int N, int K, int n_groups, bool dual) {
   if (rows <= 8 || K % 64) return false;

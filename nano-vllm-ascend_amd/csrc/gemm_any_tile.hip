@@ -174,7 +174,7 @@ static int64_t row_tiles(int rows, int n_groups, int t) { return n_groups ? rows
 // (Reached by operands that the streaming kernel does not take - x off 16 bytes -, and by mi_expert_ff_bytes, which is 0 here: these products are
 // two calls.)
 // Few pairs over small experts: the operand pass and the rings' first round trips are longer than the general kernels' whole walk (us with
-// weights not in the L2s, both products, general / tile kernels: 8 experts of 256 x 1024, 64 pairs 15.8 / 18.2; 16 of 256 x 512, 96 pairs
+// weights not in the L2s and the tile kernels' K loop longer than now, both products, general / tile kernels: 8 experts of 256 x 1024, 64 pairs 15.8 / 18.2; 16 of 256 x 512, 96 pairs
 // 12.0 / 14.8; 32 of 256 x 512, 32 pairs 13.3 / 14.7, 48 pairs 16.6 / 14.6; 128 of 256 x 256, 24 pairs 12.4 / 13.3; 8 of 512 x 1024,
 // 32 pairs 17.0 / 19.1, 64 pairs 18.8 / 19.1; 128 of 192 x 512, 24 pairs 13.7 / 16.9).  Their time grows with the experts that have a pair
 // (some G P / (G + P)) and their rows of weights; beyond eight pairs an expert they take other kernels.
@@ -190,6 +190,8 @@ static bool few_pairs(int64_t pairs, int N, int K, int64_t G) {
 // misses the best tile's time of by 1.2 % in the mean from K 512 on, 3.7 over all with the line below; by lines in rows per group and tiles, before, 5.2: 64 groups of 276
 // rows, two weights of 320 x 192 35 us for 22, 16 of 1974, 256 x 384 and back 67 for 52, 32 of 145, 1664 x 3456 and back 442 for 367.  1.1: over another 1588
 // products of 24 to 112 rows the larger tile was the better one where the two are near (1.6 % missed in the mean with it, 1.8 without, 2.5 by the lines).
+// The small tiles' K loop has become shorter since, all sizes alike: over 277 other products the choice misses the best tile's time by 1.1 % in the mean from
+// K 512 on and by 6 over all, with the loop of the fit by 5.7.
 static double grouped_us(int t, int rows, int N, int K, int G, bool dual) {
   const int f = t == 64 || !dual ? t : t / 2;
   const int64_t row_tiles = rows / t + G / 2, tiles = (row_tiles < G ? G : row_tiles) * ((N + f - 1) / f), c = (tiles + 255) / 256;
@@ -222,10 +224,11 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
   const int64_t limit = (int64_t)1 << 31;
   if (((int64_t)(n_groups ? n_groups : 1) * N + 256) * K * 2 >= limit || ((int64_t)rows + 256) * K * 2 >= limit) return 0;
   if (N < 64) return 0;
-  // Where the lines lie (us, these kernels incl. the 2 us of the operand pass against gemm_any.hip's; up to 8 rows those do not round x,
-  // and they stay).  No groups, N 2048: K 2048 at 9 rows 13.0 / 13.2, at 32 13.2 / 19.1, at 128 14.4 / 43.2; K 512 at 16 rows 7.1 / 5.9,
-  // at 24 7.2 / 7.2, at 64 7.3 / 10.8; K 256 at 32 rows 6.3 / 5.4, at 64 6.4 / 7.9; K 64 from 65 rows on 5.1 / 5.2.  Experts' pair of
-  // products, 32 of 512 x 1024 (64 of 768 x 2048): 16 pairs 19 / 20 (32 / 50), 128 pairs 28 / 37, (64 pairs 82 / 106).
+  // Where the lines lie (us, these kernels incl. the 2 us of the operand pass against gemm_any.hip's other than the streaming one; up to 8 rows those
+  // do not round x, and they stay).  No groups, N 2048, rows off 16 bytes: K 2048 at 9 rows 11.9 / 17.2, at 32 12.7 / 33.6, at 128 14.3 / 78; K 512
+  // at 16 rows not taken / 7.8, at 24 6.7 / 10.3, at 64 7.0 / 19.7; K 256 at 32 rows not taken / 7.6, at 64 6.3 / 12.5; K 64 from 65 rows on 5.5 / 6.6
+  // (on rows at 16 bytes, with a longer K loop here, the kernels met at those lines: K 512 at 16 rows 7.1 / 5.9, at 24 7.2 / 7.2; K 256 at 32 rows 6.3 / 5.4).
+  // Experts' pair of products, with that loop, 32 of 512 x 1024 (64 of 768 x 2048): 16 pairs 19 / 20 (32 / 50), 128 pairs 28 / 37, (64 pairs 82 / 106).
   if (n_groups ? rows < 16 || (rows < 128 && K < 256) || (pays && few_pairs(rows, N, K, n_groups))
                : !(rows > 64 || (rows > 32 && K >= 128) || (rows > 16 && K >= 512) ||
                    (rows > 8 && !dual && (K >= 2048 || N >= 8192))))
@@ -235,9 +238,10 @@ static int tile_rows_for(int rows, int N, int K, int n_groups, bool dual, int ac
     return cheapest_tile(rows, n_groups, short_k_64(rows, K, n_groups, dual), [=](int t) { return grouped_us(t, rows, N, K, n_groups, dual); });
   // 64-row tiles while they are few; the persistent kernel's 256-row ones where 128-row ones are more than the chip holds (two workgroups per CU).
   const auto tiles = [=](int t, int f) { return (int64_t)((rows + t - 1) / t) * ((N + f - 1) / f); };
-  // us, cold weights, 64- / 128- / 256-row tiles: 2000 x 1024 x 1024 (512 / 128 / 32 tiles) 12 / 16 / 26, 2000 x 2048 x 1024 (1024 / 256 / 64) 23 / 18 / 28,
-  // 4000 x 2048 x 1024 (2016 / 512 / 128) 33 / 27 / 30, 3000 x 3072 x 1024 (2256 / 576 / 144) 41 / 37 / 31; 1000 x 2048 x 2048 (512 / 128 / 32) 22 / 26 / 47,
-  // 1300 (672 / 176 / 48) 29 / 27 / 44, 4000 (2016 / 512 / 128) 53 / 42 / 48, 1300 x 6144 x 2048 (2016 / 528 / 144) 76 / 61 / 46
+  // us, cold weights, 64- / 128- / 256-row tiles: 2000 x 1024 x 1024 (512 / 128 / 32 tiles) 11 / 14 / 26, 2000 x 2048 x 1024 (1024 / 256 / 64) 24 / 17 / 30,
+  // 4000 x 2048 x 1024 (2016 / 512 / 128) 33 / 25 / 30, 3000 x 3072 x 1024 (2256 / 576 / 144) 41 / 35 / 30; 1000 x 2048 x 2048 (512 / 128 / 32) 22 / 24 / 46,
+  // 1300 (672 / 176 / 48) 30 / 22 / 44, 4000 (2016 / 512 / 128) 55 / 40 / 48, 1300 x 6144 x 2048 (2016 / 528 / 144) 77 / 59 / 47; over 200 drawn products the
+  // choice misses the best tile's time by 0.4 % in the mean
   if (tiles(64, 64) <= 512) return 64;
   return act != MI_ACT_SOFTCAP && tiles(128, dual ? 64 : 128) > 512 ? 256 : 128;
 }
@@ -272,7 +276,7 @@ static int launch_any_tile(const AnyTileArgs<ACT, DUAL, GATHER, HALF>& args, int
     }
   } else if (tile_rows == 64) {
     // two weights: 128 feature rows (64 outputs); one: 64, or 128 where that leaves at least four tiles per CU (the experts' second
-    // product, us, 64 / 128 features: 32 experts of 1024 x 512 8.9 / 9.6, 64 of 2048 x 768 41 / 39.5)
+    // product, us, 64 / 128 features: 32 experts of 1024 x 512 8.9 / 9.6, 64 of 2048 x 768 41 / 39.5; with a longer K loop than now)
     const int64_t narrow = row_tiles_max * ((a.N + 63) / 64);
     const bool wide = DUAL || narrow > 4 * kPersistentGrid;
     a.tiles_f = !DUAL && wide ? (a.N + 127) / 128 : (a.N + 63) / 64;
@@ -421,7 +425,8 @@ extern "C" int mi_gemm_any_fit_rounded(const float* x, int64_t ldx, const void* 
 
 // ---- the experts of moe.hip (bf16 activations and weights as they are stored, row-major) on the tile kernels: steps that bring prompts ----
 // moe.hip's kernels keep 16 features' weights in registers and walk an expert's pairs 16 at a time, a round trip and two barriers each:
-// made for the few pairs of a decode step.  us of a block (route to combine) with them / here on 64- / 128- / 256-row tiles:
+// made for the few pairs of a decode step.  us of a block (route to combine) with them / here on 64- / 128- / 256-row tiles (the first two with a longer
+// K loop than now):
 //   64 experts of 768 x 2048     8 pairs each 127 / 146 / 162 / 185   16 153 / 148 / 164 / 188   64 306 / 173 / 183 / 197   128 530 / 229 / 236 / 212
 //                                512 1843 / 620 / 524 / 385
 //   32 of 512 x 1024             8 34 / 34 / 38 / 56   16 40 / 35 / 38 / 56   64 72 / 44 / 44 / 57   192 155 / 62 / 56 / 63   512 360 / 115 / 110 / 106

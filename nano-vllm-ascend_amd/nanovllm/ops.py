@@ -431,9 +431,9 @@ def silu_mul(x, out=None) -> torch.Tensor:
 # fast path of the models, the in-graph sampler and the engine's lookahead all go up to this many sequences
 SKINNY_MAX_M = 512
 # ... but a WIDE projection (qkv, gate_up) goes to the MFMA tile kernels above 64 rows, where the streaming kernel begins to read the
-# rows' weights once per 64 (us: 4096 x 1024 at 72 rows 7.1 vs 10.5, at 200 7.1 vs 18.6; gate_up + SwiGLU of 6144 9.2 vs 11.5 and
-# 9.4 vs 17.1; 2048 x 2048 at 100 rows 10.2 vs 8.1, at 137 10.1 vs 14.0); the narrow ones (1024 x 2048 without K slices at 256 rows
-# 10.6 vs 7.6, at 400 10.7 vs 13.1) stay up to SKINNY_MAX_M rows: steps that are launched eagerly pay more on the host than that gains
+# rows' weights once per 64 (us: 4096 x 1024 at 72 rows 6.2 vs 10.5, at 200 6.5 vs 19.0; gate_up + SwiGLU of 6144 9.5 vs 12.1 and
+# 9.6 vs 18.0; 2048 x 2048 at 100 rows 9.9 vs 8.1, at 137 9.2 vs 13.9); the narrow ones (1024 x 2048 at 256 rows 10.5 vs 7.9, at 400
+# 9.2 vs 13.5) stay up to SKINNY_MAX_M rows: steps that are launched eagerly pay more on the host than that gains
 # (270 rows of a sparse model's 4 layers of width 1024: 770 us per step, 838 with tiles from 257 rows on)
 TILE_MIN_ROWS = 64
 
@@ -668,7 +668,7 @@ def gemm_packed_splitk(x, w_packed, ksplit: int, out=None) -> torch.Tensor:
 
 def gemm_tile_splitk(x, w, ksplit: int, out=None) -> torch.Tensor:
     """fp32 partials [ksplit, M, N] of x @ w.T on the tile kernels (w as stored): gemm_packed_splitk above 64 rows (200 rows, four
-    slices: 1024 x 2048 6.7 vs 8.8 us, 1024 x 3072 6.9 vs 15.2)."""
+    slices: 1024 x 2048 5.3 vs 8.9 us, 1024 x 3072 6.1 vs 15.5)."""
     require_gpu(x, w)
     _bf16(x, w)
     assert x.is_contiguous() and w.is_contiguous() and w.dim() == 2 and x.shape[-1] == w.shape[1]
@@ -1153,8 +1153,10 @@ def _grouped_tiles(x, x_rows, w, w2, act: int, offsets, rows_max: int, y, y_rows
 
 def product_operand(x, dtype) -> torch.Tensor | None:
     """Where a norm puts its rows rounded to bf16 beside x, its fp32 rows, for the products over weights of `dtype` that read them next (their
-    `rounded`), or None.  From 512 rows on: those go to the tile kernels, each of which would otherwise round the rows in a pass of its own
-    (fewer are left as they are: a decode step's products read fp32 rows)."""
+    `rounded`), or None.  From 512 rows on: those go to the tile kernels, each of which would otherwise round the rows in a pass of its own.
+    Fewer are left as they are (a decode step's products of up to 64 rows read fp32 rows), though prompts of 65 to 511 rows would gain about as
+    much.  us of a step of four layers without / with: Felolorn, width 1024, 640 rows 898 / 870, 260 rows 892 / 859; width 2048, 640 rows
+    1591 / 1567, 260 rows 1267 / 1251; Gazutar, width 1024, 640 rows 714 / 706, 260 rows 719 / 712; width 2048 1427 / 1423 and 1174 / 1169."""
     return torch.empty(x.shape, dtype=_BF16, device=x.device) if dtype == _BF16 and x.shape[0] >= 512 and x.shape[1] % 64 == 0 else None
 
 
