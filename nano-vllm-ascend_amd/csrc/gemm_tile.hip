@@ -498,7 +498,7 @@ static int launch_tile(const TileArgs& a, hipStream_t st, int ksplit = 1) {
 // 29; 886 x 5120 x 2048 35 / 33 / 32 / 24.8 / 43; 1260 x 1024 x 2048 14.4 / 11.9 / 14.8 / 19.6 / 40, 2450 rows 21.7 / 20.7 / 16.6 / 20.2 / 40; 128 x 64 / 64 x
 // 128 (another card): with SwiGLU 215 x 6400 x 832 9.6 / 7.9, 314 x 2304 x 2752 22.2 / 19.1, without 348 x 4672 x 1152 11.2 / 9.2.  Against the choice among 64 x 64,
 // 64 x 128, 128 x 128 and 256 x 256 by one time per step each (and that kernel's longer steps), 500 products with weights from memory: 0.89 of the
-// time in the geometric mean, 8 of them slower by more than 2 % (17 % at most).
+// time in the geometric mean, 9 of them slower by more than 2 % (17 % at most).
 struct MidTile {
   int f, t, places;  // features, tokens; tiles that share a CU
   double launch_us, round_us, step_us, step_load_us, pair_us, pair_load_us;
